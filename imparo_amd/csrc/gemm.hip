@@ -1,7 +1,7 @@
 // Y[m, n] = X[m, k] . W[n, k]^T with float32 accumulation.
 //
-// float32: a register-tiled FMA kernel; every output element sums its products
-// in the order k = 0, 1, 2, ... whatever the tile it falls in, so a row's
+// float32: kernels on the matrix cores' float32 products; every output element sums
+// its products in the order k = 0, 1, 2, ... whatever the tile it falls in, so a row's
 // result does not depend on how many other rows are in the batch.
 // bfloat16: MFMA kernels, a 128x128 LDS-tiled one for many rows and a
 // weight-streaming one with the K range split over the waves of a block for
@@ -58,144 +58,256 @@ __device__ __forceinline__ uint4 zero_if(bool out, uint4 v) {
 }
 
 // ------------------------------------------------------------------ float32
+// The float32 matrix instructions round exactly as a chain of fused multiply-adds over k = 0, 1, 2, ... does
+// (checked against fmaf on normal, widely spread and subnormal values: the same bits everywhere), so both kernels
+// below run on the matrix cores, at twice the vector units' rate, and still sum every output in that order.
+//
+// Many rows: a 64x64 tile per block of four waves, 32x32 each, K in steps of 32 through LDS, the loads of
+// three further steps in flight while one is multiplied. Of 8 neighbouring k the even ones lie together in LDS and then the
+// odd ones: lane / 32 picks a half of each product's two k, so one 16-byte read feeds four products. Bound by
+// the matrix cores where there are enough tiles; a long K with few tiles is bound by the chain of a wave's
+// products, 32 cycles a k. Measured, 666 rows: 143 us by 9,216 by 1,024 (88 TFLOP/s), 103 us by 1,024 by 4,608; the
+// LFM2-350M shape's four products 88 us on average where a register-tiled kernel on the vector units took 281.
 #define F32_BM 64
 #define F32_BN 64
-#define F32_BK 16
+#define F32_BK 32
+#define F32_LD 40   // floats from row to row in LDS: 32 bytes beyond a row's own, which keeps 16-byte reads free of conflicts
 
-template <typename TOut>
+// VEC: K is a multiple of 4 and both operands' rows start 16 bytes aligned; else they are read value by value.
+template <typename TOut, bool VEC>
 __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, const float* __restrict__ W,
                                                   const float* __restrict__ bias, TOut* __restrict__ Y,
-                                                  int M, int N, int K, Epilogue epilogue) {
-    __shared__ float As[F32_BK][F32_BM + 4];
-    __shared__ float Bs[F32_BK][F32_BN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16, ty = tid / 16;
-    const int m0 = blockIdx.y * F32_BM, n0 = blockIdx.x * F32_BN;
-    float acc[4][4];
+                                                  int M, int N, int K, int tiles_m, int tiles_n, Epilogue epilogue) {
+    __shared__ __attribute__((aligned(16))) float xs[2][F32_BM * F32_LD];
+    __shared__ __attribute__((aligned(16))) float ws[2][F32_BN * F32_LD];
+    // blocks that share weight rows are neighbours on one XCD (they go to the 8 XCDs in turn, each has an L2)
+    const int total = tiles_m * tiles_n;
+    const int per_xcd = (total + 7) / 8;
+    const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if (logical >= total) return;
+    const int m0 = (logical % tiles_m) * F32_BM, n0 = (logical / tiles_m) * F32_BN;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int row = tid >> 2, part = (tid & 3) * 8;          // a thread brings 8 neighbouring k of one row of each operand
+    const float* xrow = X + (size_t)min(m0 + row, M - 1) * K;
+    const float* wrow = W + (size_t)min(n0 + row, N - 1) * K;
+    struct Ahead {
+        float x[8], w[8];
+    };
+    auto fetch = [&](int k0, Ahead& f) __attribute__((always_inline)) {     // no load under a branch; what lies past K is zero
+        const int k = k0 + part;
+        if (VEC) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+            for (int j = 0; j < 8; j += 4) {
+                const int at = min(k + j, K - 4);
+                const float4 a = *reinterpret_cast<const float4*>(xrow + at), b = *reinterpret_cast<const float4*>(wrow + at);
+                f.x[j] = a.x, f.x[j + 1] = a.y, f.x[j + 2] = a.z, f.x[j + 3] = a.w;
+                f.w[j] = b.x, f.w[j + 1] = b.y, f.w[j + 2] = b.z, f.w[j + 3] = b.w;
+            }
+        } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-
-    for (int k0 = 0; k0 < K; k0 += F32_BK) {
-        // 64 rows x 16 k per operand = 1024 values, 4 per thread
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int e = tid + j * 256;
-            const int r = e / F32_BK, kk = e % F32_BK;
-            const int k = k0 + kk;
-            const int ma = m0 + r, nb = n0 + r;
-            As[kk][r] = (ma < M && k < K) ? X[(size_t)ma * K + k] : 0.f;
-            Bs[kk][r] = (nb < N && k < K) ? W[(size_t)nb * K + k] : 0.f;
+            for (int j = 0; j < 8; ++j) f.x[j] = xrow[min(k + j, K - 1)], f.w[j] = wrow[min(k + j, K - 1)];
         }
-        __syncthreads();
+    };
+    f32x16 acc;
 #pragma unroll
-        for (int kk = 0; kk < F32_BK; ++kk) {
-            float a[4], b[4];
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    const int put = row * F32_LD + part;
+    const int get_x = (wm + (lane & 31)) * F32_LD + (lane >> 5) * 4, get_w = (wn + (lane & 31)) * F32_LD + (lane >> 5) * 4;
+    // One step: its operands leave the registers for LDS, the step after the next two is asked for in their place
+    // (a step takes half a microsecond, a trip to memory one or two), and the products run.
+    auto step = [&](int k0, int buf, Ahead& now) __attribute__((always_inline)) {
+        float x[8], w[8];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < 8; ++j) {
+            const bool in = k0 + part + j < K;
+            x[j] = in ? now.x[j] : 0.f;
+            w[j] = in ? now.w[j] : 0.f;
         }
-        __syncthreads();
+        *reinterpret_cast<float4*>(&xs[buf][put]) = make_float4(x[0], x[2], x[4], x[6]);
+        *reinterpret_cast<float4*>(&xs[buf][put + 4]) = make_float4(x[1], x[3], x[5], x[7]);
+        *reinterpret_cast<float4*>(&ws[buf][put]) = make_float4(w[0], w[2], w[4], w[6]);
+        *reinterpret_cast<float4*>(&ws[buf][put + 4]) = make_float4(w[1], w[3], w[5], w[7]);
+        // (the other buffer was read before the barrier of the step before; the loads in flight are not waited for)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        fetch(k0 + 4 * F32_BK, now);
+        __builtin_amdgcn_sched_barrier(0);   // (left alone, the compiler sinks these loads to where they are used)
+#pragma unroll
+        for (int kb = 0; kb < F32_BK; kb += 8) {
+            const float4 a = *reinterpret_cast<const float4*>(&xs[buf][get_x + kb]);
+            const float4 b = *reinterpret_cast<const float4*>(&ws[buf][get_w + kb]);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Ahead s0, s1, s2, s3;
+    // (in the order they are used: a first use whose loads were issued last would wait for all of them, every round)
+    fetch(0, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(F32_BK, s1);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(2 * F32_BK, s2);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(3 * F32_BK, s3);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int k0 = 0; k0 < K; k0 += 4 * F32_BK) {      // (steps past the end add products of zeros: the sums keep their bits)
+        step(k0, 0, s0);
+        step(k0 + F32_BK, 1, s1);
+        step(k0 + 2 * F32_BK, 0, s2);
+        step(k0 + 3 * F32_BK, 1, s3);
     }
+    // a lane holds one column (a weight row) of 16 activation rows
+    const int n = n0 + wn + (lane & 31);
+    const float bn = bias && n < N ? bias[n] : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
-        if (bias) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int n = n0 + tx * 4 + j;
-                if (n < N) acc[i][j] += bias[n];
-            }
-        }
+    for (int r = 0; r < 16; ++r) {
+        const int m = m0 + wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+        const float v = bias ? acc[r] + bn : acc[r];
         if (epilogue == EPI_SWIGLU) {
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                const int n = n0 + tx * 4 + j;
-                if (n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, acc[i][j], acc[i][j + 1]));
-            }
-            continue;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) store_f32<TOut>(Y, (size_t)m * N + n, acc[i][j]);
+            const float up = __shfl_xor(v, 1, WAVE);             // gate and up rows are neighbours
+            if (m < M && !(lane & 1) && n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, v, up));
+        } else if (m < M && n < N) {
+            store_f32<TOut>(Y, (size_t)m * N + n, v);
         }
     }
 }
 
-// The same sums for at most 16 rows (a decode step in the float32 engine): the tile above would
-// leave three quarters of its rows empty and, with a weight of few rows, most CUs idle. A block
-// takes 32 weight rows; thread (row, pair of weight rows) adds k = 0, 1, 2, ... exactly as the
-// tile kernel does, so a token's sums are the same bits whichever kernel its batch met. The next
-// chunk of K is asked for before the current one is multiplied.
-#define F32R_BN 32
-#define F32R_BK 64
+// At most 16 rows (a decode step in the float32 engine): a wave takes 16 weight rows and all the activation rows
+// and walks K alone, operands from memory straight into registers, 16 bytes a lane: lane (row, g) asks for
+// k = 4g .. 4g + 3 of 16, and a transposition over the four groups of lanes (four lane swaps) gives it
+// k = g, 4 + g, 8 + g, 12 + g, which is how the products want them. Loads run seven chunks of 32 ahead in eight
+// register sets. A weight of many rows is bound by its bytes, one of few rows by the chain of a wave's products (each
+// waits for the one before it). Measured, cold weights, 2 rows: 65,536 by 1,024 57 us (4.7 TB/s), 9,216 by 1,024 14 us,
+// 1,024 by 4,608 33 us; 17 us on average over a decode step where two weight rows a thread through LDS took 79.
+#define F32R_BK 32
+#define F32R_SETS 8
+struct RowsF32Set {
+    f32x4 w[F32R_BK / 16], x[F32R_BK / 16];     // (whole vectors until they are used)
+};
+
+__device__ __forceinline__ void swap_lanes_16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap_lanes_32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+// lane group g, component c  ->  lane group c, component g
+__device__ __forceinline__ void transpose_over_groups(const f32x4& from, float (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = from[i];
+    swap_lanes_32(v[0], v[2]);
+    swap_lanes_32(v[1], v[3]);
+    swap_lanes_16(v[0], v[1]);
+    swap_lanes_16(v[2], v[3]);
+}
+
 template <typename TOut>
-__global__ __launch_bounds__(256) void k_gemm_f32_rows(const float* __restrict__ X, const float* __restrict__ W,
-                                                       const float* __restrict__ bias, TOut* __restrict__ Y,
-                                                       int M, int N, int K, Epilogue epilogue) {
-    __shared__ float Ws[F32R_BK][F32R_BN + 1];
-    __shared__ float Xs[F32R_BK][16 + 1];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16, ty = tid / 16;
-    const int n0 = blockIdx.x * F32R_BN;
-    float acc0 = 0.f, acc1 = 0.f;
-    float wr[8], xr[4];
-    auto fetch = [&](int k0) __attribute__((always_inline)) {
+__global__ __launch_bounds__(64) void k_gemm_f32_rows(const float* __restrict__ X, const float* __restrict__ W,
+                                                      const float* __restrict__ bias, TOut* __restrict__ Y,
+                                                      int M, int N, int K, Epilogue epilogue) {
+    const int lane = threadIdx.x, r16 = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    // (uniform bases and 32-bit offsets inside 16 rows: a load in the loop costs no address arithmetic)
+    const float* wbase = W + (size_t)n0 * K;
+    const unsigned woff = (unsigned)min(r16, N - 1 - n0) * (unsigned)K + g * 4, xoff = (unsigned)min(r16, M - 1) * (unsigned)K + g * 4;
+    const int full = K / F32R_BK;                        // whole chunks; the rest of K, a multiple of 4, comes last
+    auto fetch = [&](int chunk, RowsF32Set& f) __attribute__((always_inline)) {
+        const char* w0 = reinterpret_cast<const char*>(wbase + min(chunk, full - 1) * F32R_BK);
+        const char* x0 = reinterpret_cast<const char*>(X + min(chunk, full - 1) * F32R_BK);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {                    // 32 weight rows x 64 k, a row's 64 values side by side
-            const int e = tid + j * 256;
-            const int r = e / F32R_BK, k = k0 + e % F32R_BK;
-            wr[j] = (n0 + r < N && k < K) ? W[(size_t)(n0 + r) * K + k] : 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {                    // 16 activation rows x 64 k
-            const int e = tid + j * 256;
-            const int r = e / F32R_BK, k = k0 + e % F32R_BK;
-            xr[j] = (r < M && k < K) ? X[(size_t)r * K + k] : 0.f;
+        for (int j = 0; j < F32R_BK / 16; ++j) {
+            f.w[j] = *reinterpret_cast<const f32x4*>(w0 + woff * 4u + j * 64);
+            f.x[j] = *reinterpret_cast<const f32x4*>(x0 + xoff * 4u + j * 64);
         }
     };
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += F32R_BK) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const RowsF32Set& f) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int e = tid + j * 256;
-            Ws[e % F32R_BK][e / F32R_BK] = wr[j];
+        for (int j = 0; j < F32R_BK / 16; ++j) {
+            float w[4], x[4];
+            transpose_over_groups(f.w[j], w);
+            transpose_over_groups(f.x[j], x);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[i], acc, 0, 0, 0);
+        }
+    };
+    if (full > 0) {
+        RowsF32Set set[F32R_SETS];
+        // (in the order they are used: a first use whose loads were issued last would wait for all of them, every round)
+#pragma unroll
+        for (int i = 0; i < F32R_SETS - 1; ++i) {
+            fetch(i, set[i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int rounds = full / F32R_SETS * F32R_SETS;
+        for (int c = 0; c < rounds; c += F32R_SETS) {
+#pragma unroll
+            for (int i = 0; i < F32R_SETS; ++i) {
+                fetch(c + i + F32R_SETS - 1, set[(i + F32R_SETS - 1) % F32R_SETS]);
+                __builtin_amdgcn_sched_barrier(0);       // (left alone, the compiler sinks the loads to where they are used)
+                multiply(set[i]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int e = tid + j * 256;
-            Xs[e % F32R_BK][e / F32R_BK] = xr[j];
-        }
-        __syncthreads();
-        fetch(k0 + F32R_BK);                             // (past the end: nothing is read, zeros)
-#pragma unroll 16
-        for (int kk = 0; kk < F32R_BK; ++kk) {
-            const float a = Xs[kk][ty];
-            acc0 = fmaf(a, Ws[kk][2 * tx], acc0);
-            acc1 = fmaf(a, Ws[kk][2 * tx + 1], acc1);
-        }
-        __syncthreads();
+        for (int i = 0; i < F32R_SETS - 1; ++i)          // the chunks beyond whole rounds: their loads are on their way
+            if (rounds + i < full) multiply(set[i]);
     }
-    const int m = ty, n = n0 + 2 * tx;
+    if (full * F32R_BK < K) {
+        RowsF32Set f;
+#pragma unroll
+        for (int j = 0; j < F32R_BK / 16; ++j) {         // what lies past K counts as zeros
+            const int k = full * F32R_BK + j * 16, at = min(k, K - 4 - g * 4);
+            const bool in = k + g * 4 < K;
+            const float4 w = *reinterpret_cast<const float4*>(wbase + ((long long)woff + at));
+            const float4 x = *reinterpret_cast<const float4*>(X + ((long long)xoff + at));
+            f.w[j] = f32x4{in ? w.x : 0.f, in ? w.y : 0.f, in ? w.z : 0.f, in ? w.w : 0.f};
+            f.x[j] = f32x4{in ? x.x : 0.f, in ? x.y : 0.f, in ? x.z : 0.f, in ? x.w : 0.f};
+        }
+        multiply(f);
+    }
+    // lane: token lane % 16, weight rows 4 * (lane / 16) + i
+    const int m = r16, n = n0 + g * 4;
     if (m >= M) return;
-    if (bias) {
-        if (n < N) acc0 += bias[n];
-        if (n + 1 < N) acc1 += bias[n + 1];
-    }
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = bias && n + i < N ? acc[i] + bias[n + i] : acc[i];
     if (epilogue == EPI_SWIGLU) {
-        if (n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, acc0, acc1));
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            if (n + i + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + (n + i) / 2, gated_mul(epilogue, v[i], v[i + 1]));
         return;
     }
-    if (n < N) store_f32<TOut>(Y, (size_t)m * N + n, acc0);
-    if (n + 1 < N) store_f32<TOut>(Y, (size_t)m * N + n + 1, acc1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < N) store_f32<TOut>(Y, (size_t)m * N + n + i, v[i]);
+}
+
+template <typename TOut>
+static int launch_f32(const float* x, const float* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
+                      hipStream_t s) {
+    const bool vec = k % 4 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w & 15);
+    if (m <= 16 && vec && k < (1 << 25)) {           // (offsets inside 16 rows are kept in 32 bits)
+        k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
+        return launch_status();
+    }
+    const int tiles_m = (m + F32_BM - 1) / F32_BM, tiles_n = (n + F32_BN - 1) / F32_BN;
+    const long long total = (long long)tiles_m * tiles_n;
+    if (total > 0x7ffffff0LL) return IMPARO_BAD_ARGUMENT;
+    const unsigned blocks = (unsigned)((total + 7) / 8 * 8);
+    if (vec)
+        k_gemm_f32<TOut, true><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
+    else
+        k_gemm_f32<TOut, false><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
+    return launch_status();
 }
 
 // ------------------------------------------------------------------ bfloat16, many rows
@@ -1638,25 +1750,11 @@ static int gemm_variant(const void* x, const void* w, const float* bias, void* y
     if (m == 0) return IMPARO_OK;
     hipStream_t s = (hipStream_t)stream;
     if (dtype == IMPARO_F32) {
-        if (m <= 16 && out_dtype == IMPARO_F32) {
-            k_gemm_f32_rows<float><<<(n + F32R_BN - 1) / F32R_BN, 256, 0, s>>>((const float*)x, (const float*)w, bias,
-                                                                             (float*)y, m, n, k, epilogue);
-            return launch_status();
-        }
-        if (m <= 16 && out_dtype == IMPARO_BF16) {
-            k_gemm_f32_rows<bf16_t><<<(n + F32R_BN - 1) / F32R_BN, 256, 0, s>>>((const float*)x, (const float*)w, bias,
-                                                                              (bf16_t*)y, m, n, k, epilogue);
-            return launch_status();
-        }
-        dim3 grid((n + F32_BN - 1) / F32_BN, (m + F32_BM - 1) / F32_BM);
-        if (grid.y > 65535) return IMPARO_BAD_ARGUMENT;
         if (out_dtype == IMPARO_F32)
-            k_gemm_f32<float><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, bias, (float*)y, m, n, k, epilogue);
-        else if (out_dtype == IMPARO_BF16)
-            k_gemm_f32<bf16_t><<<grid, 256, 0, s>>>((const float*)x, (const float*)w, bias, (bf16_t*)y, m, n, k, epilogue);
-        else
-            return IMPARO_BAD_ARGUMENT;
-        return launch_status();
+            return launch_f32<float>((const float*)x, (const float*)w, bias, (float*)y, m, n, k, epilogue, s);
+        if (out_dtype == IMPARO_BF16)
+            return launch_f32<bf16_t>((const float*)x, (const float*)w, bias, (bf16_t*)y, m, n, k, epilogue, s);
+        return IMPARO_BAD_ARGUMENT;
     }
     if (dtype != IMPARO_BF16) return IMPARO_BAD_ARGUMENT;
     // 16-byte loads along K: rows must start 16-byte aligned

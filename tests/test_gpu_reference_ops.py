@@ -34,6 +34,23 @@ def test_float32_product_is_the_statement_bit_for_bit(m, n, k):
     assert np.abs(out.cpu().numpy() - ref).max() <= 1e-6 * math.sqrt(k) * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (16, 17, 60), (16, 33, 1028), (17, 64, 32), (63, 65, 36), (64, 66, 260), (129, 31, 100)])
+def test_float32_product_at_the_edges_of_its_tiles(m, n, k):
+    """Rows and columns beside whole tiles, K beside whole steps, operands that start 4 bytes off 16 (read value by
+    value), and the gated epilogue, bit for bit."""
+    for shift in (0, 1):
+        x, w = torch.empty(m * k + shift, device=DEV)[shift:].view(m, k), torch.empty(n * k + shift, device=DEV)[shift:].view(n, k)
+        x.copy_(rnd(m, k, seed=1)), w.copy_(rnd(n, k, seed=2))
+        out = torch.full((m + 1, n), 7.0, device=DEV)
+        ops().gemm(x, w, out[:m])
+        assert np.array_equal(out[:m].cpu().numpy(), R.gemm(x.cpu(), w.cpu()))
+        assert bool((out[m] == 7.0).all())
+        if n % 2 == 0:
+            gated, gu = torch.empty(m, n // 2, device=DEV), R.gemm(x.cpu(), w.cpu())
+            ops().gemm(x, w, gated, swiglu=True)
+            np.testing.assert_allclose(gated.cpu().numpy(), R.swiglu(gu[:, 0::2], gu[:, 1::2]), rtol=2e-6, atol=1e-6)
+
+
 def test_embedding_norm_and_gate():
     table = rnd(37, 24, seed=4)
     ids = [36, 0, 5, 5]
