@@ -42,21 +42,37 @@ template <typename T> __device__ __forceinline__ void store_f32(T* p, size_t i, 
 template <> __device__ __forceinline__ void store_f32<float>(float* p, size_t i, float v) { p[i] = v; }
 template <> __device__ __forceinline__ void store_f32<bf16_t>(bf16_t* p, size_t i, float v) { p[i] = f32_to_bf16(v); }
 
+// Sums and maxima over a wave, the same in every lane: lanes 32 apart first, then 16, 8, 4, 2, 1. On lane swaps and
+// moves inside rows of 16, which take a few cycles where a shuffle through LDS takes about a hundred: after a step all
+// lanes that far apart agree, so "rotated by n" stands for "n apart" (and a sum of two is the same either way round).
+#define WAVE_STEPS(v, OP)                                                                                              \
+    do {                                                                                                               \
+        auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);          \
+        v = OP(__uint_as_float(halves[0]), __uint_as_float(halves[1]));                                                \
+        halves = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);               \
+        v = OP(__uint_as_float(halves[0]), __uint_as_float(halves[1]));                                                \
+        v = OP(v, rotated_in_row<8>(v));                                                                               \
+        v = OP(v, rotated_in_row<4>(v));                                                                               \
+        v = OP(v, rotated_in_row<2>(v));                                                                               \
+        v = OP(v, rotated_in_row<1>(v));                                                                               \
+    } while (0)
+
+template <int N>
+__device__ __forceinline__ float rotated_in_row(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + N, 0xf, 0xf, false));   // row_ror:N
+}
+__device__ __forceinline__ float plain_sum(float a, float b) { return a + b; }
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, WAVE);
+    WAVE_STEPS(v, plain_sum);
     return v;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, WAVE));
+    WAVE_STEPS(v, fmaxf);
     return v;
 }
 
-// Sum over a block of up to 1024 threads; every thread gets the result.
-// `scratch` holds at least 16 floats of LDS. The order of the additions
-// depends only on the block size, never on the data.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     v = wave_sum(v);
     const int lane = threadIdx.x & (WAVE - 1);
