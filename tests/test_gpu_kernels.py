@@ -898,6 +898,26 @@ def test_sample_rows(vocab):
     assert (freq - torch.softmax(row[0], 0)).abs().max() < 0.03
 
 
+@pytest.mark.parametrize("vocab", [1, 255, 4096, 50257, 65552, 1200000])
+def test_sample_rows_at_the_edges_of_its_pieces(vocab):
+    """Pieces of whole vectors and not, shorter than a vector, longer than the block; logits of minus infinity and NaN
+    are never picked, and a uniform number just below one picks the last token with weight."""
+    n = 6
+    x = rnd(n, vocab, seed=4, scale=2.0)
+    if vocab > 2:
+        x[1, vocab // 2:] = float("-inf")
+        x[2, ::2] = float("nan")
+    u = torch.tensor([0.3, 0.99999994, 0.7, 0.0, 0.999, 0.5])
+    out = torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    ops().sample_rows(x.to(DEV), torch.full((n,), 0.8, device=DEV), u.to(DEV), out)
+    for r, got in enumerate(out.cpu().tolist()):
+        z = torch.where(x[r].isnan(), float("-inf"), x[r].double()) / 0.8
+        cdf = torch.cumsum(torch.softmax(z, 0), 0)
+        assert 0 <= got < vocab and torch.isfinite(z[got])
+        # the pick's interval holds the target up to float32 rounding of the sums (2^-24 an addition, 2,200 in a chain)
+        assert (float(cdf[got - 1]) if got else 0.0) - 2e-4 <= float(u[r]) <= float(cdf[got]) + 2e-4
+
+
 # ---------------------------------------------------------------- products with a folded norm (at most 16 rows)
 from imparo_amd.kernels import ops as _rows_ops
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (5, 200, 136), (13, 1536, 1536), (16, 2048, 8192), (8, 96, 320),
