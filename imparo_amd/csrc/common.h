@@ -127,6 +127,27 @@ __device__ __forceinline__ float head_norm_scale(float sum_squares, int head_dim
     return 1.0f / sqrtf(sum_squares / (float)head_dim + eps);
 }
 
+// 16 bytes a lane from memory straight into LDS, lane after lane from `dst_wave_uniform` on
+__device__ __forceinline__ void load_to_lds(const bf16_t* src, bf16_t* dst_wave_uniform) {
+    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
+                                     (void __attribute__((address_space(3)))*)dst_wave_uniform, 16, 0, 0);
+}
+
+// The same load written out, for kernels that keep the loads of several K-steps in flight. The compiler
+// answers a fragment read from LDS that follows any load into LDS it knows of with a wait for every load
+// (it counts such a load as one that may come back out of order), which empties the pipeline; a load it
+// does not know of it does not wait for, and the kernel waits itself, by count. `lds_byte` is the same
+// for the whole wave.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void load_to_lds_uncounted(const bf16_t* src, unsigned lds_byte) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                 :
+                 : "v"(src), "s"(lds_byte)
+                 : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 // Orders LDS traffic between the lanes of one wave: what any lane wrote before
 // is visible to every lane after.
 __device__ __forceinline__ void wave_lds_sync() {

@@ -703,26 +703,6 @@ template <> __device__ __forceinline__ void store_vector<bf16_t>(bf16_t* dst, co
         *reinterpret_cast<uint2*>(dst) = make_uint2(lo, f32x2_to_bf16x2(o[2], o[3]));
 }
 
-__device__ __forceinline__ void load_to_lds(const bf16_t* src, bf16_t* dst_wave_uniform) {
-    __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)src,
-                                     (void __attribute__((address_space(3)))*)dst_wave_uniform, 16, 0, 0);
-}
-
-// The same load written out, for the kernel that keeps the loads of several K-steps in flight. The compiler
-// answers a fragment read from LDS that follows any load into LDS it knows of with a wait for every load
-// (it counts such a load as one that may come back out of order), which empties the pipeline; a load it
-// does not know of it does not wait for, and the kernel waits itself, by count. `lds_byte` is the same
-// for the whole wave.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_to_lds_uncounted(const bf16_t* src, unsigned lds_byte) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
-                 :
-                 : "v"(src), "s"(lds_byte)
-                 : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 // TMI, TN: MFMA tiles of 32x32 down a wave's part of the activation rows and across its part of
 // the weight rows; NWM, NWN: waves down and across (eight in all). The launcher's plan chooses
 // the tile so that the blocks come out in whole rounds of the CUs.

@@ -21,6 +21,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define MOE_MAX_EXPERTS 1024        // real experts the plan kernel keeps counters for
 #define MOE_MAX_TOP 16              // experts a token chooses
 #define MOE_MAX_USED 24             // experts a token uses: those and the ones that every token uses
+#define MOE_COUNTED -1              // the rows of an empty tile that holds the number of tiles before the empty ones
 #define MOE_SCORE_SOFTMAX 0         // scores = softmax over all router outputs
 #define MOE_SCORE_SIGMOID 1         // scores = sigmoid of each output
 #define MOE_SCORE_CHOSEN 2          // scores = the outputs themselves; a token's weights = softmax over its chosen ones
@@ -236,8 +237,8 @@ __device__ __forceinline__ void moe_plan_block(MoePlanShared& sh, const int32_t*
     }
     for (int i = first_tile[n_experts] + tid; i < max_tiles; i += blockDim.x) {
         tiles[3 * i] = -1;
-        tiles[3 * i + 1] = 0;
-        tiles[3 * i + 2] = 0;
+        tiles[3 * i + 1] = first_tile[n_experts];       // an empty tile says how many come before the first empty one,
+        tiles[3 * i + 2] = MOE_COUNTED;                 // and that it says so
     }
     __syncthreads();
     for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;      // now the cursor of each expert
@@ -379,6 +380,45 @@ __device__ __forceinline__ float moe_epilogue(float v, int epi) {
     return v;
 }
 
+// What a tile's products become: a wave's WM x WN of 32 x 32 at (wave / ACROSS, wave % ACROSS) of the block's tile go
+// through the epilogue to their slots' rows.
+template <int WM, int WN, int ACROSS, typename TOut, bool GATED>
+__device__ __forceinline__ void moe_store_tile(const f32x16 (&acc)[WM][WN], TOut* __restrict__ out,
+                                               const int32_t* __restrict__ entry_of_slot, const MoeGate& gate, int expert,
+                                               int row0, int rows, int n0, int N, int epi) {
+    static_assert(!GATED || WN == 2, "a wave's two tiles side by side are a gate's and its up's");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = wave / ACROSS, wn = wave % ACROSS;
+    // a lane holds column lane % 32 of a 32 x 32 product, rows 8 (r / 4) + 4 (lane / 32) + r % 4
+    if constexpr (GATED) {
+        const float limit = gate.limits ? gate.limits[expert] : 0.f;
+        const int n = (n0 + wn * 64) / 2 + (lane & 31);
+        if (n < N / 2)
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int m = wm * 32 * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                    if (m >= rows) continue;
+                    const float w = moe_slot_weight(gate, entry_of_slot, row0 + m);
+                    store_f32<TOut>(out, (size_t)(row0 + m) * (N / 2) + n,
+                                    moe_act_fast(w * acc[i][0][r], w * acc[i][WN - 1][r], limit, gate.alpha));
+                }
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            const int n = n0 + wn * 32 * WN + j * 32 + (lane & 31);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = wm * 32 * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                if (m < rows && n < N) store_f32<TOut>(out, (size_t)(row0 + m) * N + n, moe_epilogue(acc[i][j][r], epi));
+            }
+        }
+}
+
 // out[slot, n] = epi(sum_k a[row(slot), k] * w[expert, n, k]) for the slots of one tile. row(slot) is the
 // slot itself, or with gather_div the token of the slot's entry (entry / gather_div). Four waves as 2 x 2,
 // each WM x WN products of 32 x 32; K in steps of 64 through two LDS stages, the next step's loads in
@@ -389,7 +429,6 @@ __global__ __launch_bounds__(256) void k_moe_gemm_bf16(const bf16_t* __restrict_
                                                        const bf16_t* __restrict__ W, TOut* __restrict__ out,
                                                        const int32_t* __restrict__ tiles, int N, int K, int epi,
                                                        MoeGate gate = {}) {
-    static_assert(!GATED || WN == 2, "a wave's two tiles side by side are a gate's and its up's");
     constexpr int TM = 64 * WM, TN = 64 * WN, LD = 72, BK = 64;
     __shared__ __attribute__((aligned(16))) bf16_t As[2][TM * LD];
     __shared__ __attribute__((aligned(16))) bf16_t Bs[2][TN * LD];
@@ -482,34 +521,127 @@ __global__ __launch_bounds__(256) void k_moe_gemm_bf16(const bf16_t* __restrict_
 #undef MOE_FETCH
 #undef MOE_STASH
 #undef MOE_MULTIPLY
-    // a lane holds column lane % 32 of a 32 x 32 product, rows 8 (r / 4) + 4 (lane / 32) + r % 4
-    if constexpr (GATED) {
-        const float limit = gate.limits ? gate.limits[expert] : 0.f;
-        const int n = (n0 + wn * 64) / 2 + (lane & 31);
-        if (n < N / 2)
+    moe_store_tile<WM, WN, 2, TOut, GATED>(acc, out, entry_of_slot, gate, expert, row0, rows, n0, N, epi);
+}
+
+// The same product for tiles of 128 rows by 256 whose K is a multiple of 64: operands go from memory straight into LDS
+// (16 bytes a lane, eight rows of 128 bytes a load, the pieces of a row exchanged by its number instead of padded: no
+// bank conflicts), three stages, the loads of two K-steps in flight while one is multiplied; eight waves of 64 x 64, one
+// block a CU. A K-step is four sub-steps of 16; the barrier sits before the last one's products, which cover the reads
+// of the next step's first sub-step. Each output is summed over k in the same order as above: the same bits. Tiles that
+// share an expert's weight rows or its slots are neighbours on one XCD. Bound by the path into LDS and out of it (a
+// wave's outputs read 16 KB of fragments a step). Measured, 10,240 slots of 9 experts: 1,536 by 1,024, gated, 52 us
+// (the kernel above: 85); 1,024 by 768, float32 out, 34 us (53). Tiles of 128
+// by 128 on two stages, two blocks a CU, were no faster.
+#define MOE_DMA_BK 64
+#define MOE_DMA_M 128
+#define MOE_DMA_N 256
+#define MOE_DMA_STAGE ((MOE_DMA_M + MOE_DMA_N) * MOE_DMA_BK)      // elements of a stage: slots' rows, then weight rows
+#define MOE_DMA_LDS (3 * MOE_DMA_STAGE * (int)sizeof(bf16_t))
+#define MOE_GROUP_M 8
+template <typename TOut, bool GATED>
+__global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__ A, int a_ld, int gather_div,
+                                                      const int32_t* __restrict__ entry_of_slot,
+                                                      const bf16_t* __restrict__ W, TOut* __restrict__ out,
+                                                      const int32_t* __restrict__ tiles, int max_tiles, int tiles_n, int N,
+                                                      int K, int epi, MoeGate gate) {
+    constexpr int BK = MOE_DMA_BK, LA = MOE_DMA_M / 64, LW = MOE_DMA_N / 64;   // load instructions a wave and a step
+    extern __shared__ __attribute__((aligned(1024))) bf16_t stages[];
+    // the tiles that hold slots are dealt to the XCDs evenly (the grid is sized for more, and an XCD with a few blocks
+    // more than its CUs take at once runs a round of its own for them)
+    const int32_t* last = tiles + 3 * (max_tiles - 1);
+    const int n_tiles = last[0] < 0 && last[2] == MOE_COUNTED ? min(last[1], max_tiles) : max_tiles;
+    const int total = n_tiles * tiles_n;
+    const int per_xcd = (total + 7) / 8;
+    const int logical = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per_xcd || logical >= total) return;
+    const int per_group = MOE_GROUP_M * tiles_n;
+    const int first_m = (logical / per_group) * MOE_GROUP_M;
+    const int gsize = min(n_tiles - first_m, MOE_GROUP_M);
+    const int tile = first_m + (logical % per_group) % gsize;
+    const int n0 = (logical % per_group) / gsize * MOE_DMA_N;
+    const int expert = tiles[3 * tile];
+    if (expert < 0) return;
+    const int row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int wm = wave >> 2, wn = wave & 3;
+    // loading: instruction j of a wave fills rows 64 j + 8 wave .. + 7; lane -> row lane / 8, place lane % 8, where the
+    // piece lane % 8 ^ swz(row) lies, swz(r) = (r & 7) ^ ((r >> 3) & 1)
+    const int load_row = wave * 8 + (lane >> 3);
+    const int load_piece = ((lane & 7) ^ (lane >> 3) ^ (wave & 1)) * 8;
+    const bf16_t* from[LA + LW];
 #pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int m = wm * 32 * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                    if (m >= rows) continue;
-                    const float w = moe_slot_weight(gate, entry_of_slot, row0 + m);
-                    store_f32<TOut>(out, (size_t)(row0 + m) * (N / 2) + n,
-                                    moe_act_fast(w * acc[i][0][r], w * acc[i][WN - 1][r], limit, gate.alpha));
-                }
-        return;
+    for (int j = 0; j < LA; ++j) {
+        const int slot = row0 + min(load_row + 64 * j, rows - 1);
+        const int src = gather_div ? entry_of_slot[slot] / gather_div : slot;
+        from[j] = A + (size_t)src * a_ld + load_piece;
     }
 #pragma unroll
-    for (int i = 0; i < WM; ++i)
+    for (int j = 0; j < LW; ++j) from[LA + j] = W + ((size_t)expert * N + min(n0 + load_row + 64 * j, N - 1)) * K + load_piece;
+    const unsigned lds = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)stages;
+    auto load_step = [&](int stage, int kt) __attribute__((always_inline)) {
+        const unsigned to = __builtin_amdgcn_readfirstlane(lds + (stage * MOE_DMA_STAGE + wave * 8 * BK) * 2);
 #pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            const int n = n0 + wn * 32 * WN + j * 32 + (lane & 31);
+        for (int j = 0; j < LA + LW; ++j) load_to_lds_uncounted(from[j] + kt * BK, to + j * 64 * BK * 2);
+    };
+    // fragments: lane holds row lane % 32, K-half lane / 32 of a 32 x 16 piece; sub-step ks is pieces 2 ks, 2 ks + 1
+    const int frag_row = lane & 31;
+    const int swz = (frag_row & 7) ^ ((frag_row >> 3) & 1);
+    const int a_base = (wm * 64 + frag_row) * BK + (((lane >> 5) ^ swz) << 3);
+    const int b_base = (MOE_DMA_M + wn * 64 + frag_row) * BK + (((lane >> 5) ^ swz) << 3);
+    f32x16 acc[2][2];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int m = wm * 32 * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (m < rows && n < N) store_f32<TOut>(out, (size_t)(row0 + m) * N + n, moe_epilogue(acc[i][j][r], epi));
-            }
-        }
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    auto read = [&](int stage, int ks, bf16x8 (&fa)[2], bf16x8 (&fb)[2]) __attribute__((always_inline)) {
+        const bf16_t* at = stages + stage * MOE_DMA_STAGE;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) fa[i] = *reinterpret_cast<const bf16x8*>(&at[(a_base ^ (ks << 4)) + i * 32 * BK]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) fb[j] = *reinterpret_cast<const bf16x8*>(&at[(b_base ^ (ks << 4)) + j * 32 * BK]);
+    };
+    auto multiply = [&](const bf16x8 (&fa)[2], const bf16x8 (&fb)[2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+    };
+    const int nk = K / BK;
+    bf16x8 fa0[2], fb0[2], fa1[2], fb1[2];
+    load_step(0, 0);
+    load_step(1, min(1, nk - 1));
+    load_step(2, min(2, nk - 1));
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (LA + LW)) : "memory");
+    __builtin_amdgcn_s_barrier();
+    read(0, 0, fa0, fb0);
+    int cur = 0;
+    // K-step kt out of stage `cur`: on entry set 0 holds its first sub-step and the loads of steps kt + 1 and kt + 2 are
+    // in flight; on exit set 0 holds the first sub-step of kt + 1 and those of kt + 2 and kt + 3 are
+    for (int kt = 0; kt < nk; ++kt) {
+        const int next = cur == 2 ? 0 : cur + 1;
+        read(cur, 1, fa1, fb1);
+        multiply(fa0, fb0);
+        __builtin_amdgcn_sched_barrier(0);                   // (reads and products stay where they are written)
+        read(cur, 2, fa0, fb0);
+        multiply(fa1, fb1);
+        __builtin_amdgcn_sched_barrier(0);
+        read(cur, 3, fa1, fb1);
+        multiply(fa0, fb0);
+        __builtin_amdgcn_sched_barrier(0);
+        // this wave's part of `next` has landed and `cur` is read; after the barrier, so for every wave
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LA + LW) : "memory");
+        __builtin_amdgcn_s_barrier();
+        read(next, 0, fa0, fb0);
+        load_step(cur, min(kt + 3, nk - 1));                 // (past the end: the last step again, nobody reads it)
+        multiply(fa1, fb1);
+        __builtin_amdgcn_sched_barrier(0);
+        cur = next;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the loads past the end have landed
+    moe_store_tile<2, 2, 4, TOut, GATED>(acc, out, entry_of_slot, gate, expert, row0, rows, n0, N, epi);
 }
 
 // Few rows an expert (a decode step): a block takes 16 outputs of one expert and up to 16 slots. The expert's
@@ -695,6 +827,27 @@ extern "C" int imparo_moe_gemm(const void* a, int a_ld, int gather_div, const in
 #define MOE_LAUNCH_GATED(WM)                                                                                         \
     k_moe_gemm_bf16<WM, 2, bf16_t, true><<<dim3(max_tiles, (n + 127) / 128), 256, 0, s>>>(                           \
         (const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (bf16_t*)out, tiles, n, k, epilogue, gate)
+    // tiles of 128 rows whose K comes in the steps that go straight into LDS, unless 256 columns a tile leave more than a
+    // quarter of the columns empty beside tiles of 128 (the kernels' rates are 1.6 to 1)
+    const int tiles_n = (n + MOE_DMA_N - 1) / MOE_DMA_N;
+    const long long blocks = ((long long)max_tiles * tiles_n + 7) / 8 * 8;
+    if (tile_rows == 128 && k % MOE_DMA_BK == 0 && 4 * tiles_n * MOE_DMA_N <= 5 * ((n + 127) / 128 * 128) && blocks < (1LL << 31)) {
+#define MOE_LAUNCH_DMA(TO, G)                                                                                        \
+    do {                                                                                                             \
+        if (hipFuncSetAttribute((const void*)k_moe_gemm_dma<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize,      \
+                                MOE_DMA_LDS) != hipSuccess)                                                          \
+            return IMPARO_LAUNCH_FAILED;                                                                             \
+        k_moe_gemm_dma<TO, G><<<(unsigned)blocks, 512, MOE_DMA_LDS, s>>>(                                            \
+            (const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (TO*)out, tiles, max_tiles, tiles_n, n, k, \
+            epilogue, gate);                                                                                         \
+    } while (0)
+        if (epilogue == MOE_EPI_GATED) MOE_LAUNCH_DMA(bf16_t, true);
+        else if (out_dtype == IMPARO_BF16) MOE_LAUNCH_DMA(bf16_t, false);
+        else if (out_dtype == IMPARO_F32) MOE_LAUNCH_DMA(float, false);
+        else return IMPARO_BAD_ARGUMENT;
+#undef MOE_LAUNCH_DMA
+        return launch_status();
+    }
     if (epilogue == MOE_EPI_GATED) {
         if (tile_rows == 16)
             k_moe_gemm_rows16<bf16_t, true><<<dim3(max_tiles, n / 32), 256, 0, s>>>(

@@ -461,6 +461,40 @@ def test_product_of_the_experts_with_the_unit_behind_it(T, X, top, F, K, bounds)
         near(got[:, j], want, 8e-3, f"choice {j}")
 
 
+@pytest.mark.parametrize("counts,N,K", [((128, 127, 129, 1, 0, 300), 256, 64), ((200, 256), 500, 128), ((513, 100, 60), 448, 192),
+                                        ((128, 128, 128), 768, 1024)])
+@pytest.mark.parametrize("epilogue,out_dtype", [("relu2", torch.bfloat16), (None, torch.float32), ("gated", torch.bfloat16)])
+def test_product_of_the_experts_at_the_edges_of_wide_tiles(counts, N, K, epilogue, out_dtype):
+    """Tiles of 128 slots by 256 columns beside experts with a row more or less, none, or one; columns and K-steps beside
+    whole tiles and rounds; with empty tiles in the list and without. Sums of K products of bfloat16 in float32."""
+    from imparo_amd.kernels import ops
+    N = N // 64 * 64 if epilogue == "gated" else N
+    g = torch.Generator().manual_seed(N + K)
+    X, n = len(counts), sum(counts)
+    choice = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])[torch.randperm(n, generator=g)]
+    h = torch.randn(n, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(X, N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
+    slot, entry = torch.empty(n, dtype=torch.int32, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
+    live = sum(-(-c // 128) for c in counts)
+    for length in (ops.moe_max_tiles(n, X, 128), live + 1):
+        if length < ops.moe_max_tiles(n, X, 128):
+            tiles = tiles[:length].contiguous() if length > live else tiles
+        else:
+            tiles = torch.empty(length, 3, dtype=torch.int32, device=DEV)
+            ops.moe_plan(i32(choice), X, 128, slot, entry, tiles)
+        assert (tiles[:, 0] >= 0).sum() == live
+        cols = N // 2 if epilogue == "gated" else N
+        out = torch.full((n, cols), 7.0, dtype=out_dtype, device=DEV)
+        ops.moe_gemm(dev(h, torch.bfloat16), dev(w, torch.bfloat16), out, tiles, 128, entry, gather_div=1, epilogue=epilogue)
+        z = torch.stack([h[i].double() @ w[int(choice[i])].double().t() for i in range(n)])
+        if epilogue == "gated":
+            z = z.view(n, N // 64, 2, 32)
+            z = (z[:, :, 0] * torch.sigmoid(z[:, :, 0]) * z[:, :, 1]).reshape(n, cols)
+        elif epilogue == "relu2":
+            z = torch.relu(z).square()
+        near(out.float().cpu()[slot.cpu().long()], z, 8e-3 if out_dtype == torch.bfloat16 else 1e-6 * math.sqrt(K))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T", [1, 9, 70, 300])
 @pytest.mark.parametrize("ff,shared_ff,E,X,top", [(24, 40, 64, 6, 2), (13, 9, 48, 3, 3), (64, None, 128, 16, 4), (16, 16, 36, 1, 1),
