@@ -331,8 +331,13 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
     }
 }
 
-template <int ND, bool FROM_QKV, bool EXT = false>
-__global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decode(
+// SPLITS > 1: the block has the waves of that many splits, all that a row can have, and adds their results itself, in
+// the merge kernel's order, so there is no launch for that. A short context is bound by launches (a merge behind this
+// kernel takes 4.5 us however little it adds), a long one by how many CUs draw on the cache, which wants a block a split.
+// Measured, 8 rows of 32 heads of 64 over 300 keys, two splits, the projection's rows normed and rotated here: 11.2 us where
+// the two launches took 9.3 and 4.6; one row of 16 heads over 50 keys 8.5 where they took 7.1 and 4.5.
+template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1>
+__global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decode(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ seg_start, const int32_t* __restrict__ positions,
@@ -340,12 +345,13 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decod
     float scale, int window, int n_splits, FromQkv fq, int exact, Rule rule) {
     constexpr int D = ND * 16, NK = (ND + 1) / 2;
     constexpr int TILES = DEC_SPLIT / (MFMA_WAVES * 32);   // tiles a wave takes at most
-    __shared__ float sm[MFMA_WAVES][16], sl[MFMA_WAVES][16];
-    __shared__ float so[MFMA_WAVES][16][D + 1];
+    __shared__ float sm[SPLITS * MFMA_WAVES][16], sl[SPLITS * MFMA_WAVES][16];
+    __shared__ float so[SPLITS * MFMA_WAVES][16][D + 1];
     __shared__ float sn_tab[FROM_QKV ? D / 2 : 1], cs_tab[FROM_QKV ? D / 2 : 1];
     __shared__ __attribute__((aligned(16))) float qw_tab[FROM_QKV ? D : 1], kw_tab[FROM_QKV ? D : 1];
     __shared__ __attribute__((aligned(16))) float k_raw[FROM_QKV ? D : 1], v_raw[FROM_QKV ? D : 1];
-    const int split = blockIdx.x, ri = blockIdx.z;
+    const int all_waves = threadIdx.x >> 6;                 // of the block; `wave` is one of its split's
+    const int split = SPLITS == 1 ? blockIdx.x : __builtin_amdgcn_readfirstlane(all_waves / MFMA_WAVES), ri = blockIdx.z;
     const int G = heads / kv_heads, passes = (G + 15) / 16;
     const int kvh = blockIdx.y / passes, pass = blockIdx.y % passes;
     const int row = rows[ri];
@@ -360,8 +366,8 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decod
     const int k_begin = EXT ? split * DEC_SPLIT : max(split * DEC_SPLIT, lo & ~31);
     const int k_end = min((split + 1) * DEC_SPLIT, last + 1 - walk.gap);
     const bool own = FROM_QKV && split == pos / DEC_SPLIT;  // this block weighs the row's own key in
-    if (k_begin >= k_end && !own) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (SPLITS == 1 && k_begin >= k_end && !own) return;    // (with others' splits beside it: nothing of its own to add)
+    const int lane = threadIdx.x & 63, wave = all_waves % MFMA_WAVES;
     const int c = lane & 15, g = lane >> 4;
     const int hq = pass * 16 + c;               // query head inside the group
     const bool qvalid = hq < G;
@@ -472,28 +478,68 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decod
         }
     }
     if (g == 0) {
-        sm[wave][c] = st.m;
-        sl[wave][c] = st.l;
+        sm[all_waves][c] = st.m;
+        sl[all_waves][c] = st.l;
     }
 #pragma unroll
     for (int dt = 0; dt < ND; ++dt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) so[wave][c][dt * 16 + 4 * g + i] = st.o[dt][i];
+        for (int i = 0; i < 4; ++i) so[all_waves][c][dt * 16 + 4 * g + i] = st.o[dt][i];
     __syncthreads();
-    for (int e = threadIdx.x; e < 16 * D; e += MFMA_WAVES * 64) {
+    for (int e = threadIdx.x; e < 16 * D; e += SPLITS * MFMA_WAVES * 64) {
         const int qc = e / D, d = e - qc * D;
         if (pass * 16 + qc >= G) continue;
-        float ms = sm[0][qc];
+        float m_of[SPLITS], acc_of[SPLITS], l_of[SPLITS];
 #pragma unroll
-        for (int w = 1; w < MFMA_WAVES; ++w) ms = fmaxf(ms, sm[w][qc]);
-        float acc = 0.f, ls = 0.f;
+        for (int sp = 0; sp < SPLITS; ++sp) {
+            float ms = sm[sp * MFMA_WAVES][qc];
 #pragma unroll
-        for (int w = 0; w < MFMA_WAVES; ++w) {
-            const float f = (sm[w][qc] == -INFINITY) ? 0.f : __expf(sm[w][qc] - ms);
-            acc += so[w][qc][d] * f;
-            ls += sl[w][qc] * f;
+            for (int w = 1; w < MFMA_WAVES; ++w) ms = fmaxf(ms, sm[sp * MFMA_WAVES + w][qc]);
+            float acc = 0.f, ls = 0.f;
+#pragma unroll
+            for (int w = 0; w < MFMA_WAVES; ++w) {
+                const float mw = sm[sp * MFMA_WAVES + w][qc];
+                const float f = (mw == -INFINITY) ? 0.f : __expf(mw - ms);
+                acc += so[sp * MFMA_WAVES + w][qc][d] * f;
+                ls += sl[sp * MFMA_WAVES + w][qc] * f;
+            }
+            m_of[sp] = ms, acc_of[sp] = acc, l_of[sp] = ls;
         }
         const int head_out = kvh * G + pass * 16 + qc;
+        if constexpr (SPLITS > 1) {
+            // as the merge kernel adds them: the splits the row has, counted from its first, dealt to as many sides as
+            // heads of this size let a wave take at once
+            constexpr int SIDE = WAVE / (D / 4);
+            const int s_lo = EXT ? 0 : (lo & ~15) / DEC_SPLIT;
+            const int s_hi = min((EXT ? pos - walk.gap : pos) / DEC_SPLIT, SPLITS - 1);
+            float ms = -INFINITY;
+#pragma unroll
+            for (int sp = 0; sp < SPLITS; ++sp) ms = fmaxf(ms, m_of[sp]);
+            float part[4] = {0.f, 0.f, 0.f, 0.f}, l_part[4] = {0.f, 0.f, 0.f, 0.f};     // counted from the first split
+#pragma unroll
+            for (int sp = 0; sp < SPLITS; ++sp) {
+                const float w = (m_of[sp] == -INFINITY) ? 0.f : __expf(m_of[sp] - ms);
+#pragma unroll
+                for (int i = 0; i < SPLITS; ++i)
+                    if (sp >= s_lo && sp <= s_hi && sp - s_lo == i) {
+                        part[i] = __fmul_rn(acc_of[sp], w);
+                        l_part[i] = __fmul_rn(l_of[sp], w);
+                    }
+            }
+            const float ls = (l_part[0] + l_part[2]) + (l_part[1] + l_part[3]);
+            float total = 0.f;
+#pragma unroll
+            for (int side = 0; side < SIDE && side < 4; ++side) {
+                float a = 0.f;
+#pragma unroll
+                for (int i = side; i < 4; i += SIDE) a += part[i];
+                total += a;
+            }
+            const float inv = EXT ? ruled_inverse(rule, t, head_out, ms, ls) : (ls > 0.f ? 1.0f / ls : 0.f);
+            out[((size_t)t * heads + head_out) * D + d] = f32_to_bf16(total * inv);
+            continue;
+        }
+        const float ms = m_of[0], acc = acc_of[0], ls = l_of[0];
         if (n_splits == 1) {
             const float o = EXT ? acc * ruled_inverse(rule, t, head_out, ms, ls) : (ls > 0.f ? acc / ls : 0.f);
             out[((size_t)t * heads + head_out) * D + d] = f32_to_bf16(o);
@@ -1371,29 +1417,33 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
     if (given && from_qkv) return IMPARO_BAD_ARGUMENT;
     // the merge moves four elements of a head in one access
     if (n_splits > 1 && (((uintptr_t)part_o & 15) || ((uintptr_t)out & 7))) return IMPARO_BAD_ARGUMENT;
-    dim3 grid(n_splits, kv_heads * ((G + 15) / 16), n_rows);
+    // Two splits, or up to four with heads of at most 64: one block takes them all and there is no merge. (Sixteen waves
+    // of larger heads would not find registers; from five splits on a block a split draws on more CUs.)
+    const int in_block = n_splits == 2 ? 2 : n_splits <= 4 && n_splits > 2 && head_dim <= 64 ? 4 : 1;
+    dim3 grid(in_block > 1 ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
+#define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT)                                                                \
+    k_attn_decode<ND, QKV, EXT, SPLITS><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                                   \
+        Q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,           \
+        positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, EXACT, rule)
+#define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT)                                                                       \
+    do {                                                                                                             \
+        if (in_block == 2) DECODE_GO(ND, QKV, EXT, 2, Q, FQ, EXACT);                                                 \
+        else if (in_block == 4) DECODE_GO(ND, QKV, EXT, (ND <= 4 ? 4 : 2), Q, FQ, EXACT);                            \
+        else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT);                                                               \
+    } while (0)
     if (from_qkv) {
-#define DECODE_FROM_QKV(ND)                                                                                          \
-    k_attn_decode<ND, true><<<grid, MFMA_WAVES * 64, 0, s>>>(                                                        \
-        nullptr, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,     \
-        positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, *from_qkv, 0, rule)
-        if (head_dim == 64) DECODE_FROM_QKV(4);
-        else if (head_dim == 128) DECODE_FROM_QKV(8);
+        if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, 0);
+        else if (head_dim == 128) DECODE_ANY(8, true, false, nullptr, *from_qkv, 0);
         else return IMPARO_BAD_ARGUMENT;
-#undef DECODE_FROM_QKV
     } else if (given) {
-        DISPATCH_ND(head_dim / 16, (k_attn_decode<ND, false, true><<<grid, MFMA_WAVES * 64, 0, s>>>(
-            (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows,
-            seg_start, positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window,
-            n_splits, FromQkv{}, exact, rule)));
+        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, true, (const bf16_t*)q, FromQkv{}, exact));
     } else {
-        DISPATCH_ND(head_dim / 16, (k_attn_decode<ND, false><<<grid, MFMA_WAVES * 64, 0, s>>>(
-            (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows,
-            seg_start, positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window,
-            n_splits, FromQkv{}, exact, rule)));
+        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, false, (const bf16_t*)q, FromQkv{}, exact));
     }
+#undef DECODE_ANY
+#undef DECODE_GO
     if (launch_status()) return IMPARO_LAUNCH_FAILED;
-    if (n_splits == 1) return IMPARO_OK;
+    if (n_splits == 1 || in_block > 1) return IMPARO_OK;
     if (given)
         k_attn_decode_merge<true><<<n_rows * heads, 64, 0, s>>>(part_o, part_ml, (bf16_t*)out, rows, seg_start, positions,
                                                                 heads, head_dim, n_splits, window, rule);

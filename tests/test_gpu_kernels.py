@@ -613,6 +613,19 @@ def test_matrix_core_attention_with_32_queries_a_wave(H, Hk, D, ctx, q):
     torch.testing.assert_close(wide, narrow, rtol=2 ** -7, atol=2 ** -7)
 
 
+@pytest.mark.parametrize("H,Hk,D", [(8, 2, 64), (40, 2, 64), (5, 5, 48), (4, 1, 16), (4, 1, 80), (4, 1, 128)])
+@pytest.mark.parametrize("lens", [(1, 255, 256, 257, 512, 70), (1, 512, 513, 768, 1000, 1024, 257)])
+@pytest.mark.parametrize("window", [None, 300, 1])
+def test_decode_attention_merges_few_splits_in_the_block(H, Hk, D, lens, window):
+    """Contexts of up to two splits of 256 keys, and of up to four: one launch. The same rows with block tables that have
+    room for nine splits take the merge launch: the same bits, a row of one split among many included."""
+    n, lens, one = len(lens), lens + (40,), [1] * len(lens) + [5]            # (a portion beside them: the case wants one)
+    got, ref = _attention_case(H, Hk, D, 64, window, torch.bfloat16, kernel="mfma", ctx_lens=lens, q_lens=one)
+    torch.testing.assert_close(got, ref, rtol=2 ** -6, atol=2 ** -6)
+    merged, _ = _attention_case(H, Hk, D, 64, window, torch.bfloat16, kernel="mfma", ctx_lens=lens, q_lens=one, table_width=33)
+    assert torch.equal(got[:n], merged[:n])
+
+
 @pytest.mark.parametrize("H,Hk,D", [(8, 2, 64), (5, 5, 64), (40, 2, 64), (4, 1, 128)])
 @pytest.mark.parametrize("page_size,window,interleaved,normed,rotated", [
     (16, None, False, True, True), (64, None, False, True, True), (64, 100, True, True, True),
