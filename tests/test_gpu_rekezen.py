@@ -408,6 +408,39 @@ def test_weights_over_the_chosen_outputs(X, top, T):
         assert sorted(s1.cpu().tolist()) == list(range(n)) and bool((choice.cpu()[s2.cpu().long() // (top + 1), top] == X).all())
 
 
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
+@pytest.mark.parametrize("X,top", [(1, 1), (8, 4), (16, 16), (63, 5), (64, 16)])
+def test_choice_among_few_outputs_is_the_general_one(X, top, scoring):
+    """At most 64 outputs are ranked by counting; the same rows with outputs past the 64th that cannot be chosen go the
+    general way and give the same choices and weights, bit for bit: equal outputs, rows with too few that can be chosen
+    (minus infinity, NaN), and infinity. The plan made in the same launch holds every chosen entry once."""
+    from imparo_amd.kernels import ops
+    T, wide = 40, 65
+    z = torch.randn(T, X, generator=torch.Generator().manual_seed(X)) * 2
+    z[1], z[2], z[3, 0], z[4, X // 2], z[5, X // 2:] = 0.5, z[2].round(), float("inf"), float("nan"), -float("inf")
+    corr = (0.3 * torch.randn(X, generator=torch.Generator().manual_seed(top))).round(decimals=1)
+    pad = lambda t: torch.cat([t, torch.full((*t.shape[:-1], wide - X), -float("inf"))], -1)
+    got = []
+    for logits, c in ((z, corr), (pad(z), pad(corr))):
+        choice, weight = torch.empty(T, top, dtype=torch.int32, device=DEV), torch.empty(T, top, device=DEV)
+        ops.moe_route(dev(logits), dev(c), choice, weight, top, scoring=scoring, normalize=True, scale=1.3)
+        got.append((choice.cpu(), weight.cpu()))
+    assert torch.equal(got[0][0], got[1][0])
+    assert torch.equal(got[0][1].view(torch.int32), got[1][1].view(torch.int32)) or \
+        torch.equal(got[0][1].nan_to_num(7.0), got[1][1].nan_to_num(7.0))
+    rows, n = ops.moe_tile_rows(T * top, X, torch.bfloat16), T * top
+    tiles = torch.empty(ops.moe_max_tiles(n, X, rows), 3, dtype=torch.int32, device=DEV)
+    s1, s2 = torch.empty(n, dtype=torch.int32, device=DEV), torch.full((n,), -1, dtype=torch.int32, device=DEV)
+    ops.moe_route_plan(dev(z), dev(corr), choice, weight, top, X, rows, s1, s2, tiles, scoring=scoring, normalize=True, scale=1.3)
+    assert torch.equal(choice.cpu(), got[0][0])
+    e, slot = choice.cpu().flatten(), s1.cpu()
+    real = e < X
+    assert bool((slot[~real] == -1).all()) and sorted(slot[real].tolist()) == list(range(int(real.sum())))
+    assert bool((e[s2.cpu()[:int(real.sum())].long()].diff() >= 0).all())          # an expert's slots lie together
+    used = tiles.cpu()[tiles.cpu()[:, 0] >= 0]
+    assert int(used[:, 2].sum()) == int(real.sum())
+
+
 @pytest.mark.parametrize("n,half", [(7, 24), (5, 13), (900, 64)])
 def test_gated_unit_with_bounds_over_experts_rows(n, half):
     from imparo_amd.kernels import ops
