@@ -477,9 +477,10 @@ class Engine:
 
         for rows in range(1, max_requests + 1):
             shape(rows, rows, True, longest)
-        # (the products' slices of K depend on the rows: every count to 64, then every 16th to 512, then doublings)
-        sizes = {n for n in list(range(2, 65)) + list(range(80, 513, 16)) if n <= self.max_step_tokens}
-        sizes |= {n for n in (1024, 2048, 4096, 8192, 16384) if n < self.max_step_tokens} | {self.max_step_tokens}
+        # (the products' slices of K depend on the rows: every count to 64, then every 16th to 512, then every 128th,
+        # where a range of rows cut alike mostly ends, to 8,192, then doublings)
+        sizes = {n for n in list(range(2, 65)) + list(range(80, 513, 16)) + list(range(640, 8193, 128)) + [16384]
+                 if n < self.max_step_tokens} | {self.max_step_tokens}
         for tokens in sorted(sizes):
             shape(tokens, 1, False, min(longest, max(tokens, self.page_size)))
             shape(tokens, 1, False, longest)

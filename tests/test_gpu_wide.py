@@ -199,3 +199,17 @@ def test_many_decoding_rows_beside_portions_in_one_step(wide, dtype, decoding):
         check_logits(rows_single, torch.stack([w[j] for w in want]), dtype, f"{decoding} single rows beside portions, step {j}")
     check_logits(torch.cat(got_short), want_short, dtype, "the 33-token portions")
     check_logits(torch.cat(got_long), want_long, dtype, "the 300-token portions")
+
+
+def test_a_step_between_the_doublings_finds_its_scratch_reserved(wide):
+    """The most slices of K a row count takes change at the ends of tiles: a step of 2,560 rows cuts the way back in three and
+    needs more for them than the engine's largest step, of 3,000 rows in two. Nothing may grow then, as growing allocates inside
+    a step and has every recorded graph recorded again."""
+    from imparo_amd.engine import StepEntry
+    from imparo_amd.kernels import ops
+    cut = {m: ops.gemm_slices(m, 2048, 8192, torch.bfloat16) * m for m in (2560, 3000)}
+    assert cut[2560] > cut[3000]
+    eng = make_engine(wide[0], "bfloat16", page_size=64, max_tokens=4096, max_requests=2, max_step_tokens=3000)
+    before = eng.workspace.version
+    out = eng.step([StepEntry("a", prompt_tokens(65536, 2560, 5), [2559])])
+    assert bool(torch.isfinite(out).all()) and eng.workspace.version == before
