@@ -971,27 +971,16 @@ static bool dma_tile_takes(int m, int n, int k) {
 //     once (5.5 TB/s) and the results have to go there (7.6 TB/s); a slice beyond the first costs
 //     its consumer one more pass over rows x width of float32 (5 TB/s).
 // `fixed_slices` > 0: the caller has decided (1: its consumer cannot add slices).
-// A K of 2^n has even cuts into 2, 4 and 8 only; where 2 leave a third of the CUs idle and 4 need a second round of
-// them, 3 slices, the last one shorter, are the better cut. Product and the norm that adds its slices, K = 8,192, us
-// with even slices -> 3: 2,048 weight rows: 520 rows 41.0 -> 35.8, 640 rows 47.0 -> 39.0, 1,280 rows 69.3 -> 66.5, 2,560
-// rows 109.5 -> 107.4; 1,024 weight rows: 1,100 rows 42.3 -> 36.8, 2,600 rows (1 -> 3) 68.2 -> 66.8. Only with slices of
-// 2,048 of K and more: of K = 4,096 the product itself gains little (540 rows by 4,096, 1 -> 3: 32.6 -> 32.1 us; 1,025 rows
-// by 2,048: 32.0 -> 31.5), less than two more slices of results to write and to add cost.
 struct DmaPlan {
     int bm, tn, slices, stages;
 };
-// K of a slice but the last: in whole turns of the kernel's loop
-static int dma_slice(int k, int slices, int stages) {
-    const int turn = stages * DM_BK;
-    return ((k + slices - 1) / slices + turn - 1) / turn * turn;
-}
 static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
     DmaPlan best{0, 0, fixed_slices > 0 ? fixed_slices : 1, 2};
     if (m <= 64 || !dma_tile_takes(m, n, k)) return best;
     double best_cost = 0.0;
     for (int slices : {1, 2, 3, 4, 6, 8}) {                 // (3 and 6: a K of 27 or 9 times 256 has no other cut)
         if (fixed_slices > 0 && slices != fixed_slices) continue;
-        if ((slices != 3 && k % (128 * slices) != 0) || (slices > 1 && k / slices < 512)) continue;
+        if (k % (128 * slices) != 0 || (slices > 1 && k / slices < 512)) continue;
         for (int bm = 256; bm >= 128; bm /= 2) {
             const int tiles_m = (m + bm - 1) / bm;
             for (int tn = 4; tn >= 1; --tn) {
@@ -1000,11 +989,8 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
                 const int bn = 64 * tn;
                 for (int stages = 2; stages <= 4; stages += 2) {
                     // four stages: the 128x128 tile and the 128x64 one (which runs on four only), K-steps in fours
-                    if (stages == 4 && (bm != 128 || tn > 2)) continue;
+                    if (stages == 4 && (bm != 128 || tn > 2 || (k / slices) % (4 * DM_BK) != 0)) continue;
                     if (stages == 2 && tn == 1) continue;
-                    const int k_per = dma_slice(k, slices, stages), k_last = k - (slices - 1) * k_per;
-                    if (k_last % (stages * DM_BK) != 0 || (slices > 1 && k_last < 512)) continue;
-                    if (k_per != k_last && (slices != 3 || k / slices < 2048)) continue;
                     const long long blocks = (long long)tiles_m * ((n + bn - 1) / bn) * slices;
                     const int at_once = 256 * ((bm + bn) * DM_BK * 2 * stages <= 80 * 1024 ? 2 : 1);
                     const long long rounds = (blocks + at_once - 1) / at_once;
@@ -1026,7 +1012,7 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
                     if (tiles_m == 1) step = std::max(step, bn * 128.0 / 28e3);
                     const double ends = 4.3 + 0.116 * (bm * bn / 1024.0);
                     const double from_memory = ((double)m + n) * k * 2.0 / 5.5e6;
-                    const double cost = std::max(rounds * (k_per / DM_BK * step + ends), from_memory + ends) +
+                    const double cost = std::max(rounds * (k / slices / DM_BK * step + ends), from_memory + ends) +
                                         (double)slices * m * n * 4.0 / 7.6e6 + (slices - 1) * ((double)m * n * 4.0 / 5e6);
                     if (best.tn == 0 || cost < best_cost) {
                         best = DmaPlan{bm, tn, slices, stages};
@@ -1039,32 +1025,31 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
     return best;
 }
 
-// `slices` must leave every slice of dma_slice, the last one too, whole turns of the kernel's loop (at least one).
+// `slices` must leave every slice a multiple of 128 of K (dma_tile_takes(m, n, k / slices) and k % slices == 0).
 // bm: 256 or 128 activation rows to a tile; tn: 4, 3 (bm 256 only), 2 or 1 (bm 128 only) for 256, 192, 128 or 64 weight rows.
 template <typename TOut>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                       int bm, int tn, int slices, hipStream_t s, int stages = 2) {
-    const int k_per = dma_slice(k, slices, stages);
     const int tiles_m = (m + bm - 1) / bm, tiles_n = (n + 64 * tn - 1) / (64 * tn);
     const long long total = (long long)tiles_m * tiles_n;
     const dim3 grid((unsigned)(((total + N_XCD - 1) / N_XCD) * N_XCD), (unsigned)slices);
 #define DMA_GO(TMI, TN, NWN)                                                                                         \
-    k_gemm_bf16_dma<TOut, TMI, TN, NWN><<<grid, 128 * NWN, 0, s>>>(x, w, bias, y, m, n, k, k_per, tiles_m,     \
+    k_gemm_bf16_dma<TOut, TMI, TN, NWN><<<grid, 128 * NWN, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m,     \
                                                                    tiles_n, epilogue)
     if (bm == 128 && tn == 1 && stages == 4)   // 64 wide: four waves of 64 rows by 32
-        k_gemm_bf16_dma<TOut, 2, 1, 2, 2, 4><<<grid, 256, 0, s>>>(x, w, bias, y, m, n, k, k_per, tiles_m, tiles_n, epilogue);
+        k_gemm_bf16_dma<TOut, 2, 1, 2, 2, 4><<<grid, 256, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m, tiles_n, epilogue);
     else if (bm == 128 && tn == 1)
-        k_gemm_bf16_dma<TOut, 2, 1, 2, 2, 2><<<grid, 256, 0, s>>>(x, w, bias, y, m, n, k, k_per, tiles_m, tiles_n, epilogue);
+        k_gemm_bf16_dma<TOut, 2, 1, 2, 2, 2><<<grid, 256, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m, tiles_n, epilogue);
     else if (bm == 128 && tn == 4)
         DMA_GO(2, 2, 4);
     else if (bm == 128 && stages == 4)
-        k_gemm_bf16_dma<TOut, 2, 1, 4, 2, 4><<<grid, 512, 0, s>>>(x, w, bias, y, m, n, k, k_per, tiles_m, tiles_n, epilogue);
+        k_gemm_bf16_dma<TOut, 2, 1, 4, 2, 4><<<grid, 512, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m, tiles_n, epilogue);
     else if (bm == 128)
         DMA_GO(2, 1, 4);
     else if (tn == 4)     // 256 wide: eight waves
         DMA_GO(4, 2, 4);
     else if (tn == 3)     // 192 wide: eight waves of 64 rows by 96
-        k_gemm_bf16_dma<TOut, 2, 3, 2, 4><<<grid, 512, 0, s>>>(x, w, bias, y, m, n, k, k_per, tiles_m, tiles_n, epilogue);
+        k_gemm_bf16_dma<TOut, 2, 3, 2, 4><<<grid, 512, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m, tiles_n, epilogue);
     else                  // 128 wide: eight waves
         DMA_GO(4, 1, 4);
 #undef DMA_GO

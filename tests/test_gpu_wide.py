@@ -202,14 +202,14 @@ def test_many_decoding_rows_beside_portions_in_one_step(wide, dtype, decoding):
 
 
 def test_a_step_between_the_doublings_finds_its_scratch_reserved(wide):
-    """The most slices of K a row count takes change at the ends of tiles: a step of 2,560 rows cuts the way back in three and
-    needs more for them than the engine's largest step, of 3,000 rows in two. Nothing may grow then, as growing allocates inside
+    """The most slices of K a row count takes change at the ends of tiles: a step of 1,280 rows cuts the way back in four and
+    needs more for them than the engine's largest step, of 2,500 rows in two. Nothing may grow then, as growing allocates inside
     a step and has every recorded graph recorded again."""
     from imparo_amd.engine import StepEntry
     from imparo_amd.kernels import ops
-    cut = {m: ops.gemm_slices(m, 2048, 8192, torch.bfloat16) * m for m in (2560, 3000)}
-    assert cut[2560] > cut[3000]
-    eng = make_engine(wide[0], "bfloat16", page_size=64, max_tokens=4096, max_requests=2, max_step_tokens=3000)
+    cut = {m: ops.gemm_slices(m, 2048, 8192, torch.bfloat16) * m for m in (1280, 2500)}
+    assert cut[1280] > cut[2500]
+    eng = make_engine(wide[0], "bfloat16", page_size=64, max_tokens=4096, max_requests=2, max_step_tokens=2500)
     before = eng.workspace.version
-    out = eng.step([StepEntry("a", prompt_tokens(65536, 2560, 5), [2559])])
+    out = eng.step([StepEntry("a", prompt_tokens(65536, 1280, 5), [1279])])
     assert bool(torch.isfinite(out).all()) and eng.workspace.version == before
