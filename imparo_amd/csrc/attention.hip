@@ -181,11 +181,12 @@ __global__ __launch_bounds__(ATT_WAVES * WAVE) void k_attention_wave_f32(
     const int lo_chunk = (lo / WAVE) * WAVE;
     const int keep = rule.keep_first;
     auto next_of = [&](int c) { return (c + WAVE >= keep && c + WAVE < lo_chunk) ? lo_chunk : c + WAVE; };
-    // which row of the caches holds this lane's key of chunk c, -1: none
+    // which row of the caches holds this lane's key of chunk c, -1: none (a token at a position below 0 has no keys, and its
+    // place in the table is read all the same)
     auto row_of = [&](int c) __attribute__((always_inline)) {
         const int p = c + lane;
         const bool valid = p <= pos && (p >= lo || p < keep);
-        const int page = table[min(p, pos) / page_size];
+        const int page = table[max(min(p, pos), 0) / page_size];
         return valid && page >= 0 && page < n_pages ? (page * kv_heads + kvh) * page_size + p % page_size : -1;
     };
     float4 key[HD / 4];

@@ -175,3 +175,33 @@ def test_float32_attention_sums_alike_whether_the_head_size_is_known_or_not(H, H
     general, _ = _attention_case(H, Hk, D, page_size, window, torch.float32, v_transposed=True, **lens)
     assert torch.equal(got, general)
     torch.testing.assert_close(got, ref, rtol=2e-5, atol=2e-5)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("page_size,window", [(1, 0), (5, 0), (16, 20)])
+def test_float32_attention_of_a_token_before_the_first_position(D, page_size, window):
+    """A token at a position below 0 sees no key and gives zeros; its block table is read at its first entry at the lowest (the
+    table here lies behind numbers that are no pages, and a cache of NaN shows a row read and used). Tokens beside it are
+    what they are without it."""
+    H, n_pages = 2, 40
+    g = torch.Generator().manual_seed(D)
+    k, v = (torch.full((n_pages, 1, page_size, D), float("nan")) for _ in range(2))
+    pages = torch.randperm(n_pages, generator=g)[:24].int()
+    ctx = min(30, 24 * page_size)
+    for p in range(ctx):
+        k[pages[p // page_size], 0, p % page_size] = torch.randn(D, generator=g)
+        v[pages[p // page_size], 0, p % page_size] = torch.randn(D, generator=g)
+    table = torch.cat([torch.full((24,), 1 << 30, dtype=torch.int32), pages]).to(DEV)[24:].view(1, 24)
+    k, v, q = k.to(DEV), v.to(DEV), torch.randn(4, H, D, generator=g).to(DEV)
+
+    def attend(positions):
+        n = len(positions)
+        out = torch.full((n, H * D), 7.0, device=DEV)
+        ops().attention(q[:n].contiguous(), k, v, out, torch.tensor(positions, dtype=torch.int32, device=DEV),
+                        torch.zeros(n, dtype=torch.int32, device=DEV), table, 0.125, window or None)
+        return out.cpu()
+
+    plain = attend([ctx - 1, 0])
+    assert bool(torch.isfinite(plain).all())
+    got = attend([ctx - 1, 0, -1, -20 * page_size])
+    assert torch.equal(got[:2], plain) and bool((got[2:] == 0).all())
