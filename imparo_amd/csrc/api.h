@@ -592,6 +592,9 @@ const char* imparo_program_region_name(const ImparoProgram* p, int region);
 int imparo_program_bind(ImparoProgram* p, int region, void* ptr, int64_t bytes);
 // needs[region] = bytes of each region that a step of this shape uses (0: not used)
 int imparo_program_needs(ImparoProgram* p, const ImparoStepArgs* args, int64_t* needs);
+// needs[region] = the most bytes of each region that a step of one portion of 1 to args->n_tokens tokens uses, at the
+// context of `args`. Every count is asked: a product's slices of K change with its rows, also between the ends of tiles.
+int imparo_program_needs_up_to(ImparoProgram* p, const ImparoStepArgs* args, int64_t* needs);
 // Runs the step on `stream`. *logits = where the float32 [n_want, vocab] logits are (inside the
 // "logits" region), or null if nothing is wanted. IMPARO_SCRATCH_TOO_SMALL: nothing was launched,
 // imparo_program_needs says what to bind. Any other failure: imparo_program_error names the operation.

@@ -126,6 +126,18 @@ struct Walk {
         int slices;      // > 0: [slices, m, width] (1: plain); 0: added into the stream
     };
 
+    // How the library cuts a product of this shape, asked once a walk: a model's layers share a few shapes.
+    struct Cut {
+        int m, n, k, dtype, slices;
+    };
+    std::vector<Cut> cuts;
+    int slices_of(int m, const ImparoLinearDesc& lin) {
+        for (const Cut& c : cuts)
+            if (c.m == m && c.n == lin.n && c.k == lin.k && c.dtype == lin.dtype) return c.slices;
+        cuts.push_back(Cut{m, lin.n, lin.k, lin.dtype, imparo_gemm_slices(m, lin.n, lin.k, lin.dtype)});
+        return cuts.back().slices;
+    }
+
     // A projection of m rows, as a part's Linear runs it: in slices of K where the consumer adds
     // slices and the library says that pays, added into `into` where the library's epilogue can,
     // else plain into `region`.
@@ -137,7 +149,7 @@ struct Walk {
         }
         const int width = swiglu ? lin.n / 2 : lin.n;
         if (sliced_ok && !swiglu && out_dtype == IMPARO_F32) {
-            const int slices = imparo_gemm_slices(m, lin.n, lin.k, lin.dtype);
+            const int slices = slices_of(m, lin);
             if (slices > 1) {
                 void* out = get(sliced_region, (int64_t)slices * m * width * 4);
                 launch("imparo_gemm (slices of K)", [&] {
@@ -568,6 +580,24 @@ extern "C" int imparo_program_needs(ImparoProgram* p, const ImparoStepArgs* args
     w.run();
     for (size_t i = 0; i < w.need.size(); ++i) needs[i] = w.need[i];
     return w.status;
+}
+
+extern "C" int imparo_program_needs_up_to(ImparoProgram* p, const ImparoStepArgs* args, int64_t* needs) {
+    if (!p || !args || !needs) return IMPARO_BAD_ARGUMENT;
+    for (size_t i = 0; i < p->regions.size(); ++i) needs[i] = 0;
+    ImparoStepArgs a = *args;
+    const int tile = imparo_attention_prefill_tile();
+    for (int tokens = 1; tokens <= args->n_tokens; ++tokens) {
+        a.n_tokens = a.max_seg_len = tokens;
+        a.n_rows = a.n_portion = 1;
+        a.n_single = 0;
+        a.portion_tiles = (tokens + tile - 1) / tile;
+        Walk w(p, &a, nullptr, true);
+        w.run();
+        if (w.status != IMPARO_OK) return w.status;
+        for (size_t i = 0; i < w.need.size(); ++i) needs[i] = std::max(needs[i], w.need[i]);
+    }
+    return IMPARO_OK;
 }
 
 extern "C" int imparo_program_run(ImparoProgram* p, const ImparoStepArgs* args, float** logits, imparo_stream stream) {

@@ -155,6 +155,7 @@ _SIGNATURES = {
     "imparo_program_region_name": ([P, I], ctypes.c_char_p),
     "imparo_program_bind": [P, I, P, c_int64],
     "imparo_program_needs": [P, P, P],
+    "imparo_program_needs_up_to": [P, P, P],
     "imparo_program_run": [P, P, P, P],
     "imparo_program_error": ([P], ctypes.c_char_p),
 }

@@ -141,6 +141,11 @@ class Program:
         self._ok(self._lib.imparo_program_needs(self._h, byref(args), self._needs), "needs")
         return {name: int(self._needs[i]) for i, name in enumerate(self.region_names) if self._needs[i]}
 
+    def needs_up_to(self, args: StepArgs) -> Dict[str, int]:
+        """The most bytes of every region that a step of one portion of 1 to `args.n_tokens` tokens uses."""
+        self._ok(self._lib.imparo_program_needs_up_to(self._h, byref(args), self._needs), "needs_up_to")
+        return {name: int(self._needs[i]) for i, name in enumerate(self.region_names) if self._needs[i]}
+
     def bind(self, workspace) -> None:
         """Binds every region to the workspace buffer of its name, as it is now."""
         for i, name in enumerate(self.region_names):

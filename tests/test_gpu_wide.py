@@ -213,3 +213,16 @@ def test_a_step_between_the_doublings_finds_its_scratch_reserved(wide):
     before = eng.workspace.version
     out = eng.step([StepEntry("a", prompt_tokens(65536, 1280, 5), [1279])])
     assert bool(torch.isfinite(out).all()) and eng.workspace.version == before
+
+
+def test_every_count_of_rows_finds_its_scratch_reserved(wide):
+    """The output projections, 2,048 by 2,048, come in four slices up to 485 rows and in two from there on: a step of 485 rows needs
+    more than any of 480, of 496 and of the engine's largest, 512."""
+    from imparo_amd.engine import StepEntry
+    from imparo_amd.kernels import ops
+    cut = {m: ops.gemm_slices(m, 2048, 2048, torch.bfloat16) * m for m in (480, 485, 496, 512)}
+    assert max(cut, key=cut.get) == 485
+    eng = make_engine(wide[0], "bfloat16", page_size=64, max_tokens=1024, max_requests=2, max_step_tokens=512)
+    before = eng.workspace.version
+    out = eng.step([StepEntry("a", prompt_tokens(65536, 485, 5), [484])])
+    assert bool(torch.isfinite(out).all()) and eng.workspace.version == before
