@@ -182,9 +182,12 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
 // k = g, 4 + g, 8 + g, 12 + g, which is how the products want them. Loads run seven chunks of 32 ahead in eight
 // register sets. A weight of many rows is bound by its bytes, one of few rows by the chain of a wave's products (each
 // waits for the one before it). Measured, cold weights, 2 rows: 65,536 by 1,024 57 us (4.7 TB/s), 9,216 by 1,024 14 us,
-// 1,024 by 4,608 33 us; 17 us on average over a decode step where two weight rows a thread through LDS took 79.
+// 1,024 by 4,608 33 us; 17 us on average over a decode step where two weight rows a thread through LDS took 79. The loads ask
+// for 4-byte alignment only, so a K that is no multiple of 4 and operands that start anywhere come this way too: 2 rows of 1,024 by
+// 1,026 9.9 us, 65,536 by 1,022 44 (value by value in tiles of 64 rows 50 and 144, the kernel before both 45 and 111).
 #define F32R_BK 32
 #define F32R_SETS 8
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // four floats wherever they lie
 struct RowsF32Set {
     f32x4 w[F32R_BK / 16], x[F32R_BK / 16];     // (whole vectors until they are used)
 };
@@ -218,14 +221,14 @@ __global__ __launch_bounds__(64) void k_gemm_f32_rows(const float* __restrict__ 
     // (uniform bases and 32-bit offsets inside 16 rows: a load in the loop costs no address arithmetic)
     const float* wbase = W + (size_t)n0 * K;
     const unsigned woff = (unsigned)min(r16, N - 1 - n0) * (unsigned)K + g * 4, xoff = (unsigned)min(r16, M - 1) * (unsigned)K + g * 4;
-    const int full = K / F32R_BK;                        // whole chunks; the rest of K, a multiple of 4, comes last
+    const int full = K / F32R_BK;                        // whole chunks; the rest of K comes last
     auto fetch = [&](int chunk, RowsF32Set& f) __attribute__((always_inline)) {
         const char* w0 = reinterpret_cast<const char*>(wbase + min(chunk, full - 1) * F32R_BK);
         const char* x0 = reinterpret_cast<const char*>(X + min(chunk, full - 1) * F32R_BK);
 #pragma unroll
         for (int j = 0; j < F32R_BK / 16; ++j) {
-            f.w[j] = *reinterpret_cast<const f32x4*>(w0 + woff * 4u + j * 64);
-            f.x[j] = *reinterpret_cast<const f32x4*>(x0 + xoff * 4u + j * 64);
+            f.w[j] = *reinterpret_cast<const f32x4_any*>(w0 + woff * 4u + j * 64);
+            f.x[j] = *reinterpret_cast<const f32x4_any*>(x0 + xoff * 4u + j * 64);
         }
     };
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -265,12 +268,24 @@ __global__ __launch_bounds__(64) void k_gemm_f32_rows(const float* __restrict__ 
         RowsF32Set f;
 #pragma unroll
         for (int j = 0; j < F32R_BK / 16; ++j) {         // what lies past K counts as zeros
-            const int k = full * F32R_BK + j * 16, at = min(k, K - 4 - g * 4);
-            const bool in = k + g * 4 < K;
-            const float4 w = *reinterpret_cast<const float4*>(wbase + ((long long)woff + at));
-            const float4 x = *reinterpret_cast<const float4*>(X + ((long long)xoff + at));
-            f.w[j] = f32x4{in ? w.x : 0.f, in ? w.y : 0.f, in ? w.z : 0.f, in ? w.w : 0.f};
-            f.x[j] = f32x4{in ? x.x : 0.f, in ? x.y : 0.f, in ? x.z : 0.f, in ? x.w : 0.f};
+            const int k = full * F32R_BK + j * 16 + g * 4;
+            if (K % 4 == 0) {
+                const int at = min(k, K - 4) - g * 4;
+                f.w[j] = *reinterpret_cast<const f32x4_any*>(wbase + ((long long)woff + at));
+                f.x[j] = *reinterpret_cast<const f32x4_any*>(X + ((long long)xoff + at));
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int at = min(k + i, K - 1) - g * 4;
+                    f.w[j][i] = wbase[(long long)woff + at];
+                    f.x[j][i] = X[(long long)xoff + at];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                f.w[j][i] = k + i < K ? f.w[j][i] : 0.f;
+                f.x[j][i] = k + i < K ? f.x[j][i] : 0.f;
+            }
         }
         multiply(f);
     }
@@ -295,7 +310,7 @@ template <typename TOut>
 static int launch_f32(const float* x, const float* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                       hipStream_t s) {
     const bool vec = k % 4 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w & 15);
-    if (m <= 16 && vec && k < (1 << 25)) {           // (offsets inside 16 rows are kept in 32 bits)
+    if (m <= 16 && k < (1 << 25)) {                  // (offsets inside 16 rows are kept in 32 bits)
         k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
         return launch_status();
     }
