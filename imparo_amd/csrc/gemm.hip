@@ -114,13 +114,14 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
     const int put = row * F32_LD + part;
     const int get_x = (wm + (lane & 31)) * F32_LD + (lane >> 5) * 4, get_w = (wn + (lane & 31)) * F32_LD + (lane >> 5) * 4;
-    // One step: its operands leave the registers for LDS, the step after the next two is asked for in their place
+    // One step: its operands leave the registers for LDS, the fourth step from here is asked for in their place
     // (a step takes half a microsecond, a trip to memory one or two), and the products run.
-    auto step = [&](int k0, int buf, Ahead& now) __attribute__((always_inline)) {
+    auto step = [&](int k0, int buf, Ahead& now, const bool more) __attribute__((always_inline)) {
         float x[8], w[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const bool in = k0 + part + j < K;
+            const bool in = k0 + part + j < K;           // (also where it always holds: without a choice here the compiler
+                                                         // sorts what comes as it comes, and waits for it there)
             x[j] = in ? now.x[j] : 0.f;
             w[j] = in ? now.w[j] : 0.f;
         }
@@ -131,7 +132,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
         // (the other buffer was read before the barrier of the step before; the loads in flight are not waited for)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
-        fetch(k0 + 4 * F32_BK, now);
+        if (more) fetch(k0 + 4 * F32_BK, now);
         __builtin_amdgcn_sched_barrier(0);   // (left alone, the compiler sinks these loads to where they are used)
 #pragma unroll
         for (int kb = 0; kb < F32_BK; kb += 8) {
@@ -154,12 +155,19 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
     __builtin_amdgcn_sched_barrier(0);
     fetch(3 * F32_BK, s3);
     __builtin_amdgcn_sched_barrier(0);
-    for (int k0 = 0; k0 < K; k0 += 4 * F32_BK) {      // (steps past the end add products of zeros: the sums keep their bits)
-        step(k0, 0, s0);
-        step(k0 + F32_BK, 1, s1);
-        step(k0 + 2 * F32_BK, 0, s2);
-        step(k0 + 3 * F32_BK, 1, s3);
+    const int turns = K / (4 * F32_BK) * (4 * F32_BK);
+    for (int k0 = 0; k0 < turns; k0 += 4 * F32_BK) {
+        step(k0, 0, s0, true);
+        step(k0 + F32_BK, 1, s1, true);
+        step(k0 + 2 * F32_BK, 0, s2, true);
+        step(k0 + 3 * F32_BK, 1, s3, true);
     }
+    // what is left of K, up to four steps, the last one filled up with zeros (a short K is nothing else: 4,096 rows by 1,024
+    // by 8 9.3 us where steps to the end of the turn took 18 and steps of 16 on the vector units 11)
+    if (turns < K) step(turns, 0, s0, false);
+    if (turns + F32_BK < K) step(turns + F32_BK, 1, s1, false);
+    if (turns + 2 * F32_BK < K) step(turns + 2 * F32_BK, 0, s2, false);
+    if (turns + 3 * F32_BK < K) step(turns + 3 * F32_BK, 1, s3, false);
     // a lane holds one column (a weight row) of 16 activation rows
     const int n = n0 + wn + (lane & 31);
     const float bn = bias && n < N ? bias[n] : 0.f;

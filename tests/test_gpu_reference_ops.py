@@ -34,7 +34,8 @@ def test_float32_product_is_the_statement_bit_for_bit(m, n, k):
     assert np.abs(out.cpu().numpy() - ref).max() <= 1e-6 * math.sqrt(k) * np.abs(ref).max()
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (1, 1, 1), (2, 16, 3), (5, 18, 33), (16, 15, 290), (9, 40, 1023), (16, 17, 60), (16, 33, 1028), (17, 64, 32), (63, 65, 36), (64, 66, 260), (129, 31, 100)])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 4), (1, 1, 1), (2, 16, 3), (5, 18, 33), (16, 15, 290), (9, 40, 1023), (16, 17, 60), (16, 33, 1028), (17, 64, 32), (63, 65, 36), (64, 66, 260), (129, 31, 100),
+                                   (17, 20, 1), (18, 66, 3), (65, 64, 5), (64, 33, 257), (70, 65, 258), (33, 130, 1155)])
 def test_float32_product_at_the_edges_of_its_tiles(m, n, k):
     """Rows and columns beside whole tiles, K beside whole steps and no multiple of 4, operands that start 4 bytes off 16, and
     the gated epilogue, bit for bit."""
