@@ -73,7 +73,10 @@ __device__ __forceinline__ uint4 zero_if(bool out, uint4 v) {
 #define F32_BK 32
 #define F32_LD 40   // floats from row to row in LDS: 32 bytes beyond a row's own, which keeps 16-byte reads free of conflicts
 
-// VEC: K is a multiple of 4 and both operands' rows start 16 bytes aligned; else they are read value by value.
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // four floats wherever they lie
+// VEC: K is at least 4, and rows are read in vectors of four floats that may start anywhere; the end of a K that is no
+// multiple of 4, and a shorter K, value by value. (666 rows by 9,216 by 1,024 that start 4 bytes off 16:
+// 140 us, 395 value by value.)
 template <typename TOut, bool VEC>
 __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, const float* __restrict__ W,
                                                   const float* __restrict__ bias, TOut* __restrict__ Y,
@@ -94,19 +97,22 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
     struct Ahead {
         float x[8], w[8];
     };
+    auto fetch_values = [&](int k0, Ahead& f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f.x[j] = xrow[min(k0 + part + j, K - 1)], f.w[j] = wrow[min(k0 + part + j, K - 1)];
+    };
     auto fetch = [&](int k0, Ahead& f) __attribute__((always_inline)) {     // no load under a branch; what lies past K is zero
         const int k = k0 + part;
         if (VEC) {
 #pragma unroll
             for (int j = 0; j < 8; j += 4) {
                 const int at = min(k + j, K - 4);
-                const float4 a = *reinterpret_cast<const float4*>(xrow + at), b = *reinterpret_cast<const float4*>(wrow + at);
+                const f32x4_any a = *reinterpret_cast<const f32x4_any*>(xrow + at), b = *reinterpret_cast<const f32x4_any*>(wrow + at);
                 f.x[j] = a.x, f.x[j + 1] = a.y, f.x[j + 2] = a.z, f.x[j + 3] = a.w;
                 f.w[j] = b.x, f.w[j + 1] = b.y, f.w[j + 2] = b.z, f.w[j + 3] = b.w;
             }
         } else {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) f.x[j] = xrow[min(k + j, K - 1)], f.w[j] = wrow[min(k + j, K - 1)];
+            fetch_values(k0, f);
         }
     };
     f32x16 acc;
@@ -164,10 +170,15 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
     }
     // what is left of K, up to four steps, the last one filled up with zeros (a short K is nothing else: 4,096 rows by 1,024
     // by 8 9.3 us where steps to the end of the turn took 18 and steps of 16 on the vector units 11)
-    if (turns < K) step(turns, 0, s0, false);
-    if (turns + F32_BK < K) step(turns + F32_BK, 1, s1, false);
-    if (turns + 2 * F32_BK < K) step(turns + 2 * F32_BK, 0, s2, false);
-    if (turns + 3 * F32_BK < K) step(turns + 3 * F32_BK, 1, s3, false);
+    auto rest = [&](int k0, int buf, Ahead& f) __attribute__((always_inline)) {
+        if (k0 >= K) return;
+        if (VEC && K % 4 && k0 + F32_BK > K) fetch_values(k0, f);
+        step(k0, buf, f, false);
+    };
+    rest(turns, 0, s0);
+    rest(turns + F32_BK, 1, s1);
+    rest(turns + 2 * F32_BK, 0, s2);
+    rest(turns + 3 * F32_BK, 1, s3);
     // a lane holds one column (a weight row) of 16 activation rows
     const int n = n0 + wn + (lane & 31);
     const float bn = bias && n < N ? bias[n] : 0.f;
@@ -195,7 +206,6 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
 // 1,026 9.9 us, 65,536 by 1,022 44 (value by value in tiles of 64 rows 50 and 144, the kernel before both 45 and 111).
 #define F32R_BK 32
 #define F32R_SETS 8
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // four floats wherever they lie
 struct RowsF32Set {
     f32x4 w[F32R_BK / 16], x[F32R_BK / 16];     // (whole vectors until they are used)
 };
@@ -317,7 +327,6 @@ __global__ __launch_bounds__(64) void k_gemm_f32_rows(const float* __restrict__ 
 template <typename TOut>
 static int launch_f32(const float* x, const float* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                       hipStream_t s) {
-    const bool vec = k % 4 == 0 && !((uintptr_t)x & 15) && !((uintptr_t)w & 15);
     if (m <= 16 && k < (1 << 25)) {                  // (offsets inside 16 rows are kept in 32 bits)
         k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
         return launch_status();
@@ -326,7 +335,7 @@ static int launch_f32(const float* x, const float* w, const float* bias, TOut* y
     const long long total = (long long)tiles_m * tiles_n;
     if (total > 0x7ffffff0LL) return IMPARO_BAD_ARGUMENT;
     const unsigned blocks = (unsigned)((total + 7) / 8 * 8);
-    if (vec)
+    if (k >= 4)
         k_gemm_f32<TOut, true><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
     else
         k_gemm_f32<TOut, false><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
