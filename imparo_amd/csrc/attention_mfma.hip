@@ -331,11 +331,13 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
     }
 }
 
-// SPLITS > 1: the block has the waves of that many splits, all that a row can have, and adds their results itself, in
-// the merge kernel's order, so there is no launch for that. A short context is bound by launches (a merge behind this
-// kernel takes 4.5 us however little it adds), a long one by how many CUs draw on the cache, which wants a block a split.
-// Measured, 8 rows of 32 heads of 64 over 300 keys, two splits, the projection's rows normed and rotated here: 11.2 us where
-// the two launches took 9.3 and 4.6; one row of 16 heads over 50 keys 8.5 where they took 7.1 and 4.5.
+// SPLITS 2: the block has the waves of both splits, all that a row can have, and adds their results itself, in the merge
+// kernel's order, so there is no launch for that. A short context is bound by launches, and a merge behind this kernel takes
+// 2 to 5 us however little it adds; a longer one by how many CUs draw on the cache, which wants a block a split. Measured
+// launch behind launch, us here | with the merge: 8 rows of 32 heads of 64 over 300 keys, the projection's rows normed and
+// rotated here, 9.6 | 11.1, over 60 keys 7.2 | 10.5, queries given 7.1 | 10.1; 24 heads of 128, queries given, 11.4 | 12.7. Not
+// from the projection's rows with heads above 64 (15.4 | 14.4: both splits' waves make the rotations one CU's four SIMDs then
+// share), nor three or four splits (16 waves on one CU: 1,000 keys 17.7 | 13.4, queries given 12.9 | 11.7).
 template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1>
 __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decode(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -507,33 +509,17 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         }
         const int head_out = kvh * G + pass * 16 + qc;
         if constexpr (SPLITS > 1) {
-            // as the merge kernel adds them: the splits the row has, counted from its first, dealt to as many sides as
-            // heads of this size let a wave take at once
-            constexpr int SIDE = WAVE / (D / 4);
-            const int s_lo = EXT ? 0 : (lo & ~15) / DEC_SPLIT;
-            const int s_hi = min((EXT ? pos - walk.gap : pos) / DEC_SPLIT, SPLITS - 1);
-            float ms = -INFINITY;
-#pragma unroll
-            for (int sp = 0; sp < SPLITS; ++sp) ms = fmaxf(ms, m_of[sp]);
-            float part[4] = {0.f, 0.f, 0.f, 0.f}, l_part[4] = {0.f, 0.f, 0.f, 0.f};     // counted from the first split
+#pragma clang fp contract(off)
+            // as the merge kernel adds them: products rounded before they are added, in the order of the splits (one without
+            // keys weighs nothing)
+            static_assert(SPLITS == 2, "the sums below are two splits'");
+            const float ms = fmaxf(m_of[0], m_of[1]);
+            float total = 0.f, ls = 0.f;
 #pragma unroll
             for (int sp = 0; sp < SPLITS; ++sp) {
                 const float w = (m_of[sp] == -INFINITY) ? 0.f : __expf(m_of[sp] - ms);
-#pragma unroll
-                for (int i = 0; i < SPLITS; ++i)
-                    if (sp >= s_lo && sp <= s_hi && sp - s_lo == i) {
-                        part[i] = __fmul_rn(acc_of[sp], w);
-                        l_part[i] = __fmul_rn(l_of[sp], w);
-                    }
-            }
-            const float ls = (l_part[0] + l_part[2]) + (l_part[1] + l_part[3]);
-            float total = 0.f;
-#pragma unroll
-            for (int side = 0; side < SIDE && side < 4; ++side) {
-                float a = 0.f;
-#pragma unroll
-                for (int i = side; i < 4; i += SIDE) a += part[i];
-                total += a;
+                total += acc_of[sp] * w;
+                ls += l_of[sp] * w;
             }
             const float inv = EXT ? ruled_inverse(rule, t, head_out, ms, ls) : (ls > 0.f ? 1.0f / ls : 0.f);
             out[((size_t)t * heads + head_out) * D + d] = f32_to_bf16(total * inv);
@@ -1417,18 +1403,16 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
     if (given && from_qkv) return IMPARO_BAD_ARGUMENT;
     // the merge moves four elements of a head in one access
     if (n_splits > 1 && (((uintptr_t)part_o & 15) || ((uintptr_t)out & 7))) return IMPARO_BAD_ARGUMENT;
-    // Two splits, or up to four with heads of at most 64: one block takes them all and there is no merge. (Sixteen waves
-    // of larger heads would not find registers; from five splits on a block a split draws on more CUs.)
-    const int in_block = n_splits == 2 ? 2 : n_splits <= 4 && n_splits > 2 && head_dim <= 64 ? 4 : 1;
-    dim3 grid(in_block > 1 ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
+    // two splits: one block takes both and there is no merge, where that is the faster way (k_attn_decode)
+    const bool in_block = n_splits == 2 && !(from_qkv && head_dim > 64);
+    dim3 grid(in_block ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
 #define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT)                                                                \
     k_attn_decode<ND, QKV, EXT, SPLITS><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                                   \
         Q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,           \
         positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, EXACT, rule)
 #define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT)                                                                       \
     do {                                                                                                             \
-        if (in_block == 2) DECODE_GO(ND, QKV, EXT, 2, Q, FQ, EXACT);                                                 \
-        else if (in_block == 4) DECODE_GO(ND, QKV, EXT, (ND <= 4 ? 4 : 2), Q, FQ, EXACT);                            \
+        if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT);                                \
         else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT);                                                               \
     } while (0)
     if (from_qkv) {
@@ -1443,7 +1427,7 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
 #undef DECODE_ANY
 #undef DECODE_GO
     if (launch_status()) return IMPARO_LAUNCH_FAILED;
-    if (n_splits == 1 || in_block > 1) return IMPARO_OK;
+    if (n_splits == 1 || in_block) return IMPARO_OK;
     if (given)
         k_attn_decode_merge<true><<<n_rows * heads, 64, 0, s>>>(part_o, part_ml, (bf16_t*)out, rows, seg_start, positions,
                                                                 heads, head_dim, n_splits, window, rule);

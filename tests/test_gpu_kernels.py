@@ -617,13 +617,49 @@ def test_matrix_core_attention_with_32_queries_a_wave(H, Hk, D, ctx, q):
 @pytest.mark.parametrize("lens", [(1, 255, 256, 257, 512, 70), (1, 512, 513, 768, 1000, 1024, 257)])
 @pytest.mark.parametrize("window", [None, 300, 1])
 def test_decode_attention_merges_few_splits_in_the_block(H, Hk, D, lens, window):
-    """Contexts of up to two splits of 256 keys, and of up to four: one launch. The same rows with block tables that have
-    room for nine splits take the merge launch: the same bits, a row of one split among many included."""
+    """Contexts of up to two splits of 256 keys: one launch; of up to four: a block a split and a merge. The same rows with
+    block tables that have room for nine splits: the same bits, a row of one split among many included."""
     n, lens, one = len(lens), lens + (40,), [1] * len(lens) + [5]            # (a portion beside them: the case wants one)
     got, ref = _attention_case(H, Hk, D, 64, window, torch.bfloat16, kernel="mfma", ctx_lens=lens, q_lens=one)
     torch.testing.assert_close(got, ref, rtol=2 ** -6, atol=2 ** -6)
     merged, _ = _attention_case(H, Hk, D, 64, window, torch.bfloat16, kernel="mfma", ctx_lens=lens, q_lens=one, table_width=33)
     assert torch.equal(got[:n], merged[:n])
+
+
+@pytest.mark.parametrize("form", ["qkv", "exact", "ruled"])
+@pytest.mark.parametrize("H,Hk,D", [(8, 2, 64), (40, 2, 64), (4, 1, 128), (6, 2, 80)])
+@pytest.mark.parametrize("window", [None, 300])
+def test_every_form_of_decode_attention_merges_two_splits_as_the_merge_does(form, H, Hk, D, window, monkeypatch):
+    """Contexts of up to 512 keys with partial results for two splits (one launch where it is the faster way) and for nine (a
+    block a split and the merge): the same bits for the projection's rows, exact weights, and a rule with first positions
+    that stay, a cap, a sink and a gate. The row's own key is the last of the first split, alone in the second, and the
+    last of both; from the projection's rows the same keys and values are written."""
+    if form == "qkv" and D not in (64, 128):
+        pytest.skip("the projection's rows: heads of 64 and 128")
+    monkeypatch.setattr(ops(), "attention_ruled_keys", lambda max_context, window, rule: max_context)
+    lens, page = (1, 255, 256, 257, 300, 512, 40), 64
+    R, n_pages = len(lens), sum(-(-c // page) for c in lens) + 2
+    ctx = hand_context([(c - 1, 1) for c in lens], page, n_pages, torch.bfloat16, DEV, kv_sites={0: (Hk, D)}, v_transposed=True)
+    k0, v0, table = ctx.kv(0)
+    k0.copy_(rnd(*k0.shape, seed=1)), v0.copy_(rnd(*v0.shape, seed=2))
+    qkv, q = rnd(R, (H + 2 * Hk) * D, seed=3).to(DEV), rnd(R, H, D, seed=4).to(torch.bfloat16).to(DEV)
+    weight, freq = (1 + 0.1 * rnd(D, seed=5)).to(DEV), torch.linspace(1.0, 0.01, D // 2, device=DEV)
+    gates = rnd(R, H, seed=6).to(DEV)
+    rule = ops().attention_rule(H, keep_first=70 if window else 0, softcap=20.0, sink=rnd(H, seed=7).to(DEV)).with_gate(gates, 0)
+    got = []
+    for splits in (2, 9):
+        k, v = k0.clone(), v0.clone()
+        out = torch.full((R, H * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        part_o, part_ml = (torch.full((R * H * splits * n,), float("nan"), device=DEV) for n in (D, 2))
+        tail = (part_o, part_ml, ctx.single_rows, R, ctx.seg_start, ctx.positions, table)
+        if form == "qkv":
+            ops().attention_decode_qkv(qkv, weight, weight, 1e-5, freq, k, v, out, *tail, H, 0.125, window, 256 * splits)
+        else:
+            ops().attention_decode(q, k, v, out, *tail, 0.125, window, 256 * splits, exact=True, rule=rule if form == "ruled" else None)
+        got.append((out.cpu(), k.cpu(), v.cpu()))
+    assert bool(torch.isfinite(got[0][0]).all())
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("H,Hk,D", [(8, 2, 64), (5, 5, 64), (40, 2, 64), (4, 1, 128)])
