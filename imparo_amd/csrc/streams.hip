@@ -51,7 +51,7 @@ __device__ __forceinline__ void stream_store(float* __restrict__ p, const float 
 }
 
 // One block a row; a thread keeps PER pieces of V neighbouring values of u in registers. S: at least `streams`.
-template <int S, int V, int PER>
+template <int S, int V, int PER, bool EARLY>
 __global__ __launch_bounds__(1024) void k_stream_norm(
     const float* x, int in_streams, float* x_out, const float* __restrict__ delta, int n_delta,
     size_t delta_stride, StreamExperts moe, const int32_t* __restrict__ rows, int streams,
@@ -66,12 +66,24 @@ __global__ __launch_bounds__(1024) void k_stream_norm(
     const size_t t = rows ? rows[i_out] : i_out;
     const bool adds = moe.y || n_delta;
     const int pieces = width / V;
-    // What depends on nothing is asked for first, all of it before anything is waited for: with few rows (a decode step)
+    // What depends on nothing is asked for first (EARLY), all of it before anything is waited for: with few rows (a decode step)
     // this kernel is a chain of trips to memory, and these are then one. (8 rows of 1,024 on four copies: 6.0 us where
     // it took 7.8 with the weights, the experts' places and the row one after the other.) Threads that keep several
     // pieces of a wide row ask for each piece's row where they use it.
-    constexpr bool EARLY = PER == 1;
+    static_assert(!EARLY || PER == 1, "a thread's only piece");
+    // Experts' rows are asked for without a branch (FREE), but for many single values a thread: sixteen times the code in
+    // the unrolled pieces pushes 16 copies out of the registers (one row of 2,048 by 16 copies 421 us with the branch, 505
+    // without).
+    constexpr bool FREE = PER == 1 || V == 4;
     const int c_own = min(tid, pieces - 1) * V;
+    auto passed = [&](int c) __attribute__((always_inline)) {          // what an expert that passes its input through gives
+        StreamPiece<V> r;
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            r.e[i] = moe.h_is_bf16 ? load_f32<bf16_t>((const bf16_t*)moe.h, t * width + c + i)
+                                   : load_f32<float>((const float*)moe.h, t * width + c + i);
+        return r;
+    };
     StreamPiece<V> v_own[S], w_own, b_own, d_own;
     if (EARLY) {
 #pragma unroll
@@ -117,16 +129,13 @@ __global__ __launch_bounds__(1024) void k_stream_norm(
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int sl = slot[min(k0 + j, moe.top - 1)];
-                    y[j] = stream_load<V>(moe.y + (size_t)max(sl, 0) * width + c);      // (no load under a branch)
+                    if (FREE || sl >= 0) y[j] = stream_load<V>(moe.y + (size_t)max(sl, 0) * width + c);
+                    else y[j] = passed(c);
                 }
+                if (FREE)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (__builtin_amdgcn_readfirstlane(slot[min(k0 + j, moe.top - 1)]) < 0) {    // passes its input through
-#pragma unroll
-                        for (int i = 0; i < V; ++i)
-                            y[j].e[i] = moe.h_is_bf16 ? load_f32<bf16_t>((const bf16_t*)moe.h, t * width + c + i)
-                                                      : load_f32<float>((const float*)moe.h, t * width + c + i);
-                    }
+                    for (int j = 0; j < 4; ++j)
+                        if (__builtin_amdgcn_readfirstlane(slot[min(k0 + j, moe.top - 1)]) < 0) y[j] = passed(c);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const float w = k0 + j < moe.top ? wt[k0 + j] : 0.f;
@@ -257,12 +266,20 @@ extern "C" int imparo_stream_norm(const float* x, int in_streams, float* x_out, 
     const int threads = pieces >= 1024 ? 1024 : (pieces + WAVE - 1) / WAVE * WAVE;
     const int per = (pieces + threads - 1) / threads;
     const int out_is_bf16 = out_dtype == IMPARO_BF16;
+    // Once there are several rounds of blocks, how many of them a CU holds is what counts, and what is asked for early takes
+    // registers, of more copies more: 2,048 rows of 2,048, early | late: 18.4 | 17.4 us by 2 copies, 36.6 | 33.4 by 5, 59 | 54 by
+    // 8; 8,192 rows of 1,024 by 4 60 | 56; 1,023 rows of 2,048 by 4 still 14.3 | 16.1, of 1,280 by 8 18.6 | 17.5. With experts' rows
+    // early is the faster way at any count (2,048 rows of 2,048 by 8 copies 74 | 86).
+    const bool late = !y && per <= 1 && (long long)n_out * threads >= (streams > 4 ? 1 << 18 : 600000);
 #define STREAM_NORM(S, V, PER)                                                                                       \
-    k_stream_norm<S, V, PER><<<n_out, threads, 0, s>>>(x, in_streams, x_out, delta, n_delta, stride, moe, rows, streams, \
+    k_stream_norm<S, V, PER, (PER == 1)><<<n_out, threads, 0, s>>>(x, in_streams, x_out, delta, n_delta, stride, moe, rows, streams, \
                                                        mix, join, read, norm, weight, bias, eps, out, out_is_bf16, width)
 #define STREAM_WIDTHS(S)                                                                                             \
     if (four) {                                                                                                      \
-        if (per <= 1) STREAM_NORM(S, 4, 1);                                                                          \
+        if (late) k_stream_norm<S, 4, 1, false><<<n_out, threads, 0, s>>>(                                           \
+            x, in_streams, x_out, delta, n_delta, stride, moe, rows, streams, mix, join, read, norm, weight, bias,   \
+            eps, out, out_is_bf16, width);                                                                           \
+        else if (per <= 1) STREAM_NORM(S, 4, 1);                                                                     \
         else STREAM_NORM(S, 4, 4);                                                                                   \
     } else {                                                                                                         \
         if (per <= 1) STREAM_NORM(S, 1, 1);                                                                          \
@@ -281,6 +298,6 @@ extern "C" int imparo_stream_norm(const float* x, int in_streams, float* x_out, 
 
 int imparo_load_code_streams() {
     hipFuncAttributes attributes;
-    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_stream_norm<4, 4, 1>)) == hipSuccess
+    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_stream_norm<4, 4, 1, true>)) == hipSuccess
                ? IMPARO_OK : IMPARO_LAUNCH_FAILED;
 }

@@ -408,6 +408,26 @@ def test_weights_over_the_chosen_outputs(X, top, T):
         assert sorted(s1.cpu().tolist()) == list(range(n)) and bool((choice.cpu()[s2.cpu().long() // (top + 1), top] == X).all())
 
 
+@pytest.mark.parametrize("S,E,T", [(1, 2048, 1200), (2, 1028, 2001), (4, 1024, 2500), (8, 2048, 520)])
+@pytest.mark.parametrize("n_delta", [1, 3])
+def test_streams_of_many_rows_are_those_of_few(S, E, T, n_delta):
+    """From some rows on a block asks for a row where it uses it, and not ahead: the same bits as in thirds of the rows, the copies
+    that are written back and the normed rows."""
+    from imparo_amd.kernels import ops
+    g = torch.Generator().manual_seed(S)
+    r = lambda *shape: dev(torch.randn(*shape, generator=g))
+    x, delta, w, b, mix, join, read = r(T, S, E), r(n_delta, T, E), r(E), r(E), r(S, S), r(S), r(S)
+
+    def run(lo, hi):
+        x_out, out = torch.empty(hi - lo, S, E, device=DEV), torch.empty(hi - lo, E, device=DEV)
+        ops.stream_norm(x[lo:hi], "layer", w, b, 1e-5, out, delta=delta[:, lo:hi].contiguous(), mix=mix, join=join, read=read, x_out=x_out)
+        return x_out, out
+
+    many, thirds = run(0, T), [run(T * i // 3, T * (i + 1) // 3) for i in range(3)]
+    for i in range(2):
+        assert torch.equal(many[i], torch.cat([part[i] for part in thirds]))
+
+
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
 @pytest.mark.parametrize("X,top", [(1, 1), (8, 4), (16, 16), (63, 5), (64, 16)])
 def test_choice_among_few_outputs_is_the_general_one(X, top, scoring):
