@@ -429,7 +429,7 @@ def test_streams_of_many_rows_are_those_of_few(S, E, T, n_delta):
 
 
 @pytest.mark.parametrize("scoring", ["softmax", "sigmoid", "chosen"])
-@pytest.mark.parametrize("X,top", [(1, 1), (8, 4), (16, 16), (63, 5), (64, 16)])
+@pytest.mark.parametrize("X,top", [(1, 1), (8, 4), (16, 16), (32, 1), (33, 1), (33, 3), (64, 2), (63, 5), (64, 16)])
 def test_choice_among_few_outputs_is_the_general_one(X, top, scoring):
     """At most 64 outputs are ranked by counting; the same rows with outputs past the 64th that cannot be chosen go the
     general way and give the same choices and weights, bit for bit: equal outputs, rows with too few that can be chosen
