@@ -918,11 +918,16 @@ extern "C" int imparo_moe_gemm(const void* a, int a_ld, int gather_div, const in
 #define MOE_LAUNCH_GATED(WM)                                                                                         \
     k_moe_gemm_bf16<WM, 2, bf16_t, true><<<dim3(max_tiles, (n + 127) / 128), 256, 0, s>>>(                           \
         (const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (bf16_t*)out, tiles, n, k, epilogue, gate)
-    // tiles of 128 rows whose K comes in the steps that go straight into LDS, unless 256 columns a tile leave more than a
-    // quarter of the columns empty beside tiles of 128 (the kernels' rates are 1.6 to 1)
-    const int tiles_n = (n + MOE_DMA_N - 1) / MOE_DMA_N;
+    // Tiles of 128 rows whose K comes in the steps that go straight into LDS: where 256 columns a tile leave no more than a
+    // quarter of the columns empty beside tiles of 128, and cost no more rounds of the CUs (256 blocks of these at once, 512
+    // of the others; a round of these is the shorter one by a quarter and more). 8,192 slots of 8 experts, 896 columns, K = 512: 2
+    // rounds 25.6 us, the other kernel's one 21.6; 32,768 slots, 5 rounds 65, the others' 4 73. From K = 128 on: with 64 there
+    // is nothing to keep in flight (8,192 slots, 1,024 columns 16.8 us, 16.0).
+    const int tiles_n = (n + MOE_DMA_N - 1) / MOE_DMA_N, narrow_n = (n + 127) / 128;
     const long long blocks = ((long long)max_tiles * tiles_n + 7) / 8 * 8;
-    if (tile_rows == 128 && k % MOE_DMA_BK == 0 && 4 * tiles_n * MOE_DMA_N <= 5 * ((n + 127) / 128 * 128) && blocks < (1LL << 31)) {
+    const long long rounds = ((long long)max_tiles * tiles_n + 255) / 256, narrow_rounds = ((long long)max_tiles * narrow_n + 511) / 512;
+    if (tile_rows == 128 && k % MOE_DMA_BK == 0 && k > MOE_DMA_BK && 4 * tiles_n * MOE_DMA_N <= 5 * narrow_n * 128 &&
+        4 * rounds <= 5 * narrow_rounds && blocks < (1LL << 31)) {
 #define MOE_LAUNCH_DMA(TO, G)                                                                                        \
     do {                                                                                                             \
         if (hipFuncSetAttribute((const void*)k_moe_gemm_dma<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize,      \

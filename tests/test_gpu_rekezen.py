@@ -514,7 +514,7 @@ def test_product_of_the_experts_with_the_unit_behind_it(T, X, top, F, K, bounds)
         near(got[:, j], want, 8e-3, f"choice {j}")
 
 
-@pytest.mark.parametrize("counts,N,K", [((128, 127, 129, 1, 0, 300), 256, 64), ((200, 256), 500, 128), ((513, 100, 60), 448, 192),
+@pytest.mark.parametrize("counts,N,K", [((128, 127, 129, 1, 0, 300), 256, 64), ((128, 127, 129, 1, 0, 300), 256, 128), ((200, 256), 500, 128), ((513, 100, 60), 448, 192),
                                         ((128, 128, 128), 768, 1024)])
 @pytest.mark.parametrize("epilogue,out_dtype", [("relu2", torch.bfloat16), (None, torch.float32), ("gated", torch.bfloat16)])
 def test_product_of_the_experts_at_the_edges_of_wide_tiles(counts, N, K, epilogue, out_dtype):
@@ -529,13 +529,11 @@ def test_product_of_the_experts_at_the_edges_of_wide_tiles(counts, N, K, epilogu
     w = (torch.randn(X, N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16)
     slot, entry = torch.empty(n, dtype=torch.int32, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
     live = sum(-(-c // 128) for c in counts)
-    for length in (ops.moe_max_tiles(n, X, 128), live + 1):
-        if length < ops.moe_max_tiles(n, X, 128):
-            tiles = tiles[:length].contiguous() if length > live else tiles
-        else:
-            tiles = torch.empty(length, 3, dtype=torch.int32, device=DEV)
-            ops.moe_plan(i32(choice), X, 128, slot, entry, tiles)
-        assert (tiles[:, 0] >= 0).sum() == live
+    tiles = torch.empty(ops.moe_max_tiles(n, X, 128), 3, dtype=torch.int32, device=DEV)
+    ops.moe_plan(i32(choice), X, 128, slot, entry, tiles)
+    for length in (tiles.shape[0], live + 1, live):
+        tiles = tiles[:length].contiguous()
+        assert (tiles[:, 0] >= 0).sum() == live and (length > live) == bool((tiles[-1, 0] < 0).item())
         cols = N // 2 if epilogue == "gated" else N
         out = torch.full((n, cols), 7.0, dtype=out_dtype, device=DEV)
         ops.moe_gemm(dev(h, torch.bfloat16), dev(w, torch.bfloat16), out, tiles, 128, entry, gather_div=1, epilogue=epilogue)
