@@ -86,8 +86,9 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
     // blocks that share weight rows are neighbours on one XCD (they go to the 8 XCDs in turn, each has an L2)
     const int total = tiles_m * tiles_n;
     const int per_xcd = (total + 7) / 8;
-    const int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (logical >= total) return;
+    const int block = blockIdx.y * gridDim.x + blockIdx.x;   // (a row of the grid is a multiple of 8)
+    const int logical = (block % 8) * per_xcd + block / 8;
+    if (block / 8 >= per_xcd || logical >= total) return;
     const int m0 = (logical % tiles_m) * F32_BM, n0 = (logical / tiles_m) * F32_BN;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
@@ -331,10 +332,13 @@ static int launch_f32(const float* x, const float* w, const float* bias, TOut* y
         k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
         return launch_status();
     }
-    const int tiles_m = (m + F32_BM - 1) / F32_BM, tiles_n = (n + F32_BN - 1) / F32_BN;
+    if (m > 65535 * F32_BM) return IMPARO_BAD_ARGUMENT;
+    const int tiles_m = (m + F32_BM - 1) / F32_BM, tiles_n = (n - 1) / F32_BN + 1;
     const long long total = (long long)tiles_m * tiles_n;
-    if (total > 0x7ffffff0LL) return IMPARO_BAD_ARGUMENT;
-    const unsigned blocks = (unsigned)((total + 7) / 8 * 8);
+    if (total > 0x7f000000LL) return IMPARO_BAD_ARGUMENT;
+    // (a launch holds fewer than 2^32 threads along x)
+    const long long row = std::min<long long>((total + 7) / 8 * 8, 1LL << 23);
+    const dim3 blocks((unsigned)row, (unsigned)((total + row - 1) / row));
     if (k >= 4)
         k_gemm_f32<TOut, true><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
     else

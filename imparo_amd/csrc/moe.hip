@@ -927,7 +927,7 @@ extern "C" int imparo_moe_gemm(const void* a, int a_ld, int gather_div, const in
     const long long blocks = ((long long)max_tiles * tiles_n + 7) / 8 * 8;
     const long long rounds = ((long long)max_tiles * tiles_n + 255) / 256, narrow_rounds = ((long long)max_tiles * narrow_n + 511) / 512;
     if (tile_rows == 128 && k % MOE_DMA_BK == 0 && k > MOE_DMA_BK && 4 * tiles_n * MOE_DMA_N <= 5 * narrow_n * 128 &&
-        4 * rounds <= 5 * narrow_rounds && blocks < (1LL << 31)) {
+        4 * rounds <= 5 * narrow_rounds && blocks < (1LL << 23)) {       // (a launch holds fewer than 2^32 threads along x)
 #define MOE_LAUNCH_DMA(TO, G)                                                                                        \
     do {                                                                                                             \
         if (hipFuncSetAttribute((const void*)k_moe_gemm_dma<TO, G>, hipFuncAttributeMaxDynamicSharedMemorySize,      \

@@ -51,3 +51,12 @@ def test_what_steps_up_to_a_size_need_is_the_most_of_every_count(width, ff, toke
     assert list(most) == want
     slices = [ops.gemm_slices(t, width, ff, torch.bfloat16) for t in range(1, tokens + 1)]
     assert most[names.index("ffn_out_sliced")] == 4 * width * max(s * (t + 1) if s > 1 else 0 for t, s in enumerate(slices))
+
+
+@pytest.mark.parametrize("m", [65535 * 64 + 1, 2 ** 31 - 1])
+@pytest.mark.parametrize("out_dtype", [0, 1])
+def test_float32_product_refuses_more_rows_than_its_grid_takes(m, out_dtype):
+    """Refused by its sizes, before anything is launched (the addresses are nobody's), also where rounding the rows up to tiles
+    would pass 2^31."""
+    at, refused = 1 << 20, 1
+    assert library().imparo_gemm(at, at, None, at, 0, out_dtype, m, 64, 4, 0, 1, None) == refused
