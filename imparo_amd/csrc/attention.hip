@@ -155,7 +155,10 @@ __global__ void k_attention_wave(const T* __restrict__ q, const T* __restrict__ 
 // chunk ahead; value rows come 32 at a time (16 of 128 numbers), their places and weights from lane registers, no load under a branch.
 // Measured, two decoded tokens at 340 keys, 16 heads of 64: 30 us where the general kernel takes 200; two prompts of
 // 333 tokens: 120 us where it takes 270.
-template <int HD>
+// ONE: the block table has room for 64 keys at most, so one chunk holds them all: nothing is asked for ahead, no row without a
+// key, value rows eight at a time, a third of the registers. (Many short prompts fill the chip and are bound by what they ask
+// for: 64 of 30 tokens, 16 heads of 64, 76 us in the loop, 38 here, 73 in the general kernel.)
+template <int HD, bool ONE>
 __global__ __launch_bounds__(ATT_WAVES * WAVE) void k_attention_wave_f32(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, float* __restrict__ out,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ row_of_token, const int32_t* __restrict__ block_table,
@@ -200,9 +203,9 @@ __global__ __launch_bounds__(ATT_WAVES * WAVE) void k_attention_wave_f32(
     for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
     float m = -INFINITY, l = 0.f;
     int c = keep > 0 ? 0 : lo_chunk;
-    int row = row_of(c), row_next = row_of(min(next_of(c), pos));      // (places are looked up two chunks ahead of their rows)
-    ask(row);
-    while (c <= pos) {
+    if constexpr (ONE) {
+        const int row = row_of(c);
+        if (row >= 0) ask(row);
         float s = 0.f;
 #pragma unroll
         for (int i = 0; i < HD / 4; ++i) {
@@ -215,35 +218,70 @@ __global__ __launch_bounds__(ATT_WAVES * WAVE) void k_attention_wave_f32(
         s *= scale;
         if (rule.softcap > 0.f) s = rule.softcap * tanhf(s / rule.softcap);
         if (row < 0) s = -INFINITY;
-        const int c_next = next_of(c);
-        ask(row_next);
-        const int row_after = row_of(min(next_of(c_next), pos));       // (past the end: nobody looks at it)
-        const float m_new = fmaxf(m, wave_max(s));
-        const float pe = row >= 0 ? expf(s - m_new) : 0.f;
-        const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
-        l = fmaf(l, corr, wave_sum(pe));
-        m = m_new;
-        const int n_keys = min(WAVE, pos - c + 1);
+        m = fmaxf(m, wave_max(s));
+        const float pe = row >= 0 ? expf(s - m) : 0.f;
+        l = wave_sum(pe);
+        for (int k0 = 0; k0 <= pos - c; k0 += 8) {
+            float v[8][DPL], w[8];
+            int at[8];
 #pragma unroll
-        for (int j = 0; j < DPL; ++j) acc[j] *= corr;
-        for (int k0 = 0; k0 < n_keys; k0 += AHEAD) {
-            float v[AHEAD][DPL], w[AHEAD];
-            int at[AHEAD];
-#pragma unroll
-            for (int kk = 0; kk < AHEAD; ++kk) {
+            for (int kk = 0; kk < 8; ++kk) {
                 at[kk] = __builtin_amdgcn_readlane(row, k0 + kk);
                 w[kk] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pe), k0 + kk));
 #pragma unroll
                 for (int j = 0; j < DPL; ++j) v[kk][j] = v_cache[(size_t)max(at[kk], 0) * HD + lane + j * WAVE];
             }
 #pragma unroll
-            for (int kk = 0; kk < AHEAD; ++kk)
+            for (int kk = 0; kk < 8; ++kk)
 #pragma unroll
                 for (int j = 0; j < DPL; ++j) acc[j] = at[kk] >= 0 ? fmaf(w[kk], v[kk][j], acc[j]) : acc[j];
         }
-        c = c_next;
-        row = row_next;
-        row_next = row_after;
+    } else {
+        int row = row_of(c), row_next = row_of(min(next_of(c), pos));      // (places are looked up two chunks ahead of their rows)
+        ask(row);
+        while (c <= pos) {
+            float s = 0.f;
+#pragma unroll
+            for (int i = 0; i < HD / 4; ++i) {
+                const float4 qv = *reinterpret_cast<const float4*>(&qr[4 * i]);
+                s = fmaf(qv.x, key[i].x, s);
+                s = fmaf(qv.y, key[i].y, s);
+                s = fmaf(qv.z, key[i].z, s);
+                s = fmaf(qv.w, key[i].w, s);
+            }
+            s *= scale;
+            if (rule.softcap > 0.f) s = rule.softcap * tanhf(s / rule.softcap);
+            if (row < 0) s = -INFINITY;
+            const int c_next = next_of(c);
+            ask(row_next);
+            const int row_after = row_of(min(next_of(c_next), pos));       // (past the end: nobody looks at it)
+            const float m_new = fmaxf(m, wave_max(s));
+            const float pe = row >= 0 ? expf(s - m_new) : 0.f;
+            const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
+            l = fmaf(l, corr, wave_sum(pe));
+            m = m_new;
+            const int n_keys = min(WAVE, pos - c + 1);
+#pragma unroll
+            for (int j = 0; j < DPL; ++j) acc[j] *= corr;
+            for (int k0 = 0; k0 < n_keys; k0 += AHEAD) {
+                float v[AHEAD][DPL], w[AHEAD];
+                int at[AHEAD];
+#pragma unroll
+                for (int kk = 0; kk < AHEAD; ++kk) {
+                    at[kk] = __builtin_amdgcn_readlane(row, k0 + kk);
+                    w[kk] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pe), k0 + kk));
+#pragma unroll
+                    for (int j = 0; j < DPL; ++j) v[kk][j] = v_cache[(size_t)max(at[kk], 0) * HD + lane + j * WAVE];
+                }
+#pragma unroll
+                for (int kk = 0; kk < AHEAD; ++kk)
+#pragma unroll
+                    for (int j = 0; j < DPL; ++j) acc[j] = at[kk] >= 0 ? fmaf(w[kk], v[kk][j], acc[j]) : acc[j];
+            }
+            c = c_next;
+            row = row_next;
+            row_next = row_after;
+        }
     }
     float inv = l > 0.f ? 1.0f / l : 0.f;
     if (rule.sink) {                        // one more term of the denominator, without a key or a value
@@ -294,14 +332,24 @@ static int attention_wave(const void* q, const void* k_cache, const void* v_cach
     // heads of 64 or 128 whose values lie as the keys do, rows 16 bytes aligned and counted in 32 bits
     const bool plain = dtype == IMPARO_F32 && head_dim == value_dim && v_ld == head_dim && !v_transposed &&
                        !((uintptr_t)k_cache & 15) && (long long)n_pages * kv_heads * page_size < (1LL << 31);
-#define WAVE_F32_GO(HD)                                                                                                 \
-    k_attention_wave_f32<HD><<<blocks, ATT_WAVES * WAVE, 0, s>>>(                                                       \
+#define WAVE_F32_GO(HD, ONE)                                                                                            \
+    k_attention_wave_f32<HD, ONE><<<blocks, ATT_WAVES * WAVE, 0, s>>>(                                                  \
         (const float*)q, (const float*)k_cache, (const float*)v_cache, (float*)out, positions, row_of_token, block_table, \
         table_stride, page_size, n_tokens, heads, kv_heads, out_ld, n_pages, scale, window, r)
-    if (plain && head_dim == 64)
-        WAVE_F32_GO(64);
-    else if (plain && head_dim == 128)
-        WAVE_F32_GO(128);
+    // One chunk where the table has no room for more keys. Otherwise, where the waves are many and not bound by their trips, the
+    // general kernel: for windows of less than a chunk (1,000 tokens, 64 heads of 64, 20 keys: 222 us in the loop, 206 there),
+    // and with heads of 128, whose registers leave a SIMD one wave where it has four, for any window (64 heads, 128 keys: 1,292
+    // and 1,146) and short contexts (4 prompts of 100 tokens, 64 heads 251 and 216; one of 333 537 and 554).
+    const long long room = (long long)table_stride * page_size;
+    const bool one = room <= WAVE, few = total <= 4096;
+    if (plain && head_dim == 64 && one)
+        WAVE_F32_GO(64, true);
+    else if (plain && head_dim == 64 && (few || window <= 0 || window >= WAVE))
+        WAVE_F32_GO(64, false);
+    else if (plain && head_dim == 128 && one)
+        WAVE_F32_GO(128, true);
+    else if (plain && head_dim == 128 && (few || (window <= 0 && room >= 320)))
+        WAVE_F32_GO(128, false);
 #undef WAVE_F32_GO
     else if (dtype == IMPARO_F32)
         k_attention_wave<float><<<blocks, ATT_WAVES * WAVE, 0, s>>>(

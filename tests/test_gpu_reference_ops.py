@@ -167,11 +167,13 @@ def test_picks(vocab):
     assert vocab > 1000 or same >= n - 4
 
 
-@pytest.mark.parametrize("H,Hk,D,page_size,window", [(4, 2, 64, 16, None), (3, 1, 64, 8, 67), (2, 2, 128, 64, None), (4, 1, 128, 5, 130)])
-def test_float32_attention_sums_alike_whether_the_head_size_is_known_or_not(H, Hk, D, page_size, window):
-    """Heads of 64 and 128 have a kernel of their own; values transposed in their pages go through the general one.
-    Both walk the same chunks in the same order: the same bits, at contexts beside whole chunks of 64 keys."""
-    lens = dict(ctx_lens=(64, 65, 1, 200, 129), q_lens=(3, 65, 1, 2, 1))
+@pytest.mark.parametrize("H,Hk,D,page_size,window", [(4, 2, 64, 16, None), (3, 1, 64, 8, 67), (2, 2, 128, 64, None), (4, 1, 128, 5, 130), (2, 1, 64, 16, 20), (2, 1, 128, 16, 20)])
+@pytest.mark.parametrize("ctx_lens,q_lens", [((64, 65, 1, 200, 129), (3, 65, 1, 2, 1)), ((64, 1, 9, 33, 60, 48), (64, 1, 9, 2, 1, 48))])
+def test_float32_attention_sums_alike_whether_the_head_size_is_known_or_not(H, Hk, D, page_size, window, ctx_lens, q_lens):
+    """Heads of 64 and 128 have a kernel of their own, in one form for block tables of one chunk of 64 keys and one for
+    longer ones; values transposed in their pages go through the general one. All walk the same chunks in the same order: the
+    same bits, at contexts beside whole chunks."""
+    lens = dict(ctx_lens=ctx_lens, q_lens=q_lens)
     got, ref = _attention_case(H, Hk, D, page_size, window, torch.float32, v_transposed=False, **lens)
     general, _ = _attention_case(H, Hk, D, page_size, window, torch.float32, v_transposed=True, **lens)
     assert torch.equal(got, general)
