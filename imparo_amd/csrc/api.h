@@ -660,7 +660,8 @@ int imparo_qk_row_norm_rope_store(const float* qkv, int row_ld, const float* q_w
                                   int n_pages, int v_transposed, imparo_stream stream);
 // plan: entries are (token, choice) pairs in row-major order; those whose expert is below n_experts get a slot,
 // an expert's slots side by side (slot_of_entry, -1 for the others; entry_of_slot), and `tiles` [max_tiles, 3]
-// lists (expert, first slot, rows <= tile_rows) of every tile of rows, expert -1 past the list's end.
+// lists (expert, first slot, rows <= tile_rows) of every tile of rows; past the list's end come empty tiles (-1, how many tiles
+// hold rows, -1).
 int imparo_moe_tile_rows(int n_entries, int n_experts, int dtype);
 int imparo_moe_max_tiles(int n_entries, int n_experts, int tile_rows);
 int imparo_moe_plan(const int32_t* choice, int n_entries, int n_experts, int tile_rows,
@@ -668,7 +669,8 @@ int imparo_moe_plan(const int32_t* choice, int n_entries, int n_experts, int til
                     imparo_stream stream);
 // product: out[slot, :n] = epilogue(a[row(slot), :k] . w[expert(slot), :n, :k]); row(slot) is the slot, or with
 // gather_div > 0 entry_of_slot[slot] / gather_div. epilogue 0: none, 1: max(z, 0)^2. bfloat16 operands (k a
-// multiple of 8, out bfloat16 or float32; tile_rows 16, 64 or 128) or float32 throughout (tile_rows 64).
+// multiple of 8, out bfloat16 or float32; tile_rows 16, 64 or 128) or float32 throughout (tile_rows 64). A list may end in
+// empty tiles as the plan writes them, of which the last one's count is believed, in tiles of expert -1 with other numbers, or in none.
 // epilogue 2 (bfloat16 operands and out, n a multiple of 64): an expert's rows are 32 gate rows, the 32 up rows that
 // belong to them, and so on; out [slots, n / 2] = act(w g, w u) as in imparo_moe_gated, with limits [experts] (null:
 // SiLU) and w = entry_weight[entry_of_slot[slot]] (null: 1).

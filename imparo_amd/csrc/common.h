@@ -45,6 +45,7 @@ template <> __device__ __forceinline__ void store_f32<bf16_t>(bf16_t* p, size_t 
 // Sums and maxima over a wave, the same in every lane: lanes 32 apart first, then 16, 8, 4, 2, 1. On lane swaps and
 // moves inside rows of 16, which take a few cycles where a shuffle through LDS takes about a hundred: after a step all
 // lanes that far apart agree, so "rotated by n" stands for "n apart" (and a sum of two is the same either way round).
+// All 64 lanes must be active: no call where lanes have left or taken another branch.
 #define WAVE_STEPS(v, OP)                                                                                              \
     do {                                                                                                               \
         auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);          \
@@ -73,6 +74,9 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Sum over a block of up to 1024 threads in whole waves; every thread gets the result.
+// `scratch` holds at least 16 floats of LDS. The order of the additions
+// depends only on the block size, never on the data.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     v = wave_sum(v);
     const int lane = threadIdx.x & (WAVE - 1);

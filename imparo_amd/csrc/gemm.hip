@@ -200,8 +200,9 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
 // and walks K alone, operands from memory straight into registers, 16 bytes a lane: lane (row, g) asks for
 // k = 4g .. 4g + 3 of 16, and a transposition over the four groups of lanes (four lane swaps) gives it
 // k = g, 4 + g, 8 + g, 12 + g, which is how the products want them. Loads run seven chunks of 32 ahead in eight
-// register sets. A weight of many rows is bound by its bytes, one of few rows by the chain of a wave's products (each
-// waits for the one before it). Measured, cold weights, 2 rows: 65,536 by 1,024 57 us (4.7 TB/s), 9,216 by 1,024 14 us,
+// register sets. A weight of many rows is bound by its bytes. One of few rows leaves most CUs idle and is
+// bound by one wave's walk: products that each wait for the one before them, 32 cycles for 4 k (16 us for K = 4,608), and
+// about as much again for the lane swaps and waits between them. Measured, cold weights, 2 rows: 65,536 by 1,024 57 us (4.7 TB/s), 9,216 by 1,024 14 us,
 // 1,024 by 4,608 33 us; 17 us on average over a decode step where two weight rows a thread through LDS took 79. The loads ask
 // for 4-byte alignment only, so a K that is no multiple of 4 and operands that start anywhere come this way too: 2 rows of 1,024 by
 // 1,026 9.9 us, 65,536 by 1,022 44 (value by value in tiles of 64 rows 50 and 144, the kernel before both 45 and 111).

@@ -261,7 +261,8 @@ extern "C" int imparo_moe_route(const float* logits, const float* correction, in
 }
 
 // ---------------------------------------------------------------- plan
-// tiles[3 i ..]: expert, first slot, rows of tile i; expert -1 where the list has ended.
+// tiles[3 i ..]: expert, first slot, rows of tile i; where the list has ended expert -1, the number of tiles that hold rows,
+// MOE_COUNTED (k_moe_gemm_dma deals the tiles to the XCDs by that number).
 struct MoePlanShared {
     int count[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], first_tile[MOE_MAX_EXPERTS + 1];
 };

@@ -93,7 +93,7 @@ extern "C" int imparo_argmax_rows(const float* logits, int32_t* out, int n_rows,
 // The sums' order is part of the result (two machines that draw the same number pick the same token), so the scan
 // over the pieces and the walk inside one stay chains of additions; what a chain adds is fetched ahead of it, sixteen
 // values a time, and all that is no addition (exponentials, comparisons) is done by the whole block. Measured, 64
-// rows of 65,536 logits: 150 us with both chains reading LDS and memory value by value, 38 us so (28 us for rows of 16,384).
+// rows of 65,536 logits: 153 us with both chains reading LDS and memory value by value, 38 us so (28 us for rows of 16,384).
 #define SAMPLE_THREADS 1024
 __global__ __launch_bounds__(SAMPLE_THREADS) void k_sample_rows(
     const float* __restrict__ logits, const float* __restrict__ temperature, const float* __restrict__ uniform,

@@ -967,6 +967,32 @@ def test_sample_rows_at_the_edges_of_its_pieces(vocab):
         assert (float(cdf[got - 1]) if got else 0.0) - 2e-4 <= float(u[r]) <= float(cdf[got]) + 2e-4
 
 
+@pytest.mark.parametrize("vocab", [255, 4096, 50257, 65536, 128256, 1200000])
+@pytest.mark.parametrize("gaps", ["none", "every other", "first half", "ends"])
+def test_sample_rows_counts_equal_logits_exactly(vocab, gaps):
+    """Equal logits have exponentials of exactly one and sums that are whole numbers below 2^24, so a uniform number names one
+    token: around the edges of pieces (a thread's share of the row, 256 or 1,024 of them), of 16 values and of 1,024, first and
+    last; tokens without weight (minus infinity, NaN) between them are passed over."""
+    x = torch.zeros(vocab)
+    if gaps == "every other":
+        x[::2] = float("-inf")
+    elif gaps == "first half":
+        x[:vocab // 2] = float("nan")
+    elif gaps == "ends":
+        x[:3], x[-vocab // 3:] = float("-inf"), float("nan")
+    live = torch.nonzero(x == 0).flatten().tolist()
+    n, threads = len(live), 1024 if vocab >= 16384 else 256
+    piece = -(-vocab // threads)
+    edges = {p + d for p in (0, 16, 1024, piece, 2 * piece, 16 * piece, 17 * piece, 5 * 1024, threads // 2 * piece, n - 16, n) for d in (-1, 0, 1)}
+    edges = sorted(e for e in edges if 0 <= e < n)
+    u = np.array([(e + 0.5) / n for e in edges] + [0.0, 0.99999994], dtype=np.float32)
+    target = u * np.float32(n)
+    want = [live[min(int(math.floor(t)), n - 1)] for t in target.tolist()]
+    out = torch.full((len(u),), -7, dtype=torch.int32, device=DEV)
+    ops().sample_rows(x.repeat(len(u), 1).to(DEV), torch.ones(len(u), device=DEV), torch.from_numpy(u).to(DEV), out)
+    assert out.cpu().tolist() == want and want[-1] == live[-1]
+
+
 # ---------------------------------------------------------------- products with a folded norm (at most 16 rows)
 from imparo_amd.kernels import ops as _rows_ops
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (5, 200, 136), (13, 1536, 1536), (16, 2048, 8192), (8, 96, 320),
