@@ -267,10 +267,20 @@ extern "C" int imparo_stream_norm(const float* x, int in_streams, float* x_out, 
     const int per = (pieces + threads - 1) / threads;
     const int out_is_bf16 = out_dtype == IMPARO_BF16;
     // Once there are several rounds of blocks, how many of them a CU holds is what counts, and what is asked for early takes
-    // registers, of more copies more: 2,048 rows of 2,048, early | late: 18.4 | 17.4 us by 2 copies, 36.6 | 33.4 by 5, 59 | 54 by
-    // 8; 8,192 rows of 1,024 by 4 60 | 56; 1,023 rows of 2,048 by 4 still 14.3 | 16.1, of 1,280 by 8 18.6 | 17.5. With experts' rows
-    // early is the faster way at any count (2,048 rows of 2,048 by 8 copies 74 | 86).
-    const bool late = !y && per <= 1 && (long long)n_out * threads >= (streams > 4 ? 1 << 18 : 600000);
+    // registers, of more copies more. Late where that costs more than the wait for memory: without a norm to wait for; and of
+    // several copies, while blocks have at most 512 threads (of 1,024 a CU holds two either way) and few slices of a
+    // pending result, which late are asked for one trip later than the row. us early | late, layer norm unless said, 2,048 rows of 2,048:
+    // one slice by 2 copies 18.8 | 17.4, by 5 37.5 | 33.3, by 8 56.6 | 52.1; by one copy 13.2 | 13.8; four slices by 4 31.6 | 34.7, by 8
+    // 68.6 | 72.9, two by 4 27.9 | 29.4, by 5 39.0 | 36.0; no norm, by 4 26.6 | 25.0. Rows of 4,096, two slices by 4 copies, 1,200 rows: 33.0 | 35.0,
+    // but 8,192 rows, one slice by 2 copies 145 | 138. From few rows on by many copies (600 of 2,048 by 5 14.5 | 13.8, by 4 with 1,200
+    // rows still 17.1 | 17.6, without a norm 600 9.0 | 9.6), two slices of few copies from more rows on (8,192 of 1,024 by 2 36.3 |
+    // 34.7). With experts' rows early is the faster way at any count (2,048 rows of 2,048 by 8 copies 74 | 86).
+    const long long at_work = (long long)n_out * threads;
+    const bool late = !y && per <= 1 &&
+                      (norm == STREAM_NORM_NONE ? at_work >= (streams == 3 || streams == 4 ? 600000 : 1 << 18)
+                                                : at_work >= (streams > 4 ? 1 << 18 : 1 << 20) && streams > 1 &&
+                                                      n_delta <= (streams > 4 || at_work >= 1 << 21 ? 2 : 1) &&
+                                                      (threads <= 512 || (streams == 2 && n_delta == 1)));
 #define STREAM_NORM(S, V, PER)                                                                                       \
     k_stream_norm<S, V, PER, (PER == 1)><<<n_out, threads, 0, s>>>(x, in_streams, x_out, delta, n_delta, stride, moe, rows, streams, \
                                                        mix, join, read, norm, weight, bias, eps, out, out_is_bf16, width)

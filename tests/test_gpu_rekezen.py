@@ -408,9 +408,10 @@ def test_weights_over_the_chosen_outputs(X, top, T):
         assert sorted(s1.cpu().tolist()) == list(range(n)) and bool((choice.cpu()[s2.cpu().long() // (top + 1), top] == X).all())
 
 
-@pytest.mark.parametrize("S,E,T", [(1, 2048, 1200), (2, 1028, 2001), (4, 1024, 2500), (8, 2048, 520)])
-@pytest.mark.parametrize("n_delta", [1, 3])
-def test_streams_of_many_rows_are_those_of_few(S, E, T, n_delta):
+@pytest.mark.parametrize("S,E,T", [(1, 2048, 1200), (2, 1028, 2001), (4, 1024, 2500), (8, 2048, 520), (2, 1028, 3500), (4, 1024, 4200), (2, 256, 33000)])
+@pytest.mark.parametrize("n_delta", [1, 2, 3])
+@pytest.mark.parametrize("norm", ["layer", "none"])
+def test_streams_of_many_rows_are_those_of_few(S, E, T, n_delta, norm):
     """From some rows on a block asks for a row where it uses it, and not ahead: the same bits as in thirds of the rows, the copies
     that are written back and the normed rows."""
     from imparo_amd.kernels import ops
@@ -420,7 +421,8 @@ def test_streams_of_many_rows_are_those_of_few(S, E, T, n_delta):
 
     def run(lo, hi):
         x_out, out = torch.empty(hi - lo, S, E, device=DEV), torch.empty(hi - lo, E, device=DEV)
-        ops.stream_norm(x[lo:hi], "layer", w, b, 1e-5, out, delta=delta[:, lo:hi].contiguous(), mix=mix, join=join, read=read, x_out=x_out)
+        weights = (w, b) if norm != "none" else (None, None)
+        ops.stream_norm(x[lo:hi], norm, *weights, 1e-5, out, delta=delta[:, lo:hi].contiguous(), mix=mix, join=join, read=read, x_out=x_out)
         return x_out, out
 
     many, thirds = run(0, T), [run(T * i // 3, T * (i + 1) // 3) for i in range(3)]
