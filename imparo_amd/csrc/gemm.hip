@@ -3,9 +3,8 @@
 // float32: kernels on the matrix cores' float32 products; every output element sums
 // its products in the order k = 0, 1, 2, ... whatever the tile it falls in, so a row's
 // result does not depend on how many other rows are in the batch.
-// bfloat16: MFMA kernels, a 128x128 LDS-tiled one for many rows and a
-// weight-streaming one with the K range split over the waves of a block for
-// few rows (decode).
+// bfloat16: MFMA kernels, LDS-tiled ones for many rows and weight-streaming ones for some
+// (at most 16 rows: decode_rows.hip).
 #include "common.h"
 
 #include <algorithm>
@@ -20,38 +19,6 @@ union Frag8 {
     uint4 u;
     bf16x8 v;
 };
-
-#define EPI_NONE 0
-#define EPI_SWIGLU 1   // weight rows interleaved gate, up, gate, up...: out[m, j] = act(y[m, 2j], y[m, 2j+1])
-#define EPI_ADD 2      // float32 out only: Y += y, what Y holds being read where the result is stored
-
-// What happens to a product before it is stored: its kind (one of the above) and, for the gated kind, a constant
-// the result is multiplied by in float32 before it is rounded (a factor on the whole sublayer, carried by the input
-// of the product that follows), and the bound of a unit that has one: act(g, u) = silu(g) u with limit 0, else
-// g' sigmoid(alpha g') (u' + 1) with g' = min(g, limit), u' = clamp(u, -limit, limit).
-struct Epilogue {
-    int kind;
-    float scale, limit, alpha;
-    __host__ __device__ Epilogue(int k, float s = 1.0f, float l = 0.0f, float a = 1.0f) : kind(k), scale(s), limit(l), alpha(a) {}
-    __host__ __device__ operator int() const { return kind; }
-};
-
-__device__ __forceinline__ void gated_bounds(const Epilogue& e, float& g, float& u) {
-    if (e.limit > 0.f) {
-        g = fminf(g, e.limit);
-        u = fminf(fmaxf(u, -e.limit), e.limit) + 1.0f;
-    }
-}
-__device__ __forceinline__ float gated_mul(const Epilogue& e, float g, float u) {
-    gated_bounds(e, g, u);
-    return g / (1.0f + expf(-e.alpha * g)) * u * e.scale;
-}
-// The same with the hardware's exp2 and reciprocal (an ulp each) for the bfloat16 kernels: the exact
-// division and exponential cost some thirty instructions per output, ten microseconds per 256x256 tile
-__device__ __forceinline__ float gated_mul_fast(const Epilogue& e, float g, float u) {
-    gated_bounds(e, g, u);
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.44269504f * e.alpha * g)) * u * e.scale;
-}
 
 __device__ __forceinline__ uint4 zero_if(bool out, uint4 v) {
     return make_uint4(out ? 0u : v.x, out ? 0u : v.y, out ? 0u : v.z, out ? 0u : v.w);
@@ -1093,7 +1060,7 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
     return launch_status();
 }
 
-// ------------------------------------------------------------------ bfloat16, few rows
+// ------------------------------------------------------------------ bfloat16, some rows (17..64), K split over waves
 // One block per 16 weight rows. Its NW waves split K in chunks of 128: wave w
 // takes chunks w, w + NW, ... so the block reads each weight row as one
 // contiguous stream. The 16 weight rows are the MFMA's M side, up to 16*MT
@@ -1221,108 +1188,130 @@ static void launch_skinny(const bf16_t* x, const bf16_t* w, const float* bias, T
 // For a decode step's rows (one token each, at most 16): the projection to [B | C | x] and the
 // gated short convolution that consumes it in one launch. A block takes 8 channels: its first
 // MFMA tile holds the B rows of those channels (tile rows 0..7) and their x rows (8..15), its
-// second the C rows (0..7, and again in 8..15: the same cache lines, nothing more to fetch).
-// K is split over the waves as in the kernel above and the partial sums meet in LDS in wave
+// second the C rows (0..7; its other lanes ask for nothing).
+// K is split over the waves in chunks of 128, all of whose loads go out at once (CH chunks a wave and
+// round, as the products of decode_rows.hip have them), and the partial sums meet in LDS in wave
 // order; then 32 lanes of wave 0 each own one token and four channels: u = B * x, the taps
 // oldest first exactly as the conv kernels sum them, the C gate, and the shift of the state
 // (a lane owns its channels' history, so nothing races). With HIST > 0 the history, the taps
-// and the biases are asked for before the walk along K, so they are there when it ends.
+// and the biases are asked for before the walk along K, so they are there when it ends. Measured: 8 rows
+// of 2,048 9.3 -> 8.5 us, one row of 1,024 6.2 -> 5.4 (a chunk ahead of the one that is multiplied before).
 // With ssq_in, X is the residual stream times a norm's weight, not yet scaled: the partial sums of
 // squares of its rows [n_parts, 16] give each row's scale, which multiplies B, C and x at the end (rows.h).
-template <typename TOut, int NW, int HIST>
-__global__ __launch_bounds__(NW * 64) void k_in_proj_conv_decode(
+template <typename TOut, int CH, int HIST>
+__global__ __launch_bounds__(512) void k_in_proj_conv_decode(
     const bf16_t* __restrict__ X, const float* __restrict__ ssq_in, int n_parts, float eps,
     const bf16_t* __restrict__ W, const float* __restrict__ in_bias,
     const float* __restrict__ conv_w, const float* __restrict__ conv_b, float* __restrict__ state,
     const int32_t* __restrict__ slot, TOut* __restrict__ out, int M, int E, int K, int taps) {
-    __shared__ float red[NW][2][64][4];
-    __shared__ float norm_part[NW * 4 * 16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ float4 red[8][2][64];
+    __shared__ __attribute__((aligned(16))) float norm_part[8 * 16];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int r16 = lane & 15, g = lane >> 4;
     const int c0 = blockIdx.x * 8;
-    const bf16_t* wrow0 = W + (size_t)(r16 < 8 ? c0 + r16 : 2 * E + c0 + (r16 - 8)) * K + g * 8;
-    const bf16_t* wrow1 = W + (size_t)(E + c0 + (r16 & 7)) * K + g * 8;
-    const bf16_t* xrow = X + (size_t)min(r16, M - 1) * K + g * 8;
+    const bf16_t* wrow0 = W + (size_t)(r16 < 8 ? c0 + r16 : 2 * E + c0 + (r16 - 8)) * K;
+    const bf16_t* wrow1 = W + (size_t)(E + c0 + (r16 & 7)) * K;
+    const bf16_t* xrow = X + (size_t)min(r16, M - 1) * K;
+    const int n_chunks = (K + 127) / 128;
     const int history = HIST > 0 ? HIST : taps - 1;
-    // the lanes that finish the block: token r16, channels cb .. cb+3
+    // the lanes that finish the block: token r16, channels cb .. cb+3. Where a token's state lies is asked for before all
+    // else and its state after the weights: who waits for the one to ask for the other waits with the weights on their way.
     const bool finisher = wave == 0 && g < 2 && r16 < M;
     const int cb = c0 + 4 * (g & 1);
-    float* st = state + (size_t)(finisher ? slot[r16] : 0) * history * E;
+    const int my_slot = finisher ? slot[r16] : 0;
+    __builtin_amdgcn_sched_barrier(0);
+    Frag8 w0[CH][4], w1[CH][4], x[CH][4];
+    auto ask = [&](int first) __attribute__((always_inline)) {
+        int k[CH][4];
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2) k[j][s2] = min(min(first + j * waves, n_chunks - 1) * 128 + s2 * 32 + g * 8, K - 8);
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2) x[j][s2].u = *reinterpret_cast<const uint4*>(xrow + k[j][s2]);
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2) {
+                w0[j][s2].u = *reinterpret_cast<const uint4*>(wrow0 + k[j][s2]);
+                w1[j][s2].u = make_uint4(0u, 0u, 0u, 0u);
+                if (r16 < 8) w1[j][s2].u = *reinterpret_cast<const uint4*>(wrow1 + k[j][s2]);
+            }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // (the rows' sums of squares before the weights: they are added up while those are on their way)
+    RowsSsq early;
+    if (ssq_in) rows_ssq_ask(early, ssq_in, n_parts, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    ask(wave);
+    if (ssq_in) rows_ssq_share(norm_part, early, ssq_in, n_parts);
+    float* st = state + (size_t)my_slot * history * E;
     constexpr int HN = HIST > 0 ? HIST : 1;
     float hist[HN][4], tap[HN + 1][4], bias_b[4], bias_c[4], bias_x[4], bias_conv[4];
     if (HIST > 0 && finisher) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
 #pragma unroll
-            for (int k = 0; k < HIST; ++k) hist[k][i] = st[(size_t)k * E + cb + i];
-#pragma unroll
             for (int k = 0; k <= HIST; ++k) tap[k][i] = conv_w[(size_t)(cb + i) * (HIST + 1) + k];
             bias_b[i] = in_bias ? in_bias[cb + i] : 0.f;
             bias_c[i] = in_bias ? in_bias[E + cb + i] : 0.f;
             bias_x[i] = in_bias ? in_bias[2 * E + cb + i] : 0.f;
             bias_conv[i] = conv_b ? conv_b[cb + i] : 0.f;
+#pragma unroll
+            for (int k = 0; k < HIST; ++k) hist[k][i] = st[(size_t)k * E + cb + i];
         }
     }
-    struct Frags {
-        Frag8 w0[4], w1[4], x[4];
-    };
     f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    auto load = [&](int k0, Frags& f) {
+    for (int first = wave; first < n_chunks;) {
 #pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2) {
-            const int k = k0 + s2 * 32;
-            const bool in = k + g * 8 < K;
-            f.w0[s2].u = in ? *reinterpret_cast<const uint4*>(wrow0 + k) : make_uint4(0, 0, 0, 0);
-            f.w1[s2].u = in ? *reinterpret_cast<const uint4*>(wrow1 + k) : make_uint4(0, 0, 0, 0);
-            f.x[s2].u = in ? *reinterpret_cast<const uint4*>(xrow + k) : make_uint4(0, 0, 0, 0);
+        for (int j = 0; j < CH; ++j) {
+            if (first + j * waves >= n_chunks) continue;
+#pragma unroll
+            for (int s2 = 0; s2 < 4; ++s2) {             // (weights beyond K count as zeros)
+                const bool beyond = (first + j * waves) * 128 + s2 * 32 + g * 8 >= K;
+                w0[j][s2].u = zero_if(beyond, w0[j][s2].u);
+                w1[j][s2].u = zero_if(beyond, w1[j][s2].u);
+                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[j][s2].v, x[j][s2].v, acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1[j][s2].v, x[j][s2].v, acc1, 0, 0, 0);
+            }
         }
-    };
-    auto multiply = [&](const Frags& f) {
-#pragma unroll
-        for (int s2 = 0; s2 < 4; ++s2) {
-            acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w0[s2].v, f.x[s2].v, acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w1[s2].v, f.x[s2].v, acc1, 0, 0, 0);
-        }
-    };
-    Frags cur, nxt;
-    int k0 = wave * 128;
-    if (k0 < K) load(k0, cur);
-    // the row's scale multiplies the sums at the end: its sums of squares are asked for now
-    RowsSsq early;
-    if (ssq_in) rows_ssq_ask(early, ssq_in, n_parts, 0);
-    while (k0 < K) {
-        const int k1 = k0 + NW * 128;
-        if (k1 < K) load(k1, nxt);
-        multiply(cur);
-        cur = nxt;
-        k0 = k1;
+        first += waves * CH;
+        if (first < n_chunks) ask(first);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        red[wave][0][lane][i] = acc0[i];
-        red[wave][1][lane][i] = acc1[i];
-    }
-    if (ssq_in) norm_part[(threadIdx.x >> 4) * 16 + (threadIdx.x & 15)] = rows_ssq_sum(early, ssq_in, n_parts);
+    red[wave][0][lane] = make_float4(acc0[0], acc0[1], acc0[2], acc0[3]);
+    red[wave][1][lane] = make_float4(acc1[0], acc1[1], acc1[2], acc1[3]);
     __syncthreads();
     if (!finisher) return;
     const float scale = ssq_in ? rows_scale(norm_part, r16, K, eps) : 1.f;
     // D layout: lane holds column lane%16 (a token), tile rows 4*(lane/16) + i: B and C of channel
     // cb + i sit in this lane's entries, x of the same channel 8 tile rows further: lane + 32
-    float b[4], c[4], x[4];
+    float b[4], c[4], xc[4];
+    {
+        float4 sb[8], sx[8], sc[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        b[i] = red[0][0][lane][i];
-        x[i] = red[0][0][lane + 32][i];
-        c[i] = red[0][1][lane][i];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            b[i] += red[w][0][lane][i];
-            x[i] += red[w][0][lane + 32][i];
-            c[i] += red[w][1][lane][i];
+        for (int q = 0; q < 8; ++q) {
+            const int w = min(q, waves - 1);
+            sb[q] = red[w][0][lane], sx[q] = red[w][0][lane + 32], sc[q] = red[w][1][lane];
         }
-        if (ssq_in) {
+        float4 tb = sb[0], tx = sx[0], tc = sc[0];
+#pragma unroll
+        for (int q = 1; q < 8; ++q)
+            if (q < waves) {
+                tb.x += sb[q].x, tb.y += sb[q].y, tb.z += sb[q].z, tb.w += sb[q].w;
+                tx.x += sx[q].x, tx.y += sx[q].y, tx.z += sx[q].z, tx.w += sx[q].w;
+                tc.x += sc[q].x, tc.y += sc[q].y, tc.z += sc[q].z, tc.w += sc[q].w;
+            }
+        b[0] = tb.x, b[1] = tb.y, b[2] = tb.z, b[3] = tb.w;
+        xc[0] = tx.x, xc[1] = tx.y, xc[2] = tx.z, xc[3] = tx.w;
+        c[0] = tc.x, c[1] = tc.y, c[2] = tc.z, c[3] = tc.w;
+    }
+    if (ssq_in) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
             b[i] = __fmul_rn(b[i], scale);
-            x[i] = __fmul_rn(x[i], scale);
+            xc[i] = __fmul_rn(xc[i], scale);
             c[i] = __fmul_rn(c[i], scale);
         }
     }
@@ -1330,7 +1319,7 @@ __global__ __launch_bounds__(NW * 64) void k_in_proj_conv_decode(
     if (HIST > 0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float u = (b[i] + bias_b[i]) * (x[i] + bias_x[i]);
+            const float u = (b[i] + bias_b[i]) * (xc[i] + bias_x[i]);
             float a = 0.f;
 #pragma unroll
             for (int k = 0; k < HIST; ++k) {
@@ -1346,7 +1335,7 @@ __global__ __launch_bounds__(NW * 64) void k_in_proj_conv_decode(
             const int ch = cb + i;
             const float bv = b[i] + (in_bias ? in_bias[ch] : 0.f);
             const float cv = c[i] + (in_bias ? in_bias[E + ch] : 0.f);
-            const float xv = x[i] + (in_bias ? in_bias[2 * E + ch] : 0.f);
+            const float xv = xc[i] + (in_bias ? in_bias[2 * E + ch] : 0.f);
             const float u = bv * xv;
             float a = 0.f;
             float prev = st[ch];                                  // oldest
@@ -1365,20 +1354,28 @@ __global__ __launch_bounds__(NW * 64) void k_in_proj_conv_decode(
     for (int i = 0; i < 4; ++i) store_f32<TOut>(out, (size_t)r16 * E + cb + i, y[i]);
 }
 
-template <typename TOut, int NW>
+template <typename TOut>
 static void launch_in_proj_conv(const bf16_t* x, const float* ssq_in, int n_parts, float eps, const bf16_t* w,
                                 const float* in_bias, const float* conv_w, const float* conv_b, float* state,
                                 const int32_t* slot, TOut* out, int m, int e, int k, int taps, hipStream_t s) {
     const unsigned blocks = (unsigned)(e / 8);
-#define CONV_GO(HIST)                                                                                              \
-    k_in_proj_conv_decode<TOut, NW, HIST><<<blocks, NW * 64, 0, s>>>(x, ssq_in, n_parts, eps, w, in_bias, conv_w, conv_b, \
+    const int chunks = (k + 127) / 128;                 // as many waves as there are chunks, or pairs of chunks
+    const int waves = chunks <= 8 ? chunks : std::min(8, (chunks + 1) / 2);
+#define CONV_GO(CH, HIST)                                                                                              \
+    k_in_proj_conv_decode<TOut, CH, HIST><<<blocks, waves * 64, 0, s>>>(x, ssq_in, n_parts, eps, w, in_bias, conv_w, conv_b, \
                                                                    state, slot, out, m, e, k, taps)
-    switch (taps - 1) {
-        case 1: CONV_GO(1); break;
-        case 2: CONV_GO(2); break;
-        case 3: CONV_GO(3); break;
-        default: CONV_GO(0);
-    }
+#define CONV_HIST(CH)                                                                                                  \
+    do {                                                                                                             \
+        switch (taps - 1) {                                                                                          \
+            case 1: CONV_GO(CH, 1); break;                                                                             \
+            case 2: CONV_GO(CH, 2); break;                                                                             \
+            case 3: CONV_GO(CH, 3); break;                                                                             \
+            default: CONV_GO(CH, 0);                                                                                   \
+        }                                                                                                            \
+    } while (0)
+    if (chunks <= 8) CONV_HIST(1);
+    else CONV_HIST(2);
+#undef CONV_HIST
 #undef CONV_GO
 }
 
@@ -1401,18 +1398,10 @@ extern "C" int imparo_in_proj_conv_decode_normed(const void* x, const float* ssq
     hipStream_t s = (hipStream_t)stream;
     const bf16_t* xb = (const bf16_t*)x;
     const bf16_t* wb = (const bf16_t*)w;
-    // waves over K as the K-split kernel has them: chunks of 128, few per wave
-#define CONV_CALL(TOut, NW)                                                                                          \
-    launch_in_proj_conv<TOut, NW>(xb, ssq_in, n_parts, eps, wb, in_bias, conv_w, conv_b, state, slot, (TOut*)out, m, e, \
-                                  k, taps, s)
-    if (out_dtype == IMPARO_F32) {
-        if (k <= 512) CONV_CALL(float, 4);
-        else CONV_CALL(float, 8);
-    } else {
-        if (k <= 512) CONV_CALL(bf16_t, 4);
-        else CONV_CALL(bf16_t, 8);
-    }
-#undef CONV_CALL
+    if (out_dtype == IMPARO_F32)
+        launch_in_proj_conv<float>(xb, ssq_in, n_parts, eps, wb, in_bias, conv_w, conv_b, state, slot, (float*)out, m, e, k, taps, s);
+    else
+        launch_in_proj_conv<bf16_t>(xb, ssq_in, n_parts, eps, wb, in_bias, conv_w, conv_b, state, slot, (bf16_t*)out, m, e, k, taps, s);
     return launch_status();
 }
 
@@ -1425,7 +1414,7 @@ extern "C" int imparo_in_proj_conv_decode(const void* x, const void* w, const fl
 }
 
 
-// Which kernel takes a product of up to 64 rows: 0 for the K-split kernel, else the waves per
+// Which kernel takes a product of 17 to 64 rows: 0 for the K-split kernel, else the waves per
 // block of the shared-activation kernel. Measured with cold weights (they never stay in cache
 // between decode steps): from about 12k weight rows on the shared-activation kernel wins at
 // any number of rows; below that it wins when every wave would fetch its own copy of more
@@ -1498,18 +1487,11 @@ struct StreamSet {
     uint4 x[XP];      // this thread's pieces of the activation chunk
 };
 
-// With ssq_in (at most 16 rows, K in one piece) the activations are the residual stream times a norm's
-// weight, and each row's result is multiplied at the end by the row's scale rsqrt(sum of squares / K +
-// eps) (rows.h): the partial sums are asked for at the start and needed only then.
 template <typename TOut, int MT, int ST_WAVES>
 __global__ __launch_bounds__(ST_WAVES * 64) void k_gemm_bf16_stream(
     const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, const float* __restrict__ bias,
-    TOut* __restrict__ Y, int M, int N, int K_all, int k_per, Epilogue epilogue, const float* __restrict__ ssq_in,
-    int n_parts, float eps) {
+    TOut* __restrict__ Y, int M, int N, int K_all, int k_per, Epilogue epilogue) {
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][MT * 16 * ST_LD];
-    __shared__ float norm_part[ST_WAVES * 4 * 16];
-    RowsSsq early;
-    if (ssq_in) rows_ssq_ask(early, ssq_in, n_parts, 0);
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, g = lane >> 4;
@@ -1621,12 +1603,6 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_gemm_bf16_stream(
         step(kt + 2, s2, s3, s1);
         step(kt + 3, s3, s0, s2);
     }
-    float row_scale = 1.f;
-    if (ssq_in) {        // (rows beyond 16 have no sums: the host sends such products elsewhere)
-        norm_part[(tid >> 4) * 16 + (tid & 15)] = rows_ssq_sum(early, ssq_in, n_parts);
-        __syncthreads();
-        row_scale = rows_scale(norm_part, min(r16, M - 1), K_all, eps);
-    }
     // D layout of the 16x16 tile: lane holds column lane%16 (an activation row), rows 4*(lane/16)+i (weight rows)
     const int nq = n0 + g * 4;
 #pragma unroll
@@ -1636,7 +1612,7 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_gemm_bf16_stream(
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            v[i] = (ssq_in ? __fmul_rn(acc[mt][i], row_scale) : acc[mt][i]) + ((bias && nq + i < N) ? bias[nq + i] : 0.f);
+            v[i] = acc[mt][i] + ((bias && nq + i < N) ? bias[nq + i] : 0.f);
         if (epilogue == EPI_SWIGLU) {
 #pragma unroll
             for (int i = 0; i < 4; i += 2)
@@ -1651,31 +1627,15 @@ __global__ __launch_bounds__(ST_WAVES * 64) void k_gemm_bf16_stream(
 
 template <typename TOut, int MT>
 static void launch_stream(const bf16_t* x, const bf16_t* w, const float* bias, TOut* y, int m, int n, int k,
-                          Epilogue epilogue, int nw, int slices, hipStream_t s, const float* ssq_in = nullptr,
-                          int n_parts = 0, float eps = 0.f) {
+                          Epilogue epilogue, int nw, int slices, hipStream_t s) {
     const int k_per = ((k + slices - 1) / slices + ST_BK - 1) / ST_BK * ST_BK;
     dim3 grid((unsigned)((n + nw * 16 - 1) / (nw * 16)), (unsigned)((k + k_per - 1) / k_per));
     if (nw == 8)
-        k_gemm_bf16_stream<TOut, MT, 8><<<grid, 8 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue, ssq_in, n_parts, eps);
+        k_gemm_bf16_stream<TOut, MT, 8><<<grid, 8 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
     else if (nw == 4)
-        k_gemm_bf16_stream<TOut, MT, 4><<<grid, 4 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue, ssq_in, n_parts, eps);
+        k_gemm_bf16_stream<TOut, MT, 4><<<grid, 4 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
     else
-        k_gemm_bf16_stream<TOut, MT, 2><<<grid, 2 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue, ssq_in, n_parts, eps);
-}
-
-// For the products of a step of at most 16 rows (decode_rows.hip): a weight of many rows is streamed
-// faster by this kernel, whose waves share the activations, than by one block per 16 weight rows.
-bool imparo_stream_rows_pays(int m, int n, int k) { return m <= 16 && stream_waves(m, n, k) == 4; }
-
-int imparo_stream_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
-                       int epilogue, const float* ssq_in, int n_parts, float eps, hipStream_t s) {
-    const int nw = stream_waves(m, n, k);
-    if (!nw || m > 16) return IMPARO_BAD_ARGUMENT;
-    if (out_dtype == IMPARO_F32)
-        launch_stream<float, 1>(x, w, bias, (float*)y, m, n, k, epilogue, nw, 1, s, ssq_in, n_parts, eps);
-    else
-        launch_stream<bf16_t, 1>(x, w, bias, (bf16_t*)y, m, n, k, epilogue, nw, 1, s, ssq_in, n_parts, eps);
-    return launch_status();
+        k_gemm_bf16_stream<TOut, MT, 2><<<grid, 2 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
 }
 
 // With a K that the kernel with loads straight into LDS does not take: the 256x256 tile with register
@@ -1693,22 +1653,21 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
     // 452: the 128 by 128 tile on four stages, at any number of rows
     if (force == 452 && k % slices == 0 && (k / slices) % (4 * DM_BK) == 0 && dma_tile_takes(m, n, k))
         return launch_dma<TOut>(x, w, bias, y, m, n, k, epilogue, 128, 2, slices, s, 4);
+    if (m <= ROWS_MAX && force == 0)
+        return imparo_few_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue, slices,
+                               nullptr, 0, 0.f, s);
     int nw = stream_waves(m, n, k);
     if (force == 1) nw = 0;
     if (force == 2 || force == 4 || force == 8) nw = force;
     if (m <= 64 && nw) {
-        if (m <= 16)
-            launch_stream<TOut, 1>(x, w, bias, y, m, n, k, epilogue, nw, slices, s);
-        else if (m <= 32)
+        if (m <= 32)
             launch_stream<TOut, 2>(x, w, bias, y, m, n, k, epilogue, nw, slices, s);
         else
             launch_stream<TOut, 4>(x, w, bias, y, m, n, k, epilogue, nw, slices, s);
         return launch_status();
     }
     if (m <= 64) {
-        if (m <= 16)
-            launch_skinny<TOut, 1>(x, w, bias, y, m, n, k, epilogue, slices, s);
-        else if (m <= 32)
+        if (m <= 32)
             launch_skinny<TOut, 2>(x, w, bias, y, m, n, k, epilogue, slices, s);
         else
             launch_skinny<TOut, 4>(x, w, bias, y, m, n, k, epilogue, slices, s);
