@@ -12,6 +12,8 @@
 // a product is summed over k in one order wherever the row lies in its tile, and a token's sum
 // over its experts runs in the order of its own choice.
 #include "common.h"
+
+#include <algorithm>
 #include "api.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -736,101 +738,167 @@ __global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__
     moe_store_tile<2, 2, 4, TOut, GATED>(acc, out, entry_of_slot, gate, expert, row0, rows, n0, N, epi);
 }
 
-// Few rows an expert (a decode step): a block takes 16 outputs of one expert and up to 16 slots. The expert's
-// 16 weight rows are the M side of 16x16x32 products and go from memory straight into the operand registers,
-// K cut over the block's four waves and, inside a wave, walked in runs of 64 with four runs' loads in flight (two
-// where each run has a gate row and an up row)
-// (a lane takes 16 consecutive k of its row, so that four lanes read a row's 128 bytes side by side; the
-// slots' rows are read with the same k order, which is all a dot product asks for). The waves' partial sums
-// meet in LDS and are added in wave order.
-// GATED: the block's 16 outputs come from 16 gate rows and the 16 up rows that belong to them, 32 rows further on.
-template <typename TOut, bool GATED = false>
-__global__ __launch_bounds__(256) void k_moe_gemm_rows16(const bf16_t* __restrict__ A, int a_ld, int gather_div,
+// Few rows an expert (a decode step): a block takes RT tiles of 16 weight rows of one expert and up to 16 slots. A tile is
+// the M side of 16x16x32 products; K is cut in runs of 64 over the block's waves, U neighbouring ones a wave and round, and
+// everything a wave needs is asked for at once, from memory straight into the operand registers, as in decode_rows.hip
+// (what bounds it is reading the experts' matrices and the trips to memory behind one another: the tile list, then the
+// weights and the slots' tokens, whose rows come last). A lane takes 16 consecutive k of its row, so that four lanes read
+// a row's 128 bytes side by side; the slots' rows are read with the same k order, which is all a dot product asks for.
+// The waves' partial sums meet in LDS and are added in wave order.
+// GATED: half of a block's tiles are gate rows, the other half the up rows that belong to them, 32 rows further on.
+// 8 tokens, 4 of 8 experts and a shared one: gate and up, 1,536 rows by 1,024 an expert, 9.1 us (two runs a wave at a time,
+// the blocks unevenly over the XCDs: 12.0), the way back, 1,024 by 768, 6.1 (6.3); one token 6.3 and 4.9 (7.5 and 4.7).
+#define MOE_ROWS_WAVES 8
+template <typename TOut, bool GATED, int RT, int U>
+__global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const bf16_t* __restrict__ A, int a_ld, int gather_div,
                                                          const int32_t* __restrict__ entry_of_slot,
                                                          const bf16_t* __restrict__ W, TOut* __restrict__ out,
-                                                         const int32_t* __restrict__ tiles, int N, int K, int epi,
-                                                         MoeGate gate = {}) {
-    constexpr int S = GATED ? 2 : 1;       // weight rows a lane walks side by side
-    constexpr int U = GATED ? 2 : 4;       // runs whose loads are under way at once
+                                                         const int32_t* __restrict__ tiles, int max_tiles, int across,
+                                                         int N, int K, int epi, MoeGate gate) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    __shared__ f32x4 part[4][S][WAVE];
-    const int expert = tiles[3 * blockIdx.x];
+    constexpr int GROUPS = GATED ? RT / 2 : RT;          // of 16 outputs a block
+    static_assert(!GATED || RT % 2 == 0, "as many gate tiles as up tiles");
+    extern __shared__ float4 moe_part[];                 // [waves][RT][WAVE]
+    // The tiles that hold slots come first in the grid, so that the XCDs, which take its blocks in turn, have equally many of
+    // them (9 tiles of 12 by 24 blocks, tile after tile along the grid: 36 on two XCDs of 32 CUs and 24 on the others, 12.0 us
+    // where this way it is 9.1).
+    const int32_t* last = tiles + 3 * (max_tiles - 1);
+    const int n_tiles = last[0] < 0 && last[2] == MOE_COUNTED ? min(last[1], max_tiles) : max_tiles;
+    const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;
+    const int tile = block / (unsigned)across;
+    if (tile >= n_tiles) return;
+    const int expert = tiles[3 * tile];
     if (expert < 0) return;
-    const int row0 = tiles[3 * blockIdx.x + 1], rows = tiles[3 * blockIdx.x + 2];
-    const int n0 = blockIdx.y * 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
+    const int n0 = (int)(block - (unsigned)tile * across) * 16 * GROUPS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int c = lane & 15, g = lane >> 4;
-    const int f = n0 + c;
-    const bf16_t* wrow = W + ((size_t)expert * N + (GATED ? (f >> 5) * 64 + (f & 31) : min(f, N - 1))) * K;
     const int slot = row0 + min(c, rows - 1);
-    const bf16_t* arow = A + (size_t)(gather_div ? entry_of_slot[slot] / gather_div : slot) * a_ld;
-    // this wave's part of K, in whole runs of 64
+    const int entry = entry_of_slot ? entry_of_slot[slot] : 0;
+    const bf16_t* wrow[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+        const int f = n0 + (t % GROUPS) * 16 + c;
+        wrow[t] = W + ((size_t)expert * N + (GATED ? (f >> 5) * 64 + (f & 31) + (t / GROUPS) * 32 : min(f, N - 1))) * K;
+    }
     const int runs = (K + 63) / 64;
-    const int per_wave = (runs + 3) / 4;
-    const int run_lo = wave * per_wave, run_hi = min(runs, run_lo + per_wave);
-    f32x4 acc[S];
+    u32x4 w[RT][U][2], x[U][2];
+    // (no load under a branch: what lies past K is read again from inside the row, and its weights count as zeros)
+    auto k_of = [&](int run, int h) { return min(min(run, runs - 1) * 64 + g * 16 + h * 8, K - 8); };
+    auto ask_weights = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < S; ++s) acc[s] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    for (int r0 = run_lo; r0 < run_hi; r0 += U) {
-        u32x4 w[S][U][2], a[U][2];
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[t][u][h] = *reinterpret_cast<const u32x4*>(wrow[t] + k_of(first + u, h));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ask_weights(wave * U);
+    const bf16_t* arow = A + (size_t)(gather_div ? entry / gather_div : slot) * a_ld;
+    auto ask_rows = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int k = min(r0 + u, run_hi - 1) * 64 + g * 16 + h * 8;
-                const bool in = k < K && r0 + u < run_hi;
-                const int kk = k < K ? k : 0;
+            for (int h = 0; h < 2; ++h) x[u][h] = *reinterpret_cast<const u32x4*>(arow + k_of(first + u, h));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    ask_rows(wave * U);
+    const float limit = GATED && gate.limits ? gate.limits[expert] : 0.f;
+    const float sw = GATED ? moe_slot_weight(gate, entry_of_slot, slot) : 1.f;
+    f32x4 acc[RT];
 #pragma unroll
-                for (int s = 0; s < S; ++s) {
-                    const u32x4 wv = *reinterpret_cast<const u32x4*>(wrow + (size_t)s * 32 * K + kk);
-                    w[s][u][h] = in ? wv : zero;
+    for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int first = wave * U; first < runs;) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (first + u >= runs) continue;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool in = (first + u) * 64 + g * 16 + h * 8 < K;
+                    const u32x4 wv = in ? w[t][u][h] : u32x4{0u, 0u, 0u, 0u}, xv = in ? x[u][h] : u32x4{0u, 0u, 0u, 0u};
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv), __builtin_bit_cast(bf16x8, xv),
+                                                                     acc[t], 0, 0, 0);
                 }
-                const u32x4 av = *reinterpret_cast<const u32x4*>(arow + kk);
-                a[u][h] = in ? av : zero;
             }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int s = 0; s < S; ++s)
-                    acc[s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[s][u][h]),
-                                                                     __builtin_bit_cast(bf16x8, a[u][h]), acc[s], 0, 0, 0);
+        first += waves * U;
+        if (first < runs) {
+            ask_weights(first);
+            ask_rows(first);
+        }
     }
 #pragma unroll
-    for (int s = 0; s < S; ++s) part[wave][s][lane] = acc[s];
+    for (int t = 0; t < RT; ++t) moe_part[(wave * RT + t) * WAVE + lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
     __syncthreads();
-    if (wave != 0) return;
-    f32x4 total[S];
+    auto total = [&](int t, float (&v)[4]) __attribute__((always_inline)) {
+        float4 p[MOE_ROWS_WAVES];
 #pragma unroll
-    for (int s = 0; s < S; ++s) total[s] = part[0][s][lane];
+        for (int q = 0; q < MOE_ROWS_WAVES; ++q) p[q] = moe_part[(min(q, waves - 1) * RT + t) * WAVE + lane];
+        v[0] = p[0].x, v[1] = p[0].y, v[2] = p[0].z, v[3] = p[0].w;
 #pragma unroll
-    for (int w2 = 1; w2 < 4; ++w2)
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const f32x4 p = part[w2][s][lane];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) total[s][i] += p[i];
-        }
-    // a lane holds slot c, outputs n0 + 4 g + i
-    if (c < rows) {
+        for (int q = 1; q < MOE_ROWS_WAVES; ++q)
+            if (q < waves) v[0] += p[q].x, v[1] += p[q].y, v[2] += p[q].z, v[3] += p[q].w;
+    };
+    // a lane holds slot c, outputs 4 g + i of a group
+    for (int t = wave; t < GROUPS; t += waves) {
+        float v[4];
+        total(t, v);
+        const int n = n0 + t * 16 + 4 * g;
         if constexpr (GATED) {
-            const float limit = gate.limits ? gate.limits[expert] : 0.f;
-            const float sw = moe_slot_weight(gate, entry_of_slot, row0 + c);
+            float up[4];
+            total(t + GROUPS, up);
+            if (c >= rows) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = moe_act_fast(sw * v[i], sw * up[i], limit, gate.alpha);
+            TOut* dst = out + (size_t)(row0 + c) * (N / 2) + n;
+            if (((uintptr_t)out & 7) == 0)               // (N / 2 is a multiple of 32, and the output bfloat16)
+                *reinterpret_cast<uint2*>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+            else
+                for (int i = 0; i < 4; ++i) store_f32<TOut>(dst, i, v[i]);
+        } else if (c < rows) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                store_f32<TOut>(out, (size_t)(row0 + c) * (N / 2) + n0 + 4 * g + i,
-                                moe_act_fast(sw * total[0][i], sw * total[S - 1][i], limit, gate.alpha));
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int n = n0 + 4 * g + i;
-            if (n < N) store_f32<TOut>(out, (size_t)(row0 + c) * N + n, moe_epilogue(total[0][i], epi));
+                if (n + i < N) store_f32<TOut>(out, (size_t)(row0 + c) * N + n + i, moe_epilogue(v[i], epi));
         }
     }
+}
+
+// A block a CU, as far as the list's length tells before it is known (tiles may be empty): tiles of 16 rows a block
+template <typename TOut, bool GATED>
+static void launch_rows16(const bf16_t* a, int a_ld, int gather_div, const int32_t* entry_of_slot, const bf16_t* w, TOut* out,
+                          const int32_t* tiles, int max_tiles, int n, int k, int epi, const MoeGate& gate, hipStream_t s) {
+    const int runs = (k + 63) / 64;
+    const int u = runs <= MOE_ROWS_WAVES ? 1 : runs <= 2 * MOE_ROWS_WAVES ? 2 : 4;
+    const int waves = std::min(MOE_ROWS_WAVES, (runs + u - 1) / u);
+    const long long all = (long long)std::max(1, max_tiles - 1) * ((n + 15) / 16);
+    const int rt = GATED ? (all <= 512 ? 2 : 4) : (all <= 1024 ? 1 : 4);
+    const int outputs = 16 * (GATED ? rt / 2 : rt), columns = GATED ? n / 2 : n;
+    const int across = (columns + outputs - 1) / outputs;
+    const long long blocks = (long long)max_tiles * across, row = std::min<long long>(blocks, 1 << 22);
+    const dim3 grid((unsigned)row, (unsigned)((blocks + row - 1) / row));    // (a launch holds fewer than 2^32 threads along x)
+    const size_t lds = (size_t)waves * rt * WAVE * sizeof(float4);
+#define ROWS16_U(RT, U)                                                                                              \
+    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, waves * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles, \
+                                                                      max_tiles, across, n, k, epi, gate)
+#define ROWS16_GO(RT)                                                                                                \
+    do {                                                                                                             \
+        if (u == 1) ROWS16_U(RT, 1);                                                                                 \
+        else if (u == 2) ROWS16_U(RT, 2);                                                                            \
+        else ROWS16_U(RT, 4);                                                                                        \
+    } while (0)
+    if constexpr (!GATED) {
+        if (rt == 1) {
+            ROWS16_GO(1);
+            return;
+        }
+    }
+    if (rt == 2) ROWS16_GO(2);
+    else ROWS16_GO(4);
+#undef ROWS16_GO
+#undef ROWS16_U
 }
 
 // The same in float32: a tile of 64 slots by 64 outputs, K in steps of 16 through LDS, every output
@@ -947,19 +1015,18 @@ extern "C" int imparo_moe_gemm(const void* a, int a_ld, int gather_div, const in
     }
     if (epilogue == MOE_EPI_GATED) {
         if (tile_rows == 16)
-            k_moe_gemm_rows16<bf16_t, true><<<dim3(max_tiles, n / 32), 256, 0, s>>>(
-                (const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (bf16_t*)out, tiles, n, k, epilogue, gate);
+            launch_rows16<bf16_t, true>((const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (bf16_t*)out, tiles,
+                                        max_tiles, n, k, epilogue, gate, s);
         else if (tile_rows == 64) MOE_LAUNCH_GATED(1);
         else if (tile_rows == 128) MOE_LAUNCH_GATED(2);
         else return IMPARO_BAD_ARGUMENT;
     } else if (tile_rows == 16) {
-        const dim3 grid16(max_tiles, (n + 15) / 16);
         if (out_dtype == IMPARO_BF16)
-            k_moe_gemm_rows16<bf16_t><<<grid16, 256, 0, s>>>((const bf16_t*)a, a_ld, gather_div, entry_of_slot,
-                                                             (const bf16_t*)w, (bf16_t*)out, tiles, n, k, epilogue);
+            launch_rows16<bf16_t, false>((const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (bf16_t*)out, tiles,
+                                         max_tiles, n, k, epilogue, gate, s);
         else if (out_dtype == IMPARO_F32)
-            k_moe_gemm_rows16<float><<<grid16, 256, 0, s>>>((const bf16_t*)a, a_ld, gather_div, entry_of_slot,
-                                                            (const bf16_t*)w, (float*)out, tiles, n, k, epilogue);
+            launch_rows16<float, false>((const bf16_t*)a, a_ld, gather_div, entry_of_slot, (const bf16_t*)w, (float*)out, tiles,
+                                        max_tiles, n, k, epilogue, gate, s);
         else
             return IMPARO_BAD_ARGUMENT;
     } else if (tile_rows == 128) {

@@ -63,3 +63,53 @@ def test_rows_scaled_at_the_end(m, k, parts):
     ops.rows_gemm(x, w, out=plain)
     scale = torch.rsqrt(ssq.double()[:, :m].sum(0) / k + 1e-5)
     torch.testing.assert_close(out.cpu().double(), plain.cpu().double() * scale[:, None], rtol=parts * EPS + 1e-6, atol=0.0)
+
+
+# one to four tiles of weight rows a block, a last block partly past the end, K of less than a run, ragged, one round of
+# runs and more than one; experts that nobody chose, so that the list ends in empty tiles
+@pytest.mark.parametrize("n, k", [(64, 8), (192, 72), (1536, 1024), (1088, 136), (64, 2120), (832, 768)])
+@pytest.mark.parametrize("tokens, experts, top", [(1, 3, 2), (8, 9, 4), (16, 4, 4)])
+def test_experts_products_of_few_rows(n, k, tokens, experts, top):
+    g = torch.Generator().manual_seed(n + k + tokens)
+    choice = torch.stack([torch.randperm(max(top, experts - 2), generator=g)[:top] for _ in range(tokens)]).int()
+    entries = tokens * top
+    rows = ops.moe_tile_rows(entries, experts, torch.bfloat16)
+    assert rows == 16
+    tiles = torch.empty(ops.moe_max_tiles(entries, experts, rows), 3, device=DEV, dtype=torch.int32)
+    slot, entry = torch.empty(entries, device=DEV, dtype=torch.int32), torch.empty(entries, device=DEV, dtype=torch.int32)
+    ops.moe_plan(choice.to(DEV), experts, rows, slot, entry, tiles)
+    x, w = rnd(tokens, k, seed=1).bfloat16().to(DEV), rnd(experts, n, k, seed=2, scale=0.1).bfloat16().to(DEV)
+    weight = torch.rand(entries, generator=g).to(DEV)
+    per_entry, expert = x.double().repeat_interleave(top, 0), choice.flatten().long().to(DEV)
+    plain = torch.bmm(w.double()[expert], per_entry[:, :, None])[:, :, 0]
+    bound = torch.bmm(w.double().abs()[expert], per_entry.abs()[:, :, None])[:, :, 0] * (k + 2) * EPS
+    at = slot.long()
+    out = torch.full((entries, n), float("nan"), device=DEV)
+    ops.moe_gemm(x, w, out, tiles, rows, entry_of_slot=entry, gather_div=top)
+    assert bool(((out[at].double() - plain).abs() <= bound).all())
+    half = torch.empty(entries, n, device=DEV, dtype=torch.bfloat16)
+    ops.moe_gemm(x, w, half, tiles, rows, entry_of_slot=entry, gather_div=top)
+    assert torch.equal(half, out.bfloat16())
+    gated = torch.full((entries, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.moe_gemm(x, w, gated, tiles, rows, entry_of_slot=entry, gather_div=top, epilogue="gated", weight=weight)
+    z = out[at].double().view(entries, n // 64, 2, 32) * weight.double()[:, None, None, None]
+    want = (z[:, :, 0] / (1.0 + torch.exp(-z[:, :, 0])) * z[:, :, 1]).reshape(entries, n // 2)
+    torch.testing.assert_close(gated[at].double(), want, rtol=2.0 ** -8 + 1e-5, atol=1e-6)
+
+
+# float32 through the ring: fewer chunks of 64 than stages, as many, an odd number, more than one turn; weight rows that are no
+# multiple of 16; one load of activations a stage and four; a K that goes the other way; few blocks and more than 512
+@pytest.mark.parametrize("n, k", [(5, 64), (33, 256), (70, 704), (40, 768), (16, 832), (130, 1600), (8200, 320), (24, 68)])
+@pytest.mark.parametrize("m", [1, 4, 5, 16])
+def test_float32_few_rows_are_the_many_rows_bits(m, n, k):
+    x, w, b = rnd(20, k, seed=1).to(DEV), rnd(n, k, seed=2, scale=0.1).to(DEV), rnd(n, seed=3).to(DEV)
+    many = torch.empty(20, n, device=DEV)
+    ops.gemm(x, w, many, bias=b)                 # (more than 16 rows: the tile kernel, held to the statement elsewhere)
+    few = torch.full((m, n), float("nan"), device=DEV)
+    ops.gemm(x[:m].contiguous(), w, few, bias=b)
+    assert torch.equal(few, many[:m])
+    if n % 2 == 0:
+        many, few = torch.empty(20, n // 2, device=DEV), torch.full((m, n // 2), float("nan"), device=DEV)
+        ops.gemm(x, w, many, bias=b, swiglu=True)
+        ops.gemm(x[:m].contiguous(), w, few, bias=b, swiglu=True)
+        assert torch.equal(few, many[:m])
