@@ -150,6 +150,13 @@ __device__ __forceinline__ void load_to_lds_uncounted(const bf16_t* src, unsigne
                  : "v"(src), "s"(lds_byte)
                  : "memory", "m0");
 }
+// The same from a uniform base and a byte offset a lane
+__device__ __forceinline__ void load_to_lds_uncounted(const float* base, unsigned byte_offset, unsigned lds_byte) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(byte_offset), "s"(base), "s"(lds_byte)
+                 : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // Orders LDS traffic between the lanes of one wave: what any lane wrote before

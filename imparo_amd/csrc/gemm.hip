@@ -167,12 +167,11 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
 // and walks K alone, operands from memory straight into registers, 16 bytes a lane: lane (row, g) asks for
 // k = 4g .. 4g + 3 of 16, and a transposition over the four groups of lanes (four lane swaps) gives it
 // k = g, 4 + g, 8 + g, 12 + g, which is how the products want them. Loads run seven chunks of 32 ahead in eight
-// register sets. A weight of many rows is bound by its bytes. One of few rows leaves most CUs idle and is
-// bound by one wave's walk: products that each wait for the one before them, 32 cycles for 4 k (16 us for K = 4,608), and
-// about as much again for the lane swaps and waits between them. Measured, cold weights, 2 rows: 65,536 by 1,024 57 us (4.7 TB/s), 9,216 by 1,024 14 us,
-// 1,024 by 4,608 33 us; 17 us on average over a decode step where two weight rows a thread through LDS took 79. The loads ask
-// for 4-byte alignment only, so a K that is no multiple of 4 and operands that start anywhere come this way too: 2 rows of 1,024 by
-// 1,026 9.9 us, 65,536 by 1,022 44 (value by value in tiles of 64 rows 50 and 144, the kernel before both 45 and 111).
+// register sets. For any K and operands that start anywhere, as its loads ask for 4-byte alignment only (2 rows of 1,024 by
+// 1,026 9.9 us, 65,536 by 1,022 44; value by value in tiles of 64 rows 50 and 144); a K that is a multiple of 64 goes
+// through the ring below. Bound by the weight's bytes, or, where few rows leave most CUs idle, by one wave's walk: products
+// that each wait for the one before them, 32 cycles for 4 k (16 us for K = 4,608), and about as much again for the lane swaps
+// and waits between them.
 #define F32R_BK 32
 #define F32R_SETS 8
 struct RowsF32Set {
@@ -197,6 +196,25 @@ __device__ __forceinline__ void transpose_over_groups(const f32x4& from, float (
     swap_lanes_32(v[1], v[3]);
     swap_lanes_16(v[0], v[1]);
     swap_lanes_16(v[2], v[3]);
+}
+
+// lane: token m, weight rows n .. n + 3
+template <typename TOut>
+__device__ __forceinline__ void f32_rows_out(const f32x4& acc, const float* __restrict__ bias, TOut* __restrict__ Y, int m, int n, int M,
+                                             int N, const Epilogue& epilogue) {
+    if (m >= M) return;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = bias && n + i < N ? acc[i] + bias[n + i] : acc[i];
+    if (epilogue == EPI_SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            if (n + i + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + (n + i) / 2, gated_mul(epilogue, v[i], v[i + 1]));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < N) store_f32<TOut>(Y, (size_t)m * N + n + i, v[i]);
 }
 
 template <typename TOut>
@@ -276,26 +294,111 @@ __global__ __launch_bounds__(64) void k_gemm_f32_rows(const float* __restrict__ 
         }
         multiply(f);
     }
-    // lane: token lane % 16, weight rows 4 * (lane / 16) + i
-    const int m = r16, n = n0 + g * 4;
-    if (m >= M) return;
-    float v[4];
+    f32_rows_out<TOut>(acc, bias, Y, r16, n0 + g * 4, M, N, epilogue);
+}
+
+// The same with K a multiple of 64 and operands that start at multiples of 16 bytes: through a ring of S stages of 64 k in
+// LDS that the loads go straight into, no more than the chain of products in the wave's way. A row's 16 pieces of four k lie
+// in the order piece ^ (row % 16): product i wants k = 4 i + g of row r in lane (r, g), which are 64 different banks, so the
+// operands come from LDS as the products want them, without lane swaps. A wave is a block and has its ring to itself: no
+// barriers, it counts its own loads. XI: load instructions for the activations of a stage, four rows each. Bound by the
+// chain, 32 cycles for 4 k, where the weight has few rows, by its bytes where it has many.
+// Measured, cold weights, 2 rows (the kernel above): 1,024 by 1,024 6.5 us (9.0), 1,024 by 4,608 20 (33), 9,216 by 1,024 10.6
+// (12.0), 65,536 by 1,024 51 (56); 16 rows of 9,216 by 1,024 11 (15.6).
+template <typename TOut, int S, int XI>
+__global__ __launch_bounds__(64) void k_gemm_f32_rows_ring(const float* __restrict__ X, const float* __restrict__ W,
+                                                           const float* __restrict__ bias, TOut* __restrict__ Y,
+                                                           int M, int N, int K, Epilogue epilogue) {
+    constexpr int STAGE = (16 + 4 * XI) * 64;               // floats
+    static_assert((S - 1) * (4 + XI) <= 63 && S * STAGE * 4 <= 65536, "loads a wave can count, and LDS in reach of an offset");
+    __shared__ __attribute__((aligned(1024))) float ring[S * STAGE];
+    const int lane = threadIdx.x, r16 = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    const int n_chunks = K / 64;
+    // loading: an instruction fills four rows; lane -> row lane / 16, place lane % 16, where piece place ^ (row % 16) lies.
+    // Uniform bases that walk along K and offsets inside 16 rows that stay: a load takes three instructions.
+    unsigned offset[4 + XI];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = bias && n + i < N ? acc[i] + bias[n + i] : acc[i];
-    if (epilogue == EPI_SWIGLU) {
-#pragma unroll
-        for (int i = 0; i < 4; i += 2)
-            if (n + i + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + (n + i) / 2, gated_mul(epilogue, v[i], v[i + 1]));
-        return;
+    for (int q = 0; q < 4 + XI; ++q) {
+        const int row = (q < 4 ? q * 4 : (q - 4) * 4) + (lane >> 4);
+        offset[q] = ((unsigned)(q < 4 ? min(row, N - 1 - n0) : min(row, M - 1)) * (unsigned)K + ((lane & 15) ^ row) * 4) * 4u;
     }
+    const float* wbase = W + (size_t)n0 * K;
+    const unsigned lds = (unsigned)(size_t)(__attribute__((address_space(3))) float*)ring;
+    auto load = [&](int stage, int chunk, int q) __attribute__((always_inline)) {      // (past the end: the last chunk again, nobody reads it)
+        load_to_lds_uncounted((q < 4 ? wbase : X) + min(chunk, n_chunks - 1) * 64, offset[q],
+                              __builtin_amdgcn_readfirstlane(lds + stage * STAGE * 4 + q * 1024));
+    };
+    const int x_row = min(r16, M - 1);
+    int w_at[16], x_at[16];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (n + i < N) store_f32<TOut>(Y, (size_t)m * N + n + i, v[i]);
+    for (int i = 0; i < 16; ++i) {
+        w_at[i] = r16 * 64 + ((i ^ r16) << 2) + g;
+        x_at[i] = 1024 + x_row * 64 + ((i ^ x_row) << 2) + g;
+    }
+    struct Operands {
+        float w[16], x[16];
+    };
+    auto read = [&](int stage, Operands& o, int i) __attribute__((always_inline)) {
+        o.w[i] = ring[stage * STAGE + w_at[i]];
+        o.x[i] = ring[stage * STAGE + x_at[i]];
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    Operands even, odd;
+    // Chunk c of 16 products: its operands are in registers or about to be, chunks c + 1 to c + S - 1 are on their way.
+    // Between one product and the next, which waits for it, the operands of chunk c + 1 are read and the loads of chunk
+    // c + S go out into the stage that chunk c was read from.
+    auto step = [&](int stage, int c, const Operands& now, Operands& next) __attribute__((always_inline)) {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * (4 + XI)) : "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(now.w[i], now.x[i], acc, 0, 0, 0);
+            if (i < 8) {                                  // (so early that the last of them is there when the chunk ends)
+                read((stage + 1) % S, next, 2 * i);
+                read((stage + 1) % S, next, 2 * i + 1);
+            }
+            if (i < 4 + XI) load(stage, c + S, i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int q = 0; q < 4 + XI; ++q) load(i, i, q);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * (4 + XI)) : "memory");
+#pragma unroll
+    for (int i = 0; i < 16; ++i) read(0, even, i);
+    static_assert(S % 2 == 0, "two register sets in turn");
+    for (int c = 0; c < n_chunks; c += S) {
+#pragma unroll
+        for (int i = 0; i < S; i += 2) {
+            if (c + i < n_chunks) step(i, c + i, even, odd);
+            if (c + i + 1 < n_chunks) step(i + 1, c + i + 1, odd, even);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // nothing may land in LDS that is another block's
+    f32_rows_out<TOut>(acc, bias, Y, r16, n0 + g * 4, M, N, epilogue);
 }
 
 template <typename TOut>
 static int launch_f32(const float* x, const float* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                       hipStream_t s) {
+    const unsigned rows_blocks = (unsigned)((n + 15) / 16);
+    if (m <= 16 && k % 64 == 0 && k < (1 << 25) && !(((uintptr_t)x | (uintptr_t)w) & 15)) {
+        // stages: as many as keep a wave alone on its CU supplied, fewer where more waves share the CU and its LDS (9,216 by
+        // 1,024: 8 stages 11.1 us, 4 10.6)
+        if (m <= 4 && rows_blocks <= 512)
+            k_gemm_f32_rows_ring<TOut, 12, 1><<<rows_blocks, 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
+        else if (m <= 4)
+            k_gemm_f32_rows_ring<TOut, 4, 1><<<rows_blocks, 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
+        else if (rows_blocks <= 512)
+            k_gemm_f32_rows_ring<TOut, 8, 4><<<rows_blocks, 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
+        else
+            k_gemm_f32_rows_ring<TOut, 4, 4><<<rows_blocks, 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
+        return launch_status();
+    }
     if (m <= 16 && k < (1 << 25)) {                  // (offsets inside 16 rows are kept in 32 bits)
         k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
         return launch_status();
