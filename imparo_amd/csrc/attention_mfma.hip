@@ -160,6 +160,25 @@ __device__ __forceinline__ void decode_load(DecodeTile<ND>& r, const Paged& kv, 
         r.v[dt].u = *reinterpret_cast<const uint4*>(vbase + (size_t)(dt * 16 + c) * kv.page_size);
 }
 
+// The same for pages of 32 keys and more, where a tile lies in one page: `page` is the same for the whole wave, and no
+// address waits for anything else. What the page holds outside the live keys is forced to zero before use.
+template <int ND>
+__device__ __forceinline__ void decode_load_paged(DecodeTile<ND>& r, const Paged& kv, int key_base, int page, int lane) {
+    constexpr int D = ND * 16, NK = (ND + 1) / 2;
+    const int c = lane & 15, g = lane >> 4;
+    const size_t head_of_page = (size_t)page * kv.kv_heads + kv.kvh;
+    const int first = key_base & (kv.page_size - 1);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const bf16_t* krow = kv.k + (head_of_page * kv.page_size + first + 8 * (c >> 2) + 4 * t + (c & 3)) * D;
+#pragma unroll
+        for (int dk = 0; dk < NK; ++dk) r.k[t][dk].u = *reinterpret_cast<const uint4*>(krow + min(dk * 32 + 8 * g, D - 8));
+    }
+    const bf16_t* vbase = kv.v + head_of_page * kv.page_size * D + first + 8 * g;
+#pragma unroll
+    for (int dt = 0; dt < ND; ++dt) r.v[dt].u = *reinterpret_cast<const uint4*>(vbase + (size_t)(dt * 16 + c) * kv.page_size);
+}
+
 // One softmax step over a loaded tile of 32 keys. [lo_q, hi_q] is the key range of this
 // lane's query. `full`: every key of the tile is inside every query's range.
 template <int ND>
@@ -352,8 +371,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     __shared__ float sn_tab[FROM_QKV ? D / 2 : 1], cs_tab[FROM_QKV ? D / 2 : 1];
     __shared__ __attribute__((aligned(16))) float qw_tab[FROM_QKV ? D : 1], kw_tab[FROM_QKV ? D : 1];
     __shared__ __attribute__((aligned(16))) float k_raw[FROM_QKV ? D : 1], v_raw[FROM_QKV ? D : 1];
-    const int all_waves = threadIdx.x >> 6;                 // of the block; `wave` is one of its split's
-    const int split = SPLITS == 1 ? blockIdx.x : __builtin_amdgcn_readfirstlane(all_waves / MFMA_WAVES), ri = blockIdx.z;
+    const int all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // of the block; `wave` is one of its split's
+    const int split = SPLITS == 1 ? blockIdx.x : all_waves / MFMA_WAVES, ri = blockIdx.z;
     const int G = heads / kv_heads, passes = (G + 15) / 16;
     const int kvh = blockIdx.y / passes, pass = blockIdx.y % passes;
     const int row = rows[ri];
@@ -384,11 +403,44 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     const int hi_q = qvalid ? last : -1;
     // (a block with the row's own key only: one clamped tile is loaded and none is used)
     const int lo_c = (EXT && keep > 0) ? 0 : min(lo, max(last, 0)), last_c = max(last, 0);
+    // What the block shares and the projection's rows are asked for before the tiles: loads come back in order, and who waits
+    // for one behind the tiles' waits for the tiles too, at the barrier the whole block with it (one row over 50 keys 6.3 us,
+    // so 5.7; 8 rows over 300 keys 8.7 and 7.9).
+    HeadElements<ND> qh;
+    const int units = heads + 2 * kv_heads;
+    float freq;
+    float2 q_norm, k_norm;
+    float4 own_raw;
+    const int norm_at = 2 * ((int)threadIdx.x - 128);       // (another wave's lanes than the sines and cosines)
+    const int own_at = 4 * (lane % (D / 4));
+    if constexpr (FROM_QKV) {                               // (every lane asks, for something: no load under a branch)
+        const float* row_in = fq.qkv + (size_t)t * units * D;
+        const int norm_from = min(max(norm_at, 0), D - 2);
+        head_elements<ND>(qh, row_in + (size_t)head * D, g);
+        freq = (fq.inv_freq ? fq.inv_freq : row_in)[min((int)threadIdx.x, D / 2 - 1)];
+        q_norm = make_float2((fq.q_weight ? fq.q_weight : row_in)[norm_from], (fq.q_weight ? fq.q_weight : row_in)[norm_from + 1]);
+        k_norm = make_float2((fq.q_weight ? fq.k_weight : row_in)[norm_from], (fq.q_weight ? fq.k_weight : row_in)[norm_from + 1]);
+        own_raw = *reinterpret_cast<const float4*>(row_in + (size_t)(lane < D / 4 ? heads + kvh : heads + kv_heads + kvh) * D + own_at);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     DecodeTile<ND> regs[TILES];
+    // (with the queries given, where nothing else waits for scalar loads, the lanes' own are no slower: 4.3 us, 4.5 so)
+    if (FROM_QKV && page_size >= 32) {
+        int page[TILES];
 #pragma unroll
-    for (int j = 0; j < TILES; ++j)             // past the split's end: clamped addresses, never used
-        decode_load<ND>(regs[j], kv, walk.key(k_begin + (wave + j * MFMA_WAVES) * 32), lo_c, last_c, lane);
-    if (!FROM_QKV) {
+        for (int j = 0; j < TILES; ++j) {       // past the split's end: some page, never used
+            const int base = walk.key(k_begin + (wave + j * MFMA_WAVES) * 32);
+            page[j] = min(max(kv.table[min(base >> kv.page_shift, table_stride - 1)], 0), n_pages - 1);
+        }
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)
+            decode_load_paged<ND>(regs[j], kv, walk.key(k_begin + (wave + j * MFMA_WAVES) * 32), page[j], lane);
+    } else {
+#pragma unroll
+        for (int j = 0; j < TILES; ++j)         // past the split's end: clamped addresses, never used
+            decode_load<ND>(regs[j], kv, walk.key(k_begin + (wave + j * MFMA_WAVES) * 32), lo_c, last_c, lane);
+    }
+    if constexpr (!FROM_QKV) {
         const bf16_t* qrow = q + ((size_t)t * heads + head) * D;
 #pragma unroll
         for (int dk = 0; dk < NK; ++dk) {
@@ -396,24 +448,16 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
             st.q[dk].u = zero_unless(qvalid && d < D, *reinterpret_cast<const uint4*>(qrow + min(d, D - 8)));
         }
     }
-    const int units = heads + 2 * kv_heads;
     if constexpr (FROM_QKV) {
-        // The tiles' loads are on their way; so is the query's row, before anything waits. Meanwhile the
-        // block's sines and cosines are worked out and the norms' weights go to LDS.
-        HeadElements<ND> qh;
-        head_elements<ND>(qh, fq.qkv + ((size_t)t * units + head) * D, g);
-        if (fq.inv_freq && (int)threadIdx.x < D / 2)
-            rotation_of(pos, fq.inv_freq[threadIdx.x], sn_tab[threadIdx.x], cs_tab[threadIdx.x]);
-        if (fq.q_weight && (int)threadIdx.x >= 128 && (int)threadIdx.x < 128 + D / 2) {     // (another wave's lanes)
-            const int i = (int)threadIdx.x - 128;
-            qw_tab[2 * i] = fq.q_weight[2 * i], qw_tab[2 * i + 1] = fq.q_weight[2 * i + 1];
-            kw_tab[2 * i] = fq.k_weight[2 * i], kw_tab[2 * i + 1] = fq.k_weight[2 * i + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        // while the tiles are on their way: the block's sines and cosines, the norms' weights, and the row's new key and
+        // value, which wait in LDS for the last wave
+        if (fq.inv_freq && (int)threadIdx.x < D / 2) rotation_of(pos, freq, sn_tab[threadIdx.x], cs_tab[threadIdx.x]);
+        if (norm_at >= 0 && norm_at < D) {
+            *reinterpret_cast<float2*>(qw_tab + norm_at) = q_norm;
+            *reinterpret_cast<float2*>(kw_tab + norm_at) = k_norm;
         }
-        if (own && wave == 1 && lane < D / 2) {      // the row's new key and value wait in LDS for the first wave
-            const int u = lane < D / 4 ? heads + kvh : heads + kv_heads + kvh, at = 4 * (lane % (D / 4));
-            const float4 x = *reinterpret_cast<const float4*>(fq.qkv + ((size_t)t * units + u) * D + at);
-            *reinterpret_cast<float4*>((lane < D / 4 ? k_raw : v_raw) + at) = x;
-        }
+        if (own && wave == 1 && lane < D / 2) *reinterpret_cast<float4*>((lane < D / 4 ? k_raw : v_raw) + own_at) = own_raw;
         __syncthreads();
         normed_rotated<ND>(st.q, qh, fq.q_weight ? qw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
                            sn_tab, cs_tab, qvalid, g);
@@ -428,7 +472,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         }
     }
     if constexpr (FROM_QKV) {
-        if (own && wave == 0) {
+        // (by the wave that has the fewest tiles, which is done first where the split is not full)
+        if (own && wave == MFMA_WAVES - 1) {
             // the row's own key and value, from the projection's row: every lane holds the key's dims
             // dk*32 + 8*g + j (the same for all 16 heads) and the value's dims dt*16 + 4*g + i
             Frag8 kf[NK];
