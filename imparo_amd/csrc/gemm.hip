@@ -769,7 +769,7 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
 }
 
 // ------------------------------------------------------------------ bfloat16, many rows, loads straight into LDS
-// A tile of 256 or 128 activation rows by 256, 192 or 128 weight rows on eight waves, two per
+// A tile of 256 or 128 activation rows by 256, 192 or 128 weight rows, or of 192 by 256, on eight waves, two per
 // SIMD, so that one's products run while the other waits or writes its results (12% faster than
 // four waves of 128x128 on the gate/up product at 2,048 rows, 5 to 15% on the narrower tiles).
 // A wave has 128 (or 64) rows by 64 or 32 of it, 4x2 or 4x1 MFMA tiles of 32x32 (2x2, 2x1 with
@@ -1053,15 +1053,18 @@ static bool dma_tile_takes(int m, int n, int k) {
     return k % (2 * DM_BK) == 0 && (long long)m * k < (1LL << 31) && (long long)n * k < (1LL << 31);
 }
 
-// Which tile (bm = 256 or 128 activation rows, tn = 4, 3, 2, 1 for 256, 192, 128, 64 weight rows; 192 with
-// bm 256 only, 64 with bm 128 only), on how many stages, and how many slices of K suit a product of many rows; tn = 0:
+// Which tile (bm = 256, 192 or 128 activation rows, tn = 4, 3, 2, 1 for 256, 192, 128, 64 weight rows; 192 with
+// bm 256 only, 64 with bm 128 only, bm 192 with 256 only), on how many stages, and how many slices of K suit a product of many rows; tn = 0:
 // none (a K the kernel does not take). A model of the time, fitted to this machine over 128 to 8,192
 // rows and seven weight shapes, every tile and 1 to 8 slices measured (what it picks is within 1 % of
 // the fastest on average and within 7 % on every shape whose consumer can add slices):
 //   - a K-step of 64 takes a block alone on its CU the first figure below with few CUs busy and the
 //     second with all 256 (clocks, L2), in between in proportion:
 //         128x128 0.46 .. 0.78 us    128x256 0.70 .. 1.08    256x128 0.66 .. 1.08
-//         256x192 0.89 .. 1.30       256x256 1.03 .. 1.58
+//         256x192 0.89 .. 1.30       256x256 1.03 .. 1.58       192x256 0.95 .. 1.25
+//     (192 activation rows suit portions a little over a power of two, a prompt's beside the tokens of other requests:
+//     gate and up of 520 rows 57 us on the 256x256 tile and 51, 1,536 rows 117 and 104, 2,300 rows 174 and 149. K in one
+//     piece and rows of at most 4,096 only: with 8,192 a step took 1.13 us on 24 CUs where 2,048 took 0.85);
 //   - a tile of 128 rows by 64 weight rows on four waves and four stages takes 0.35 .. 0.50 us a step: with at
 //     most 128 rows (one tile down the rows) it makes twice the blocks of the 128x128 tile out of a weight
 //     that is streamed once, and a block's share of the weights is what bounds such a product (measured at
@@ -1088,11 +1091,12 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
     for (int slices : {1, 2, 3, 4, 6, 8}) {                 // (3 and 6: a K of 27 or 9 times 256 has no other cut)
         if (fixed_slices > 0 && slices != fixed_slices) continue;
         if (k % (128 * slices) != 0 || (slices > 1 && k / slices < 512)) continue;
-        for (int bm = 256; bm >= 128; bm /= 2) {
+        for (int bm = 256; bm >= 128; bm -= 64) {
             const int tiles_m = (m + bm - 1) / bm;
             for (int tn = 4; tn >= 1; --tn) {
                 if (tn == 3 && bm != 256) continue;
                 if (tn == 1 && bm != 128) continue;
+                if (bm == 192 && (tn != 4 || slices > 1 || k > 4096)) continue;
                 const int bn = 64 * tn;
                 for (int stages = 2; stages <= 4; stages += 2) {
                     // four stages: the 128x128 tile and the 128x64 one (which runs on four only), K-steps in fours
@@ -1104,7 +1108,8 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
                     const long long per_round = (blocks + rounds - 1) / rounds;
                     const double cus = (double)std::min<long long>(256, per_round);
                     double few, all;
-                    if (bm == 128 && tn == 1) few = 0.35, all = 0.50;
+                    if (bm == 192) few = 0.95, all = 1.25;
+                    else if (bm == 128 && tn == 1) few = 0.35, all = 0.50;
                     else if (bm == 128 && tn == 2) few = stages == 4 ? 0.33 : 0.46, all = stages == 4 ? 0.53 : 0.78;
                     else if (bm == 128) few = 0.70, all = 1.08;
                     else if (tn == 2) few = 0.66, all = 1.08;
@@ -1133,7 +1138,7 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
 }
 
 // `slices` must leave every slice a multiple of 128 of K (dma_tile_takes(m, n, k / slices) and k % slices == 0).
-// bm: 256 or 128 activation rows to a tile; tn: 4, 3 (bm 256 only), 2 or 1 (bm 128 only) for 256, 192, 128 or 64 weight rows.
+// bm: 256, 192 or 128 activation rows to a tile; tn: 4, 3 (bm 256 only), 2 or 1 (bm 128 only) for 256, 192, 128 or 64 weight rows.
 template <typename TOut>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                       int bm, int tn, int slices, hipStream_t s, int stages = 2) {
@@ -1153,6 +1158,8 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
         k_gemm_bf16_dma<TOut, 2, 1, 4, 2, 4><<<grid, 512, 0, s>>>(x, w, bias, y, m, n, k, k / slices, tiles_m, tiles_n, epilogue);
     else if (bm == 128)
         DMA_GO(2, 1, 4);
+    else if (bm == 192)   // 256 wide: eight waves of 96 rows by 64
+        DMA_GO(3, 2, 4);
     else if (tn == 4)     // 256 wide: eight waves
         DMA_GO(4, 2, 4);
     else if (tn == 3)     // 192 wide: eight waves of 64 rows by 96
@@ -1788,6 +1795,9 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
         if ((force == 258 || force == 262 || force == 263) && k % slices == 0 && dma_tile_takes(m, n, k / slices) &&
             dma_tile_takes(m, n, k))
             return launch_dma<TOut>(x, w, bias, y, m, n, k, epilogue, 256, force == 258 ? 4 : force - 260, slices, s);
+        // 558: 192 activation rows to a tile, 256 wide
+        if (force == 558 && k % slices == 0 && dma_tile_takes(m, n, k / slices) && dma_tile_takes(m, n, k))
+            return launch_dma<TOut>(x, w, bias, y, m, n, k, epilogue, 192, 4, slices, s);
         // 358, 352: 128 activation rows to a tile, 256 and 128 wide
         if ((force == 358 || force == 352) && k % slices == 0 && dma_tile_takes(m, n, k / slices) && dma_tile_takes(m, n, k))
             return launch_dma<TOut>(x, w, bias, y, m, n, k, epilogue, 128, force == 358 ? 4 : 2, slices, s);
@@ -1811,7 +1821,7 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
 // that each kernel can be met at any shape: 1 the K-split kernel, 2, 4 or 8 the shared-activation
 // kernel with that many waves, 256 the 256x256 tile with register staging, 258 / 263 / 262 the tile
 // with loads straight into LDS at 256 rows by 256 / 192 / 128, 358 / 352 the same at 128 rows by
-// 256 / 128, 452 the 128 by 128 tile on four stages, 351 / 451 the 128 by 64 tile on two / four stages;
+// 256 / 128, 558 at 192 rows by 256, 452 the 128 by 128 tile on four stages, 351 / 451 the 128 by 64 tile on two / four stages;
 // with a variant, any number of K slices is taken.
 static int gemm_variant(const void* x, const void* w, const float* bias, void* y, int dtype, int out_dtype,
                         int m, int n, int k, Epilogue epilogue, int slices, int variant, imparo_stream stream) {
