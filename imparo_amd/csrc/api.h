@@ -268,6 +268,16 @@ int imparo_head_prepare(float* rows, int ld, int off, int n_tokens, int heads, i
 int imparo_gated_group_norm(const float* x, const float* gate, int gate_ld, int gate_off, const float* w, void* out,
                             int out_dtype, int n_tokens, int width, int groups, float eps, int gate_first, int gate_act,
                             imparo_stream stream);
+// One token a request of the delta rule with a decay a channel, from the projections' rows (q | k | v .. b, and steps |
+// gate) to sigmoid(gate) * rms_norm(o) * norm: causal conv with SiLU of q, k and v and the shift of their history (conv
+// [n_slots, taps - 1, channels]), unit length of q (times q_scale) and k, the state's step, o. Takes heads of 128 by 128,
+// one or two a query/key head, and up to four taps. slot [n_rows]: distinct.
+int imparo_channel_delta_step_takes(int heads, int kv_heads, int dim, int vdim, int taps);
+int imparo_channel_delta_step(const float* rows, int ld, int beta_off, const float* steps, int steps_ld, int gate_off,
+                              const float* conv_w, float* conv, int taps, const float* step_bias, const float* rate,
+                              float* state, int n_slots, const int32_t* slot, const float* norm, void* out, int out_dtype,
+                              int n_rows, int heads, int kv_heads, int dim, int vdim, float unit_eps, float q_scale, float eps,
+                              imparo_stream stream);
 // out[t] = factor (rms_norm(a[t]) wa + rms_norm(b[t]) wb); a and b float32 [slices, tokens, width], added in order.
 int imparo_normed_sum(const float* a, int a_slices, const float* wa, const float* b, int b_slices, const float* wb,
                       float* out, int n_tokens, int width, float eps, float factor, imparo_stream stream);

@@ -1066,6 +1066,186 @@ extern "C" int imparo_gated_row_add(float* out, const float* y, int y_slices, co
     return launch_status();
 }
 
+// ---------------------------------------------------------------- one token of the channel delta rule, whole
+// A decode step of the delta rule with a decay a channel, from the projections' rows to the rows the output projection
+// reads: conv and SiLU of q, k and v with the shift of their history, unit length, the decays, the state's step, and the
+// norm and gate of the heads behind it, one launch where there were four (the conv, the heads' preparation, the walk, the
+// norm: 19.7 us in a step of 4 requests with 8 heads, each launch a trip through memory to the next; now 9.3). Heads of 128 by
+// 128 and up to four taps. A block has one request's query/key head and the PER heads that share it, so that no other block
+// reads the history it shifts; its 1,024 threads keep a piece of four rows by four columns of each head's state, asked for
+// before anything else. Bound by the state's trips to memory and five meetings of the block between them.
+#define CDS_DIM 128
+#define CDS_MAX_TAPS 4
+struct ChannelStepArgs {
+    const float* rows; int ld, beta_off;         // q | k | v | .., b from beta_off on
+    const float* steps; int steps_ld, gate_off;  // the decays' raw steps, the gate from gate_off on
+    const float* conv_w; float* conv; int taps;  // [channels, taps], [slots, taps - 1, channels]
+    const float* step_bias; const float* rate;   // [heads * dim], [heads]
+    float* state;                                // [slots, heads, dim, vdim]
+    const int32_t* slot;
+    const float* norm;                           // [heads * vdim]
+    int heads, kv_heads;
+    float unit_eps, q_scale, eps;
+};
+
+__device__ __forceinline__ float cds_halves(float v) {       // the sum of the two lanes 32 apart
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+template <typename TOut, int PER>
+__global__ __launch_bounds__(1024) void k_channel_delta_step(const ChannelStepArgs A, TOut* __restrict__ out) {
+    constexpr int D = CDS_DIM, WAVES = 16;
+    __shared__ __attribute__((aligned(16))) float sq[D], sk[D], sv[PER][D], sg[PER][D], su[PER][D];
+    __shared__ __attribute__((aligned(16))) float red[PER][WAVES][D];
+    __shared__ float squares[4], beta[PER], part[2 * PER];
+    const int r = blockIdx.x, kh = blockIdx.y, h0 = kh * PER;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c4 = (tid & 31) * 4, k0 = (tid >> 5) * 4;      // this thread's columns and rows of a head's state
+    const int H = A.heads, Hk = A.kv_heads, channels = 2 * Hk * D + H * D;
+    const size_t at = A.slot[r];
+    float* S_at = A.state + (at * H + h0) * (D * D);
+    float4 S[PER][4];
+#pragma unroll
+    for (int p = 0; p < PER; ++p)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) S[p][j] = *reinterpret_cast<const float4*>(S_at + ((size_t)p * D + k0 + j) * D + c4);
+    const float* row = A.rows + (size_t)r * A.ld;
+    const float* step = A.steps + (size_t)r * A.steps_ld;
+    const bool finishes = tid < PER * D;                     // one output
+    const float gate = finishes ? step[A.gate_off + h0 * D + tid] : 0.f, norm = finishes ? A.norm[h0 * D + tid] : 0.f;
+    if (tid < (2 + PER) * D) {                               // one channel: 128 of q, 128 of k, the heads' values
+        const int ch = tid < D ? kh * D + tid : tid < 2 * D ? Hk * D + kh * D + (tid - D) : 2 * Hk * D + h0 * D + (tid - 2 * D);
+        const int history = A.taps - 1;
+        float* hist = A.conv + at * (size_t)history * channels + ch;
+        float old[CDS_MAX_TAPS - 1], w[CDS_MAX_TAPS];
+#pragma unroll
+        for (int i = 0; i < CDS_MAX_TAPS - 1; ++i) old[i] = i < history ? hist[(size_t)i * channels] : 0.f;
+#pragma unroll
+        for (int i = 0; i < CDS_MAX_TAPS; ++i) w[i] = i < A.taps ? A.conv_w[(size_t)ch * A.taps + i] : 0.f;
+        const float now = row[ch];
+        float acc = 0.f, last = 0.f;
+#pragma unroll
+        for (int i = 0; i < CDS_MAX_TAPS; ++i) {
+            if (i < history) acc += w[i] * old[i < CDS_MAX_TAPS - 1 ? i : 0];
+            last = i == history ? w[i] : last;
+        }
+        acc += last * now;
+#pragma unroll
+        for (int i = 0; i < CDS_MAX_TAPS - 1; ++i)
+            if (i < history) hist[(size_t)i * channels] = i + 1 < history ? old[i + 1 < CDS_MAX_TAPS - 1 ? i + 1 : 0] : now;
+        const float y = ds_silu(acc);
+        if (tid < 2 * D) {
+            (tid < D ? sq : sk)[tid & (D - 1)] = y;
+            const float ss = wave_sum(y * y);                // (whole waves: a head's 128 channels are two)
+            if (lane == 0) squares[wave] = ss;
+        } else {
+            sv[(tid - 2 * D) / D][(tid - 2 * D) & (D - 1)] = y;
+        }
+    } else if (tid >= 1024 - PER * D) {                      // one decay a state row (other waves than the channels')
+        const int i = tid - (1024 - PER * D);
+        sg[i / D][i & (D - 1)] = expf(-A.rate[h0 + i / D] * ds_softplus(step[h0 * D + i] + A.step_bias[h0 * D + i]));
+        if (i < PER) beta[i] = ds_sigmoid(row[A.beta_off + h0 + i]);
+    }
+    __syncthreads();
+    const float fq = A.q_scale * (1.0f / sqrtf(squares[0] + squares[1] + A.unit_eps));
+    const float fk = 1.0f / sqrtf(squares[2] + squares[3] + A.unit_eps);
+    float4 kk = *reinterpret_cast<const float4*>(&sk[k0]), qq = *reinterpret_cast<const float4*>(&sq[k0]);
+    const float kj[4] = {kk.x * fk, kk.y * fk, kk.z * fk, kk.w * fk}, qj[4] = {qq.x * fq, qq.y * fq, qq.z * fq, qq.w * fq};
+    // a sum over the state's rows: four a thread, two threads a wave, the waves' through LDS in wave order
+    auto leave = [&](int p, const float (&v)[4]) __attribute__((always_inline)) {
+        const float4 s = make_float4(cds_halves(v[0]), cds_halves(v[1]), cds_halves(v[2]), cds_halves(v[3]));
+        if (lane < 32) *reinterpret_cast<float4*>(&red[p][wave][c4]) = s;
+    };
+    auto gather = [&]() __attribute__((always_inline)) {     // column tid % 128 of head tid / 128
+        float v[WAVES], sum = 0.f;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) v[w] = red[tid / D][w][tid & (D - 1)];
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) sum += v[w];
+        return sum;
+    };
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const float4 g4 = *reinterpret_cast<const float4*>(&sg[p][k0]);
+        const float g[4] = {g4.x, g4.y, g4.z, g4.w};
+        float seen[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            S[p][j] = make_float4(S[p][j].x * g[j], S[p][j].y * g[j], S[p][j].z * g[j], S[p][j].w * g[j]);
+            seen[0] = fmaf(S[p][j].x, kj[j], seen[0]);
+            seen[1] = fmaf(S[p][j].y, kj[j], seen[1]);
+            seen[2] = fmaf(S[p][j].z, kj[j], seen[2]);
+            seen[3] = fmaf(S[p][j].w, kj[j], seen[3]);
+        }
+        leave(p, seen);
+    }
+    __syncthreads();
+    if (finishes) su[tid / D][tid & (D - 1)] = beta[tid / D] * (sv[tid / D][tid & (D - 1)] - gather());
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const float4 u = *reinterpret_cast<const float4*>(&su[p][c4]);
+        float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            S[p][j] = make_float4(fmaf(kj[j], u.x, S[p][j].x), fmaf(kj[j], u.y, S[p][j].y), fmaf(kj[j], u.z, S[p][j].z),
+                                  fmaf(kj[j], u.w, S[p][j].w));
+            o[0] = fmaf(S[p][j].x, qj[j], o[0]);
+            o[1] = fmaf(S[p][j].y, qj[j], o[1]);
+            o[2] = fmaf(S[p][j].z, qj[j], o[2]);
+            o[3] = fmaf(S[p][j].w, qj[j], o[3]);
+            *reinterpret_cast<float4*>(S_at + ((size_t)p * D + k0 + j) * D + c4) = S[p][j];
+        }
+        leave(p, o);
+    }
+    __syncthreads();
+    float y = 0.f;
+    if (finishes) {                                          // (whole waves)
+        y = gather();
+        const float ss = wave_sum(y * y);
+        if (lane == 0) part[wave] = ss;
+    }
+    __syncthreads();
+    if (!finishes) return;
+    const int p = tid / D;
+    const float rs = 1.0f / sqrtf((part[2 * p] + part[2 * p + 1]) / (float)D + A.eps);
+    store_f32<TOut>(out, ((size_t)r * H + h0) * D + tid, y * rs * norm * ds_sigmoid(gate));
+}
+
+// Whether the launch below takes a mixer of these sizes.
+extern "C" int imparo_channel_delta_step_takes(int heads, int kv_heads, int dim, int vdim, int taps) {
+    return dim == CDS_DIM && vdim == CDS_DIM && taps >= 1 && taps <= CDS_MAX_TAPS && kv_heads > 0 &&
+           (heads == kv_heads || heads == 2 * kv_heads);
+}
+
+extern "C" int imparo_channel_delta_step(const float* rows, int ld, int beta_off, const float* steps, int steps_ld, int gate_off,
+                                         const float* conv_w, float* conv, int taps, const float* step_bias, const float* rate,
+                                         float* state, int n_slots, const int32_t* slot, const float* norm, void* out,
+                                         int out_dtype, int n_rows, int heads, int kv_heads, int dim, int vdim, float unit_eps,
+                                         float q_scale, float eps, imparo_stream stream) {
+    if (!rows || !steps || !conv_w || !step_bias || !rate || !state || !slot || !norm || !out || n_rows < 0 || n_slots < 1)
+        return IMPARO_BAD_ARGUMENT;
+    if (!imparo_channel_delta_step_takes(heads, kv_heads, dim, vdim, taps) || (taps > 1 && !conv)) return IMPARO_BAD_ARGUMENT;
+    if (kv_heads > 65535 || beta_off < 0 || gate_off < heads * dim || ld < (2 * kv_heads + heads) * CDS_DIM ||
+        ld < beta_off + heads || steps_ld < gate_off + heads * vdim || ((uintptr_t)state & 15))
+        return IMPARO_BAD_ARGUMENT;
+    if (out_dtype != IMPARO_F32 && out_dtype != IMPARO_BF16) return IMPARO_BAD_ARGUMENT;
+    if (n_rows == 0) return IMPARO_OK;
+    const ChannelStepArgs a{rows, ld, beta_off, steps, steps_ld, gate_off, conv_w, conv, taps, step_bias, rate,
+                            state, slot, norm, heads, kv_heads, unit_eps, q_scale, eps};
+    const dim3 grid((unsigned)n_rows, (unsigned)kv_heads);
+    hipStream_t s = (hipStream_t)stream;
+    if (heads == kv_heads) {
+        if (out_dtype == IMPARO_BF16) k_channel_delta_step<bf16_t, 1><<<grid, 1024, 0, s>>>(a, (bf16_t*)out);
+        else k_channel_delta_step<float, 1><<<grid, 1024, 0, s>>>(a, (float*)out);
+    } else {
+        if (out_dtype == IMPARO_BF16) k_channel_delta_step<bf16_t, 2><<<grid, 1024, 0, s>>>(a, (bf16_t*)out);
+        else k_channel_delta_step<float, 2><<<grid, 1024, 0, s>>>(a, (float*)out);
+    }
+    return launch_status();
+}
+
 int imparo_load_code_decay_scan() {
     hipFuncAttributes attributes;
     return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_decay_carry)) == hipSuccess

@@ -115,6 +115,8 @@ _SIGNATURES = {
     "imparo_delta_chunk_tokens": [],
     "imparo_delta_chunk_max_dim": [],
     "imparo_head_prepare": [P, I, I, I, I, I, I, F, P, I, I, P, I, F, F, P],
+    "imparo_channel_delta_step_takes": [I, I, I, I, I],
+    "imparo_channel_delta_step": [P, I, I, P, I, I, P, P, I, P, P, P, I, P, P, P, I, I, I, I, I, I, F, F, F, P],
     "imparo_gated_group_norm": [P, P, I, I, P, P, I, I, I, I, F, I, I, P],
     "imparo_normed_sum": [P, I, P, P, I, P, P, I, I, F, F, P],
     "imparo_gated_row_add": [P, P, I, P, I, I, I, I, P],

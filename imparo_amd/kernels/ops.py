@@ -1488,6 +1488,37 @@ def channel_delta_scan(q: torch.Tensor, q_off: int, q_div: int, k: torch.Tensor,
     return out
 
 
+def channel_delta_step_takes(heads: int, kv_heads: int, dim: int, vdim: int, taps: int) -> bool:
+    """Whether channel_delta_step takes a mixer of these sizes."""
+    return bool(library().imparo_channel_delta_step_takes(int(heads), int(kv_heads), int(dim), int(vdim), int(taps)))
+
+
+def channel_delta_step(rows: torch.Tensor, beta_off: int, steps: torch.Tensor, gate_off: int, conv_weight: torch.Tensor,
+                       conv_state: Optional[torch.Tensor], step_bias: torch.Tensor, rate: torch.Tensor, state: torch.Tensor,
+                       slot: torch.Tensor, norm: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, dim: int,
+                       vdim: int, unit_eps: float, q_scale: float, eps: float) -> torch.Tensor:
+    """causal_conv (with SiLU), head_prepare, channel_delta_scan and gated_group_norm in one launch, for rows of one token
+    each (row r of `rows` is the token of the request with slot[r]): rows hold q | k | v and, from beta_off on, b; steps
+    hold the decays' raw steps and, from gate_off on, the gate, whose sigmoid multiplies the normed heads."""
+    n, ld = rows.shape
+    channels, taps = conv_weight.shape
+    n_slots = state.shape[0]
+    if not channel_delta_step_takes(heads, kv_heads, dim, vdim, taps) or channels != (2 * kv_heads + heads) * dim:
+        raise KernelArgumentError("channel_delta_step: heads of 128 by 128, one or two a query/key head, and up to four taps")
+    if ld < channels or ld < beta_off + heads or steps.shape[0] != n or gate_off < heads * dim or steps.shape[1] < gate_off + heads * vdim:
+        raise KernelArgumentError("channel_delta_step: the projections' rows do not hold what the mixer reads")
+    _check(library().imparo_channel_delta_step(
+        _dev(rows, "projected rows", torch.float32), ld, int(beta_off), _dev(steps, "steps", torch.float32), steps.shape[1],
+        int(gate_off), _dev(conv_weight, "conv weight", torch.float32),
+        _dev(conv_state, "conv state", torch.float32, (n_slots, taps - 1, channels)), taps,
+        _dev(step_bias, "step bias", torch.float32, (heads * dim,)), _dev(rate, "rate", torch.float32, (heads,)),
+        _dev(state, "state", torch.float32, (n_slots, heads, dim, vdim)), n_slots, _dev(slot, "slot", torch.int32, (n,)),
+        _dev(norm, "norm weight", torch.float32, (heads * vdim,)), _dev(out, "normed heads", None, (n, heads * vdim)),
+        _code(out, "normed heads"), n, heads, kv_heads, dim, vdim, float(unit_eps), float(q_scale), float(eps), _stream()),
+        "channel_delta_step")
+    return out
+
+
 def silu_columns(rows: torch.Tensor, off: int, n: int) -> torch.Tensor:
     """SiLU in place on columns off .. off + n - 1 of float32 rows."""
     if off < 0 or n < 1 or off + n > rows.shape[1]:

@@ -135,6 +135,12 @@ class ChannelDelta:
         rows = self.proj(ctx, h, torch.float32, "delta_rows", alias="mixer_in")              # q k v | b
         low = self.low(ctx, h, self.high.in_dtype, "delta_low")
         steps = self.high(ctx, low, torch.float32, "delta_steps")                            # decays' steps | gate
+        gated = ctx.workspace.get("delta_gated", (T, H * dv), self.out.in_dtype, alias="mixer_mid")
+        if ctx.max_seg_len == 1 and ops.channel_delta_step_takes(H, Hk, dk, dv, self.taps):
+            # a decode step: everything between the projections in one launch
+            ops.channel_delta_step(rows, C, steps, H * dk, self.conv_weight, state.get("conv"), self.dt_bias, self.rate,
+                                   state["state"], ctx.slot, self.norm, gated, H, Hk, dk, dv, UNIT_EPS, float(dk) ** -0.5, self.eps)
+            return self.out(ctx, gated, torch.float32, "mixer_out", sliced_ok=True, into=ctx.stream)
         qkv = ctx.workspace.get("delta_qkv", (T, C), torch.float32)
         ops.causal_conv(rows, C, self.conv_weight, None, state.get("conv"), ctx.row_of_token, ctx.seg_start,
                         ctx.seg_len, ctx.slot, qkv, silu=True, single_tokens=ctx.max_seg_len == 1)
@@ -150,7 +156,6 @@ class ChannelDelta:
         ops.channel_delta_scan(qkv, 0, H // Hk, qkv, Hk * dk, H // Hk, qkv, 2 * Hk * dk, steps, 0, self.dt_bias, self.rate,
                                rows, C, state["state"], ctx.seg_start, ctx.seg_len, ctx.slot, o, H, dk, dv,
                                chunk_tokens=chunk_tokens, max_chunks=max_chunks, scratch=scratch)
-        gated = ctx.workspace.get("delta_gated", (T, H * dv), self.out.in_dtype, alias="mixer_mid")
         ops.gated_group_norm(o, steps, H * dk, self.norm, H, self.eps, gated, gate_first=False, gate_act="sigmoid")
         return self.out(ctx, gated, torch.float32, "mixer_out", sliced_ok=True, into=ctx.stream)
 
