@@ -739,16 +739,17 @@ __global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__
 }
 
 // Few rows an expert (a decode step): a block takes RT tiles of 16 weight rows of one expert and up to 16 slots. A tile is
-// the M side of 16x16x32 products; K is cut in runs of 64 over the block's waves, U neighbouring ones a wave and round, and
-// everything a wave needs is asked for at once, from memory straight into the operand registers, as in decode_rows.hip
+// the M side of 16x16x32 products; K is cut in four neighbouring parts over the block's waves, walked in runs of 64, U of
+// them a round, and everything a round needs is asked for at once, from memory straight into the operand registers, as in decode_rows.hip
 // (what bounds it is reading the experts' matrices and the trips to memory behind one another: the tile list, then the
 // weights and the slots' tokens, whose rows come last). A lane takes 16 consecutive k of its row, so that four lanes read
 // a row's 128 bytes side by side; the slots' rows are read with the same k order, which is all a dot product asks for.
 // The waves' partial sums meet in LDS and are added in wave order.
 // GATED: half of a block's tiles are gate rows, the other half the up rows that belong to them, 32 rows further on.
-// 8 tokens, 4 of 8 experts and a shared one: gate and up, 1,536 rows by 1,024 an expert, 9.1 us (two runs a wave at a time,
-// the blocks unevenly over the XCDs: 12.0), the way back, 1,024 by 768, 6.1 (6.3); one token 6.3 and 4.9 (7.5 and 4.7).
-#define MOE_ROWS_WAVES 8
+// 8 tokens, 4 of 8 experts and a shared one: gate and up, 1,536 rows by 1,024 an expert, 10.1 us (two runs a wave at a time,
+// the blocks unevenly over the XCDs: 12.0), the way back, 1,024 by 768, 5.9 (6.3); one token 6.5 and 4.7 (7.5 and 4.7). With
+// eight waves of two runs 9.1, but sums in another order, which turn a router's near ties behind them.
+#define MOE_ROWS_WAVES 4
 template <typename TOut, bool GATED, int RT, int U>
 __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const bf16_t* __restrict__ A, int a_ld, int gather_div,
                                                          const int32_t* __restrict__ entry_of_slot,
@@ -762,7 +763,7 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     extern __shared__ float4 moe_part[];                 // [waves][RT][WAVE]
     // The tiles that hold slots come first in the grid, so that the XCDs, which take its blocks in turn, have equally many of
     // them (9 tiles of 12 by 24 blocks, tile after tile along the grid: 36 on two XCDs of 32 CUs and 24 on the others, 12.0 us
-    // where this way it is 9.1).
+    // where this way it is 10.1).
     const int32_t* last = tiles + 3 * (max_tiles - 1);
     const int n_tiles = last[0] < 0 && last[2] == MOE_COUNTED ? min(last[1], max_tiles) : max_tiles;
     const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;
@@ -772,7 +773,7 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     if (expert < 0) return;
     const int row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
     const int n0 = (int)(block - (unsigned)tile * across) * 16 * GROUPS;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
     const int slot = row0 + min(c, rows - 1);
     const int entry = entry_of_slot ? entry_of_slot[slot] : 0;
@@ -782,7 +783,8 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
         const int f = n0 + (t % GROUPS) * 16 + c;
         wrow[t] = W + ((size_t)expert * N + (GATED ? (f >> 5) * 64 + (f & 31) + (t / GROUPS) * 32 : min(f, N - 1))) * K;
     }
-    const int runs = (K + 63) / 64;
+    const int runs = (K + 63) / 64, a_wave = (runs + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES;
+    const int run_lo = wave * a_wave, run_hi = min(runs, run_lo + a_wave);
     u32x4 w[RT][U][2], x[U][2];
     // (no load under a branch: what lies past K is read again from inside the row, and its weights count as zeros)
     auto k_of = [&](int run, int h) { return min(min(run, runs - 1) * 64 + g * 16 + h * 8, K - 8); };
@@ -795,7 +797,7 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
                 for (int h = 0; h < 2; ++h) w[t][u][h] = *reinterpret_cast<const u32x4*>(wrow[t] + k_of(first + u, h));
         __builtin_amdgcn_sched_barrier(0);
     };
-    ask_weights(wave * U);
+    ask_weights(run_lo);
     const bf16_t* arow = A + (size_t)(gather_div ? entry / gather_div : slot) * a_ld;
     auto ask_rows = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
@@ -804,18 +806,18 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
             for (int h = 0; h < 2; ++h) x[u][h] = *reinterpret_cast<const u32x4*>(arow + k_of(first + u, h));
         __builtin_amdgcn_sched_barrier(0);
     };
-    ask_rows(wave * U);
+    ask_rows(run_lo);
     const float limit = GATED && gate.limits ? gate.limits[expert] : 0.f;
     const float sw = GATED ? moe_slot_weight(gate, entry_of_slot, slot) : 1.f;
     f32x4 acc[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int first = wave * U; first < runs;) {
+    for (int first = run_lo; first < run_hi;) {
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if (first + u >= runs) continue;
+                if (first + u >= run_hi) continue;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     const bool in = (first + u) * 64 + g * 16 + h * 8 < K;
@@ -824,8 +826,8 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
                                                                      acc[t], 0, 0, 0);
                 }
             }
-        first += waves * U;
-        if (first < runs) {
+        first += U;
+        if (first < run_hi) {
             ask_weights(first);
             ask_rows(first);
         }
@@ -836,14 +838,14 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     auto total = [&](int t, float (&v)[4]) __attribute__((always_inline)) {
         float4 p[MOE_ROWS_WAVES];
 #pragma unroll
-        for (int q = 0; q < MOE_ROWS_WAVES; ++q) p[q] = moe_part[(min(q, waves - 1) * RT + t) * WAVE + lane];
+        for (int q = 0; q < MOE_ROWS_WAVES; ++q) p[q] = moe_part[(q * RT + t) * WAVE + lane];
         v[0] = p[0].x, v[1] = p[0].y, v[2] = p[0].z, v[3] = p[0].w;
 #pragma unroll
         for (int q = 1; q < MOE_ROWS_WAVES; ++q)
-            if (q < waves) v[0] += p[q].x, v[1] += p[q].y, v[2] += p[q].z, v[3] += p[q].w;
+            v[0] += p[q].x, v[1] += p[q].y, v[2] += p[q].z, v[3] += p[q].w;
     };
     // a lane holds slot c, outputs 4 g + i of a group
-    for (int t = wave; t < GROUPS; t += waves) {
+    for (int t = wave; t < GROUPS; t += MOE_ROWS_WAVES) {
         float v[4];
         total(t, v);
         const int n = n0 + t * 16 + 4 * g;
@@ -870,23 +872,22 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
 template <typename TOut, bool GATED>
 static void launch_rows16(const bf16_t* a, int a_ld, int gather_div, const int32_t* entry_of_slot, const bf16_t* w, TOut* out,
                           const int32_t* tiles, int max_tiles, int n, int k, int epi, const MoeGate& gate, hipStream_t s) {
-    const int runs = (k + 63) / 64;
-    const int u = runs <= MOE_ROWS_WAVES ? 1 : runs <= 2 * MOE_ROWS_WAVES ? 2 : 4;
-    const int waves = std::min(MOE_ROWS_WAVES, (runs + u - 1) / u);
+    const int a_wave = ((k + 63) / 64 + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES, u = std::min(a_wave, 4);
     const long long all = (long long)std::max(1, max_tiles - 1) * ((n + 15) / 16);
-    const int rt = GATED ? (all <= 512 ? 2 : 4) : (all <= 1024 ? 1 : 4);
+    const int rt = GATED ? (all <= 1024 ? 2 : 4) : (all <= 1024 ? 1 : 4);
     const int outputs = 16 * (GATED ? rt / 2 : rt), columns = GATED ? n / 2 : n;
     const int across = (columns + outputs - 1) / outputs;
     const long long blocks = (long long)max_tiles * across, row = std::min<long long>(blocks, 1 << 22);
     const dim3 grid((unsigned)row, (unsigned)((blocks + row - 1) / row));    // (a launch holds fewer than 2^32 threads along x)
-    const size_t lds = (size_t)waves * rt * WAVE * sizeof(float4);
+    const size_t lds = (size_t)MOE_ROWS_WAVES * rt * WAVE * sizeof(float4);
 #define ROWS16_U(RT, U)                                                                                              \
-    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, waves * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles, \
+    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, MOE_ROWS_WAVES * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles, \
                                                                       max_tiles, across, n, k, epi, gate)
 #define ROWS16_GO(RT)                                                                                                \
     do {                                                                                                             \
         if (u == 1) ROWS16_U(RT, 1);                                                                                 \
         else if (u == 2) ROWS16_U(RT, 2);                                                                            \
+        else if (u == 3) ROWS16_U(RT, 3);                                                                            \
         else ROWS16_U(RT, 4);                                                                                        \
     } while (0)
     if constexpr (!GATED) {
