@@ -70,7 +70,7 @@ template <typename TOut> __device__ __forceinline__ void rows_store(TOut* dst, c
 
 // RB: weight rows of a tile, 16 or 8 (the other lanes ask for nothing; RT 1). CH: chunks of 128 of K that a wave has in
 // flight at once. RAGGED: K is no multiple of 128, or not all slices are alike: addresses are clamped into the row and
-// weights beyond K count as zeros. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per) into
+// what lies beyond K counts as zeros. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per) into
 // Y + y * M * N and the consumer adds the slices.
 template <typename TOut, int RB, int RT, int CH, int EPI, bool RAGGED>
 __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
@@ -153,7 +153,8 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                 if (first + j * waves >= n_chunks) continue;
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    if (RAGGED && (first + j * waves) * 128 + s * 32 + g * 8 >= K) w[t][j][s].u = make_uint4(0u, 0u, 0u, 0u);
+                    if (RAGGED && (first + j * waves) * 128 + s * 32 + g * 8 >= K)
+                        w[t][j][s].u = x[j][s].u = make_uint4(0u, 0u, 0u, 0u);       // (both: zero times infinity is none)
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][j][s].v, x[j][s].v, acc[t], 0, 0, 0);
                 }
             }

@@ -1379,8 +1379,9 @@ __global__ __launch_bounds__(512) void k_in_proj_conv_decode(
         for (int j = 0; j < CH; ++j) {
             if (first + j * waves >= n_chunks) continue;
 #pragma unroll
-            for (int s2 = 0; s2 < 4; ++s2) {             // (weights beyond K count as zeros)
+            for (int s2 = 0; s2 < 4; ++s2) {             // (what lies beyond K counts as zeros: activations too, which may be infinite)
                 const bool beyond = (first + j * waves) * 128 + s2 * 32 + g * 8 >= K;
+                x[j][s2].u = zero_if(beyond, x[j][s2].u);
                 w0[j][s2].u = zero_if(beyond, w0[j][s2].u);
                 w1[j][s2].u = zero_if(beyond, w1[j][s2].u);
                 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0[j][s2].v, x[j][s2].v, acc0, 0, 0, 0);

@@ -1,4 +1,6 @@
 """Products of at most 16 rows at the edges of how they are shared out: tiles a block, chunks of K a wave, rounds, ragged K."""
+import math
+
 import pytest
 import torch
 
@@ -113,3 +115,31 @@ def test_float32_few_rows_are_the_many_rows_bits(m, n, k):
         ops.gemm(x, w, many, bias=b, swiglu=True)
         ops.gemm(x[:m].contiguous(), w, few, bias=b, swiglu=True)
         assert torch.equal(few, many[:m])
+
+
+# K that is no multiple of 128: the last eight activations are what a chunk would read again past K
+@pytest.mark.parametrize("k", [8, 24, 136, 392, 1032, 1288, 2312, 5000])
+def test_an_infinite_last_activation_stays_one(k):
+    m, n = 3, 48
+    x, w = rnd(m, k, seed=1).bfloat16(), rnd(n, k, seed=2, scale=0.1).bfloat16()
+    x[1, k - 1] = math.inf
+    want = (w[:, k - 1].float().sign() * math.inf).to(DEV)
+    finite = x.clone()
+    finite[1, k - 1] = 0.0
+    xg, fg, wg = x.to(DEV), finite.to(DEV), w.to(DEV)
+    out, plain, rows = (torch.empty(m, n, device=DEV) for _ in range(3))
+    ops.gemm(fg, wg, plain)
+    ops.gemm(xg, wg, out)
+    ops.rows_gemm(xg, wg, out=rows)
+    stream, ssq = torch.zeros(m, n, device=DEV), torch.empty(ops.rows_parts(n), 16, device=DEV)
+    ops.rows_gemm(xg, wg, into=stream, ssq_out=ssq)
+    for y in (out, rows, stream):
+        assert torch.equal(y[1], want)
+        assert torch.equal(y[[0, 2]], plain[[0, 2]]) or y is stream
+    # the conv's input projection: B, C and x of the row are infinite, one tap of 1 on the token itself
+    e = n // 3
+    state, slot = torch.zeros(m, 1, e, device=DEV), torch.arange(m, device=DEV, dtype=torch.int32)
+    conv, taps = torch.empty(m, e, device=DEV), torch.tensor([[0.0, 1.0]] * e, device=DEV)
+    ops.in_proj_conv_decode(xg, wg, None, taps, None, state, slot, conv)
+    b, c, u = want[:e], want[e:2 * e], want[2 * e:]
+    assert torch.equal(conv[1], c * (b * u)) and bool(conv[[0, 2]].isfinite().all())
