@@ -68,18 +68,19 @@ template <typename TOut> __device__ __forceinline__ void rows_store(TOut* dst, c
         if (n + i < N) store_f32<TOut>(dst, i, v[i]);
 }
 
+// CHAINS: sums that a wave's chunks go into by turns; the chains' sums are added in the order of their first chunks.
 // RB: weight rows of a tile, 16 or 8 (the other lanes ask for nothing; RT 1). CH: chunks of 128 of K that a wave has in
 // flight at once. RAGGED: K is no multiple of 128, or not all slices are alike: addresses are clamped into the row and
 // what lies beyond K counts as zeros. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per) into
 // Y + y * M * N and the consumer adds the slices.
-template <typename TOut, int RB, int RT, int CH, int EPI, bool RAGGED>
+template <typename TOut, int RB, int RT, int CH, int CHAINS, int EPI, bool RAGGED>
 __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     const bf16_t* __restrict__ X, const float* __restrict__ ssq_in, int n_parts, float eps,
     const bf16_t* __restrict__ W, const float* __restrict__ bias, TOut* __restrict__ Y, float* __restrict__ x_io,
     float* __restrict__ ssq_out, bf16_t* __restrict__ weighted_out, const float* __restrict__ weighted_by, int M, int N,
     int K_all, int k_per, Epilogue unit) {
     static_assert(RB == 16 || RT == 1, "half tiles one by one");
-    extern __shared__ float4 red[];                     // [waves][RT][64]
+    extern __shared__ float4 red[];                     // [CHAINS][waves][RT][64]
     __shared__ __attribute__((aligned(16))) float part[ROWS_WAVES * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int r16 = lane & 15, g = lane >> 4;
@@ -142,9 +143,11 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
             if (weighted_by) by[i] = weighted_by[n];
         }
     }
-    f32x4 acc[RT];
+    f32x4 acc[CHAINS][RT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+        for (int t = 0; t < RT; ++t) acc[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int first = wave; first < n_chunks;) {
 #pragma unroll
         for (int t = 0; t < RT; ++t)
@@ -155,26 +158,29 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                 for (int s = 0; s < 4; ++s) {
                     if (RAGGED && (first + j * waves) * 128 + s * 32 + g * 8 >= K)
                         w[t][j][s].u = x[j][s].u = make_uint4(0u, 0u, 0u, 0u);       // (both: zero times infinity is none)
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][j][s].v, x[j][s].v, acc[t], 0, 0, 0);
+                    acc[j % CHAINS][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][j][s].v, x[j][s].v, acc[j % CHAINS][t], 0, 0, 0);
                 }
             }
         first += waves * CH;
         if (first < n_chunks) ask(first);
     }
 #pragma unroll
-    for (int t = 0; t < RT; ++t) red[(wave * RT + t) * 64 + lane] = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+    for (int c = 0; c < CHAINS; ++c)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+            red[((c * waves + wave) * RT + t) * 64 + lane] = make_float4(acc[c][t][0], acc[c][t][1], acc[c][t][2], acc[c][t][3]);
     __syncthreads();
     if (g * 4 >= RB) return;
     // D layout of the 16x16 tile: lane holds column lane % 16 (a token), rows 4 * (lane / 16) + i (weight rows)
     for (int t = wave; t < RT; t += waves) {
-        float4 sums[ROWS_WAVES];
+        float4 sums[CHAINS * ROWS_WAVES];
 #pragma unroll
-        for (int q = 0; q < ROWS_WAVES; ++q) sums[q] = red[(min(q, waves - 1) * RT + t) * 64 + lane];
+        for (int q = 0; q < CHAINS * ROWS_WAVES; ++q) sums[q] = red[(min(q, CHAINS * waves - 1) * RT + t) * 64 + lane];
         const float scale = ssq_in ? rows_scale(part, token, K, eps) : 1.f;
         float v[4] = {sums[0].x, sums[0].y, sums[0].z, sums[0].w};
 #pragma unroll
-        for (int q = 1; q < ROWS_WAVES; ++q)
-            if (q < waves) v[0] += sums[q].x, v[1] += sums[q].y, v[2] += sums[q].z, v[3] += sums[q].w;
+        for (int q = 1; q < CHAINS * ROWS_WAVES; ++q)
+            if (q < CHAINS * waves) v[0] += sums[q].x, v[1] += sums[q].y, v[2] += sums[q].z, v[3] += sums[q].w;
         const int n = n0 + t * 16 + g * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -216,26 +222,22 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     }
 }
 
-// How a product is shared out: `waves` with `ch` chunks of 128 in flight each, as many as there are chunks and no more (a
-// chunk too many is read and thrown away), more than 32 chunks in rounds; `rt` tiles of 16 weight rows a block so that
-// there is a block a CU (1,024 by 1,024, 8 rows: one tile 3.5 us, four 6.2; 9,216 by 1,024: one 7.1, three, which is 192
-// blocks, 6.0; 16,384 by 2,048: one 14.7, four, 256 blocks, 13.0). A weight of more rows than four tiles a CU runs several
-// blocks one after the other on a CU: those of many short rows are then the smallest, whose ends the others' loads cover
-// (65,536 by 1,024, one row: one tile 22 us, four 26), unless there are more activations to share (8 rows: 28 and 25).
+// How a product is shared out: as many waves as there are chunks, eight at most, with `ch` chunks of 128 in flight each;
+// `rt` tiles of 16 weight rows a block so that there is a block a CU (1,024 by 1,024, 8 rows: one tile 3.5 us, four 6.2; 9,216
+// by 1,024: one 7.1, three, which is 192 blocks, 6.0; 16,384 by 2,048: one 14.7, four, 256 blocks, 13.0). A weight of more rows
+// than four tiles a CU runs several blocks one after the other on a CU: those of many short rows are then the smallest, whose
+// ends the others' loads cover (65,536 by 1,024, one row: one tile 22 us, four 26), unless there are more activations to share
+// (8 rows: 28 and 25). The more chains a column is summed in, the nearer it is to 64 bits: fewer waves with more chunks each
+// were 1.12e-7 off at K of 1,152, where eight are 8.8e-8, and eight with three chunks in one chain 1.21e-7 at 3,072, in two 1.14e-7.
+// Eight chains up to 16 chunks and sixteen beyond, in this order, are the sums of before there was this kernel.
 struct RowsShape {
-    int waves, ch, rt;
+    int waves, ch, rt, chains;
 };
 static RowsShape rows_shape(int m, int n, int k_per, int slices, bool ragged, int rb) {
     const int chunks = (k_per + 127) / 128;
-    RowsShape sh{ROWS_WAVES, 4, 1};
-    if (chunks <= 8) {
-        sh = {chunks, 1, 1};
-    } else if (chunks <= 24) {
-        const int two = (chunks + 1) / 2, three = (chunks + 2) / 3;
-        sh = two <= ROWS_WAVES && two * 2 - chunks <= three * 3 - chunks ? RowsShape{two, 2, 1} : RowsShape{three, 3, 1};
-    } else if (chunks <= 32) {
-        sh.waves = (chunks + 3) / 4;
-    }
+    RowsShape sh{std::min(chunks, ROWS_WAVES), 4, 1, 1};
+    sh.ch = std::min((chunks + sh.waves - 1) / sh.waves, 4);
+    if (sh.ch > 2 && (rb == 16 ? n < 12288 : chunks > 32)) sh.chains = 2;
     if (rb == 16) {
         const long long tiles = (long long)((n + 15) / 16) * slices;
         const int most = ragged || sh.ch > 2 ? 2 : 4;
@@ -267,17 +269,19 @@ static void rows_launch(const RowsCall& c, hipStream_t s) {
     const bool ragged = c.k % 128 != 0 || c.k >= (1 << 25);      // (offsets inside 64 rows are kept in 32 bits)
     const RowsShape sh = rows_shape(c.m, c.n, std::min(k_per, c.k), c.slices, ragged, RB);
     const dim3 grid((unsigned)((c.n + (long long)RB * sh.rt - 1) / (RB * sh.rt)), (unsigned)((c.k + k_per - 1) / k_per));
-    const size_t lds = (size_t)sh.waves * sh.rt * 64 * sizeof(float4);          // (32 KB at most)
-#define ROWS_GO(RT, CH, RG)                                                                                          \
-    k_rows_gemm<TOut, RB, RT, CH, EPI, RG><<<grid, sh.waves * 64, lds, s>>>(                                           \
+    const size_t lds = (size_t)sh.chains * sh.waves * sh.rt * 64 * sizeof(float4);          // (32 KB at most)
+#define ROWS_GO(RT, CH, CHAINS, RG)                                                                                  \
+    k_rows_gemm<TOut, RB, RT, CH, CHAINS, EPI, RG><<<grid, sh.waves * 64, lds, s>>>(                                   \
         c.x, c.ssq_in, c.n_parts, c.eps, c.w, c.bias, (TOut*)c.y, c.x_io, c.ssq_out, c.weighted_out, c.weighted_by, c.m, \
         c.n, c.k, k_per, c.unit)
 #define ROWS_CH(RT, RG)                                                                                              \
     do {                                                                                                             \
-        if (sh.ch == 1) ROWS_GO(RT, 1, RG);                                                                          \
-        else if (sh.ch == 2) ROWS_GO(RT, 2, RG);                                                                     \
-        else if (sh.ch == 3) ROWS_GO(RT, 3, RG);                                                                     \
-        else ROWS_GO(RT, 4, RG);                                                                                     \
+        if (sh.ch == 1) ROWS_GO(RT, 1, 1, RG);                                                                       \
+        else if (sh.ch == 2) ROWS_GO(RT, 2, 1, RG);                                                                  \
+        else if (sh.ch == 3 && sh.chains == 2) ROWS_GO(RT, 3, 2, RG);                                                \
+        else if (sh.ch == 3) ROWS_GO(RT, 3, 1, RG);                                                                  \
+        else if (sh.chains == 2) ROWS_GO(RT, 4, 2, RG);                                                              \
+        else ROWS_GO(RT, 4, 1, RG);                                                                                  \
     } while (0)
     if constexpr (RB == 16) {
         if (ragged) {
@@ -288,11 +292,11 @@ static void rows_launch(const RowsCall& c, hipStream_t s) {
         } else if (sh.rt == 2) {
             ROWS_CH(2, false);
         } else if (sh.rt == 3) {
-            if (sh.ch == 1) ROWS_GO(3, 1, false);
-            else ROWS_GO(3, 2, false);
+            if (sh.ch == 1) ROWS_GO(3, 1, 1, false);
+            else ROWS_GO(3, 2, 1, false);
         } else {
-            if (sh.ch == 1) ROWS_GO(4, 1, false);
-            else ROWS_GO(4, 2, false);
+            if (sh.ch == 1) ROWS_GO(4, 1, 1, false);
+            else ROWS_GO(4, 2, 1, false);
         }
     } else {
         if (ragged) ROWS_CH(1, true);
@@ -354,7 +358,7 @@ extern "C" int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts,
 // cannot do that).
 int imparo_load_code_decode_rows() {
     hipFuncAttributes attributes;
-    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_rows_gemm<float, 8, 1, 1, ROWS_RESID, false>)) ==
+    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_rows_gemm<float, 8, 1, 1, 1, ROWS_RESID, false>)) ==
                    hipSuccess
                ? IMPARO_OK
                : IMPARO_LAUNCH_FAILED;

@@ -1470,8 +1470,9 @@ static void launch_in_proj_conv(const bf16_t* x, const float* ssq_in, int n_part
                                 const float* in_bias, const float* conv_w, const float* conv_b, float* state,
                                 const int32_t* slot, TOut* out, int m, int e, int k, int taps, hipStream_t s) {
     const unsigned blocks = (unsigned)(e / 8);
-    const int chunks = (k + 127) / 128;                 // as many waves as there are chunks, or pairs of chunks
-    const int waves = chunks <= 8 ? chunks : std::min(8, (chunks + 1) / 2);
+    // (eight waves from eight chunks on, though some have a chunk less than others: the sums' order of before, and nearer to
+    // 64 bits than fewer longer ones)
+    const int chunks = (k + 127) / 128, waves = std::min(chunks, 8);
 #define CONV_GO(CH, HIST)                                                                                              \
     k_in_proj_conv_decode<TOut, CH, HIST><<<blocks, waves * 64, 0, s>>>(x, ssq_in, n_parts, eps, w, in_bias, conv_w, conv_b, \
                                                                    state, slot, out, m, e, k, taps)

@@ -143,3 +143,17 @@ def test_an_infinite_last_activation_stays_one(k):
     ops.in_proj_conv_decode(xg, wg, None, taps, None, state, slot, conv)
     b, c, u = want[:e], want[e:2 * e], want[2 * e:]
     assert torch.equal(conv[1], c * (b * u)) and bool(conv[[0, 2]].isfinite().all())
+
+
+# The root mean square of the errors against 64 bits, in units of the outputs', goes by how many chains of sums a column has
+# and how long they are: eight chains of two chunks of 128 at the most up to K = 2,048 and sixteen beyond measured 8.8e-8,
+# 9.8e-8, 1.02e-7, 1.04e-7, 1.09e-7 and 1.15e-7 here; three to seven waves with longer chains 1.15e-7, 9.9e-8, 1.2e-7, 1.2e-7,
+# 1.2e-7 and 1.35e-7. The limits lie between (16,384 outputs of independent roundings: the figures stray by less than 1 %).
+@pytest.mark.parametrize("k, limit", [(1152, 1.0e-7), (1920, 1.1e-7), (2304, 1.1e-7), (2560, 1.12e-7), (3584, 1.24e-7)])
+def test_sums_stay_as_near_to_64_bits(k, limit):
+    m, n = 16, 1024
+    x, w = rnd(m, k, seed=1).bfloat16().to(DEV), rnd(n, k, seed=2, scale=0.02).bfloat16().to(DEV)
+    out = torch.empty(m, n, device=DEV)
+    ops.rows_gemm(x, w, out=out)
+    want = x.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) < limit
