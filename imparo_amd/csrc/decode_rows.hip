@@ -22,15 +22,19 @@
 // RT, how many waves and chunks a wave: rows_shape. Measured, cold weights, launch behind launch (before: walks along K
 // in steps of 128 to 1,024 with the activations through LDS):
 //
-//   rows, weight (gated unless said)      before      now
-//   1, 9,216 by 1,024, scaled             7.9 us      6.5 us
-//   8, 16,384 by 2,048, scaled            16.0        13.9
-//   1, 65,536 by 1,024, plain             31.4        23.7
-//   8, 65,536 by 2,048, plain             51.8        51.2
-//   1, 1,024 by 4,608, 8 slices           6.0         4.5
-//   8, 2,048 by 8,192, 4 slices           9.6         8.8
-//   8, 3,072 by 2,048, plain              6.4         5.7
-//   8, 2,048 by 2,048, into the stream    5.8         5.4
+//   rows, weight                               before      now
+//   1, 9,216 by 1,024, gated, scaled           8.3 us      6.8 us
+//   8 / 16, 16,384 by 2,048, gated, scaled     17.3 / 17.3 15.4 / 15.9
+//   1, 65,536 by 1,024                         32.7        24.9
+//   8 / 16, 65,536 by 2,048                    55.9 / 57.2 54.0 / 56.0
+//   1, 1,024 by 4,608, 8 slices                6.1         4.5
+//   8 / 16, 2,048 by 8,192, 4 slices           10.2 / 10.5 9.2 / 9.8
+//   8 / 16, 3,072 by 2,048                     6.5 / 7.4   5.9 / 6.4
+//   8 / 16, 2,048 by 2,048, into the stream    5.8 / 6.8   5.4 / 5.9
+//   16, 9,216 by 3,072                         24.6        15.3
+//   8, 12,288 by 4,608                         26.1        23.6
+//   16, 16,384 by 4,096                        41.5        27.6
+//   8, 16,384 by 11,008                        69.0        67.7
 //
 // (a kernel that only reads 8 / 34 / 67 / 134 / 268 MB takes 3.8 / 7.4 / 12.3 / 22 / 48 us).
 #include "common.h"
@@ -52,6 +56,17 @@ union RowFrag {
 #define ROWS_SWIGLU 1
 #define ROWS_RESID 2
 #define ROWS_WAVES 8         // of a block at most
+#define ROWS_TURNED 8192     // from this K on blocks start their walks at different places
+
+// K_KIND
+#define ROWS_WHOLE 0         // K is a multiple of 128, and every wave has as many chunks of it as its rounds ask for
+#define ROWS_UNEVEN 1        // K is a multiple of 128
+#define ROWS_RAGGED 2        // any other K: addresses are clamped into the row, and what a chunk has beyond K counts as zeros
+#define ROWS_HUGE 3          // K from 2^25 on: the same, with 64-bit offsets inside a block's rows
+
+__device__ __forceinline__ uint4 rows_zero_if(bool out, uint4 v) {
+    return make_uint4(out ? 0u : v.x, out ? 0u : v.y, out ? 0u : v.z, out ? 0u : v.w);
+}
 
 // Four results of a token, columns n .. n + 3 of N (n a multiple of 4), in one store where rows keep it aligned
 template <typename TOut> __device__ __forceinline__ void rows_store(TOut* dst, const float (&v)[4], int n, int N, bool whole) {
@@ -70,16 +85,16 @@ template <typename TOut> __device__ __forceinline__ void rows_store(TOut* dst, c
 
 // CHAINS: sums that a wave's chunks go into by turns; the chains' sums are added in the order of their first chunks.
 // RB: weight rows of a tile, 16 or 8 (the other lanes ask for nothing; RT 1). CH: chunks of 128 of K that a wave has in
-// flight at once. RAGGED: K is no multiple of 128, or not all slices are alike: addresses are clamped into the row and
-// what lies beyond K counts as zeros. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per) into
-// Y + y * M * N and the consumer adds the slices.
-template <typename TOut, int RB, int RT, int CH, int CHAINS, int EPI, bool RAGGED>
+// flight at once. SCALED: ssq_in is there. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per)
+// into Y + y * M * N and the consumer adds the slices.
+template <typename TOut, int RB, int RT, int CH, int CHAINS, int EPI, int K_KIND, bool SCALED>
 __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     const bf16_t* __restrict__ X, const float* __restrict__ ssq_in, int n_parts, float eps,
     const bf16_t* __restrict__ W, const float* __restrict__ bias, TOut* __restrict__ Y, float* __restrict__ x_io,
     float* __restrict__ ssq_out, bf16_t* __restrict__ weighted_out, const float* __restrict__ weighted_by, int M, int N,
-    int K_all, int k_per, Epilogue unit) {
+    int K_all, int k_per, int rounds, int turned, Epilogue unit) {
     static_assert(RB == 16 || RT == 1, "half tiles one by one");
+    constexpr bool RAGGED = K_KIND == ROWS_RAGGED || K_KIND == ROWS_HUGE;
     extern __shared__ float4 red[];                     // [CHAINS][waves][RT][64]
     __shared__ __attribute__((aligned(16))) float part[ROWS_WAVES * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
@@ -91,48 +106,62 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     if (blockIdx.y > 0) bias = nullptr;                 // the bias belongs to one slice only
     const int token = min(r16, M - 1);
     const int n_chunks = (K + 127) / 128;
-    // uniform bases and 32-bit offsets inside a block's rows: a load costs no address arithmetic (RAGGED: any K)
-    typedef typename std::conditional<RAGGED, size_t, unsigned>::type Offset;
+    // uniform bases and 32-bit byte offsets inside a block's rows: a load costs next to no address arithmetic
+    typedef typename std::conditional<K_KIND == ROWS_HUGE, size_t, unsigned>::type Offset;
     const bf16_t* xbase = X + k_lo;
     const bf16_t* wbase = W + (size_t)n0 * K_all + k_lo;
-    const Offset xoff = (Offset)token * (unsigned)K_all;
+    const Offset xoff = (Offset)token * (unsigned)K_all * 2u;
     Offset woff[RT];
 #pragma unroll
-    for (int t = 0; t < RT; ++t) woff[t] = (Offset)min(t * 16 + (r16 & (RB - 1)), N - 1 - n0) * (unsigned)K_all;
+    for (int t = 0; t < RT; ++t) woff[t] = (Offset)min(t * 16 + (r16 & (RB - 1)), N - 1 - n0) * (unsigned)K_all * 2u;
     RowFrag x[CH][4], w[RT][CH][4];
     // This wave's chunks are first, first + waves, ...: CH of them a round. No load under a branch (the compiler would wait
     // for every load in flight at the next use of any): past the last chunk the last one again, which no product reads.
+    // A long walk starts at a round that goes by the block's place: rows of a long K lie so far apart that blocks in step keep
+    // asking the same few channels (8 rows of 16,384 by 11,008 82 us in step, 67 so; of 8,192 by 16,384 68 and 52). The
+    // place is hashed, as rounds that follow the row's number undo what the address's own hash does (8,192 by 8,192 41 us).
+    const int turn = waves * CH;
+    int round = (int)__umulhi((unsigned)(n0 / 64) * 2654435761u, (unsigned)turned);      // (no branch in front of the loads)
     auto at = [&](const bf16_t* base, Offset row, int chunk, int s) __attribute__((always_inline)) {
         if constexpr (RAGGED)
-            return reinterpret_cast<const uint4*>(base + row + min(chunk * 128 + s * 32 + g * 8, K - 8));
+            return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base) +
+                                                  (row + (Offset)min(chunk * 128 + s * 32 + g * 8, K - 8) * 2u));
         else
-            return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base + chunk * 128) + (row + g * 8) * 2u + s * 64);
+            return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(base + chunk * 128) + (row + g * 16) + s * 64);
     };
     // (A tile's chunks one after the other: chunk after chunk over all tiles, every block would read the first half of its
     // rows and then the second, at any time half of the memory's channels: 8 rows of 16,384 by 2,048 15.1 us and not 13.9.)
-    auto ask = [&](int first) __attribute__((always_inline)) {
+    auto ask_some = [&](int first, int n) __attribute__((always_inline)) {     // (n: known when this is compiled)
 #pragma unroll
-        for (int j = 0; j < CH; ++j)
+        for (int j = 0; j < n; ++j)
 #pragma unroll
             for (int s = 0; s < 4; ++s) x[j][s].u = *at(xbase, xoff, min(first + j * waves, n_chunks - 1), s);
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
-            for (int j = 0; j < CH; ++j)
+            for (int j = 0; j < n; ++j)
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
                     // (lanes of weight rows beyond RB ask for nothing: their rows of the tile are nobody's)
                     if (RB < 16) w[t][j][s].u = make_uint4(0u, 0u, 0u, 0u);
                     if (RB == 16 || r16 < RB) w[t][j][s].u = *at(wbase, woff[t], min(first + j * waves, n_chunks - 1), s);
                 }
+    };
+    auto ask = [&](int first) __attribute__((always_inline)) {
+        if constexpr (CH > 1 && K_KIND != ROWS_WHOLE) {      // (a wave may have a chunk less than others)
+            if (first + (CH - 1) * waves < n_chunks) ask_some(first, CH);
+            else ask_some(first, CH - 1);
+        } else {
+            ask_some(first, CH);
+        }
         __builtin_amdgcn_sched_barrier(0);
     };
     // the rows' sums of squares first: they are added up while the weights are on their way
     RowsSsq early;
-    if (ssq_in) rows_ssq_ask(early, ssq_in, n_parts, 0);
+    if (SCALED) rows_ssq_ask(early, ssq_in, n_parts, 0);
     __builtin_amdgcn_sched_barrier(0);
-    ask(wave);
-    if (ssq_in) rows_ssq_share(part, early, ssq_in, n_parts);
+    ask(wave + round * turn);
+    if (SCALED) rows_ssq_share(part, early, ssq_in, n_parts);
     // needed when the walk is over: what the finishing lanes add to
     float x_old[4] = {0.f, 0.f, 0.f, 0.f}, by[4] = {0.f, 0.f, 0.f, 0.f};
     if (EPI == ROWS_RESID && wave == 0 && g * 4 < RB && r16 < M) {
@@ -148,22 +177,40 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
         for (int t = 0; t < RT; ++t) acc[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int first = wave; first < n_chunks;) {
+    int left = rounds;                                   // (at least one)
+    do {
+        const int first = wave + round * turn;
+        if constexpr (RAGGED) {                              // what the last steps of 32 have beyond K counts as zeros
 #pragma unroll
-        for (int t = 0; t < RT; ++t)
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                if (first + j * waves >= n_chunks) continue;
+            for (int j = 0; j < CH; ++j)
 #pragma unroll
                 for (int s = 0; s < 4; ++s) {
-                    if (RAGGED && (first + j * waves) * 128 + s * 32 + g * 8 >= K)
-                        w[t][j][s].u = x[j][s].u = make_uint4(0u, 0u, 0u, 0u);       // (both: zero times infinity is none)
-                    acc[j % CHAINS][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][j][s].v, x[j][s].v, acc[j % CHAINS][t], 0, 0, 0);
+                    const int k0 = (first + j * waves) * 128 + s * 32;
+                    if (k0 >= K || k0 + 32 <= K) continue;
+                    x[j][s].u = rows_zero_if(k0 + g * 8 >= K, x[j][s].u);
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) w[t][j][s].u = rows_zero_if(k0 + g * 8 >= K, w[t][j][s].u);
                 }
-            }
-        first += waves * CH;
-        if (first < n_chunks) ask(first);
-    }
+        }
+        auto multiply = [&](int odd) __attribute__((always_inline)) {       // (a wave's chunks by turns into its chains)
+#pragma unroll
+            for (int t = 0; t < RT; ++t)
+#pragma unroll
+                for (int j = 0; j < CH; ++j) {
+                    if (first + j * waves >= n_chunks) continue;
+                    f32x4& sum = acc[(j + odd) % CHAINS][t];
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        if (RAGGED && (first + j * waves) * 128 + s * 32 >= K) continue;
+                        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t][j][s].v, x[j][s].v, sum, 0, 0, 0);
+                    }
+                }
+        };
+        if (CHAINS == 2 && CH % 2 == 1 && (round & 1)) multiply(1);
+        else multiply(0);
+        round = round + 1 == rounds ? 0 : round + 1;
+        if (left > 1 && wave + round * turn < n_chunks) ask(wave + round * turn);
+    } while (--left > 0);
 #pragma unroll
     for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
@@ -176,7 +223,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
         float4 sums[CHAINS * ROWS_WAVES];
 #pragma unroll
         for (int q = 0; q < CHAINS * ROWS_WAVES; ++q) sums[q] = red[(min(q, CHAINS * waves - 1) * RT + t) * 64 + lane];
-        const float scale = ssq_in ? rows_scale(part, token, K, eps) : 1.f;
+        const float scale = SCALED ? rows_scale(part, token, K, eps) : 1.f;
         float v[4] = {sums[0].x, sums[0].y, sums[0].z, sums[0].w};
 #pragma unroll
         for (int q = 1; q < CHAINS * ROWS_WAVES; ++q)
@@ -185,7 +232,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             // each step rounded on its own (no fused multiply-add), so that every epilogue gives the same bits
-            if (ssq_in) v[i] = __fmul_rn(v[i], scale);
+            if (SCALED) v[i] = __fmul_rn(v[i], scale);
             if (bias && n + i < N) v[i] = __fadd_rn(v[i], bias[n + i]);
         }
         const bool live = r16 < M;
@@ -222,27 +269,61 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     }
 }
 
-// How a product is shared out: as many waves as there are chunks, eight at most, with `ch` chunks of 128 in flight each;
-// `rt` tiles of 16 weight rows a block so that there is a block a CU (1,024 by 1,024, 8 rows: one tile 3.5 us, four 6.2; 9,216
-// by 1,024: one 7.1, three, which is 192 blocks, 6.0; 16,384 by 2,048: one 14.7, four, 256 blocks, 13.0). A weight of more rows
-// than four tiles a CU runs several blocks one after the other on a CU: those of many short rows are then the smallest, whose
-// ends the others' loads cover (65,536 by 1,024, one row: one tile 22 us, four 26), unless there are more activations to share
-// (8 rows: 28 and 25). The more chains a column is summed in, the nearer it is to 64 bits: fewer waves with more chunks each
-// were 1.12e-7 off at K of 1,152, where eight are 8.8e-8, and eight with three chunks in one chain 1.21e-7 at 3,072, in two 1.14e-7.
-// Eight chains up to 16 chunks and sixteen beyond, in this order, are the sums of before there was this kernel.
+// How a product is shared out, measured against the kernels before over 2,500 random forms of 1 to 16 rows (1.25 times as
+// fast on average, 1 in 100 slower by more than 3 % and 0.1 us: K below 540 and no multiple of 128, by 0.2 us at the most, and
+// into the stream over K of 14,336, by 9 %).
+//
+// Waves: as many as there are chunks, eight at most. Chains: two a wave from 17 chunks on (into the stream from 33), where the
+// kernels before had sixteen sums, too. The more chains a column is summed in, the nearer it is to 64 bits: fewer waves with
+// more chunks each were 1.12e-7 off at K of 1,152, where eight are 8.8e-8, and eight with three chunks in one chain 1.21e-7 at
+// 3,072, in two 1.14e-7. Waves, chains and where a walk starts do not go by the rows: a row has the same bits among others
+// and by itself. (Weights of 12,288 rows and more had one chain a column, 3.4e-7 at 3,072; one a wave, 1.2e-7, saves registers.)
+//
+// Tiles a block: as many (up to four) as still load the CUs evenly, as they share the activations: 16 rows of 9,216 by 3,072
+// three tiles (192 blocks) 15.2 us, two (288 blocks, some CUs with two) 21.5; of 24,576 by 4,608 three (two blocks a CU) 47.5,
+// four 54.1. One or two chunks of K have nothing to share, and a block a tile is there sooner (8 rows of 9,216 by 128: one tile
+// 3.4 us, three 4.2); nor do short slices of K (1,024 by 4,608 in eight) or up to four rows of a weight of many rows (1 row of
+// 65,536 by 1,536: one 38.7, four 41.1), unless their walk is turned, for that goes by the block.
+//
+// Chunks in flight: all that a wave has, up to four, where a block is alone on its CU. With three or four tiles and in a walk
+// of more than one round one, or two where rows lie a multiple of 4 KB apart and every wave has whole pairs: blocks of few
+// registers share a CU, and one's loads cover the other's waits (16 rows of 65,536 by 4,608: one 115 us, two 122, four 160;
+// of 16,384 by 4,096: one 31.1, two 27.9, four 31.5: rows that far apart lie on the same few channels, and longer pieces of
+// each spread the load).
+//
+// Turned: 16 rows of 8,192 by 8,192 in step 35.0 us, turned 29.5; of 12,288 by 5,504 42.3 and 34.3, as whenever rows are an odd
+// multiple of 256 or 512 bytes apart; of 6,144 by 4,608 16.3 and 17.6, so not below 8,192 otherwise.
 struct RowsShape {
     int waves, ch, rt, chains;
+    bool turned;
 };
-static RowsShape rows_shape(int m, int n, int k_per, int slices, bool ragged, int rb) {
-    const int chunks = (k_per + 127) / 128;
-    RowsShape sh{std::min(chunks, ROWS_WAVES), 4, 1, 1};
-    sh.ch = std::min((chunks + sh.waves - 1) / sh.waves, 4);
-    if (sh.ch > 2 && (rb == 16 ? n < 12288 : chunks > 32)) sh.chains = 2;
+static RowsShape rows_shape(int m, int n, int k, int k_per, int slices, int rb) {
+    const int chunks = (k_per + 127) / 128, waves = std::min(chunks, ROWS_WAVES), a_wave = (chunks + waves - 1) / waves;
+    const bool ragged = k % 128 != 0;
+    RowsShape sh{waves, 1, 1, 1, k >= ROWS_TURNED || (chunks > 32 && !ragged && k % 512 != 0)};
+    // a whole number of pairs of chunks for every wave, and rows a multiple of 4 KB apart
+    const int pairs = k % 2048 == 0 && k_per % (256 * waves) == 0 && k % k_per == 0 ? 2 : 1;
+    bool spread = a_wave > 4;                            // one or two chunks at a time
     if (rb == 16) {
         const long long tiles = (long long)((n + 15) / 16) * slices;
-        const int most = ragged || sh.ch > 2 ? 2 : 4;
-        const int a_cu = slices > 1 && tiles <= 512 ? 1 : tiles <= 1024 ? (int)((tiles + 255) / 256) : k_per < 2048 && m <= 4 ? 1 : 4;
-        sh.rt = std::max(1, std::min(a_cu, most));
+        auto a_cu = [&](int rt) { return ((tiles + rt - 1) / rt + 255) / 256 * rt; };
+        const long long least = a_cu(1);
+        for (int rt = 2; rt <= 4; ++rt)
+            if (a_cu(rt) * 6 <= least * 7) sh.rt = rt;
+        if (chunks <= 2 && tiles <= 1024) sh.rt = 1;
+        if (slices > 1 && tiles <= 512 && chunks <= 8) sh.rt = 1;
+        if (m <= 4 && tiles > 1024 && !sh.turned) sh.rt = 1;
+        if (tiles > 768 && a_wave > 2) spread = true;
+        if (m <= 4 && tiles > 1024) spread = true;
+        if (sh.rt > 2 && !(sh.rt == 3 && a_wave == 3 && tiles <= 768 && !ragged)) spread = true;
+        if (slices > 1 && a_wave == 4 && pairs == 2) spread = true;
+        sh.ch = spread ? pairs : a_wave;
+        sh.chains = chunks > 2 * ROWS_WAVES && (n < 12288 || sh.ch > 2) ? 2 : 1;
+    } else {
+        // half tiles: one chunk at a time where a CU has several blocks, else two of four, which leaves room for a second block
+        if (n > 4096 || (n > 2048 && a_wave == 4)) sh.ch = spread ? pairs : 1;
+        else sh.ch = spread || (a_wave == 4 && pairs == 2) ? pairs : a_wave;
+        sh.chains = chunks > 4 * ROWS_WAVES ? 2 : 1;
     }
     return sh;
 }
@@ -263,47 +344,75 @@ struct RowsCall {
     Epilogue unit;
 };
 
-template <typename TOut, int RB, int EPI>
-static void rows_launch(const RowsCall& c, hipStream_t s) {
+template <typename TOut, int RB, int EPI, bool SCALED>
+static void rows_launch_as(const RowsCall& c, hipStream_t s) {
     const int k_per = ((c.k + c.slices - 1) / c.slices + 127) / 128 * 128;
-    const bool ragged = c.k % 128 != 0 || c.k >= (1 << 25);      // (offsets inside 64 rows are kept in 32 bits)
-    const RowsShape sh = rows_shape(c.m, c.n, std::min(k_per, c.k), c.slices, ragged, RB);
+    const bool huge = c.k >= (1 << 25), ragged = c.k % 128 != 0 || huge;      // (byte offsets inside 64 rows stay in 32 bits)
+    RowsShape sh = rows_shape(c.m, c.n, c.k, std::min(k_per, c.k), c.slices, RB);
+    if (huge) sh.rt = 1, sh.ch = 1, sh.chains = 1;
     const dim3 grid((unsigned)((c.n + (long long)RB * sh.rt - 1) / (RB * sh.rt)), (unsigned)((c.k + k_per - 1) / k_per));
-    const size_t lds = (size_t)sh.chains * sh.waves * sh.rt * 64 * sizeof(float4);          // (32 KB at most)
-#define ROWS_GO(RT, CH, CHAINS, RG)                                                                                  \
-    k_rows_gemm<TOut, RB, RT, CH, CHAINS, EPI, RG><<<grid, sh.waves * 64, lds, s>>>(                                   \
+    const int rounds = ((std::min(k_per, c.k) + 127) / 128 + sh.waves * sh.ch - 1) / (sh.waves * sh.ch);
+    const int turned = sh.turned ? rounds : 0;
+    const bool even = c.k % (128 * sh.waves * sh.ch) == 0 && k_per % (128 * sh.waves * sh.ch) == 0;
+    const size_t lds = (size_t)sh.chains * sh.waves * sh.rt * 64 * sizeof(float4);          // (48 KB at most)
+#define ROWS_GO(RT, CH, CHAINS, KIND)                                                                                \
+    k_rows_gemm<TOut, RB, RT, CH, CHAINS, EPI, KIND, SCALED><<<grid, sh.waves * 64, lds, s>>>(                         \
         c.x, c.ssq_in, c.n_parts, c.eps, c.w, c.bias, (TOut*)c.y, c.x_io, c.ssq_out, c.weighted_out, c.weighted_by, c.m, \
-        c.n, c.k, k_per, c.unit)
-#define ROWS_CH(RT, RG)                                                                                              \
+        c.n, c.k, k_per, rounds, turned, c.unit)
+#define ROWS_CHAINS(RT, CH, KIND)                                                                                    \
     do {                                                                                                             \
-        if (sh.ch == 1) ROWS_GO(RT, 1, 1, RG);                                                                       \
-        else if (sh.ch == 2) ROWS_GO(RT, 2, 1, RG);                                                                  \
-        else if (sh.ch == 3 && sh.chains == 2) ROWS_GO(RT, 3, 2, RG);                                                \
-        else if (sh.ch == 3) ROWS_GO(RT, 3, 1, RG);                                                                  \
-        else if (sh.chains == 2) ROWS_GO(RT, 4, 2, RG);                                                              \
-        else ROWS_GO(RT, 4, 1, RG);                                                                                  \
+        if (sh.chains == 2) ROWS_GO(RT, CH, 2, KIND);                                                                \
+        else ROWS_GO(RT, CH, 1, KIND);                                                                               \
     } while (0)
-    if constexpr (RB == 16) {
-        if (ragged) {
-            if (sh.rt == 1) ROWS_CH(1, true);
-            else ROWS_CH(2, true);
-        } else if (sh.rt == 1) {
-            ROWS_CH(1, false);
-        } else if (sh.rt == 2) {
-            ROWS_CH(2, false);
-        } else if (sh.rt == 3) {
-            if (sh.ch == 1) ROWS_GO(3, 1, 1, false);
-            else ROWS_GO(3, 2, 1, false);
-        } else {
-            if (sh.ch == 1) ROWS_GO(4, 1, 1, false);
-            else ROWS_GO(4, 2, 1, false);
-        }
+// (three and four chunks a wave are a walk of one round: two chains, but into the stream)
+#define ROWS_LONG(RT, CH, KIND)                                                                                      \
+    do {                                                                                                             \
+        if constexpr (RB == 8) ROWS_CHAINS(RT, CH, KIND);                                                            \
+        else ROWS_GO(RT, CH, 2, KIND);                                                                               \
+    } while (0)
+#define ROWS_CH(RT)                                                                                                  \
+    do {                                                                                                             \
+        if (sh.ch == 1 && ragged) ROWS_CHAINS(RT, 1, ROWS_RAGGED);                                                   \
+        else if (sh.ch == 1) ROWS_CHAINS(RT, 1, ROWS_WHOLE);                                                         \
+        else if (sh.ch == 2 && ragged) ROWS_GO(RT, 2, 1, ROWS_RAGGED);                                               \
+        else if (sh.ch == 2 && even) ROWS_CHAINS(RT, 2, ROWS_WHOLE);                                                 \
+        else if (sh.ch == 2) ROWS_GO(RT, 2, 1, ROWS_UNEVEN);                                                         \
+        else if (sh.ch == 3 && ragged) ROWS_LONG(RT, 3, ROWS_RAGGED);                                                \
+        else if (sh.ch == 3 && even) ROWS_LONG(RT, 3, ROWS_WHOLE);                                                   \
+        else if (sh.ch == 3) ROWS_LONG(RT, 3, ROWS_UNEVEN);                                                          \
+        else if (ragged) ROWS_LONG(RT, 4, ROWS_RAGGED);                                                              \
+        else if (even) ROWS_LONG(RT, 4, ROWS_WHOLE);                                                                 \
+        else ROWS_LONG(RT, 4, ROWS_UNEVEN);                                                                          \
+    } while (0)
+    if (huge) {
+        ROWS_GO(1, 1, 1, ROWS_HUGE);
+    } else if constexpr (RB == 8) {
+        ROWS_CH(1);
+    } else if (sh.rt == 1) {
+        ROWS_CH(1);
+    } else if (sh.rt == 2) {
+        ROWS_CH(2);
+    } else if (sh.rt == 3) {
+        if (ragged) ROWS_CHAINS(3, 1, ROWS_RAGGED);
+        else if (sh.ch == 1) ROWS_CHAINS(3, 1, ROWS_WHOLE);
+        else if (sh.ch == 2) ROWS_CHAINS(3, 2, ROWS_WHOLE);
+        else if (even) ROWS_GO(3, 3, 2, ROWS_WHOLE);
+        else ROWS_GO(3, 3, 2, ROWS_UNEVEN);
     } else {
-        if (ragged) ROWS_CH(1, true);
-        else ROWS_CH(1, false);
+        if (ragged) ROWS_GO(4, 1, 1, ROWS_RAGGED);
+        else if (sh.ch == 1) ROWS_GO(4, 1, 1, ROWS_WHOLE);
+        else ROWS_GO(4, 2, 1, ROWS_WHOLE);
     }
+#undef ROWS_LONG
+#undef ROWS_CHAINS
 #undef ROWS_CH
 #undef ROWS_GO
+}
+
+template <typename TOut, int RB, int EPI>
+static void rows_launch(const RowsCall& c, hipStream_t s) {
+    if (c.ssq_in) rows_launch_as<TOut, RB, EPI, true>(c, s);
+    else rows_launch_as<TOut, RB, EPI, false>(c, s);
 }
 
 int imparo_few_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
@@ -358,7 +467,7 @@ extern "C" int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts,
 // cannot do that).
 int imparo_load_code_decode_rows() {
     hipFuncAttributes attributes;
-    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_rows_gemm<float, 8, 1, 1, 1, ROWS_RESID, false>)) ==
+    return hipFuncGetAttributes(&attributes, reinterpret_cast<const void*>(&k_rows_gemm<float, 8, 1, 1, 1, ROWS_RESID, ROWS_WHOLE, false>)) ==
                    hipSuccess
                ? IMPARO_OK
                : IMPARO_LAUNCH_FAILED;

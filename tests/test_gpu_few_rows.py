@@ -157,3 +157,34 @@ def test_sums_stay_as_near_to_64_bits(k, limit):
     ops.rows_gemm(x, w, out=out)
     want = x.double() @ w.double().t()
     assert float((out.double() - want).norm() / want.norm()) < limit
+
+
+# every way to share a product out: three and four tiles a block with one, two and three chunks in flight, walks of several
+# rounds with waves that have a chunk less, turned walks whose rounds end unevenly, pairs of chunks, slices of two rounds
+@pytest.mark.parametrize("n, k", [(9200, 1152), (9216, 3072), (12288, 2304), (17600, 3072), (20010, 2312), (24576, 2048), (6144, 5504),
+                                  (9000, 4224), (12300, 4608), (16400, 6144), (3072, 12288), (2048, 16384), (1030, 14336), (70, 8968)])
+def test_few_rows_have_the_same_bits_however_they_are_shared_out(n, k):
+    x, w = rnd(16, k, seed=1).bfloat16().to(DEV), rnd(n, k, seed=2, scale=0.02).bfloat16().to(DEV)
+    plain, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    whole = torch.full((16, n), float("nan"), device=DEV)
+    ops.rows_gemm(x, w, out=whole)
+    assert bool(((whole.double() - plain).abs() <= size * (k + 2) * EPS).all())
+    ssq = torch.full((1, 16), float(k), device=DEV)          # (a scale of one, but for eps)
+    for m in (1, 2, 4, 5, 9):
+        out = torch.full((m, n), float("nan"), device=DEV)
+        ops.rows_gemm(x[:m].contiguous(), w, out=out)
+        assert torch.equal(out, whole[:m])
+        ops.rows_gemm(x[:m].contiguous(), w, out=out, ssq_in=ssq, eps=1e-12)
+        assert torch.equal(out, whole[:m])
+    slices = ops.gemm_slices(16, n, k, torch.bfloat16)
+    if slices > 1:
+        parts, one = torch.full((slices, 16, n), float("nan"), device=DEV), torch.full((slices, 1, n), float("nan"), device=DEV)
+        ops.gemm(x, w, parts)
+        ops.gemm(x[3:4].contiguous(), w, one)
+        assert bool(((parts.double().sum(0) - plain).abs() <= size * (k + 2) * EPS).all()) and torch.equal(one[:, 0], parts[:, 3])
+    if n <= 9216:
+        stream = torch.zeros(16, n, device=DEV)
+        ssq = torch.full((ops.rows_parts(n), 16), float("nan"), device=DEV)
+        ops.rows_gemm(x, w, into=stream, ssq_out=ssq)
+        assert bool(((stream.double() - plain).abs() <= size * (k + 2) * EPS).all())
+        torch.testing.assert_close(ssq.double().sum(0), stream.double().square().sum(1), rtol=1e-5, atol=0.0)
