@@ -738,23 +738,24 @@ __global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__
     moe_store_tile<2, 2, 4, TOut, GATED>(acc, out, entry_of_slot, gate, expert, row0, rows, n0, N, epi);
 }
 
-// Few rows an expert (a decode step): a block takes RT tiles of 16 weight rows of one expert and up to 16 slots. A tile is
-// the M side of 16x16x32 products; K is cut in four neighbouring parts over the block's waves, walked in runs of 64, U of
-// them a round, and everything a round needs is asked for at once, from memory straight into the operand registers, as in decode_rows.hip
-// (what bounds it is reading the experts' matrices and the trips to memory behind one another: the tile list, then the
-// weights and the slots' tokens, whose rows come last). A lane takes 16 consecutive k of its row, so that four lanes read
-// a row's 128 bytes side by side; the slots' rows are read with the same k order, which is all a dot product asks for.
-// The waves' partial sums meet in LDS and are added in wave order.
-// GATED: half of a block's tiles are gate rows, the other half the up rows that belong to them, 32 rows further on.
-// 8 tokens, 4 of 8 experts and a shared one: gate and up, 1,536 rows by 1,024 an expert, 10.1 us (two runs a wave at a time,
-// the blocks unevenly over the XCDs: 12.0), the way back, 1,024 by 768, 5.9 (6.3); one token 6.5 and 4.7 (7.5 and 4.7). With
-// eight waves of two runs 9.1, but sums in another order, which turn a router's near ties behind them.
+// Few rows an expert (a decode step): a block takes a tile of 16 weight rows of one expert, gated a tile of gate rows and the
+// up rows that belong to them, 32 rows further on, and up to 16 slots. A tile is the M side of 16x16x32 products; K is cut in
+// four neighbouring parts over the block's waves, walked in runs of 64, U of them a round, and everything a round needs is
+// asked for at once, from memory straight into the operand registers, as in decode_rows.hip (what bounds it is reading the
+// experts' matrices and the trips to memory behind one another: the tile list, then the weights and the slots' tokens, whose
+// rows come last, so nothing but products stands behind them). A lane takes 16 consecutive k of its row, so that four lanes
+// read a row's 128 bytes side by side; the slots' rows are read with the same k order, which is all a dot product asks for.
+// The waves' partial sums meet in LDS and are added in wave order. 4 of 8 experts and a shared one, 8 tokens: gate and up,
+// 1,536 rows by 1,024 an expert, 9.4 us (12.0 with two runs a wave at a time, selects before every product and the blocks
+// unevenly over the XCDs), the way back, 1,024 by 768, 6.2 (7.1); one token 6.3 and 4.6 (7.4 and 5.2). Over 3,920 forms of 4 to
+// 128 experts 1.23 times as fast as that on average, 90 slower by more than 3 % and 0.1 us: gated, K of 1,024 and 2,048 over
+// few rows, by 12 % at the most.
 #define MOE_ROWS_WAVES 4
 template <typename TOut, bool GATED, int RT, int U>
 __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const bf16_t* __restrict__ A, int a_ld, int gather_div,
                                                          const int32_t* __restrict__ entry_of_slot,
                                                          const bf16_t* __restrict__ W, TOut* __restrict__ out,
-                                                         const int32_t* __restrict__ tiles, int max_tiles, int across,
+                                                         const int32_t* __restrict__ tiles, int max_tiles,
                                                          int N, int K, int epi, MoeGate gate) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -765,15 +766,17 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     // them (9 tiles of 12 by 24 blocks, tile after tile along the grid: 36 on two XCDs of 32 CUs and 24 on the others, 12.0 us
     // where this way it is 10.1).
     const int32_t* last = tiles + 3 * (max_tiles - 1);
-    const int n_tiles = last[0] < 0 && last[2] == MOE_COUNTED ? min(last[1], max_tiles) : max_tiles;
-    const unsigned block = blockIdx.y * gridDim.x + blockIdx.x;
-    const int tile = block / (unsigned)across;
-    if (tile >= n_tiles) return;
-    const int expert = tiles[3 * tile];
-    if (expert < 0) return;
-    const int row0 = tiles[3 * tile + 1], rows = tiles[3 * tile + 2];
-    const int n0 = (int)(block - (unsigned)tile * across) * 16 * GROUPS;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // (what the tile holds is read beside the number of tiles, and nothing of either under a condition: one trip to memory of
+    // 0.6 us, and not three)
+    const unsigned tile = blockIdx.z * gridDim.y + blockIdx.y, listed = min(tile, (unsigned)max_tiles - 1);
+    const int expert = tiles[3 * listed], row0 = tiles[3 * listed + 1], rows = tiles[3 * listed + 2];
+    const int last_expert = last[0], last_rows = last[2];
+    int counted = last[1];
+    asm volatile("" : "+s"(counted));                    // (or it is asked for when the others have come)
+    const int n_tiles = (last_expert < 0) & (last_rows == MOE_COUNTED) ? min(counted, max_tiles) : max_tiles;
+    if ((int)(tile >= (unsigned)n_tiles) | (expert < 0) | (row0 < 0) | (rows < 1)) return;
+    const int n0 = (int)blockIdx.x * 16 * GROUPS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int c = lane & 15, g = lane >> 4;
     const int slot = row0 + min(c, rows - 1);
     const int entry = entry_of_slot ? entry_of_slot[slot] : 0;
@@ -813,6 +816,17 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int first = run_lo; first < run_hi;) {
+        if ((first + U) * 64 > K) {                      // (for the last runs of a K that is no multiple of 64 only)
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const bool in = (first + u) * 64 + g * 16 + h * 8 < K;
+                    x[u][h] = in ? x[u][h] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                    for (int t = 0; t < RT; ++t) w[t][u][h] = in ? w[t][u][h] : u32x4{0u, 0u, 0u, 0u};
+                }
+        }
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -820,10 +834,8 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
                 if (first + u >= run_hi) continue;
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const bool in = (first + u) * 64 + g * 16 + h * 8 < K;
-                    const u32x4 wv = in ? w[t][u][h] : u32x4{0u, 0u, 0u, 0u}, xv = in ? x[u][h] : u32x4{0u, 0u, 0u, 0u};
-                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wv), __builtin_bit_cast(bf16x8, xv),
-                                                                     acc[t], 0, 0, 0);
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[t][u][h]),
+                                                                     __builtin_bit_cast(bf16x8, x[u][h]), acc[t], 0, 0, 0);
                 }
             }
         first += U;
@@ -838,11 +850,11 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     auto total = [&](int t, float (&v)[4]) __attribute__((always_inline)) {
         float4 p[MOE_ROWS_WAVES];
 #pragma unroll
-        for (int q = 0; q < MOE_ROWS_WAVES; ++q) p[q] = moe_part[(q * RT + t) * WAVE + lane];
+        for (int q = 0; q < MOE_ROWS_WAVES; ++q) p[q] = moe_part[(min(q, waves - 1) * RT + t) * WAVE + lane];
         v[0] = p[0].x, v[1] = p[0].y, v[2] = p[0].z, v[3] = p[0].w;
 #pragma unroll
         for (int q = 1; q < MOE_ROWS_WAVES; ++q)
-            v[0] += p[q].x, v[1] += p[q].y, v[2] += p[q].z, v[3] += p[q].w;
+            if (q < waves) v[0] += p[q].x, v[1] += p[q].y, v[2] += p[q].z, v[3] += p[q].w;
     };
     // a lane holds slot c, outputs 4 g + i of a group
     for (int t = wave; t < GROUPS; t += MOE_ROWS_WAVES) {
@@ -868,37 +880,26 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     }
 }
 
-// A block a CU, as far as the list's length tells before it is known (tiles may be empty): tiles of 16 rows a block
+// One tile a block whatever the number of tiles: with four (fewer blocks that share the slots' rows) every form but short rows
+// of many experts was slower, by up to 1.4 times (20 slots of 128 experts, 1,024 by 1,024: 9.5 us and 13.6). Runs at once: all
+// of a wave up to three, then four where they come out even, or two where a run is a gate row's and an up row's (K of 2,048,
+// gated, one slot: four 7.4 us, two 6.8).
 template <typename TOut, bool GATED>
 static void launch_rows16(const bf16_t* a, int a_ld, int gather_div, const int32_t* entry_of_slot, const bf16_t* w, TOut* out,
                           const int32_t* tiles, int max_tiles, int n, int k, int epi, const MoeGate& gate, hipStream_t s) {
-    const int a_wave = ((k + 63) / 64 + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES, u = std::min(a_wave, 4);
-    const long long all = (long long)std::max(1, max_tiles - 1) * ((n + 15) / 16);
-    const int rt = GATED ? (all <= 1024 ? 2 : 4) : (all <= 1024 ? 1 : 4);
-    const int outputs = 16 * (GATED ? rt / 2 : rt), columns = GATED ? n / 2 : n;
-    const int across = (columns + outputs - 1) / outputs;
-    const long long blocks = (long long)max_tiles * across, row = std::min<long long>(blocks, 1 << 22);
-    const dim3 grid((unsigned)row, (unsigned)((blocks + row - 1) / row));    // (a launch holds fewer than 2^32 threads along x)
-    const size_t lds = (size_t)MOE_ROWS_WAVES * rt * WAVE * sizeof(float4);
-#define ROWS16_U(RT, U)                                                                                              \
-    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, MOE_ROWS_WAVES * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles, \
-                                                                      max_tiles, across, n, k, epi, gate)
-#define ROWS16_GO(RT)                                                                                                \
-    do {                                                                                                             \
-        if (u == 1) ROWS16_U(RT, 1);                                                                                 \
-        else if (u == 2) ROWS16_U(RT, 2);                                                                            \
-        else if (u == 3) ROWS16_U(RT, 3);                                                                            \
-        else ROWS16_U(RT, 4);                                                                                        \
-    } while (0)
-    if constexpr (!GATED) {
-        if (rt == 1) {
-            ROWS16_GO(1);
-            return;
-        }
-    }
-    if (rt == 2) ROWS16_GO(2);
-    else ROWS16_GO(4);
-#undef ROWS16_GO
+    constexpr int RT = GATED ? 2 : 1;
+    const int runs = (k + 63) / 64, a_wave = (runs + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES;
+    const int waves = (runs + a_wave - 1) / a_wave;      // (all that have a run: four, or fewer with a short K)
+    const int tall = std::min(max_tiles, 32768);
+    const dim3 grid((unsigned)(((GATED ? n / 2 : n) + 15) / 16), (unsigned)tall, (unsigned)((max_tiles + tall - 1) / tall));
+    const size_t lds = (size_t)waves * RT * WAVE * sizeof(float4);
+#define ROWS16_U(U)                                                                                                  \
+    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, waves * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles,   \
+                                                                max_tiles, n, k, epi, gate)
+    if (a_wave == 1) ROWS16_U(1);
+    else if (a_wave == 3) ROWS16_U(3);
+    else if (!GATED && a_wave % 4 == 0) ROWS16_U(4);
+    else ROWS16_U(2);
 #undef ROWS16_U
 }
 

@@ -67,8 +67,8 @@ def test_rows_scaled_at_the_end(m, k, parts):
     torch.testing.assert_close(out.cpu().double(), plain.cpu().double() * scale[:, None], rtol=parts * EPS + 1e-6, atol=0.0)
 
 
-# one to four tiles of weight rows a block, a last block partly past the end, K of less than a run, ragged, one round of
-# runs and more than one; experts that nobody chose, so that the list ends in empty tiles
+# K of less than a run, ragged, one round of runs and more than one; experts that nobody chose, so that the list ends in
+# empty tiles (many tiles, and a last tile of weight rows partly past the end: below)
 @pytest.mark.parametrize("n, k", [(64, 8), (192, 72), (1536, 1024), (1088, 136), (64, 2120), (832, 768)])
 @pytest.mark.parametrize("tokens, experts, top", [(1, 3, 2), (8, 9, 4), (16, 4, 4)])
 def test_experts_products_of_few_rows(n, k, tokens, experts, top):
@@ -188,3 +188,40 @@ def test_few_rows_have_the_same_bits_however_they_are_shared_out(n, k):
         ops.rows_gemm(x, w, into=stream, ssq_out=ssq)
         assert bool(((stream.double() - plain).abs() <= size * (k + 2) * EPS).all())
         torch.testing.assert_close(ssq.double().sum(0), stream.double().square().sum(1), rtol=1e-5, atol=0.0)
+
+
+# more tiles of weight rows than blocks run at once, a last one partly past the end, waves without a run (K up to 128), with one
+# to five; lists with an empty tile at the end and without one, and lists that do not count them
+@pytest.mark.parametrize("n, k", [(1700, 136), (4100, 72), (1536, 1024), (1000, 320), (24, 8), (2050, 1288)])
+@pytest.mark.parametrize("tokens, experts, top", [(8, 9, 5), (16, 40, 5), (1, 1, 1)])
+def test_experts_products_of_many_tiles(n, k, tokens, experts, top):
+    g = torch.Generator().manual_seed(n + k + tokens)
+    choice = torch.stack([torch.randperm(experts, generator=g)[:top] for _ in range(tokens)]).int()
+    entries = tokens * top
+    rows = ops.moe_tile_rows(entries, experts, torch.bfloat16)
+    assert rows == 16
+    tiles = torch.empty(ops.moe_max_tiles(entries, experts, rows), 3, device=DEV, dtype=torch.int32)
+    slot, entry = torch.empty(entries, device=DEV, dtype=torch.int32), torch.empty(entries, device=DEV, dtype=torch.int32)
+    ops.moe_plan(choice.to(DEV), experts, rows, slot, entry, tiles)
+    x, w = rnd(tokens, k, seed=1).bfloat16().to(DEV), rnd(experts, n, k, seed=2, scale=0.1).bfloat16().to(DEV)
+    expert, token = choice.flatten().long().to(DEV), torch.arange(entries, device=DEV) // top
+    plain, size = (torch.empty(entries, n, device=DEV, dtype=torch.float64) for _ in range(2))
+    for e in range(experts):
+        of = expert == e
+        plain[of] = x[token[of]].double() @ w[e].double().t()
+        size[of] = x[token[of]].double().abs() @ w[e].double().abs().t()
+    at = slot.long()
+    out = torch.full((entries, n), float("nan"), device=DEV)
+    ops.moe_gemm(x, w, out, tiles, rows, entry_of_slot=entry, gather_div=top)
+    assert bool(((out[at].double() - plain).abs() <= size * (k + 2) * EPS).all())
+    live = tiles[tiles[:, 0] >= 0]
+    for listed in (live, torch.cat([live, torch.tensor([[-1, 0, 0]] * 3, device=DEV, dtype=torch.int32), live[:1]])):
+        again = torch.full_like(out, float("nan"))
+        ops.moe_gemm(x, w, again, listed.contiguous(), rows, entry_of_slot=entry, gather_div=top)
+        assert torch.equal(again, out)
+    if n % 64 == 0:
+        gated = torch.full((entries, n // 2), float("nan"), device=DEV, dtype=torch.bfloat16)
+        ops.moe_gemm(x, w, gated, tiles, rows, entry_of_slot=entry, gather_div=top, epilogue="gated")
+        z = out[at].double().view(entries, n // 64, 2, 32)
+        want = (z[:, :, 0] / (1.0 + torch.exp(-z[:, :, 0])) * z[:, :, 1]).reshape(entries, n // 2)
+        torch.testing.assert_close(gated[at].double(), want, rtol=2.0 ** -8 + 1e-5, atol=1e-6)
