@@ -42,6 +42,20 @@ __device__ __forceinline__ Best row_best(const float* __restrict__ row, int voca
         // and a choice of index for every value were a third of the time (one row of 65,536 9.0 us, so 6.2).
         const float4* row4 = reinterpret_cast<const float4*>(row);
         const int n4 = vocab >> 2;
+        if (n4 <= (int)blockDim.x) {
+            // one load a thread: the maximum and its index together, one meeting of the block (a row of 1,000 in two 3.8 us)
+            const float4 v = row4[min((int)threadIdx.x, n4 - 1)];
+            const float vs[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if ((int)threadIdx.x < n4 && (vs[j] > b.v || (vs[j] == b.v && 4 * (int)threadIdx.x + j < b.i))) {
+                    b.v = vs[j];
+                    b.i = 4 * (int)threadIdx.x + j;
+                }
+            b = block_best(b, scratch);
+            if (b.i == INT_MAX) b.i = 0;   // every value was NaN
+            return b;
+        }
         constexpr int DEEP = 16;
         float m = -INFINITY;
         int met = 0;
