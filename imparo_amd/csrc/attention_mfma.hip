@@ -405,7 +405,9 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     const int lo_c = (EXT && keep > 0) ? 0 : min(lo, max(last, 0)), last_c = max(last, 0);
     // What the block shares and the projection's rows are asked for before the tiles: loads come back in order, and who waits
     // for one behind the tiles' waits for the tiles too, at the barrier the whole block with it (one row over 50 keys 6.3 us,
-    // so 5.7; 8 rows over 300 keys 8.7 and 7.9).
+    // so 5.7; 8 rows over 300 keys 8.7 and 7.9). Not with heads of 128, whose tiles leave no registers for what comes first:
+    // 8 rows over 1,000 keys, 32 heads by 8, so 17.9 us, behind the tiles 16.3.
+    constexpr bool AHEAD = FROM_QKV && ND <= 4;
     HeadElements<ND> qh;
     const int units = heads + 2 * kv_heads;
     float freq;
@@ -413,7 +415,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     float4 own_raw;
     const int norm_at = 2 * ((int)threadIdx.x - 128);       // (another wave's lanes than the sines and cosines)
     const int own_at = 4 * (lane % (D / 4));
-    if constexpr (FROM_QKV) {                               // (every lane asks, for something: no load under a branch)
+    auto ask_shared = [&]() __attribute__((always_inline)) {      // (every lane asks, for something: no load under a branch)
         const float* row_in = fq.qkv + (size_t)t * units * D;
         const int norm_from = min(max(norm_at, 0), D - 2);
         head_elements<ND>(qh, row_in + (size_t)head * D, g);
@@ -422,10 +424,11 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         k_norm = make_float2((fq.q_weight ? fq.k_weight : row_in)[norm_from], (fq.q_weight ? fq.k_weight : row_in)[norm_from + 1]);
         own_raw = *reinterpret_cast<const float4*>(row_in + (size_t)(lane < D / 4 ? heads + kvh : heads + kv_heads + kvh) * D + own_at);
         __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    if constexpr (AHEAD) ask_shared();
     DecodeTile<ND> regs[TILES];
     // (with the queries given, where nothing else waits for scalar loads, the lanes' own are no slower: 4.3 us, 4.5 so)
-    if (FROM_QKV && page_size >= 32) {
+    if (AHEAD && page_size >= 32) {
         int page[TILES];
 #pragma unroll
         for (int j = 0; j < TILES; ++j) {       // past the split's end: some page, never used
@@ -449,9 +452,10 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         }
     }
     if constexpr (FROM_QKV) {
-        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+        else ask_shared();
         // while the tiles are on their way: the block's sines and cosines, the norms' weights, and the row's new key and
-        // value, which wait in LDS for the last wave
+        // value, which wait in LDS for the wave that takes them
         if (fq.inv_freq && (int)threadIdx.x < D / 2) rotation_of(pos, freq, sn_tab[threadIdx.x], cs_tab[threadIdx.x]);
         if (norm_at >= 0 && norm_at < D) {
             *reinterpret_cast<float2*>(qw_tab + norm_at) = q_norm;
@@ -472,8 +476,9 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         }
     }
     if constexpr (FROM_QKV) {
-        // (by the wave that has the fewest tiles, which is done first where the split is not full)
-        if (own && wave == MFMA_WAVES - 1) {
+        // (by the wave that has the fewest tiles, which is done first where the split is not full; the first with heads of 128,
+        // which keeps the order of the sums there)
+        if (own && wave == (AHEAD ? MFMA_WAVES - 1 : 0)) {
             // the row's own key and value, from the projection's row: every lane holds the key's dims
             // dk*32 + 8*g + j (the same for all 16 heads) and the value's dims dt*16 + 4*g + i
             Frag8 kf[NK];
