@@ -118,8 +118,9 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     // This wave's chunks are first, first + waves, ...: CH of them a round. No load under a branch (the compiler would wait
     // for every load in flight at the next use of any): past the last chunk the last one again, which no product reads.
     // A long walk starts at a round that goes by the block's place: rows of a long K lie so far apart that blocks in step keep
-    // asking the same few channels (8 rows of 16,384 by 11,008 82 us in step, 67 so; of 8,192 by 16,384 68 and 52). The
-    // place is hashed, as rounds that follow the row's number undo what the address's own hash does (8,192 by 8,192 41 us).
+    // asking the same few channels (8 rows of 16,384 by 11,008 82 us in step, 68 so; of 8,192 by 16,384 68 and 53). The
+    // place is hashed, as rounds that follow the row's number undo what the address's own hash does (8 rows of 8,192 by
+    // 8,192: in step 32 us, hashed 28, by the row 46).
     const int turn = waves * CH;
     int round = (int)__umulhi((unsigned)(n0 / 64) * 2654435761u, (unsigned)turned);      // (no branch in front of the loads)
     auto at = [&](const bf16_t* base, Offset row, int chunk, int s) __attribute__((always_inline)) {
@@ -312,7 +313,8 @@ static RowsShape rows_shape(int m, int n, int k, int k_per, int slices, int rb) 
             if (a_cu(rt) * 6 <= least * 7) sh.rt = rt;
         if (chunks <= 2 && tiles <= 1024) sh.rt = 1;
         if (slices > 1 && tiles <= 512 && chunks <= 8) sh.rt = 1;
-        if (m <= 4 && tiles > 1024 && !sh.turned) sh.rt = 1;
+        // (a launch holds fewer than 2^32 threads along x: a tile a block of several waves would pass that at 2^29 rows)
+        if (m <= 4 && tiles > 1024 && tiles < (1 << 22) && !sh.turned) sh.rt = 1;
         if (tiles > 768 && a_wave > 2) spread = true;
         if (m <= 4 && tiles > 1024) spread = true;
         if (sh.rt > 2 && !(sh.rt == 3 && a_wave == 3 && tiles <= 768 && !ragged)) spread = true;

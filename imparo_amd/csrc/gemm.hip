@@ -387,7 +387,7 @@ static int launch_f32(const float* x, const float* w, const float* bias, TOut* y
                       hipStream_t s) {
     const unsigned rows_blocks = (unsigned)((n + 15) / 16);
     // (from K of 256 on: with less the ring is hardly filled before it is empty, 1 row of 512 by 64 2.6 us and 2.2 without, by 128
-    // 3.1 and 2.9, by 256 3.6 and 4.1)
+    // 3.1 and 2.9, by 256 3.6 and 3.8)
     if (m <= 16 && k % 64 == 0 && k >= 256 && k < (1 << 25) && !(((uintptr_t)x | (uintptr_t)w) & 15)) {
         // stages: as many as keep a wave alone on its CU supplied, fewer where more waves share the CU and its LDS (9,216 by
         // 1,024: 8 stages 11.1 us, 4 10.6)
