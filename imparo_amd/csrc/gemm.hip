@@ -40,7 +40,6 @@ __device__ __forceinline__ uint4 zero_if(bool out, uint4 v) {
 #define F32_BK 32
 #define F32_LD 40   // floats from row to row in LDS: 32 bytes beyond a row's own, which keeps 16-byte reads free of conflicts
 
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // four floats wherever they lie
 // VEC: K is at least 4, and rows are read in vectors of four floats that may start anywhere; the end of a K that is no
 // multiple of 4, and a shorter K, value by value. (666 rows by 9,216 by 1,024 that start 4 bytes off 16:
 // 140 us, 395 value by value.)

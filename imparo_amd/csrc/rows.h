@@ -7,6 +7,8 @@
 #pragma once
 #include "common.h"
 
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));     // four floats wherever they lie
+
 #define EPI_NONE 0
 #define EPI_SWIGLU 1   // weight rows interleaved gate, up, gate, up...: out[m, j] = act(y[m, 2j], y[m, 2j+1])
 #define EPI_ADD 2      // float32 out only: Y += y, what Y holds being read where the result is stored
@@ -44,7 +46,7 @@ __device__ __forceinline__ float gated_mul_fast(const Epilogue& e, float g, floa
 #define ROWS_ASK 4           // partial sums of four tokens that a thread has in flight at once
 
 struct RowsSsq {
-    float4 v[ROWS_ASK];
+    f32x4_any v[ROWS_ASK];
 };
 
 // Thread i gathers the partials p = first + i / 4, + threads / 4, ... of tokens 4 * (i % 4) to 4 * (i % 4) + 3: every block
@@ -53,7 +55,7 @@ __device__ __forceinline__ void rows_ssq_ask(RowsSsq& r, const float* __restrict
     const int at = first + (threadIdx.x >> 2), step = blockDim.x >> 2;
 #pragma unroll
     for (int j = 0; j < ROWS_ASK; ++j)
-        r.v[j] = *reinterpret_cast<const float4*>(ssq + (size_t)min(at + j * step, n_parts - 1) * ROWS_PARTS + (threadIdx.x & 3) * 4);
+        r.v[j] = *reinterpret_cast<const f32x4_any*>(ssq + (size_t)min(at + j * step, n_parts - 1) * ROWS_PARTS + (threadIdx.x & 3) * 4);
 }
 
 __device__ __forceinline__ float rows_fold(float v) {       // over the lanes 4, 8, 16 and 32 apart
@@ -75,7 +77,7 @@ __device__ __forceinline__ void rows_ssq_share(float* part, const RowsSsq& early
 #pragma unroll
         for (int j = 0; j < ROWS_ASK; ++j) {
             const bool in = first + at + j * step < n_parts;
-            s.x += in ? r.v[j].x : 0.f, s.y += in ? r.v[j].y : 0.f, s.z += in ? r.v[j].z : 0.f, s.w += in ? r.v[j].w : 0.f;
+            s.x += in ? r.v[j][0] : 0.f, s.y += in ? r.v[j][1] : 0.f, s.z += in ? r.v[j][2] : 0.f, s.w += in ? r.v[j][3] : 0.f;
         }
     };
     add(early, 0);
