@@ -1065,7 +1065,7 @@ static bool dma_tile_takes(int m, int n, int k) {
 //         256x192 0.89 .. 1.30       256x256 1.03 .. 1.58       192x256 0.95 .. 1.25
 //     (192 activation rows suit portions a little over a power of two, a prompt's beside the tokens of other requests:
 //     gate and up of 520 rows 57 us on the 256x256 tile and 51, 1,536 rows 117 and 104, 2,300 rows 174 and 149. K in one
-//     piece and rows of at most 4,096 only: with 8,192 a step took 1.13 us on 24 CUs where 2,048 took 0.85);
+//     piece and of at most 4,096 only: with 8,192 a step took 1.13 us on 24 CUs where 2,048 took 0.85);
 //   - a tile of 128 rows by 64 weight rows on four waves and four stages takes 0.35 .. 0.50 us a step: with at
 //     most 128 rows (one tile down the rows) it makes twice the blocks of the 128x128 tile out of a weight
 //     that is streamed once, and a block's share of the weights is what bounds such a product (measured at
@@ -1171,130 +1171,6 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
         DMA_GO(4, 1, 4);
 #undef DMA_GO
     return launch_status();
-}
-
-// ------------------------------------------------------------------ bfloat16, some rows (17..64), K split over waves
-// One block per 16 weight rows. Its NW waves split K in chunks of 128: wave w
-// takes chunks w, w + NW, ... so the block reads each weight row as one
-// contiguous stream. The 16 weight rows are the MFMA's M side, up to 16*MT
-// activation rows its N side. A decode step is a chain of such products, each
-// a few megabytes: what counts is how few memory round trips one of them
-// takes, so a wave has the loads of its next chunk in flight while it
-// multiplies the current one, and NW is chosen so that a wave has few chunks.
-// Partial sums meet in LDS and are added in wave order, so the result is the
-// same from run to run.
-template <int MT>
-struct SkinnyFrags {
-    Frag8 w[4];
-    Frag8 x[MT][4];
-};
-
-// With slices (gridDim.y > 1) block (x, y) sums only K range [y * k_per, (y+1) * k_per) and
-// writes it to Y + y * M * N: the consumer adds the slices in order.
-template <typename TOut, int MT, int NW>
-__global__ __launch_bounds__(NW * 64) void k_gemm_bf16_skinny(const bf16_t* __restrict__ X,
-                                                              const bf16_t* __restrict__ W,
-                                                              const float* __restrict__ bias,
-                                                              TOut* __restrict__ Y, int M, int N, int K_all,
-                                                              int k_per, Epilogue epilogue) {
-    __shared__ float red[NW][MT][64][4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0 = blockIdx.x * 16;
-    const int k_lo = blockIdx.y * k_per;
-    const int K = min(K_all, k_lo + k_per) - k_lo;       // this block's part of K, re-based to 0
-    X += k_lo;
-    W += k_lo;
-    Y += (size_t)blockIdx.y * M * N;
-    if (blockIdx.y > 0) bias = nullptr;                  // the bias belongs to one slice only
-    const int r16 = lane & 15, g = lane >> 4;
-    const bf16_t* wrow = W + (size_t)min(n0 + r16, N - 1) * K_all + g * 8;
-    const bf16_t* xrow[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xrow[mt] = X + (size_t)min(mt * 16 + r16, M - 1) * K_all + g * 8;
-    f32x4 acc[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    auto load = [&](int k0, SkinnyFrags<MT>& f) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int k = k0 + s * 32;
-            const bool in = k + g * 8 < K;
-            f.w[s].u = in ? *reinterpret_cast<const uint4*>(wrow + k) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                f.x[mt][s].u = in ? *reinterpret_cast<const uint4*>(xrow[mt] + k) : make_uint4(0, 0, 0, 0);
-        }
-    };
-    auto multiply = [&](const SkinnyFrags<MT>& f) {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-                acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[s].v, f.x[mt][s].v, acc[mt], 0, 0, 0);
-    };
-
-    SkinnyFrags<MT> cur, nxt;
-    int k0 = wave * 128;
-    if (k0 < K) load(k0, cur);
-    while (k0 < K) {
-        const int k1 = k0 + NW * 128;
-        if (k1 < K) load(k1, nxt);
-        multiply(cur);
-        cur = nxt;
-        k0 = k1;
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) red[wave][mt][lane][i] = acc[mt][i];
-    __syncthreads();
-    if (wave != 0) return;
-    // D layout of the 16x16 tile: lane holds column lane%16 (an activation row),
-    // rows 4*(lane/16) + i (weight rows)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int m = mt * 16 + r16;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            v[i] = red[0][mt][lane][i];
-#pragma unroll
-            for (int w = 1; w < NW; ++w) v[i] += red[w][mt][lane][i];
-            const int n = n0 + g * 4 + i;
-            if (bias && n < N) v[i] += bias[n];
-        }
-        if (m >= M) continue;
-        if (epilogue == EPI_SWIGLU) {
-#pragma unroll
-            for (int i = 0; i < 4; i += 2) {
-                const int n = n0 + g * 4 + i;
-                if (n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul_fast(epilogue, v[i], v[i + 1]));
-            }
-            continue;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int n = n0 + g * 4 + i;
-            if (n < N) store_f32<TOut>(Y, (size_t)m * N + n, v[i]);
-        }
-    }
-}
-
-template <typename TOut, int MT>
-static void launch_skinny(const bf16_t* x, const bf16_t* w, const float* bias, TOut* y, int m, int n, int k,
-                          Epilogue epilogue, int slices, hipStream_t s) {
-    const int k_per = ((k + slices - 1) / slices + 127) / 128 * 128;
-    dim3 grid((unsigned)((n + 15) / 16), (unsigned)((k + k_per - 1) / k_per));
-    // few chunks of 128 per wave: 4 waves up to 512 of K per block, 8 up to 2048, 16 beyond
-    if (k_per <= 512)
-        k_gemm_bf16_skinny<TOut, MT, 4><<<grid, 4 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
-    else if (k_per <= 2048)
-        k_gemm_bf16_skinny<TOut, MT, 8><<<grid, 8 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
-    else if constexpr (MT <= 2)
-        k_gemm_bf16_skinny<TOut, MT, 16><<<grid, 16 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
-    else   // 64 activation rows keep too many fragments in registers for 1024 threads
-        k_gemm_bf16_skinny<TOut, MT, 8><<<grid, 8 * 64, 0, s>>>(x, w, bias, y, m, n, k, k_per, epilogue);
 }
 
 // ------------------------------------------------------------------ conv input projection + gated conv, single tokens
@@ -1529,16 +1405,9 @@ extern "C" int imparo_in_proj_conv_decode(const void* x, const void* w, const fl
 }
 
 
-// Which kernel takes a product of 17 to 64 rows: 0 for the K-split kernel, else the waves per
-// block of the shared-activation kernel. Measured with cold weights (they never stay in cache
-// between decode steps): from about 12k weight rows on the shared-activation kernel wins at
-// any number of rows; below that it wins when every wave would fetch its own copy of more
-// than 16 activation rows, or when K is long.
-static int stream_waves(int m, int n, int k) {
-    if (n >= 12288) return 4;
-    if (m > 16 || k >= 4096) return 2;
-    return 0;
-}
+// The waves a block of the shared-activation kernel, for products of 17 to 64 rows. Measured with cold weights (they never
+// stay in cache between decode steps): four from about 12k weight rows on, two below.
+static int stream_waves(int n) { return n >= 12288 ? 4 : 2; }
 
 // A slice's length is rounded up to the kernel's step along K; with a ragged K that can leave the
 // last slices empty. The consumer adds every slice it was promised: fewer slices then, all of
@@ -1568,8 +1437,9 @@ extern "C" int imparo_gemm_slices(int m, int n, int k, int dtype) {
         while (slices < 4 && tiles * slices * 2 <= 512 && k / (slices * 2) >= 1024) slices *= 2;
         return whole_slices(slices, k, BG_BK);
     }
-    const int nw = stream_waves(m, n, k);
-    const int rows_per_block = nw ? nw * 16 : 16;
+    // (weight rows a block that the count goes by; with at most 16 rows the kernel takes 16 to 64 as the slices and the CUs
+    // have it, so that 2,048 by 8,192 in four slices are 256 blocks of 32 and 1,024 by 4,608 in eight 512 of 16)
+    const int rows_per_block = n >= 12288 ? 64 : m > 16 || k >= 4096 ? 32 : 16;
     const int blocks = (n + rows_per_block - 1) / rows_per_block;
     int slices = 1;
     while (slices < 8 && blocks * slices * 2 <= 256 && k / (slices * 2) >= 512) slices *= 2;
@@ -1764,28 +1634,19 @@ static bool big_tile_pays(int m, int n, int k) {
 template <typename TOut>
 static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut* y, int m, int n, int k, Epilogue epilogue,
                        int force, int slices, hipStream_t s) {
-    // `force` (for measurements): 1 = K-split kernel, 2/4/8 = shared activations with that many waves
+    // `force` (for measurements): 2/4/8 = shared activations with that many waves
     // 452: the 128 by 128 tile on four stages, at any number of rows
     if (force == 452 && k % slices == 0 && (k / slices) % (4 * DM_BK) == 0 && dma_tile_takes(m, n, k))
         return launch_dma<TOut>(x, w, bias, y, m, n, k, epilogue, 128, 2, slices, s, 4);
     if (m <= ROWS_MAX && force == 0)
         return imparo_few_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue, slices,
                                nullptr, 0, 0.f, s);
-    int nw = stream_waves(m, n, k);
-    if (force == 1) nw = 0;
-    if (force == 2 || force == 4 || force == 8) nw = force;
-    if (m <= 64 && nw) {
+    if (m <= 64) {
+        const int nw = force == 2 || force == 4 || force == 8 ? force : stream_waves(n);
         if (m <= 32)
             launch_stream<TOut, 2>(x, w, bias, y, m, n, k, epilogue, nw, slices, s);
         else
             launch_stream<TOut, 4>(x, w, bias, y, m, n, k, epilogue, nw, slices, s);
-        return launch_status();
-    }
-    if (m <= 64) {
-        if (m <= 32)
-            launch_skinny<TOut, 2>(x, w, bias, y, m, n, k, epilogue, slices, s);
-        else
-            launch_skinny<TOut, 4>(x, w, bias, y, m, n, k, epilogue, slices, s);
     } else {
         // by shape: the tile kernel with loads straight into LDS where it takes the K, as its plan says;
         // `force` (for measurements) 256: the 256x256 tile with register staging
@@ -1823,15 +1684,14 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
 
 
 // `variant` 0 lets the library choose the kernel. The others are for measurements and tests only, so
-// that each kernel can be met at any shape: 1 the K-split kernel, 2, 4 or 8 the shared-activation
-// kernel with that many waves, 256 the 256x256 tile with register staging, 258 / 263 / 262 the tile
+// that each kernel can be met at any shape: 2, 4 or 8 the shared-activation kernel with that many waves (up to 64 rows), 256 the 256x256 tile with register staging, 258 / 263 / 262 the tile
 // with loads straight into LDS at 256 rows by 256 / 192 / 128, 358 / 352 the same at 128 rows by
 // 256 / 128, 558 at 192 rows by 256, 452 the 128 by 128 tile on four stages, 351 / 451 the 128 by 64 tile on two / four stages;
 // with a variant, any number of K slices is taken.
 static int gemm_variant(const void* x, const void* w, const float* bias, void* y, int dtype, int out_dtype,
                         int m, int n, int k, Epilogue epilogue, int slices, int variant, imparo_stream stream) {
     if (!x || !w || !y || m < 0 || n <= 0 || k <= 0) return IMPARO_BAD_ARGUMENT;
-    if (slices < 1) return IMPARO_BAD_ARGUMENT;
+    if (slices < 1 || variant == 1) return IMPARO_BAD_ARGUMENT;      // (1: a kernel that is no more)
     // slices: only what imparo_gemm_slices allows, float32 out, no epilogue that is not linear
     const int slices_ok = imparo_gemm_slices(m, n, k, dtype);
     if (slices > 1 && ((slices != slices_ok && variant == 0) || out_dtype != IMPARO_F32 || epilogue != EPI_NONE))
