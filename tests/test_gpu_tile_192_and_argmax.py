@@ -28,6 +28,12 @@ def test_tile_of_192_rows_against_float64(m, n, k):
     torch.testing.assert_close(gated.double(), u / (1.0 + torch.exp(-u)) * v, rtol=2.0 ** -8 + 1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("m, n, k", [(151, 69516, 3584), (167, 67434, 3584)])
+def test_the_tile_takes_no_slices_place(m, n, k):
+    """Two slices of K are nearer to 64 bits than one piece: these shapes had two before there was the tile."""
+    assert ops.gemm_slices(m, n, k, torch.bfloat16) == 2
+
+
 @pytest.mark.parametrize("vocab", [64, 4096, 65536, 65540, 200000])
 def test_argmax_of_special_rows(vocab):
     g = torch.Generator().manual_seed(vocab)
