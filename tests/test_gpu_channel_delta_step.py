@@ -43,3 +43,24 @@ def test_one_launch_is_the_four(heads, kv_heads, taps, rows_n):
     with pytest.raises(ops.KernelArgumentError):
         ops.channel_delta_step(rows[:, :C].contiguous(), C, steps, H * D, conv_w, conv, bias, rate, state, slot, norm, half, H, Hk, D, D,
                                1e-6, 1.0, 1e-5)
+
+
+@pytest.mark.parametrize("heads, kv_heads, taps", [(1, 1, 4), (4, 2, 3)])
+def test_bfloat16_out_is_the_float32_rounded(heads, kv_heads, taps):
+    """What a bfloat16 engine reads, and a second step on what the first one left."""
+    g = torch.Generator().manual_seed(heads)
+    rnd = lambda *s, scale=1.0: (torch.randn(*s, generator=g) * scale).to(DEV)
+    D, H, Hk, n, slots = 128, heads, kv_heads, 3, 4
+    C = (2 * Hk + H) * D
+    conv_w, conv, state = rnd(C, taps, scale=0.5), rnd(slots, taps - 1, C), rnd(slots, H, D, D, scale=0.3)
+    bias, rate, norm = rnd(H * D, scale=0.5), rnd(H).exp() * 0.1, rnd(H * D)
+    slot = torch.tensor([2, 0, 3], device=DEV, dtype=torch.int32)
+    sides = [(conv.clone(), state.clone(), torch.full((n, H * D), float("nan"), device=DEV, dtype=t)) for t in (torch.float32, torch.bfloat16)]
+    for _ in range(2):
+        rows, steps = rnd(n, C + H), rnd(n, 2 * H * D)
+        for history, kept, out in sides:
+            ops.channel_delta_step(rows, C, steps, H * D, conv_w, history, bias, rate, kept, slot, norm, out, H, Hk, D, D, 1e-6,
+                                   D ** -0.5, 1e-5)
+        (history, kept, whole), (history2, kept2, half) = sides
+        assert torch.equal(half, whole.bfloat16()) and torch.equal(history, history2) and torch.equal(kept, kept2)
+    assert torch.equal(kept[1], state[1]) and torch.equal(history[1], conv[1])       # nobody's slot

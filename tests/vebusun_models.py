@@ -98,8 +98,19 @@ CONFIG_E = dict(
         layer(parallel(left(3, 3, 80, 80, softcap=9.0, window=70, keep=66, rot=80), right(1, 16, 16, [0.97])), None),
     ])
 
-CONFIGS = {"A": (CONFIG_A, 51), "B": (CONFIG_B, 52), "C": (CONFIG_C, 53), "D": (CONFIG_D, 54), "E": (CONFIG_E, 55)}
-RANKS = {"A": (12, 20), "B": (1, 1), "C": (5, 9), "D": (32, 24), "E": (16, 16)}       # inner ranks of decays and gates
+# F: heads of 128 by 128, one and two a query/key head, whose decode steps take everything between the projections in one
+# launch; four, three and one taps
+CONFIG_F = dict(
+    architecture="Vebusun", vocab=150, width=96, norm=dict(eps=1e-5), residual_mult=0.5, embedding=dict(scale=2.0),
+    layers=[
+        layer(delta(2, 1, 128, 128, 4), 64),
+        layer(delta(2, 2, 128, 128, 3), 48),
+        layer(parallel(left(4, 2, 16, 16, softcap=9.0, window=33, keep=20, rot=8, base=2000.0), right(2, 24, 16, [0.85, 0.99])), 56),
+        layer(delta(4, 2, 128, 128, 1), None),
+    ])
+
+CONFIGS = {"A": (CONFIG_A, 51), "B": (CONFIG_B, 52), "C": (CONFIG_C, 53), "D": (CONFIG_D, 54), "E": (CONFIG_E, 55), "F": (CONFIG_F, 56)}
+RANKS = {"A": (12, 20), "B": (1, 1), "C": (5, 9), "D": (32, 24), "E": (16, 16), "F": (24, 16)}       # inner ranks of decays and gates
 
 
 def runs_of(config):
