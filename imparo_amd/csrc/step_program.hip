@@ -487,7 +487,8 @@ extern "C" int imparo_program_set_fold(ImparoProgram* p, int mode) {
 // 2048) with everything folded, with only the products over K <= 2048 folded (the mixers' output
 // projections), and with nothing folded: the second is the fastest everywhere (a step of 8 rows at
 // width 1024: 0.670 ms against 0.702 and 0.718; at width 2048: 0.915 against 0.942 and 0.934); a block
-// that walks a K of 4,608 or more alone takes longer than the norm's launch it saves.
+// that walked a K of 4,608 or more alone took longer than the norm's launch it saved. (With the kernels of then. Whole steps
+// have not been measured since; a row of 1,024 by 4,608 now takes 7.0 us into the stream, in eight slices 4.5.)
 extern "C" int imparo_rows_fold_pays(int m, int n, int k) {
     (void)n;
     return m <= 16 && k <= 2048;
