@@ -183,6 +183,7 @@ int imparo_load_code_rope_cache();
 int imparo_load_code_row_ops();
 int imparo_load_code_sampling();
 int imparo_load_code_selective_scan();
+int imparo_load_code_some_rows();
 int imparo_load_code_streams();
 
 static inline int launch_status() {

@@ -4,7 +4,7 @@
 // its products in the order k = 0, 1, 2, ... whatever the tile it falls in, so a row's
 // result does not depend on how many other rows are in the batch.
 // bfloat16: MFMA kernels, LDS-tiled ones for many rows and weight-streaming ones for some
-// (at most 16 rows: decode_rows.hip).
+// (17 to 128 rows: some_rows.hip; at most 16: decode_rows.hip).
 #include "common.h"
 
 #include <algorithm>
@@ -1410,7 +1410,7 @@ extern "C" int imparo_in_proj_conv_decode(const void* x, const void* w, const fl
 }
 
 
-// The waves a block of the shared-activation kernel, for products of 17 to 64 rows. Measured with cold weights (they never
+// The waves a block of the shared-activation kernel, for products of 17 to 64 rows with a K that is no multiple of 128. Measured with cold weights (they never
 // stay in cache between decode steps): four from about 12k weight rows on, two below.
 static int stream_waves(int n) { return n >= 12288 ? 4 : 2; }
 
@@ -1458,7 +1458,8 @@ extern "C" int imparo_gemm_adds(int m, int n, int k, int dtype) {
 }
 
 
-// ------------------------------------------------------------------ bfloat16, some rows (17..64)
+// ------------------------------------------------------------------ bfloat16, some rows (17..64), any K
+// (K a multiple of 128: some_rows.hip)
 // A block of ST_WAVES waves takes 16 weight rows per wave and up to 16*MT
 // activation rows, and walks its part of K in chunks of 128. The activation
 // chunk is staged in LDS once per block and shared by the waves (with more
@@ -1646,6 +1647,16 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
     if (m <= ROWS_MAX && force == 0)
         return imparo_few_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue, slices,
                                nullptr, 0, 0.f, s);
+    // up to 96 rows the kernel of some_rows.hip, and up to 128 where it takes few weight rows a block: with 64 the tile of 128 by
+    // 64 draws the same bytes a CU with less to do about them (128 rows of 16,384 by 2,048 gated 20.0 us, 20.8 there; 96 rows 19.3
+    // and 18.9, 65 rows 18.9 and 17.5; 128 rows of 6,144 by 2,048 16.9 and 14.5).
+    // 616, 632, 664: that kernel with 16, 32 and 64 weight rows a block
+    if (imparo_some_rows_takes(m, n, k) && (force == 0 || force == 616 || force == 632 || force == 664)) {
+        const int tile = force ? force - 600 : imparo_some_rows_tile(m, n, slices);
+        if (force || m <= 96 || tile <= 32)
+            return imparo_some_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue,
+                                    slices, tile, s);
+    }
     if (m <= 64) {
         const int nw = force == 2 || force == 4 || force == 8 ? force : stream_waves(n);
         if (m <= 32)
@@ -1691,7 +1702,7 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
 // `variant` 0 lets the library choose the kernel. The others are for measurements and tests only, so
 // that each kernel can be met at any shape: 2, 4 or 8 the shared-activation kernel with that many waves (up to 64 rows), 256 the 256x256 tile with register staging, 258 / 263 / 262 the tile
 // with loads straight into LDS at 256 rows by 256 / 192 / 128, 358 / 352 the same at 128 rows by
-// 256 / 128, 558 at 192 rows by 256, 452 the 128 by 128 tile on four stages, 351 / 451 the 128 by 64 tile on two / four stages;
+// 256 / 128, 558 at 192 rows by 256, 616 / 632 / 664 the kernel of 17 to 128 rows with 16 / 32 / 64 weight rows a block, 452 the 128 by 128 tile on four stages, 351 / 451 the 128 by 64 tile on two / four stages;
 // with a variant, any number of K slices is taken.
 static int gemm_variant(const void* x, const void* w, const float* bias, void* y, int dtype, int out_dtype,
                         int m, int n, int k, Epilogue epilogue, int slices, int variant, imparo_stream stream) {

@@ -108,3 +108,11 @@ __device__ __forceinline__ float rows_scale(const float* part, int token, int wi
 // says, each a float32 result of its own in Y; ssq_in (null: none): the rows are scaled at the end.
 int imparo_few_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
                     const Epilogue& epilogue, int slices, const float* ssq_in, int n_parts, float eps, hipStream_t s);
+
+// (some_rows.hip) Products of 17 to SOME_ROWS_MAX rows with a K that is a multiple of 128, any kind; `tile`: weight rows a block, 64, 32 or 16,
+// as imparo_some_rows_tile says.
+#define SOME_ROWS_MAX 128
+bool imparo_some_rows_takes(int m, int n, int k);
+int imparo_some_rows_tile(int m, int n, int slices);
+int imparo_some_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
+                     const Epilogue& epilogue, int slices, int tile, hipStream_t s);
