@@ -412,6 +412,10 @@ int imparo_rows_parts(int n);
 int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts, float eps, const void* w, const float* bias,
                      void* y, int out_dtype, float* x_io, float* ssq_out, void* weighted_out, const float* weighted_by,
                      int m, int n, int k, int epilogue, imparo_stream stream);
+// The same with a norm that has no statistic: x_io [m, n] += the result, and with norm_w and norm_b [n], out [m, n] bfloat16 = tanh(alpha
+// x) norm_w + norm_b of the new rows (all three null: the stream alone).
+int imparo_rows_gemm_tanh(const void* x, const void* w, const float* bias, float* x_io, void* out, float alpha, const float* norm_w,
+                          const float* norm_b, int m, int n, int k, imparo_stream stream);
 
 // state' = the last taps-1 rows of (state ++ B*x) for every request; runs after
 // imparo_short_conv on the same stream.

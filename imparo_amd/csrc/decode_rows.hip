@@ -7,6 +7,8 @@
 //     norm needs is there. Told the weight of the norm that reads the stream next, it also leaves
 //     the new rows times that weight in bfloat16. A block adds the whole of K (no slices of K over
 //     blocks): nothing meets across blocks, so there are no counters and no fences;
+//     Where that norm has no statistic (dynamic tanh), the block leaves the rows behind it: every element is its own, and
+//     nothing is left for the reader to do;
 //   * the activations may be such rows (the stream times a norm's weight, not yet scaled) with the
 //     partial sums of squares beside them: the block multiplies each row's result by the row's scale
 //     rsqrt(sum / K + eps) at the end, in float32 -- no norm launch.
@@ -91,8 +93,8 @@ template <typename TOut, int RB, int RT, int CH, int CHAINS, int EPI, int K_KIND
 __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     const bf16_t* __restrict__ X, const float* __restrict__ ssq_in, int n_parts, float eps,
     const bf16_t* __restrict__ W, const float* __restrict__ bias, TOut* __restrict__ Y, float* __restrict__ x_io,
-    float* __restrict__ ssq_out, bf16_t* __restrict__ weighted_out, const float* __restrict__ weighted_by, int M, int N,
-    int K_all, int k_per, int rounds, int turned, Epilogue unit) {
+    float* __restrict__ ssq_out, bf16_t* __restrict__ weighted_out, const float* __restrict__ weighted_by,
+    const float* __restrict__ tanh_bias, float tanh_alpha, int M, int N, int K_all, int k_per, int rounds, int turned, Epilogue unit) {
     static_assert(RB == 16 || RT == 1, "half tiles one by one");
     constexpr bool RAGGED = K_KIND == ROWS_RAGGED || K_KIND == ROWS_HUGE;
     extern __shared__ float4 red[];                     // [CHAINS][waves][RT][64]
@@ -164,13 +166,14 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     ask(wave + round * turn);
     if (SCALED) rows_ssq_share(part, early, ssq_in, n_parts);
     // needed when the walk is over: what the finishing lanes add to
-    float x_old[4] = {0.f, 0.f, 0.f, 0.f}, by[4] = {0.f, 0.f, 0.f, 0.f};
+    float x_old[4] = {0.f, 0.f, 0.f, 0.f}, by[4] = {0.f, 0.f, 0.f, 0.f}, plus[4] = {0.f, 0.f, 0.f, 0.f};
     if (EPI == ROWS_RESID && wave == 0 && g * 4 < RB && r16 < M) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int n = min(n0 + g * 4 + i, N - 1);
             x_old[i] = x_io[(size_t)r16 * N + n];
             if (weighted_by) by[i] = weighted_by[n];
+            if (tanh_bias) plus[i] = tanh_bias[n];
         }
     }
     f32x4 acc[CHAINS][RT];
@@ -261,11 +264,13 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                     const float xn = __fadd_rn(x_old[i], v[i]);
                     x_io[(size_t)r16 * N + n + i] = xn;
                     sq = fmaf(xn, xn, sq);
-                    if (weighted_out) weighted_out[(size_t)r16 * N + n + i] = f32_to_bf16(xn * by[i]);
+                    if (weighted_out)
+                        weighted_out[(size_t)r16 * N + n + i] =
+                            f32_to_bf16(tanh_bias ? fmaf(tanhf(tanh_alpha * xn), by[i], plus[i]) : xn * by[i]);
                 }
             }
             sq += __shfl_xor(sq, 16, WAVE);             // the two lanes of a token sit 16 apart
-            if (g == 0) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
+            if (g == 0 && ssq_out) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
         }
     }
 }
@@ -342,6 +347,8 @@ struct RowsCall {
     float* ssq_out;
     bf16_t* weighted_out;
     const float* weighted_by;
+    const float* tanh_bias;
+    float tanh_alpha;
     int m, n, k, slices;
     Epilogue unit;
 };
@@ -359,8 +366,8 @@ static void rows_launch_as(const RowsCall& c, hipStream_t s) {
     const size_t lds = (size_t)sh.chains * sh.waves * sh.rt * 64 * sizeof(float4);          // (48 KB at most)
 #define ROWS_GO(RT, CH, CHAINS, KIND)                                                                                \
     k_rows_gemm<TOut, RB, RT, CH, CHAINS, EPI, KIND, SCALED><<<grid, sh.waves * 64, lds, s>>>(                         \
-        c.x, c.ssq_in, c.n_parts, c.eps, c.w, c.bias, (TOut*)c.y, c.x_io, c.ssq_out, c.weighted_out, c.weighted_by, c.m, \
-        c.n, c.k, k_per, rounds, turned, c.unit)
+        c.x, c.ssq_in, c.n_parts, c.eps, c.w, c.bias, (TOut*)c.y, c.x_io, c.ssq_out, c.weighted_out, c.weighted_by, \
+        c.tanh_bias, c.tanh_alpha, c.m, c.n, c.k, k_per, rounds, turned, c.unit)
 #define ROWS_CHAINS(RT, CH, KIND)                                                                                    \
     do {                                                                                                             \
         if (sh.chains == 2) ROWS_GO(RT, CH, 2, KIND);                                                                \
@@ -419,7 +426,8 @@ static void rows_launch(const RowsCall& c, hipStream_t s) {
 
 int imparo_few_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
                     const Epilogue& epilogue, int slices, const float* ssq_in, int n_parts, float eps, hipStream_t s) {
-    const RowsCall c{x, ssq_in, n_parts, eps, w, bias, y, nullptr, nullptr, nullptr, nullptr, m, n, k, slices, epilogue};
+    const RowsCall c{x, ssq_in, n_parts, eps, w, bias, y, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, m, n, k, slices,
+                     epilogue};
     if (m <= 0 || m > ROWS_MAX || n <= 0 || k < 8 || k % 8 || slices < 1) return IMPARO_BAD_ARGUMENT;
     if (epilogue == EPI_SWIGLU && out_dtype == IMPARO_BF16)
         rows_launch<bf16_t, 16, ROWS_SWIGLU>(c, s);
@@ -456,12 +464,24 @@ extern "C" int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts,
     const bf16_t* wb = (const bf16_t*)w;
     bf16_t* wo = (bf16_t*)weighted_out;
     if (epilogue == ROWS_RESID) {
-        rows_launch<float, 8, ROWS_RESID>(RowsCall{xb, ssq_in, n_parts, eps, wb, bias, nullptr, x_io, ssq_out, wo, weighted_by, m, n,
-                                                   k, 1, Epilogue(EPI_NONE)}, s);
+        rows_launch<float, 8, ROWS_RESID>(RowsCall{xb, ssq_in, n_parts, eps, wb, bias, nullptr, x_io, ssq_out, wo, weighted_by, nullptr,
+                                                   0.f, m, n, k, 1, Epilogue(EPI_NONE)}, s);
         return launch_status();
     }
     return imparo_few_rows(xb, wb, bias, y, out_dtype, m, n, k, Epilogue(epilogue == ROWS_SWIGLU ? EPI_SWIGLU : EPI_NONE), 1, ssq_in,
                            n_parts, eps, s);
+}
+
+extern "C" int imparo_rows_gemm_tanh(const void* x, const void* w, const float* bias, float* x_io, void* out, float alpha,
+                                     const float* norm_w, const float* norm_b, int m, int n, int k, imparo_stream stream) {
+    if (!x || !w || !x_io || m < 0 || m > ROWS_MAX || n <= 0 || k <= 0 || k % 8 != 0) return IMPARO_BAD_ARGUMENT;
+    if ((out != nullptr) != (norm_w != nullptr) || (out != nullptr) != (norm_b != nullptr)) return IMPARO_BAD_ARGUMENT;
+    if (((uintptr_t)w & 15) || ((uintptr_t)x & 15)) return IMPARO_BAD_ARGUMENT;
+    if (m == 0) return IMPARO_OK;
+    rows_launch<float, 8, ROWS_RESID>(RowsCall{(const bf16_t*)x, nullptr, 0, 0.f, (const bf16_t*)w, bias, nullptr, x_io, nullptr,
+                                               (bf16_t*)out, norm_w, norm_b, alpha, m, n, k, 1, Epilogue(EPI_NONE)},
+                                      (hipStream_t)stream);
+    return launch_status();
 }
 
 // Asks the runtime about one kernel of this file, which makes it load the file's code onto the

@@ -101,6 +101,9 @@ class Model:
                 if res.streams is not None or res.link is not None:
                     raise ValueError("a stream kept as several copies does not take the embedding's output in again")
                 ops.add_rows(res.x, kept)        # (what is pending on the stream is added by the next norm, as ever)
+            after = self.plan.order[i + 1] if i + 1 < len(self.plan.order) else None
+            tells = after is not None and not after.add_input and emits(self.blocks[after.layer], "first_norm")
+            ctx.next_norm = self.blocks[after.layer].first_norm() if tells else None
             self.blocks[call.layer].forward(ctx, res, self.site_of_call[i], call.cache_of is None)
         if want_rows is None or want_rows.shape[0] == 0:
             return None

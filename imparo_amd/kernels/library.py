@@ -140,6 +140,7 @@ _SIGNATURES = {
     "imparo_post_norm_add": [P, P, I, I, P, P, F, P, F, P, I, I, I, P],
     "imparo_rows_parts": [I],
     # x, ssq_in, n_parts, eps, w, bias, y, out_dtype, x_io, ssq_out, weighted_out, weighted_by, m, n, k, epilogue, stream
+    "imparo_rows_gemm_tanh": [P, P, P, P, P, F, P, P, I, I, I, P],
     "imparo_rows_gemm": [P, P, I, F, P, P, P, I, P, P, P, P, I, I, I, I, P],
     "imparo_in_proj_conv_decode_normed": [P, P, I, F, P, P, P, P, P, P, P, I, I, I, I, I, I, P],
     "imparo_rows_fold_pays": [I, I, I],

@@ -17,6 +17,7 @@ from .library import library
 
 F32, BF16 = 0, 1
 ATTENTION_MAX_HEAD_DIM = 576      # the wave attention kernel's longest key row
+ROWS_MAX = 16                     # tokens of a step that the few-row products with a norm folded in take
 HGRN2_MAX_DIM = 512               # state rows a head of the gated linear recurrence
 _CODES = {torch.float32: F32, torch.bfloat16: BF16}
 
@@ -695,6 +696,26 @@ def rows_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = No
         _dev(weighted_out, "weighted out", torch.bfloat16, (m, n)), _dev(weighted_by, "weighted by", torch.float32, (n,)),
         m, n, k, epilogue, _stream()), "rows_gemm")
     return into if into is not None else out
+
+
+def rows_gemm_tanh(x: torch.Tensor, w: torch.Tensor, into: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                   out: Optional[torch.Tensor] = None, alpha: float = 0.0, norm_weight: Optional[torch.Tensor] = None,
+                   norm_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A product of at most 16 rows, x [m, k] and w [n, k] bfloat16, added to `into` [m, n] float32 in place; `out` [m, n]
+    bfloat16 receives tanh(alpha * row) * norm_weight + norm_bias of the new rows."""
+    m, k = x.shape
+    n, kw = w.shape
+    if kw != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not 0 < m <= 16 or k % 8:
+        raise KernelArgumentError("rows_gemm_tanh: 1 to 16 bfloat16 rows, a bfloat16 weight over the same inner size, "
+                                  "a multiple of 8")
+    if len({t is None for t in (out, norm_weight, norm_bias)}) > 1:
+        raise KernelArgumentError("rows_gemm_tanh: the rows behind the norm need its weight and bias")
+    _check(library().imparo_rows_gemm_tanh(
+        _dev(x, "x"), _dev(w, "weight"), _dev(bias, "bias", torch.float32, (n,)), _dev(into, "stream", torch.float32, (m, n)),
+        _dev(out, "rows behind the norm", torch.bfloat16, (m, n)), float(alpha),
+        _dev(norm_weight, "norm weight", torch.float32, (n,)), _dev(norm_bias, "norm bias", torch.float32, (n,)), m, n, k,
+        _stream()), "rows_gemm_tanh")
+    return into
 
 
 def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> torch.Tensor:

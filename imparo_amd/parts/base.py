@@ -112,6 +112,10 @@ class StepContext:
     # The float32 residual stream while a block runs the part whose result goes into it, with nothing pending
     # on it: the part may add its result there itself and return the stream instead of a delta. None: return a delta.
     stream: Optional[torch.Tensor] = None
+    # With it, the norm that reads the stream next: a product that adds to the stream may take it into its launch.
+    ride: Optional["NormRide"] = None
+    # The norm behind the running block and the dtype its reader asks for, where the next block tells.
+    next_norm: Optional[Tuple[object, torch.dtype]] = None
     # The step's token ids (int32, one a token), for a part that looks a token up in a table of its own.
     token_ids: Optional[torch.Tensor] = None
 
@@ -143,6 +147,15 @@ def emits(part, emit: str = "emit", forward: str = "forward") -> bool:
 
 
 @dataclass
+class NormRide:
+    """The norm that reads the stream next (None: another part adds to the stream first) and the dtype its reader asks
+    for. The product that adds the last of what the norm reads may leave the rows behind the norm in `rows`."""
+    norm: Optional[object]
+    out_dtype: torch.dtype
+    rows: Optional[torch.Tensor] = None
+
+
+@dataclass
 class Residual:
     """The residual stream in float32 and a delta not yet added to it. The
     next norm adds the delta while it reads the row anyway. The delta is
@@ -159,6 +172,8 @@ class Residual:
     # the stream next mixes them in its own launch.
     streams: Optional[torch.Tensor] = None
     link: Optional[object] = None
+    # Left by the product before, where the next norm rode in its launch: that norm and its rows.
+    normed: Optional[NormRide] = None
 
 
 def one_delta(res: Residual) -> None:

@@ -17,7 +17,7 @@ import torch
 
 from ..cache.pages import with_fixed_arrays
 from ..kernels import ops
-from .base import Residual, StepContext, emits
+from .base import NormRide, Residual, StepContext, emits
 from .registry import register_part
 
 
@@ -54,10 +54,16 @@ class PreNormBlock:
         else:
             h = self.shift.forward(ctx, site, self.mixer_norm.forward(ctx, res, torch.float32, name="normed_f32"),
                                    self.mixer.in_dtype)
-        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h))
+        behind = ctx.next_norm if self.ffn is None else (self.ffn_norm, self.ffn.in_dtype)
+        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h), behind)
         if self.ffn is not None:
             n = self.ffn_norm.forward(ctx, res, self.ffn.in_dtype)
-            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n))
+            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n), ctx.next_norm)
+
+    def first_norm(self):
+        """The norm that reads the stream first and the dtype its rows are asked for in, if it may ride with the product before
+        this block."""
+        return None if self.shift is not None else (self.mixer_norm, self.mixer.in_dtype)
 
     def can_emit(self) -> bool:
         if self.shift is not None or self.ffn is None:
@@ -73,14 +79,19 @@ class PreNormBlock:
         self.ffn.emit(program)
 
     @staticmethod
-    def _delta(ctx: StepContext, res: Residual, run):
+    def _delta(ctx: StepContext, res: Residual, run, behind=None):
         """Runs a part whose result goes into the stream. With nothing pending the part may add its
-        result to the stream itself (it then returns the stream); otherwise it returns a delta."""
+        result to the stream itself (it then returns the stream); otherwise it returns a delta.
+        `behind`: the norm that reads the stream next and the dtype of its rows; a norm that can rides with
+        the part's last product."""
         ctx.stream = res.x if res.pending is None else None
+        ctx.ride = NormRide(*behind) if ctx.stream is not None and behind and hasattr(behind[0], "ride") else None
+        ride = ctx.ride
         try:
             delta = run()
         finally:
-            ctx.stream = None
+            ctx.stream = ctx.ride = None
+        res.normed = ride if ride is not None and ride.rows is not None and delta is res.x else None
         return None if delta is res.x else delta
 
 
@@ -109,6 +120,9 @@ class SandwichBlock(PreNormBlock):
             # a feed-forward that can leave its last sum to the norm's launch does (`forward_rows`)
             run = getattr(self.ffn, "forward_rows", None) or self.ffn.forward
             res.pending, res.post = run(ctx, n), self.ffn_post.as_post()
+
+    def first_norm(self):
+        return None
 
     def can_emit(self) -> bool:
         return False          # the step program knows the pre-norm block only

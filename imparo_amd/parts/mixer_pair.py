@@ -29,7 +29,7 @@ from ..cache.pages import FixedArray, FixedSpec, PagedSpec, fixed_part
 from ..config.plan import PartSpec
 from ..kernels import ops
 from ..weights.loader import TensorDecl
-from .base import Declared, StepContext
+from .base import Declared, NormRide, StepContext
 from .linear import place_vector
 from .registry import part_class, register_part
 
@@ -55,8 +55,8 @@ class _Scoped:
     its own, under its own names; the stream to add into only where the pair's result is the plain sum."""
 
     def __init__(self, ctx: StepContext, prefix: str, scratch_prefix: str = "",
-                 stream: Optional[torch.Tensor] = None):
-        self._ctx, self._prefix = ctx, prefix
+                 stream: Optional[torch.Tensor] = None, ride: Optional[NormRide] = None):
+        self._ctx, self._prefix, self.ride = ctx, prefix, ride
         self.workspace = _ScopedWorkspace(ctx.workspace, scratch_prefix) if scratch_prefix else ctx.workspace
         self.stream = stream
 
@@ -129,8 +129,11 @@ class MixerPair:
     def forward(self, ctx: StepContext, site: int, owns_cache: bool, h: torch.Tensor) -> torch.Tensor:
         if not self.normed:
             stream = ctx.stream
-            a = self.left.forward(_Scoped(ctx, "left.", "left:", stream), site, owns_cache, h)
-            b = self.right.forward(_Scoped(ctx, "right.", stream=stream), site, owns_cache, h)
+            ride = ctx.ride
+            first = None if ride is None else NormRide(None, ride.out_dtype)      # (the norm behind both rides with the second)
+            a = self.left.forward(_Scoped(ctx, "left.", "left:", stream, first), site, owns_cache, h)
+            ride = ride if stream is not None and a is stream else None
+            b = self.right.forward(_Scoped(ctx, "right.", stream=stream, ride=ride), site, owns_cache, h)
             deltas = tuple(d for d in (a, b) if stream is None or d is not stream)
             return stream if not deltas else deltas[0] if len(deltas) == 1 else deltas
         a = self.left.forward(_Scoped(ctx, "left.", "left:"), site, owns_cache, h)

@@ -260,9 +260,19 @@ class DynamicTanh:
 
     def forward(self, ctx: StepContext, res: Residual, out_dtype: torch.dtype, name: str = "normed") -> torch.Tensor:
         """Adds what is pending into the stream (if anything) and returns the rows behind the norm in `out_dtype`."""
+        normed, res.normed = res.normed, None
+        if normed is not None and normed.norm is self and normed.out_dtype == out_dtype and res.pending is None:
+            return normed.rows
         out = ctx.workspace.get(name, tuple(res.x.shape), out_dtype)
         deltas, res.pending = self._deltas(res), None
         return ops.dynamic_tanh(res.x, self.alpha, self.weight, self.bias, out, deltas, write_back=bool(deltas))
+
+    def ride(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], into: torch.Tensor,
+             rows: torch.Tensor) -> torch.Tensor:
+        """into += x . weight^T (+ bias), and `rows` the new stream behind this norm, in one launch (a part that has this
+        method may ride with the product before it)."""
+        return ops.rows_gemm_tanh(x, weight, into, bias=bias, out=rows, alpha=self.alpha, norm_weight=self.weight,
+                                  norm_bias=self.bias)
 
     def forward_rows(self, ctx: StepContext, res: Residual, rows: torch.Tensor, out_dtype: torch.dtype,
                      name: str = "normed_rows") -> torch.Tensor:

@@ -1,0 +1,69 @@
+"""A norm without a statistic in the launch of the product before it: against the two launches, and whole models with and without."""
+import pytest
+import torch
+
+from imparo_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def rnd(*shape, seed, scale=1.0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale
+
+
+# one block partly past the end, more columns than blocks of 8, one chunk of K, a ragged K, two chains of sums
+@pytest.mark.parametrize("n, k", [(8, 128), (41, 72), (1024, 1024), (130, 3072), (2056, 4224)])
+@pytest.mark.parametrize("m", [1, 5, 16])
+@pytest.mark.parametrize("biased", [False, True])
+def test_product_with_the_norm_behind_it(n, k, m, biased):
+    x, w = rnd(m, k, seed=1).bfloat16().to(DEV), rnd(n, k, seed=2, scale=0.05).bfloat16().to(DEV)
+    b = rnd(n, seed=3).to(DEV) if biased else None
+    held, nw, nb = (rnd(*s, seed=i).to(DEV) for i, s in ((4, (m, n)), (5, (n,)), (6, (n,))))
+    stream, plain = held.clone(), held.clone()
+    rows = torch.full((m, n), float("nan"), device=DEV, dtype=torch.bfloat16)
+    ops.rows_gemm_tanh(x, w, stream, bias=b, out=rows, alpha=0.7, norm_weight=nw, norm_bias=nb)
+    ssq = torch.empty(ops.rows_parts(n), 16, device=DEV)
+    ops.rows_gemm(x, w, bias=b, into=plain, ssq_out=ssq)
+    assert torch.equal(stream, plain)                        # the stream has the bits it has without a norm
+    want = torch.empty_like(rows)
+    ops.dynamic_tanh(plain, 0.7, nw, nb, want, ())
+    assert torch.equal(rows, want)
+    alone = held.clone()
+    ops.rows_gemm_tanh(x, w, alone, bias=b)
+    assert torch.equal(alone, plain)
+    with pytest.raises(ops.KernelArgumentError):
+        ops.rows_gemm_tanh(x, w, alone, out=rows, alpha=0.7)
+    with pytest.raises(ops.KernelArgumentError):
+        ops.rows_gemm_tanh(x, w, alone[:, :n - 1].contiguous())
+
+
+def test_a_models_steps_with_and_without(tmp_path, monkeypatch):
+    """Prompts and decoded tokens of a model whose layers' norms ride (delta rule, and attention beside lightning attention)."""
+    from imparo_amd import Engine, StepEntry, write_random_model
+    from imparo_amd.parts import linear
+    mixers = [dict(type="channel_delta", mixer=dict(heads=2, kv_heads=1, dim=128, vdim=128, conv=4)),
+              dict(type="parallel", mixer=dict(
+                  left=dict(heads=4, kv_heads=2, dim=64, vdim=64, scale=0.125, softcap=30.0, mask=dict(size=64, keep_first=4),
+                            rot=dict(dims=64, base=10000.0)),
+                  right=dict(heads=2, dim=128, vdim=128, decay=[0.9, 0.99]), left_scale=0.8, right_scale=0.6))]
+    config = dict(architecture="Vebusun", vocab=256, width=256, norm=dict(eps=1e-5), residual_mult=0.5, embedding=dict(scale=1.0),
+                  layers=[dict(mixers[i % 2], mlp=dict(kind="dense", ff=512)) for i in range(4)])
+    folder = str(tmp_path)
+    write_random_model(config, 3, folder, layer_gain=4.0)
+    calls, ride = [], ops.rows_gemm_tanh
+    monkeypatch.setattr(ops, "rows_gemm_tanh", lambda *a, **k: (calls.append(k.get("out") is not None), ride(*a, **k))[1])
+    results = []
+    for most in (linear.RIDE_MAX_K, 0):
+        monkeypatch.setattr(linear, "RIDE_MAX_K", most)
+        engine, logits = Engine(folder, dtype="bfloat16", max_tokens=512, max_requests=4), []
+        for step in range(5):
+            tokens = [[(7 * i + j) % 256 for j in range(5 + i)] if step == 0 else [(31 * step + i) % 256] for i in range(3)]
+            logits.append(engine.step([StepEntry(i, t, [len(t) - 1]) for i, t in enumerate(tokens)]).clone())
+        results.append((torch.stack(logits), len(calls), sum(calls)))
+        calls.clear()
+    # the first step's 18 tokens have kernels of their own; then every product into the stream but a last block's way back rides
+    (with_, n, normed), (without, none, _) = results
+    assert n > 0 and n % 9 == 0 and normed * 9 == n * 7 and none == 0
+    # (bfloat16 rows of the same float32 stream, whose sums come in another order)
+    assert float((with_ - without).norm() / without.norm()) < 0.02
