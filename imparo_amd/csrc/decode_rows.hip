@@ -57,6 +57,7 @@ union RowFrag {
 #define ROWS_STORE 0
 #define ROWS_SWIGLU 1
 #define ROWS_RESID 2
+#define ROWS_TANH 3          // into the stream, and the rows behind a norm without a statistic
 #define ROWS_WAVES 8         // of a block at most
 #define ROWS_TURNED 8192     // from this K on blocks start their walks at different places
 
@@ -86,7 +87,7 @@ template <typename TOut> __device__ __forceinline__ void rows_store(TOut* dst, c
 }
 
 // CHAINS: sums that a wave's chunks go into by turns; the chains' sums are added in the order of their first chunks.
-// RB: weight rows of a tile, 16 or 8 (the other lanes ask for nothing; RT 1). CH: chunks of 128 of K that a wave has in
+// RB: weight rows of a tile, 16, 8 or 4 (the other lanes ask for nothing; RT 1). CH: chunks of 128 of K that a wave has in
 // flight at once. SCALED: ssq_in is there. With slices (gridDim.y > 1) block (x, y) sums K range [y * k_per, (y+1) * k_per)
 // into Y + y * M * N and the consumer adds the slices.
 template <typename TOut, int RB, int RT, int CH, int CHAINS, int EPI, int K_KIND, bool SCALED>
@@ -167,13 +168,13 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     if (SCALED) rows_ssq_share(part, early, ssq_in, n_parts);
     // needed when the walk is over: what the finishing lanes add to
     float x_old[4] = {0.f, 0.f, 0.f, 0.f}, by[4] = {0.f, 0.f, 0.f, 0.f}, plus[4] = {0.f, 0.f, 0.f, 0.f};
-    if (EPI == ROWS_RESID && wave == 0 && g * 4 < RB && r16 < M) {
+    if ((EPI == ROWS_RESID || EPI == ROWS_TANH) && wave == 0 && g * 4 < RB && r16 < M) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int n = min(n0 + g * 4 + i, N - 1);
             x_old[i] = x_io[(size_t)r16 * N + n];
             if (weighted_by) by[i] = weighted_by[n];
-            if (tanh_bias) plus[i] = tanh_bias[n];
+            if (EPI == ROWS_TANH && tanh_bias) plus[i] = tanh_bias[n];
         }
     }
     f32x4 acc[CHAINS][RT];
@@ -215,8 +216,16 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
         round = round + 1 == rounds ? 0 : round + 1;
         if (left > 1 && wave + round * turn < n_chunks) ask(wave + round * turn);
     } while (--left > 0);
+    // into the stream in one piece stands for slices of K and may not be further from 64 bits than they are: a wave's chains are
+    // added in pairs here, the waves' sums in pairs below
+    if constexpr (EPI == ROWS_TANH) {
 #pragma unroll
-    for (int c = 0; c < CHAINS; ++c)
+        for (int c = 0; c + 1 < CHAINS; c += 2) acc[c][0] += acc[c + 1][0];
+        if constexpr (CHAINS > 2) acc[0][0] += acc[2][0];
+    }
+    constexpr int LEFT = EPI == ROWS_TANH ? 1 : CHAINS;      // sums a wave leaves
+#pragma unroll
+    for (int c = 0; c < LEFT; ++c)
 #pragma unroll
         for (int t = 0; t < RT; ++t)
             red[((c * waves + wave) * RT + t) * 64 + lane] = make_float4(acc[c][t][0], acc[c][t][1], acc[c][t][2], acc[c][t][3]);
@@ -224,14 +233,26 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     if (g * 4 >= RB) return;
     // D layout of the 16x16 tile: lane holds column lane % 16 (a token), rows 4 * (lane / 16) + i (weight rows)
     for (int t = wave; t < RT; t += waves) {
-        float4 sums[CHAINS * ROWS_WAVES];
+        float4 sums[LEFT * ROWS_WAVES];
 #pragma unroll
-        for (int q = 0; q < CHAINS * ROWS_WAVES; ++q) sums[q] = red[(min(q, CHAINS * waves - 1) * RT + t) * 64 + lane];
+        for (int q = 0; q < LEFT * ROWS_WAVES; ++q) sums[q] = red[(min(q, LEFT * waves - 1) * RT + t) * 64 + lane];
         const float scale = SCALED ? rows_scale(part, token, K, eps) : 1.f;
-        float v[4] = {sums[0].x, sums[0].y, sums[0].z, sums[0].w};
+        if constexpr (EPI == ROWS_TANH) {
 #pragma unroll
-        for (int q = 1; q < CHAINS * ROWS_WAVES; ++q)
-            if (q < CHAINS * waves) v[0] += sums[q].x, v[1] += sums[q].y, v[2] += sums[q].z, v[3] += sums[q].w;
+            for (int w = 1; w < ROWS_WAVES; ++w)
+                if (w >= waves) sums[w] = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int half = ROWS_WAVES / 2; half > 0; half /= 2)
+#pragma unroll
+                for (int w = 0; w < half; ++w)
+                    sums[w].x += sums[w + half].x, sums[w].y += sums[w + half].y, sums[w].z += sums[w + half].z, sums[w].w += sums[w + half].w;
+        }
+        float v[4] = {sums[0].x, sums[0].y, sums[0].z, sums[0].w};
+        if constexpr (EPI != ROWS_TANH) {
+#pragma unroll
+            for (int q = 1; q < CHAINS * ROWS_WAVES; ++q)
+                if (q < CHAINS * waves) v[0] += sums[q].x, v[1] += sums[q].y, v[2] += sums[q].z, v[3] += sums[q].w;
+        }
         const int n = n0 + t * 16 + g * 4;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -266,11 +287,12 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                     sq = fmaf(xn, xn, sq);
                     if (weighted_out)
                         weighted_out[(size_t)r16 * N + n + i] =
-                            f32_to_bf16(tanh_bias ? fmaf(tanhf(tanh_alpha * xn), by[i], plus[i]) : xn * by[i]);
+                            f32_to_bf16(EPI == ROWS_TANH ? fmaf(tanhf(tanh_alpha * xn), by[i], plus[i]) : xn * by[i]);
                 }
             }
+            if (EPI == ROWS_TANH) continue;
             sq += __shfl_xor(sq, 16, WAVE);             // the two lanes of a token sit 16 apart
-            if (g == 0 && ssq_out) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
+            if (g == 0) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
         }
     }
 }
@@ -418,6 +440,24 @@ static void rows_launch_as(const RowsCall& c, hipStream_t s) {
 #undef ROWS_GO
 }
 
+// A sum for every chunk a wave has in flight (up to four; K of 4,096 is one round), added in pairs: errors of 1,024 weight rows
+// against 64 bits 7.7e-8 over K of 1,024 and 8.7e-8 over 3,072, where a chain a wave, added one after the other, had 8.3e-8 and
+// 1.2e-7 and slices of K that the norm adds have 7.8e-8 and 8.7e-8.
+template <int RB, int CH>
+static void rows_launch_tanh(const RowsCall& c, const RowsShape& sh, hipStream_t s) {
+    const int rounds = ((c.k + 127) / 128 + sh.waves * CH - 1) / (sh.waves * CH), turned = sh.turned ? rounds : 0;
+    const dim3 grid((unsigned)((c.n + RB - 1LL) / RB));
+    const size_t lds = (size_t)sh.waves * 64 * sizeof(float4);
+#define ROWS_GO(KIND)                                                                                                  \
+    k_rows_gemm<float, RB, 1, CH, CH, ROWS_TANH, KIND, false><<<grid, sh.waves * 64, lds, s>>>(                          \
+        c.x, nullptr, 0, 0.f, c.w, c.bias, nullptr, c.x_io, nullptr, c.weighted_out, c.weighted_by, c.tanh_bias, c.tanh_alpha, \
+        c.m, c.n, c.k, c.k, rounds, turned, c.unit)
+    if (c.k % 128) ROWS_GO(ROWS_RAGGED);
+    else if (CH == 1 || c.k % (128 * sh.waves * CH) == 0) ROWS_GO(ROWS_WHOLE);
+    else ROWS_GO(ROWS_UNEVEN);
+#undef ROWS_GO
+}
+
 template <typename TOut, int RB, int EPI>
 static void rows_launch(const RowsCall& c, hipStream_t s) {
     if (c.ssq_in) rows_launch_as<TOut, RB, EPI, true>(c, s);
@@ -476,11 +516,25 @@ extern "C" int imparo_rows_gemm_tanh(const void* x, const void* w, const float* 
                                      const float* norm_w, const float* norm_b, int m, int n, int k, imparo_stream stream) {
     if (!x || !w || !x_io || m < 0 || m > ROWS_MAX || n <= 0 || k <= 0 || k % 8 != 0) return IMPARO_BAD_ARGUMENT;
     if ((out != nullptr) != (norm_w != nullptr) || (out != nullptr) != (norm_b != nullptr)) return IMPARO_BAD_ARGUMENT;
-    if (((uintptr_t)w & 15) || ((uintptr_t)x & 15)) return IMPARO_BAD_ARGUMENT;
+    if (((uintptr_t)w & 15) || ((uintptr_t)x & 15) || k >= (1 << 25)) return IMPARO_BAD_ARGUMENT;
     if (m == 0) return IMPARO_OK;
-    rows_launch<float, 8, ROWS_RESID>(RowsCall{(const bf16_t*)x, nullptr, 0, 0.f, (const bf16_t*)w, bias, nullptr, x_io, nullptr,
-                                               (bf16_t*)out, norm_w, norm_b, alpha, m, n, k, 1, Epilogue(EPI_NONE)},
-                                      (hipStream_t)stream);
+    const RowsCall c{(const bf16_t*)x, nullptr, 0, 0.f, (const bf16_t*)w, bias, nullptr, x_io, nullptr, (bf16_t*)out, norm_w, norm_b,
+                     alpha, m, n, k, 1, Epilogue(EPI_NONE)};
+    const RowsShape sh = rows_shape(m, n, k, k, 1, 8);
+    const int a_wave = ((k + 127) / 128 + sh.waves - 1) / sh.waves;
+    hipStream_t s = (hipStream_t)stream;
+    // four weight rows a block while those make no more blocks than CUs: 4 rows of 1,024 by 3,072 5.9 -> 5.5 us, by 1,024 4.1 -> 3.8; of
+    // 1,536 by 3,072 6.3 -> 8.8
+#define ROWS_TANH_GO(RB)                                     \
+    do {                                                     \
+        if (a_wave == 1) rows_launch_tanh<RB, 1>(c, sh, s);  \
+        else if (a_wave == 2) rows_launch_tanh<RB, 2>(c, sh, s); \
+        else if (a_wave == 3) rows_launch_tanh<RB, 3>(c, sh, s); \
+        else rows_launch_tanh<RB, 4>(c, sh, s);              \
+    } while (0)
+    if (n <= 1024) ROWS_TANH_GO(4);
+    else ROWS_TANH_GO(8);
+#undef ROWS_TANH_GO
     return launch_status();
 }
 

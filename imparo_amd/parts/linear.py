@@ -14,10 +14,11 @@ import torch
 from ..kernels import ops
 from .base import StepContext
 
-# Up to this inner size a product of at most 16 rows that sums the whole of K in a block and takes a norm without a statistic
-# along beats slices of K and a launch for the norm: 1,024 weight rows over 1,024 4.8 us against 4.2 and 3.3, over 3,072 6.0 against
-# 4.3 and 3.3, over 4,608 8.2 against 4.8 and 3.3.
+# Up to this inner size and this many activations a product of at most 16 rows that sums the whole of K in a block and takes a norm
+# without a statistic along beats slices of K and a launch for the norm (in a graph, cold weights): 4 rows of 1,024 weight rows
+# over 1,024 3.8 us against 5.8, over 3,072 5.5 against 6.4, 8 rows 5.8 and 6.4, but 16 rows 7.0 and 6.7: every block reads all of them.
 RIDE_MAX_K = 4096
+RIDE_MAX_ACTIVATIONS = 36864
 
 
 class Linear:
@@ -47,7 +48,8 @@ class Linear:
         width = self.out_features // 2 if swiglu else self.out_features
         m = x.shape[0]
         ride = ctx.ride if into is not None else None
-        if (ride is not None and not swiglu and m <= ops.ROWS_MAX and self.in_features <= RIDE_MAX_K and x.dtype == torch.bfloat16
+        if (ride is not None and not swiglu and m <= ops.ROWS_MAX and self.in_features <= RIDE_MAX_K
+                and m * self.in_features <= RIDE_MAX_ACTIVATIONS and x.dtype == torch.bfloat16
                 and self.weight.dtype == torch.bfloat16 and self.in_features % 8 == 0 and ride.out_dtype == torch.bfloat16
                 and into.dtype == torch.float32 and tuple(into.shape) == (m, width) and into.is_contiguous()):
             # a few rows: the product adds to the stream and takes the norm behind it along

@@ -13,25 +13,37 @@ def rnd(*shape, seed, scale=1.0):
 
 
 # one block partly past the end, more columns than blocks of 8, one chunk of K, a ragged K, two chains of sums
-@pytest.mark.parametrize("n, k", [(8, 128), (41, 72), (1024, 1024), (130, 3072), (2056, 4224)])
+@pytest.mark.parametrize("n, k", [(8, 128), (41, 72), (1024, 1024), (130, 3072), (72, 4096), (2056, 4224)])
 @pytest.mark.parametrize("m", [1, 5, 16])
 @pytest.mark.parametrize("biased", [False, True])
 def test_product_with_the_norm_behind_it(n, k, m, biased):
     x, w = rnd(m, k, seed=1).bfloat16().to(DEV), rnd(n, k, seed=2, scale=0.05).bfloat16().to(DEV)
     b = rnd(n, seed=3).to(DEV) if biased else None
     held, nw, nb = (rnd(*s, seed=i).to(DEV) for i, s in ((4, (m, n)), (5, (n,)), (6, (n,))))
-    stream, plain = held.clone(), held.clone()
+    stream = held.clone()
     rows = torch.full((m, n), float("nan"), device=DEV, dtype=torch.bfloat16)
     ops.rows_gemm_tanh(x, w, stream, bias=b, out=rows, alpha=0.7, norm_weight=nw, norm_bias=nb)
-    ssq = torch.empty(ops.rows_parts(n), 16, device=DEV)
-    ops.rows_gemm(x, w, bias=b, into=plain, ssq_out=ssq)
-    assert torch.equal(stream, plain)                        # the stream has the bits it has without a norm
+    y = x.double() @ w.double().t() + (0.0 if b is None else b.double())
+    # a float32 sum of k products and of two more terms, in any order
+    bound = (x.double().abs() @ w.double().abs().t() + held.double().abs() + 4.0) * (k + 3) * 2.0 ** -24
+    assert bool(((stream.double() - (held.double() + y)).abs() <= bound).all())
     want = torch.empty_like(rows)
-    ops.dynamic_tanh(plain, 0.7, nw, nb, want, ())
-    assert torch.equal(rows, want)
+    ops.dynamic_tanh(stream, 0.7, nw, nb, want, ())
+    assert torch.equal(rows, want)                           # the rows that the norm's own launch makes of that stream
     alone = held.clone()
     ops.rows_gemm_tanh(x, w, alone, bias=b)
-    assert torch.equal(alone, plain)
+    assert torch.equal(alone, stream)
+    # and no further from 64 bits than the slices of K that it stands for, added in order
+    slices = ops.gemm_slices(m, n, k, torch.bfloat16)
+    if slices > 1 and k <= 4096 and not biased:
+        parts, zero = torch.empty(slices, m, n, device=DEV), torch.zeros(m, n, device=DEV)
+        ops.gemm(x, w, parts)
+        ops.rows_gemm_tanh(x, w, zero)
+        total = parts[0]
+        for part in parts[1:]:
+            total = total + part
+        # (errors of 8e-8 over thousands of outputs; a tenth is more than samples of one row differ by)
+        assert float((zero.double() - y).norm()) <= 1.1 * float((total.double() - y).norm())
     with pytest.raises(ops.KernelArgumentError):
         ops.rows_gemm_tanh(x, w, alone, out=rows, alpha=0.7)
     with pytest.raises(ops.KernelArgumentError):
