@@ -278,6 +278,15 @@ int imparo_channel_delta_step(const float* rows, int ld, int beta_off, const flo
                               float* state, int n_slots, const int32_t* slot, const float* norm, void* out, int out_dtype,
                               int n_rows, int heads, int kv_heads, int dim, int vdim, float unit_eps, float q_scale, float eps,
                               imparo_stream stream);
+// The same behind a projection that has done the conv (imparo_rows_gemm_conv), for any number of heads a query/key head: rows hold
+// q | k | v behind conv and SiLU, b from beta_off on, and from low_off on rank_a + rank_g inner numbers of the decays' and the gate's
+// bottlenecks, which are rounded to bfloat16 and multiplied by high [2 heads dim, high_ld] bfloat16 (the first heads dim rows
+// by the first rank_a of them, the others by the rest).
+int imparo_channel_delta_heads_takes(int heads, int kv_heads, int dim, int vdim, int taps, int rank_a, int rank_g);
+int imparo_channel_delta_heads(const float* rows, int ld, int beta_off, int low_off, const void* high, int high_ld, int rank_a,
+                               int rank_g, const float* step_bias, const float* rate, float* state, int n_slots,
+                               const int32_t* slot, const float* norm, void* out, int out_dtype, int n_rows, int heads,
+                               int kv_heads, float unit_eps, float q_scale, float eps, imparo_stream stream);
 // out[t] = factor (rms_norm(a[t]) wa + rms_norm(b[t]) wb); a and b float32 [slices, tokens, width], added in order.
 int imparo_normed_sum(const float* a, int a_slices, const float* wa, const float* b, int b_slices, const float* wb,
                       float* out, int n_tokens, int width, float eps, float factor, imparo_stream stream);
@@ -412,7 +421,11 @@ int imparo_rows_parts(int n);
 int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts, float eps, const void* w, const float* bias,
                      void* y, int out_dtype, float* x_io, float* ssq_out, void* weighted_out, const float* weighted_by,
                      int m, int n, int k, int epilogue, imparo_stream stream);
-// The same with a norm that has no statistic: x_io [m, n] += the result, and with norm_w and norm_b [n], out [m, n] bfloat16 = tanh(alpha
+// y [m, n] float32, the first `channels` columns (a multiple of 4) through a causal conv a channel (conv_w [channels, taps], at most four
+// taps, hist [slots, taps - 1, channels] the request's last inputs, shifted in place, row r in slot[r]) and SiLU. slot: distinct.
+int imparo_rows_gemm_conv(const void* x, const void* w, float* y, const float* conv_w, float* hist, const int32_t* slot, int taps,
+                          int channels, int m, int n, int k, imparo_stream stream);
+// Epilogue 2 with a norm that has no statistic: x_io [m, n] += the result, and with norm_w and norm_b [n], out [m, n] bfloat16 = tanh(alpha
 // x) norm_w + norm_b of the new rows (all three null: the stream alone).
 int imparo_rows_gemm_tanh(const void* x, const void* w, const float* bias, float* x_io, void* out, float alpha, const float* norm_w,
                           const float* norm_b, int m, int n, int k, imparo_stream stream);

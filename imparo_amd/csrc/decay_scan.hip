@@ -1216,6 +1216,180 @@ __global__ __launch_bounds__(1024) void k_channel_delta_step(const ChannelStepAr
     store_f32<TOut>(out, ((size_t)r * H + h0) * D + tid, y * rs * norm * ds_sigmoid(gate));
 }
 
+// The same a head and block, where the conv is done (it rides in the projection's launch) and the decays and the gate come
+// through their bottleneck here: the head's rows of the matrix that leads back up, 64 KB of bfloat16 for a rank of 128, are
+// asked for together with its state and multiplied while that is on its way, where they were a launch of their own. Nothing is
+// left that two heads would share and change, so a query/key head's heads no longer share a block. Four neighbouring
+// threads have a decay's or gate's sum. Measured in a graph, 4 rows of 8 heads, rank 128, width 1,024: 7.1 -> 6.0 us, and from
+// the normed rows to the output projection's 17.3 us in four launches -> 10.5 in two; 1 row 16.7 -> 10.2, 16 rows 21.5 -> 13.6.
+struct ChannelHeadArgs {
+    const float* rows; int ld, beta_off, low_off;            // q | k | v behind conv and SiLU .., b, the bottlenecks' inner numbers
+    const bf16_t* high; int high_ld, rank_a, rank_g;         // [2 * heads * 128, high_ld]: decays read columns 0 .. rank_a - 1,
+                                                             // gates (from row heads * 128 on) rank_a .. rank_a + rank_g - 1
+    const float* step_bias; const float* rate;               // [heads * 128], [heads]
+    float* state;                                            // [slots, heads, 128, 128]
+    const int32_t* slot;
+    const float* norm;                                       // [heads * 128]
+    int heads, kv_heads;
+    float unit_eps, q_scale, eps;
+};
+#define CDH_RANK 128
+
+template <int N>
+__device__ __forceinline__ float cdh_quad(float v) {         // the lane N (1 or 2) apart among four neighbours
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), N == 1 ? 0xB1 : 0x4E, 0xf, 0xf, false));
+}
+
+template <typename TOut>
+__global__ __launch_bounds__(1024) void k_channel_delta_head(const ChannelHeadArgs A, TOut* __restrict__ out) {
+    constexpr int D = CDS_DIM, WAVES = 16;
+    __shared__ __attribute__((aligned(16))) float sq[D], sk[D], sv[D], sg[D], su[D], gates[D], low[2 * CDH_RANK];
+    __shared__ __attribute__((aligned(16))) float red[WAVES][D];
+    __shared__ float squares[4], part[2], beta;
+    const int r = blockIdx.x, h = blockIdx.y, kh = h / (A.heads / A.kv_heads);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c4 = (tid & 31) * 4, k0 = (tid >> 5) * 4;      // this thread's columns and rows of the state
+    const float* row = A.rows + (size_t)r * A.ld;
+    const int ranks = A.rank_a + A.rank_g;
+    // what the block needs first, then the weights, then the state
+    float mine = 0.f;
+    if (tid < 3 * D) mine = row[tid < D ? kh * D + tid : tid < 2 * D ? (A.kv_heads + kh) * D + (tid - D) : (2 * A.kv_heads + h) * D + (tid - 2 * D)];
+    else if (tid >= 512 && tid < 512 + ranks) mine = row[A.low_off + tid - 512];
+    else if (tid == 3 * D) mine = row[A.beta_off + h];
+    const int dot = tid >> 2, piece = tid & 3;               // decays 0 .. 127, then gates
+    const bool gate = dot >= D;
+    const int rank = gate ? A.rank_g : A.rank_a;
+    const bf16_t* high = A.high + (size_t)((gate ? A.heads * D : 0) + h * D + (dot & (D - 1))) * A.high_ld + (gate ? A.rank_a : 0);
+    uint4 w[CDH_RANK / 32];
+#pragma unroll
+    for (int j = 0; j < CDH_RANK / 32; ++j) w[j] = *reinterpret_cast<const uint4*>(high + min((j * 4 + piece) * 8, rank - 8));
+    const float bias = A.step_bias[h * D + (dot & (D - 1))], rate = A.rate[h];
+    const float norm = A.norm[h * D + (tid & (D - 1))];
+    float* S_at = A.state + ((size_t)A.slot[r] * A.heads + h) * (D * D);
+    float4 S[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S[j] = *reinterpret_cast<const float4*>(S_at + (k0 + j) * D + c4);
+    if (tid < 3 * D) {
+        (tid < D ? sq : tid < 2 * D ? sk : sv)[tid & (D - 1)] = mine;
+        if (tid < 2 * D) {
+            const float ss = wave_sum(mine * mine);          // (whole waves: a head's 128 channels are two)
+            if (lane == 0) squares[wave] = ss;
+        }
+    } else if (tid >= 512 && tid < 512 + ranks) {
+        low[tid - 512] = bf16_to_f32(f32_to_bf16(mine));     // (what the matrix that leads back up reads is bfloat16)
+    } else if (tid == 3 * D) {
+        beta = ds_sigmoid(mine);
+    }
+    __syncthreads();
+    {
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < CDH_RANK / 32; ++j) {
+            const int at = (j * 4 + piece) * 8;
+            if (at >= rank) continue;
+            const float4 a = *reinterpret_cast<const float4*>(&low[(gate ? A.rank_a : 0) + at]);
+            const float4 b = *reinterpret_cast<const float4*>(&low[(gate ? A.rank_a : 0) + at + 4]);
+            const float l[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+            const unsigned u[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                sum = fmaf(__uint_as_float(u[i] << 16), l[2 * i], sum);
+                sum = fmaf(__uint_as_float(u[i] & 0xffff0000u), l[2 * i + 1], sum);
+            }
+        }
+        sum += cdh_quad<1>(sum);
+        sum += cdh_quad<2>(sum);
+        if (piece == 0) {
+            if (gate) gates[dot - D] = sum;
+            else sg[dot] = expf(-rate * ds_softplus(sum + bias));
+        }
+    }
+    __syncthreads();
+    const float fq = A.q_scale * (1.0f / sqrtf(squares[0] + squares[1] + A.unit_eps));
+    const float fk = 1.0f / sqrtf(squares[2] + squares[3] + A.unit_eps);
+    const float4 kk = *reinterpret_cast<const float4*>(&sk[k0]), qq = *reinterpret_cast<const float4*>(&sq[k0]);
+    const float4 gg = *reinterpret_cast<const float4*>(&sg[k0]);
+    const float kj[4] = {kk.x * fk, kk.y * fk, kk.z * fk, kk.w * fk}, qj[4] = {qq.x * fq, qq.y * fq, qq.z * fq, qq.w * fq};
+    const float g[4] = {gg.x, gg.y, gg.z, gg.w};
+    // sums over the state's rows as the kernel above has them
+    auto leave = [&](const float (&v)[4]) __attribute__((always_inline)) {
+        const float4 s = make_float4(cds_halves(v[0]), cds_halves(v[1]), cds_halves(v[2]), cds_halves(v[3]));
+        if (lane < 32) *reinterpret_cast<float4*>(&red[wave][c4]) = s;
+    };
+    auto gather = [&]() __attribute__((always_inline)) {
+        float v[WAVES];
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) v[i] = red[i][tid & (D - 1)];
+#pragma unroll
+        for (int half = WAVES / 2; half > 0; half /= 2)
+#pragma unroll
+            for (int i = 0; i < half; ++i) v[i] += v[i + half];
+        return v[0];
+    };
+    float seen[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        S[j] = make_float4(S[j].x * g[j], S[j].y * g[j], S[j].z * g[j], S[j].w * g[j]);
+        seen[0] = fmaf(S[j].x, kj[j], seen[0]);
+        seen[1] = fmaf(S[j].y, kj[j], seen[1]);
+        seen[2] = fmaf(S[j].z, kj[j], seen[2]);
+        seen[3] = fmaf(S[j].w, kj[j], seen[3]);
+    }
+    leave(seen);
+    __syncthreads();
+    if (tid < D) su[tid] = beta * (sv[tid] - gather());
+    __syncthreads();
+    const float4 u = *reinterpret_cast<const float4*>(&su[c4]);
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        S[j] = make_float4(fmaf(kj[j], u.x, S[j].x), fmaf(kj[j], u.y, S[j].y), fmaf(kj[j], u.z, S[j].z), fmaf(kj[j], u.w, S[j].w));
+        o[0] = fmaf(S[j].x, qj[j], o[0]);
+        o[1] = fmaf(S[j].y, qj[j], o[1]);
+        o[2] = fmaf(S[j].z, qj[j], o[2]);
+        o[3] = fmaf(S[j].w, qj[j], o[3]);
+        *reinterpret_cast<float4*>(S_at + (k0 + j) * D + c4) = S[j];
+    }
+    leave(o);
+    __syncthreads();
+    float y = 0.f;
+    if (tid < D) {                                           // (whole waves)
+        y = gather();
+        const float ss = wave_sum(y * y);
+        if (lane == 0) part[wave] = ss;
+    }
+    __syncthreads();
+    if (tid >= D) return;
+    const float rs = 1.0f / sqrtf((part[0] + part[1]) / (float)D + A.eps);
+    store_f32<TOut>(out, ((size_t)r * A.heads + h) * D + tid, y * rs * norm * ds_sigmoid(gates[tid]));
+}
+
+extern "C" int imparo_channel_delta_heads_takes(int heads, int kv_heads, int dim, int vdim, int taps, int rank_a, int rank_g) {
+    return dim == CDS_DIM && vdim == CDS_DIM && taps >= 1 && taps <= CDS_MAX_TAPS && kv_heads > 0 && heads % kv_heads == 0 &&
+           heads <= 65535 && rank_a >= 8 && rank_a <= CDH_RANK && rank_a % 8 == 0 && rank_g >= 8 && rank_g <= CDH_RANK && rank_g % 8 == 0;
+}
+
+extern "C" int imparo_channel_delta_heads(const float* rows, int ld, int beta_off, int low_off, const void* high, int high_ld,
+                                          int rank_a, int rank_g, const float* step_bias, const float* rate, float* state,
+                                          int n_slots, const int32_t* slot, const float* norm, void* out, int out_dtype, int n_rows,
+                                          int heads, int kv_heads, float unit_eps, float q_scale, float eps, imparo_stream stream) {
+    if (!rows || !high || !step_bias || !rate || !state || !slot || !norm || !out || n_rows < 0 || n_slots < 1) return IMPARO_BAD_ARGUMENT;
+    if (!imparo_channel_delta_heads_takes(heads, kv_heads, CDS_DIM, CDS_DIM, 1, rank_a, rank_g)) return IMPARO_BAD_ARGUMENT;
+    const int channels = (2 * kv_heads + heads) * CDS_DIM;
+    if (beta_off < channels || ld < beta_off + heads || low_off < channels || ld < low_off + rank_a + rank_g ||
+        high_ld < rank_a + rank_g || high_ld % 8 || ((uintptr_t)high & 15) || ((uintptr_t)state & 15))
+        return IMPARO_BAD_ARGUMENT;
+    if (out_dtype != IMPARO_F32 && out_dtype != IMPARO_BF16) return IMPARO_BAD_ARGUMENT;
+    if (n_rows == 0) return IMPARO_OK;
+    const ChannelHeadArgs a{rows, ld, beta_off, low_off, (const bf16_t*)high, high_ld, rank_a, rank_g, step_bias, rate, state, slot,
+                            norm, heads, kv_heads, unit_eps, q_scale, eps};
+    const dim3 grid((unsigned)n_rows, (unsigned)heads);
+    hipStream_t s = (hipStream_t)stream;
+    if (out_dtype == IMPARO_BF16) k_channel_delta_head<bf16_t><<<grid, 1024, 0, s>>>(a, (bf16_t*)out);
+    else k_channel_delta_head<float><<<grid, 1024, 0, s>>>(a, (float*)out);
+    return launch_status();
+}
+
 // Whether the launch below takes a mixer of these sizes.
 extern "C" int imparo_channel_delta_step_takes(int heads, int kv_heads, int dim, int vdim, int taps) {
     return dim == CDS_DIM && vdim == CDS_DIM && taps >= 1 && taps <= CDS_MAX_TAPS && kv_heads > 0 &&

@@ -9,6 +9,8 @@
 //     blocks): nothing meets across blocks, so there are no counters and no fences;
 //     Where that norm has no statistic (dynamic tanh), the block leaves the rows behind it: every element is its own, and
 //     nothing is left for the reader to do;
+//   * the first columns may be channels of a causal conv with SiLU behind it: the lane that ends up with a channel's sum has
+//     its history and taps by then, and shifts the history;
 //   * the activations may be such rows (the stream times a norm's weight, not yet scaled) with the
 //     partial sums of squares beside them: the block multiplies each row's result by the row's scale
 //     rsqrt(sum / K + eps) at the end, in float32 -- no norm launch.
@@ -61,6 +63,18 @@ union RowFrag {
 #define ROWS_WAVES 8         // of a block at most
 #define ROWS_TURNED 8192     // from this K on blocks start their walks at different places
 
+#define ROWS_CONV 4          // the first columns through a causal conv a channel and SiLU
+
+// ROWS_CONV: columns 0 .. channels - 1 are channels of a causal conv (at most ROWS_TAPS taps, the last one the current row's) whose
+// last inputs a request keeps: hist [slots, taps - 1, channels], row r in slot[r], shifted in place by the lane that owns the channel.
+#define ROWS_TAPS 4
+struct RowsConv {
+    const float* w;          // [channels, taps]
+    float* hist;
+    const int32_t* slot;
+    int taps, channels;
+};
+
 // K_KIND
 #define ROWS_WHOLE 0         // K is a multiple of 128, and every wave has as many chunks of it as its rounds ask for
 #define ROWS_UNEVEN 1        // K is a multiple of 128
@@ -95,7 +109,8 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
     const bf16_t* __restrict__ X, const float* __restrict__ ssq_in, int n_parts, float eps,
     const bf16_t* __restrict__ W, const float* __restrict__ bias, TOut* __restrict__ Y, float* __restrict__ x_io,
     float* __restrict__ ssq_out, bf16_t* __restrict__ weighted_out, const float* __restrict__ weighted_by,
-    const float* __restrict__ tanh_bias, float tanh_alpha, int M, int N, int K_all, int k_per, int rounds, int turned, Epilogue unit) {
+    const float* __restrict__ tanh_bias, float tanh_alpha, int M, int N, int K_all, int k_per, int rounds, int turned, Epilogue unit,
+    RowsConv conv) {
     static_assert(RB == 16 || RT == 1, "half tiles one by one");
     constexpr bool RAGGED = K_KIND == ROWS_RAGGED || K_KIND == ROWS_HUGE;
     extern __shared__ float4 red[];                     // [CHAINS][waves][RT][64]
@@ -177,6 +192,23 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
             if (EPI == ROWS_TANH && tanh_bias) plus[i] = tanh_bias[n];
         }
     }
+    // (and what a conv's channels had before, for the tile that this wave finishes first)
+    float taps_of[EPI == ROWS_CONV ? 4 : 1][ROWS_TAPS], old[EPI == ROWS_CONV ? ROWS_TAPS - 1 : 1][4];
+    auto ask_conv = [&](int t) __attribute__((always_inline)) {
+        const int n = n0 + t * 16 + g * 4, history = conv.taps - 1;
+        if (n >= conv.channels || r16 >= M) return;
+        const float* hist = conv.hist + (size_t)conv.slot[r16] * history * conv.channels + n;
+#pragma unroll
+        for (int i = 0; i < ROWS_TAPS - 1; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) old[EPI == ROWS_CONV ? i : 0][j] = i < history ? hist[(size_t)i * conv.channels + j] : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < ROWS_TAPS; ++i)
+                taps_of[EPI == ROWS_CONV ? j : 0][i] = i < conv.taps ? conv.w[(size_t)(n + j) * conv.taps + i] : 0.f;
+    };
+    if (EPI == ROWS_CONV && wave < RT) ask_conv(wave);
     f32x4 acc[CHAINS][RT];
 #pragma unroll
     for (int c = 0; c < CHAINS; ++c)
@@ -274,6 +306,29 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                 if (n + 1 < N) store_f32<TOut>(dst, 0, a);
                 if (n + 3 < N) store_f32<TOut>(dst, 1, b);
             }
+        } else if (EPI == ROWS_CONV) {
+            if (!live) continue;
+            if (n < conv.channels) {                     // (channels are a multiple of 4)
+                if (t != wave) ask_conv(t);
+                const int history = conv.taps - 1;
+                float* hist = conv.hist + (size_t)conv.slot[r16] * history * conv.channels + n;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float now = v[j];
+                    float sum = 0.f, last = taps_of[EPI == ROWS_CONV ? j : 0][0];
+#pragma unroll
+                    for (int i = 0; i < ROWS_TAPS - 1; ++i) {          // (what lies past the history is zero)
+                        const int at = EPI == ROWS_CONV ? i : 0;
+                        sum = fmaf(i < history ? taps_of[EPI == ROWS_CONV ? j : 0][i] : 0.f, old[at][j], sum);
+                        last = i + 1 == history ? taps_of[EPI == ROWS_CONV ? j : 0][i + 1] : last;
+                        if (i < history)
+                            hist[(size_t)i * conv.channels + j] = i + 1 < history ? old[EPI == ROWS_CONV && i + 1 < ROWS_TAPS - 1 ? i + 1 : 0][j] : now;
+                    }
+                    const float z = fmaf(last, now, sum);
+                    v[j] = z / (1.0f + expf(-z));
+                }
+            }
+            rows_store<TOut>(Y + (size_t)r16 * N + n, v, n, N, N % 4 == 0 && ((uintptr_t)Y & (4 * sizeof(TOut) - 1)) == 0);
         } else if (EPI == ROWS_STORE) {
             if (live) rows_store<TOut>(Y + (size_t)r16 * N + n, v, n, N, N % 4 == 0 && ((uintptr_t)Y & (4 * sizeof(TOut) - 1)) == 0);
         } else {
@@ -373,6 +428,7 @@ struct RowsCall {
     float tanh_alpha;
     int m, n, k, slices;
     Epilogue unit;
+    RowsConv conv;
 };
 
 template <typename TOut, int RB, int EPI, bool SCALED>
@@ -380,6 +436,7 @@ static void rows_launch_as(const RowsCall& c, hipStream_t s) {
     const int k_per = ((c.k + c.slices - 1) / c.slices + 127) / 128 * 128;
     const bool huge = c.k >= (1 << 25), ragged = c.k % 128 != 0 || huge;      // (byte offsets inside 64 rows stay in 32 bits)
     RowsShape sh = rows_shape(c.m, c.n, c.k, std::min(k_per, c.k), c.slices, RB);
+    if (EPI == ROWS_CONV && sh.rt > 2) sh.rt = 2;
     if (huge) sh.rt = 1, sh.ch = 1, sh.chains = 1;
     const dim3 grid((unsigned)((c.n + (long long)RB * sh.rt - 1) / (RB * sh.rt)), (unsigned)((c.k + k_per - 1) / k_per));
     const int rounds = ((std::min(k_per, c.k) + 127) / 128 + sh.waves * sh.ch - 1) / (sh.waves * sh.ch);
@@ -389,7 +446,7 @@ static void rows_launch_as(const RowsCall& c, hipStream_t s) {
 #define ROWS_GO(RT, CH, CHAINS, KIND)                                                                                \
     k_rows_gemm<TOut, RB, RT, CH, CHAINS, EPI, KIND, SCALED><<<grid, sh.waves * 64, lds, s>>>(                         \
         c.x, c.ssq_in, c.n_parts, c.eps, c.w, c.bias, (TOut*)c.y, c.x_io, c.ssq_out, c.weighted_out, c.weighted_by, \
-        c.tanh_bias, c.tanh_alpha, c.m, c.n, c.k, k_per, rounds, turned, c.unit)
+        c.tanh_bias, c.tanh_alpha, c.m, c.n, c.k, k_per, rounds, turned, c.unit, c.conv)
 #define ROWS_CHAINS(RT, CH, KIND)                                                                                    \
     do {                                                                                                             \
         if (sh.chains == 2) ROWS_GO(RT, CH, 2, KIND);                                                                \
@@ -421,8 +478,9 @@ static void rows_launch_as(const RowsCall& c, hipStream_t s) {
         ROWS_CH(1);
     } else if (sh.rt == 1) {
         ROWS_CH(1);
-    } else if (sh.rt == 2) {
+    } else if (EPI == ROWS_CONV || sh.rt == 2) {
         ROWS_CH(2);
+    } else if constexpr (EPI == ROWS_CONV) {
     } else if (sh.rt == 3) {
         if (ragged) ROWS_CHAINS(3, 1, ROWS_RAGGED);
         else if (sh.ch == 1) ROWS_CHAINS(3, 1, ROWS_WHOLE);
@@ -451,7 +509,7 @@ static void rows_launch_tanh(const RowsCall& c, const RowsShape& sh, hipStream_t
 #define ROWS_GO(KIND)                                                                                                  \
     k_rows_gemm<float, RB, 1, CH, CH, ROWS_TANH, KIND, false><<<grid, sh.waves * 64, lds, s>>>(                          \
         c.x, nullptr, 0, 0.f, c.w, c.bias, nullptr, c.x_io, nullptr, c.weighted_out, c.weighted_by, c.tanh_bias, c.tanh_alpha, \
-        c.m, c.n, c.k, c.k, rounds, turned, c.unit)
+        c.m, c.n, c.k, c.k, rounds, turned, c.unit, c.conv)
     if (c.k % 128) ROWS_GO(ROWS_RAGGED);
     else if (CH == 1 || c.k % (128 * sh.waves * CH) == 0) ROWS_GO(ROWS_WHOLE);
     else ROWS_GO(ROWS_UNEVEN);
@@ -467,7 +525,7 @@ static void rows_launch(const RowsCall& c, hipStream_t s) {
 int imparo_few_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* y, int out_dtype, int m, int n, int k,
                     const Epilogue& epilogue, int slices, const float* ssq_in, int n_parts, float eps, hipStream_t s) {
     const RowsCall c{x, ssq_in, n_parts, eps, w, bias, y, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, m, n, k, slices,
-                     epilogue};
+                     epilogue, {}};
     if (m <= 0 || m > ROWS_MAX || n <= 0 || k < 8 || k % 8 || slices < 1) return IMPARO_BAD_ARGUMENT;
     if (epilogue == EPI_SWIGLU && out_dtype == IMPARO_BF16)
         rows_launch<bf16_t, 16, ROWS_SWIGLU>(c, s);
@@ -505,11 +563,26 @@ extern "C" int imparo_rows_gemm(const void* x, const float* ssq_in, int n_parts,
     bf16_t* wo = (bf16_t*)weighted_out;
     if (epilogue == ROWS_RESID) {
         rows_launch<float, 8, ROWS_RESID>(RowsCall{xb, ssq_in, n_parts, eps, wb, bias, nullptr, x_io, ssq_out, wo, weighted_by, nullptr,
-                                                   0.f, m, n, k, 1, Epilogue(EPI_NONE)}, s);
+                                                   0.f, m, n, k, 1, Epilogue(EPI_NONE), {}}, s);
         return launch_status();
     }
     return imparo_few_rows(xb, wb, bias, y, out_dtype, m, n, k, Epilogue(epilogue == ROWS_SWIGLU ? EPI_SWIGLU : EPI_NONE), 1, ssq_in,
                            n_parts, eps, s);
+}
+
+extern "C" int imparo_rows_gemm_conv(const void* x, const void* w, float* y, const float* conv_w, float* hist, const int32_t* slot,
+                                     int taps, int channels, int m, int n, int k, imparo_stream stream) {
+    if (!x || !w || !y || !conv_w || !slot || m < 0 || m > ROWS_MAX || n <= 0 || k <= 0 || k % 8 != 0 || k >= (1 << 25))
+        return IMPARO_BAD_ARGUMENT;
+    if (taps < 1 || taps > ROWS_TAPS || (taps > 1 && !hist) || channels < 0 || channels > n || channels % 4)
+        return IMPARO_BAD_ARGUMENT;
+    if (((uintptr_t)w & 15) || ((uintptr_t)x & 15)) return IMPARO_BAD_ARGUMENT;
+    if (m == 0) return IMPARO_OK;
+    rows_launch_as<float, 16, ROWS_CONV, false>(
+        RowsCall{(const bf16_t*)x, nullptr, 0, 0.f, (const bf16_t*)w, nullptr, y, nullptr, nullptr, nullptr, nullptr, nullptr, 0.f, m, n,
+                 k, 1, Epilogue(EPI_NONE), RowsConv{conv_w, hist, slot, taps, channels}},
+        (hipStream_t)stream);
+    return launch_status();
 }
 
 extern "C" int imparo_rows_gemm_tanh(const void* x, const void* w, const float* bias, float* x_io, void* out, float alpha,
@@ -519,7 +592,7 @@ extern "C" int imparo_rows_gemm_tanh(const void* x, const void* w, const float* 
     if (((uintptr_t)w & 15) || ((uintptr_t)x & 15) || k >= (1 << 25)) return IMPARO_BAD_ARGUMENT;
     if (m == 0) return IMPARO_OK;
     const RowsCall c{(const bf16_t*)x, nullptr, 0, 0.f, (const bf16_t*)w, bias, nullptr, x_io, nullptr, (bf16_t*)out, norm_w, norm_b,
-                     alpha, m, n, k, 1, Epilogue(EPI_NONE)};
+                     alpha, m, n, k, 1, Epilogue(EPI_NONE), {}};
     const RowsShape sh = rows_shape(m, n, k, k, 1, 8);
     const int a_wave = ((k + 127) / 128 + sh.waves - 1) / sh.waves;
     hipStream_t s = (hipStream_t)stream;

@@ -115,6 +115,8 @@ _SIGNATURES = {
     "imparo_delta_chunk_tokens": [],
     "imparo_delta_chunk_max_dim": [],
     "imparo_head_prepare": [P, I, I, I, I, I, I, F, P, I, I, P, I, F, F, P],
+    "imparo_channel_delta_heads_takes": [I, I, I, I, I, I, I],
+    "imparo_channel_delta_heads": [P, I, I, I, P, I, I, I, P, P, P, I, P, P, P, I, I, I, I, F, F, F, P],
     "imparo_channel_delta_step_takes": [I, I, I, I, I],
     "imparo_channel_delta_step": [P, I, I, P, I, I, P, P, I, P, P, P, I, P, P, P, I, I, I, I, I, I, F, F, F, P],
     "imparo_gated_group_norm": [P, P, I, I, P, P, I, I, I, I, F, I, I, P],
@@ -140,6 +142,7 @@ _SIGNATURES = {
     "imparo_post_norm_add": [P, P, I, I, P, P, F, P, F, P, I, I, I, P],
     "imparo_rows_parts": [I],
     # x, ssq_in, n_parts, eps, w, bias, y, out_dtype, x_io, ssq_out, weighted_out, weighted_by, m, n, k, epilogue, stream
+    "imparo_rows_gemm_conv": [P, P, P, P, P, P, I, I, I, I, I, P],
     "imparo_rows_gemm_tanh": [P, P, P, P, P, F, P, P, I, I, I, P],
     "imparo_rows_gemm": [P, P, I, F, P, P, P, I, P, P, P, P, I, I, I, I, P],
     "imparo_in_proj_conv_decode_normed": [P, P, I, F, P, P, P, P, P, P, P, I, I, I, I, I, I, P],

@@ -698,6 +698,27 @@ def rows_gemm(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = No
     return into if into is not None else out
 
 
+def rows_gemm_conv(x: torch.Tensor, w: torch.Tensor, conv_weight: torch.Tensor, conv_state: Optional[torch.Tensor],
+                   slot: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """A product of at most 16 rows of one token each, x [m, k] and w [n, k] bfloat16, out [m, n] float32, whose first columns go
+    through a causal conv a channel (conv_weight [channels, taps], conv_state [slots, taps - 1, channels] shifted in
+    place, row r is the token of the request in slot[r]) and SiLU."""
+    m, k = x.shape
+    n, kw = w.shape
+    channels, taps = conv_weight.shape
+    if kw != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not 0 < m <= ROWS_MAX or k % 8:
+        raise KernelArgumentError("rows_gemm_conv: 1 to 16 bfloat16 rows, a bfloat16 weight over the same inner size, "
+                                  "a multiple of 8")
+    if channels > n or channels % 4 or not 1 <= taps <= 4:
+        raise KernelArgumentError("rows_gemm_conv: the conv's channels are the first columns, a multiple of 4, with up to four taps")
+    slots = 0 if conv_state is None else conv_state.shape[0]
+    _check(library().imparo_rows_gemm_conv(
+        _dev(x, "x"), _dev(w, "weight"), _dev(out, "out", torch.float32, (m, n)), _dev(conv_weight, "conv weight", torch.float32),
+        _dev(conv_state, "conv state", torch.float32, (slots, taps - 1, channels)), _dev(slot, "slot", torch.int32, (m,)), taps,
+        channels, m, n, k, _stream()), "rows_gemm_conv")
+    return out
+
+
 def rows_gemm_tanh(x: torch.Tensor, w: torch.Tensor, into: torch.Tensor, bias: Optional[torch.Tensor] = None,
                    out: Optional[torch.Tensor] = None, alpha: float = 0.0, norm_weight: Optional[torch.Tensor] = None,
                    norm_bias: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -1512,6 +1533,37 @@ def channel_delta_scan(q: torch.Tensor, q_off: int, q_div: int, k: torch.Tensor,
 def channel_delta_step_takes(heads: int, kv_heads: int, dim: int, vdim: int, taps: int) -> bool:
     """Whether channel_delta_step takes a mixer of these sizes."""
     return bool(library().imparo_channel_delta_step_takes(int(heads), int(kv_heads), int(dim), int(vdim), int(taps)))
+
+
+def channel_delta_heads_takes(heads: int, kv_heads: int, dim: int, vdim: int, taps: int, rank_a: int, rank_g: int) -> bool:
+    """Whether rows_gemm_conv and channel_delta_heads take a mixer of these sizes."""
+    return bool(library().imparo_channel_delta_heads_takes(int(heads), int(kv_heads), int(dim), int(vdim), int(taps), int(rank_a),
+                                                           int(rank_g)))
+
+
+def channel_delta_heads(rows: torch.Tensor, beta_off: int, low_off: int, high: torch.Tensor, rank_a: int, rank_g: int,
+                        step_bias: torch.Tensor, rate: torch.Tensor, state: torch.Tensor, slot: torch.Tensor, norm: torch.Tensor,
+                        out: torch.Tensor, heads: int, kv_heads: int, unit_eps: float, q_scale: float, eps: float) -> torch.Tensor:
+    """channel_delta_step for rows that rows_gemm_conv left: q | k | v behind conv and SiLU, b from beta_off on, and from low_off on
+    the inner numbers of the decays' (rank_a) and the gate's (rank_g) bottleneck, which `high` [2 heads 128, ..] bfloat16
+    leads back up: its first heads * 128 rows from the first rank_a numbers, the others from the rank_g behind them."""
+    n, ld = rows.shape
+    n_slots, dim = state.shape[0], 128
+    if not channel_delta_heads_takes(heads, kv_heads, dim, dim, 1, rank_a, rank_g):
+        raise KernelArgumentError("channel_delta_heads: heads of 128 by 128 and ranks that are multiples of 8 up to 128")
+    channels = (2 * kv_heads + heads) * dim
+    if beta_off < channels or ld < beta_off + heads or low_off < channels or ld < low_off + rank_a + rank_g:
+        raise KernelArgumentError("channel_delta_heads: the projection's rows do not hold what the mixer reads")
+    if high.shape[0] != 2 * heads * dim or high.shape[1] < rank_a + rank_g or high.shape[1] % 8:
+        raise KernelArgumentError("channel_delta_heads: the matrix that leads back up does not fit the heads and ranks")
+    _check(library().imparo_channel_delta_heads(
+        _dev(rows, "projected rows", torch.float32), ld, int(beta_off), int(low_off), _dev(high, "way up", torch.bfloat16),
+        high.shape[1], int(rank_a), int(rank_g), _dev(step_bias, "step bias", torch.float32, (heads * dim,)),
+        _dev(rate, "rate", torch.float32, (heads,)), _dev(state, "state", torch.float32, (n_slots, heads, dim, dim)), n_slots,
+        _dev(slot, "slot", torch.int32, (n,)), _dev(norm, "norm weight", torch.float32, (heads * dim,)),
+        _dev(out, "normed heads", None, (n, heads * dim)), _code(out, "normed heads"), n, heads, kv_heads, float(unit_eps),
+        float(q_scale), float(eps), _stream()), "channel_delta_heads")
+    return out
 
 
 def channel_delta_step(rows: torch.Tensor, beta_off: int, steps: torch.Tensor, gate_off: int, conv_weight: torch.Tensor,

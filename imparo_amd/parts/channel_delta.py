@@ -95,15 +95,23 @@ class ChannelDelta:
             ws = [tensors[n[x]] for x in names]
             return ws if len({w.dtype for w in ws}) == 1 else [w.to(torch.float32) for w in ws]
 
-        # one projection for q | k | v | b: the same dot products, one launch
-        self.proj = Linear(place_projection(torch.cat(side("q", "k", "v", "b"), dim=0), engine_dtype, device))
-        # The two bottlenecks side by side: one projection down, and one up whose matrix has a block for each (the
-        # other block's columns are zero and add nothing). Filled up with rows of zero weight to a multiple of 8
-        # inner numbers, which the bfloat16 kernels walk.
+        # One projection for q | k | v | b, and one for the two bottlenecks side by side: the same dot products, one launch
+        # each, or one for both (their rows lie in one matrix). The way up from the bottlenecks is one matrix with a block
+        # for each (the other block's columns are zero and add nothing). Filled up with rows of zero weight to a multiple
+        # of 8 inner numbers, which the bfloat16 kernels walk.
+        wide = torch.cat(side("q", "k", "v", "b"), dim=0)
         a1, g1, a2, g2 = side("a1", "g1", "a2", "g2")
         ra, rg = a1.shape[0], g1.shape[0]
         fill = (-(ra + rg)) % 8
-        self.low = Linear(place_projection(torch.cat([a1, g1, a1.new_zeros(fill, self.width)], dim=0), engine_dtype, device))
+        down = torch.cat([a1, g1, a1.new_zeros(fill, self.width)], dim=0)
+        self.rows_weight = None
+        if wide.dtype == down.dtype:
+            self.rows_weight = place_projection(torch.cat([wide, down], dim=0), engine_dtype, device)
+            self.proj, self.low = Linear(self.rows_weight[:wide.shape[0]]), Linear(self.rows_weight[wide.shape[0]:])
+        else:
+            self.proj = Linear(place_projection(wide, engine_dtype, device))
+            self.low = Linear(place_projection(down, engine_dtype, device))
+        self.ranks = ra, rg
         high = a2.new_zeros(H * dk + H * dv, ra + rg + fill)
         high[:H * dk, :ra] = a2
         high[H * dk:, ra:ra + rg] = g2
@@ -132,6 +140,17 @@ class ChannelDelta:
             raise ValueError("a recurrence's state cannot be read from another layer")
         T, H, Hk, dk, dv, C = h.shape[0], self.heads, self.kv_heads, self.dim, self.vdim, self.conv_channels
         state = ctx.fixed_arrays(site)
+        if (ctx.max_seg_len == 1 and T <= ops.ROWS_MAX and self.rows_weight is not None and h.dtype == torch.bfloat16
+                and self.rows_weight.dtype == torch.bfloat16 and self.high.in_dtype == torch.bfloat16
+                and ops.channel_delta_heads_takes(H, Hk, dk, dv, self.taps, *self.ranks)):
+            # a decode step of a few rows: everything that reads h in one launch, with the conv, and the rest in another
+            n = self.rows_weight.shape[0]
+            rows = ctx.workspace.get("delta_rows", (T, n), torch.float32, alias="mixer_in")          # q k v | b | bottlenecks
+            ops.rows_gemm_conv(h, self.rows_weight, self.conv_weight, state.get("conv"), ctx.slot, rows)
+            gated = ctx.workspace.get("delta_gated", (T, H * dv), self.out.in_dtype, alias="mixer_mid")
+            ops.channel_delta_heads(rows, C, C + H, self.high.weight, *self.ranks, self.dt_bias, self.rate, state["state"], ctx.slot,
+                                    self.norm, gated, H, Hk, UNIT_EPS, float(dk) ** -0.5, self.eps)
+            return self.out(ctx, gated, torch.float32, "mixer_out", sliced_ok=True, into=ctx.stream)
         rows = self.proj(ctx, h, torch.float32, "delta_rows", alias="mixer_in")              # q k v | b
         low = self.low(ctx, h, self.high.in_dtype, "delta_low")
         steps = self.high(ctx, low, torch.float32, "delta_steps")                            # decays' steps | gate
