@@ -787,28 +787,10 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
 // work queued while the waves meet. Needs K a multiple of 128 (two K-steps).
 #define DM_BK 64
 
-// What the output holds where four results of a row will go (the epilogue that adds; float32 out only)
-template <typename T> __device__ __forceinline__ float4 held_vector(const T*) { return make_float4(0.f, 0.f, 0.f, 0.f); }
-template <> __device__ __forceinline__ float4 held_vector<float>(const float* dst) {
-    return *reinterpret_cast<const float4*>(dst);
-}
-template <typename T> __device__ __forceinline__ float held_f32(const T*, int) { return 0.f; }
-template <> __device__ __forceinline__ float held_f32<float>(const float* dst, int c) { return dst[c]; }
-
-// Two (`pair`) or four outputs of one row in one store; the address is aligned to the store
-template <typename T> __device__ __forceinline__ void store_vector(T* dst, const float (&o)[4], bool pair);
-template <> __device__ __forceinline__ void store_vector<float>(float* dst, const float (&o)[4], bool pair) {
-    if (pair)
-        *reinterpret_cast<float2*>(dst) = make_float2(o[0], o[1]);
-    else
-        *reinterpret_cast<float4*>(dst) = make_float4(o[0], o[1], o[2], o[3]);
-}
-template <> __device__ __forceinline__ void store_vector<bf16_t>(bf16_t* dst, const float (&o)[4], bool pair) {
-    const unsigned lo = f32x2_to_bf16x2(o[0], o[1]);
-    if (pair)
-        *reinterpret_cast<unsigned*>(dst) = lo;
-    else
-        *reinterpret_cast<uint2*>(dst) = make_uint2(lo, f32x2_to_bf16x2(o[2], o[3]));
+// What the lane N (1 or 2) apart among four neighbours has
+template <int N>
+__device__ __forceinline__ float lane_xor(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), N == 1 ? 0xB1 : 0x4E, 0xf, 0xf, false));
 }
 
 // TMI, TN: MFMA tiles of 32x32 down a wave's part of the activation rows and across its part of
@@ -911,8 +893,11 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
     Frag8 fa0[TMI], fb0[TN], fa1[TMI], fb1[TN];
     // K-step kt from `cur`: on entry set 0 holds its first sub-step and the loads of step kt+1
     // into `next` are in flight (and with four stages those of kt+2 and kt+3); on exit set 0 holds
-    // the first sub-step of kt+1 and the loads of kt+STAGES into `cur` are in flight
-    auto k_step = [&](bf16_t* cur, bf16_t* next, int kt) __attribute__((always_inline)) {
+    // the first sub-step of kt+1 and the loads of kt+STAGES into `cur` are in flight. `after`: how many steps
+    // follow, as far as it matters (the last ones ask for nothing: with the last step loaded again and again a block
+    // of 16 steps on four stages moved a quarter more than it needs)
+    auto k_step = [&](bf16_t* cur, bf16_t* next, int kt, auto after) __attribute__((always_inline)) {
+        constexpr int AFTER = decltype(after)::value;
         // (the scheduling barriers keep each sub-step's reads and products where they are written:
         // left alone, the compiler sinks the loads of the next step to just before the wait for them)
         read(cur, 1, fa1, fb1);
@@ -924,28 +909,36 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
         read(cur, 3, fa1, fb1);
         multiply(fa0, fb0);
         __builtin_amdgcn_sched_barrier(0);
+        if constexpr (AFTER == 0) {
+            multiply(fa1, fb1);
+            return;
+        }
         // this wave's part of `next` has landed and `cur` is read; after the barrier, so for every wave
-        if (STAGES == 4) {             // the loads of the two steps after `next` stay in flight: a bare barrier
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * (LX + LW)) : "memory");
+        if (STAGES == 4) {             // the loads of the steps after `next` stay in flight: a bare barrier
+            constexpr int BEYOND = AFTER - 1 < 2 ? (AFTER > 0 ? AFTER - 1 : 0) : 2;
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(BEYOND * (LX + LW)) : "memory");
             __builtin_amdgcn_s_barrier();
         } else {
             __syncthreads();
         }
         read(next, 0, fa0, fb0);
-        load_step(cur, min(kt + STAGES, nk - 1));   // past the end: the last step again, into a stage nobody reads any more
+        if constexpr (AFTER >= STAGES) load_step(cur, kt + STAGES);
         multiply(fa1, fb1);
+        if constexpr (AFTER >= STAGES) {
 #pragma unroll
-        for (int q = 0; q < TMI * TN; ++q) {        // one product, (one fragment read,) one load or two
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            if (q < TMI + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-            if (q < LX + LW - TMI * TN)
-                __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-            else if (q < LX + LW)
-                __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            for (int q = 0; q < TMI * TN; ++q) {        // one product, (one fragment read,) one load or two
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (q < TMI + TN) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                if (q < LX + LW - TMI * TN)
+                    __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+                else if (q < LX + LW)
+                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    if (STAGES == 4) {
+    constexpr std::integral_constant<int, STAGES> many{};
+    if constexpr (STAGES == 4) {
         load_step(stage0, 0);
         load_step(stage1, 1);
         load_step(stage2, 2);
@@ -953,99 +946,128 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * (LX + LW)) : "memory");
         __builtin_amdgcn_s_barrier();
         read(stage0, 0, fa0, fb0);
-        for (int kt = 0; kt < nk; kt += 4) {           // K-steps in fours: one loop, one way round it
-            k_step(stage0, stage1, kt);
-            k_step(stage1, stage2, kt + 1);
-            k_step(stage2, stage3, kt + 2);
-            k_step(stage3, stage0, kt + 3);
+        int kt = 0;
+        for (; kt + 4 < nk; kt += 4) {                 // K-steps in fours: one loop, one way round it
+            k_step(stage0, stage1, kt, many);
+            k_step(stage1, stage2, kt + 1, many);
+            k_step(stage2, stage3, kt + 2, many);
+            k_step(stage3, stage0, kt + 3, many);
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the loads past the end: nothing may land in what the tile leaves through
+        k_step(stage0, stage1, kt, std::integral_constant<int, 3>{});
+        k_step(stage1, stage2, kt + 1, std::integral_constant<int, 2>{});
+        k_step(stage2, stage3, kt + 2, std::integral_constant<int, 1>{});
+        k_step(stage3, stage0, kt + 3, std::integral_constant<int, 0>{});
     } else {
         load_step(stage0, 0);
         __syncthreads();
         load_step(stage1, 1);
         read(stage0, 0, fa0, fb0);
-        for (int kt = 0; kt < nk; kt += 2) {           // an even number of K-steps: one loop, one way round it
-            k_step(stage0, stage1, kt);
-            k_step(stage1, stage0, kt + 1);
+        int kt = 0;
+        for (; kt + 2 < nk; kt += 2) {                 // an even number of K-steps: one loop, one way round it
+            k_step(stage0, stage1, kt, many);
+            k_step(stage1, stage0, kt + 1, many);
         }
+        k_step(stage0, stage1, kt, std::integral_constant<int, 1>{});
+        k_step(stage1, stage0, kt + 1, std::integral_constant<int, 0>{});
     }
-    // The tile leaves through LDS, a wave's 32 rows x 128 columns at a time (one row of its MFMA
-    // tiles): the wave writes the accumulators as the matrix pipe left them, reads whole rows
-    // back, four columns per lane, and stores 16 (or 8, or 4) bytes per lane, half a wave to a row.
-    // That keeps the 256 accumulators out of the vector registers (where the compiler would
-    // otherwise gather them all at once, spilling what the K loop needs) and gives row-long
-    // stores. A staged row is 136 floats: the two rows a store instruction touches, 4 apart,
-    // fall on disjoint banks. Each wave has a region of its own, so no barrier between passes.
-    __syncthreads();                                   // every wave is done with the operands in LDS
-    constexpr int EP_LD = (NWN == 2 && NWM == 2 && TN > 1) ? 136 : WN + 8;
-    constexpr int LPR = ((NWN == 2 && NWM == 2 && TN > 1) || 64 % (WN / 4)) ? 32 : WN / 4;   // lanes to a staged row
-    static_assert((4 * EP_LD) % 64 == 32 && NW / 2 * 32 * EP_LD * 4 <= (BM + BN) * DM_BK * 2, "staging layout");
-    float* staged = reinterpret_cast<float*>(wave >= NW / 2 ? stage1 : stage0) + (wave % (NW / 2)) * (32 * EP_LD);
-    const int out_col = (lane % LPR) * 4;              // of the wave's columns: lanes past them (narrow tiles) sit out
-    const bool lane_on = out_col < WN;
-    const int n = n0 + wn * WN + out_col;
-    float bn[4] = {0.f, 0.f, 0.f, 0.f};
-    if (bias && lane_on) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (n + c < N) bn[c] = bias[n + c];
-    }
+    // The tile leaves from the accumulators, as the matrix pipe left them: a lane has one column (a weight row), lane % 32 of a
+    // 32x32 product, of 16 rows, so a store of 64 lanes is two rows of 128 bytes, and the stores of a tile go out one after the
+    // other without waiting for anything. Through LDS, 32 rows at a time and 16 bytes a lane as it was before, the waves wrote,
+    // waited and read back in turn. Measured with the last steps' loads left out, us before and now: 8,192 rows of 6,144 by 2,048
+    // 201 and 178, gate and up of 16,384 by 2,048 469 and 458; 2,048 rows 57.4 and 51.0, 124 and 121, of 2,048 by 2,048 added
+    // 27.5 and 24.0, by 8,192 76.4 and 74.9; 520 rows of 6,144 by 2,048 24.0 and 21.4, of 2,048 by 2,048 in two slices 13.3 and 10.9.
+    const int l32 = lane & 31, m_lane = m0 + wm * WM + 4 * (lane >> 5), n_lane = n0 + wn * WN + l32;
     const bool swiglu = epilogue == EPI_SWIGLU;
     const bool adds = epilogue == EPI_ADD;             // (float32 out; the launcher sees to it)
-    const int out_n = swiglu ? N / 2 : N;              // columns of Y
-    const int per_lane = swiglu ? 2 : 4;               // outputs a lane holds of a row
-    // whole vectors: every row of this tile inside, the lane's columns inside, rows of Y aligned
-    const bool vectors = m0 + BM <= M && n0 + BN <= N && out_n % per_lane == 0 &&
-                         ((uintptr_t)Y % (per_lane * sizeof(TOut))) == 0;
-    constexpr int ITS = 32 * LPR / 64;                 // rows of a pass that a lane stores
-    constexpr bool CAN_ADD = std::is_same<TOut, float>::value;
+    const bool inside = m0 + BM <= M && n0 + BN <= N;
+    constexpr bool FLOAT = std::is_same<TOut, float>::value;
+    float bn[TN];
 #pragma unroll
-    for (int i = 0; i < TMI; ++i) {
-        // what the output holds (the epilogue that adds): a pass's rows asked for together, before the
-        // accumulators go through LDS, so that the trips to memory overlap each other and the staging
-        float4 held[CAN_ADD ? ITS : 1];
-        if (CAN_ADD && adds && vectors && lane_on) {
+    for (int j = 0; j < TN; ++j) bn[j] = bias && n_lane + j * 32 < N ? bias[n_lane + j * 32] : 0.f;
+    if (swiglu) {
+        // Gates and ups are neighbouring lanes: of two rows the even lane takes the first one's pair and the odd lane the
+        // second's. In bfloat16 two such results of neighbouring columns go on to one lane, of two rows and the next two again.
+        const int out_n = N / 2;
+        const bool odd = lane & 1, upper = lane & 2;
+        const bool pairs = !FLOAT && inside && out_n % 2 == 0 && ((uintptr_t)Y & 3) == 0;
+        auto gated = [&](const f32x16& a, float b, int r) __attribute__((always_inline)) {       // row r + odd, column l32 / 2
+            const float first = a[r] + b, second = a[r + 1] + b;
+            const float other = lane_xor<1>(odd ? first : second);
+            return gated_mul_fast(epilogue, odd ? other : first, odd ? second : other);
+        };
 #pragma unroll
-            for (int it = 0; it < ITS; ++it) {
-                const int m = m0 + wm * WM + i * 32 + it * (64 / LPR) + lane / LPR;
-                held[CAN_ADD ? it : 0] = held_vector<TOut>(Y + (size_t)m * out_n + n);
-            }
-        }
+        for (int i = 0; i < TMI; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j) {
+                const int col = (n0 + wn * WN + j * 32) / 2;
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                staged[((r >> 2) * 8 + (lane >> 5) * 4 + (r & 3)) * EP_LD + j * 32 + (lane & 31)] = acc[i][j][r];
-#pragma unroll
-        for (int it = 0; it < ITS; ++it) {
-            if (!lane_on) continue;
-            const int row = it * (64 / LPR) + lane / LPR;
-            const float4 v = *reinterpret_cast<const float4*>(&staged[row * EP_LD + out_col]);
-            const int m = m0 + wm * WM + i * 32 + row;
-            float o[4] = {v.x + bn[0], v.y + bn[1], v.z + bn[2], v.w + bn[3]};
-            if (swiglu) {
-                o[0] = gated_mul_fast(epilogue, o[0], o[1]);
-                o[1] = gated_mul_fast(epilogue, o[2], o[3]);
-            }
-            TOut* dst = Y + (size_t)m * out_n + (swiglu ? n / 2 : n);
-            if (vectors) {
-                if (CAN_ADD && adds) {
-                    const float4 h = held[CAN_ADD ? it : 0];
-                    o[0] = h.x + o[0], o[1] = h.y + o[1], o[2] = h.z + o[2], o[3] = h.w + o[3];
-                }
-                store_vector<TOut>(dst, o, swiglu);
-            } else if (m < M) {
-                if (swiglu) {
-                    if (n + 1 < N) store_f32<TOut>(dst, 0, o[0]);
-                    if (n + 3 < N) store_f32<TOut>(dst, 1, o[1]);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < 4; ++c)
-                        if (n + c < N) store_f32<TOut>(dst, c, adds ? held_f32<TOut>(dst, c) + o[c] : o[c]);
+                for (int r = 0; r < 16; r += 4) {
+                    const float lo = gated(acc[i][j], bn[j], r), hi = gated(acc[i][j], bn[j], r + 2);
+                    const int m = m_lane + i * 32 + (r >> 2) * 8 + odd;
+                    if (pairs) {
+                        const float other = lane_xor<2>(upper ? lo : hi);
+                        *reinterpret_cast<uint32_t*>(Y + (size_t)(m + (upper ? 2 : 0)) * out_n + col + (l32 >> 2) * 2) =
+                            upper ? f32x2_to_bf16x2(other, hi) : f32x2_to_bf16x2(lo, other);
+                    } else if (col + (l32 >> 1) < out_n) {
+                        if (m < M) store_f32<TOut>(Y, (size_t)m * out_n + col + (l32 >> 1), lo);
+                        if (m + 2 < M) store_f32<TOut>(Y, (size_t)(m + 2) * out_n + col + (l32 >> 1), hi);
+                    }
                 }
             }
+        return;
+    }
+    if constexpr (FLOAT) {
+#pragma unroll
+        for (int i = 0; i < TMI; ++i) {
+            float* dst = Y + (size_t)(m_lane + i * 32) * N + n_lane;
+            if (inside) {
+                // what the output holds (the epilogue that adds): the rows of a product asked for together
+                float held[TN][16];
+                if (adds) {
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) held[j][r] = dst[(size_t)((r >> 2) * 8 + (r & 3)) * N + j * 32];
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const float v = acc[i][j][r] + bn[j];
+                        dst[(size_t)((r >> 2) * 8 + (r & 3)) * N + j * 32] = adds ? held[j][r] + v : v;
+                    }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        const int row = (r >> 2) * 8 + (r & 3);
+                        if (m_lane + i * 32 + row >= M || n_lane + j * 32 >= N) continue;
+                        float* at = dst + (size_t)row * N + j * 32;
+                        const float v = acc[i][j][r] + bn[j];
+                        *at = adds ? *at + v : v;
+                    }
+            }
         }
+    } else {
+        const bool odd = lane & 1, pairs = inside && N % 2 == 0 && ((uintptr_t)Y & 3) == 0;
+#pragma unroll
+        for (int i = 0; i < TMI; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; r += 2) {
+                    const float first = acc[i][j][r] + bn[j], second = acc[i][j][r + 1] + bn[j];
+                    const int m = m_lane + i * 32 + (r >> 2) * 8 + (r & 3), n = n_lane + j * 32;
+                    if (pairs) {                       // (two neighbouring columns of the first row in the even lane, of the second in the odd)
+                        const float other = lane_xor<1>(odd ? first : second);
+                        *reinterpret_cast<uint32_t*>(Y + (size_t)(m + odd) * N + n - odd) =
+                            odd ? f32x2_to_bf16x2(other, second) : f32x2_to_bf16x2(first, other);
+                    } else if (n < N) {
+                        if (m < M) store_f32<TOut>(Y, (size_t)m * N + n, first);
+                        if (m + 1 < M) store_f32<TOut>(Y, (size_t)(m + 1) * N + n, second);
+                    }
+                }
     }
 }
 
