@@ -1078,24 +1078,17 @@ static bool dma_tile_takes(int m, int n, int k) {
 
 // Which tile (bm = 256, 192 or 128 activation rows, tn = 4, 3, 2, 1 for 256, 192, 128, 64 weight rows; 192 with
 // bm 256 only, 64 with bm 128 only, bm 192 with 256 only), on how many stages, and how many slices of K suit a product of many rows; tn = 0:
-// none (a K the kernel does not take). A model of the time, fitted to this machine over 128 to 8,192
-// rows and seven weight shapes, every tile and 1 to 8 slices measured (what it picks is within 1 % of
-// the fastest on average and within 7 % on every shape whose consumer can add slices):
-//   - a K-step of 64 takes a block alone on its CU the first figure below with few CUs busy and the
-//     second with all 256 (clocks, L2), in between in proportion:
-//         128x128 0.46 .. 0.78 us    128x256 0.70 .. 1.08    256x128 0.66 .. 1.08
-//         256x192 0.89 .. 1.30       256x256 1.03 .. 1.58       192x256 0.95 .. 1.25
-//     (192 activation rows suit portions a little over a power of two, a prompt's beside the tokens of other requests:
-//     gate and up of 520 rows 57 us on the 256x256 tile and 51, 1,536 rows 117 and 104, 2,300 rows 174 and 149. K in one
-//     piece and of at most 4,096 only: with 8,192 a step took 1.13 us on 24 CUs where 2,048 took 0.85);
-//   - a tile of 128 rows by 64 weight rows on four waves and four stages takes 0.35 .. 0.50 us a step: with at
-//     most 128 rows (one tile down the rows) it makes twice the blocks of the 128x128 tile out of a weight
-//     that is streamed once, and a block's share of the weights is what bounds such a product (measured at
-//     96 and 128 rows: 21 us against 27 on gate/up, 8 to 13 against 11 to 18 on the sliced products);
+// none (a K the kernel does not take). A model of the time, fitted to this machine:
+//   - a K-step of 64 takes a block alone on its CU `few` us with few CUs busy and `all` with all 256 (clocks, L2), in
+//     between in proportion (the tables below; 192 activation rows suit portions a little over a power of two, a prompt's beside
+//     the tokens of other requests);
+//   - a tile of 128 rows by 64 weight rows on four waves and four stages makes twice the blocks of the 128x128 tile: with at most
+//     128 rows out of a weight that is streamed once, where a block's share of the weights is what bounds such a product, and
+//     wherever the larger tiles leave CUs idle (520 rows of 3,072 by 2,048 13.7 us against 16.2);
 //   - two blocks fit a CU where their stages take 80 KB or less each (the 128x128 tile on two
-//     stages); a step of both then takes 1.09 us, and with two on some CUs only, in between;
-//   - the 128x128 tile can instead keep four stages (one block a CU, three steps' loads in flight):
-//     0.33 .. 0.53 us a step, which pays where the tiles are one round of the CUs or less;
+//     stages); a step of both then takes `both`, and with two on some CUs only, in between;
+//   - the 128x128 tile can instead keep four stages (one block a CU, three steps' loads in flight),
+//     which pays where the tiles are one round of the CUs or less;
 //   - with one or two tiles down the rows (a decode batch of 65 to 256 rows) every block meets its
 //     weights first, and cold: a step then takes 0.55 us at least on two stages and 0.36 on four;
 //   - a block's beginning and end take 4.3 us + 0.116 us per MFMA of a SIMD in a K-step
@@ -1103,20 +1096,31 @@ static bool dma_tile_takes(int m, int n, int k) {
 //   - blocks run in rounds of what fits the chip at once; the operands have to come from memory
 //     once (5.5 TB/s) and the results have to go there (7.6 TB/s); a slice beyond the first costs
 //     its consumer one more pass over rows x width of float32 (5 TB/s).
-// `fixed_slices` > 0: the caller has decided (1: its consumer cannot add slices).
+// `fixed_slices` > 0: the caller has decided. Then the tile is chosen by what the kernel takes now (18 numbers of rows from 136
+// to 8,192, 18 weights, every tile measured: 0.6 % above the fastest on average, where the figures of before were 5 %; one
+// product in 471 more than 3 % slower than the tile they chose). Else the slices are, by the figures they were always
+// chosen with: a count once chosen stays, as fewer slices are further from 64 bits (151 rows of 69,516 by 3,584 in two 2.5e-7 and in one
+// 3.7e-7), and what a tile is does not change a sum.
 struct DmaPlan {
     int bm, tn, slices, stages;
 };
+struct DmaStep {
+    double few, all;
+};
+struct DmaRates {
+    DmaStep t256x256, t256x192, t256x128, t192x256, t128x256, t128x128, t128x128_four, t128x64_four;
+    double both;
+};
+static const DmaRates dma_rates_slices = {{1.03, 1.58}, {0.89, 1.30}, {0.66, 1.08}, {0.95, 1.25}, {0.70, 1.08}, {0.46, 0.78}, {0.33, 0.53},
+                                          {0.35, 0.50}, 1.09};
+static const DmaRates dma_rates_tile = {{1.06, 1.63}, {0.89, 1.30}, {0.49, 1.13}, {0.94, 1.29}, {0.62, 1.08}, {0.46, 0.84}, {0.37, 0.58},
+                                        {0.35, 0.48}, 1.15};
 static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
     DmaPlan best{0, 0, fixed_slices > 0 ? fixed_slices : 1, 2};
     if (m <= 64 || !dma_tile_takes(m, n, k)) return best;
+    const DmaRates& rates = fixed_slices > 0 ? dma_rates_tile : dma_rates_slices;
     double best_cost = 0.0;
-    // (the 192-row tile at the end, and only where the others leave K in one piece: it takes no slices' place, whose sums are
-    // nearer to 64 bits, 151 rows of 69,516 by 3,584 in two 2.5e-7 and in one 3.7e-7)
-    for (int turn = 0; turn < 7; ++turn) {
-        const bool narrow = turn == 6;
-        const int slices = narrow ? 1 : (const int[]){1, 2, 3, 4, 6, 8}[turn];     // (3 and 6: a K of 27 or 9 times 256 has no other cut)
-        if (narrow && best.slices > 1) break;
+    for (int slices : {1, 2, 3, 4, 6, 8}) {            // (3 and 6: a K of 27 or 9 times 256 has no other cut)
         if (fixed_slices > 0 && slices != fixed_slices) continue;
         if (k % (128 * slices) != 0 || (slices > 1 && k / slices < 512)) continue;
         for (int bm = 256; bm >= 128; bm -= 64) {
@@ -1124,9 +1128,8 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
             for (int tn = 4; tn >= 1; --tn) {
                 if (tn == 3 && bm != 256) continue;
                 if (tn == 1 && bm != 128) continue;
-                // (K of 128 is all beginning and end, and up to 128 rows one tile of 128 has them all: 65 rows of 16,384 by
-                // 3,072 29.8 us on it, 31.4; 5,000 rows of 4,608 by 128 31.2 on 256 rows, 34.4)
-                if ((bm == 192) != narrow || (narrow && (tn != 4 || k > 4096 || k < 256 || m <= 128))) continue;
+                // (192 rows: the tile is chosen among all, the slices never were)
+                if (bm == 192 && (tn != 4 || fixed_slices <= 0 || m <= 128 || k / slices < 256)) continue;
                 const int bn = 64 * tn;
                 for (int stages = 2; stages <= 4; stages += 2) {
                     // four stages: the 128x128 tile and the 128x64 one (which runs on four only), K-steps in fours
@@ -1137,16 +1140,11 @@ static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
                     const long long rounds = (blocks + at_once - 1) / at_once;
                     const long long per_round = (blocks + rounds - 1) / rounds;
                     const double cus = (double)std::min<long long>(256, per_round);
-                    double few, all;
-                    if (bm == 192) few = 0.95, all = 1.25;
-                    else if (bm == 128 && tn == 1) few = 0.35, all = 0.50;
-                    else if (bm == 128 && tn == 2) few = stages == 4 ? 0.33 : 0.46, all = stages == 4 ? 0.53 : 0.78;
-                    else if (bm == 128) few = 0.70, all = 1.08;
-                    else if (tn == 2) few = 0.66, all = 1.08;
-                    else if (tn == 3) few = 0.89, all = 1.30;
-                    else few = 1.03, all = 1.58;
-                    double step = per_round > 256 ? all + (1.09 - all) * (per_round - 256) / 256.0    // some CUs, or all, with two
-                                                  : few + (all - few) * cus / 256.0;
+                    const DmaStep& a_step = bm == 192 ? rates.t192x256 : bm == 128 && tn == 1 ? rates.t128x64_four
+                                          : bm == 128 && tn == 2 ? (stages == 4 ? rates.t128x128_four : rates.t128x128)
+                                          : bm == 128 ? rates.t128x256 : tn == 2 ? rates.t256x128 : tn == 3 ? rates.t256x192 : rates.t256x256;
+                    double step = per_round > 256 ? a_step.all + (rates.both - a_step.all) * (per_round - 256) / 256.0    // some CUs, or all, with two
+                                                  : a_step.few + (a_step.all - a_step.few) * cus / 256.0;
                     if (tiles_m <= 2) step = std::max(step, stages == 4 ? 0.36 : 0.55);
                     // one tile down the rows: a block streams its weight rows alone, 128 bytes of each a
                     // step, and one CU draws about 28 GB/s of cold weights (0.60 us a step measured on the
