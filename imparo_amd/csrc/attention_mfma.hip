@@ -210,8 +210,7 @@ __device__ __forceinline__ void decode_tile(DecodeState<ND>& st, const DecodeTil
         sv[j] = ok ? score : -INFINITY;
         mx = fmaxf(mx, sv[j]);
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+    mx = max_16_32(mx);
     const float m_new = fmaxf(st.m, mx);
     const float corr = (st.m == -INFINITY) ? 0.f : __expf(st.m - m_new);
     union {
@@ -230,8 +229,7 @@ __device__ __forceinline__ void decode_tile(DecodeState<ND>& st, const DecodeTil
         if (exact) pl.h[j] = f32_to_bf16(p - bf16_to_f32(pb.h[j]));
         psum += exact ? p : bf16_to_f32(pb.h[j]);             // the denominator sums what the product uses
     }
-    psum += __shfl_xor(psum, 16, WAVE);
-    psum += __shfl_xor(psum, 32, WAVE);
+    psum = sum_16_32(psum);
     st.l = st.l * corr + psum;
     st.m = m_new;
     // ---- weighted values
@@ -311,8 +309,7 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
         for (int dk = 0; dk < NK; ++dk)
 #pragma unroll
             for (int j = 0; j < 8; ++j) ss = fmaf(e[dk][j], e[dk][j], ss);
-        ss += __shfl_xor(ss, 16, WAVE);
-        ss += __shfl_xor(ss, 32, WAVE);
+        ss = sum_16_32(ss);
         const float scale = head_norm_scale(ss, D, eps);
 #pragma unroll
         for (int dk = 0; dk < NK; ++dk)
@@ -357,13 +354,15 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
 // rotated here, 9.6 | 11.1, over 60 keys 7.2 | 10.5, queries given 7.1 | 10.1; 24 heads of 128, queries given, 11.4 | 12.7. Not
 // from the projection's rows with heads above 64 (15.4 | 14.4: both splits' waves make the rotations one CU's four SIMDs then
 // share), nor three or four splits (16 waves on one CU: 1,000 keys 17.7 | 13.4, queries given 12.9 | 11.7).
-template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1>
+// EXACT: see decode_tile; part of the kernel's type, as branches on it inside a tile kept the scheduler from filling one weight's
+// waits with the next one's work.
+template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1, bool EXACT = false>
 __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decode(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ seg_start, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ block_table, int table_stride, int page_size, int heads, int kv_heads, int n_pages,
-    float scale, int window, int n_splits, FromQkv fq, int exact, Rule rule) {
+    float scale, int window, int n_splits, FromQkv fq, Rule rule) {
     constexpr int D = ND * 16, NK = (ND + 1) / 2;
     constexpr int TILES = DEC_SPLIT / (MFMA_WAVES * 32);   // tiles a wave takes at most
     __shared__ float sm[SPLITS * MFMA_WAVES][16], sl[SPLITS * MFMA_WAVES][16];
@@ -472,7 +471,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         if (kv_base < k_end) {
             const int kb = walk.key(kv_base);
             const bool full = (kb >= lo || kb + 31 < keep) && kb + 31 <= last;
-            decode_tile<ND>(st, regs[j], kb, lo, hi_q, lo, last, full, scale, lane, exact != 0, keep, cap);
+            decode_tile<ND>(st, regs[j], kb, lo, hi_q, lo, last, full, scale, lane, EXACT, keep, cap);
         }
     }
     if constexpr (FROM_QKV) {
@@ -501,8 +500,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
             for (int dk = 0; dk < NK; ++dk)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) dot = fmaf((float)st.q[dk].v[j], (float)kf[dk].v[j], dot);
-            dot += __shfl_xor(dot, 16, WAVE);
-            dot += __shfl_xor(dot, 32, WAVE);
+            dot = sum_16_32(dot);
             if (qvalid) {
                 const float sc = dot * scale;
                 const float m_new = fmaxf(st.m, sc);
@@ -857,8 +855,7 @@ __global__ __launch_bounds__(MFMA_WAVES * 64) void k_attn_prefill(
                         mx = fmaxf(mx, sc[kt][i]);
                     }
             }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+            mx = max_16_32(mx);
             const float m_new = fmaxf(st.m, mx);
             const float corr = (st.m == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(st.m - m_new);
             const float m_sub = (m_new == -INFINITY) ? 0.f : m_new;        // exp2(-inf - 0) = 0: masked keys
@@ -884,8 +881,7 @@ __global__ __launch_bounds__(MFMA_WAVES * 64) void k_attn_prefill(
                 pb[kt] = pk.v;
                 pl[kt] = lo.v;
             }
-            psum += __shfl_xor(psum, 16, WAVE);
-            psum += __shfl_xor(psum, 32, WAVE);
+            psum = sum_16_32(psum);
             st.l = st.l * corr + psum;
             st.m = m_new;
 #pragma unroll
@@ -937,14 +933,18 @@ __global__ __launch_bounds__(MFMA_WAVES * 64) void k_attn_prefill(
 // block table a tile then serves every thread, and what a thread reads of a tile is at a fixed place
 // inside the page: a quarter of the instructions of the general staging, which was a quarter to a
 // third of the kernel's time.
-template <int ND, int HALVES, bool PAGE_TILE, bool EXT>
-__global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 2 : 1) void k_attn_prefill_x32(
+// EXACT: what the rounding to bfloat16 takes off a weight goes through second products (part of the kernel's type: branches on
+// it inside a tile kept the scheduler from mixing one weight's instructions with the next one's).
+// (three waves a SIMD with heads of up to 64: with one register more than that leaves, 8,192 exact queries over 16,384 keys took 1,614
+// us and not 1,415; 1,497 before)
+template <int ND, int HALVES, bool PAGE_TILE, bool EXT, bool EXACT>
+__global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 3 : 1) void k_attn_prefill_x32(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     bf16_t* __restrict__ out, const int32_t* __restrict__ rows, int n_rows,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_len, const int32_t* __restrict__ positions,
     const int32_t* __restrict__ block_table, int table_stride, int page_size, int heads, int kv_heads, int n_pages,
     float scale, int window, int heads_per_block, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int exact, Rule rule) {
+    Rule rule) {
     constexpr int D = ND * 16, NK = ND / 2;
     const int keep = EXT ? rule.keep : 0;
     // Rows of K lie their length + 32 bytes apart: the fragment reads (row lane % 16, 16-byte piece lane / 16) then
@@ -1219,8 +1219,7 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 2 : 1) void k_attn_prefi
                             mx = fmaxf(mx, sc[h][s16][i]);
                         }
                 }
-                mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-                mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+                mx = max_16_32(mx);
                 const float m_new = fmaxf(m_run[h], mx);
                 const float m_sub = (m_new == -INFINITY) ? 0.f : m_new * scale_log2;   // exp2(-inf - 0) = 0: masked keys
 #pragma unroll
@@ -1231,8 +1230,8 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 2 : 1) void k_attn_prefi
                         const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[h][s16][i], scale_log2, -m_sub));
                         const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[h][s16][i + 1], scale_log2, -m_sub));
                         pk[i >> 1] = f32x2_to_bf16x2(p0, p1);
-                        // `exact`: what the rounding took off a weight goes through second products (sum and values)
-                        if (exact)
+                        // EXACT: what the rounding took off a weight goes through second products (sum and values)
+                        if constexpr (EXACT)
                             lk[i >> 1] = f32x2_to_bf16x2(p0 - __uint_as_float(pk[i >> 1] << 16),
                                                          p1 - __uint_as_float(pk[i >> 1] & 0xffff0000u));
                     }
@@ -1261,7 +1260,7 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 2 : 1) void k_attn_prefi
 #pragma unroll
                 for (int G = 0; G < 2; ++G)
                     l_acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pb[h][G].v, l_acc[h], 0, 0, 0);
-                if (exact) {
+                if constexpr (EXACT) {
 #pragma unroll
                     for (int G = 0; G < 2; ++G)
                         l_acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones.v, pl[h][G].v, l_acc[h], 0, 0, 0);
@@ -1277,7 +1276,7 @@ __global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 2 : 1) void k_attn_prefi
 #pragma unroll
                     for (int h = 0; h < HALVES; ++h)
                         o[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pb[h][G].v, o[h][dt], 0, 0, 0);
-                    if (exact) {
+                    if constexpr (EXACT) {
 #pragma unroll
                         for (int h = 0; h < HALVES; ++h)
                             o[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pl[h][G].v, o[h][dt], 0, 0, 0);
@@ -1457,22 +1456,25 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
     const bool in_block = n_splits == 2 && !(from_qkv && head_dim > 64);
     dim3 grid(in_block ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
 #define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT)                                                                \
-    k_attn_decode<ND, QKV, EXT, SPLITS><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                                   \
+    k_attn_decode<ND, QKV, EXT, SPLITS, EXACT><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                            \
         Q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,           \
-        positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, EXACT, rule)
+        positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, rule)
 #define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT)                                                                       \
     do {                                                                                                             \
         if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT);                                \
         else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT);                                                               \
     } while (0)
+    if (given && !exact) return IMPARO_BAD_ARGUMENT;         // (the rules run with exact weights)
     if (from_qkv) {
-        if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, 0);
-        else if (head_dim == 128) DECODE_ANY(8, true, false, nullptr, *from_qkv, 0);
+        if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, false);
+        else if (head_dim == 128) DECODE_ANY(8, true, false, nullptr, *from_qkv, false);
         else return IMPARO_BAD_ARGUMENT;
     } else if (given) {
-        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, true, (const bf16_t*)q, FromQkv{}, exact));
+        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, true, (const bf16_t*)q, FromQkv{}, true));
+    } else if (exact) {
+        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, false, (const bf16_t*)q, FromQkv{}, true));
     } else {
-        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, false, (const bf16_t*)q, FromQkv{}, exact));
+        DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, false, (const bf16_t*)q, FromQkv{}, false));
     }
 #undef DECODE_ANY
 #undef DECODE_GO
@@ -1708,7 +1710,7 @@ static int attention_prefill_entry(const void* q, const void* k_cache, const voi
                                    const int32_t* block_table, int table_stride, int page_size,
                                    int heads, int kv_heads, int head_dim, int n_pages, float scale, int window,
                                    imparo_stream stream, int exact, const ImparoAttentionRule* given = nullptr) {
-    if (given && imparo_attention_rule_bad(*given, window)) return IMPARO_BAD_ARGUMENT;
+    if (given && (imparo_attention_rule_bad(*given, window) || !exact)) return IMPARO_BAD_ARGUMENT;     // (rules run with exact weights)
     const Rule rule = rule_of(given);
     const int bad = check_common(q, k_cache, v_cache, out, rows, seg_start, positions, block_table, table_stride,
                                  page_size, heads, kv_heads, head_dim, n_pages, window);
@@ -1726,15 +1728,16 @@ static int attention_prefill_entry(const void* q, const void* k_cache, const voi
         const int hpb = p.hpb;
         const bool wide = p.wide;
         dim3 grid32((unsigned)(n_tiles * (p.qt < 64 ? 64 / p.qt : 1)), heads / hpb, n_splits);
-#define PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, EXT)                                                                 \
-    k_attn_prefill_x32<ND, HALVES, PAGE_TILE, EXT><<<grid32, MFMA_WAVES * 64, 0, s>>>(                               \
+#define PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, EXT, EXACT)                                                          \
+    k_attn_prefill_x32<ND, HALVES, PAGE_TILE, EXT, EXACT><<<grid32, MFMA_WAVES * 64, 0, s>>>(                        \
         (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, (bf16_t*)out, rows, n_rows, seg_start,     \
         seg_len, positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, hpb,      \
-        part_o, part_ml, exact, rule)
+        part_o, part_ml, rule)
 #define PREFILL_X32_GO(ND, HALVES, PAGE_TILE)                                                                       \
     do {                                                                                                             \
-        if (given) PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, true);                                                     \
-        else PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, false);                                                          \
+        if (given) PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, true, true);                                               \
+        else if (exact) PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, false, true);                                         \
+        else PREFILL_X32_RUN(ND, HALVES, PAGE_TILE, false, false);                                                   \
     } while (0)
 #define PREFILL_X32(ND)                                                                                              \
     if (wide && page_size >= PX_KEYS) PREFILL_X32_GO(ND, 2, true);                                                   \

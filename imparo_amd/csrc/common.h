@@ -74,6 +74,54 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// What the lane N apart (lane ^ N) holds, on moves inside rows of 16 and lane swaps: a few cycles each, where a shuffle is a trip
+// through LDS. Both lanes must be active (for 16 and 32 the whole wave).
+template <int N>
+__device__ __forceinline__ uint32_t lane_xor_bits(uint32_t v) {
+    static_assert(N == 1 || N == 2 || N == 4 || N == 8 || N == 16 || N == 32, "a power of two inside a wave");
+    if constexpr (N == 1) return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);           // quad_perm:[1,0,3,2]
+    if constexpr (N == 2) return __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);           // quad_perm:[2,3,0,1]
+    if constexpr (N == 4) {                                                                          // row_shl:4 into quads 0 and 2,
+        const uint32_t up = __builtin_amdgcn_update_dpp(v, v, 0x104, 0xf, 0x5, false);               // row_shr:4 into quads 1 and 3
+        return __builtin_amdgcn_update_dpp(up, v, 0x114, 0xf, 0xA, false);
+    }
+    if constexpr (N == 8) return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);          // row_ror:8
+    if constexpr (N == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return threadIdx.x & 16 ? r[0] : r[1];
+    }
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return threadIdx.x & 32 ? r[0] : r[1];
+}
+template <int N> __device__ __forceinline__ float lane_xor(float v) { return __uint_as_float(lane_xor_bits<N>(__float_as_uint(v))); }
+template <int N> __device__ __forceinline__ int lane_xor(int v) { return (int)lane_xor_bits<N>((uint32_t)v); }
+
+// Sums and maxima over the lanes 16 and then 32 apart (all 64 lanes active); a sum of two is the same either way round
+__device__ __forceinline__ float sum_16_32(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max_16_32(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// The sum over LANES neighbouring lanes (a power of two), the nearest first (1, 2, 4, ... apart): after a step all lanes that near
+// agree, so a mirrored quad or half row stands for the one 4 or 8 apart
+template <int LANES>
+__device__ __forceinline__ float sum_near_first(float v) {
+    if constexpr (LANES > 1) v += lane_xor<1>(v);
+    if constexpr (LANES > 2) v += lane_xor<2>(v);
+    if constexpr (LANES > 4) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x141, 0xf, 0xf, false));   // row_half_mirror
+    if constexpr (LANES > 8) v += __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x140, 0xf, 0xf, false));   // row_mirror
+    if constexpr (LANES > 16) v += lane_xor<16>(v);
+    if constexpr (LANES > 32) v += lane_xor<32>(v);
+    return v;
+}
+
 // Sum over a block of up to 1024 threads in whole waves; every thread gets the result.
 // `scratch` holds at least 16 floats of LDS. The order of the additions
 // depends only on the block size, never on the data.

@@ -179,8 +179,7 @@ __global__ __launch_bounds__(DS_MAX_THREADS) void k_decay_scan(const DecayScanAr
                         S[j] *= CHAN ? gg[CHAN ? j : 0] : a;
                         seen = fmaf(S[j], kk[j], seen);
                     }
-#pragma unroll
-                for (int off = 1; off < KS; off <<= 1) seen += __shfl_xor(seen, off, WAVE);
+                seen = sum_near_first<KS>(seen);
                 val = sb[tok] * (val - seen);
 #pragma unroll
                 for (int j = 0; j < DS_KPT; ++j)
@@ -198,8 +197,7 @@ __global__ __launch_bounds__(DS_MAX_THREADS) void k_decay_scan(const DecayScanAr
                 if constexpr (MODE == 1) decay_all *= a;
             }
             if (MODE != 1) {
-#pragma unroll
-                for (int off = 1; off < KS; off <<= 1) acc += __shfl_xor(acc, off, WAVE);
+                acc = sum_near_first<KS>(acc);
                 if (ks == 0 && live)
                     A.out[(size_t)(first + t0 + tok) * heads * vdim + (size_t)h * vdim + v] = fmaf(skip, raw, acc);
             }
@@ -1235,11 +1233,6 @@ struct ChannelHeadArgs {
 };
 #define CDH_RANK 128
 
-template <int N>
-__device__ __forceinline__ float cdh_quad(float v) {         // the lane N (1 or 2) apart among four neighbours
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), N == 1 ? 0xB1 : 0x4E, 0xf, 0xf, false));
-}
-
 template <typename TOut>
 __global__ __launch_bounds__(1024) void k_channel_delta_head(const ChannelHeadArgs A, TOut* __restrict__ out) {
     constexpr int D = CDS_DIM, WAVES = 16;
@@ -1297,8 +1290,7 @@ __global__ __launch_bounds__(1024) void k_channel_delta_head(const ChannelHeadAr
                 sum = fmaf(__uint_as_float(u[i] & 0xffff0000u), l[2 * i + 1], sum);
             }
         }
-        sum += cdh_quad<1>(sum);
-        sum += cdh_quad<2>(sum);
+        sum = sum_near_first<4>(sum);
         if (piece == 0) {
             if (gate) gates[dot - D] = sum;
             else sg[dot] = expf(-rate * ds_softplus(sum + bias));

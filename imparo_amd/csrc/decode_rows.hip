@@ -346,7 +346,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                 }
             }
             if (EPI == ROWS_TANH) continue;
-            sq += __shfl_xor(sq, 16, WAVE);             // the two lanes of a token sit 16 apart
+            sq += lane_xor<16>(sq);             // the two lanes of a token sit 16 apart
             if (g == 0) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
         }
     }

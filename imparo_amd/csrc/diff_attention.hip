@@ -472,8 +472,7 @@ __global__ __launch_bounds__(256) void k_diff_attention_tiles(
                         tile_max = fmaxf(tile_max, sc[mb][i]);
                     }
             }
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, WAVE));
-            tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, WAVE));
+            tile_max = max_16_32(tile_max);
             const float m_new = fmaxf(mx[m], tile_max);
             const float m_use = m_new == -INFINITY ? 0.f : m_new;
             corr[m] = mx[m] == -INFINITY ? 0.f : __expf(mx[m] - m_use);
@@ -486,8 +485,7 @@ __global__ __launch_bounds__(256) void k_diff_attention_tiles(
                     p[mb][i] = __expf(sc[mb][i] - m_use);       // exp(-inf) = 0 for keys that are not seen
                     tile_sum += p[mb][i];
                 }
-            tile_sum += __shfl_xor(tile_sum, 16, WAVE);
-            tile_sum += __shfl_xor(tile_sum, 32, WAVE);
+            tile_sum = sum_16_32(tile_sum);
             sum[m] = sum[m] * corr[m] + tile_sum;
             mx[m] = m_new;
 #pragma unroll
@@ -540,8 +538,7 @@ __global__ __launch_bounds__(256) void k_diff_attention_tiles(
                 ss += v * v;
             }
         }
-    ss += __shfl_xor(ss, 16, WAVE);
-    ss += __shfl_xor(ss, 32, WAVE);
+    ss = sum_16_32(ss);
     const float rr = out_scale / sqrtf(ss / (float)vdim + eps);
     if (col < n_q) {
         const float* gt = gate ? gate + (size_t)t * gate_ld + (size_t)h * vdim : nullptr;
@@ -742,8 +739,7 @@ __global__ __launch_bounds__(256, 2) void k_diff_attention_shared(
                             tile_max = fmaxf(tile_max, sc[mb][i]);
                         }
                 }
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, WAVE));
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, WAVE));
+                tile_max = max_16_32(tile_max);
                 const float m_new = fmaxf(mx[m], tile_max);
                 const float m_use = m_new == -INFINITY ? 0.f : m_new;
                 corr[m] = mx[m] == -INFINITY ? 0.f : __expf(mx[m] - m_use);
@@ -756,8 +752,7 @@ __global__ __launch_bounds__(256, 2) void k_diff_attention_shared(
                         p[mb][i] = __expf(sc[mb][i] - m_use);
                         tile_sum += p[mb][i];
                     }
-                tile_sum += __shfl_xor(tile_sum, 16, WAVE);
-                tile_sum += __shfl_xor(tile_sum, 32, WAVE);
+                tile_sum = sum_16_32(tile_sum);
                 sum[m] = sum[m] * corr[m] + tile_sum;
                 mx[m] = m_new;
 #pragma unroll
@@ -808,8 +803,7 @@ __global__ __launch_bounds__(256, 2) void k_diff_attention_shared(
                 ss += v * v;
             }
         }
-    ss += __shfl_xor(ss, 16, WAVE);
-    ss += __shfl_xor(ss, 32, WAVE);
+    ss = sum_16_32(ss);
     const float rr = out_scale / sqrtf(ss / (float)vdim + eps);
     if (col < n_q) {
         const float* gt = gate ? gate + (size_t)t * gate_ld + (size_t)h * vdim : nullptr;

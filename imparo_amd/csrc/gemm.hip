@@ -154,7 +154,7 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
         const int m = m0 + wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
         const float v = bias ? acc[r] + bn : acc[r];
         if (epilogue == EPI_SWIGLU) {
-            const float up = __shfl_xor(v, 1, WAVE);             // gate and up rows are neighbours
+            const float up = lane_xor<1>(v);             // gate and up rows are neighbours
             if (m < M && !(lane & 1) && n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, v, up));
         } else if (m < M && n < N) {
             store_f32<TOut>(Y, (size_t)m * N + n, v);
@@ -586,7 +586,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_bf16_tile(const bf16_t* __restr
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float mine = acc[i][j][r] + bn;
-                    const float other = __shfl_xor(mine, 1, WAVE);
+                    const float other = lane_xor<1>(mine);
                     const int m = m0 + wm * 64 + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
                     if (!(lane & 1) && n + 1 < N && m < M)
                         store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul_fast(epilogue, mine, other));
@@ -733,7 +733,7 @@ __global__ __launch_bounds__(WM * WN * 64) void k_gemm_bf16_big(const bf16_t* __
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const float mine = acc[i][j][r] + bn;
-                    const float other = __shfl_xor(mine, 1, WAVE);
+                    const float other = lane_xor<1>(mine);
                     const int m = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
                     if (!(lane & 1) && n + 1 < N && m < M)
                         store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul_fast(epilogue, mine, other));
@@ -786,12 +786,6 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TOut*
 // barrier of a K-step sits before the last sub-step's products, so the matrix pipe has
 // work queued while the waves meet. Needs K a multiple of 128 (two K-steps).
 #define DM_BK 64
-
-// What the lane N (1 or 2) apart among four neighbours has
-template <int N>
-__device__ __forceinline__ float lane_xor(float v) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), N == 1 ? 0xB1 : 0x4E, 0xf, 0xf, false));
-}
 
 // TMI, TN: MFMA tiles of 32x32 down a wave's part of the activation rows and across its part of
 // the weight rows; NWM, NWN: waves down and across (eight in all). The launcher's plan chooses

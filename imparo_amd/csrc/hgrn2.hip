@@ -100,8 +100,7 @@ __global__ __launch_bounds__(HG2_THREADS) void k_hgrn2_scan(
                 }
             }
             if (MODE != 1) {
-#pragma unroll
-                for (int off = 1; off < KS; off <<= 1) acc += __shfl_xor(acc, off, WAVE);
+                acc = sum_near_first<KS>(acc);
                 if (ks == 0 && live) out[(size_t)(first + t0 + tok) * heads * vdim + (size_t)h * vdim + v] = acc;
             }
         }

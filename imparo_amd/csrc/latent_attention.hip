@@ -289,8 +289,7 @@ __global__ __launch_bounds__(LAT_WAVES * WAVE, QT == 1 ? 2 : 1) void k_latent_at
                     sv[j] = (key >= k_lo && key <= k_hi) ? s[u][j >> 2][j & 3] * scale : -INFINITY;
                     tile_max = fmaxf(tile_max, sv[j]);
                 }
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, WAVE));
-                tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, WAVE));
+                tile_max = max_16_32(tile_max);
                 const float m_new = fmaxf(m[u], tile_max);  // finite: every tile holds a key of the range
                 const float corr = __expf(m[u] - m_new);
                 float p[8], p_sum = 0.f;
@@ -329,8 +328,7 @@ __global__ __launch_bounds__(LAT_WAVES * WAVE, QT == 1 ? 2 : 1) void k_latent_at
         extern __shared__ float lat_parts[];         // [3][NV * 4 + 2][64]
         constexpr int PER = (NV * 4 + 2) * WAVE;
         float lu = l[0];
-        lu += __shfl_xor(lu, 16, WAVE);
-        lu += __shfl_xor(lu, 32, WAVE);
+        lu = sum_16_32(lu);
         if (wave > 0) {
             float* mine = lat_parts + (size_t)(wave - 1) * PER;
 #pragma unroll
@@ -382,8 +380,7 @@ __global__ __launch_bounds__(LAT_WAVES * WAVE, QT == 1 ? 2 : 1) void k_latent_at
 #pragma unroll
     for (int u = 0; u < QT; ++u) {
         float lu = l[u];
-        lu += __shfl_xor(lu, 16, WAVE);
-        lu += __shfl_xor(lu, 32, WAVE);
+        lu = sum_16_32(lu);
         const int h = h0 + 16 * u;
         if (h >= heads) continue;
         const float inv = lu > 0.f ? 1.0f / lu : 0.f;

@@ -45,6 +45,22 @@ struct MoeRouteRules {
     int always;
 };
 
+template <int N>
+__device__ __forceinline__ void moe_better_of(float& best, int& at) {
+    const float ob = lane_xor<N>(best);
+    const int oa = lane_xor<N>(at);
+    if (ob > best || (ob == best && oa < at)) best = ob, at = oa;
+}
+// the largest of the wave's, of equal ones the lowest index, in every lane
+__device__ __forceinline__ void moe_best_of_wave(float& best, int& at) {
+    moe_better_of<32>(best, at);
+    moe_better_of<16>(best, at);
+    moe_better_of<8>(best, at);
+    moe_better_of<4>(best, at);
+    moe_better_of<2>(best, at);
+    moe_better_of<1>(best, at);
+}
+
 __device__ __forceinline__ void moe_route_token(const float* __restrict__ logits, const float* __restrict__ correction,
                                                 int32_t* __restrict__ choice, float* __restrict__ weight, int t,
                                                 int n_router, int top, int scoring, const MoeRouteRules rules) {
@@ -111,12 +127,7 @@ __device__ __forceinline__ void moe_route_token(const float* __restrict__ logits
         for (int k = 0; k < rules.keep; ++k) {
             float best = gscore;
             int at = lane < rules.groups ? lane : 0x7fffffff;
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const float ob = __shfl_xor(best, off, WAVE);
-                const int oa = __shfl_xor(at, off, WAVE);
-                if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-            }
+            moe_best_of_wave(best, at);
             if (at < rules.groups) kept |= 1ull << at;
             if (lane == at) gscore = -INFINITY;
         }
@@ -136,12 +147,7 @@ __device__ __forceinline__ void moe_route_token(const float* __restrict__ logits
             const int i = lane + j * WAVE;
             if (pick[j] > best) { best = pick[j]; at = i; }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const float ob = __shfl_xor(best, off, WAVE);
-            const int oa = __shfl_xor(at, off, WAVE);
-            if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
-        }
+        moe_best_of_wave(best, at);
         float s = 0.f;
 #pragma unroll
         for (int j = 0; j < PER; ++j)

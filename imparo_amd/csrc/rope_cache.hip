@@ -11,11 +11,7 @@
 // tokens came with it, and its results must not.
 // The sum over a wave's lanes, nearest lanes first (1, 2, 4, ... apart): the kernel below that gives a lane
 // four neighbouring elements adds them in this same order, inside the lane first.
-__device__ __forceinline__ float wave_sum_near_first(float v) {
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) v += __shfl_xor(v, off, WAVE);
-    return v;
-}
+__device__ __forceinline__ float wave_sum_near_first(float v) { return sum_near_first<WAVE>(v); }
 // lane-owned pair i of a row staged in LDS: elements (i, i + n_freq), or with `interleaved`
 // (2i, 2i + 1); reads both, then writes both
 __device__ __forceinline__ void rotate_pair(float* row, int i, int n_freq, int interleaved, float sn, float cs) {
@@ -296,14 +292,13 @@ __global__ __launch_bounds__(ROPE_WAVES * WAVE) void k_qk_norm_rope_store_token6
         const float e[4] = {rows[r].x, rows[r].y, rows[r].z, rows[r].w};
         // (every lane takes part in the exchanges, also those of a value head or past the last unit)
         float ss = squares_of_four(e);
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) ss += __shfl_xor(ss, off, WAVE);
+        ss = sum_near_first<16>(ss);
         const float scale = head_norm_scale(ss, D, eps);
         float n[4], partner[4], o[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) n[j] = q_weight ? e[j] * scale * (is_q ? wq[j] : wk[j]) : e[j];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) partner[j] = interleaved ? n[j ^ 1] : __shfl_xor(n[j], 8, WAVE);
+        for (int j = 0; j < 4; ++j) partner[j] = interleaved ? n[j ^ 1] : lane_xor<8>(n[j]);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const float x0 = second[j] ? partner[j] : n[j], x1 = second[j] ? n[j] : partner[j];

@@ -14,13 +14,12 @@ __device__ __forceinline__ Best better(Best a, Best b) {
 }
 
 __device__ __forceinline__ Best block_best(Best b, Best* scratch) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        Best o;
-        o.v = __shfl_xor(b.v, off, WAVE);
-        o.i = __shfl_xor(b.i, off, WAVE);
-        b = better(b, o);
-    }
+    b = better(b, Best{lane_xor<32>(b.v), lane_xor<32>(b.i)});
+    b = better(b, Best{lane_xor<16>(b.v), lane_xor<16>(b.i)});
+    b = better(b, Best{lane_xor<8>(b.v), lane_xor<8>(b.i)});
+    b = better(b, Best{lane_xor<4>(b.v), lane_xor<4>(b.i)});
+    b = better(b, Best{lane_xor<2>(b.v), lane_xor<2>(b.i)});
+    b = better(b, Best{lane_xor<1>(b.v), lane_xor<1>(b.i)});
     const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
     const int n_waves = (blockDim.x + WAVE - 1) / WAVE;
     __syncthreads();
