@@ -29,36 +29,64 @@ __device__ __forceinline__ uint4 zero_if(bool out, uint4 v) {
 // (checked against fmaf on normal, widely spread and subnormal values: the same bits everywhere), so both kernels
 // below run on the matrix cores, at twice the vector units' rate, and still sum every output in that order.
 //
-// Many rows: a 64x64 tile per block of four waves, 32x32 each, K in steps of 32 through LDS, the loads of
-// three further steps in flight while one is multiplied. Of 8 neighbouring k the even ones lie together in LDS and then the
-// odd ones: lane / 32 picks a half of each product's two k, so one 16-byte read feeds four products. Bound by
-// the matrix cores where there are enough tiles; a long K with few tiles is bound by the chain of a wave's
-// products, 32 cycles a k. Measured, 666 rows: 143 us by 9,216 by 1,024 (88 TFLOP/s), 103 us by 1,024 by 4,608; the
-// LFM2-350M shape's four products 88 us on average where a register-tiled kernel on the vector units took 281.
-#define F32_BM 64
-#define F32_BN 64
-#define F32_BK 32
-#define F32_LD 40   // floats from row to row in LDS: 32 bytes beyond a row's own, which keeps 16-byte reads free of conflicts
+// Many rows: a tile of 64x64 or 32x32 per block of four waves, a quarter each, K in steps of 32 or 64 through LDS; a thread
+// brings 8 neighbouring k of a row of each operand, the loads of four further steps in flight.
+// 64x64: a wave has 32x32 on the 32x32x2 product, 32 cycles a k. Of 8 neighbouring k the even ones lie together in LDS
+// and then the odd ones: lane / 32 picks a half of each product's two k, so one 16-byte read feeds four products.
+// 32x32: a wave has 16x16 on the 16x16x4 product, whose chain takes 8 cycles a k; k = 4p + lane / 16 of product p comes out
+// of LDS as it lies there, value by value (rows 68 floats apart: 64 lanes, 64 banks).
+// A step's operands go to LDS while the products of the step before run, and the barrier stands before its last four products, with
+// the next step's first operands asked for behind it, so that neither is waited for.
+// Bound by the matrix cores where there are enough tiles, and with few by the chain of a wave's products (64x64) or what a CU
+// brings in, 30 to 40 GB/s (32x32). Measured, 666 rows: 131 us by 9,216 by 1,024 (96 TFLOP/s; 140 when a step's writes, barrier and
+// reads stood between its products and the last step's), 89 by 1,024 by 4,608 (107); 64 rows by 1,024 by 4,608 41 (106).
+template <bool SMALL>
+struct F32Tile {
+    static constexpr int M = SMALL ? 32 : 64, K = SMALL ? 64 : 32;
+    static constexpr int LD = SMALL ? 68 : 40;      // (40: 32 bytes beyond a row's own keep 16-byte reads free of conflicts)
+    static constexpr int SUB = K / 4;               // k of four products
+    using Acc = typename std::conditional<SMALL, f32x4, f32x16>::type;
+};
+
+// lane: token m, weight rows n .. n + 3
+template <typename TOut>
+__device__ __forceinline__ void f32_rows_out(const f32x4& acc, const float* __restrict__ bias, TOut* __restrict__ Y, int m, int n, int M,
+                                             int N, const Epilogue& epilogue) {
+    if (m >= M) return;
+    float v[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = bias && n + i < N ? acc[i] + bias[n + i] : acc[i];
+    if (epilogue == EPI_SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < 4; i += 2)
+            if (n + i + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + (n + i) / 2, gated_mul(epilogue, v[i], v[i + 1]));
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (n + i < N) store_f32<TOut>(Y, (size_t)m * N + n + i, v[i]);
+}
 
 // VEC: K is at least 4, and rows are read in vectors of four floats that may start anywhere; the end of a K that is no
 // multiple of 4, and a shorter K, value by value. (666 rows by 9,216 by 1,024 that start 4 bytes off 16:
-// 140 us, 395 value by value.)
-template <typename TOut, bool VEC>
-__global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, const float* __restrict__ W,
+// 136 us, 395 value by value.)
+template <typename TOut, bool VEC, bool SMALL>
+__global__ __launch_bounds__(256, VEC ? 4 : 3) void k_gemm_f32(const float* __restrict__ X, const float* __restrict__ W,
                                                   const float* __restrict__ bias, TOut* __restrict__ Y,
                                                   int M, int N, int K, int tiles_m, int tiles_n, Epilogue epilogue) {
-    __shared__ __attribute__((aligned(16))) float xs[2][F32_BM * F32_LD];
-    __shared__ __attribute__((aligned(16))) float ws[2][F32_BN * F32_LD];
+    using T = F32Tile<SMALL>;
+    __shared__ __attribute__((aligned(16))) float xs[2][T::M * T::LD];
+    __shared__ __attribute__((aligned(16))) float ws[2][T::M * T::LD];
     // blocks that share weight rows are neighbours on one XCD (they go to the 8 XCDs in turn, each has an L2)
     const int total = tiles_m * tiles_n;
     const int per_xcd = (total + 7) / 8;
     const int block = blockIdx.y * gridDim.x + blockIdx.x;   // (a row of the grid is a multiple of 8)
     const int logical = (block % 8) * per_xcd + block / 8;
     if (block / 8 >= per_xcd || logical >= total) return;
-    const int m0 = (logical % tiles_m) * F32_BM, n0 = (logical / tiles_m) * F32_BN;
+    const int m0 = (logical % tiles_m) * T::M, n0 = (logical / tiles_m) * T::M;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    const int row = tid >> 2, part = (tid & 3) * 8;          // a thread brings 8 neighbouring k of one row of each operand
+    const int wm = (wave >> 1) * (T::M / 2), wn = (wave & 1) * (T::M / 2);
+    const int row = tid / (T::K / 8), part = tid % (T::K / 8) * 8;
     const float* xrow = X + (size_t)min(m0 + row, M - 1) * K;
     const float* wrow = W + (size_t)min(n0 + row, N - 1) * K;
     struct Ahead {
@@ -82,82 +110,130 @@ __global__ __launch_bounds__(256) void k_gemm_f32(const float* __restrict__ X, c
             fetch_values(k0, f);
         }
     };
-    f32x16 acc;
+    const int at = row * T::LD + part;
+    auto put_row = [&](int k0, float* to, const float (&f)[8]) __attribute__((always_inline)) {
+        float v[8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    const int put = row * F32_LD + part;
-    const int get_x = (wm + (lane & 31)) * F32_LD + (lane >> 5) * 4, get_w = (wn + (lane & 31)) * F32_LD + (lane >> 5) * 4;
-    // One step: its operands leave the registers for LDS, the fourth step from here is asked for in their place
-    // (a step takes half a microsecond, a trip to memory one or two), and the products run.
-    auto step = [&](int k0, int buf, Ahead& now, const bool more) __attribute__((always_inline)) {
-        float x[8], w[8];
+        for (int j = 0; j < 8; ++j)                      // (the choice also where it always holds: without it the compiler
+            v[SMALL ? j : (j & 1) * 4 + j / 2] = k0 + part + j < K ? f[j] : 0.f;   // sorts what comes as it comes, and waits there)
+        *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4*>(to + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    };
+    auto put = [&](int k0, int buf, const Ahead& f) __attribute__((always_inline)) {
+        put_row(k0, &xs[buf][at], f.x);
+        __builtin_amdgcn_sched_barrier(0);               // (one after the other: registers)
+        put_row(k0, &ws[buf][at], f.w);
+    };
+    struct Operands {
+        float x[4], w[4];
+    };
+    const int get_x = SMALL ? (wm + (lane & 15)) * T::LD + (lane >> 4) : (wm + (lane & 31)) * T::LD + (lane >> 5) * 4;
+    const int get_w = SMALL ? (wn + (lane & 15)) * T::LD + (lane >> 4) : (wn + (lane & 31)) * T::LD + (lane >> 5) * 4;
+    auto get = [&](int buf, int sub, Operands& o) __attribute__((always_inline)) {
+        if (SMALL) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const bool in = k0 + part + j < K;           // (also where it always holds: without a choice here the compiler
-                                                         // sorts what comes as it comes, and waits for it there)
-            x[j] = in ? now.x[j] : 0.f;
-            w[j] = in ? now.w[j] : 0.f;
+            for (int i = 0; i < 4; ++i) {
+                o.x[i] = xs[buf][get_x + sub * T::SUB + i * 4];
+                o.w[i] = ws[buf][get_w + sub * T::SUB + i * 4];
+            }
+        } else {
+            const float4 a = *reinterpret_cast<const float4*>(&xs[buf][get_x + sub * T::SUB]);
+            const float4 b = *reinterpret_cast<const float4*>(&ws[buf][get_w + sub * T::SUB]);
+            o.x[0] = a.x, o.x[1] = a.y, o.x[2] = a.z, o.x[3] = a.w;
+            o.w[0] = b.x, o.w[1] = b.y, o.w[2] = b.z, o.w[3] = b.w;
         }
-        *reinterpret_cast<float4*>(&xs[buf][put]) = make_float4(x[0], x[2], x[4], x[6]);
-        *reinterpret_cast<float4*>(&xs[buf][put + 4]) = make_float4(x[1], x[3], x[5], x[7]);
-        *reinterpret_cast<float4*>(&ws[buf][put]) = make_float4(w[0], w[2], w[4], w[6]);
-        *reinterpret_cast<float4*>(&ws[buf][put + 4]) = make_float4(w[1], w[3], w[5], w[7]);
-        // (the other buffer was read before the barrier of the step before; the loads in flight are not waited for)
+    };
+    typename T::Acc acc = {};
+    auto multiply = [&](const Operands& o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (SMALL)
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[i], o.x[i], acc, 0, 0, 0);
+            else
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(o.x[i], o.w[i], acc, 0, 0, 0);
+        }
+    };
+    Operands even, odd;
+    // One step, whose first operands are in `even`; `next` holds the step behind it, which goes to LDS here (if it is not
+    // the last), and is asked for the fourth step behind that one.
+    auto step = [&](int k0, int buf, Ahead& next, const bool more, const bool puts) __attribute__((always_inline)) {
+        get(buf, 1, odd);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(even);
+        if (puts) put(k0 + T::K, buf ^ 1, next);
+        if (more) fetch(k0 + 5 * T::K, next);
+        __builtin_amdgcn_sched_barrier(0);   // (left alone, the compiler sinks these loads to where they are used)
+        get(buf, 2, even);
+        multiply(odd);
+        __builtin_amdgcn_sched_barrier(0);
+        get(buf, 3, odd);
+        multiply(even);
+        // (nobody reads the other buffer any more, nobody will read this one; the loads in flight are not waited for)
+        __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
-        if (more) fetch(k0 + 4 * F32_BK, now);
-        __builtin_amdgcn_sched_barrier(0);   // (left alone, the compiler sinks these loads to where they are used)
-#pragma unroll
-        for (int kb = 0; kb < F32_BK; kb += 8) {
-            const float4 a = *reinterpret_cast<const float4*>(&xs[buf][get_x + kb]);
-            const float4 b = *reinterpret_cast<const float4*>(&ws[buf][get_w + kb]);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc, 0, 0, 0);
-        }
+        asm volatile("" ::: "memory");
+        get(buf ^ 1, 0, even);               // (behind the last step: for nothing)
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(odd);
         __builtin_amdgcn_sched_barrier(0);
     };
+    const int steps = (K + T::K - 1) / T::K;
     Ahead s0, s1, s2, s3;
     // (in the order they are used: a first use whose loads were issued last would wait for all of them, every round)
     fetch(0, s0);
     __builtin_amdgcn_sched_barrier(0);
-    fetch(F32_BK, s1);
+    fetch(T::K, s1);
     __builtin_amdgcn_sched_barrier(0);
-    fetch(2 * F32_BK, s2);
+    fetch(2 * T::K, s2);
     __builtin_amdgcn_sched_barrier(0);
-    fetch(3 * F32_BK, s3);
+    fetch(3 * T::K, s3);
     __builtin_amdgcn_sched_barrier(0);
-    const int turns = K / (4 * F32_BK) * (4 * F32_BK);
-    for (int k0 = 0; k0 < turns; k0 += 4 * F32_BK) {
-        step(k0, 0, s0, true);
-        step(k0 + F32_BK, 1, s1, true);
-        step(k0 + 2 * F32_BK, 0, s2, true);
-        step(k0 + 3 * F32_BK, 1, s3, true);
+    if (VEC && K % 4 && steps == 1) fetch_values(0, s0);
+    put(0, 0, s0);
+    fetch(4 * T::K, s0);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    get(0, 0, even);
+    // turns of four steps that two steps at least come behind, so that the last step, which may end inside a vector, is none that
+    // a turn puts into LDS
+    const int turns = steps < 2 ? 0 : (steps - 2) / 4 * 4 * T::K;
+    for (int k0 = 0; k0 < turns; k0 += 4 * T::K) {
+        step(k0, 0, s1, true, true);
+        step(k0 + T::K, 1, s2, true, true);
+        step(k0 + 2 * T::K, 0, s3, true, true);
+        step(k0 + 3 * T::K, 1, s0, true, true);
     }
-    // what is left of K, up to four steps, the last one filled up with zeros (a short K is nothing else: 4,096 rows by 1,024
+    // what is left of K, up to five steps, the last one filled up with zeros (a short K is nothing else: 4,096 rows by 1,024
     // by 8 9.3 us where steps to the end of the turn took 18 and steps of 16 on the vector units 11)
-    auto rest = [&](int k0, int buf, Ahead& f) __attribute__((always_inline)) {
+    auto rest = [&](int k0, int buf, Ahead& next) __attribute__((always_inline)) {
         if (k0 >= K) return;
-        if (VEC && K % 4 && k0 + F32_BK > K) fetch_values(k0, f);
-        step(k0, buf, f, false);
+        if (VEC && K % 4 && k0 + T::K < K && k0 + 2 * T::K > K) fetch_values(k0 + T::K, next);
+        step(k0, buf, next, false, k0 + T::K < K);
     };
-    rest(turns, 0, s0);
-    rest(turns + F32_BK, 1, s1);
-    rest(turns + 2 * F32_BK, 0, s2);
-    rest(turns + 3 * F32_BK, 1, s3);
-    // a lane holds one column (a weight row) of 16 activation rows
-    const int n = n0 + wn + (lane & 31);
-    const float bn = bias && n < N ? bias[n] : 0.f;
+    rest(turns, 0, s1);
+    rest(turns + T::K, 1, s2);
+    rest(turns + 2 * T::K, 0, s3);
+    rest(turns + 3 * T::K, 1, s0);
+    rest(turns + 4 * T::K, 0, s1);
+    if constexpr (SMALL) {
+        f32_rows_out<TOut>(acc, bias, Y, m0 + wm + (lane & 15), n0 + wn + (lane >> 4) * 4, M, N, epilogue);
+    } else {
+        // a lane holds one column (a weight row) of 16 activation rows
+        const int n = n0 + wn + (lane & 31);
+        const float bn = bias && n < N ? bias[n] : 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        const float v = bias ? acc[r] + bn : acc[r];
-        if (epilogue == EPI_SWIGLU) {
-            const float up = lane_xor<1>(v);             // gate and up rows are neighbours
-            if (m < M && !(lane & 1) && n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, v, up));
-        } else if (m < M && n < N) {
-            store_f32<TOut>(Y, (size_t)m * N + n, v);
+        for (int r = 0; r < 16; ++r) {
+            const int m = m0 + wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
+            const float v = bias ? acc[r] + bn : acc[r];
+            if (epilogue == EPI_SWIGLU) {
+                const float up = lane_xor<1>(v);             // gate and up rows are neighbours
+                if (m < M && !(lane & 1) && n + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + n / 2, gated_mul(epilogue, v, up));
+            } else if (m < M && n < N) {
+                store_f32<TOut>(Y, (size_t)m * N + n, v);
+            }
         }
     }
 }
@@ -195,25 +271,6 @@ __device__ __forceinline__ void transpose_over_groups(const f32x4& from, float (
     swap_lanes_32(v[1], v[3]);
     swap_lanes_16(v[0], v[1]);
     swap_lanes_16(v[2], v[3]);
-}
-
-// lane: token m, weight rows n .. n + 3
-template <typename TOut>
-__device__ __forceinline__ void f32_rows_out(const f32x4& acc, const float* __restrict__ bias, TOut* __restrict__ Y, int m, int n, int M,
-                                             int N, const Epilogue& epilogue) {
-    if (m >= M) return;
-    float v[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = bias && n + i < N ? acc[i] + bias[n + i] : acc[i];
-    if (epilogue == EPI_SWIGLU) {
-#pragma unroll
-        for (int i = 0; i < 4; i += 2)
-            if (n + i + 1 < N) store_f32<TOut>(Y, (size_t)m * (N / 2) + (n + i) / 2, gated_mul(epilogue, v[i], v[i + 1]));
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-        if (n + i < N) store_f32<TOut>(Y, (size_t)m * N + n + i, v[i]);
 }
 
 template <typename TOut>
@@ -404,17 +461,28 @@ static int launch_f32(const float* x, const float* w, const float* bias, TOut* y
         k_gemm_f32_rows<TOut><<<(unsigned)((n + 15) / 16), 64, 0, s>>>(x, w, bias, y, m, n, k, epilogue);
         return launch_status();
     }
-    if (m > 65535 * F32_BM) return IMPARO_BAD_ARGUMENT;
-    const int tiles_m = (m + F32_BM - 1) / F32_BM, tiles_n = (n - 1) / F32_BN + 1;
+    if (m > 65535 * F32Tile<false>::M) return IMPARO_BAD_ARGUMENT;
+    auto tiles = [](int rows, bool small) { return (rows - 1) / (small ? F32Tile<true>::M : F32Tile<false>::M) + 1; };
+    // The smaller tile where it loads the CUs so much more evenly that its twice the operands a product cost less: what a launch takes
+    // goes by the blocks of its fullest CU. 2,048 rows of weight by 8,192, us by blocks a CU: 64x64 one 162, two 284, three 424; 32x32 one
+    // 70, two 110, three 154, four 197, six 292. (So 16 to 128 rows by 2,048 by 1,024 24.4 -> 12.3 us, 666 by 1,024 by 4,608 95 -> 89.)
+    auto a_cu = [&](bool small) { return ((long long)tiles(m, small) * tiles(n, small) + 255) / 256; };
+    // (With three blocks a CU it takes a longer K and rows on 16 bytes: 666 rows by 1,024 by 8 6.0 us and 4.7, by 300 11.3 and 11.7, 64
+    // rows by 9,216 by 1,024 off 16 30.1 and 28.6.)
+    const bool at_16 = k % 4 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15);
+    const bool small = k >= 4 && 5 * a_cu(true) + 3 < 14 * a_cu(false) + 5 && (a_cu(true) <= 2 || (k >= 256 && at_16));
+    const int tiles_m = tiles(m, small), tiles_n = tiles(n, small);
     const long long total = (long long)tiles_m * tiles_n;
     if (total > 0x7f000000LL) return IMPARO_BAD_ARGUMENT;
     // (a launch holds fewer than 2^32 threads along x)
     const long long row = std::min<long long>((total + 7) / 8 * 8, 1LL << 23);
     const dim3 blocks((unsigned)row, (unsigned)((total + row - 1) / row));
-    if (k >= 4)
-        k_gemm_f32<TOut, true><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
+    if (small)
+        k_gemm_f32<TOut, true, true><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
+    else if (k >= 4)
+        k_gemm_f32<TOut, true, false><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
     else
-        k_gemm_f32<TOut, false><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
+        k_gemm_f32<TOut, false, false><<<blocks, 256, 0, s>>>(x, w, bias, y, m, n, k, tiles_m, tiles_n, epilogue);
     return launch_status();
 }
 
