@@ -55,10 +55,10 @@ class PreNormBlock:
             h = self.shift.forward(ctx, site, self.mixer_norm.forward(ctx, res, torch.float32, name="normed_f32"),
                                    self.mixer.in_dtype)
         behind = ctx.next_norm if self.ffn is None else (self.ffn_norm, self.ffn.in_dtype)
-        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h), behind)
+        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h), self.mixer, behind)
         if self.ffn is not None:
             n = self.ffn_norm.forward(ctx, res, self.ffn.in_dtype)
-            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n), ctx.next_norm)
+            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n), self.ffn, ctx.next_norm)
 
     def first_norm(self):
         """The norm that reads the stream first and the dtype its rows are asked for in, if it may ride with the product before
@@ -79,13 +79,15 @@ class PreNormBlock:
         self.ffn.emit(program)
 
     @staticmethod
-    def _delta(ctx: StepContext, res: Residual, run, behind=None):
+    def _delta(ctx: StepContext, res: Residual, run, part=None, behind=None):
         """Runs a part whose result goes into the stream. With nothing pending the part may add its
         result to the stream itself (it then returns the stream); otherwise it returns a delta.
         `behind`: the norm that reads the stream next and the dtype of its rows; a norm that can rides with
-        the part's last product."""
+        the last product of a `part` that says `adds_last`. Both have to say so of the `forward` they run: a part that
+        goes on adding to the stream, or a norm that does more, would leave rows of a stream that is not the one read."""
         ctx.stream = res.x if res.pending is None else None
-        ctx.ride = NormRide(*behind) if ctx.stream is not None and behind and hasattr(behind[0], "ride") else None
+        rides = ctx.stream is not None and behind and emits(behind[0], "ride") and emits(part, "adds_last")
+        ctx.ride = NormRide(*behind) if rides else None
         ride = ctx.ride
         try:
             delta = run()

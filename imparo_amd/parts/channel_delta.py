@@ -43,6 +43,7 @@ _DEFAULT_NAMES = dict(q="q", k="k", v="v", q_conv="q.conv", k_conv="k.conv", v_c
 class ChannelDelta:
     role = "mixer"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:

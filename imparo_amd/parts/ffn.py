@@ -26,6 +26,7 @@ _DEFAULT_NAMES = dict(gate="gate_proj", up="up_proj", down="down_proj")
 class SwiGlu:
     role = "feed_forward"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
     limit, alpha = 0.0, 1.0          # (no bounds: SiLU)
 
     @staticmethod
@@ -95,6 +96,7 @@ class SwiGlu:
 class PolyNormFfn:
     role = "feed_forward"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:

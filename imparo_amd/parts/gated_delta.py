@@ -41,6 +41,7 @@ UNIT_EPS = 1e-6          # inside the root that makes q and k unit vectors
 class GatedDelta:
     role = "mixer"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:

@@ -38,6 +38,7 @@ _DEFAULT_NAMES = {"in": "in", "conv": "conv", "conv_bias": "conv.b", "dt_bias": 
 class Mamba2:
     role = "mixer"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:

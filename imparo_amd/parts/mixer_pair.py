@@ -29,7 +29,7 @@ from ..cache.pages import FixedArray, FixedSpec, PagedSpec, fixed_part
 from ..config.plan import PartSpec
 from ..kernels import ops
 from ..weights.loader import TensorDecl
-from .base import Declared, NormRide, StepContext
+from .base import Declared, NormRide, StepContext, emits
 from .linear import place_vector
 from .registry import part_class, register_part
 
@@ -74,6 +74,7 @@ class _Scoped:
 
 class MixerPair:
     role = "mixer"
+    adds_last = True      # (where its right side says so; see `forward`)
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:
@@ -130,9 +131,10 @@ class MixerPair:
         if not self.normed:
             stream = ctx.stream
             ride = ctx.ride
-            first = None if ride is None else NormRide(None, ride.out_dtype)      # (the norm behind both rides with the second)
+            # (the norm behind both rides with the second)
+            first = NormRide(None, ride.out_dtype) if ride is not None and emits(self.left, "adds_last") else None
             a = self.left.forward(_Scoped(ctx, "left.", "left:", stream, first), site, owns_cache, h)
-            ride = ride if stream is not None and a is stream else None
+            ride = ride if stream is not None and a is stream and emits(self.right, "adds_last") else None
             b = self.right.forward(_Scoped(ctx, "right.", stream=stream, ride=ride), site, owns_cache, h)
             deltas = tuple(d for d in (a, b) if stream is None or d is not stream)
             return stream if not deltas else deltas[0] if len(deltas) == 1 else deltas

@@ -40,6 +40,7 @@ _DEFAULT_NAMES = dict(q="q", k="k", v="v", g="g", o="o")
 class Retention:
     role = "mixer"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:

@@ -25,6 +25,7 @@ from .registry import register_part
 class ShortConv:
     role = "mixer"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    adds_last = True      # the last thing `forward` launches is the product into ctx.stream: a norm may ride with it
 
     @staticmethod
     def declare(spec: PartSpec) -> Declared:
