@@ -132,17 +132,19 @@ class Model:
         return program
 
     def weight_bytes(self) -> int:
-        seen, total = set(), 0
+        """Bytes of device memory that the model's tensors take; what several of them view is counted once."""
+        spans = set()
         def walk(obj):
-            nonlocal total
             for v in vars(obj).values():
                 if isinstance(v, torch.Tensor):
-                    if v.data_ptr() not in seen:
-                        seen.add(v.data_ptr())
-                        total += v.numel() * v.element_size()
+                    spans.add((v.data_ptr(), v.data_ptr() + v.numel() * v.element_size()))
                 elif hasattr(v, "__dict__") and not isinstance(v, type):
                     walk(v)
         walk(self.embedding); walk(self.final_norm); walk(self.head)
         for b in self.blocks:
             walk(b)
+        total, counted = 0, 0                    # (addresses up to `counted` are in the total)
+        for start, end in sorted(spans):
+            total += max(0, end - max(start, counted))
+            counted = max(counted, end)
         return total
