@@ -14,11 +14,23 @@ import torch
 from ..kernels import ops
 from .base import StepContext
 
-# Up to this inner size and this many activations a product of at most 16 rows that sums the whole of K in a block and takes a norm
-# without a statistic along beats slices of K and a launch for the norm (in a graph, cold weights): 4 rows of 1,024 weight rows
-# over 1,024 3.8 us against 5.8, over 3,072 5.5 against 6.4, 8 rows 5.8 and 6.4, but 16 rows 7.0 and 6.7: every block reads all of them.
+# Most of K where a product of at most 16 rows that sums the whole of K in a block and takes a norm without a statistic along beats
+# slices of K and a launch for the norm, by how many blocks of eight weight rows the fullest CU has (one up to 2,048 weight rows, where
+# up to 1,024 a block has four; every block reads all activations, so that the price goes by the blocks and by K). By the weight and K
+# alone: a row's sums then come in one order in all steps of 1 to 16 rows. Measured in a graph, cold weights, us for 1 / 4 / 8 / 16 rows
+# with the norm's launch counted in, riding and not: 1,024 weight rows over 1,024 3.7 3.9 4.0 4.3 and 5.6 5.8 5.9 6.0, over 3,072 5.4 5.8 6.2
+# 7.1 and 6.4 6.6 6.7 6.9, over 3,584 16 rows 7.6 and 7.2; 2,048 over 4,096 7.5 7.7 8.2 9.4 and 8.6 8.8 9.1 9.4; 3,072 over 2,048 7.0 7.4 8.1 9.2
+# and 8.5 8.6 8.8 9.3, over 3,072 16 rows 12.9 and 11.2; 5,120 over 1,024 6.1 6.4 6.9 8.1 and 7.8 8.1 8.1 8.5, over 2,048 16 rows 12.8 and
+# 11.1; 8,192 over 512 6.9 and 7.5, over 1,024 10.3 and 9.0; 16,384 over 512 11.7 and 9.3.
 RIDE_MAX_K = 4096
-RIDE_MAX_ACTIVATIONS = 36864
+_RIDE_MOST_K = (4096, 2048, 1024, 512)
+
+
+def _rides(weight_rows: int, k: int) -> bool:
+    a_cu = -(-weight_rows // 2048)
+    if a_cu > len(_RIDE_MOST_K):
+        return False
+    return k <= min(RIDE_MAX_K, 3072 if weight_rows <= 1024 else _RIDE_MOST_K[a_cu - 1])
 
 
 class Linear:
@@ -48,8 +60,7 @@ class Linear:
         width = self.out_features // 2 if swiglu else self.out_features
         m = x.shape[0]
         ride = ctx.ride if into is not None else None
-        if (ride is not None and not swiglu and m <= ops.ROWS_MAX and self.in_features <= RIDE_MAX_K
-                and m * self.in_features <= RIDE_MAX_ACTIVATIONS and x.dtype == torch.bfloat16
+        if (ride is not None and not swiglu and m <= ops.ROWS_MAX and _rides(self.out_features, self.in_features) and x.dtype == torch.bfloat16
                 and self.weight.dtype == torch.bfloat16 and self.in_features % 8 == 0 and ride.out_dtype == torch.bfloat16
                 and into.dtype == torch.float32 and tuple(into.shape) == (m, width) and into.is_contiguous()):
             # a few rows: the product adds to the stream and takes the norm behind it along

@@ -50,6 +50,31 @@ def test_product_with_the_norm_behind_it(n, k, m, biased):
         ops.rows_gemm_tanh(x, w, alone[:, :n - 1].contiguous())
 
 
+# weights that ride and that do not, at the lines between them
+@pytest.mark.parametrize("n, k, rides", [(1024, 3072, True), (1024, 3080, False), (1032, 4096, True), (2048, 4104, False), (2056, 2048, True),
+                                         (2056, 2056, False), (4104, 1024, True), (4104, 1032, False), (6152, 512, True), (8200, 256, False)])
+def test_a_row_is_summed_in_one_order_in_all_steps_of_few_rows(n, k, rides):
+    """A request's stream and rows do not depend on how many others decode beside it."""
+    import types
+    from imparo_amd.parts.base import NormRide, Residual, Workspace
+    from imparo_amd.parts.linear import Linear
+    from imparo_amd.parts.norm import DynamicTanh
+    x, held = rnd(16, k, seed=1).bfloat16().to(DEV), rnd(16, n, seed=2).to(DEV)
+    linear = Linear(rnd(n, k, seed=3, scale=k ** -0.5).bfloat16().to(DEV))
+    norm = DynamicTanh.__new__(DynamicTanh)
+    norm.alpha, norm.weight, norm.bias = 0.7, rnd(n, seed=4).to(DEV), rnd(n, seed=5).to(DEV)
+    first = None
+    for m in (16, 1, 2, 4, 8, 9, 12, 13, 15):
+        res = Residual(held[:m].clone())
+        ctx = types.SimpleNamespace(workspace=Workspace(torch.device(DEV)), stream=res.x, ride=NormRide(norm, torch.bfloat16))
+        delta = linear(ctx, x[:m], torch.float32, "out", sliced_ok=True, into=res.x)
+        assert (ctx.ride.rows is not None) == rides and (delta is res.x) == rides
+        res.pending, res.normed = (None, ctx.ride) if rides else (delta, None)
+        rows = norm.forward(ctx, res, torch.bfloat16)
+        first = first if first is not None else (res.x.clone(), rows.clone())
+        assert torch.equal(res.x, first[0][:m]) and torch.equal(rows, first[1][:m])
+
+
 def test_a_models_steps_with_and_without(tmp_path, monkeypatch):
     """Prompts and decoded tokens of a model whose layers' norms ride (delta rule, and attention beside lightning attention)."""
     from imparo_amd import Engine, StepEntry, write_random_model
