@@ -60,10 +60,9 @@ union RowFrag {
 #define ROWS_SWIGLU 1
 #define ROWS_RESID 2
 #define ROWS_TANH 3          // into the stream, and the rows behind a norm without a statistic
+#define ROWS_CONV 4          // the first columns through a causal conv a channel and SiLU
 #define ROWS_WAVES 8         // of a block at most
 #define ROWS_TURNED 8192     // from this K on blocks start their walks at different places
-
-#define ROWS_CONV 4          // the first columns through a causal conv a channel and SiLU
 
 // ROWS_CONV: columns 0 .. channels - 1 are channels of a causal conv (at most ROWS_TAPS taps, the last one the current row's) whose
 // last inputs a request keeps: hist [slots, taps - 1, channels], row r in slot[r], shifted in place by the lane that owns the channel.
@@ -346,7 +345,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) void k_rows_gemm(
                 }
             }
             if (EPI == ROWS_TANH) continue;
-            sq += lane_xor<16>(sq);             // the two lanes of a token sit 16 apart
+            sq += __shfl_xor(sq, 16, WAVE);             // the two lanes of a token sit 16 apart
             if (g == 0) ssq_out[(size_t)blockIdx.x * ROWS_PARTS + r16] = sq;
         }
     }

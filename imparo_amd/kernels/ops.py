@@ -726,7 +726,7 @@ def rows_gemm_tanh(x: torch.Tensor, w: torch.Tensor, into: torch.Tensor, bias: O
     bfloat16 receives tanh(alpha * row) * norm_weight + norm_bias of the new rows."""
     m, k = x.shape
     n, kw = w.shape
-    if kw != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not 0 < m <= 16 or k % 8:
+    if kw != k or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not 0 < m <= ROWS_MAX or k % 8:
         raise KernelArgumentError("rows_gemm_tanh: 1 to 16 bfloat16 rows, a bfloat16 weight over the same inner size, "
                                   "a multiple of 8")
     if len({t is None for t in (out, norm_weight, norm_bias)}) > 1:
