@@ -289,7 +289,12 @@ __global__ __launch_bounds__(LAT_WAVES * WAVE, QT == 1 ? 2 : 1) void k_latent_at
                     sv[j] = (key >= k_lo && key <= k_hi) ? s[u][j >> 2][j & 3] * scale : -INFINITY;
                     tile_max = fmaxf(tile_max, sv[j]);
                 }
-                tile_max = max_16_32(tile_max);
+                if constexpr (NK + NV > 25 && QT == 1) {       // (with lane swaps the largest form holds six registers too many: 64 rows over
+                    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16, WAVE));        // 2,000 keys of 320 and 256 46.8 us, 43.1 so)
+                    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32, WAVE));
+                } else {
+                    tile_max = max_16_32(tile_max);
+                }
                 const float m_new = fmaxf(m[u], tile_max);  // finite: every tile holds a key of the range
                 const float corr = __expf(m[u] - m_new);
                 float p[8], p_sum = 0.f;
