@@ -936,9 +936,12 @@ __global__ __launch_bounds__(MFMA_WAVES * 64) void k_attn_prefill(
 // EXACT: what the rounding to bfloat16 takes off a weight goes through second products (part of the kernel's type: branches on
 // it inside a tile kept the scheduler from mixing one weight's instructions with the next one's).
 // (three waves a SIMD with heads of up to 64: with one register more than that leaves, 8,192 exact queries over 16,384 keys took 1,614
-// us and not 1,415; 1,497 before)
+// us and not 1,415; 1,497 before. Three also where it costs spills, three to eight registers with 32 queries a wave and small pages or
+// rules: 8,192 exact queries of 16 heads on pages of 32 373 us, in two waves that spill nothing 398; 4,096 capped ones with sinks over
+// 16,384 keys 1,239 and 1,371. Four with heads of 32, rules and small pages, which would take 130 registers and lose the fourth: 8,192
+// queries 330 us, in three 428)
 template <int ND, int HALVES, bool PAGE_TILE, bool EXT, bool EXACT>
-__global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 4 ? 3 : 1) void k_attn_prefill_x32(
+__global__ __launch_bounds__(MFMA_WAVES * 64, ND <= 2 && EXT && !PAGE_TILE ? 4 : ND <= 4 ? 3 : 1) void k_attn_prefill_x32(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     bf16_t* __restrict__ out, const int32_t* __restrict__ rows, int n_rows,
     const int32_t* __restrict__ seg_start, const int32_t* __restrict__ seg_len, const int32_t* __restrict__ positions,
