@@ -1038,7 +1038,11 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
     // waited and read back in turn. Measured with the last steps' loads left out, us before and now: 8,192 rows of 6,144 by 2,048
     // 201 and 178, gate and up of 16,384 by 2,048 469 and 458; 2,048 rows 57.4 and 51.0, 124 and 121, of 2,048 by 2,048 added
     // 27.5 and 24.0, by 8,192 76.4 and 74.9; 520 rows of 6,144 by 2,048 24.0 and 21.4, of 2,048 by 2,048 in two slices 13.3 and 10.9.
+    // Of a tile that is cut, every product that lies whole inside goes the same way, and only those on the edge value by value: all
+    // value by value 198 rows of 220 by 256 added took 15.0 us, now 5.9, 5,292 of 6,656 by 768 added 167 and 81, 1,881 of 512 by 256
+    // 7.7 and 5.0.
     const int l32 = lane & 31, m_lane = m0 + wm * WM + 4 * (lane >> 5), n_lane = n0 + wn * WN + l32;
+    const int m_wave = __builtin_amdgcn_readfirstlane(m0 + wm * WM), n_wave = __builtin_amdgcn_readfirstlane(n0 + wn * WN);
     const bool swiglu = epilogue == EPI_SWIGLU;
     const bool adds = epilogue == EPI_ADD;             // (float32 out; the launcher sees to it)
     const bool inside = m0 + BM <= M && n0 + BN <= N;
@@ -1046,12 +1050,14 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
     float bn[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j) bn[j] = bias && n_lane + j * 32 < N ? bias[n_lane + j * 32] : 0.f;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(bn[j]));     // waited for here: a store under a condition would wait for it, and for the store before
     if (swiglu) {
         // Gates and ups are neighbouring lanes: of two rows the even lane takes the first one's pair and the odd lane the
         // second's. In bfloat16 two such results of neighbouring columns go on to one lane, of two rows and the next two again.
         const int out_n = N / 2;
         const bool odd = lane & 1, upper = lane & 2;
-        const bool pairs = !FLOAT && inside && out_n % 2 == 0 && ((uintptr_t)Y & 3) == 0;
+        const bool fits = !FLOAT && out_n % 2 == 0 && ((uintptr_t)Y & 3) == 0;
         auto gated = [&](const f32x16& a, float b, int r) __attribute__((always_inline)) {       // row r + odd, column l32 / 2
             const float first = a[r] + b, second = a[r + 1] + b;
             const float other = lane_xor<1>(odd ? first : second);
@@ -1062,6 +1068,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 const int col = (n0 + wn * WN + j * 32) / 2;
+                const bool pairs = fits && (inside || (m_wave + i * 32 + 32 <= M && n_wave + j * 32 + 32 <= N));
 #pragma unroll
                 for (int r = 0; r < 16; r += 4) {
                     const float lo = gated(acc[i][j], bn[j], r), hi = gated(acc[i][j], bn[j], r + 2);
@@ -1098,25 +1105,50 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
                         const float v = acc[i][j][r] + bn[j];
                         dst[(size_t)((r >> 2) * 8 + (r & 3)) * N + j * 32] = adds ? held[j][r] + v : v;
                     }
-            } else {
+                continue;
+            }
 #pragma unroll
-                for (int r = 0; r < 16; ++r)
+            for (int j = 0; j < TN; ++j) {
+                const int m_first = m_wave + i * 32, n_first = n_wave + j * 32;
+                if (m_first >= M || n_first >= N) continue;
+                float held[16];
+                if (m_first + 32 <= M && n_first + 32 <= N) {
+                    if (adds) {
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        const int row = (r >> 2) * 8 + (r & 3);
-                        if (m_lane + i * 32 + row >= M || n_lane + j * 32 >= N) continue;
-                        float* at = dst + (size_t)row * N + j * 32;
-                        const float v = acc[i][j][r] + bn[j];
-                        *at = adds ? *at + v : v;
+                        for (int r = 0; r < 16; ++r) held[r] = dst[(size_t)((r >> 2) * 8 + (r & 3)) * N + j * 32];
                     }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const float v = acc[i][j][r] + bn[j];
+                        dst[(size_t)((r >> 2) * 8 + (r & 3)) * N + j * 32] = adds ? held[r] + v : v;
+                    }
+                    continue;
+                }
+                const int left = n_lane + j * 32 < N ? M - (m_lane + i * 32) : 0;      // rows of this lane's column, four of every eight
+                if (adds) {                            // (a row outside asks for the first activations: no load under a branch)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = (r >> 2) * 8 + (r & 3);
+                        held[r] = *(row < left ? dst + (size_t)row * N + j * 32 : reinterpret_cast<const float*>(X));
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) asm volatile("" : "+v"(held[r]));     // (waited for together, as the bias)
+                }
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = (r >> 2) * 8 + (r & 3);
+                    const float v = acc[i][j][r] + bn[j];
+                    if (row < left) dst[(size_t)row * N + j * 32] = adds ? held[r] + v : v;
+                }
             }
         }
     } else {
-        const bool odd = lane & 1, pairs = inside && N % 2 == 0 && ((uintptr_t)Y & 3) == 0;
+        const bool odd = lane & 1, fits = N % 2 == 0 && ((uintptr_t)Y & 3) == 0;
 #pragma unroll
         for (int i = 0; i < TMI; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
+            for (int j = 0; j < TN; ++j) {
+                const bool pairs = fits && (inside || (m_wave + i * 32 + 32 <= M && n_wave + j * 32 + 32 <= N));
 #pragma unroll
                 for (int r = 0; r < 16; r += 2) {
                     const float first = acc[i][j][r] + bn[j], second = acc[i][j][r + 1] + bn[j];
@@ -1130,6 +1162,7 @@ __global__ __launch_bounds__(64 * NWM * NWN) void k_gemm_bf16_dma(const bf16_t* 
                         if (m + 1 < M) store_f32<TOut>(Y, (size_t)(m + 1) * N + n, second);
                     }
                 }
+            }
     }
 }
 
