@@ -643,12 +643,16 @@ __global__ __launch_bounds__(256, 2) void k_gemm_bf16_tile(const bf16_t* __restr
         if (kt + 1 < nk) step(kt + 1, a2, b2);
     }
     // D layout of the 32x32 tile: lane holds column lane%32, rows 8*(r/4) + 4*(lane/32) + r%4
+    float bns[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) bns[j] = bias && n0 + wn * 64 + j * 32 + (lane & 31) < N ? bias[n0 + wn * 64 + j * 32 + (lane & 31)] : 0.f;
+    asm volatile("" : "+v"(bns[0]), "+v"(bns[1]));     // waited for here: a store under a condition would wait for it, and for the store before
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-            const float bn = (bias && n < N) ? bias[n] : 0.f;
+            const float bn = bns[j];
             if (epilogue == EPI_SWIGLU) {
                 // gate and up of one output sit in neighbouring lanes (n even, n odd)
 #pragma unroll
