@@ -1191,13 +1191,14 @@ static bool dma_tile_takes(int m, int n, int k) {
 //   - with one or two tiles down the rows (a decode batch of 65 to 256 rows) every block meets its
 //     weights first, and cold: a step then takes 0.55 us at least on two stages and 0.36 on four;
 //   - a block's beginning and end take 4.3 us + 0.116 us per MFMA of a SIMD in a K-step
-//     (bm * bn / 1024 of them);
+//     (bm * bn / 1024 of them; measured when tiles left through LDS, and kept: the figures for the tiles are fitted beside it);
 //   - blocks run in rounds of what fits the chip at once; the operands have to come from memory
 //     once (5.5 TB/s) and the results have to go there (7.6 TB/s); a slice beyond the first costs
 //     its consumer one more pass over rows x width of float32 (5 TB/s).
-// `fixed_slices` > 0: the caller has decided. Then the tile is chosen by what the kernel takes now (18 numbers of rows from 136
-// to 8,192, 18 weights, every tile measured: 0.6 % above the fastest on average, where the figures of before were 5 %; one
-// product in 471 more than 3 % slower than the tile they chose). Else the slices are, by the figures they were always
+// `fixed_slices` > 0: the caller has decided. Then the tile is chosen by what the kernel takes now (240 products of 129 to 6,000 rows,
+// two thirds of them over K of 4,224 to 12,800, every tile measured: 0.14 % above the fastest on average and 8 % at most; with
+// figures fitted up to K of 4,608 the long ones were 2.8 % above it and 22 % at most, as two 128x128 tiles a CU were held to be
+// slower than they are: 641 rows of 8,192 by 9,088 166 us on 128x256, 135 on 128x128). Else the slices are, by the figures they were always
 // chosen with: a count once chosen stays, as fewer slices are further from 64 bits (151 rows of 69,516 by 3,584 in two 2.5e-7 and in one
 // 3.7e-7), and what a tile is does not change a sum.
 struct DmaPlan {
@@ -1212,8 +1213,8 @@ struct DmaRates {
 };
 static const DmaRates dma_rates_slices = {{1.03, 1.58}, {0.89, 1.30}, {0.66, 1.08}, {0.95, 1.25}, {0.70, 1.08}, {0.46, 0.78}, {0.33, 0.53},
                                           {0.35, 0.50}, 1.09};
-static const DmaRates dma_rates_tile = {{1.06, 1.63}, {0.89, 1.30}, {0.49, 1.13}, {0.94, 1.29}, {0.62, 1.08}, {0.46, 0.84}, {0.37, 0.58},
-                                        {0.35, 0.48}, 1.15};
+static const DmaRates dma_rates_tile = {{1.06, 1.63}, {0.89, 1.30}, {0.49, 1.13}, {0.96, 1.29}, {0.62, 1.08}, {0.46, 0.81}, {0.37, 0.58},
+                                        {0.35, 0.48}, 1.05};
 static DmaPlan dma_plan(int m, int n, int k, int fixed_slices) {
     DmaPlan best{0, 0, fixed_slices > 0 ? fixed_slices : 1, 2};
     if (m <= 64 || !dma_tile_takes(m, n, k)) return best;
