@@ -1767,13 +1767,17 @@ static int launch_bf16(const bf16_t* x, const bf16_t* w, const float* bias, TOut
     if (m <= ROWS_MAX && force == 0)
         return imparo_few_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue, slices,
                                nullptr, 0, 0.f, s);
-    // up to 96 rows the kernel of some_rows.hip, and up to 128 where it takes few weight rows a block: with 64 the tile of 128 by
-    // 64 draws the same bytes a CU with less to do about them (128 rows of 16,384 by 2,048 gated 20.0 us, 20.8 there; 96 rows 19.3
-    // and 18.9, 65 rows 18.9 and 17.5; 128 rows of 6,144 by 2,048 16.9 and 14.5).
-    // 616, 632, 664: that kernel with 16, 32 and 64 weight rows a block
+    // Up to 64 rows the kernel of some_rows.hip, and up to 128 where it takes few weight rows a block: with 64 the tile of 128 by
+    // 64 draws the same bytes a CU with less to do about them (128 rows of 16,384 by 2,048 gated 20.0 us, 20.8 there; 96 rows 18.9
+    // and 19.3, 65 rows 17.5 and 18.9; 79 rows of 60,418 by 128 8.6 and 21.5, 93 of 49,664 by 1,024 gated 26.8 and 39.1). But that
+    // tile's four stages take K-steps in fours: where K does not come in fours, up to 96 rows and in one round of the CUs this kernel is the
+    // faster one again (72 rows of 12,288 by 9,344 gated 68.7 us, 125.5 on the tile; 78 of 9,090 by 3,456 27.2 and 47.1, 71 of
+    // 9,216 by 640 8.9 and 11.8; in two rounds 70 of 17,920 by 2,688 40.1 and 39.2; 73 of 9,216 by 128 5.7 and 4.4).
+    // 616, 632, 664: this kernel with 16, 32 and 64 weight rows a block
     if (imparo_some_rows_takes(m, n, k) && (force == 0 || force == 616 || force == 632 || force == 664)) {
-        const int tile = force ? force - 600 : imparo_some_rows_tile(m, n, slices);
-        if (force || m <= 96 || tile <= 32)
+        const int tile = force ? force - 600 : imparo_some_rows_tile(m, n, slices), k_slice = k / slices;
+        const bool odd_steps = k_slice % (4 * DM_BK) != 0 && k_slice > 2 * DM_BK && (long long)((n + 63) / 64) * slices <= 256;
+        if (force || m <= 64 || tile <= 32 || (m <= 96 && odd_steps))
             return imparo_some_rows(x, w, bias, y, std::is_same<TOut, float>::value ? IMPARO_F32 : IMPARO_BF16, m, n, k, epilogue,
                                     slices, tile, s);
     }
