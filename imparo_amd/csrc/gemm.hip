@@ -468,9 +468,10 @@ static int launch_f32(const float* x, const float* w, const float* bias, TOut* y
     // 70, two 110, three 154, four 197, six 292. (So 16 to 128 rows by 2,048 by 1,024 24.4 -> 12.3 us, 666 by 1,024 by 4,608 95 -> 89.)
     auto a_cu = [&](bool small) { return ((long long)tiles(m, small) * tiles(n, small) + 255) / 256; };
     // (With three blocks a CU it takes a longer K and rows on 16 bytes: 666 rows by 1,024 by 8 6.0 us and 4.7, by 300 11.3 and 11.7, 64
-    // rows by 9,216 by 1,024 off 16 30.1 and 28.6.)
+    // rows by 9,216 by 1,024 off 16 30.1 and 28.6. With two more than one step of the other tile: 541 rows by 768 by 4 to 32 4.3 us and
+    // 3.9, by 48 4.3 and 4.8.)
     const bool at_16 = k % 4 == 0 && !(((uintptr_t)x | (uintptr_t)w) & 15);
-    const bool small = k >= 4 && 5 * a_cu(true) + 3 < 14 * a_cu(false) + 5 && (a_cu(true) <= 2 || (k >= 256 && at_16));
+    const bool small = k >= 4 && 5 * a_cu(true) + 3 < 14 * a_cu(false) + 5 && (a_cu(true) <= (k > 32 ? 2 : 1) || (k >= 256 && at_16));
     const int tiles_m = tiles(m, small), tiles_n = tiles(n, small);
     const long long total = (long long)tiles_m * tiles_n;
     if (total > 0x7f000000LL) return IMPARO_BAD_ARGUMENT;
