@@ -1563,8 +1563,9 @@ extern "C" int imparo_gemm_slices(int m, int n, int k, int dtype) {
         while (slices < 4 && tiles * slices * 2 <= 512 && k / (slices * 2) >= 1024) slices *= 2;
         return whole_slices(slices, k, BG_BK);
     }
-    // (weight rows a block that the count goes by; with at most 16 rows the kernel takes 16 to 64 as the slices and the CUs
-    // have it, so that 2,048 by 8,192 in four slices are 256 blocks of 32 and 1,024 by 4,608 in eight 512 of 16)
+    // (weight rows a block that the count goes by, those of the kernels it was measured with. The kernels of now take 16 to 64 as
+    // the slices and the CUs have it, so that 2,048 by 8,192 in four slices are 256 blocks of 32 and 1,024 by 4,608 in eight 512 of 16;
+    // the counts stay, as fewer slices are further from 64 bits)
     const int rows_per_block = n >= 12288 ? 64 : m > 16 || k >= 4096 ? 32 : 16;
     const int blocks = (n + rows_per_block - 1) / rows_per_block;
     int slices = 1;

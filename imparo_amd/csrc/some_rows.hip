@@ -237,6 +237,8 @@ bool imparo_some_rows_takes(int m, int n, int k) {
     return m > 16 && m <= SOME_ROWS_MAX && k % SR_BK == 0 && k < (1 << 23) && n < (1 << 25);
 }
 
+// What the fullest CU draws, weights and activations: the fewest weight rows a block whose blocks are still one round of the CUs, else 64
+// (but for a few shapes of more than 64 rows in three or six slices, where 32 take no more rounds than 64 do).
 int imparo_some_rows_tile(int m, int n, int slices) {
     const int rows = (m <= 64 ? (m + 15) / 16 : (m + 31) / 32 * 2) * 16;
     int best = 0;
