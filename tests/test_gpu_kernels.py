@@ -138,8 +138,8 @@ def test_gemm_in_slices_of_k_and_the_norm_that_adds_them(m):
 @pytest.mark.parametrize("m", [3, 16, 24, 64])
 @pytest.mark.parametrize("k", [264, 1024])
 def test_gemm_with_many_weight_rows(m, k):
-    """From about 12k weight rows on, few-row products go to the kernel that shares the
-    activations between the waves of a block: ragged K, a last block that is cut, bias, SwiGLU."""
+    """Few rows over about 12k weight rows: a last block that is cut, bias, SwiGLU. With more than 16 rows the ragged K runs on
+    the kernel that shares staged activations between the waves of a block, the other one on that of 17 to 128 rows."""
     n = 12288 + 2 * 37
     x, w, b = rnd(m, k, seed=1).to(torch.bfloat16), rnd(n, k, seed=2, scale=0.1).to(torch.bfloat16), rnd(n, seed=3)
     y = x.double() @ w.double().t() + b.double()
@@ -162,10 +162,10 @@ def test_gemm_with_many_weight_rows(m, k):
                                         (128, 16384, 2048, 0), (96, 2048, 8192, 0), (65, 3072, 2048, 0)])
 def test_gemm_with_large_tiles(m, n, k, tile):
     """Many rows: K a multiple of 128 goes to the kernel that loads straight into LDS, with a tile
-    of 256 or 128 rows by 256, 192, 128 or 64 weight rows, whichever its plan finds fastest (`tile`
+    of 256, 192 or 128 rows by 256, 192, 128 or 64 weight rows, whichever its plan finds fastest (`tile`
     other than 0 names one, an argument of the entry point for tests and measurements, so that each is met);
-    another K to the tile kernels with register staging. Edges in both directions, an odd number
-    of column pairs, a bias, both epilogues and output types."""
+    another K to the tile kernels with register staging, and up to 128 rows that would take fewer than 64 weight rows a block
+    to the kernel of 17 to 128 rows. Edges in both directions, an odd number of column pairs, a bias, both epilogues and output types."""
     _large_tile_case(m, n, k, tile)
 
 
