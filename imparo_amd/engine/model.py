@@ -79,6 +79,10 @@ class Model:
                 if owner != spec:
                     raise ValueError(f"run order entry {i} reads the cache of entry {call.cache_of}, "
                                      f"whose state has another shape")
+        # the norm that reads the stream behind each call and the dtype of its rows, where the next block tells and it may ride
+        # with the product before it
+        self.next_norm_of_call = [None if after.add_input or not emits(self.blocks[after.layer], "first_norm")
+                                  else self.blocks[after.layer].first_norm() for after in plan.order[1:]] + [None]
         # what the embedding keeps per request (the token before, say) is one more site, behind the layers'
         own = getattr(self.embedding, "cache_spec", lambda page_size: None)(page_size)
         if own is not None:
@@ -101,9 +105,7 @@ class Model:
                 if res.streams is not None or res.link is not None:
                     raise ValueError("a stream kept as several copies does not take the embedding's output in again")
                 ops.add_rows(res.x, kept)        # (what is pending on the stream is added by the next norm, as ever)
-            after = self.plan.order[i + 1] if i + 1 < len(self.plan.order) else None
-            tells = after is not None and not after.add_input and emits(self.blocks[after.layer], "first_norm")
-            ctx.next_norm = self.blocks[after.layer].first_norm() if tells else None
+            ctx.next_norm = self.next_norm_of_call[i]
             self.blocks[call.layer].forward(ctx, res, self.site_of_call[i], call.cache_of is None)
         if want_rows is None or want_rows.shape[0] == 0:
             return None

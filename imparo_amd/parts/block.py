@@ -25,6 +25,8 @@ class PreNormBlock:
     """Reads its parts by name: mixer_norm, mixer, ffn_norm, ffn; optionally shift; ffn_norm and ffn may be absent."""
     role = "block"
     graph_safe = True     # launches kernels only: a step made of such parts can be captured
+    # which norms may ride with the product before them, and which parts end with a product that takes one along
+    first_rides = ffn_norm_rides = mixer_takes = ffn_takes = False
 
     def __init__(self, parts: Dict[str, object]):
         self.parts = parts
@@ -33,6 +35,9 @@ class PreNormBlock:
         self.shift = parts.get("shift")
         if (self.ffn is None) != (self.ffn_norm is None):
             raise ValueError("a block has a feed-forward and the norm before it, or neither")
+        self.first_rides = self.shift is None and emits(self.mixer_norm, "ride")
+        self.ffn_norm_rides = emits(self.ffn_norm, "ride")
+        self.mixer_takes, self.ffn_takes = emits(self.mixer, "adds_last"), emits(self.ffn, "adds_last")
 
     def cache_spec(self, page_size: int):
         """What a call of this block keeps between steps: its mixer's state and,
@@ -54,16 +59,16 @@ class PreNormBlock:
         else:
             h = self.shift.forward(ctx, site, self.mixer_norm.forward(ctx, res, torch.float32, name="normed_f32"),
                                    self.mixer.in_dtype)
-        behind = ctx.next_norm if self.ffn is None else (self.ffn_norm, self.ffn.in_dtype)
-        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h), self.mixer, behind)
+        behind = ctx.next_norm if self.ffn is None else (self.ffn_norm, self.ffn.in_dtype) if self.ffn_norm_rides else None
+        res.pending = self._delta(ctx, res, lambda: self.mixer.forward(ctx, site, owns_cache, h), behind if self.mixer_takes else None)
         if self.ffn is not None:
             n = self.ffn_norm.forward(ctx, res, self.ffn.in_dtype)
-            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n), self.ffn, ctx.next_norm)
+            res.pending = self._delta(ctx, res, lambda: self.ffn.forward(ctx, n), ctx.next_norm if self.ffn_takes else None)
 
     def first_norm(self):
         """The norm that reads the stream first and the dtype its rows are asked for in, if it may ride with the product before
         this block."""
-        return None if self.shift is not None else (self.mixer_norm, self.mixer.in_dtype)
+        return (self.mixer_norm, self.mixer.in_dtype) if self.first_rides else None
 
     def can_emit(self) -> bool:
         if self.shift is not None or self.ffn is None:
@@ -79,15 +84,14 @@ class PreNormBlock:
         self.ffn.emit(program)
 
     @staticmethod
-    def _delta(ctx: StepContext, res: Residual, run, part=None, behind=None):
+    def _delta(ctx: StepContext, res: Residual, run, behind=None):
         """Runs a part whose result goes into the stream. With nothing pending the part may add its
         result to the stream itself (it then returns the stream); otherwise it returns a delta.
-        `behind`: the norm that reads the stream next and the dtype of its rows; a norm that can rides with
-        the last product of a `part` that says `adds_last`. Both have to say so of the `forward` they run: a part that
-        goes on adding to the stream, or a norm that does more, would leave rows of a stream that is not the one read."""
+        `behind`: the norm that reads the stream next and the dtype of its rows, where that norm can ride with the part's last
+        product. Both have to say so of the `forward` they run (`ride`, `adds_last`): a part that goes on adding to the
+        stream, or a norm that does more, would leave rows of a stream that is not the one read."""
         ctx.stream = res.x if res.pending is None else None
-        rides = ctx.stream is not None and behind and emits(behind[0], "ride") and emits(part, "adds_last")
-        ctx.ride = NormRide(*behind) if rides else None
+        ctx.ride = NormRide(*behind) if ctx.stream is not None and behind else None
         ride = ctx.ride
         try:
             delta = run()

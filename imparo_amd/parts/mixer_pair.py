@@ -75,6 +75,7 @@ class _Scoped:
 class MixerPair:
     role = "mixer"
     adds_last = True      # (where its right side says so; see `forward`)
+    left_takes = right_takes = False
 
     @staticmethod
     def _names(spec: PartSpec) -> Dict[str, str]:
@@ -102,6 +103,7 @@ class MixerPair:
         self.right = part_class("mixer", spec["right"].kind)(spec["right"], tensors, device, engine_dtype)
         if self.left.in_dtype != self.right.in_dtype:
             raise ValueError("two mixers side by side read their input in one dtype")
+        self.left_takes, self.right_takes = emits(self.left, "adds_last"), emits(self.right, "adds_last")
         self.normed = bool(spec.get("normed", True))
         if self.normed:
             self.left_out = place_vector(tensors[n["left_out"]], device)
@@ -132,9 +134,9 @@ class MixerPair:
             stream = ctx.stream
             ride = ctx.ride
             # (the norm behind both rides with the second)
-            first = NormRide(None, ride.out_dtype) if ride is not None and emits(self.left, "adds_last") else None
+            first = NormRide(None, ride.out_dtype) if ride is not None and self.left_takes else None
             a = self.left.forward(_Scoped(ctx, "left.", "left:", stream, first), site, owns_cache, h)
-            ride = ride if stream is not None and a is stream and emits(self.right, "adds_last") else None
+            ride = ride if stream is not None and a is stream and self.right_takes else None
             b = self.right.forward(_Scoped(ctx, "right.", stream=stream, ride=ride), site, owns_cache, h)
             deltas = tuple(d for d in (a, b) if stream is None or d is not stream)
             return stream if not deltas else deltas[0] if len(deltas) == 1 else deltas

@@ -6,20 +6,8 @@ import pytest
 import torch
 
 from imparo_amd.parts import attention, channel_delta, ffn, mixer_pair, norm, retention
-from imparo_amd.parts.base import Residual
+from imparo_amd.parts.base import Residual, emits
 from imparo_amd.parts.block import PreNormBlock
-
-
-def ride_of(part, behind):
-    """The ride that a block's part is offered while it runs."""
-    ctx, res, seen = types.SimpleNamespace(stream=None, ride=None), Residual(torch.zeros(2, 8)), []
-
-    def run():
-        seen.append(ctx.ride)
-        return torch.zeros(2, 8)
-    PreNormBlock._delta(ctx, res, run, part, (behind, torch.bfloat16))
-    assert ctx.ride is None and ctx.stream is None
-    return seen[0]
 
 
 new = lambda cls: cls.__new__(cls)
@@ -27,11 +15,15 @@ new = lambda cls: cls.__new__(cls)
 
 @pytest.mark.parametrize("part", [ffn.SwiGlu, ffn.ClampedGlu, ffn.PolyNormFfn, attention.Attention, channel_delta.ChannelDelta,
                                   retention.Retention, mixer_pair.MixerPair])
-def test_a_part_that_ends_with_its_product_is_offered_the_norm(part):
-    tanh = new(norm.DynamicTanh)
-    ride = ride_of(new(part), tanh)
-    assert ride.norm is tanh and ride.rows is None
-    assert ride_of(new(part), new(norm.RmsNorm)) is None
+def test_parts_that_end_with_their_product_say_so(part):
+    class Further(part):
+        def forward(self, *args):
+            raise NotImplementedError
+
+    block = PreNormBlock(dict(mixer_norm=new(norm.DynamicTanh), mixer=new(part), ffn_norm=new(norm.DynamicTanh), ffn=new(part)))
+    assert block.mixer_takes and block.ffn_takes and block.first_rides and block.ffn_norm_rides
+    block = PreNormBlock(dict(mixer_norm=new(norm.RmsNorm), mixer=new(Further), ffn_norm=new(norm.RmsNorm), ffn=new(Further)))
+    assert not (block.mixer_takes or block.ffn_takes or block.first_rides or block.ffn_norm_rides) and block.first_norm() is None
 
 
 class Recorder:
@@ -76,14 +68,32 @@ class Reads:                                     # (what runs here reads no rows
         return res.x
 
 
-@pytest.mark.parametrize("mixer, behind, rides", [(Ends, Tanh, True), (TwiceAndSaysSo, Tanh, True), (Twice, Tanh, False),
-                                                  (Recorder, Tanh, False), (Ends, Louder, False), (Ends, Reads, False)])
-def test_a_block_offers_the_norm_to_who_says_so(mixer, behind, rides):
-    """A part that goes on adding to the stream, or a norm that does more than ride, is left alone."""
-    block = PreNormBlock(dict(mixer_norm=Reads(), mixer=mixer()))
-    ctx, res = types.SimpleNamespace(stream=None, ride=None, max_seg_len=1, next_norm=(behind(), torch.bfloat16)), Residual(torch.zeros(2, 8))
-    block.forward(ctx, res, 0, True)
-    assert (block.mixer.ride is not None) == rides and res.pending is None and res.normed is None
+class TanhThatReads(Tanh):
+    """A norm that rides, for a block that runs: it says so of its own `forward`."""
+    def forward(self, ctx, res, out_dtype, name="normed"):
+        return res.x
+
+    ride = norm.DynamicTanh.ride
+
+
+@pytest.mark.parametrize("part, behind, rides", [(Ends, Tanh, True), (TwiceAndSaysSo, Tanh, True), (Twice, Tanh, False),
+                                                 (Recorder, Tanh, False), (Ends, Louder, False), (Ends, Reads, False)])
+def test_a_block_offers_the_norm_to_who_says_so(part, behind, rides):
+    """A part that goes on adding to the stream, or a norm that does more than ride, is left alone: behind a mixer, and
+    behind the feed-forward of the block before."""
+    after = PreNormBlock(dict(mixer_norm=behind(), mixer=Recorder()))
+    before = PreNormBlock(dict(mixer_norm=Reads(), mixer=Recorder(), ffn_norm=TanhThatReads(), ffn=part()))
+    ctx, res = types.SimpleNamespace(stream=None, ride=None, max_seg_len=1, next_norm=after.first_norm()), Residual(torch.zeros(2, 8))
+    before.forward(ctx, res, 0, True)
+    assert before.mixer.ride is None             # (that mixer does not say)
+    assert (before.ffn.ride is not None) == rides and (not rides or before.ffn.ride.norm is after.mixer_norm)
+    alone = PreNormBlock(dict(mixer_norm=Reads(), mixer=part()))
+    alone.forward(ctx, res, 0, True)
+    assert (alone.mixer.ride is not None) == rides
+    both = PreNormBlock(dict(mixer_norm=Reads(), mixer=part(), ffn_norm=TanhThatReads(), ffn=Recorder()))
+    both.forward(ctx, res, 0, True)
+    assert (both.mixer.ride is not None) == both.mixer_takes and both.ffn.ride is None
+    assert res.pending is None and res.normed is None and ctx.ride is None and ctx.stream is None
 
 
 def test_both_sides_of_a_pair_are_asked():
@@ -102,6 +112,7 @@ def test_both_sides_of_a_pair_are_asked():
     for left, right in ((Side(), Side()), (Silent(), Side()), (Side(), Silent())):
         pair, tanh = new(mixer_pair.MixerPair), new(norm.DynamicTanh)
         pair.left, pair.right, pair.normed = left, right, False
+        pair.left_takes, pair.right_takes = emits(left, "adds_last"), emits(right, "adds_last")
         ride = types.SimpleNamespace(norm=tanh, out_dtype=torch.bfloat16, rows=None)
         ctx = types.SimpleNamespace(stream=torch.zeros(2, 8), ride=ride, workspace=None)
         assert pair.forward(ctx, 0, True, torch.zeros(2, 8)) is ctx.stream
