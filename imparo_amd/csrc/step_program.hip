@@ -484,12 +484,12 @@ extern "C" int imparo_program_set_fold(ImparoProgram* p, int mode) {
 // Whether a product of m <= 16 rows over a [n, k] weight that feeds the residual stream should add its
 // result there itself and fold the next norm away: one launch less, at the price of every block
 // summing the whole of K (no slices of K over blocks) and of a product behind the norm that scales its
-// rows at its end. Measured on whole decode steps of 1 to 16 rows at three model widths (1024, 1536,
-// 2048) with everything folded, with only the products over K <= 2048 folded (the mixers' output
-// projections), and with nothing folded: the second is the fastest everywhere (a step of 8 rows at
-// width 1024: 0.670 ms against 0.702 and 0.718; at width 2048: 0.915 against 0.942 and 0.934); a block
-// that walked a K of 4,608 or more alone took longer than the norm's launch it saved. (With the kernels of then. Whole steps
-// have not been measured since; a row of 1,024 by 4,608 now takes 7.0 us into the stream, in eight slices 4.5.)
+// rows at its end. Measured on whole decode steps of 1 to 16 rows at three model widths (1,024, 1,536 and
+// 2,048; contexts of 100 tokens) with everything folded, with only the products over K <= 2,048 folded (the mixers' output
+// projections), and with nothing folded: the second is the fastest everywhere (us of a step of 1 / 8 / 16 rows at width
+// 1,024 474 509 548, 471 500 523 and 499 531 550; at 2,048 721 773 846, 722 756 797 and 751 779 819); a block
+// that walks a K of 4,608 or more alone takes longer than the norm's launch it saves (a row of 1,024 by 4,608 7.0 us into
+// the stream, in eight slices 4.5).
 extern "C" int imparo_rows_fold_pays(int m, int n, int k) {
     (void)n;
     return m <= 16 && k <= 2048;
