@@ -342,6 +342,19 @@ int imparo_attention_decode_qkv(const float* qkv, const float* q_weight, const f
                                 const int32_t* block_table, int table_stride, int page_size, int heads,
                                 int kv_heads, int head_dim, int n_pages, float scale, int window, int n_splits,
                                 imparo_stream stream);
+// The same under a rule, with exact weights (imparo_attention_decode_ruled), out of rows row_ld floats apart (a multiple of 4).
+// brings: the rows hold the new keys and values, which go into their pages; 0: queries only, of a layer that reads another
+// layer's cache, where the row's own key is already. magnitude: a factor on sines and cosines. whole: the norms run over all
+// query heads and over all key heads, weights as wide.
+int imparo_attention_decode_qkv_ruled_takes(int heads, int kv_heads, int head_dim, int n_freq, int whole);
+int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int whole);
+int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, int brings, const float* q_weight, const float* k_weight,
+                                      float eps, const float* inv_freq, int n_freq, int interleaved, float magnitude, int whole,
+                                      void* k_cache, void* v_cache, void* out, float* part_o, float* part_ml,
+                                      const int32_t* rows, int n_rows, const int32_t* seg_start, const int32_t* positions,
+                                      const int32_t* block_table, int table_stride, int page_size, int heads, int kv_heads,
+                                      int head_dim, int n_pages, float scale, int window, int n_splits,
+                                      const ImparoAttentionRule* rule, imparo_stream stream);
 
 // imparo_attention_decode for callers that cannot allocate device memory: code under HIP graph
 // capture, tight serving loops, harnesses that forbid hipMalloc. It has no counterpart in the

@@ -265,7 +265,12 @@ __device__ __forceinline__ void decode_tile(DecodeState<ND>& st, const DecodeTil
 // it and the new value in from registers (the cached keys end one position earlier), and, for a layer
 // that owns its cache, writes both into their page: the launch that would do all this ahead of the
 // attention is gone. Head sizes of 64 and 128 rotated whole, where both elements of a pair (i, i + D/2)
-// or (2i, 2i + 1) sit in one lane.
+// or (2i, 2i + 1) sit in one lane. Under a rule (EXT) heads of 64 only; the new key and value take their places in the loaded tile
+// there, so that a row has the bits of the two launches, and a layer without keys of its own brings queries alone. Bound by the
+// trips to memory behind one another, the rotation's float64 and the tiles' exponentials; 16 heads by 8, exact weights and a cap,
+// 8 rows over 200 keys 9.7 us in two launches and 8.5 in one, queries alone 9.1 and 7.0; 8 chats of a mixture 33.0 -> 32.1 ms.
+#define WHOLE_Q 2048            // the widest query part of a row, all heads, whose norm over all of it the kernel makes
+#define WHOLE_K 1024            // and the widest key part
 struct FromQkv {
     const float* qkv;
     const float* q_weight;      // per-head norm weights [D], or null: no norm
@@ -275,6 +280,11 @@ struct FromQkv {
     bf16_t* v_out;
     float eps;
     int interleaved;
+    // Where the kernel is built with EXT (else heads + 2 kv_heads units a row, the new key and value among them, and 1):
+    int row_ld;                 // floats from one token's row to the next
+    int brings;                 // the rows hold the new key and value; 0: queries only, all keys are in the cache
+    float magnitude;            // a factor on sines and cosines
+    int whole;                  // norms over all query heads and all key heads of a row, weights as wide
 };
 
 // One head's 8 x NK elements of a lane (dims dk*32 + 8*g + j): asked for early (`head_elements`, with the
@@ -299,18 +309,21 @@ __device__ __forceinline__ void head_elements(HeadElements<ND>& h, const float* 
 template <int ND>
 __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadElements<ND>& h, const float* weight,
                                                float eps, bool rotate, int interleaved, const float* sn_tab,
-                                               const float* cs_tab, bool valid, int g) {
+                                               const float* cs_tab, bool valid, int g, float given = 0.f) {
     constexpr int D = ND * 16, NK = (ND + 1) / 2;
     static_assert(D % 64 == 0, "pairs inside a lane");
     auto& e = h.e;
     if (weight) {                      // (in LDS)
-        float ss = 0.f;
+        float scale = given;           // (of a norm over more than the head)
+        if (given == 0.f) {
+            float ss = 0.f;
 #pragma unroll
-        for (int dk = 0; dk < NK; ++dk)
+            for (int dk = 0; dk < NK; ++dk)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) ss = fmaf(e[dk][j], e[dk][j], ss);
-        ss = sum_16_32(ss);
-        const float scale = head_norm_scale(ss, D, eps);
+                for (int j = 0; j < 8; ++j) ss = fmaf(e[dk][j], e[dk][j], ss);
+            ss = sum_16_32(ss);
+            scale = head_norm_scale(ss, D, eps);
+        }
 #pragma unroll
         for (int dk = 0; dk < NK; ++dk)
 #pragma unroll
@@ -356,8 +369,10 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
 // share), nor three or four splits (16 waves on one CU: 1,000 keys 17.7 | 13.4, queries given 12.9 | 11.7).
 // EXACT: see decode_tile; part of the kernel's type, as branches on it inside a tile kept the scheduler from filling one weight's
 // waits with the next one's work.
-template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1, bool EXACT = false>
-__global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_attn_decode(
+// WHOLE (from the projection's rows): the norms run over all query heads and over all key heads of a token, weights as wide as
+// those; every block adds up the squares of its whole row, 6 KB of 16 heads and 8, beside the sines and cosines.
+template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1, bool EXACT = false, bool WHOLE = false>
+__global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - SPLITS : 4) void k_attn_decode(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ seg_start, const int32_t* __restrict__ positions,
@@ -368,7 +383,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     __shared__ float sm[SPLITS * MFMA_WAVES][16], sl[SPLITS * MFMA_WAVES][16];
     __shared__ float so[SPLITS * MFMA_WAVES][16][D + 1];
     __shared__ float sn_tab[FROM_QKV ? D / 2 : 1], cs_tab[FROM_QKV ? D / 2 : 1];
-    __shared__ __attribute__((aligned(16))) float qw_tab[FROM_QKV ? D : 1], kw_tab[FROM_QKV ? D : 1];
+    __shared__ __attribute__((aligned(16))) float qw_tab[FROM_QKV ? (WHOLE ? 16 : 1) * D : 1], kw_tab[FROM_QKV ? D : 1];
+    __shared__ float sq_of[WHOLE ? MFMA_WAVES : 1], sk_of[WHOLE ? MFMA_WAVES : 1];
     __shared__ __attribute__((aligned(16))) float k_raw[FROM_QKV ? D : 1], v_raw[FROM_QKV ? D : 1];
     const int all_waves = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);     // of the block; `wave` is one of its split's
     const int split = SPLITS == 1 ? blockIdx.x : all_waves / MFMA_WAVES, ri = blockIdx.z;
@@ -378,14 +394,15 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     const int t = seg_start[row];
     const int pos = positions[t];
     const int lo = first_seen(pos, window);
-    const int last = FROM_QKV ? pos - 1 : pos;              // the last key that is in the cache
+    const bool brings = FROM_QKV && (!EXT || fq.brings);    // the row's own key and value are not in the cache
+    const int last = FROM_QKV && !EXT ? pos - 1 : pos;      // the last key that the tiles hold
     // (EXT: splits count keys in the numbering without the gap behind the first positions that stay)
     const TileWalk<32> walk(EXT ? rule.keep : 0, EXT ? lo : 0);
     const int keep = EXT ? rule.keep : 0;
     const float cap = EXT ? rule.cap : 0.f;
     const int k_begin = EXT ? split * DEC_SPLIT : max(split * DEC_SPLIT, lo & ~31);
     const int k_end = min((split + 1) * DEC_SPLIT, last + 1 - walk.gap);
-    const bool own = FROM_QKV && split == pos / DEC_SPLIT;  // this block weighs the row's own key in
+    const bool own = brings && split == (EXT ? pos - walk.gap : pos) / DEC_SPLIT;      // this block weighs the row's own key in
     if (SPLITS == 1 && k_begin >= k_end && !own) return;    // (with others' splits beside it: nothing of its own to add)
     const int lane = threadIdx.x & 63, wave = all_waves % MFMA_WAVES;
     const int c = lane & 15, g = lane >> 4;
@@ -414,16 +431,32 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
     float4 own_raw;
     const int norm_at = 2 * ((int)threadIdx.x - 128);       // (another wave's lanes than the sines and cosines)
     const int own_at = 4 * (lane % (D / 4));
+    constexpr int THREADS = SPLITS * MFMA_WAVES * 64, QW = WHOLE ? (16 * D / 4 + THREADS - 1) / THREADS : 1;
+    constexpr int PIECES = (WHOLE_Q + WHOLE_K) / 1024;
+    float4 piece[PIECES], qw_piece[QW];      // (WHOLE)
+    const int heads_at = brings ? (heads + kv_heads) * D : heads * D;       // where queries and keys end
     auto ask_shared = [&]() __attribute__((always_inline)) {      // (every lane asks, for something: no load under a branch)
-        const float* row_in = fq.qkv + (size_t)t * units * D;
+        const float* row_in = fq.qkv + (EXT ? (size_t)t * fq.row_ld : (size_t)t * units * D);
         const int norm_from = min(max(norm_at, 0), D - 2);
+        if constexpr (WHOLE) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+                piece[i] = *reinterpret_cast<const float4*>(row_in + min(4 * (int)(threadIdx.x & 255) + i * 1024, heads_at - 4));
+#pragma unroll
+            for (int i = 0; i < QW; ++i) {
+                const int at = min((int)threadIdx.x + i * THREADS, 16 * D / 4 - 1), of = at / (D / 4);
+                qw_piece[i] = *reinterpret_cast<const float4*>(fq.q_weight + (size_t)(kvh * G + min(pass * 16 + of, G - 1)) * D + at % (D / 4) * 4);
+            }
+        }
         head_elements<ND>(qh, row_in + (size_t)head * D, g);
         freq = (fq.inv_freq ? fq.inv_freq : row_in)[min((int)threadIdx.x, D / 2 - 1)];
         q_norm = make_float2((fq.q_weight ? fq.q_weight : row_in)[norm_from], (fq.q_weight ? fq.q_weight : row_in)[norm_from + 1]);
-        k_norm = make_float2((fq.q_weight ? fq.k_weight : row_in)[norm_from], (fq.q_weight ? fq.k_weight : row_in)[norm_from + 1]);
-        own_raw = *reinterpret_cast<const float4*>(row_in + (size_t)(lane < D / 4 ? heads + kvh : heads + kv_heads + kvh) * D + own_at);
+        const float* kw_in = fq.q_weight ? fq.k_weight + (WHOLE && brings ? kvh * D : 0) : row_in;
+        k_norm = make_float2(kw_in[norm_from], kw_in[norm_from + 1]);
+        own_raw = *reinterpret_cast<const float4*>(row_in + (size_t)(!brings ? 0 : lane < D / 4 ? heads + kvh : heads + kv_heads + kvh) * D + own_at);
         __builtin_amdgcn_sched_barrier(0);
     };
+    const int own_page = FROM_QKV && EXT ? kv.table[min(pos >> kv.page_shift, table_stride - 1)] : 0;
     if constexpr (AHEAD) ask_shared();
     DecodeTile<ND> regs[TILES];
     // (with the queries given, where nothing else waits for scalar loads, the lanes' own are no slower: 4.3 us, 4.5 so)
@@ -455,39 +488,112 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND <= 4 ? 4 : 2) void k_a
         else ask_shared();
         // while the tiles are on their way: the block's sines and cosines, the norms' weights, and the row's new key and
         // value, which wait in LDS for the wave that takes them
-        if (fq.inv_freq && (int)threadIdx.x < D / 2) rotation_of(pos, freq, sn_tab[threadIdx.x], cs_tab[threadIdx.x]);
+        if (fq.inv_freq && (int)threadIdx.x < D / 2) {
+            float sn, cs;
+            rotation_of(pos, freq, sn, cs);
+            sn_tab[threadIdx.x] = EXT ? sn * fq.magnitude : sn;
+            cs_tab[threadIdx.x] = EXT ? cs * fq.magnitude : cs;
+        }
         if (norm_at >= 0 && norm_at < D) {
-            *reinterpret_cast<float2*>(qw_tab + norm_at) = q_norm;
+            if (!WHOLE) *reinterpret_cast<float2*>(qw_tab + norm_at) = q_norm;
             *reinterpret_cast<float2*>(kw_tab + norm_at) = k_norm;
+        }
+        float q_given = 0.f;
+        if constexpr (WHOLE) {
+            // (256 threads, four neighbouring values each, as the launch that does this for many rows adds them: the same bits)
+            float sq = 0.f, sk = 0.f;
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) {
+                const int at = 4 * (int)(threadIdx.x & 255) + i * 1024;
+                float sum = 0.f;
+                sum = fmaf(piece[i].x, piece[i].x, sum);
+                sum = fmaf(piece[i].y, piece[i].y, sum);
+                sum = fmaf(piece[i].z, piece[i].z, sum);
+                sum = fmaf(piece[i].w, piece[i].w, sum);
+                sq += at < heads * D ? sum : 0.f;
+                sk += at >= heads * D && at < heads_at ? sum : 0.f;
+            }
+            sq = wave_sum(sq);
+            sk = wave_sum(sk);
+            if (lane == 0 && all_waves < MFMA_WAVES) sq_of[all_waves] = sq, sk_of[all_waves] = sk;
+#pragma unroll
+            for (int i = 0; i < QW; ++i)
+                if ((int)threadIdx.x + i * THREADS < 16 * D / 4)
+                    *reinterpret_cast<float4*>(qw_tab + 4 * (threadIdx.x + i * THREADS)) = qw_piece[i];
         }
         if (own && wave == 1 && lane < D / 2) *reinterpret_cast<float4*>((lane < D / 4 ? k_raw : v_raw) + own_at) = own_raw;
         __syncthreads();
-        normed_rotated<ND>(st.q, qh, fq.q_weight ? qw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
-                           sn_tab, cs_tab, qvalid, g);
+        if constexpr (WHOLE) {
+            q_given = head_norm_scale(sq_of[0] + sq_of[1] + sq_of[2] + sq_of[3], heads * D, fq.eps);
+        }
+        normed_rotated<ND>(st.q, qh, fq.q_weight ? qw_tab + (WHOLE ? c * D : 0) : nullptr, fq.eps, fq.inv_freq != nullptr,
+                           fq.interleaved, sn_tab, cs_tab, qvalid, g, q_given);
     }
+    // the row's own key from the projection's row, in the layout of a tile's rows: dims dk*32 + 8*g + j
+    auto own_key = [&](auto& kf) __attribute__((always_inline)) {
+        HeadElements<ND> kh;
+        head_elements<ND>(kh, k_raw, g);
+        float k_given = 0.f;
+        if constexpr (WHOLE) k_given = head_norm_scale(sk_of[0] + sk_of[1] + sk_of[2] + sk_of[3], kv_heads * D, fq.eps);
+        normed_rotated<ND>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
+                           sn_tab, cs_tab, true, g, k_given);
+    };
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
         const int kv_base = k_begin + (wave + j * MFMA_WAVES) * 32;
         if (kv_base < k_end) {
             const int kb = walk.key(kv_base);
+            if constexpr (FROM_QKV && EXT) if (own && pos >= kb && pos < kb + 32) {
+                // under a rule the own key and value take their places in the tile: the bits of a launch that finds them in
+                // the cache (models that route by what follows turn at near ties)
+                Frag8 kf[NK];
+                own_key(kf);
+                const int at = pos - kb;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int dk = 0; dk < NK; ++dk) {
+                        const bool here = 8 * (c >> 2) + 4 * t + (c & 3) == at;
+                        const uint4 was = regs[j].k[t][dk].u, is = kf[dk].u;
+                        regs[j].k[t][dk].u = make_uint4(here ? is.x : was.x, here ? is.y : was.y, here ? is.z : was.z, here ? is.w : was.w);
+                    }
+                const int page = own_page;
+                const bool writes = fq.k_out && pass == 0 && page >= 0 && page < n_pages;      // never outside the pool
+                const int slot = pos & (page_size - 1);
+                if (writes && c == 0) {
+                    bf16_t* kdst = fq.k_out + (((size_t)page * kv_heads + kvh) * page_size + slot) * D + 8 * g;
+#pragma unroll
+                    for (int dk = 0; dk < NK; ++dk) *reinterpret_cast<uint4*>(kdst + dk * 32) = kf[dk].u;
+                }
+#pragma unroll
+                for (int dt = 0; dt < ND; ++dt) {
+                    const uint32_t value = f32_to_bf16(v_raw[dt * 16 + c]);
+                    uint32_t w[4] = {regs[j].v[dt].u.x, regs[j].v[dt].u.y, regs[j].v[dt].u.z, regs[j].v[dt].u.w};
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int key = 8 * g + 2 * i;
+                        w[i] = key == at ? (w[i] & 0xffff0000u) | value : key + 1 == at ? (w[i] & 0xffffu) | value << 16 : w[i];
+                    }
+                    regs[j].v[dt].u = make_uint4(w[0], w[1], w[2], w[3]);
+                    if (writes && g == 0)
+                        fq.v_out[((size_t)page * kv_heads + kvh) * page_size * D + (size_t)(dt * 16 + c) * page_size + slot] = (bf16_t)value;
+                }
+            }
             const bool full = (kb >= lo || kb + 31 < keep) && kb + 31 <= last;
             decode_tile<ND>(st, regs[j], kb, lo, hi_q, lo, last, full, scale, lane, EXACT, keep, cap);
         }
     }
-    if constexpr (FROM_QKV) {
+    if constexpr (FROM_QKV && !EXT) {
         // (by the wave that has the fewest tiles, which is done first where the split is not full; the first with heads of 128,
         // which keeps the order of the sums there)
         if (own && wave == (AHEAD ? MFMA_WAVES - 1 : 0)) {
             // the row's own key and value, from the projection's row: every lane holds the key's dims
             // dk*32 + 8*g + j (the same for all 16 heads) and the value's dims dt*16 + 4*g + i
             Frag8 kf[NK];
-            HeadElements<ND> kh;
-            head_elements<ND>(kh, k_raw, g);
+            own_key(kf);
             float4 vnew[ND];
 #pragma unroll
             for (int dt = 0; dt < ND; ++dt) vnew[dt] = *reinterpret_cast<const float4*>(v_raw + dt * 16 + 4 * g);
-            normed_rotated<ND>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
-                               sn_tab, cs_tab, true, g);
             bf16_t vb[ND][4];
 #pragma unroll
             for (int dt = 0; dt < ND; ++dt) {
@@ -1452,24 +1558,27 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
                                    const ImparoAttentionRule* given = nullptr) {
     const int G = heads / kv_heads;
     const Rule rule = rule_of(given);
-    if (given && from_qkv) return IMPARO_BAD_ARGUMENT;
     // the merge moves four elements of a head in one access
     if (n_splits > 1 && (((uintptr_t)part_o & 15) || ((uintptr_t)out & 7))) return IMPARO_BAD_ARGUMENT;
     // two splits: one block takes both and there is no merge, where that is the faster way (k_attn_decode)
     const bool in_block = n_splits == 2 && !(from_qkv && head_dim > 64);
     dim3 grid(in_block ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
-#define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT)                                                                \
-    k_attn_decode<ND, QKV, EXT, SPLITS, EXACT><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                            \
+#define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT, WHOLE)                                                         \
+    k_attn_decode<ND, QKV, EXT, SPLITS, EXACT, WHOLE><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                            \
         Q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,           \
         positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, rule)
-#define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT)                                                                       \
+#define DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, WHOLE)                                                               \
     do {                                                                                                             \
-        if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT);                                \
-        else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT);                                                               \
+        if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT, WHOLE);                         \
+        else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT, WHOLE);                                                        \
     } while (0)
+#define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT) DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, false)
     if (given && !exact) return IMPARO_BAD_ARGUMENT;         // (the rules run with exact weights)
     if (from_qkv) {
-        if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, false);
+        if (given && head_dim != 64) return IMPARO_BAD_ARGUMENT;
+        if (given && from_qkv->whole) DECODE_NORM(4, true, true, nullptr, *from_qkv, true, true);
+        else if (given) DECODE_ANY(4, true, true, nullptr, *from_qkv, true);
+        else if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, false);
         else if (head_dim == 128) DECODE_ANY(8, true, false, nullptr, *from_qkv, false);
         else return IMPARO_BAD_ARGUMENT;
     } else if (given) {
@@ -1480,6 +1589,7 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
         DISPATCH_ND(head_dim / 16, DECODE_ANY(ND, false, false, (const bf16_t*)q, FromQkv{}, false));
     }
 #undef DECODE_ANY
+#undef DECODE_NORM
 #undef DECODE_GO
     if (launch_status()) return IMPARO_LAUNCH_FAILED;
     if (n_splits == 1 || in_block) return IMPARO_OK;
@@ -1571,6 +1681,27 @@ extern "C" int imparo_attention_decode_qkv_pays(int n_rows, int n_splits) {
     return n_rows <= 16 && (long long)n_rows * n_splits <= 1024;
 }
 
+static int attention_decode_qkv_entry(FromQkv fq, int n_freq, void* k_cache, void* v_cache, void* out, float* part_o, float* part_ml,
+                                      const int32_t* rows, int n_rows, const int32_t* seg_start, const int32_t* positions,
+                                      const int32_t* block_table, int table_stride, int page_size, int heads, int kv_heads,
+                                      int head_dim, int n_pages, float scale, int window, int n_splits, imparo_stream stream,
+                                      const ImparoAttentionRule* rule = nullptr) {
+    const int bad = check_common(fq.qkv, k_cache, v_cache, out, rows, seg_start, positions, block_table, table_stride,
+                                 page_size, heads, kv_heads, head_dim, n_pages, window);
+    if (bad) return bad;
+    if (!part_o || !part_ml || n_rows < 0 || n_splits <= 0 || n_splits > 65535) return IMPARO_BAD_ARGUMENT;
+    if (!imparo_attention_decode_qkv_takes(head_dim, n_freq) || (n_freq > 0 && !fq.inv_freq)) return IMPARO_BAD_ARGUMENT;
+    if ((fq.q_weight == nullptr) != (fq.k_weight == nullptr) || (fq.q_weight && !(fq.eps > 0.f))) return IMPARO_BAD_ARGUMENT;
+    if (((uintptr_t)fq.qkv | (uintptr_t)fq.q_weight | (uintptr_t)fq.k_weight | (uintptr_t)k_cache) % 16 != 0)
+        return IMPARO_BAD_ARGUMENT;
+    if (n_rows == 0) return IMPARO_OK;
+    if (n_rows > 65535) return IMPARO_BAD_ARGUMENT;
+    if (n_freq == 0) fq.inv_freq = nullptr;
+    return attention_decode_launch(nullptr, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
+                                   block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale,
+                                   window, n_splits, (hipStream_t)stream, &fq, rule ? 1 : 0, rule);
+}
+
 extern "C" int imparo_attention_decode_qkv(const float* qkv, const float* q_weight, const float* k_weight, float eps,
                                            const float* inv_freq, int n_freq, int interleaved, void* k_cache,
                                            void* v_cache, int write_kv, void* out, float* part_o, float* part_ml,
@@ -1578,21 +1709,50 @@ extern "C" int imparo_attention_decode_qkv(const float* qkv, const float* q_weig
                                            const int32_t* positions, const int32_t* block_table, int table_stride,
                                            int page_size, int heads, int kv_heads, int head_dim, int n_pages,
                                            float scale, int window, int n_splits, imparo_stream stream) {
-    const int bad = check_common(qkv, k_cache, v_cache, out, rows, seg_start, positions, block_table, table_stride,
-                                 page_size, heads, kv_heads, head_dim, n_pages, window);
-    if (bad) return bad;
-    if (!part_o || !part_ml || n_rows < 0 || n_splits <= 0 || n_splits > 65535) return IMPARO_BAD_ARGUMENT;
-    if (!imparo_attention_decode_qkv_takes(head_dim, n_freq) || (n_freq > 0 && !inv_freq)) return IMPARO_BAD_ARGUMENT;
-    if ((q_weight == nullptr) != (k_weight == nullptr) || (q_weight && !(eps > 0.f))) return IMPARO_BAD_ARGUMENT;
-    if (((uintptr_t)qkv | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)k_cache) % 16 != 0)
+    const FromQkv fq{qkv, q_weight, k_weight, inv_freq, write_kv ? (bf16_t*)k_cache : nullptr,
+                     write_kv ? (bf16_t*)v_cache : nullptr, eps, interleaved, (heads + 2 * kv_heads) * head_dim, 1, 1.0f, 0};
+    return attention_decode_qkv_entry(fq, n_freq, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
+                                      block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale, window,
+                                      n_splits, stream);
+}
+
+// Which heads imparo_attention_decode_qkv_ruled takes: of 64 (of 128 the two launches are the faster ones: 8 rows over 200 keys,
+// norms over all heads, 14.5 us and 12.5, over 4,000 39.7 and 31.6; a norm a head, over 4,000 36.8 and 33.2), rotated whole or
+// not at all, norms over all heads up to what a block's threads add up in one load each.
+extern "C" int imparo_attention_decode_qkv_ruled_takes(int heads, int kv_heads, int head_dim, int n_freq, int whole) {
+    return head_dim == 64 && (n_freq == 0 || n_freq == 32) &&
+           (!whole || ((long long)heads * head_dim <= WHOLE_Q && (long long)kv_heads * head_dim <= WHOLE_K));
+}
+// ... and for how many rows over how many splits it is the faster way. Launch behind launch, 16 heads by 8, one launch | two, us:
+// norms over all heads 1 row over 50 keys 7.2 | 8.3, 8 over 200 8.5 | 9.7, 8 over 1,000 12.0 | 13.4, 8 over 4,000 23.0 | 22.7, 16 over
+// 4,000 33.0 | 32.1, queries alone 30.0 | 31.2; a norm a head 8 over 200 8.2 | 10.9, 16 over 4,000 29.4 | 33.1.
+extern "C" int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int whole) {
+    return n_rows <= 16 && (long long)n_rows * n_splits <= (whole ? 128 : 1024);
+}
+
+// The same under a rule, with exact weights, out of rows that may be wider than the heads (row_ld floats apart). brings: the
+// rows hold the new keys and values, which are written into their pages; 0: queries only, of a layer that reads another's cache,
+// where the new keys are already. magnitude: a factor on sines and cosines. whole: q_weight and k_weight are as wide as all
+// query heads and all key heads, and the norms run over those.
+extern "C" int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, int brings, const float* q_weight,
+                                                 const float* k_weight, float eps, const float* inv_freq, int n_freq,
+                                                 int interleaved, float magnitude, int whole, void* k_cache, void* v_cache, void* out,
+                                                 float* part_o, float* part_ml, const int32_t* rows, int n_rows,
+                                                 const int32_t* seg_start, const int32_t* positions,
+                                                 const int32_t* block_table, int table_stride, int page_size, int heads,
+                                                 int kv_heads, int head_dim, int n_pages, float scale, int window,
+                                                 int n_splits, const ImparoAttentionRule* rule, imparo_stream stream) {
+    if (!rule || imparo_attention_rule_bad(*rule, window)) return IMPARO_BAD_ARGUMENT;
+    if (heads < 1 || kv_heads < 1 || head_dim < 1 || row_ld % 4 != 0 ||
+        row_ld < (long long)(heads + (brings ? 2 * kv_heads : 0)) * head_dim)
         return IMPARO_BAD_ARGUMENT;
-    if (n_rows == 0) return IMPARO_OK;
-    if (n_rows > 65535) return IMPARO_BAD_ARGUMENT;
-    const FromQkv fq{qkv, q_weight, k_weight, n_freq > 0 ? inv_freq : nullptr, write_kv ? (bf16_t*)k_cache : nullptr,
-                     write_kv ? (bf16_t*)v_cache : nullptr, eps, interleaved};
-    return attention_decode_launch(nullptr, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
-                                   block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale,
-                                   window, n_splits, (hipStream_t)stream, &fq);
+    if (!imparo_attention_decode_qkv_ruled_takes(heads, kv_heads, head_dim, n_freq, whole) || (whole && !q_weight))
+        return IMPARO_BAD_ARGUMENT;
+    const FromQkv fq{qkv, q_weight, k_weight, inv_freq, brings ? (bf16_t*)k_cache : nullptr,
+                     brings ? (bf16_t*)v_cache : nullptr, eps, interleaved, row_ld, brings != 0, magnitude, whole != 0};
+    return attention_decode_qkv_entry(fq, n_freq, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
+                                      block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale, window,
+                                      n_splits, stream, rule);
 }
 
 // ---------------------------------------------------------------- decode without a workspace argument

@@ -514,28 +514,63 @@ def attention_decode_qkv_pays(n_rows: int, max_context: int) -> bool:
     return bool(library().imparo_attention_decode_qkv_pays(int(n_rows), n_splits))
 
 
+def attention_decode_qkv_ruled_takes(heads: int, kv_heads: int, head_dim: int, n_freq: int, whole: bool) -> bool:
+    """Whether attention_decode_qkv takes such heads under a rule, `whole`: with norms over all heads of a row."""
+    return bool(library().imparo_attention_decode_qkv_ruled_takes(int(heads), int(kv_heads), int(head_dim), int(n_freq), int(whole)))
+
+
+def attention_decode_qkv_ruled_pays(n_rows: int, keys: int, whole: bool) -> bool:
+    """Whether the one launch is the faster way under a rule, for rows that see at most so many `keys`."""
+    return bool(library().imparo_attention_decode_qkv_ruled_pays(int(n_rows), max(1, -(-int(keys) // decode_split())), int(whole)))
+
+
 def attention_decode_qkv(qkv, q_weight, k_weight, eps: float, inv_freq, k_cache, v_cache, out, part_o, part_ml,
                          rows, n_rows: int, seg_start, positions, block_table, heads: int, scale: float,
                          window: Optional[int], max_context: int, interleaved: bool = False,
-                         write_kv: bool = True) -> torch.Tensor:
+                         write_kv: bool = True, rule: Optional[AttentionRule] = None, magnitude: float = 1.0,
+                         whole: bool = False) -> torch.Tensor:
     """qk_norm_rope_store and attention_decode in one launch less, for a step whose rows all bring one
     token: `qkv` is the fused projection's float32 rows; the new keys and values are weighed in from
-    registers and, with `write_kv`, written into their pages (V pages transposed)."""
+    registers and, with `write_kv`, written into their pages (V pages transposed). With a `rule` (and exact weights) the
+    rows may be wider (gates behind the heads) and sines and cosines carry `magnitude`; without `write_kv` they then hold
+    queries only, whose keys are all in the cache; `whole`: the norms run over all query heads and all key heads of a row,
+    weights as wide as those (without `write_kv` the key weight is not read)."""
     n_pages, kv_heads, page_size, head_dim = k_cache.shape
     n = qkv.shape[0]
-    _dev(qkv, "qkv", torch.float32, (n, (heads + 2 * kv_heads) * head_dim))
+    if rule is None:
+        if magnitude != 1.0 or whole:
+            raise KernelArgumentError("attention_decode_qkv: a magnitude and norms over all heads go with a rule")
+        _dev(qkv, "qkv", torch.float32, (n, (heads + 2 * kv_heads) * head_dim))
+    else:
+        _dev(qkv, "qkv", torch.float32)
+        if qkv.dim() != 2 or qkv.shape[1] < (heads + (2 * kv_heads if write_kv else 0)) * head_dim or qkv.shape[1] % 4:
+            raise KernelArgumentError(f"attention_decode_qkv: rows of {list(qkv.shape)} do not hold {heads} heads of {head_dim} on whole vectors")
     _dev(out, "attention out", torch.bfloat16)
     if out.numel() != n * heads * head_dim:
         raise KernelArgumentError("attention_decode_qkv: the output does not match the rows")
     if k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16 or tuple(v_cache.shape) != (n_pages, kv_heads, head_dim, page_size):
         raise KernelArgumentError("attention_decode_qkv: bfloat16 caches, V pages transposed")
     n_freq = 0 if inv_freq is None else inv_freq.shape[0]
-    if not attention_decode_qkv_takes(head_dim, n_freq):
+    if not (attention_decode_qkv_takes(head_dim, n_freq) if rule is None
+            else attention_decode_qkv_ruled_takes(heads, kv_heads, head_dim, n_freq, whole)):
         raise KernelArgumentError(f"attention_decode_qkv: heads of {head_dim} with {n_freq} rotated pairs are not taken")
     split = decode_split()
-    n_splits = max(1, (max_context + split - 1) // split)
+    keys = max_context if rule is None else attention_ruled_keys(max_context, window, rule)
+    n_splits = max(1, (keys + split - 1) // split)
     if part_o.numel() < n_rows * heads * n_splits * head_dim or part_ml.numel() < n_rows * heads * n_splits * 2:
         raise KernelArgumentError("attention_decode_qkv: the scratch for partial results is too small")
+    if rule is not None:
+        _check(library().imparo_attention_decode_qkv_ruled(
+            qkv.data_ptr(), qkv.shape[1], int(bool(write_kv)),
+            _dev(q_weight, "q norm weight", torch.float32, (heads * head_dim if whole else head_dim,)),
+            _dev(k_weight, "k norm weight", torch.float32, (kv_heads * head_dim,) if whole and write_kv else None if whole else (head_dim,)),
+            float(eps), _dev(inv_freq, "inv_freq", torch.float32), n_freq, int(bool(interleaved)), float(magnitude), int(bool(whole)), k_cache.data_ptr(),
+            v_cache.data_ptr(), out.data_ptr(), _dev(part_o, "partial outputs", torch.float32),
+            _dev(part_ml, "partial sums", torch.float32), _dev(rows, "decode rows", torch.int32), n_rows,
+            _dev(seg_start, "seg_start", torch.int32), _dev(positions, "positions", torch.int32, (n,)),
+            _dev(block_table, "block table", torch.int32), block_table.shape[1], page_size, heads, kv_heads, head_dim,
+            n_pages, float(scale), int(window or 0), n_splits, _rule(rule, heads, n), _stream()), "attention_decode_qkv")
+        return out
     _check(library().imparo_attention_decode_qkv(
         qkv.data_ptr(), _dev(q_weight, "q norm weight", torch.float32, (head_dim,)),
         _dev(k_weight, "k norm weight", torch.float32, (head_dim,)), float(eps),

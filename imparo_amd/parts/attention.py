@@ -220,6 +220,18 @@ class Attention:
         part_ml = ctx.workspace.get("attn_part_ml", (ctx.n_single_rows * self.heads * n_splits * 2,), torch.float32)
         return part_o, part_ml
 
+    def _from_the_projection(self, ctx: StepContext, T: int, row_ld: int, owns_cache: bool, whole: bool) -> bool:
+        """Whether a step of `T` single tokens takes the attention kernel that reads the projection's rows. Plain: keys of its
+        own and head norms; under a rule also queries alone, rows with gates behind the heads, norms over all heads, and
+        sines and cosines that carry a magnitude."""
+        n_freq = 0 if self.position.inv_freq is None else self.position.inv_freq.shape[0]
+        if self.rule is None:
+            return (owns_cache and not self.exact_weights and not self.row_store
+                    and ops.attention_decode_qkv_pays(T, ctx.max_context) and ops.attention_decode_qkv_takes(self.head_dim, n_freq))
+        keys = ops.attention_ruled_keys(ctx.max_context, self.window, self.rule)
+        return (row_ld % 4 == 0 and ops.attention_decode_qkv_ruled_pays(T, keys, whole)
+                and ops.attention_decode_qkv_ruled_takes(self.heads, self.kv_heads, self.head_dim, n_freq, whole))
+
     def forward(self, ctx: StepContext, site: int, owns_cache: bool, h: torch.Tensor) -> torch.Tensor:
         T = h.shape[0]
         if self.shared_kv and owns_cache:
@@ -240,9 +252,9 @@ class Attention:
         inv_freq = self.position.inv_freq
         interleaved = bool(getattr(self.position, "interleaved", False))
         Dv = self.value_dim
-        if (vt and owns_cache and not self.exact_weights and not self.row_store and ctx.single_rows is not None and ctx.n_single_rows == T and not ctx.n_portion_rows
-                and ops.attention_decode_qkv_pays(T, ctx.max_context)
-                and ops.attention_decode_qkv_takes(self.head_dim, 0 if inv_freq is None else inv_freq.shape[0])):
+        whole = self.norm_over == "projection"
+        if (vt and ctx.single_rows is not None and ctx.n_single_rows == T and not ctx.n_portion_rows
+                and self._from_the_projection(ctx, T, qkv.shape[1], owns_cache, whole)):
             # every row brings one token: head norm, rotation and the write of the new key and value ride
             # in the attention launch (the new key is weighed in from registers)
             o = ctx.workspace.get("attn_out", (T, self.heads * self.head_dim), ctx.dtype, alias="mixer_mid")
@@ -250,7 +262,7 @@ class Attention:
             ops.attention_decode_qkv(qkv, self.q_norm, self.k_norm, self.norm_eps, inv_freq, k_cache, v_cache, o,
                                      part_o, part_ml, ctx.single_rows, ctx.n_single_rows, ctx.seg_start,
                                      ctx.positions, table, self.heads, self.scale, self.window, ctx.max_context,
-                                     interleaved=interleaved)
+                                     interleaved=interleaved, write_kv=owns_cache, rule=rule, magnitude=self.magnitude, whole=whole)
             return self.out(ctx, o, torch.float32, "mixer_out", sliced_ok=True, into=ctx.stream)
         q = ctx.workspace.get("q", (T, self.heads, self.head_dim), ctx.dtype)
         where = (ctx.positions, ctx.row_of_token, table if owns_cache else None, ctx.page_size, q,

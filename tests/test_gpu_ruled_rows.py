@@ -1,0 +1,87 @@
+"""Decode attention under a rule out of the projection's rows: one launch instead of two."""
+import math
+
+import pytest
+import torch
+
+from gpu_helpers import hand_context
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def ops():
+    from imparo_amd.kernels import ops
+    return ops
+
+
+def rnd(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+
+
+@pytest.mark.parametrize("over", ["head", "projection"])
+@pytest.mark.parametrize("H,Hk,D", [(8, 2, 64), (20, 1, 64), (32, 16, 64)])
+@pytest.mark.parametrize("window,keep,page", [(None, 0, 64), (300, 70, 64), (32, 33, 32), (1, 0, 16), (-100, 0, 64)])
+@pytest.mark.parametrize("brings,gated,magnitude", [(True, False, 1.0), (True, True, 1.2), (False, False, 1.2)])
+def test_ruled_attention_from_the_projection_rows(over, H, Hk, D, window, keep, page, brings, gated, magnitude):
+    """Rows that bring queries, keys and values, or queries alone (another layer's cache), as the launch that norms, turns
+    and stores and the launch that attends give them: bit for bit, but for norms a head, whose squares are added in another
+    order and may turn a rounding to bfloat16. The row's own key is the first, the last of a tile, of a split, the first of one."""
+    lens = (1, 32, 33, 256, 257, 512, 513, 700)
+    R, n_pages = len(lens), sum(-(-c // page) for c in lens) + 2
+    ctx = hand_context([(c - 1, 1) for c in lens], page, n_pages, torch.bfloat16, DEV, kv_sites={0: (Hk, D)}, v_transposed=True)
+    k0, v0, table = ctx.kv(0)
+    k0.copy_(rnd(*k0.shape, seed=1)), v0.copy_(rnd(*v0.shape, seed=2))
+    units = H + (2 * Hk if brings else 0)
+    width = units * D + ((H + 7) // 8 * 8 if gated else 0)
+    rows = rnd(R, width, seed=3).to(DEV)
+    whole = over == "projection"
+    assert ops().attention_decode_qkv_ruled_takes(H, Hk, D, D // 2, whole)
+    qw, kw = (1 + 0.1 * rnd(H * D if whole else D, seed=4)).to(DEV), (1 + 0.1 * rnd(Hk * D if whole else D, seed=5)).to(DEV)
+    freq = torch.linspace(1.0, 0.01, D // 2, device=DEV)
+    rule = ops().attention_rule(H, keep_first=keep, softcap=20.0, sink=rnd(H, seed=7).to(DEV), out_scale=0.7)
+    if gated:
+        rule = rule.with_gate(rows, units * D)
+    scale = 1.0 / math.sqrt(D)
+    seen = ops().attention_ruled_keys(max(lens), window, rule)
+    splits = -(-seen // 256)
+    part = lambda n: torch.full((R * H * splits * n,), float("nan"), device=DEV)
+    got = []
+    for one in (True, False):
+        k, v = k0.clone(), v0.clone()
+        out = torch.full((R, H * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tail = (part(D), part(2), ctx.single_rows, R, ctx.seg_start, ctx.positions, table)
+        if one:
+            ops().attention_decode_qkv(rows, qw, kw, 1e-5, freq, k, v, out, *tail, H, scale, window, max(lens), write_kv=brings,
+                                       rule=rule, magnitude=magnitude, whole=whole)
+        else:
+            q = torch.empty(R, H, D, dtype=torch.bfloat16, device=DEV)
+            ops().qk_row_norm_rope_store(rows, qw, kw, over, 1e-5, freq, magnitude, ctx.positions, ctx.row_of_token,
+                                         table if brings else None, page, q, k if brings else None, v if brings else None, H,
+                                         Hk if brings else 0, D, D, v_transposed=True)
+            ops().attention_decode(q, k, v, out, *tail, scale, window, max(lens), exact=True, rule=rule)
+        got.append((out.cpu().float(), k.cpu(), v.cpu()))
+    assert bool(torch.isfinite(got[1][0]).all())
+    if whole:
+        assert all(torch.equal(a, b) for a, b in zip(*got))
+    top = float(got[1][0].abs().max())
+    torch.testing.assert_close(got[0][0], got[1][0], rtol=2 ** -6, atol=top * 2 ** -8)
+    torch.testing.assert_close(got[0][1].float(), got[1][1].float(), rtol=2 ** -7, atol=2 ** -9)
+    assert torch.equal(got[0][2], got[1][2])
+
+
+def test_ruled_rows_of_a_wrong_width_are_refused():
+    from imparo_amd.kernels import KernelArgumentError
+    ctx = hand_context([(4, 1)], 64, 4, torch.bfloat16, DEV, kv_sites={0: (2, 64)}, v_transposed=True)
+    k, v, table = ctx.kv(0)
+    i = torch.zeros(1, dtype=torch.int32, device=DEV)
+    out, part = torch.zeros(1, 4 * 64, dtype=torch.bfloat16, device=DEV), torch.zeros(4096, device=DEV)
+    rule = ops().attention_rule(4, softcap=20.0)
+    for width in (4 * 64, 8 * 64 + 2):
+        with pytest.raises(KernelArgumentError):
+            ops().attention_decode_qkv(torch.zeros(1, width, device=DEV), None, None, 0.0, None, k, v, out, part, part, i, 1, i, i,
+                                       table, 4, 0.125, None, 5, rule=rule)
+    takes = ops().attention_decode_qkv_ruled_takes
+    assert takes(33, 33, 64, 32, False) and takes(8, 2, 64, 0, False) and not takes(8, 2, 64, 16, False)
+    assert not takes(33, 1, 64, 32, True) and not takes(17, 17, 64, 32, True) and not takes(8, 2, 128, 64, False)
