@@ -680,6 +680,27 @@ int imparo_stream_norm(const float* x, int in_streams, float* x_out, const float
                        int streams, const float* mix, const float* join, const float* read, int norm,
                        const float* weight, const float* bias, float eps, void* out, int out_dtype, int n_out,
                        int width, imparo_stream stream);
+// The same for the at most 16 rows of a decode step (imparo_stream_step_takes), written to x_out, everything asked for at once: what
+// joins is n_delta slices, or experts' rows that lie by entry, row t * top + j of y for the j-th expert in token t's list. With
+// router_w [n_router, width] bfloat16 (imparo_stream_step_routes; bfloat16 out, no groups) the row, as it is stored, goes on through
+// a mixture's router (+ router_bias) in the same launch: route_choice and route_weight [n_rows, route_top + always] as
+// imparo_moe_route leaves them. The bits are those of imparo_stream_norm, of the product of few rows, and of imparo_moe_route.
+int imparo_stream_step_takes(int n_rows, int streams, int width, int n_delta, int top);
+int imparo_stream_step_routes(int width, int n_router, int top);
+int imparo_stream_step(const float* x, int in_streams, float* x_out, const float* delta, int n_delta, const float* y,
+                       const void* h, int h_dtype, const int32_t* choice, const float* choice_weight, int top, int n_experts,
+                       int n_rows, int streams, const float* mix, const float* join, const float* read, int norm,
+                       const float* weight, const float* bias, float eps, void* out, int out_dtype, int width,
+                       const void* router_w, const float* router_bias, const float* correction, int n_router, int route_top,
+                       int scoring, int normalize, float route_scale, int always, int32_t* route_choice, float* route_weight,
+                       imparo_stream stream);
+// A mixture's bfloat16 products for a step of few tokens (imparo_moe_direct_takes) straight from the tokens' choices [n_tokens,
+// used], without a plan: out has a row an entry, token * used + place in its list; own_rows: row t of `a` is read for every entry of
+// token t, else row t * used + j. w [n_experts, n, k], epilogues and limits as imparo_moe_gemm (gated: bfloat16 out, else float32).
+int imparo_moe_direct_takes(int n_tokens, int used, int n_experts);
+int imparo_moe_gemm_direct(const void* a, int a_ld, int own_rows, const int32_t* choice, int n_tokens, int used, int n_experts,
+                           const void* w, void* out, int out_dtype, int n, int k, int epilogue, const float* limits, float alpha,
+                           imparo_stream stream);
 // x[t] = table[ids[t]] * scale + bigram[row], row = (previous * mul_prev + ids[t] * mul_cur) mod buckets, or `buckets`
 // for a token at position 0, which has none before it. The previous token is the one before it in its segment, or for
 // a segment's first token what the request left in state[slot]; with `advance` the segment's last token is left there.

@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "api.h"
+#include "moe_route.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -23,28 +24,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define MOE_MAX_ROUTER 512          // router outputs (experts of both kinds)
 #define MOE_MAX_EXPERTS 1024        // real experts the plan kernel keeps counters for
 #define MOE_MAX_TOP 16              // experts a token chooses
-#define MOE_MAX_USED 24             // experts a token uses: those and the ones that every token uses
 #define MOE_COUNTED -1              // the rows of an empty tile that holds the number of tiles before the empty ones
-#define MOE_SCORE_SOFTMAX 0         // scores = softmax over all router outputs
-#define MOE_SCORE_SIGMOID 1         // scores = sigmoid of each output
-#define MOE_SCORE_CHOSEN 2          // scores = the outputs themselves; a token's weights = softmax over its chosen ones
 
 extern "C" int imparo_moe_max_tiles(int n_entries, int n_experts, int tile_rows);
 
 // ---------------------------------------------------------------- route
-// What a router may do beyond scoring and choosing. logits_ld: floats between two tokens' logits (at least
-// n_router; further columns belong to someone else). groups > 1: the router outputs form that many equal
-// groups of neighbours, a group's score is the sum of its two largest choice scores (score + correction), and
-// only outputs of the `keep` best groups can be chosen (of equal groups the lowest). normalize: the chosen
-// scores are divided by their sum + 1e-20. scale: the weights are multiplied by it at the end. always: so many
-// experts, numbered behind the router's outputs, are used by every token with weight one; a token's list of experts
-// has them behind its `top` chosen ones.
-struct MoeRouteRules {
-    int logits_ld, groups, keep, normalize;
-    float scale;
-    int always;
-};
-
 template <int N>
 __device__ __forceinline__ void moe_better_of(float& best, int& at) {
     const float ob = lane_xor<N>(best);
@@ -172,68 +156,6 @@ __device__ __forceinline__ void moe_route_token(const float* __restrict__ logits
         if (lane == 0)
             for (int k = 0; k < top; ++k) weight[k] *= f;
     }
-}
-
-// The same for at most 64 outputs without groups: a lane holds one output and counts the ones that come before it (larger,
-// or as large with a lower index), so the k-th choice is the lane whose count is k: some five instructions an output
-// instead of twelve shuffles a choice, each of which waits for LDS. Same picks, weights and order of addition. 4 of 8
-// outputs: 2,048 rows 6.8 -> 3.9 us; 8 rows, with the plan made in the same launch from choices kept in LDS, 7.7 -> 4.1.
-__device__ __forceinline__ void moe_route_token_narrow(const float* __restrict__ logits, const float* __restrict__ correction,
-                                                       int32_t* choice, float* __restrict__ weight, int t, int n_router, int top,
-                                                       int scoring, const MoeRouteRules rules, int32_t* choice_too) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int used = top + rules.always;
-    choice += (size_t)t * used;
-    weight += (size_t)t * used;
-    const bool mine = lane < n_router;
-    float z = mine ? logits[(size_t)t * rules.logits_ld + lane] : -INFINITY;
-    const float shift = mine && correction ? correction[lane] : 0.f;
-    if (scoring == MOE_SCORE_SIGMOID) {
-        z = mine ? 1.0f / (1.0f + expf(-z)) : 0.f;
-    } else if (scoring == MOE_SCORE_SOFTMAX) {
-        const float m = wave_max(z);
-        z = mine ? expf(z - m) : 0.f;
-        z *= 1.0f / wave_sum(z);
-    }
-    const float pick = mine ? z + shift : -INFINITY;
-    int before = 0;
-    for (int i = 0; i < n_router; ++i) {
-        const float other = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(pick), i));
-        before += (other > pick || (other == pick && i < lane)) ? 1 : 0;
-    }
-    const bool valid = pick > -INFINITY;                     // (and no NaN: those are never chosen)
-    float chosen_sum = 0.f, chosen_max = -INFINITY, score = -INFINITY;      // score, at: lane k keeps the k-th choice's
-    int at = 0x7fffffff;
-    for (int k = 0; k < top; ++k) {
-        const unsigned long long who = __ballot(valid && before == k);
-        const int i = who ? __ffsll((long long)who) - 1 : 0;
-        const float s = who ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(z), i)) : 0.f;
-        chosen_sum += s;
-        chosen_max = fmaxf(chosen_max, s);
-        if (lane == k) {
-            score = s;
-            at = who ? i : 0x7fffffff;
-        }
-    }
-    float w = score;
-    if (scoring == MOE_SCORE_CHOSEN) {
-        const float e = lane < top ? expf(score - chosen_max) : 0.f;
-        w = e / wave_sum(e) * rules.scale;
-    } else if (rules.normalize || rules.scale != 1.0f) {
-        w *= (rules.normalize ? 1.0f / (chosen_sum + 1e-20f) : 1.0f) * rules.scale;
-    }
-    if (lane < used) {
-        const int e = lane < top ? at : n_router + lane - top;
-        choice[lane] = e;
-        weight[lane] = lane < top ? w : 1.0f;
-        if (choice_too) choice_too[(size_t)t * used + lane] = e;
-    }
-}
-
-// Counting costs by the output, choosing in rounds by the choice: 8,192 rows, counted | in rounds, 64 outputs: the best one 9.8 |
-// 7.6 us, two 10.0 | 9.4, four 10.4 | 13.2; 32 outputs: the best one 6.7 | 7.6.
-__device__ __forceinline__ bool moe_routes_narrow(int n_router, int top, const MoeRouteRules& rules) {
-    return n_router <= WAVE && rules.groups == 1 && (n_router <= 32 || top >= 3);
 }
 
 __global__ void k_moe_route(const float* __restrict__ logits, const float* __restrict__ correction,
@@ -769,13 +691,22 @@ __global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__
 // unevenly over the XCDs), the way back, 1,024 by 768, 6.2 (7.1); one token 6.3 and 4.6 (7.4 and 5.2). Over 3,920 forms of 4 to
 // 128 experts 1.23 times as fast as that on average, 90 slower by more than 3 % and 0.1 us: gated, K of 1,024 and 2,048 over
 // few rows, by 12 % at the most.
+// DIRECT: no plan at all. A step of at most 16 tokens fits one tile of slots, so a block of expert `y` takes all tokens, finds
+// in their choices (`tiles`: [max_tiles tokens, gather_div used]) which of them use the expert, and leaves where nobody does;
+// rows of `out` (and of A, unless the tokens' own rows are read: bit 0 of `own_rows`) go by entry, token * used + place in its list. A row of the tile sums
+// over k as it does in any other, so results have the bits of planned ones. Worth the launch of the plan and not faster by
+// itself, cold weights, direct | planned us, gate and up, way back: 9 experts of 768 by 1,024, five a token, 1 token 6.8 | 5.9, 4.6 | 4.5,
+// 8 tokens 8.1 | 8.3, 6.0 | 5.8; 16 of 512 by 2,048, four a token, 1 token 9.1 | 7.1, 4.5 | 4.0, 8 tokens 13.5 | 13.3, 8.1 | 7.5; 32 of
+// 512 by 1,024, four a token, whose blocks mostly leave, 8 tokens 11.0 | 9.9, 6.8 | 5.9.
 #define MOE_ROWS_WAVES 4
-template <typename TOut, bool GATED, int RT, int U>
+#define MOE_DIRECT_TOKENS 16
+#define MOE_DIRECT_USED 8
+template <typename TOut, bool GATED, int RT, int U, bool DIRECT = false>
 __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const bf16_t* __restrict__ A, int a_ld, int gather_div,
                                                          const int32_t* __restrict__ entry_of_slot,
                                                          const bf16_t* __restrict__ W, TOut* __restrict__ out,
                                                          const int32_t* __restrict__ tiles, int max_tiles,
-                                                         int N, int K, int epi, MoeGate gate) {
+                                                         int N, int K, int epi, MoeGate gate, int own_rows) {
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int GROUPS = GATED ? RT / 2 : RT;          // of 16 outputs a block
@@ -784,43 +715,17 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
     // The tiles that hold slots come first in the grid, so that the XCDs, which take its blocks in turn, have equally many of
     // them (9 tiles of 12 by 24 blocks, tile after tile along the grid: 36 on two XCDs of 32 CUs and 24 on the others, 12.0 us
     // where this way it is 10.1).
-    const int32_t* last = tiles + 3 * (max_tiles - 1);
-    // (what the tile holds is read beside the number of tiles, and nothing of either under a condition: one trip to memory of
-    // 0.6 us, and not three)
-    const unsigned tile = blockIdx.z * gridDim.y + blockIdx.y, listed = min(tile, (unsigned)max_tiles - 1);
-    const int expert = tiles[3 * listed], row0 = tiles[3 * listed + 1], rows = tiles[3 * listed + 2];
-    const int last_expert = last[0], last_rows = last[2];
-    int counted = last[1];
-    asm volatile("" : "+s"(counted));                    // (or it is asked for when the others have come)
-    const int n_tiles = (last_expert < 0) & (last_rows == MOE_COUNTED) ? min(counted, max_tiles) : max_tiles;
-    if ((int)(tile >= (unsigned)n_tiles) | (expert < 0) | (row0 < 0) | (rows < 1)) return;
-    const int n0 = (int)blockIdx.x * 16 * GROUPS;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
     const int c = lane & 15, g = lane >> 4;
-    const int slot = row0 + min(c, rows - 1);
-    const int entry = entry_of_slot ? entry_of_slot[slot] : 0;
-    const bf16_t* wrow[RT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int f = n0 + (t % GROUPS) * 16 + c;
-        wrow[t] = W + ((size_t)expert * N + (GATED ? (f >> 5) * 64 + (f & 31) + (t / GROUPS) * 32 : min(f, N - 1))) * K;
-    }
+    const int n0 = (int)blockIdx.x * 16 * GROUPS;
+    int expert, row0 = 0, rows, entry = 0, slot;
+    bool live;                                           // this lane's column of the tile is a slot of the expert's
+    const bf16_t* arow;
     const int runs = (K + 63) / 64, a_wave = (runs + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES;
     const int run_lo = wave * a_wave, run_hi = min(runs, run_lo + a_wave);
     u32x4 w[RT][U][2], x[U][2];
     // (no load under a branch: what lies past K is read again from inside the row, and its weights count as zeros)
     auto k_of = [&](int run, int h) { return min(min(run, runs - 1) * 64 + g * 16 + h * 8, K - 8); };
-    auto ask_weights = [&](int first) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < RT; ++t)
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) w[t][u][h] = *reinterpret_cast<const u32x4*>(wrow[t] + k_of(first + u, h));
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    ask_weights(run_lo);
-    const bf16_t* arow = A + (size_t)(gather_div ? entry / gather_div : slot) * a_ld;
     auto ask_rows = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -828,9 +733,68 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
             for (int h = 0; h < 2; ++h) x[u][h] = *reinterpret_cast<const u32x4*>(arow + k_of(first + u, h));
         __builtin_amdgcn_sched_barrier(0);
     };
-    ask_rows(run_lo);
+    auto weight_row = [&](int t) {
+        const int f = n0 + (t % GROUPS) * 16 + c;
+        return W + ((size_t)expert * N + (GATED ? (f >> 5) * 64 + (f & 31) + (t / GROUPS) * 32 : min(f, N - 1))) * K;
+    };
+    auto ask_weights = [&](int first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const bf16_t* wrow = weight_row(t);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) w[t][u][h] = *reinterpret_cast<const u32x4*>(wrow + k_of(first + u, h));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (DIRECT) {
+        expert = blockIdx.y;
+        rows = max_tiles;
+        const int token = min(c, rows - 1), used = gather_div;
+        // (all tokens' choices, at most 128, in two loads of the wave: who uses the expert is then two masks)
+        const int entries = rows * used;
+        int choice[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) choice[i] = tiles[min(lane + 64 * i, entries - 1)];
+        if (own_rows & 1) {                              // (the choices are on their way beside them)
+            arow = A + (size_t)token * a_ld;
+            ask_rows(run_lo);
+        }
+        // (where hardly an expert goes unchosen its rows are asked for before that is known: one trip to memory less)
+        if (own_rows & 2) ask_weights(run_lo);
+        const unsigned long long lo = __ballot(lane < entries && choice[0] == expert);
+        const unsigned long long hi = __ballot(lane + 64 < entries && choice[1] == expert);
+        const int bit = token * used;
+        const unsigned long long mine = bit >= 64 ? hi >> (bit - 64) : bit ? lo >> bit | hi << (64 - bit) : lo;
+        const int at = __ffsll((long long)(mine & ((1ull << used) - 1))) - 1;
+        live = at >= 0 && c < rows;
+        const unsigned long long who = __ballot(live);
+        if (who == 0) return;
+        entry = slot = token * used + max(at, 0);
+        // (a column that is nobody's reads what the first one reads)
+        if (!(own_rows & 1)) arow = A + (size_t)(live ? slot : __shfl(slot, __ffsll(who) - 1)) * a_ld;
+    } else {
+    const int32_t* last = tiles + 3 * (max_tiles - 1);
+    // (what the tile holds is read beside the number of tiles, and nothing of either under a condition: one trip to memory of
+    // 0.6 us, and not three)
+    const unsigned tile = blockIdx.z * gridDim.y + blockIdx.y, listed = min(tile, (unsigned)max_tiles - 1);
+    expert = tiles[3 * listed], row0 = tiles[3 * listed + 1], rows = tiles[3 * listed + 2];
+    const int last_expert = last[0], last_rows = last[2];
+    int counted = last[1];
+    asm volatile("" : "+s"(counted));                    // (or it is asked for when the others have come)
+    const int n_tiles = (last_expert < 0) & (last_rows == MOE_COUNTED) ? min(counted, max_tiles) : max_tiles;
+    if ((int)(tile >= (unsigned)n_tiles) | (expert < 0) | (row0 < 0) | (rows < 1)) return;
+    slot = row0 + min(c, rows - 1);
+    live = c < rows;
+    entry = entry_of_slot ? entry_of_slot[slot] : 0;
+    }
+    if (!DIRECT || !(own_rows & 2)) ask_weights(run_lo);
+    if constexpr (!DIRECT) arow = A + (size_t)(gather_div ? entry / gather_div : slot) * a_ld;
+    if (!DIRECT || !(own_rows & 1)) ask_rows(run_lo);
     const float limit = GATED && gate.limits ? gate.limits[expert] : 0.f;
-    const float sw = GATED ? moe_slot_weight(gate, entry_of_slot, slot) : 1.f;
+    const float sw = GATED && !DIRECT ? moe_slot_weight(gate, entry_of_slot, slot) : 1.f;
+    const size_t out_row = DIRECT ? entry : row0 + c;
     f32x4 acc[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -883,18 +847,18 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
         if constexpr (GATED) {
             float up[4];
             total(t + GROUPS, up);
-            if (c >= rows) continue;
+            if (!live) continue;
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = moe_act_fast(sw * v[i], sw * up[i], limit, gate.alpha);
-            TOut* dst = out + (size_t)(row0 + c) * (N / 2) + n;
+            TOut* dst = out + out_row * (N / 2) + n;
             if (((uintptr_t)out & 7) == 0)               // (N / 2 is a multiple of 32, and the output bfloat16)
                 *reinterpret_cast<uint2*>(dst) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
             else
                 for (int i = 0; i < 4; ++i) store_f32<TOut>(dst, i, v[i]);
-        } else if (c < rows) {
+        } else if (live) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (n + i < N) store_f32<TOut>(out, (size_t)(row0 + c) * N + n + i, moe_epilogue(v[i], epi));
+                if (n + i < N) store_f32<TOut>(out, out_row * N + n + i, moe_epilogue(v[i], epi));
         }
     }
 }
@@ -903,23 +867,53 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
 // of many experts was slower, by up to 1.4 times (20 slots of 128 experts, 1,024 by 1,024: 9.5 us and 13.6). Runs at once: all
 // of a wave up to three, then four where they come out even, or two where a run is a gate row's and an up row's (K of 2,048,
 // gated, one slot: four 7.4 us, two 6.8).
-template <typename TOut, bool GATED>
+template <typename TOut, bool GATED, bool DIRECT = false>
 static void launch_rows16(const bf16_t* a, int a_ld, int gather_div, const int32_t* entry_of_slot, const bf16_t* w, TOut* out,
-                          const int32_t* tiles, int max_tiles, int n, int k, int epi, const MoeGate& gate, hipStream_t s) {
+                          const int32_t* tiles, int max_tiles, int n, int k, int epi, const MoeGate& gate, hipStream_t s,
+                          int n_experts = 0, int own_rows = 0) {
     constexpr int RT = GATED ? 2 : 1;
     const int runs = (k + 63) / 64, a_wave = (runs + MOE_ROWS_WAVES - 1) / MOE_ROWS_WAVES;
     const int waves = (runs + a_wave - 1) / a_wave;      // (all that have a run: four, or fewer with a short K)
-    const int tall = std::min(max_tiles, 32768);
-    const dim3 grid((unsigned)(((GATED ? n / 2 : n) + 15) / 16), (unsigned)tall, (unsigned)((max_tiles + tall - 1) / tall));
+    const int tall = DIRECT ? n_experts : std::min(max_tiles, 32768);
+    const dim3 grid((unsigned)(((GATED ? n / 2 : n) + 15) / 16), (unsigned)tall, DIRECT ? 1u : (unsigned)((max_tiles + tall - 1) / tall));
     const size_t lds = (size_t)waves * RT * WAVE * sizeof(float4);
 #define ROWS16_U(U)                                                                                                  \
-    k_moe_gemm_rows16<TOut, GATED, RT, U><<<grid, waves * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out, tiles,   \
-                                                                max_tiles, n, k, epi, gate)
+    k_moe_gemm_rows16<TOut, GATED, RT, U, DIRECT><<<grid, waves * 64, lds, s>>>(a, a_ld, gather_div, entry_of_slot, w, out,  \
+                                                                        tiles, max_tiles, n, k, epi, gate, own_rows)
     if (a_wave == 1) ROWS16_U(1);
     else if (a_wave == 3) ROWS16_U(3);
     else if (!GATED && a_wave % 4 == 0) ROWS16_U(4);
     else ROWS16_U(2);
 #undef ROWS16_U
+}
+
+// The products of a step of few tokens straight from the tokens' choices (k_moe_gemm_rows16, DIRECT): without a plan. For few
+// experts, as the blocks of those that nobody chose come all the same.
+extern "C" int imparo_moe_direct_takes(int n_tokens, int used, int n_experts) {
+    return n_tokens >= 1 && n_tokens <= MOE_DIRECT_TOKENS && used >= 1 && used <= MOE_DIRECT_USED && n_experts >= 1 && n_experts <= 24;
+}
+
+// own_rows: row t of `a` is read for every entry of token t, else row t * used + j for its j-th; out has a row an entry.
+extern "C" int imparo_moe_gemm_direct(const void* a, int a_ld, int own_rows, const int32_t* choice, int n_tokens, int used,
+                                      int n_experts, const void* w, void* out, int out_dtype, int n, int k, int epilogue,
+                                      const float* limits, float alpha, imparo_stream stream) {
+    if (!a || !choice || !w || !out || n < 1 || k < 8 || k % 8 || a_ld < k || a_ld % 8) return IMPARO_BAD_ARGUMENT;
+    if (!imparo_moe_direct_takes(n_tokens, used, n_experts) || ((uintptr_t)a | (uintptr_t)w) % 16) return IMPARO_BAD_ARGUMENT;
+    if (epilogue < MOE_EPI_NONE || epilogue > MOE_EPI_GATED) return IMPARO_BAD_ARGUMENT;
+    hipStream_t s = (hipStream_t)stream;
+    const MoeGate gate{limits, alpha, nullptr, 0};
+    const int flags = (own_rows ? 1 : 0) | (n_tokens * used >= 2 * n_experts ? 2 : 0);
+    if (epilogue == MOE_EPI_GATED) {
+        if (out_dtype != IMPARO_BF16 || n % 64) return IMPARO_BAD_ARGUMENT;
+        launch_rows16<bf16_t, true, true>((const bf16_t*)a, a_ld, used, nullptr, (const bf16_t*)w, (bf16_t*)out, choice, n_tokens, n, k,
+                                          epilogue, gate, s, n_experts, flags);
+    } else if (out_dtype == IMPARO_F32) {
+        launch_rows16<float, false, true>((const bf16_t*)a, a_ld, used, nullptr, (const bf16_t*)w, (float*)out, choice, n_tokens, n, k,
+                                          epilogue, gate, s, n_experts, flags);
+    } else {
+        return IMPARO_BAD_ARGUMENT;
+    }
+    return launch_status();
 }
 
 // The same in float32: a tile of 64 slots by 64 outputs, K in steps of 16 through LDS, every output

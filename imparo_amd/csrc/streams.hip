@@ -8,6 +8,7 @@
 // Sums in float32, in an order that the width alone decides.
 #include "common.h"
 #include "api.h"
+#include "moe_route.h"
 
 #define STREAM_MAX 16              // copies
 #define STREAM_MAX_WIDTH 16384
@@ -234,6 +235,248 @@ __global__ __launch_bounds__(1024) void k_stream_norm(
             stream_store<V>((float*)out + dst, y);
         }
     }
+}
+
+// ---------------------------------------------------------------- a decode step's rows
+// The same for the few rows of a decode step, whose sublayer left slices of a product, or experts' rows that lie by entry
+// (token * used + place in the token's list: no places to look up first). Such a launch is a chain of trips to memory, so everything
+// is asked for at once, the small constants through the scalar cache, and the rows' sums run as in k_stream_norm, so that a row has the same bits.
+// ROUTE: the row goes on through a mixture's router in the same launch: its outputs (at most 16) are matrix products over the
+// rounded row in LDS, chunks of 128 of K summed as the product of few rows sums them (decode_rows.hip: a wave a chunk, or two, the
+// waves' sums in order), and the first wave chooses. 8 rows of 1,024 on four copies, one of 33 such launches of a step: behind a
+// mixture 6.0 -> 4.7 us; behind attention, with a router of 8 outputs, 7.7, where norm, product and choice took 6.0 + 4.2 + 4.0.
+// 8 chats of a mixture of 8 experts 32.0 -> 28.4 ms.
+#define STREAM_STEP_DELTAS 4
+#define STREAM_STEP_TOP 8
+#define STREAM_STEP_ROUTER 16
+struct StreamRouter {
+    const bf16_t* w;            // [n_router, width]
+    const float* bias;          // [n_router] or null
+    const float* correction;    // [n_router] or null
+    int32_t* choice;            // [rows, top + always]
+    float* weight;
+    int n_router, top, scoring;
+    MoeRouteRules rules;
+};
+
+template <int S, bool MOE, bool ROUTE>
+__global__ __launch_bounds__(ROUTE ? 512 : 1024) void k_stream_step(
+    const float* x, int in_streams, float* x_out, const float* __restrict__ delta, int n_delta, size_t delta_stride,
+    StreamExperts moe, int streams, const float* __restrict__ mix, const float* __restrict__ join,
+    const float* __restrict__ read, int norm, const float* __restrict__ weight, const float* __restrict__ bias, float eps,
+    void* __restrict__ out, int out_is_bf16, int width, StreamRouter router) {
+    typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int V = 4;
+    __shared__ float scratch[16];
+    __shared__ __attribute__((aligned(16))) bf16_t row_lds[ROUTE ? 2048 : 8];
+    __shared__ float z_part[ROUTE ? 8 : 1][STREAM_STEP_ROUTER];
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const size_t t = blockIdx.x;
+    const int c = tid * V;                               // (a thread has one piece: blocks have width / 4 threads)
+    StreamPiece<V> v[S], y[MOE ? STREAM_STEP_TOP : STREAM_STEP_DELTAS];
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        v[s] = stream_load<V>(x + (t * in_streams + (in_streams == 1 ? 0 : min(s, streams - 1))) * width + c);
+    if constexpr (MOE) {
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_TOP; ++k) y[k] = stream_load<V>(moe.y + (t * moe.top + min(k, moe.top - 1)) * width + c);
+    } else {
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_DELTAS; ++k) y[k] = stream_load<V>(delta + min(k, n_delta - 1) * delta_stride + t * width + c);
+    }
+    const float* some = weight ? weight : bias ? bias : x;
+    const StreamPiece<V> w = stream_load<V>((weight ? weight : some) + c), b = stream_load<V>((bias ? bias : some) + c);
+    u32x4 rw[ROUTE ? 2 : 1][4];
+    const int waves = blockDim.x / WAVE, r16 = lane & 15, g = lane >> 4;
+    if constexpr (ROUTE) {                               // two chunks of 128 of the router's rows a wave
+        const bf16_t* at = router.w + (size_t)min(r16, router.n_router - 1) * width + g * 8;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) rw[h][s] = *reinterpret_cast<const u32x4*>(at + (wave + h * waves) * 128 + s * 32);
+    }
+    float mixes[S][S], joins[S], reads[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+        const int from = min(i, streams - 1);
+        joins[i] = i >= streams ? 0.f : join ? join[from] : 1.f;
+        reads[i] = i >= streams ? 0.f : read ? read[from] : 1.f;
+#pragma unroll
+        for (int to = 0; to < S; ++to)
+            mixes[i][to] = (i >= streams || to >= streams) ? 0.f : mix ? mix[from * streams + min(to, streams - 1)] : i == to ? 1.f : 0.f;
+    }
+    float d[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) d[i] = 0.f;
+    if constexpr (MOE) {
+        float wt[STREAM_STEP_TOP];
+        bool passes[STREAM_STEP_TOP];
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_TOP; ++k) {
+            const size_t entry = t * moe.top + min(k, moe.top - 1);
+            const int e = moe.choice[entry];
+            wt[k] = moe.weight ? moe.weight[entry] : 1.0f;
+            passes[k] = e < 0 || e >= moe.n_experts;
+        }
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_TOP; ++k)
+            if (k < moe.top && passes[k]) {              // an expert that hands its input on
+#pragma unroll
+                for (int i = 0; i < V; ++i)
+                    y[k].e[i] = moe.h_is_bf16 ? load_f32<bf16_t>((const bf16_t*)moe.h, t * width + c + i)
+                                              : load_f32<float>((const float*)moe.h, t * width + c + i);
+            }
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_TOP; ++k)
+#pragma unroll
+            for (int i = 0; i < V; ++i) d[i] = k < moe.top ? fmaf(wt[k], y[k].e[i], d[i]) : d[i];
+    } else {
+        float e[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) e[i] = 0.f;
+#pragma unroll
+        for (int k = 0; k < STREAM_STEP_DELTAS; ++k)
+#pragma unroll
+            for (int i = 0; i < V; ++i) e[i] += k < n_delta ? y[k].e[i] : 0.f;
+#pragma unroll
+        for (int i = 0; i < V; ++i) d[i] += e[i];
+    }
+    float u[V];
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) u[i] = 0.f;
+#pragma unroll
+    for (int to = 0; to < S; ++to) {
+        float n[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) n[i] = joins[to] * d[i];
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int i = 0; i < V; ++i) n[i] = fmaf(mixes[s][to], v[s].e[i], n[i]);
+        if (x_out && to < streams) stream_store<V>(x_out + (t * streams + to) * width + c, n);
+#pragma unroll
+        for (int i = 0; i < V; ++i) u[i] = fmaf(reads[to], n[i], u[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) sum += norm == STREAM_NORM_RMS ? u[i] * u[i] : u[i];
+    float mean = 0.f, scale = 1.0f;
+    if (norm == STREAM_NORM_RMS) {
+        scale = 1.0f / sqrtf(block_sum(sum, scratch) / (float)width + eps);
+    } else if (norm == STREAM_NORM_LAYER) {
+        mean = block_sum(sum, scratch) / (float)width;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < V; ++i) ss = fmaf(u[i] - mean, u[i] - mean, ss);
+        scale = 1.0f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+    }
+    float o[V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        o[i] = (u[i] - mean) * scale;
+        if (weight) o[i] *= w.e[i];
+        if (bias) o[i] += b.e[i];
+    }
+    const size_t dst = t * width + c;
+    const uint2 packed = make_uint2(f32x2_to_bf16x2(o[0], o[1]), f32x2_to_bf16x2(o[2], o[3]));
+    if (out_is_bf16) *reinterpret_cast<uint2*>((bf16_t*)out + dst) = packed;
+    else stream_store<V>((float*)out + dst, o);
+    if constexpr (ROUTE) {
+        *reinterpret_cast<uint2*>(row_lds + c) = packed;
+        __syncthreads();
+        // every column of the products is this row; the router's rows are theirs. Up to eight chunks each has a sum of its own, of
+        // sixteen a wave adds its two
+        const bool pairs = 2 * waves > 8;
+        f32x4 acc[2];
+        acc[0] = acc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (h == 1 && pairs) acc[1] = acc[0];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const u32x4 a = *reinterpret_cast<const u32x4*>(row_lds + (wave + h * waves) * 128 + s * 32 + g * 8);
+                acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, rw[h][s]), __builtin_bit_cast(bf16x8, a), acc[h], 0, 0, 0);
+            }
+        }
+        if (r16 == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (!pairs) z_part[wave][4 * g + i] = acc[0][i];
+                z_part[pairs ? wave : wave + waves][4 * g + i] = acc[1][i];
+            }
+        }
+        __syncthreads();
+        if (wave == 0) {
+            const int parts = pairs ? waves : 2 * waves, e = min(lane, router.n_router - 1);
+            float p[8];                                  // (asked for together)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) p[q] = z_part[min(q, parts - 1)][e];
+            float z = p[0];
+#pragma unroll
+            for (int q = 1; q < 8; ++q) z = q < parts ? z + p[q] : z;
+            if (router.bias) z = __fadd_rn(z, router.bias[e]);
+            moe_route_lanes(z, router.correction, router.choice, router.weight, (int)t, router.n_router, router.top, router.scoring,
+                            router.rules, nullptr);
+        }
+    }
+}
+
+// Which steps imparo_stream_step takes: few rows of copies that a block keeps in registers, a piece of four a thread.
+extern "C" int imparo_stream_step_takes(int n_rows, int streams, int width, int n_delta, int top) {
+    return n_rows >= 1 && n_rows <= 16 && streams >= 1 && streams <= 4 && width >= 256 && width <= 4096 && width % 256 == 0 &&
+           (top > 0 ? top <= STREAM_STEP_TOP && n_delta == 0 : n_delta >= 1 && n_delta <= STREAM_STEP_DELTAS);
+}
+// ... and whether a router of so many outputs rides: widths whose chunks of 128 come out as the product of few rows sums them.
+extern "C" int imparo_stream_step_routes(int width, int n_router, int top) {
+    return width % 256 == 0 && (width <= 1024 || width == 2048) && n_router >= 1 && n_router <= STREAM_STEP_ROUTER && top >= 1 &&
+           top <= n_router;
+}
+
+extern "C" int imparo_stream_step(const float* x, int in_streams, float* x_out, const float* delta, int n_delta, const float* y,
+                                  const void* h, int h_dtype, const int32_t* choice, const float* choice_weight, int top,
+                                  int n_experts, int n_rows, int streams, const float* mix, const float* join, const float* read,
+                                  int norm, const float* weight, const float* bias, float eps, void* out, int out_dtype,
+                                  int width, const void* router_w, const float* router_bias, const float* correction,
+                                  int n_router, int route_top, int scoring, int normalize, float route_scale, int always,
+                                  int32_t* route_choice, float* route_weight, imparo_stream stream) {
+    if (!x || !x_out || !out || n_rows < 0 || n_delta < 0 || (n_delta && !delta) || (!y && top) || (y && top < 1)) return IMPARO_BAD_ARGUMENT;
+    if (n_rows == 0) return IMPARO_OK;
+    if (!imparo_stream_step_takes(n_rows, streams, width, n_delta, y ? top : 0)) return IMPARO_BAD_ARGUMENT;
+    if ((in_streams != streams && in_streams != 1) || (in_streams != streams && x_out == x)) return IMPARO_BAD_ARGUMENT;
+    if (y && (!h || !choice || n_experts < 0 || (h_dtype != IMPARO_F32 && h_dtype != IMPARO_BF16))) return IMPARO_BAD_ARGUMENT;
+    if (norm < STREAM_NORM_NONE || norm > STREAM_NORM_LAYER) return IMPARO_BAD_ARGUMENT;
+    if (out_dtype != IMPARO_F32 && out_dtype != IMPARO_BF16) return IMPARO_BAD_ARGUMENT;
+    if (((uintptr_t)x | (uintptr_t)x_out | (uintptr_t)delta | (uintptr_t)y | (uintptr_t)out | (uintptr_t)weight | (uintptr_t)bias |
+         (uintptr_t)router_w) & 15)
+        return IMPARO_BAD_ARGUMENT;
+    const MoeRouteRules rules{n_router, 1, 1, normalize, route_scale, always};
+    const StreamRouter router{(const bf16_t*)router_w, router_bias, correction, route_choice, route_weight, n_router, route_top, scoring, rules};
+    if (router_w) {
+        if (!imparo_stream_step_routes(width, n_router, route_top) || out_dtype != IMPARO_BF16) return IMPARO_BAD_ARGUMENT;
+        if (!route_choice || !route_weight || always < 0 || route_top + always > MOE_MAX_USED || !(route_scale == route_scale))
+            return IMPARO_BAD_ARGUMENT;
+        if (scoring < MOE_SCORE_SOFTMAX || scoring > MOE_SCORE_CHOSEN) return IMPARO_BAD_ARGUMENT;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    const StreamExperts moe{y, h, choice, choice_weight, nullptr, h_dtype == IMPARO_BF16, top, n_experts};
+    const size_t stride = (size_t)n_rows * width;
+    const int out_is_bf16 = out_dtype == IMPARO_BF16;
+#define STREAM_STEP(S, MOE, ROUTE)                                                                                   \
+    k_stream_step<S, MOE, ROUTE><<<n_rows, width / 4, 0, s>>>(x, in_streams, x_out, delta, n_delta, stride, moe, streams, mix, join, \
+                                                              read, norm, weight, bias, eps, out, out_is_bf16, width, router)
+#define STREAM_STEP_OF(S)                                                                                            \
+    if (y && router_w) STREAM_STEP(S, true, true);                                                                   \
+    else if (y) STREAM_STEP(S, true, false);                                                                         \
+    else if (router_w) STREAM_STEP(S, false, true);                                                                  \
+    else STREAM_STEP(S, false, false)
+    if (streams == 1) { STREAM_STEP_OF(1); }
+    else if (streams == 2) { STREAM_STEP_OF(2); }
+    else { STREAM_STEP_OF(4); }
+#undef STREAM_STEP_OF
+#undef STREAM_STEP
+    return launch_status();
 }
 
 extern "C" int imparo_stream_max() { return STREAM_MAX; }

@@ -89,6 +89,15 @@ _SIGNATURES = {
     # rows, streams, mix, join, read, norm, weight, bias, eps, out, out_dtype, n_out, width, stream
     "imparo_stream_norm": [P, I, P, P, I, P, P, I, P, P, P, I, I, I, P, I, P, P, P, I, P, P, F, P, I, I, I, P],
     "imparo_stream_max": [],
+    "imparo_stream_step_takes": [I, I, I, I, I],
+    "imparo_stream_step_routes": [I, I, I],
+    # x, in_streams, x_out, delta, n_delta, y, h, h_dtype, choice, choice_weight, top, n_experts, n_rows, streams, mix, join, read,
+    # norm, weight, bias, eps, out, out_dtype, width, router_w, router_bias, correction, n_router, route_top, scoring, normalize,
+    # route_scale, always, route_choice, route_weight, stream
+    "imparo_stream_step": [P, I, P, P, I, P, P, I, P, P, I, I, I, I, P, P, P, I, P, P, F, P, I, I, P, P, P, I, I, I, I, F, I, P, P, P],
+    "imparo_moe_direct_takes": [I, I, I],
+    # a, a_ld, own_rows, choice, n_tokens, used, n_experts, w, out, out_dtype, n, k, epilogue, limits, alpha, stream
+    "imparo_moe_gemm_direct": [P, I, I, P, I, I, I, P, P, I, I, I, I, P, F, P],
     # table, bigram, dtype, ids, positions, row_of_token, seg_start, seg_len, slot, state, x, n_tokens, n_rows, width, vocab,
     # n_slots, buckets, mul_prev, mul_cur, scale, advance, stream
     "imparo_embed_bigram": [P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, I, c_int64, c_int64, F, I, P],

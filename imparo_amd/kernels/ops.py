@@ -133,14 +133,15 @@ def stream_max() -> int:
 def stream_norm(x: torch.Tensor, norm: str, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], eps: float,
                 out: torch.Tensor, delta=None, mix: Optional[torch.Tensor] = None, join: Optional[torch.Tensor] = None,
                 read: Optional[torch.Tensor] = None, x_out: Optional[torch.Tensor] = None,
-                rows: Optional[torch.Tensor] = None, streams: Optional[int] = None) -> torch.Tensor:
+                rows: Optional[torch.Tensor] = None, streams: Optional[int] = None, route=None) -> torch.Tensor:
     """A norm ("none", "rms" or "layer") of a residual stream that is kept as copies of a row, together with what the
     sublayer before it left pending: x'_t = sum_s mix[s, t] x_s + join[t] delta, out = norm(sum_t read[t] x'_t).
 
     x float32 [n, streams, width], or [n, width] where all copies are equal still (or the only one). `delta`: a tensor
     [n, width] or [slices, n, width], or what a routed feed-forward left to be combined (an object with y, h, choice,
     weight, slot_of_entry, n_experts, extra). x_out [n, streams, width] (or x's own shape, for one copy) receives x';
-    without it the stream stays as it is. mix None: the identity; join, read None: ones. `rows`: those rows only."""
+    without it the stream stays as it is. mix None: the identity; join, read None: ones. `rows`: those rows only. `route`: a
+    mixture's router that the normed rows go on through where `stream_step_routes` says so of this very call."""
     n_x, width = x.shape[0], x.shape[-1]
     in_streams = x.shape[1] if x.dim() == 3 else 1
     if streams is None:
@@ -167,6 +168,26 @@ def stream_norm(x: torch.Tensor, norm: str, weight: Optional[torch.Tensor], bias
         if rows is not None or delta is None:
             raise KernelArgumentError("stream_norm: the copies are written for every row, and where something joins them")
         _dev(x_out, "stream out", torch.float32, (n_x, width) if streams == 1 and x_out.dim() == 2 else (n_x, streams, width))
+    if x_out is not None and _stream_step_takes(x, out, delta, slices, n_delta, streams, weight, bias, x_out):
+        by_entry = moe[0:5] + moe[6:] if moe[0] else (0, 0, 0, 0, 0, 0, 0)
+        router = (0, 0, 0, 0, 0, 0, 0, 0.0, 0, 0, 0)
+        if route is not None:
+            _code(out, "normed")
+            used = route.top + route.always
+            router = (_dev(route.weight, "router", torch.bfloat16, (route.weight.shape[0], width)),
+                      _dev(route.bias, "router bias", torch.float32, (route.weight.shape[0],)),
+                      _dev(route.correction, "correction", torch.float32, (route.weight.shape[0],)), route.weight.shape[0], route.top,
+                      MOE_SCORINGS[route.scoring], int(route.normalize), float(route.scale), route.always,
+                      _dev(route.choice, "choice", torch.int32, (n_x, used)), _dev(route.shares, "choice weights", torch.float32, (n_x, used)))
+        _check(library().imparo_stream_step(
+            _dev(x, "stream", torch.float32), in_streams, x_out.data_ptr(), 0 if slices is None else slices.data_ptr(), n_delta,
+            *by_entry, n_x, streams, _dev(mix, "mix", torch.float32, (streams, streams)), _dev(join, "join", torch.float32, (streams,)),
+            _dev(read, "read", torch.float32, (streams,)), STREAM_NORMS[norm], _dev(weight, "norm weight", torch.float32, (width,)),
+            _dev(bias, "norm bias", torch.float32, (width,)), float(eps), _dev(out, "normed", None, (n_out, width)),
+            _code(out, "normed"), width, *router, _stream()), "stream_step")
+        return out
+    if route is not None:
+        raise KernelArgumentError("stream_norm: no router rides with this call")
     _check(library().imparo_stream_norm(
         _dev(x, "stream", torch.float32), in_streams, 0 if x_out is None else x_out.data_ptr(),
         0 if slices is None else slices.data_ptr(), n_delta, *moe, n_x, _dev(rows, "rows", torch.int32), streams,
@@ -175,6 +196,28 @@ def stream_norm(x: torch.Tensor, norm: str, weight: Optional[torch.Tensor], bias
         _dev(bias, "norm bias", torch.float32, (width,)), float(eps), _dev(out, "normed", None, (n_out, width)),
         _code(out, "normed"), n_out, width, _stream()), "stream_norm")
     return out
+
+
+def _stream_step_takes(x, out, delta, slices, n_delta: int, streams: int, weight, bias, x_out) -> bool:
+    """Whether stream_norm's call goes to the kernel of a decode step's rows."""
+    top = 0
+    if delta is not None and not isinstance(delta, torch.Tensor):
+        if not getattr(delta, "by_entry", False):
+            return False
+        top = delta.choice.shape[1]
+    return (bool(library().imparo_stream_step_takes(x.shape[0], streams, x.shape[-1], n_delta, top))
+            and not any(t is not None and t.data_ptr() % 16 for t in (x, out, slices, weight, bias, x_out, delta.y if top else None)))
+
+
+def stream_step_routes(x: torch.Tensor, delta, streams: int, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor],
+                       router: torch.Tensor, top: int) -> bool:
+    """Whether `stream_norm`, given these, whole aligned outputs and an x_out, takes a router [n, width] of `top` choices along."""
+    if router.dtype != torch.bfloat16 or not router.is_contiguous() or router.data_ptr() % 16 or router.dim() != 2 or router.shape[1] != x.shape[-1]:
+        return False
+    slices = delta if delta is None or isinstance(delta, torch.Tensor) else delta.extra
+    n_delta = 0 if slices is None else slices.shape[0] if slices.dim() == 3 else 1
+    return (bool(library().imparo_stream_step_routes(x.shape[-1], router.shape[0], int(top))) and delta is not None
+            and _stream_step_takes(x, None, delta, slices, n_delta, streams, weight, bias, None))
 
 
 def place_tokens(ids: torch.Tensor, dst: torch.Tensor, src: torch.Tensor, src_index: torch.Tensor,
@@ -1167,6 +1210,31 @@ def moe_gemm(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, tiles: torch.T
         _dev(tiles, "tiles", torch.int32), tiles.shape[0], int(tile_rows), n, k, MOE_EPILOGUES[epilogue],
         _dev(limits, "experts' bounds", torch.float32), float(alpha), _dev(weight, "choice weights", torch.float32),
         0 if weight is None else weight.numel(), _stream()), "moe_gemm")
+    return out
+
+
+def moe_direct_takes(n_tokens: int, used: int, n_experts: int) -> bool:
+    """Whether `moe_gemm_direct` is for a step of so many tokens that use so many of the experts each."""
+    return bool(library().imparo_moe_direct_takes(int(n_tokens), int(used), int(n_experts)))
+
+
+def moe_gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, choice: torch.Tensor, own_rows: bool = False,
+                    epilogue: Optional[str] = None, limits: Optional[torch.Tensor] = None, alpha: float = 1.0) -> torch.Tensor:
+    """`moe_gemm` without a plan, for few tokens: out[entry] = epilogue(a[row] . w[choice of the entry]^T), entry = token * used +
+    place in `choice` [tokens, used], row the entry, or with `own_rows` the token. Entries of no expert are left as they are."""
+    n_experts, n, k = w.shape
+    tokens, used = choice.shape
+    gated = epilogue == "gated"
+    if a.dim() != 2 or a.shape[1] != k or a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.shape[0] < (tokens if own_rows else tokens * used):
+        raise KernelArgumentError(f"moe_gemm_direct: a is {tuple(a.shape)} {a.dtype}, the experts' matrices {tuple(w.shape)} {w.dtype}")
+    if tuple(out.shape) != (tokens * used, n // 2 if gated else n) or (gated and (n % 64 or (limits is not None and limits.numel() != n_experts))):
+        raise KernelArgumentError(f"moe_gemm_direct: out is {tuple(out.shape)}; gated experts have rows in blocks of 64 and a bound each")
+    if epilogue not in MOE_EPILOGUES:
+        raise KernelArgumentError(f"moe_gemm_direct: unknown epilogue {epilogue!r}")
+    _check(library().imparo_moe_gemm_direct(
+        _dev(a, "moe_gemm a"), a.stride(0), int(bool(own_rows)), _dev(choice, "choice", torch.int32), tokens, used, n_experts,
+        _dev(w, "experts' matrices"), _dev(out, "moe_gemm out"), _code(out, "moe_gemm out"), n, k, MOE_EPILOGUES[epilogue],
+        _dev(limits, "experts' bounds", torch.float32), float(alpha), _stream()), "moe_gemm_direct")
     return out
 
 

@@ -201,3 +201,21 @@ class RowsToCombine:
     slot_of_entry: torch.Tensor
     n_experts: int
     extra: Optional[torch.Tensor] = None
+    by_entry: bool = False          # slot_of_entry is the identity: an entry's row is its own number, token * top + place
+
+
+@dataclass
+class RouterRide:
+    """A mixture's router that the norm before it may take into its launch: its matrix and rules, and where a token's choices
+    and their weights go. `done`: the norm did."""
+    weight: torch.Tensor
+    bias: Optional[torch.Tensor]
+    correction: Optional[torch.Tensor]
+    top: int
+    always: int
+    scoring: str
+    normalize: bool
+    scale: float
+    choice: torch.Tensor
+    shares: torch.Tensor
+    done: bool = False

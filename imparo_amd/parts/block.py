@@ -149,6 +149,9 @@ class HyperBlock:
         self.ffn_norm, self.ffn, self.ffn_link = parts.get("ffn_norm"), parts.get("ffn"), parts.get("ffn_link")
         if len({self.ffn is None, self.ffn_norm is None, self.ffn_link is None}) > 1:
             raise ValueError("a block has a feed-forward, the norm before it and its link, or none of them")
+        # whether the feed-forward's router may ride with the norm: both have to say so of the methods they run
+        self.routes = (emits(self.ffn_norm, "routes", "forward_linked")
+                       and all(emits(self.ffn, "router_ride", run) for run in ("forward", "forward_parts", "_parts", "_rows")))
 
     def cache_spec(self, page_size: int):
         return self.mixer.cache_spec(page_size)
@@ -158,9 +161,11 @@ class HyperBlock:
         res.pending, res.link = self.mixer.forward(ctx, site, owns_cache, h), self.mixer_link
         if self.ffn is not None:
             # (a buffer of its own: the feed-forward may leave this input to be read by the launch of the next norm)
-            n = self.ffn_norm.forward_linked(ctx, res, self.ffn_link, self.ffn.in_dtype, name="normed_ffn")
+            ride = self.ffn.router_ride(ctx, res.x.shape[0]) if self.routes else None
+            more = {} if ride is None else dict(route=ride)
+            n = self.ffn_norm.forward_linked(ctx, res, self.ffn_link, self.ffn.in_dtype, name="normed_ffn", **more)
             run = getattr(self.ffn, "forward_parts", None) or self.ffn.forward
-            res.pending, res.link = run(ctx, n), self.ffn_link
+            res.pending, res.link = run(ctx, n, routed=ride) if ride is not None and ride.done else run(ctx, n), self.ffn_link
 
     def can_emit(self) -> bool:
         return False          # the step program knows the pre-norm block only

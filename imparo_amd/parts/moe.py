@@ -49,7 +49,7 @@ import torch
 from ..config.plan import PartSpec
 from ..kernels import ops
 from ..weights.loader import TensorDecl
-from .base import Declared, RowsToCombine, StepContext
+from .base import Declared, RouterRide, RowsToCombine, StepContext
 from .linear import Linear, place_matrix, place_projection, place_vector
 from .registry import part_class, register_part
 
@@ -156,6 +156,7 @@ class RoutedExperts:
             limits.append(float(shared.get("limit", 0.0)))
         self.used, self.n_experts = self.top + self.always, self.experts + self.always      # a token's, and all of them
         self.limits = place_vector(torch.tensor(limits), device) if limit else None
+        self.fused = False
         if not self.experts:
             self.up = self.down = None
             return
@@ -181,6 +182,8 @@ class RoutedExperts:
         self.hidden_rows = F
         self.up = place_matrix(up, engine_dtype, device)
         self.down = place_matrix(stacked["down"], engine_dtype, device)
+        # where an entry's row is its own number: the products of few tokens (as many entries as those take)
+        self.own_slots = torch.arange(128, dtype=torch.int32, device=device)
 
     @classmethod
     def _joins_experts(cls, spec: PartSpec, shared: PartSpec) -> bool:
@@ -210,13 +213,24 @@ class RoutedExperts:
         None where that result is multiplied by a gate first, or the experts' weights are spent on their input."""
         return None if self.weigh == "input" or (self.shared is not None and self.shared_gated) else self._parts
 
-    def _parts(self, ctx: StepContext, n: torch.Tensor) -> RowsToCombine:
+    def router_ride(self, ctx: StepContext, T: int) -> Optional[RouterRide]:
+        """The router, for the norm that hands this part its rows; None where it goes a launch of its own. The products then go
+        by the tokens' choices: the plan, which takes all tokens, would be a launch again."""
+        if (self.shared is not None or self.group_count > 1 or not self.fused or self.weigh != "output"
+                or not ops.moe_direct_takes(T, self.used, self.n_experts)):
+            return None
+        ws = ctx.workspace
+        return RouterRide(self.router.weight, self.router.bias, self.correction, self.top, self.always, self.scoring, self.normalize,
+                          self.route_scale, ws.get("moe_choice", (T, self.used), torch.int32), ws.get("moe_weight", (T, self.used), torch.float32))
+
+    def _parts(self, ctx: StepContext, n: torch.Tensor, routed: Optional[RouterRide] = None) -> RowsToCombine:
         extra: list = []
-        r = self._rows(ctx, n, extra if self.shared is not None else None)
+        r = self._rows(ctx, n, extra if self.shared is not None else None, routed)
         r.extra = extra[0] if extra else None
         return r
 
-    def _rows(self, ctx: StepContext, n: torch.Tensor, shared_out: Optional[list] = None) -> RowsToCombine:
+    def _rows(self, ctx: StepContext, n: torch.Tensor, shared_out: Optional[list] = None,
+              routed: Optional[RouterRide] = None) -> RowsToCombine:
         T, top, used, X = n.shape[0], self.top, self.used, self.n_experts
         ws = ctx.workspace
         rules = dict(scoring=self.scoring, n_router=self.n_router, groups=self.group_count, keep=self.group_keep,
@@ -228,12 +242,18 @@ class RoutedExperts:
                 shared_out.append(self.shared.forward(ctx, n))
             finally:
                 ctx.stream = stream
-        z = self.router(ctx, n, torch.float32, "router_logits")
+        z = None if routed is not None else self.router(ctx, n, torch.float32, "router_logits")
         if shared_out is not None:
             shared_out.append(z)
         choice = ws.get("moe_choice", (T, used), torch.int32)
         weight = ws.get("moe_weight", (T, used), torch.float32)
         entries = T * used
+        if routed is not None:
+            hidden = ws.get("moe_hidden", (entries, self.hidden_rows), self.down.dtype)
+            y = ws.get("moe_y", (entries, self.width), torch.float32)
+            ops.moe_gemm_direct(n, self.up, hidden, choice, own_rows=True, epilogue="gated", limits=self.limits, alpha=self.alpha)
+            ops.moe_gemm_direct(hidden, self.down, y, choice)
+            return RowsToCombine(y, n, choice, weight, self.own_slots[:entries], X, by_entry=True)
         slot_of_entry = ws.get("moe_slot_of_entry", (entries,), torch.int32)
         y = ws.get("moe_y", (entries, self.width), torch.float32)
         if X:

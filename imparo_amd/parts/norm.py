@@ -34,11 +34,12 @@ from .registry import register_part
 class LinkedNorm:
     """What a norm over whole rows needs to read a stream kept as several copies of a row (hyper-connections): the
     class says its `row_norm()`, (kind, weight, bias, eps) as the stream kernel takes it."""
+    routes = True         # `forward_linked` may take a mixture's router into its launch
 
     def row_norm(self):
         raise NotImplementedError
 
-    def _read(self, ctx: StepContext, res: Residual, link, out: torch.Tensor, rows: Optional[torch.Tensor] = None):
+    def _read(self, ctx: StepContext, res: Residual, link, out: torch.Tensor, rows: Optional[torch.Tensor] = None, route=None):
         """norm(sum_t read[t] x'_t) with x' the copies behind the pending add, into `out`; without `rows` the copies
         are moved on. `link` None: the plain sum of the copies is read."""
         kind, weight, bias, eps = self.row_norm()
@@ -54,16 +55,21 @@ class LinkedNorm:
         moved = None
         if rows is None:
             moved = ctx.workspace.get("streams", (res.x.shape[0], n, res.x.shape[1]), torch.float32)
+        if (route is not None and rows is None and out.dtype == torch.bfloat16
+                and ops.stream_step_routes(x, res.pending, n, weight, bias, route.weight, route.top)):
+            route.done = True
         ops.stream_norm(x, kind, weight, bias, eps, out, delta=res.pending, mix=res.link.mix, join=res.link.join,
-                        read=None if link is None else link.read, x_out=moved, rows=rows)
+                        read=None if link is None else link.read, x_out=moved, rows=rows,
+                        route=route if route is not None and route.done else None)
         if rows is None:
             res.streams, res.pending, res.link = moved, None, None
         return out
 
     def forward_linked(self, ctx: StepContext, res: Residual, link, out_dtype: torch.dtype,
-                       name: str = "normed") -> torch.Tensor:
-        """`forward` for a sublayer with a link of its own: the normed sum of the copies, weighed by its `read`."""
-        return self._read(ctx, res, link, ctx.workspace.get(name, tuple(res.x.shape), out_dtype))
+                       name: str = "normed", route=None) -> torch.Tensor:
+        """`forward` for a sublayer with a link of its own: the normed sum of the copies, weighed by its `read`. `route`: the
+        sublayer's router, which the launch takes along where it can."""
+        return self._read(ctx, res, link, ctx.workspace.get(name, tuple(res.x.shape), out_dtype), route=route)
 
 
 class RmsNorm(LinkedNorm):

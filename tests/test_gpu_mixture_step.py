@@ -1,0 +1,84 @@
+"""A mixture's decode step: the norm that takes the router along, and products that go by the tokens' choices. Both against the
+launches they stand for, whose bits they have."""
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def ops():
+    from imparo_amd.kernels import ops
+    return ops
+
+
+def rnd(*shape, seed=0, dtype=torch.float32):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV)
+
+
+@pytest.mark.parametrize("T,experts,used", [(1, 9, 5), (8, 9, 5), (16, 24, 8), (5, 2, 1), (16, 3, 3)])
+@pytest.mark.parametrize("F,E", [(32, 8), (768, 1024), (96, 200), (160, 2056)])
+def test_products_by_the_tokens_choices_have_the_planned_bits(T, experts, used, F, E):
+    choice = torch.stack([torch.randperm(experts + 1, generator=torch.Generator().manual_seed(i))[:used] for i in range(T)])
+    choice[choice == experts] = experts + 7                      # (an expert past the last one: nobody's entry)
+    choice = choice.to(torch.int32).to(DEV)
+    n, up, down = rnd(T, E, seed=1, dtype=torch.bfloat16), rnd(experts, 2 * F, E, seed=2, dtype=torch.bfloat16), rnd(experts, E, F, seed=3, dtype=torch.bfloat16)
+    limits = torch.linspace(0.5, 9.0, experts, device=DEV)
+    limits[0] = 0.0
+    entries = T * used
+    rows = 16
+    tiles = torch.empty(ops().moe_max_tiles(entries, experts, rows), 3, dtype=torch.int32, device=DEV)
+    slot, entry = (torch.zeros(entries, dtype=torch.int32, device=DEV) for _ in range(2))
+    ops().moe_plan(choice, experts, rows, slot, entry, tiles)
+    hidden, y = torch.zeros(entries, F, dtype=torch.bfloat16, device=DEV), torch.zeros(entries, E, device=DEV)
+    ops().moe_gemm(n, up, hidden, tiles, rows, entry, gather_div=used, epilogue="gated", limits=limits, alpha=1.702)
+    ops().moe_gemm(hidden, down, y, tiles, rows)
+    hidden_d, y_d = torch.full((entries, F), 3.0, dtype=torch.bfloat16, device=DEV), torch.full((entries, E), 7.0, device=DEV)
+    ops().moe_gemm_direct(n, up, hidden_d, choice, own_rows=True, epilogue="gated", limits=limits, alpha=1.702)
+    ops().moe_gemm_direct(hidden_d, down, y_d, choice)
+    has = slot >= 0
+    at = slot[has].long()
+    assert torch.equal(hidden_d[has], hidden[at]) and torch.equal(y_d[has], y[at])
+    assert bool((hidden_d[~has] == 3.0).all()) and bool((y_d[~has] == 7.0).all())
+
+
+@pytest.mark.parametrize("T,width,streams,in_streams", [(1, 256, 1, 1), (8, 1024, 4, 4), (16, 2048, 3, 1), (3, 768, 2, 2), (5, 4096, 4, 4)])
+@pytest.mark.parametrize("pending", ["one", "slices", "experts"])
+@pytest.mark.parametrize("norm", ["rms", "layer", "none"])
+def test_the_step_norm_and_its_router_have_the_bits_of_their_launches(T, width, streams, in_streams, pending, norm, monkeypatch):
+    x = rnd(T, in_streams, width, seed=1) if in_streams > 1 else rnd(T, width, seed=1)
+    weight, bias = rnd(width, seed=2), (None if norm == "rms" else rnd(width, seed=3))
+    mix, join, read = rnd(streams, streams, seed=4), rnd(streams, seed=5), rnd(streams, seed=6)
+    if pending == "experts":
+        choice = torch.stack([torch.randperm(11, generator=torch.Generator().manual_seed(i))[:6] for i in range(T)]).to(torch.int32).to(DEV)
+        delta = types.SimpleNamespace(y=rnd(T * 6, width, seed=7), h=rnd(T, width, seed=8, dtype=torch.bfloat16), choice=choice,
+                                      weight=rnd(T, 6, seed=9).abs(), slot_of_entry=torch.arange(T * 6, dtype=torch.int32, device=DEV),
+                                      n_experts=9, extra=None, by_entry=True)     # (experts 9 and 10 hand their input on)
+    else:
+        delta = rnd(T, width, seed=7) if pending == "one" else rnd(3, T, width, seed=7)
+    router, top, always = rnd(8, width, seed=10, dtype=torch.bfloat16), 4, 1
+    correction = rnd(8, seed=11)
+    got = []
+    for step in (True, False):
+        out, moved = torch.empty(T, width, dtype=torch.bfloat16, device=DEV), torch.empty(T, streams, width, device=DEV)
+        chosen, shares = torch.empty(T, top + always, dtype=torch.int32, device=DEV), torch.empty(T, top + always, device=DEV)
+        call = dict(delta=delta, mix=mix, join=join, read=read, x_out=moved)
+        rides = ops().stream_step_routes(x, delta, streams, weight, bias, router, top)
+        assert rides == (step and width in (256, 768, 1024, 2048))
+        if rides:
+            ride = types.SimpleNamespace(weight=router, bias=None, correction=correction, top=top, always=always, scoring="chosen",
+                                         normalize=False, scale=1.25, choice=chosen, shares=shares)
+            ops().stream_norm(x, norm, weight, bias, 1e-5, out, route=ride, **call)
+        else:
+            ops().stream_norm(x, norm, weight, bias, 1e-5, out, **call)
+            z = torch.empty(T, 8, device=DEV)
+            ops().gemm(out, router, z)
+            ops().moe_route(z, correction, chosen, shares, top, scoring="chosen", n_router=8, groups=1, keep=1, normalize=False, scale=1.25,
+                            always=always)
+        got.append((out, moved, chosen, shares))
+        monkeypatch.setattr(ops(), "_stream_step_takes", lambda *a: False)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
