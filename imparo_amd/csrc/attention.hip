@@ -298,6 +298,215 @@ __global__ __launch_bounds__(ATT_WAVES * WAVE) void k_attention_wave_f32(
         for (int d = HD + lane; d < out_ld - h * HD; d += WAVE) dst[d] = 0.f;
 }
 
+// The same again for few tokens (a decode step): one wave's walk leaves the chip idle behind its chain of trips, 5 us a chunk. Of
+// what a walk does only three things are a chain: the running maximum, which is the maximum of all chunks before whatever
+// order it is taken in; the denominator, one multiply-add a chunk; and the weighted sum, one multiply-add a key. So a block has all
+// heads of one kv head of a token, its waves take chunks side by side (scores, their maximum, then the weights under the
+// maximum so far), the values wait in LDS, and a wave a head adds them up in the order of the keys: the same bits. Two tokens
+// over 340 keys, 16 heads of 64 by 8, 27.4 -> 11.3 us, over 4,000 288 -> 85, of 128 50 -> 20 and 557 -> 163, 32 tokens over 340 keys 29.8 ->
+// 16.4; over 40 keys 7.1 -> 6.1. What is left is a CU's way to memory, about 1 us for the keys and values of a chunk. Two float32
+// requests of 333 tokens, 8 decoded, 15.35 -> 14.48 ms.
+template <int HD> struct SplitF32 {
+    static constexpr int WAVES = HD == 64 ? 8 : 4;           // chunks at once, whose rows, keys and then values, fill 136 KB of LDS
+    static constexpr int LD = HD + 4;                        // floats from row to row there: lanes that read a row each meet no bank twice
+};
+template <int HD, int GMAX>
+__global__ __launch_bounds__(SplitF32<HD>::WAVES * WAVE, 1) void k_attention_split_f32(
+    const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, float* __restrict__ out,
+    const int32_t* __restrict__ positions, const int32_t* __restrict__ row_of_token, const int32_t* __restrict__ block_table,
+    int table_stride, int page_size, int heads, int kv_heads, int out_ld, int n_pages, float scale, int window,
+    const ImparoAttentionRule rule) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));    // (arrays of the header's float4 end up in memory here)
+    constexpr int W = SplitF32<HD>::WAVES, LD = SplitF32<HD>::LD, DPL = HD / WAVE;
+    constexpr int PIECES = HD / 4;                           // of a row, and of a lane's share of a chunk
+    extern __shared__ __attribute__((aligned(16))) float values[];       // [W][64][LD]
+    __shared__ __attribute__((aligned(16))) float q_rows[GMAX][HD];
+    __shared__ __attribute__((aligned(16))) float weights[GMAX][W][WAVE];
+    __shared__ float top_of[GMAX][W], sum_of[GMAX][W], corr_of[GMAX][W];
+    __shared__ unsigned long long rows_of[W];                // which keys of a chunk there are
+    const int lane = threadIdx.x & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int t = blockIdx.x / kv_heads, kvh = blockIdx.x - t * kv_heads, G = heads / kv_heads;
+    const int pos = positions[t];
+    const int lo = first_seen(pos, window), keep = rule.keep_first;
+    const int32_t* table = block_table + (size_t)row_of_token[t] * table_stride;
+    // chunk i of the walk starts at 64 i, or behind the first positions that stay at 64 i + gap
+    const int keep_end = (keep + WAVE - 1) / WAVE * WAVE, gap = max(0, lo / WAVE * WAVE - keep_end);
+    const int chunks = pos < 0 ? 0 : (pos - gap) / WAVE + 1;
+    auto start_of = [&](int i) { return i * WAVE < keep_end ? i * WAVE : i * WAVE + gap; };
+    for (int i = threadIdx.x; i < G * HD; i += W * WAVE) q_rows[i / HD][i % HD] = q[((size_t)t * heads + kvh * G) * HD + i];
+    float m[GMAX], l = 0.f, acc[DPL];                        // m of every head in every wave; l and acc of the head that a wave adds up
+#pragma unroll
+    for (int g = 0; g < GMAX; ++g) m[g] = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
+    for (int first = 0; first < chunks; first += W) {
+        const bool busy = first + wave < chunks;             // (the last round: a wave may have none)
+        f32x4 key[PIECES], v[PIECES];
+        bool there = false;
+        if (busy) {
+        const int p = start_of(first + wave) + lane;
+        const int page = table[min(p, pos) / page_size];
+        there = p <= pos && (p >= lo || p < keep) && page >= 0 && page < n_pages;
+        const int row = there ? (page * kv_heads + kvh) * page_size + p % page_size : 0;
+        // 64 lanes ask for 1,024 bytes of neighbouring rows: a row a lane, each instruction would meet 64 lines
+        int at[PIECES];
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int piece = i * WAVE + lane;
+            at[i] = __shfl(row, piece / PIECES) * HD + piece % PIECES * 4;
+        }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) key[i] = *reinterpret_cast<const f32x4*>(k_cache + (size_t)(unsigned)at[i]);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) v[i] = *reinterpret_cast<const f32x4*>(v_cache + (size_t)(unsigned)at[i]);
+        }
+        float* rows_lds = values + (size_t)wave * WAVE * LD;
+        auto put = [&](const f32x4 (&piece)[PIECES]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+                *reinterpret_cast<f32x4*>(rows_lds + (i * WAVE + lane) / PIECES * LD + lane % PIECES * 4) = piece[i];
+        };
+        __syncthreads();                                     // (queries are there; the values before are read)
+        float s[GMAX];
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) s[g] = 0.f;
+        if (busy) {
+        put(key);
+        wave_lds_sync();
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) key[i] = *reinterpret_cast<const f32x4*>(rows_lds + lane * LD + 4 * i);
+        wave_lds_sync();
+        put(v);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+            for (int g = 0; g < GMAX; ++g) {
+                if (g >= G) continue;
+                const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_rows[g][4 * i]);
+                s[g] = fmaf(qv.x, key[i].x, s[g]);
+                s[g] = fmaf(qv.y, key[i].y, s[g]);
+                s[g] = fmaf(qv.z, key[i].z, s[g]);
+                s[g] = fmaf(qv.w, key[i].w, s[g]);
+            }
+        }
+        const unsigned long long keys = __ballot(there);
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) {
+            if (g >= G) continue;
+            s[g] *= scale;
+            if (rule.softcap > 0.f) s[g] = rule.softcap * tanhf(s[g] / rule.softcap);
+            if (!there) s[g] = -INFINITY;
+            const float top = wave_max(s[g]);
+            if (lane == 0) top_of[g][wave] = top;          // (of no keys: -inf)
+        }
+        if (lane == 0) rows_of[wave] = keys;
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < GMAX; ++g) {
+            if (g >= G) continue;
+            float before = m[g], all = m[g];
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                const float top = top_of[g][w];
+                before = w < wave ? fmaxf(before, top) : before;
+                all = fmaxf(all, top);
+            }
+            const float m_new = fmaxf(before, top_of[g][wave]);
+            const float pe = there ? expf(s[g] - m_new) : 0.f;
+            const float corr = (before == -INFINITY) ? 0.f : expf(before - m_new);
+            const float sum = wave_sum(pe);
+            weights[g][wave][lane] = pe;
+            if (lane == 0) sum_of[g][wave] = sum, corr_of[g][wave] = corr;
+            m[g] = all;
+        }
+        __syncthreads();
+        if (wave < G) {
+            for (int w = 0; w < min(W, chunks - first); ++w) {
+                const float corr = corr_of[wave][w];
+                l = fmaf(l, corr, sum_of[wave][w]);
+#pragma unroll
+                for (int j = 0; j < DPL; ++j) acc[j] *= corr;
+                const unsigned long long have = rows_of[w];
+                const float* vw = values + (size_t)w * WAVE * LD + lane;
+                const float* pw = weights[wave][w];
+                // (sixteen keys ahead of the chain)
+                constexpr int N = 16;
+                float vn[N][DPL], pn[N];
+                auto ask = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < N; i += 4) {
+                        const f32x4 p4 = *reinterpret_cast<const f32x4*>(pw + k + i);
+#pragma unroll
+                        for (int n = 0; n < 4; ++n) pn[i + n] = p4[n];
+                    }
+#pragma unroll
+                    for (int i = 0; i < N; ++i)
+#pragma unroll
+                        for (int j = 0; j < DPL; ++j) vn[i][j] = vw[(k + i) * LD + j * WAVE];
+                };
+                ask(0);
+#pragma unroll
+                for (int k = 0; k < WAVE; k += N) {
+                    float vk[N][DPL], pk[N];
+#pragma unroll
+                    for (int i = 0; i < N; ++i) {
+                        pk[i] = pn[i];
+#pragma unroll
+                        for (int j = 0; j < DPL; ++j) vk[i][j] = vn[i][j];
+                    }
+                    if (k + N < WAVE) ask(k + N);
+                    const unsigned some = (unsigned)(have >> k) & ((1u << N) - 1);
+                    if (some == (1u << N) - 1) {
+#pragma unroll
+                        for (int i = 0; i < N; ++i)
+#pragma unroll
+                            for (int j = 0; j < DPL; ++j) acc[j] = fmaf(pk[i], vk[i][j], acc[j]);
+                    } else if (some) {
+#pragma unroll
+                        for (int i = 0; i < N; ++i)
+#pragma unroll
+                            for (int j = 0; j < DPL; ++j) {
+                                const float to = fmaf(pk[i], vk[i][j], acc[j]);
+                                acc[j] = some >> i & 1 ? to : acc[j];
+                            }
+                    }
+                }
+            }
+        }
+    }
+    if (wave >= G) return;
+    const int h = kvh * G + wave;
+    float inv = l > 0.f ? 1.0f / l : 0.f;
+    if (rule.sink) {                        // one more term of the denominator, without a key or a value
+        float mine = m[0];
+#pragma unroll
+        for (int g = 1; g < GMAX; ++g) mine = g == wave ? m[g] : mine;
+        const float sink = rule.sink[h], top = fmaxf(mine, sink);
+        const float w = (mine == -INFINITY) ? 0.f : expf(mine - top);
+        inv = w / fmaf(l, w, expf(sink - top));
+    }
+    inv *= rule.out_scale;
+    if (rule.gate) inv *= 1.0f / (1.0f + expf(-rule.gate[(size_t)t * rule.gate_ld + h]));
+    float* dst = out + (size_t)t * out_ld + (size_t)h * HD;
+#pragma unroll
+    for (int j = 0; j < DPL; ++j) dst[lane + j * WAVE] = acc[j] * inv;
+    if (h == heads - 1)
+        for (int d = HD + lane; d < out_ld - h * HD; d += WAVE) dst[d] = 0.f;
+}
+
+template <int HD, int GMAX>
+static int launch_split_f32(const float* q, const float* k_cache, const float* v_cache, float* out, const int32_t* positions,
+                            const int32_t* row_of_token, const int32_t* block_table, int table_stride, int page_size, int n_tokens,
+                            int heads, int kv_heads, int out_ld, int n_pages, float scale, int window, const ImparoAttentionRule& r,
+                            hipStream_t s) {
+    constexpr int W = SplitF32<HD>::WAVES, LDS = W * WAVE * SplitF32<HD>::LD * 4;
+    if (hipFuncSetAttribute((const void*)k_attention_split_f32<HD, GMAX>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
+        return IMPARO_LAUNCH_FAILED;
+    k_attention_split_f32<HD, GMAX><<<n_tokens * kv_heads, W * WAVE, LDS, s>>>(q, k_cache, v_cache, out, positions, row_of_token,
+        block_table, table_stride, page_size, heads, kv_heads, out_ld, n_pages, scale, window, r);
+    return launch_status();
+}
+
 static int check_attention_args(const void* q, const void* k_cache, const void* v_cache, void* out,
                                 const int32_t* positions, const int32_t* row_of_token, const int32_t* block_table,
                                 int table_stride, int page_size, int n_tokens, int heads, int kv_heads, int head_dim,
@@ -342,6 +551,19 @@ static int attention_wave(const void* q, const void* k_cache, const void* v_cach
     // and 1,146) and short contexts (4 prompts of 100 tokens, 64 heads 251 and 216; one of 333 537 and 554).
     const long long room = (long long)table_stride * page_size;
     const bool one = room <= WAVE, few = total <= 4096;
+    // Few tokens: a block of several waves for a token's kv head (k_attention_split_f32), as long as each has a CU of its own.
+    const int G = heads / kv_heads;
+    if (plain && (head_dim == 64 || head_dim == 128) && !one && G <= 4 && (long long)n_tokens * kv_heads <= 256 && !((uintptr_t)v_cache & 15) &&
+        (long long)n_pages * kv_heads * page_size * head_dim < (1LL << 32)) {
+#define SPLIT_F32(HD, GMAX)                                                                                             \
+    return launch_split_f32<HD, GMAX>((const float*)q, (const float*)k_cache, (const float*)v_cache, (float*)out, positions, row_of_token, \
+                                      block_table, table_stride, page_size, n_tokens, heads, kv_heads, out_ld, n_pages, scale, window, r, s)
+        if (head_dim == 64 && G <= 2) SPLIT_F32(64, 2);
+        if (head_dim == 64) SPLIT_F32(64, 4);
+        if (G <= 2) SPLIT_F32(128, 2);
+        SPLIT_F32(128, 4);
+#undef SPLIT_F32
+    }
     if (plain && head_dim == 64 && one)
         WAVE_F32_GO(64, true);
     else if (plain && head_dim == 64 && (few || window <= 0 || window >= WAVE))

@@ -1,0 +1,37 @@
+"""Float32 attention of few tokens: chunks of keys side by side over a block's waves, the bits of one wave's walk."""
+import pytest
+import torch
+
+from gpu_helpers import hand_context
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def ops():
+    from imparo_amd.kernels import ops
+    return ops
+
+
+@pytest.mark.parametrize("H,Hk,D", [(16, 8, 64), (4, 4, 64), (8, 2, 64), (6, 2, 128), (4, 1, 128), (5, 1, 64)])
+@pytest.mark.parametrize("window,keep,capped", [(None, 0, False), (600, 70, True), (64, 0, False), (1, 130, True), (-100, 0, False)])
+def test_few_tokens_have_the_general_kernels_bits(H, Hk, D, window, keep, capped):
+    """Contexts at whole chunks and rounds of them (256 and 512 keys), beside them, and of one key; values transposed in their
+    pages go through the general kernel."""
+    lens, page = (1, 64, 65, 256, 257, 511, 513, 1100), 16
+    R, n_pages = len(lens), sum(-(-c // page) for c in lens) + 2
+    ctx = hand_context([(c - 1, 1) for c in lens], page, n_pages, torch.float32, DEV, kv_sites={0: (Hk, D)})
+    table = ctx.block_tables[0]
+    g = torch.Generator().manual_seed(1)
+    k, v, q = (torch.randn(*s, generator=g).to(DEV) for s in ((n_pages, Hk, page, D), (n_pages, Hk, page, D), (R, H, D)))
+    rule = None
+    if keep or capped:
+        rule = ops().attention_rule(H, keep_first=keep, softcap=8.0 if capped else None, sink=torch.randn(H, generator=g).to(DEV), out_scale=0.9)
+    got = []
+    for transposed in (False, True):
+        out = torch.full((R, H * D), float("nan"), device=DEV)
+        values = v.transpose(2, 3).contiguous() if transposed else v
+        ops().attention(q, k, values, out, ctx.positions, ctx.row_of_token, table, 0.125, window, v_transposed=transposed, rule=rule)
+        got.append(out.cpu())
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(*got)
