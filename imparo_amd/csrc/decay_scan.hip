@@ -339,89 +339,197 @@ __global__ __launch_bounds__(256) void k_delta_chunk_prepare(const DecayScanArgs
 __host__ __device__ static inline size_t channel_chunk_floats(int dp) { return 2 * DC * DC + (3 * DC + 1) * (size_t)dp; }
 __host__ __device__ static inline int channel_rows(int dim) { return dim <= 64 ? 64 : DMAXK; }
 
-__global__ __launch_bounds__(256) void k_channel_delta_prepare(const DecayScanArgs A) {
-    __shared__ float sk[DC][DMAXK + 1], sq[DC][DMAXK + 1], lg[DC][DMAXK + 1], sL[DC][DC + 1], sb[DC];
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// acc + x y on the matrix cores in float32: x's row lane % 16 and y's column lane % 16, inner numbers 4 i .. of group lane / 16 as
+// both sides have them; the result's column is lane % 16, its rows 4 (lane / 16) + i.
+__device__ __forceinline__ f32x4 dc_product(const f32x4& x, const f32x4& y, f32x4 acc) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], acc, 0, 0, 0);
+    return acc;
+}
+
+// A pair j < t belongs to the level s = 1, 2, 4, 8 or 16 of the highest bit in which t and j differ: t in the second half of a run
+// of 2 s tokens, j in the first. With e the first half's last token, g_t / g_j = (g_t / g_e) (g_e / g_j), both at most one, and
+// neither leaves float32's range where their product does not. So a level is one product of 16 tokens by 16 over the
+// state's rows, on the matrix cores, of whose result the pairs that share a run count, and needs one exponential a
+// token and row, 5 for all levels, where pair by pair it was 16 and five reads of LDS a pair and row. Each wave has a
+// quarter of the state's rows; the four sums meet in LDS. Every thread asks for its column of k, q and steps at once, and sums
+// the steps up in registers. The triangle is inverted in two halves side by side and the block below them by two products.
+// Bound by what it reads and writes, 106 KB a chunk and head. Measured, 4 requests of 1,024 tokens, 8 heads of 128: 78.5 -> 41.5 us; one of
+// 2,048 44.5 -> 27.3; results 2.8e-7 -> 2.3e-7 from 64 bits.
+template <int DP>
+__global__ __launch_bounds__(256, 3) void k_channel_delta_prepare(const DecayScanArgs A) {
+    constexpr int LD = DP + 4, RUNS = 256 / DP, TOK = DC / RUNS, KL = DP / 16, LEVELS = 5;
+    constexpr int PART = DC * DC, TRI = DC + 1;
+    constexpr int FLOATS = 3 * DC * LD > 8 * PART + DC * TRI ? 3 * DC * LD : 8 * PART + DC * TRI;
+    __shared__ __attribute__((aligned(16))) float mem[FLOATS];   // k | q | logarithms; then the waves' sums, and L
+    __shared__ float sb[DC], diagonal[DC], total[DP];
+    float* const sk = mem;
+    float* const sq = mem + DC * LD;
+    float* const lg = mem + 2 * DC * LD;
     const int r = blockIdx.x / A.max_chunks, chunk = blockIdx.x - r * A.max_chunks, h = blockIdx.y;
-    const int tid = threadIdx.x, dim = A.dim, heads = A.heads, dp = channel_rows(dim);
+    const int tid = threadIdx.x, dim = A.dim, heads = A.heads;
     const int n_all = A.seg_len[r];
     if (chunk * DC >= n_all) return;                     // (the whole block)
     const int first = A.seg_start[r] + chunk * DC, n = min(DC, n_all - chunk * DC);
     const int qh = h / A.q_div, kh = h / A.k_div;
     const float rate = A.rate[h] * 1.44269504088896340736f;      // logarithms to base 2
-    for (int i = tid; i < DC * dp; i += 256) {
-        const int t = i / dp, k = i - t * dp;
-        const bool on = t < n && k < dim;
-        const size_t row = (size_t)(first + min(t, n - 1));
-        const int kc = min(k, dim - 1);
-        const float kv = A.k[row * A.k_ld + A.k_off + kh * dim + kc], qv = A.q[row * A.q_ld + A.q_off + qh * dim + kc];
-        const float raw = A.step[row * A.step_ld + A.step_off + h * dim + kc] + A.step_bias[h * dim + kc];
-        sk[t][k] = on ? kv : 0.f;
-        sq[t][k] = on ? qv : 0.f;
-        lg[t][k] = on ? -rate * ds_softplus(raw) : 0.f;
-    }
-    if (tid < DC)
-        sb[tid] = tid < n ? ds_sigmoid(A.beta[(size_t)(first + tid) * A.beta_ld + A.beta_off + h]) : 0.f;
-    __syncthreads();
-    if (tid < dp) {
-        float sum = 0.f;
-        for (int t = 0; t < DC; ++t) {
-            sum += lg[t][tid];
-            lg[t][tid] = sum;
+    const int col = tid % DP, run = tid / DP, t0 = run * TOK;    // this thread's state row, its tokens
+    float kv[TOK], qv[TOK], la[TOK];
+    {
+        const int kc = min(col, dim - 1);
+        const float bias = A.step_bias[h * dim + kc];
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {                  // (no load under a branch)
+            const size_t row = (size_t)(first + min(t0 + i, n - 1));
+            kv[i] = A.k[row * A.k_ld + A.k_off + kh * dim + kc];
+            qv[i] = A.q[row * A.q_ld + A.q_off + qh * dim + kc];
+            la[i] = A.step[row * A.step_ld + A.step_off + h * dim + kc];
+        }
+        if (tid < DC)
+            sb[tid] = tid < n ? ds_sigmoid(A.beta[(size_t)(first + tid) * A.beta_ld + A.beta_off + h]) : 0.f;
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {
+            const bool on = t0 + i < n && col < dim;
+            kv[i] = on ? kv[i] : 0.f;
+            qv[i] = on ? qv[i] : 0.f;
+            sk[(t0 + i) * LD + col] = kv[i];
+            sq[(t0 + i) * LD + col] = qv[i];
+            la[i] = on ? -rate * ds_softplus(la[i] + bias) : 0.f;
         }
     }
-    __syncthreads();
-    float* T_out = A.chunk_state + ((size_t)blockIdx.x * heads + h) * channel_chunk_floats(dp);
+    // the logarithms add up token after token, so that of two neighbours' sums the difference is one rounding away from the step
+    // between them: one run's threads after the other's
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < RUNS; ++i) {
+        if (run == i) {                                  // (whole waves)
+            if (i > 0) sum = total[col];
+#pragma unroll
+            for (int j = 0; j < TOK; ++j) {
+                sum += la[j];
+                la[j] = sum;
+                lg[(t0 + j) * LD + col] = sum;
+            }
+            total[col] = sum;
+        }
+        __syncthreads();
+    }
+    float* T_out = A.chunk_state + ((size_t)blockIdx.x * heads + h) * channel_chunk_floats(DP);
     float* M_out = T_out + DC * DC;
     float* kg_out = M_out + DC * DC;
-    float* qg_out = kg_out + DC * dp;
-    float* ke_out = qg_out + DC * dp;
-    for (int i = tid; i < DC * DC; i += 256) {             // above the diagonals
-        const int t = i / DC, j = i - t * DC;
-        if (j >= t) sL[t][j] = 0.f;
-        if (j > t) M_out[i] = 0.f;
-    }
-    // the pairs j <= t one after the other, row by row, so that no lane idles on the other half of the square
-    for (int p = tid; p < DC * (DC + 1) / 2; p += 256) {
-        int t = (int)((sqrtf(8.0f * (float)p + 1.0f) - 1.0f) * 0.5f);
-        if (t * (t + 1) / 2 > p) --t;
-        if ((t + 1) * (t + 2) / 2 <= p) ++t;
-        const int j = p - t * (t + 1) / 2;
-        float kk = 0.f, qk = 0.f;
-#pragma unroll 8
-        for (int k = 0; k < dim; ++k) {
-            const float w = sk[j][k] * __builtin_amdgcn_exp2f(lg[t][k] - lg[j][k]);
-            kk = fmaf(sk[t][k], w, kk);
-            qk = fmaf(sq[t][k], w, qk);
+    float* qg_out = kg_out + DC * DP;
+    float* ke_out = qg_out + DC * DP;
+    {
+        const float last = lg[(DC - 1) * LD + col];
+#pragma unroll
+        for (int i = 0; i < TOK; ++i) {
+            const float g = __builtin_amdgcn_exp2f(la[i]);
+            kg_out[(t0 + i) * DP + col] = kv[i] * g;
+            qg_out[(t0 + i) * DP + col] = qv[i] * g;
         }
-        if (j < t) sL[t][j] = kk * sb[t];
-        M_out[t * DC + j] = qk;
+#pragma unroll
+        for (int i = 0; i < TOK; i += 4) {
+            f32x4 e;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) e[j] = kv[i + j] * __builtin_amdgcn_exp2f(last - la[i + j]);
+            *reinterpret_cast<f32x4*>(&ke_out[col * DC + t0 + i]) = e;
+        }
+        if (run == 0) ke_out[DC * DP + col] = __builtin_amdgcn_exp2f(last);
     }
-    for (int i = tid; i < DC * dp; i += 256) {
-        const int t = i / dp, k = i - t * dp;
-        const float g = __builtin_amdgcn_exp2f(lg[t][k]);
-        kg_out[i] = sk[t][k] * g;
-        qg_out[i] = sq[t][k] * g;
+    const int lane = tid & (WAVE - 1), wave = tid / WAVE, c = lane & 15, g = lane >> 4;
+    {                                                    // q_t . k_t: eight threads a token
+        const int t = tid >> 3, at = t * LD + (tid & 7) * (DP / 8);
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < DP / 8; ++i) sum = fmaf(sq[at + i], sk[at + i], sum);
+#pragma unroll
+        for (int m = 1; m < 8; m *= 2) sum += __shfl_xor(sum, m, WAVE);
+        if ((tid & 7) == 0) diagonal[t] = sum;
     }
-    for (int i = tid; i < DC * dp; i += 256) {
-        const int k = i / DC, t = i - k * DC;
-        ke_out[i] = sk[t][k] * __builtin_amdgcn_exp2f(lg[DC - 1][k] - lg[t][k]);
+    f32x4 kk[LEVELS], qk[LEVELS];
+#pragma unroll
+    for (int lv = 0; lv < LEVELS; ++lv) {
+        const int s = 1 << lv, t = (c / s * 2 + 1) * s + c % s, e = (c / s * 2 + 1) * s - 1;
+        const int at = wave * (DP / 4) + g * KL;         // (the state's rows in any order, the same on both sides)
+        kk[lv] = qk[lv] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = at; k < at + KL; k += 4) {
+            const f32x4 lt = *reinterpret_cast<const f32x4*>(&lg[t * LD + k]), le = *reinterpret_cast<const f32x4*>(&lg[e * LD + k]);
+            const f32x4 lj = *reinterpret_cast<const f32x4*>(&lg[(t - s) * LD + k]), kj = *reinterpret_cast<const f32x4*>(&sk[(t - s) * LD + k]);
+            const f32x4 kt = *reinterpret_cast<const f32x4*>(&sk[t * LD + k]), qt = *reinterpret_cast<const f32x4*>(&sq[t * LD + k]);
+            f32x4 a, b;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a[i] = __builtin_amdgcn_exp2f(lt[i] - le[i]);
+                b[i] = kj[i] * __builtin_amdgcn_exp2f(le[i] - lj[i]);
+            }
+            kk[lv] = dc_product(kt * a, b, kk[lv]);
+            qk[lv] = dc_product(qt * a, b, qk[lv]);
+        }
     }
-    if (tid < dp) ke_out[DC * dp + tid] = __builtin_amdgcn_exp2f(lg[DC - 1][tid]);
+    __syncthreads();                                     // k, q and the logarithms have been read
+    float* const part = mem + wave * 2 * PART;           // [t][j], of K K^T and of Q K^T
+#pragma unroll
+    for (int lv = 0; lv < LEVELS; ++lv) {
+        const int s = 1 << lv, j = c / s * 2 * s + c % s;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int row = 4 * g + i, t = (row / s * 2 + 1) * s + row % s;
+            if (row / s != c / s) continue;
+            part[t * DC + j] = kk[lv][i];
+            part[PART + t * DC + j] = qk[lv][i];
+        }
+    }
     __syncthreads();
-    if (tid < DC) {
-        // column tid of (I + L)^-1 by forward substitution, then times b of that column
-        float x[DC];
+    float* const sL = mem + 8 * PART;                    // [DC][TRI]
+    for (int i = tid; i < PART; i += 256) {
+        const int t = i / DC, j = i - t * DC;
+        float l = 0.f, m = j == t ? diagonal[t] : 0.f;
+        if (j < t) {
+            l = ((mem[i] + mem[2 * PART + i]) + (mem[4 * PART + i] + mem[6 * PART + i])) * sb[t];
+            m = (mem[PART + i] + mem[3 * PART + i]) + (mem[5 * PART + i] + mem[7 * PART + i]);
+        }
+        sL[t * TRI + j] = l;
+        M_out[i] = m;
+    }
+    __syncthreads();
+    if (wave) return;
+    // (I + L)^-1 diag(b): lanes 0 .. 15 the columns of the upper half's inverse, 16 .. 31 of the lower's, by forward
+    // substitution; the block below is -(lower inverse) L21 (upper inverse)
+    float* const inverse = mem;                          // [2][16][17]
+    if (lane < DC) {
+        const float* L = sL + (lane & 16) * (TRI + 1);
+        float x[16];
 #pragma unroll
-        for (int t = 0; t < DC; ++t) {
-            float acc = t == tid ? 1.f : 0.f;
+        for (int t = 0; t < 16; ++t) {
+            float acc = t == c ? 1.f : 0.f;
 #pragma unroll
-            for (int j = 0; j < t; ++j) acc = fmaf(-sL[t][j], x[j], acc);
+            for (int j = 0; j < t; ++j) acc = fmaf(-L[t * TRI + j], x[j], acc);
             x[t] = acc;
         }
-        const float b = sb[tid];
+        const float b = sb[lane];
 #pragma unroll
-        for (int t = 0; t < DC; ++t) T_out[t * DC + tid] = x[t] * b;
+        for (int t = 0; t < 16; ++t) {
+            inverse[(g * 16 + t) * 17 + c] = x[t];
+            T_out[((lane & 16) + t) * DC + lane] = x[t] * b;
+            if (g == 1) T_out[t * DC + lane] = 0.f;
+        }
     }
+    wave_lds_sync();
+    f32x4 l21, upper, lower;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        l21[i] = sL[(16 + c) * TRI + 4 * g + i];
+        upper[i] = inverse[(4 * g + i) * 17 + c];
+        lower[i] = -inverse[(16 + c) * 17 + 4 * g + i];
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 below = dc_product(lower, dc_product(l21, upper, zero), zero);
+    const float b = sb[c];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_out[(16 + 4 * g + i) * DC + c] = below[i] * b;
 }
 
 // The walk: a segment's chunks in order, a block a (segment, head, run of 16 value columns), every product on the
@@ -431,12 +539,14 @@ __global__ __launch_bounds__(256) void k_channel_delta_prepare(const DecayScanAr
 // register i the second operand of the next product as it is, and the first operand 16 neighbouring bytes of a row of K
 // (or Q, T, M). So nothing is staged and nothing moves between lanes; each wave multiplies its own rows of the state,
 // the four partial sums of K S and Q S meet in LDS (two buffers in turn: one barrier a chunk), every wave makes the
-// whole of U for its own update, and waves 0 and 1 finish the 16 results each. The operands of the next chunk are
-// asked for a chunk ahead.
+// whole of U for its own update, and waves 0 and 1 finish the 16 results each. An operand of the next chunk is asked for
+// right behind the last use of this chunk's, into the same registers. Bound by the chunk's chain: 60 to 68 products of 32
+// cycles a wave, with the exchange in the middle. Measured, 4 requests of 1,024 tokens, 8 heads of 128, decays a channel: 88.3 us
+// with a chunk's 27 requests in a row and the sums read from LDS one by one, 74.4 now (50 with neither requests nor results); one of
+// 2,048 158 -> 129. Uniform bases with 32-bit offsets in place of whole addresses: 73.9 and 128.8, not kept.
 // KIND: a plain decay (U is V itself), the delta rule, the delta rule with decays a channel (whose operands the first
 // launch has laid out; the others read K and Q where they lie and scale rows of the results instead). VEC: K's and
 // Q's rows can be read in 16-byte pieces.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 enum { WALK_DELTA = 0, WALK_PLAIN = 1, WALK_CHANNEL = 2 };
 
 template <int KIND, int TPW>
@@ -469,80 +579,96 @@ __global__ __launch_bounds__(256) void k_chunk_walk(const DecayScanArgs A) {
             const float x = S_at[(size_t)min(k, dim - 1) * vdim + vc];
             S[j][i] = (k < dim && live) ? x : 0.f;
         }
-    // every address is clamped and nothing is chosen here (no load may end up under a branch); tokens past the end
-    // repeat the last one and meet zeros in U
-    auto load = [&](ChunkIn<KIND, TPW>& in, int chunk) __attribute__((always_inline)) {
+    // What is asked for, a piece at a time; every address is clamped and nothing is chosen here (no load may end up under a
+    // branch); tokens past the end repeat the last one and meet zeros in U
+    struct Place {                                         // of a chunk
+        int first, n;
+        const float* T;                                    // T, M, and with decays a channel the operands
+        const float* decays;
+    };
+    constexpr int DP = TPW * 64;
+    auto place = [&](int chunk) __attribute__((always_inline)) {
         chunk = min(chunk, n_chunks - 1);
-        const int first = start + chunk * DC, n = min(DC, n_all - chunk * DC);
         const size_t at = (size_t)(r * A.max_chunks + chunk) * heads + h;
-        const float* T = A.chunk_state + at * (KIND == WALK_CHANNEL ? channel_chunk_floats(TPW * 64) : (size_t)(2 * DC * DC));
-        const float* M = T + DC * DC;
+        return Place{start + chunk * DC, min(DC, n_all - chunk * DC),
+                     A.chunk_state + at * (KIND == WALK_CHANNEL ? channel_chunk_floats(DP) : (size_t)(2 * DC * DC)),
+                     KIND == WALK_CHANNEL ? nullptr : A.chunk_decay + at * (2 * DC)};
+    };
+    ChunkIn<KIND, TPW> in;
+    auto row_of = [&](const float* rows, int ld, const Place& p, int a, int j) __attribute__((always_inline)) {    // K's or Q's piece [a][j]
+        const float* x = rows + (size_t)(p.first + min(16 * a + c, p.n - 1)) * ld;
+        const int k0 = 16 * (wave + 4 * j) + 4 * g;        // (past dim: other numbers of the row, which meet state rows that stay zero)
+        f32x4 v;
+        if constexpr (VEC) {                               // rows of whole pieces
+            v = *reinterpret_cast<const f32x4*>(x + min(k0, dim - 4));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = x[min(k0 + i, dim - 1)];
+        }
+        return v;
+    };
+    auto load_k = [&](const Place& p, int a, int j) __attribute__((always_inline)) {
+        if constexpr (KIND == WALK_CHANNEL)
+            in.k[a][j] = *reinterpret_cast<const f32x4*>(p.T + 2 * DC * DC + (16 * a + c) * DP + 16 * (wave + 4 * j) + 4 * g);
+        else if constexpr (KIND == WALK_DELTA)
+            in.k[a][j] = row_of(A.k + A.k_off + kh * dim, A.k_ld, p, a, j);
+    };
+    auto load_q = [&](const Place& p, int a, int j) __attribute__((always_inline)) {
+        if constexpr (KIND == WALK_CHANNEL)
+            in.q[a][j] = *reinterpret_cast<const f32x4*>(p.T + 2 * DC * DC + DC * DP + (16 * a + c) * DP + 16 * (wave + 4 * j) + 4 * g);
+        else
+            in.q[a][j] = row_of(A.q + A.q_off + qh * dim, A.q_ld, p, a, j);
+    };
+    auto load_e = [&](const Place& p, int a, int j) __attribute__((always_inline)) {
+        const int k = 16 * (wave + 4 * j) + c;
+        if constexpr (KIND == WALK_CHANNEL) {
+            in.e[a][j] = *reinterpret_cast<const f32x4*>(p.T + 2 * DC * DC + 2 * DC * DP + k * DC + 16 * a + 4 * g);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                in.e[a][j][i] = A.k[(size_t)(p.first + min(16 * a + 4 * g + i, p.n - 1)) * A.k_ld + A.k_off + kh * dim + min(k, dim - 1)];
+        }
+    };
+    auto load_v = [&](const Place& p, int a) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            in.v[a][i] = A.v[(size_t)(p.first + min(16 * a + 4 * g + i, p.n - 1)) * A.v_ld + A.v_off + h * vdim + vc];
+    };
+    auto load_t = [&](const Place& p) __attribute__((always_inline)) {
         if constexpr (KIND != WALK_PLAIN) {
-            in.t00 = *reinterpret_cast<const f32x4*>(T + c * DC + 4 * g);
-            in.t10 = *reinterpret_cast<const f32x4*>(T + (16 + c) * DC + 4 * g);
-            in.t11 = *reinterpret_cast<const f32x4*>(T + (16 + c) * DC + 16 + 4 * g);
-        }
-        const float* m_row = M + ((wave & 1) * 16 + c) * DC + 4 * g;
-        in.m0 = *reinterpret_cast<const f32x4*>(m_row);
-        in.m1 = *reinterpret_cast<const f32x4*>(m_row + 16);
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 16 * a + 4 * g + i;
-                const float x = A.v[(size_t)(first + min(t, n - 1)) * A.v_ld + A.v_off + h * vdim + vc];
-                in.v[a][i] = x;
-            }
-            if constexpr (KIND == WALK_CHANNEL) {
-                constexpr int DP = TPW * 64;
-                const float* kg = M + DC * DC;
-#pragma unroll
-                for (int j = 0; j < TPW; ++j) {
-                    const int T16 = 16 * (wave + 4 * j);
-                    in.k[a][j] = *reinterpret_cast<const f32x4*>(kg + (16 * a + c) * DP + T16 + 4 * g);
-                    in.q[a][j] = *reinterpret_cast<const f32x4*>(kg + DC * DP + (16 * a + c) * DP + T16 + 4 * g);
-                    in.e[a][j] = *reinterpret_cast<const f32x4*>(kg + 2 * DC * DP + (T16 + c) * DC + 16 * a + 4 * g);
-                    if (a == 0) in.gl[j] = *reinterpret_cast<const f32x4*>(kg + 3 * DC * DP + T16 + 4 * g);
-                }
-            } else {
-                const float* decays = A.chunk_decay + at * (2 * DC);
-                in.lg[a] = *reinterpret_cast<const f32x4*>(decays + 16 * a + 4 * g);
-                if constexpr (KIND == WALK_PLAIN) in.dt[a] = *reinterpret_cast<const f32x4*>(decays + DC + 16 * a + 4 * g);
-                in.last = decays[DC - 1];
-                const size_t row = (size_t)(first + min(16 * a + c, n - 1));
-                const float* kr = A.k + row * A.k_ld + A.k_off + kh * dim;
-                const float* qr = A.q + row * A.q_ld + A.q_off + qh * dim;
-#pragma unroll
-                for (int j = 0; j < TPW; ++j) {
-                    const int k0 = 16 * (wave + 4 * j) + 4 * g, kc = 16 * (wave + 4 * j) + c;
-                    // (past dim: other numbers of the row, which meet state rows that stay zero)
-                    if constexpr (VEC) {                   // rows of whole pieces
-                        in.q[a][j] = *reinterpret_cast<const f32x4*>(qr + min(k0, dim - 4));
-                        if constexpr (KIND != WALK_PLAIN) in.k[a][j] = *reinterpret_cast<const f32x4*>(kr + min(k0, dim - 4));
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            in.q[a][j][i] = qr[min(k0 + i, dim - 1)];
-                            if constexpr (KIND != WALK_PLAIN) in.k[a][j][i] = kr[min(k0 + i, dim - 1)];
-                        }
-                    }
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const size_t rt = (size_t)(first + min(16 * a + 4 * g + i, n - 1));
-                        in.e[a][j][i] = A.k[rt * A.k_ld + A.k_off + kh * dim + min(kc, dim - 1)];
-                    }
-                }
-            }
+            in.t00 = *reinterpret_cast<const f32x4*>(p.T + c * DC + 4 * g);
+            in.t10 = *reinterpret_cast<const f32x4*>(p.T + (16 + c) * DC + 4 * g);
+            in.t11 = *reinterpret_cast<const f32x4*>(p.T + (16 + c) * DC + 16 + 4 * g);
         }
     };
-    auto product = [](const f32x4& x, const f32x4& y, f32x4 acc) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i], y[i], acc, 0, 0, 0);
-        return acc;
+    auto load_m = [&](const Place& p) __attribute__((always_inline)) {
+        const float* row = p.T + DC * DC + ((wave & 1) * 16 + c) * DC + 4 * g;
+        in.m0 = *reinterpret_cast<const f32x4*>(row);
+        in.m1 = *reinterpret_cast<const f32x4*>(row + 16);
     };
+    auto load_decays = [&](const Place& p) __attribute__((always_inline)) {
+        if constexpr (KIND == WALK_CHANNEL) {
+#pragma unroll
+            for (int j = 0; j < TPW; ++j)
+                in.gl[j] = *reinterpret_cast<const f32x4*>(p.T + 2 * DC * DC + 3 * DC * DP + 16 * (wave + 4 * j) + 4 * g);
+        } else {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                in.lg[a] = *reinterpret_cast<const f32x4*>(p.decays + 16 * a + 4 * g);
+                if constexpr (KIND == WALK_PLAIN) in.dt[a] = *reinterpret_cast<const f32x4*>(p.decays + DC + 16 * a + 4 * g);
+            }
+            in.last = p.decays[DC - 1];
+        }
+    };
+    auto held = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
     const float skip = (KIND == WALK_PLAIN && A.skip) ? A.skip[h] : 0.f;
-    auto step = [&](const ChunkIn<KIND, TPW>& in, int chunk) __attribute__((always_inline)) {
+    float* out = A.out + (size_t)h * vdim + v;
+    const int out_ld = heads * vdim;
+    // Every piece of the next chunk is asked for right behind the last use of this chunk's, into the same registers: a chunk ahead,
+    // and one request between two products, so that no wave stands in line to ask
+    auto step = [&](int chunk) __attribute__((always_inline)) {
         const int first = start + chunk * DC, n = min(DC, n_all - chunk * DC), buf = chunk & 1;
+        const Place next = place(chunk + 1);
         // what the state says of the chunk's keys and queries: this wave's rows of it
         f32x4 p[2], q[2];
 #pragma unroll
@@ -551,57 +677,85 @@ __global__ __launch_bounds__(256) void k_chunk_walk(const DecayScanArgs A) {
 #pragma unroll
             for (int j = 0; j < TPW; ++j)
 #pragma unroll
-                for (int a = 0; a < 2; ++a) p[a] = product(in.k[a][j], S[j], p[a]);
+                for (int a = 0; a < 2; ++a) {
+                    p[a] = dc_product(in.k[a][j], S[j], p[a]);
+                    load_k(next, a, j);
+                    held();
+                }
             part[buf][wave][0][lane] = p[0];
             part[buf][wave][1][lane] = p[1];
         }
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
 #pragma unroll
-            for (int a = 0; a < 2; ++a) q[a] = product(in.q[a][j], S[j], q[a]);
+            for (int a = 0; a < 2; ++a) {
+                q[a] = dc_product(in.q[a][j], S[j], q[a]);
+                load_q(next, a, j);
+                held();
+            }
         part[buf][wave][2][lane] = q[0];
         part[buf][wave][3][lane] = q[1];
-        __syncthreads();
         f32x4 g_of[2], u[2], vv[2];
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int a = 0; a < 2; ++a) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) vv[a][i] = (16 * a + 4 * g + i < n && live) ? in.v[a][i] : 0.f;
-        if constexpr (KIND != WALK_CHANNEL)
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) g_of[a][i] = expf(in.lg[a][i]);
+            for (int i = 0; i < 4; ++i) {
+                vv[a][i] = (16 * a + 4 * g + i < n && live) ? in.v[a][i] : 0.f;
+                if constexpr (KIND != WALK_CHANNEL) g_of[a][i] = expf(in.lg[a][i]);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                      // (a bare one: the loads in flight are not waited for)
+        asm volatile("" ::: "memory");
         if constexpr (KIND == WALK_PLAIN) {
 #pragma unroll
             for (int a = 0; a < 2; ++a) u[a] = A.v_times_step ? vv[a] * in.dt[a] : vv[a];
         } else {
-            f32x4 res[2];
+            f32x4 res[2], of[2][4];
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) of[a][w] = part[buf][w][a][lane];
+            held();                                        // (left alone, the compiler reads and waits one by one)
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
-                f32x4 sum = part[buf][0][a][lane];
+                f32x4 sum = of[a][0];
 #pragma unroll
-                for (int w = 1; w < 4; ++w) sum = sum + part[buf][w][a][lane];
+                for (int w = 1; w < 4; ++w) sum = sum + of[a][w];
                 res[a] = KIND == WALK_CHANNEL ? vv[a] - sum : vv[a] - g_of[a] * sum;
             }
             const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-            u[0] = product(in.t00, res[0], zero);
-            u[1] = product(in.t11, res[1], product(in.t10, res[0], zero));
+            u[0] = dc_product(in.t00, res[0], zero);
+            load_v(next, 0);
+            held();
+            u[1] = dc_product(in.t10, res[0], zero);
+            load_v(next, 1);
+            held();
+            u[1] = dc_product(in.t11, res[1], u[1]);
+            load_t(next);
+            held();
         }
+        if constexpr (KIND == WALK_PLAIN) load_v(next, 0), load_v(next, 1);
         if (wave < 2) {                                    // (the whole wave) results of tokens 16 wave .. + 15
-            f32x4 o = part[buf][0][2 + wave][lane];
+            f32x4 of[4];
 #pragma unroll
-            for (int w = 1; w < 4; ++w) o = o + part[buf][w][2 + wave][lane];
+            for (int w = 0; w < 4; ++w) of[w] = part[buf][w][2 + wave][lane];
+            held();
+            f32x4 o = of[0];
+#pragma unroll
+            for (int w = 1; w < 4; ++w) o = o + of[w];
             if constexpr (KIND != WALK_CHANNEL) o = o * (wave ? g_of[1] : g_of[0]);
-            o = product(in.m0, u[0], o);
-            if (wave) o = product(in.m1, u[1], o);
+            o = dc_product(in.m0, u[0], o);
+            if (wave) o = dc_product(in.m1, u[1], o);
             if (KIND == WALK_PLAIN && skip != 0.f) o = o + skip * (wave ? vv[1] : vv[0]);
+            const int t = 16 * wave + 4 * g;
+            float* to = out + (size_t)(first + t) * out_ld;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int t = 16 * wave + 4 * g + i;
-                if (t < n && live) A.out[(size_t)(first + t) * heads * vdim + (size_t)h * vdim + v] = o[i];
-            }
+            for (int i = 0; i < 4; ++i)
+                if (t + i < n && live) to[(size_t)i * out_ld] = o[i];
         }
+        load_m(next);
+        held();
         // the state behind the chunk
         if constexpr (KIND != WALK_CHANNEL) {
             const float g_last = expf(in.last);
@@ -615,6 +769,7 @@ __global__ __launch_bounds__(256) void k_chunk_walk(const DecayScanArgs A) {
 #pragma unroll
             for (int j = 0; j < TPW; ++j) S[j] = S[j] * in.gl[j];
         }
+        load_decays(next);
 #pragma unroll
         for (int j = 0; j < TPW; ++j)
 #pragma unroll
@@ -623,18 +778,28 @@ __global__ __launch_bounds__(256) void k_chunk_walk(const DecayScanArgs A) {
                 if constexpr (KIND != WALK_CHANNEL)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) e[i] = 16 * (wave + 4 * j) + c < dim ? e[i] : 0.f;
-                S[j] = product(e, u[a], S[j]);
+                S[j] = dc_product(e, u[a], S[j]);
+                load_e(next, a, j);
+                held();
             }
     };
-    ChunkIn<KIND, TPW> even, odd;
-    load(even, 0);
-    for (int chunk = 0; chunk < n_chunks; chunk += 2) {
-        load(odd, chunk + 1);
-        step(even, chunk);
-        if (chunk + 1 >= n_chunks) break;
-        load(even, chunk + 2);
-        step(odd, chunk + 1);
+    {
+        const Place p = place(0);                          // (in the order they are used, as in the loop: a wait counts what was asked for later)
+#pragma unroll
+        for (int j = 0; j < TPW; ++j)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) load_k(p, a, j), held();
+#pragma unroll
+        for (int j = 0; j < TPW; ++j)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) load_q(p, a, j), held();
+        load_v(p, 0), held(), load_v(p, 1), held(), load_t(p), held(), load_m(p), held(), load_decays(p), held();
+#pragma unroll
+        for (int j = 0; j < TPW; ++j)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) load_e(p, a, j), held();
     }
+    for (int chunk = 0; chunk < n_chunks; ++chunk) step(chunk);
 #pragma unroll
     for (int j = 0; j < TPW; ++j)
 #pragma unroll
@@ -686,7 +851,9 @@ extern "C" int imparo_channel_delta_scan(const float* q, int q_ld, int q_off, in
     args.heads = heads, args.dim = dim, args.vdim = vdim, args.kpt = kpt;
     args.chunk_tokens = chunk_tokens, args.max_chunks = max_chunks, args.chunk_state = scratch;
     if (chunk_tokens) {
-        k_channel_delta_prepare<<<dim3(n_rows * max_chunks, heads), 256, 0, s>>>(args);
+        const dim3 pgrid(n_rows * max_chunks, heads);
+        if (channel_rows(dim) == 64) k_channel_delta_prepare<64><<<pgrid, 256, 0, s>>>(args);
+        else k_channel_delta_prepare<DMAXK><<<pgrid, 256, 0, s>>>(args);
         launch_walk<WALK_CHANNEL, true>(args, n_rows, s);
         return launch_status();
     }
