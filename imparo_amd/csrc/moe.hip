@@ -198,21 +198,12 @@ struct MoePlanShared {
     int count[MOE_MAX_EXPERTS], first[MOE_MAX_EXPERTS], first_tile[MOE_MAX_EXPERTS + 1];
 };
 
-__device__ __forceinline__ void moe_plan_block(MoePlanShared& sh, const int32_t* __restrict__ choice, int n_entries,
-                                               int n_experts, int tile_rows, int32_t* __restrict__ slot_of_entry,
-                                               int32_t* __restrict__ entry_of_slot, int32_t* __restrict__ tiles,
-                                               int max_tiles) {
+// From every expert's count its first slot and first tile
+__device__ __forceinline__ void moe_plan_firsts(MoePlanShared& sh, int n_experts, int tile_rows) {
     int* count = sh.count;
     int* first = sh.first;
     int* first_tile = sh.first_tile;
     const int tid = threadIdx.x;
-    for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;
-    __syncthreads();
-    for (int i = tid; i < n_entries; i += blockDim.x) {
-        const int e = choice[i];
-        if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
-    }
-    __syncthreads();
     if (n_experts <= WAVE) {
         if (tid < WAVE) {                    // a lane an expert
             const int c = tid < n_experts ? count[tid] : 0, t = (c + tile_rows - 1) / tile_rows;
@@ -239,7 +230,14 @@ __device__ __forceinline__ void moe_plan_block(MoePlanShared& sh, const int32_t*
         }
         first_tile[n_experts] = n_tiles;
     }
-    __syncthreads();
+}
+
+__device__ __forceinline__ void moe_plan_tiles(const MoePlanShared& sh, int n_experts, int tile_rows, int32_t* __restrict__ tiles,
+                                               int max_tiles) {
+    const int* count = sh.count;
+    const int* first = sh.first;
+    const int* first_tile = sh.first_tile;
+    const int tid = threadIdx.x;
     for (int e = tid; e < n_experts; e += blockDim.x) {
         const int n = count[e];
         int i = first_tile[e];
@@ -254,6 +252,25 @@ __device__ __forceinline__ void moe_plan_block(MoePlanShared& sh, const int32_t*
         tiles[3 * i + 1] = first_tile[n_experts];       // an empty tile says how many come before the first empty one,
         tiles[3 * i + 2] = MOE_COUNTED;                 // and that it says so
     }
+}
+
+__device__ __forceinline__ void moe_plan_block(MoePlanShared& sh, const int32_t* __restrict__ choice, int n_entries,
+                                               int n_experts, int tile_rows, int32_t* __restrict__ slot_of_entry,
+                                               int32_t* __restrict__ entry_of_slot, int32_t* __restrict__ tiles,
+                                               int max_tiles) {
+    int* count = sh.count;
+    int* first = sh.first;
+    const int tid = threadIdx.x;
+    for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;
+    __syncthreads();
+    for (int i = tid; i < n_entries; i += blockDim.x) {
+        const int e = choice[i];
+        if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+    }
+    __syncthreads();
+    moe_plan_firsts(sh, n_experts, tile_rows);
+    __syncthreads();
+    moe_plan_tiles(sh, n_experts, tile_rows, tiles, max_tiles);
     __syncthreads();
     for (int e = tid; e < n_experts; e += blockDim.x) count[e] = 0;      // now the cursor of each expert
     __syncthreads();
@@ -324,6 +341,178 @@ extern "C" int imparo_moe_route_plan(const float* logits, const float* correctio
     k_moe_route_plan<<<1, 1024, 0, (hipStream_t)stream>>>(logits, correction, choice, weight, n_tokens, n_router, top,
                                                           scoring, rules, n_experts, tile_rows, slot_of_entry, entry_of_slot,
                                                           tiles, max_tiles);
+    return launch_status();
+}
+
+// ---------------------------------------------------------------- a prompt's router, choice and plan in two launches
+// The router's product, the choice and every expert's count in one launch: a block brings 16 tokens' rows and the router's into LDS,
+// all loads at once, one wave walks K in the order of the tile products (so that the logits are their bits and no near tie
+// turns), then each of eight waves chooses for two tokens out of LDS and the block counts what they chose. The second launch places the
+// entries: a block of 64 tokens adds up the counts of all blocks and of those before it, which is where its own entries
+// start, so that no block waits for another. Bound by the trips to memory and the walk's chain of products.
+// Measured, 2,048 tokens of 1,024, 4 of 8 chosen and one for all: product, choice and plan 9.3 + 3.9 + 9.8 us, now 8.9 + 4.4.
+// The product as a tile of 128 rows had 16 blocks that streamed their activations alone, the plan one block for all entries.
+#define MOE_ROUTER_TOKENS 16
+#define MOE_ROUTER_MAX 32           // outputs, and the experts of the plan
+#define MOE_ROUTER_K 1024           // of K in LDS at once
+#define MOE_ROUTER_LD (MOE_ROUTER_K + 8)
+#define MOE_PLACE_TOKENS 64
+
+__global__ __launch_bounds__(512) void k_moe_router(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                    const float* __restrict__ bias, const float* __restrict__ correction,
+                                                    int32_t* __restrict__ choice, float* __restrict__ weight,
+                                                    int32_t* __restrict__ counts, int n_tokens, int n_router, int K, int top,
+                                                    int scoring, const MoeRouteRules rules, int n_experts) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t rows[];        // [MOE_ROUTER_TOKENS + n_router][MOE_ROUTER_LD]: tokens, then outputs
+    __shared__ float logits[MOE_ROUTER_TOKENS][MOE_ROUTER_MAX + 1];
+    __shared__ int32_t chosen[MOE_ROUTER_TOKENS * MOE_MAX_USED];
+    __shared__ int count[MOE_ROUTER_MAX];
+    constexpr int WAVES = 8, PIECES = MOE_ROUTER_K / 8, AHEAD = 8;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+    const int t0 = blockIdx.x * MOE_ROUTER_TOKENS, n = min(MOE_ROUTER_TOKENS, n_tokens - t0), used = top + rules.always;
+    if (tid < MOE_ROUTER_MAX) count[tid] = 0;
+    union Frag {
+        uint4 u;
+        bf16x8 v;
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+    for (int k0 = 0; k0 < K; k0 += MOE_ROUTER_K) {
+        const int part = min(K - k0, MOE_ROUTER_K);          // (a multiple of 128)
+        // a wave takes a row and half of what is here of it at a time, rows of tokens past the end the last one's
+        const int piece = (wave & 1) * (PIECES / 2) + lane, all = MOE_ROUTER_TOKENS + n_router;
+        const int at = k0 + min(piece * 8, part - 8);
+        __syncthreads();                                     // (the part before has been read)
+        for (int r0 = wave >> 1; r0 < all; r0 += 4 * AHEAD) {
+            uint4 v[AHEAD];
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) {
+                const int r = min(r0 + 4 * i, all - 1);
+                const bf16_t* row = r < MOE_ROUTER_TOKENS ? X + (size_t)(t0 + min(r, n - 1)) * K : W + (size_t)(r - MOE_ROUTER_TOKENS) * K;
+                v[i] = *reinterpret_cast<const uint4*>(row + at);
+            }
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i)
+                if (r0 + 4 * i < all) *reinterpret_cast<uint4*>(&rows[(r0 + 4 * i) * MOE_ROUTER_LD + piece * 8]) = v[i];
+        }
+        __syncthreads();
+        if (wave == 0) {
+            // (rows 16 .. 31 of the product are rows 0 .. 15 again)
+            const bf16_t* x = rows + (lane & 15) * MOE_ROUTER_LD + (lane >> 5) * 8;
+            const bf16_t* w = rows + (MOE_ROUTER_TOKENS + min(lane & 31, n_router - 1)) * MOE_ROUTER_LD + (lane >> 5) * 8;
+            Frag a[2][4], b[2][4];
+            auto read = [&](int k, Frag (&fa)[4], Frag (&fb)[4]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    fa[i].u = *reinterpret_cast<const uint4*>(x + k + 16 * i);
+                    fb[i].u = *reinterpret_cast<const uint4*>(w + k + 16 * i);
+                }
+                __builtin_amdgcn_sched_barrier(0);           // (the next operands are asked for before a product waits for these)
+            };
+            auto multiply = [&](const Frag (&fa)[4], const Frag (&fb)[4]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i].v, fb[i].v, acc, 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            read(0, a[0], b[0]);
+            for (int k = 0; k < part; k += 128) {
+                read(k + 64, a[1], b[1]);
+                multiply(a[0], b[0]);
+                read(min(k + 128, part - 64), a[0], b[0]);
+                multiply(a[1], b[1]);
+            }
+        }
+    }
+    if (wave == 0) {                                         // lane: output lane % 32 of 8 tokens
+        const int o = lane & 31;
+        const float bo = bias && o < n_router ? bias[o] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) logits[(i >> 2) * 8 + (lane >> 5) * 4 + (i & 3)][o] = acc[i] + bo;
+    }
+    __syncthreads();
+    for (int t = wave; t < n; t += WAVES)
+        moe_route_lanes(lane < n_router ? logits[t][min(lane, MOE_ROUTER_MAX)] : -INFINITY, correction, choice + (size_t)t0 * used,
+                        weight + (size_t)t0 * used, t, n_router, top, scoring, rules, chosen);
+    __syncthreads();
+    for (int i = tid; i < n * used; i += blockDim.x) {
+        const int e = chosen[i];
+        if (e >= 0 && e < n_experts) atomicAdd(&count[e], 1);
+    }
+    __syncthreads();
+    if (tid < n_experts) counts[(size_t)blockIdx.x * n_experts + tid] = count[tid];
+}
+
+__global__ __launch_bounds__(512) void k_moe_place(const int32_t* __restrict__ choice, const int32_t* __restrict__ counts, int n_tokens,
+                                                   int used, int n_experts, int tile_rows, int32_t* __restrict__ slot_of_entry,
+                                                   int32_t* __restrict__ entry_of_slot, int32_t* __restrict__ tiles, int max_tiles) {
+    constexpr int PER = MOE_PLACE_TOKENS / MOE_ROUTER_TOKENS;
+    __shared__ MoePlanShared sh;
+    __shared__ int next[MOE_ROUTER_MAX];                 // the block's next slot of an expert, from the expert's first
+    const int tid = threadIdx.x, blocks = (n_tokens + MOE_ROUTER_TOKENS - 1) / MOE_ROUTER_TOKENS;
+    const int first_entry = blockIdx.x * MOE_PLACE_TOKENS * used, entries = min(MOE_PLACE_TOKENS, n_tokens - (int)blockIdx.x * MOE_PLACE_TOKENS) * used;
+    if (tid < MOE_ROUTER_MAX) sh.count[tid] = 0, next[tid] = 0;
+    __syncthreads();
+    const int stripes = blockDim.x / n_experts, e = tid % n_experts;
+    if (tid < stripes * n_experts) {
+        int all = 0, before = 0;
+#pragma unroll 4
+        for (int b = tid / n_experts; b < blocks; b += stripes) {
+            const int c = counts[(size_t)b * n_experts + e];
+            all += c;
+            before += b < (int)blockIdx.x * PER ? c : 0;
+        }
+        atomicAdd(&sh.count[e], all);
+        atomicAdd(&next[e], before);
+    }
+    __syncthreads();
+    moe_plan_firsts(sh, n_experts, tile_rows);
+    __syncthreads();
+    if (blockIdx.x == 0) moe_plan_tiles(sh, n_experts, tile_rows, tiles, max_tiles);
+    for (int i = tid; i < entries; i += blockDim.x) {
+        const int mine = choice[first_entry + i];
+        int slot = -1;
+        if (mine >= 0 && mine < n_experts) {
+            slot = sh.first[mine] + atomicAdd(&next[mine], 1);
+            entry_of_slot[slot] = first_entry + i;
+        }
+        slot_of_entry[first_entry + i] = slot;
+    }
+}
+
+// Whether the two launches take so many tokens and a router of so many outputs over rows of k: where the product alone would go to
+// the tiles whose order the walk keeps (more than 128 rows, a K in 128s), and a 32 of outputs holds them.
+extern "C" int imparo_moe_router_takes(int n_tokens, int n_router, int n_experts, int top, int groups, int always, int k) {
+    return n_tokens > 128 && (long long)n_tokens * k < (1LL << 31) && n_router >= 1 && n_router <= MOE_ROUTER_MAX && n_experts >= 1 && n_experts <= MOE_ROUTER_MAX && top >= 1 && top <= n_router &&
+           top <= MOE_MAX_TOP && always >= 0 && top + always <= MOE_MAX_USED && groups == 1 &&
+           k >= 128 && k % 128 == 0;
+}
+
+extern "C" int imparo_moe_router_blocks(int n_tokens) { return (n_tokens + MOE_ROUTER_TOKENS - 1) / MOE_ROUTER_TOKENS; }
+
+extern "C" int imparo_moe_router_plan(const void* x, const void* w, const float* bias, const float* correction, int32_t* choice,
+                                      float* weight, int32_t* counts, int n_tokens, int n_router, int k, int top, int scoring,
+                                      int normalize, float scale, int always, int n_experts, int tile_rows, int32_t* slot_of_entry,
+                                      int32_t* entry_of_slot, int32_t* tiles, int max_tiles, imparo_stream stream) {
+    if (!x || !w || !choice || !weight || !counts || !slot_of_entry || !entry_of_slot || !tiles || n_tokens < 0) return IMPARO_BAD_ARGUMENT;
+    if (!imparo_moe_router_takes(n_tokens, n_router, n_experts, top, 1, always, k) || scale != scale || tile_rows < 1) return IMPARO_BAD_ARGUMENT;
+    if (scoring < MOE_SCORE_SOFTMAX || scoring > MOE_SCORE_CHOSEN || (((uintptr_t)x | (uintptr_t)w) & 15)) return IMPARO_BAD_ARGUMENT;
+    if ((long long)n_tokens * (top + always) > 0x7fffffffLL) return IMPARO_BAD_ARGUMENT;
+    if (max_tiles < imparo_moe_max_tiles(n_tokens * (top + always), n_experts, tile_rows)) return IMPARO_SCRATCH_TOO_SMALL;
+    const MoeRouteRules rules{n_router, 1, 1, normalize, scale, always};
+    const unsigned blocks = (unsigned)imparo_moe_router_blocks(n_tokens);
+    hipStream_t s = (hipStream_t)stream;
+    const int lds_bytes = (MOE_ROUTER_TOKENS + n_router) * MOE_ROUTER_LD * (int)sizeof(bf16_t);
+    if (hipFuncSetAttribute((const void*)k_moe_router, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (MOE_ROUTER_TOKENS + MOE_ROUTER_MAX) * MOE_ROUTER_LD * (int)sizeof(bf16_t)) != hipSuccess)
+        return IMPARO_LAUNCH_FAILED;
+    k_moe_router<<<blocks, 512, lds_bytes, s>>>((const bf16_t*)x, (const bf16_t*)w, bias, correction, choice, weight, counts, n_tokens,
+                                                n_router, k, top, scoring, rules, n_experts);
+    const int status = launch_status();
+    if (status != IMPARO_OK) return status;
+    k_moe_place<<<(n_tokens + MOE_PLACE_TOKENS - 1) / MOE_PLACE_TOKENS, 512, 0, s>>>(choice, counts, n_tokens, top + always, n_experts,
+                                                                                   tile_rows, slot_of_entry, entry_of_slot, tiles,
+                                                                                   max_tiles);
     return launch_status();
 }
 

@@ -142,6 +142,11 @@ _SIGNATURES = {
     "imparo_cast_rows": [P, P, P, I, I, I, P],
     "imparo_moe_route_plan_tokens": [],
     "imparo_moe_route_plan": [P, P, P, P, I, I, I, I, I, I, P, P, P, I, I, I, I, I, F, I, P],
+    "imparo_moe_router_takes": [I, I, I, I, I, I, I],
+    "imparo_moe_router_blocks": [I],
+    # x, w, bias, correction, choice, weight, counts, n_tokens, n_router, k, top, scoring, normalize, scale, always, n_experts,
+    # tile_rows, slot_of_entry, entry_of_slot, tiles, max_tiles, stream
+    "imparo_moe_router_plan": [P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, I, P, P, P, I, P],
     # x, y, h, h_dtype, choice, weight, slot_of_entry, top, n_experts, n_rows_x, rows, w_post, eps_post, w_next, eps_next,
     # out, out_dtype, n_out, width, stream
     "imparo_post_norm_add_moe": [P, P, P, I, P, P, P, I, I, I, P, P, F, P, F, P, I, I, I, P],

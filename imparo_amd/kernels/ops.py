@@ -1164,6 +1164,34 @@ def moe_route_plan(logits: torch.Tensor, correction: Optional[torch.Tensor], cho
         _dev(tiles, "tiles", torch.int32), tiles.shape[0], *rules, _stream()), "moe_route_plan")
 
 
+def moe_router_takes(n_tokens: int, n_router: int, n_experts: int, top: int, groups: int, always: int, k: int) -> bool:
+    """Whether `moe_router_plan` takes so many tokens and a router of so many outputs over rows of k."""
+    return bool(library().imparo_moe_router_takes(int(n_tokens), int(n_router), int(n_experts), int(top), int(groups), int(always), int(k)))
+
+
+def moe_router_blocks(n_tokens: int) -> int:
+    """The rows of `moe_router_plan`'s counts."""
+    return int(library().imparo_moe_router_blocks(int(n_tokens)))
+
+
+def moe_router_plan(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], correction: Optional[torch.Tensor],
+                    choice: torch.Tensor, weight: torch.Tensor, counts: torch.Tensor, top: int, n_experts: int, tile_rows: int,
+                    slot_of_entry: torch.Tensor, entry_of_slot: torch.Tensor, tiles: torch.Tensor, scoring: str = "softmax",
+                    normalize: bool = False, scale: float = 1.0, always: int = 0) -> None:
+    """The router's product x [n, k] . w [n_router, k]^T + bias (bfloat16 operands), `moe_route` and `moe_plan` in two launches.
+    The logits are the bits that the product alone gives. `counts` [moe_router_blocks(n), n_experts] int32 is scratch."""
+    n, k = x.shape
+    r, used = w.shape[0], top + always
+    _check(library().imparo_moe_router_plan(
+        _dev(x, "router input", torch.bfloat16), _dev(w, "router weight", torch.bfloat16, (r, k)),
+        _dev(bias, "router bias", torch.float32, (r,)), _dev(correction, "router correction", torch.float32, (r,)),
+        _dev(choice, "choice", torch.int32, (n, used)), _dev(weight, "choice weights", torch.float32, (n, used)),
+        _dev(counts, "counts", torch.int32, (moe_router_blocks(n), n_experts)), n, r, k, top, MOE_SCORINGS[scoring],
+        int(bool(normalize)), float(scale), always, n_experts, tile_rows, _dev(slot_of_entry, "slot_of_entry", torch.int32, (n * used,)),
+        _dev(entry_of_slot, "entry_of_slot", torch.int32, (n * used,)), _dev(tiles, "tiles", torch.int32), tiles.shape[0],
+        _stream()), "moe_router_plan")
+
+
 def moe_tile_rows(n_entries: int, n_experts: int, dtype: torch.dtype) -> int:
     return int(library().imparo_moe_tile_rows(int(n_entries), int(n_experts), 0 if dtype == torch.float32 else 1))
 

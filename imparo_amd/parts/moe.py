@@ -242,7 +242,11 @@ class RoutedExperts:
                 shared_out.append(self.shared.forward(ctx, n))
             finally:
                 ctx.stream = stream
-        z = None if routed is not None else self.router(ctx, n, torch.float32, "router_logits")
+        # a prompt's router takes choice and plan along, where nothing else reads its logits
+        rides = (routed is None and X > 0 and n.dtype == torch.bfloat16
+                 and self.router.weight.dtype == torch.bfloat16 and not (self.shared is not None and self.shared_gated)
+                 and ops.moe_router_takes(T, self.n_router, X, top, self.group_count, self.always, self.width))
+        z = None if routed is not None or rides else self.router(ctx, n, torch.float32, "router_logits")
         if shared_out is not None:
             shared_out.append(z)
         choice = ws.get("moe_choice", (T, used), torch.int32)
@@ -260,7 +264,12 @@ class RoutedExperts:
             rows = ops.moe_tile_rows(entries, X, self.up.dtype)
             tiles = ws.get("moe_tiles", (ops.moe_max_tiles(entries, X, rows), 3), torch.int32)
             entry_of_slot = ws.get("moe_entry_of_slot", (entries,), torch.int32)
-            if T <= ops.moe_route_plan_tokens():      # a decode step: choice and plan in one launch
+            if rides:
+                counts = ws.get("moe_counts", (ops.moe_router_blocks(T), X), torch.int32)
+                ops.moe_router_plan(n, self.router.weight, self.router.bias, self.correction, choice, weight, counts, top, X, rows,
+                                    slot_of_entry, entry_of_slot, tiles, scoring=self.scoring, normalize=self.normalize,
+                                    scale=self.route_scale, always=self.always)
+            elif T <= ops.moe_route_plan_tokens():      # a decode step: choice and plan in one launch
                 ops.moe_route_plan(z, self.correction, choice, weight, top, X, rows, slot_of_entry, entry_of_slot, tiles,
                                    **rules)
             else:
