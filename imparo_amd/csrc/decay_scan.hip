@@ -1026,6 +1026,23 @@ __global__ void k_head_prepare(float* __restrict__ rows, int ld, int off, int n_
     for (int i = 2 * n_freq + lane; i < dim; i += WAVE) x[i] *= f;
 }
 
+// The same without a rotation, for heads of whole 16-byte pieces, at most one a lane: LANES lanes a head, which keep it in registers
+// where it was read twice, a value a lane at a time. Bound by its bytes. 3,328 rows of 8 heads of 128 as unit vectors 9.9 -> 6.5 us.
+template <int LANES>
+__global__ __launch_bounds__(256) void k_head_prepare_four(float* __restrict__ rows, int ld, int off, int n_tokens, int heads, int dim,
+                                                           int unit, float unit_eps, int n_first, float scale_first, float scale_rest) {
+    const int lane = threadIdx.x % LANES;
+    const long long all = (long long)n_tokens * heads, at = (long long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const long long id = at < all ? at : all - 1;            // (no lane leaves before the sums)
+    const int t = (int)(id / heads), j = (int)(id - (long long)t * heads);
+    float4* x = reinterpret_cast<float4*>(rows + (size_t)t * ld + off + (size_t)j * dim) + min(lane, dim / 4 - 1);
+    const bool on = lane < dim / 4;
+    const float4 v = *x;
+    float f = j < n_first ? scale_first : scale_rest;
+    if (unit) f *= 1.0f / sqrtf(sum_near_first<LANES>(on ? fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))) : 0.f) + unit_eps);
+    if (on && at < all) *x = make_float4(v.x * f, v.y * f, v.z * f, v.w * f);
+}
+
 extern "C" int imparo_head_prepare(float* rows, int ld, int off, int n_tokens, int heads, int dim, int unit,
                                    float unit_eps, const float* inv_freq, int n_freq, int interleaved,
                                    const int32_t* positions, int n_first, float scale_first, float scale_rest,
@@ -1034,6 +1051,15 @@ extern "C" int imparo_head_prepare(float* rows, int ld, int off, int n_tokens, i
     if (n_freq < 0 || 2 * n_freq > dim || (n_freq && (!inv_freq || !positions))) return IMPARO_BAD_ARGUMENT;
     if (n_tokens == 0) return IMPARO_OK;
     const long long waves = (long long)n_tokens * heads;
+    if (!n_freq && dim % 4 == 0 && dim <= 256 && ld % 4 == 0 && off % 4 == 0 && !((uintptr_t)rows & 15)) {
+        if (dim <= 128)
+            k_head_prepare_four<32><<<(unsigned)((waves + 7) / 8), 256, 0, (hipStream_t)stream>>>(rows, ld, off, n_tokens, heads, dim, unit,
+                                                                                                unit_eps, n_first, scale_first, scale_rest);
+        else
+            k_head_prepare_four<64><<<(unsigned)((waves + 3) / 4), 256, 0, (hipStream_t)stream>>>(rows, ld, off, n_tokens, heads, dim, unit,
+                                                                                                unit_eps, n_first, scale_first, scale_rest);
+        return launch_status();
+    }
     k_head_prepare<<<(unsigned)((waves + 3) / 4), 4 * WAVE, 0, (hipStream_t)stream>>>(
         rows, ld, off, n_tokens, heads, dim, unit, unit_eps, inv_freq, n_freq, interleaved, positions, n_first,
         scale_first, scale_rest);
@@ -1075,6 +1101,60 @@ __global__ __launch_bounds__(256) void k_gated_group_norm(const float* __restric
         y = y * rs * (w ? w[(size_t)g * part + i] : 1.f);
         if (!gate_first) y *= gv;
         store_f32<TOut>(out, (size_t)t * width + (size_t)g * part + i, y);
+    }
+}
+
+// A short part of whole 16-byte pieces, Q of them a lane at most: LANES lanes a part, everything asked for at once and kept, where a
+// wave asked value by value and read the part and its gate again behind the sum. Bound by its bytes. 3,328 rows of 8 parts of 128, bfloat16
+// out, 15.5 -> 10.6 us.
+template <typename TOut, int LANES, int Q>
+__global__ __launch_bounds__(256) void k_gated_group_norm_four(const float* __restrict__ x, const float* __restrict__ gate,
+                                                               int gate_ld, int gate_off, const float* __restrict__ w,
+                                                               TOut* __restrict__ out, int n_tokens, int width, int groups,
+                                                               float eps, int gate_first, int gate_act) {
+    const int lane = threadIdx.x % LANES, part = width / groups;
+    const long long all = (long long)n_tokens * groups, at = (long long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const long long id = at < all ? at : all - 1;            // (no lane leaves before the sum)
+    const int t = (int)(id / groups), g = (int)(id - (long long)t * groups);
+    const float* xr = x + (size_t)t * width + (size_t)g * part;
+    const float* gr = gate ? gate + (size_t)t * gate_ld + gate_off + (size_t)g * part : nullptr;
+    float y[Q][4], gv[Q][4], wv[Q][4];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = min((lane + q * LANES) * 4, part - 4);
+        const float4 a = *reinterpret_cast<const float4*>(xr + i);
+        const float4 one = make_float4(1.f, 1.f, 1.f, 1.f);
+        const float4 b = gr ? *reinterpret_cast<const float4*>(gr + i) : one;
+        const float4 c = w ? *reinterpret_cast<const float4*>(w + (size_t)g * part + i) : one;
+        y[q][0] = a.x, y[q][1] = a.y, y[q][2] = a.z, y[q][3] = a.w;
+        gv[q][0] = b.x, gv[q][1] = b.y, gv[q][2] = b.z, gv[q][3] = b.w;
+        wv[q][0] = c.x, wv[q][1] = c.y, wv[q][2] = c.z, wv[q][3] = c.w;
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            gv[q][i] = gr ? ds_gate(gv[q][i], gate_act) : 1.f;
+            if (gate_first) y[q][i] *= gv[q][i];
+            if ((lane + q * LANES) * 4 < part) ss = fmaf(y[q][i], y[q][i], ss);
+        }
+    const float rs = 1.0f / sqrtf(sum_near_first<LANES>(ss) / (float)part + eps);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = (lane + q * LANES) * 4;
+        float v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = y[q][k] * rs * wv[q][k];
+            if (!gate_first) v[k] *= gv[q][k];
+        }
+        if (i >= part || at >= all) continue;
+        TOut* to = out + (size_t)t * width + (size_t)g * part + i;
+        if constexpr (sizeof(TOut) == 4)
+            *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+            *reinterpret_cast<uint2*>(to) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
     }
 }
 
@@ -1138,6 +1218,20 @@ extern "C" int imparo_gated_group_norm(const float* x, const float* gate, int ga
         if (out_dtype == IMPARO_BF16) { GGN_PER(bf16_t); } else { GGN_PER(float); }
 #undef GGN_PER
 #undef GGN_BLOCK
+        return launch_status();
+    }
+    if (part % 4 == 0 && part <= 512 && gate_ld % 4 == 0 && gate_off % 4 == 0 &&
+        !(((uintptr_t)x | (uintptr_t)gate | (uintptr_t)w | (uintptr_t)out) & 15)) {
+#define GGN_FOUR(T, LANES, Q)                                                                                        \
+    k_gated_group_norm_four<T, LANES, Q><<<(unsigned)((parts + 256 / LANES - 1) / (256 / LANES)), 256, 0, s>>>(      \
+        x, gate, gate_ld, gate_off, w, (T*)out, n_tokens, width, groups, eps, gate_first, gate_act)
+#define GGN_FIT(T)                                                                                                   \
+    if (part <= 128) GGN_FOUR(T, 32, 1);                                                                             \
+    else if (part <= 256) GGN_FOUR(T, 64, 1);                                                                        \
+    else GGN_FOUR(T, 64, 2)
+        if (out_dtype == IMPARO_BF16) { GGN_FIT(bf16_t); } else { GGN_FIT(float); }
+#undef GGN_FIT
+#undef GGN_FOUR
         return launch_status();
     }
     const unsigned blocks = (unsigned)((parts + 3) / 4);
