@@ -306,7 +306,8 @@ __device__ __forceinline__ void head_elements(HeadElements<ND>& h, const float* 
         h.e[dk][4] = b.x, h.e[dk][5] = b.y, h.e[dk][6] = b.z, h.e[dk][7] = b.w;
     }
 }
-template <int ND>
+// GIVEN: the norm runs over more than the head, and its scale is `given` (which may be 0: of a row whose squares overflow).
+template <int ND, bool GIVEN = false>
 __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadElements<ND>& h, const float* weight,
                                                float eps, bool rotate, int interleaved, const float* sn_tab,
                                                const float* cs_tab, bool valid, int g, float given = 0.f) {
@@ -314,8 +315,8 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
     static_assert(D % 64 == 0, "pairs inside a lane");
     auto& e = h.e;
     if (weight) {                      // (in LDS)
-        float scale = given;           // (of a norm over more than the head)
-        if (given == 0.f) {
+        float scale = given;
+        if constexpr (!GIVEN) {
             float ss = 0.f;
 #pragma unroll
             for (int dk = 0; dk < NK; ++dk)
@@ -531,7 +532,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
         if constexpr (WHOLE) {
             q_given = head_norm_scale(sq_of[0] + sq_of[1] + sq_of[2] + sq_of[3], heads * D, fq.eps);
         }
-        normed_rotated<ND>(st.q, qh, fq.q_weight ? qw_tab + (WHOLE ? c * D : 0) : nullptr, fq.eps, fq.inv_freq != nullptr,
+        normed_rotated<ND, WHOLE>(st.q, qh, fq.q_weight ? qw_tab + (WHOLE ? c * D : 0) : nullptr, fq.eps, fq.inv_freq != nullptr,
                            fq.interleaved, sn_tab, cs_tab, qvalid, g, q_given);
     }
     // the row's own key from the projection's row, in the layout of a tile's rows: dims dk*32 + 8*g + j
@@ -540,7 +541,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
         head_elements<ND>(kh, k_raw, g);
         float k_given = 0.f;
         if constexpr (WHOLE) k_given = head_norm_scale(sk_of[0] + sk_of[1] + sk_of[2] + sk_of[3], kv_heads * D, fq.eps);
-        normed_rotated<ND>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
+        normed_rotated<ND, WHOLE>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
                            sn_tab, cs_tab, true, g, k_given);
     };
 #pragma unroll

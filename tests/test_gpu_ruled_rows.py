@@ -85,3 +85,57 @@ def test_ruled_rows_of_a_wrong_width_are_refused():
     takes = ops().attention_decode_qkv_ruled_takes
     assert takes(33, 33, 64, 32, False) and takes(8, 2, 64, 0, False) and not takes(8, 2, 64, 16, False)
     assert not takes(33, 1, 64, 32, True) and not takes(17, 17, 64, 32, True) and not takes(8, 2, 128, 64, False)
+
+
+def _one_and_two_launches(rows, H, Hk, qw, kw, freq, over, lens, brings=True, magnitude=1.0, gated=False, interleaved=False, page=64):
+    """(outputs, keys, values) of the one launch and of the two that it stands for, on the CPU."""
+    R, D = rows.shape[0], 64
+    ctx = hand_context([(c - 1, 1) for c in lens], page, sum(-(-c // page) for c in lens) + 2, torch.bfloat16, DEV,
+                       kv_sites={0: (Hk, D)}, v_transposed=True)
+    k0, v0, table = ctx.kv(0)
+    k0.copy_(rnd(*k0.shape, seed=1)), v0.copy_(rnd(*v0.shape, seed=2))
+    rule = ops().attention_rule(H, softcap=20.0, sink=rnd(H, seed=7).to(DEV))
+    if gated:
+        rule = rule.with_gate(rows, (H + 2 * Hk) * D)
+    splits = -(-ops().attention_ruled_keys(max(lens), None, rule) // 256)
+    part = lambda n: torch.full((R * H * splits * n,), float("nan"), device=DEV)
+    got = []
+    for one in (True, False):
+        k, v = k0.clone(), v0.clone()
+        out = torch.full((R, H * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        tail = (part(D), part(2), ctx.single_rows, R, ctx.seg_start, ctx.positions, table)
+        if one:
+            ops().attention_decode_qkv(rows, qw, kw, 1e-5, freq, k, v, out, *tail, H, 0.125, None, max(lens), write_kv=brings,
+                                       rule=rule, magnitude=magnitude, whole=over == "projection", interleaved=interleaved)
+        else:
+            q = torch.empty(R, H, D, dtype=torch.bfloat16, device=DEV)
+            where = (ctx.positions, ctx.row_of_token, table if brings else None, page, q, k if brings else None,
+                     v if brings else None, H, Hk if brings else 0, D)
+            if gated or over == "projection" or magnitude != 1.0:     # (as the attention part chooses)
+                ops().qk_row_norm_rope_store(rows, qw, qw if kw is None else kw, over if qw is not None else None, 1e-5, freq, magnitude,
+                                             *where, D, v_transposed=True, interleaved=interleaved)
+            else:
+                ops().qk_norm_rope_store(rows, qw, kw, 1e-5, freq, *where, v_transposed=True, interleaved=interleaved)
+            ops().attention_decode(q, k, v, out, *tail, 0.125, None, max(lens), exact=True, rule=rule)
+        got.append([t.cpu().float() for t in (out, k, v)])
+    return got
+
+
+def _same(one, two):
+    for a, b in zip(one, two):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+@pytest.mark.parametrize("H,Hk", [(8, 2), (32, 16)])
+def test_norms_over_rows_whose_squares_leave_float32(H, Hk):
+    """A row whose sum of squares overflows has a scale of exactly zero: zeros, and not every head normed by itself; an infinity
+    gives NaN where it stands. In queries, and in the keys that are stored."""
+    D, lens = 64, (40, 300, 64, 257)
+    rows = rnd(len(lens), (H + 2 * Hk) * D, seed=3)
+    rows[0, 5] = 3e19                                    # (its square is past 3.4e38)
+    rows[1, 70] = float("inf")
+    rows[2, H * D + 9] = -2e30
+    rows[3, H * D + D + 1] = float("-inf")
+    qw, kw = (1 + 0.1 * rnd(H * D, seed=4)).to(DEV), (1 + 0.1 * rnd(Hk * D, seed=5)).to(DEV)
+    one, two = _one_and_two_launches(rows.to(DEV), H, Hk, qw, kw, torch.linspace(1.0, 0.01, 32, device=DEV), "projection", lens)
+    _same(one, two)
