@@ -457,7 +457,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
         head_elements<ND>(qh, row_in + (size_t)head * D, g);
         freq = (fq.inv_freq ? fq.inv_freq : row_in)[min((int)threadIdx.x, D / 2 - 1)];
         q_norm = make_float2((fq.q_weight ? fq.q_weight : row_in)[norm_from], (fq.q_weight ? fq.q_weight : row_in)[norm_from + 1]);
-        const float* kw_in = fq.q_weight ? fq.k_weight + (WHOLE && brings ? kvh * D : 0) : row_in;
+        // (rows of queries alone have no key weight: what is handed in its place may be shorter than a head)
+        const float* kw_in = fq.q_weight && brings ? fq.k_weight + (WHOLE ? kvh * D : 0) : row_in;
         k_norm = make_float2(kw_in[norm_from], kw_in[norm_from + 1]);
         own_raw = *reinterpret_cast<const float4*>(row_in + (size_t)(!brings ? 0 : lane < D / 4 ? heads + kvh : heads + kv_heads + kvh) * D + own_at);
         __builtin_amdgcn_sched_barrier(0);

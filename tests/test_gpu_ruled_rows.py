@@ -139,3 +139,16 @@ def test_norms_over_rows_whose_squares_leave_float32(H, Hk):
     qw, kw = (1 + 0.1 * rnd(H * D, seed=4)).to(DEV), (1 + 0.1 * rnd(Hk * D, seed=5)).to(DEV)
     one, two = _one_and_two_launches(rows.to(DEV), H, Hk, qw, kw, torch.linspace(1.0, 0.01, 32, device=DEV), "projection", lens)
     _same(one, two)
+
+
+@pytest.mark.parametrize("key_weight", [1, 4, None])
+def test_rows_of_queries_alone_read_no_key_weight(key_weight):
+    """Another layer's cache: whatever stands in the key weight's place (here shorter than a head, or the query weight) is not read."""
+    H, Hk, D, lens = 16, 8, 64, (1, 33, 256, 300)
+    rows = rnd(len(lens), H * D, seed=3).to(DEV)
+    qw = (1 + 0.1 * rnd(H * D, seed=4)).to(DEV)
+    kw = qw if key_weight is None else torch.full((key_weight,), float("nan"), device=DEV)
+    one, _ = _one_and_two_launches(rows, H, Hk, qw, kw, torch.linspace(1.0, 0.01, 32, device=DEV), "projection", lens, brings=False)
+    _, two = _one_and_two_launches(rows, H, Hk, qw, qw, torch.linspace(1.0, 0.01, 32, device=DEV), "projection", lens, brings=False)
+    assert bool(torch.isfinite(two[0]).all())
+    _same(one, two)
