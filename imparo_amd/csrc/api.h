@@ -345,11 +345,12 @@ int imparo_attention_decode_qkv(const float* qkv, const float* q_weight, const f
 // The same under a rule, with exact weights (imparo_attention_decode_ruled), out of rows row_ld floats apart (a multiple of 4).
 // brings: the rows hold the new keys and values, which go into their pages; 0: queries only, of a layer that reads another
 // layer's cache, where the row's own key is already. magnitude: a factor on sines and cosines. whole: the norms run over all
-// query heads and over all key heads, weights as wide.
+// query heads and over all key heads, weights as wide. far_first: a norm a head adds its squares in the order of
+// imparo_qk_row_norm_rope_store, else of imparo_qk_norm_rope_store: a row has the bits of the two launches.
 int imparo_attention_decode_qkv_ruled_takes(int heads, int kv_heads, int head_dim, int n_freq, int whole);
 int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int whole);
 int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, int brings, const float* q_weight, const float* k_weight,
-                                      float eps, const float* inv_freq, int n_freq, int interleaved, float magnitude, int whole,
+                                      float eps, const float* inv_freq, int n_freq, int interleaved, float magnitude, int whole, int far_first,
                                       void* k_cache, void* v_cache, void* out, float* part_o, float* part_ml,
                                       const int32_t* rows, int n_rows, const int32_t* seg_start, const int32_t* positions,
                                       const int32_t* block_table, int table_stride, int page_size, int heads, int kv_heads,

@@ -287,6 +287,43 @@ struct FromQkv {
     int whole;                  // norms over all query heads and all key heads of a row, weights as wide
 };
 
+// The sum of a head of 64's squares in the order of the launch that norms the rows of longer steps, so that a row has one sum in
+// all of them (a key in the cache keeps its bits however many rows ran beside it). That launch has a value a lane and adds
+// lanes 1, 2, 4, .. 32 apart (rope_cache.hip: a head a wave), or FAR_FIRST 32, 16, .. 1 apart (whole rows); here a lane
+// has dims 8 g + j and 32 + 8 g + j, so those 8 and 16 apart lie in lanes 16 and 32 apart. 16 heads by 8, us with a lane's own squares
+// in a chain | near | far first: 8 rows over 200 keys 8.60 | 8.70 | 9.02, 16 over 4,000 30.4 | 30.5 | 33.3 (far first takes 132
+// registers where one split has a block: three waves a SIMD, and not four).
+template <bool FAR_FIRST>
+__device__ __forceinline__ float squares_as_stored(const float (&e)[2][8]) {
+#pragma clang fp contract(off)
+    // (depth first: few sums live at a time, beside the tiles on their way)
+    if constexpr (FAR_FIRST) {
+        auto of = [&](int j) __attribute__((always_inline)) { return sum_32_16(e[0][j] * e[0][j] + e[1][j] * e[1][j]); };
+        float sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {                        // (no more of the eight at a time than registers are free)
+            float of_four = 0.f;
+#pragma unroll
+            for (int n = 0; n < 4; n += 2) {
+                const float first = of(j + n);
+                __builtin_amdgcn_sched_barrier(0);
+                const float both = first + of(j + n + 4);
+                __builtin_amdgcn_sched_barrier(0);
+                of_four = n ? of_four + both : both;
+            }
+            sum = j ? sum + of_four : of_four;
+        }
+        return sum;
+    }
+    auto of = [&](int dk) __attribute__((always_inline)) {
+        auto two = [&](int j) __attribute__((always_inline)) { return e[dk][j] * e[dk][j] + e[dk][j + 1] * e[dk][j + 1]; };
+        const float near = two(0) + two(2);
+        return sum_16_32(near + (two(4) + two(6)));
+    };
+    const float low = of(0);
+    return low + of(1);
+}
+
 // One head's 8 x NK elements of a lane (dims dk*32 + 8*g + j): asked for early (`head_elements`, with the
 // norm's weights), then normed, rotated and rounded to bfloat16 (`normed_rotated`) once the block's sines
 // and cosines are there. All lanes with the same lane % 16 share a head: the sum of squares crosses
@@ -306,8 +343,10 @@ __device__ __forceinline__ void head_elements(HeadElements<ND>& h, const float* 
         h.e[dk][4] = b.x, h.e[dk][5] = b.y, h.e[dk][6] = b.z, h.e[dk][7] = b.w;
     }
 }
-// GIVEN: the norm runs over more than the head, and its scale is `given` (which may be 0: of a row whose squares overflow).
-template <int ND, bool GIVEN = false>
+// NORM_GIVEN: the norm runs over more than the head, and its scale is `given` (which may be 0: of a row whose squares overflow).
+// NORM_NEAR_FIRST, NORM_FAR_FIRST: squares in the order of another launch (squares_as_stored).
+enum { NORM_LANES, NORM_GIVEN, NORM_NEAR_FIRST, NORM_FAR_FIRST };
+template <int ND, int NORM = NORM_LANES>
 __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadElements<ND>& h, const float* weight,
                                                float eps, bool rotate, int interleaved, const float* sn_tab,
                                                const float* cs_tab, bool valid, int g, float given = 0.f) {
@@ -316,7 +355,9 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
     auto& e = h.e;
     if (weight) {                      // (in LDS)
         float scale = given;
-        if constexpr (!GIVEN) {
+        if constexpr (NORM == NORM_NEAR_FIRST || NORM == NORM_FAR_FIRST) {
+            scale = head_norm_scale(squares_as_stored<NORM == NORM_FAR_FIRST>(e), D, eps);
+        } else if constexpr (NORM == NORM_LANES) {
             float ss = 0.f;
 #pragma unroll
             for (int dk = 0; dk < NK; ++dk)
@@ -370,10 +411,10 @@ __device__ __forceinline__ void normed_rotated(Frag8 (&out)[(ND + 1) / 2], HeadE
 // share), nor three or four splits (16 waves on one CU: 1,000 keys 17.7 | 13.4, queries given 12.9 | 11.7).
 // EXACT: see decode_tile; part of the kernel's type, as branches on it inside a tile kept the scheduler from filling one weight's
 // waits with the next one's work.
-// WHOLE (from the projection's rows): the norms run over all query heads and over all key heads of a token, weights as wide as
+// NORM (from the projection's rows): see normed_rotated. NORM_GIVEN, WHOLE: the norms run over all query heads and over all key heads of a token, weights as wide as
 // those; every block adds up the squares of its whole row, 6 KB of 16 heads and 8, beside the sines and cosines.
-template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1, bool EXACT = false, bool WHOLE = false>
-__global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - SPLITS : 4) void k_attn_decode(
+template <int ND, bool FROM_QKV, bool EXT = false, int SPLITS = 1, bool EXACT = false, int NORM = NORM_LANES>
+__global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : NORM == NORM_GIVEN ? 4 - SPLITS : NORM == NORM_FAR_FIRST && SPLITS == 1 ? 3 : 4) void k_attn_decode(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out,
     const int32_t* __restrict__ rows, const int32_t* __restrict__ seg_start, const int32_t* __restrict__ positions,
@@ -381,6 +422,7 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
     float scale, int window, int n_splits, FromQkv fq, Rule rule) {
     constexpr int D = ND * 16, NK = (ND + 1) / 2;
     constexpr int TILES = DEC_SPLIT / (MFMA_WAVES * 32);   // tiles a wave takes at most
+    constexpr bool WHOLE = NORM == NORM_GIVEN;
     __shared__ float sm[SPLITS * MFMA_WAVES][16], sl[SPLITS * MFMA_WAVES][16];
     __shared__ float so[SPLITS * MFMA_WAVES][16][D + 1];
     __shared__ float sn_tab[FROM_QKV ? D / 2 : 1], cs_tab[FROM_QKV ? D / 2 : 1];
@@ -533,8 +575,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
         if constexpr (WHOLE) {
             q_given = head_norm_scale(sq_of[0] + sq_of[1] + sq_of[2] + sq_of[3], heads * D, fq.eps);
         }
-        normed_rotated<ND, WHOLE>(st.q, qh, fq.q_weight ? qw_tab + (WHOLE ? c * D : 0) : nullptr, fq.eps, fq.inv_freq != nullptr,
-                           fq.interleaved, sn_tab, cs_tab, qvalid, g, q_given);
+        normed_rotated<ND, NORM>(st.q, qh, fq.q_weight ? qw_tab + (WHOLE ? c * D : 0) : nullptr, fq.eps, fq.inv_freq != nullptr,
+                                 fq.interleaved, sn_tab, cs_tab, qvalid, g, q_given);
     }
     // the row's own key from the projection's row, in the layout of a tile's rows: dims dk*32 + 8*g + j
     auto own_key = [&](auto& kf) __attribute__((always_inline)) {
@@ -542,8 +584,8 @@ __global__ __launch_bounds__(SPLITS * MFMA_WAVES * 64, ND > 4 ? 2 : WHOLE ? 4 - 
         head_elements<ND>(kh, k_raw, g);
         float k_given = 0.f;
         if constexpr (WHOLE) k_given = head_norm_scale(sk_of[0] + sk_of[1] + sk_of[2] + sk_of[3], kv_heads * D, fq.eps);
-        normed_rotated<ND, WHOLE>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
-                           sn_tab, cs_tab, true, g, k_given);
+        normed_rotated<ND, NORM>(kf, kh, fq.k_weight ? kw_tab : nullptr, fq.eps, fq.inv_freq != nullptr, fq.interleaved,
+                                 sn_tab, cs_tab, true, g, k_given);
     };
 #pragma unroll
     for (int j = 0; j < TILES; ++j) {
@@ -1565,7 +1607,7 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
                                    const int32_t* block_table, int table_stride, int page_size,
                                    int heads, int kv_heads, int head_dim, int n_pages, float scale, int window,
                                    int n_splits, hipStream_t s, const FromQkv* from_qkv = nullptr, int exact = 0,
-                                   const ImparoAttentionRule* given = nullptr) {
+                                   const ImparoAttentionRule* given = nullptr, bool far_first = false) {
     const int G = heads / kv_heads;
     const Rule rule = rule_of(given);
     // the merge moves four elements of a head in one access
@@ -1573,21 +1615,22 @@ static int attention_decode_launch(const void* q, const void* k_cache, const voi
     // two splits: one block takes both and there is no merge, where that is the faster way (k_attn_decode)
     const bool in_block = n_splits == 2 && !(from_qkv && head_dim > 64);
     dim3 grid(in_block ? 1 : n_splits, kv_heads * ((G + 15) / 16), n_rows);
-#define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT, WHOLE)                                                         \
-    k_attn_decode<ND, QKV, EXT, SPLITS, EXACT, WHOLE><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                            \
+#define DECODE_GO(ND, QKV, EXT, SPLITS, Q, FQ, EXACT, NORM)                                                          \
+    k_attn_decode<ND, QKV, EXT, SPLITS, EXACT, NORM><<<grid, SPLITS * MFMA_WAVES * 64, 0, s>>>(                            \
         Q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, part_o, part_ml, (bf16_t*)out, rows, seg_start,           \
         positions, block_table, table_stride, page_size, heads, kv_heads, n_pages, scale, window, n_splits, FQ, rule)
-#define DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, WHOLE)                                                               \
+#define DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, NORM)                                                                \
     do {                                                                                                             \
-        if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT, WHOLE);                         \
-        else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT, WHOLE);                                                        \
+        if (in_block) DECODE_GO(ND, QKV, EXT, (QKV && ND > 4 ? 1 : 2), Q, FQ, EXACT, NORM);                          \
+        else DECODE_GO(ND, QKV, EXT, 1, Q, FQ, EXACT, NORM);                                                         \
     } while (0)
-#define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT) DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, false)
+#define DECODE_ANY(ND, QKV, EXT, Q, FQ, EXACT) DECODE_NORM(ND, QKV, EXT, Q, FQ, EXACT, NORM_LANES)
     if (given && !exact) return IMPARO_BAD_ARGUMENT;         // (the rules run with exact weights)
     if (from_qkv) {
         if (given && head_dim != 64) return IMPARO_BAD_ARGUMENT;
-        if (given && from_qkv->whole) DECODE_NORM(4, true, true, nullptr, *from_qkv, true, true);
-        else if (given) DECODE_ANY(4, true, true, nullptr, *from_qkv, true);
+        if (given && from_qkv->whole) DECODE_NORM(4, true, true, nullptr, *from_qkv, true, NORM_GIVEN);
+        else if (given && far_first) DECODE_NORM(4, true, true, nullptr, *from_qkv, true, NORM_FAR_FIRST);
+        else if (given) DECODE_NORM(4, true, true, nullptr, *from_qkv, true, NORM_NEAR_FIRST);
         else if (head_dim == 64) DECODE_ANY(4, true, false, nullptr, *from_qkv, false);
         else if (head_dim == 128) DECODE_ANY(8, true, false, nullptr, *from_qkv, false);
         else return IMPARO_BAD_ARGUMENT;
@@ -1695,7 +1738,7 @@ static int attention_decode_qkv_entry(FromQkv fq, int n_freq, void* k_cache, voi
                                       const int32_t* rows, int n_rows, const int32_t* seg_start, const int32_t* positions,
                                       const int32_t* block_table, int table_stride, int page_size, int heads, int kv_heads,
                                       int head_dim, int n_pages, float scale, int window, int n_splits, imparo_stream stream,
-                                      const ImparoAttentionRule* rule = nullptr) {
+                                      const ImparoAttentionRule* rule = nullptr, bool far_first = false) {
     const int bad = check_common(fq.qkv, k_cache, v_cache, out, rows, seg_start, positions, block_table, table_stride,
                                  page_size, heads, kv_heads, head_dim, n_pages, window);
     if (bad) return bad;
@@ -1709,7 +1752,7 @@ static int attention_decode_qkv_entry(FromQkv fq, int n_freq, void* k_cache, voi
     if (n_freq == 0) fq.inv_freq = nullptr;
     return attention_decode_launch(nullptr, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
                                    block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale,
-                                   window, n_splits, (hipStream_t)stream, &fq, rule ? 1 : 0, rule);
+                                   window, n_splits, (hipStream_t)stream, &fq, rule ? 1 : 0, rule, far_first);
 }
 
 extern "C" int imparo_attention_decode_qkv(const float* qkv, const float* q_weight, const float* k_weight, float eps,
@@ -1743,11 +1786,12 @@ extern "C" int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, 
 // The same under a rule, with exact weights, out of rows that may be wider than the heads (row_ld floats apart). brings: the
 // rows hold the new keys and values, which are written into their pages; 0: queries only, of a layer that reads another's cache,
 // where the new keys are already. magnitude: a factor on sines and cosines. whole: q_weight and k_weight are as wide as all
-// query heads and all key heads, and the norms run over those.
+// query heads and all key heads, and the norms run over those. far_first: a norm a head adds its squares as
+// imparo_qk_row_norm_rope_store does, else as imparo_qk_norm_rope_store.
 extern "C" int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, int brings, const float* q_weight,
                                                  const float* k_weight, float eps, const float* inv_freq, int n_freq,
-                                                 int interleaved, float magnitude, int whole, void* k_cache, void* v_cache, void* out,
-                                                 float* part_o, float* part_ml, const int32_t* rows, int n_rows,
+                                                 int interleaved, float magnitude, int whole, int far_first, void* k_cache,
+                                                 void* v_cache, void* out, float* part_o, float* part_ml, const int32_t* rows, int n_rows,
                                                  const int32_t* seg_start, const int32_t* positions,
                                                  const int32_t* block_table, int table_stride, int page_size, int heads,
                                                  int kv_heads, int head_dim, int n_pages, float scale, int window,
@@ -1762,7 +1806,7 @@ extern "C" int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, i
                      brings ? (bf16_t*)v_cache : nullptr, eps, interleaved, row_ld, brings != 0, magnitude, whole != 0};
     return attention_decode_qkv_entry(fq, n_freq, k_cache, v_cache, out, part_o, part_ml, rows, n_rows, seg_start, positions,
                                       block_table, table_stride, page_size, heads, kv_heads, head_dim, n_pages, scale, window,
-                                      n_splits, stream, rule);
+                                      n_splits, stream, rule, far_first != 0);
 }
 
 // ---------------------------------------------------------------- decode without a workspace argument

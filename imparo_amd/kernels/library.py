@@ -38,9 +38,9 @@ _SIGNATURES = {
     # qkv, q_w, k_w, eps, inv_freq, n_freq, interleaved, k_cache, v_cache, write_kv, out, part_o, part_ml, rows, n_rows,
     # seg_start, positions, table, stride, page, heads, kv_heads, head_dim, n_pages, scale, window, n_splits, stream
     "imparo_attention_decode_qkv": [P, P, P, F, P, I, I, P, P, I, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, I, I, P],
-    # qkv, row_ld, brings, q_w, k_w, eps, inv_freq, n_freq, interleaved, magnitude, whole, k_cache, v_cache, out, part_o, part_ml, rows,
-    # n_rows, seg_start, positions, table, stride, page, heads, kv_heads, head_dim, n_pages, scale, window, n_splits, rule, stream
-    "imparo_attention_decode_qkv_ruled": [P, I, I, P, P, F, P, I, I, F, I, P, P, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
+    # qkv, row_ld, brings, q_w, k_w, eps, inv_freq, n_freq, interleaved, magnitude, whole, far_first, k_cache, v_cache, out, part_o,
+    # part_ml, rows, n_rows, seg_start, positions, table, stride, page, heads, kv_heads, head_dim, n_pages, scale, window, n_splits, rule, stream
+    "imparo_attention_decode_qkv_ruled": [P, I, I, P, P, F, P, I, I, F, I, I, P, P, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
     "imparo_attention_decode_exact": [P, P, P, P, P, P, P, I, P, P, P, I, I, I, I, I, I, F, I, I, P],
     "imparo_attention_prefill_exact": [P, P, P, P, P, P, I, P, I, I, P, P, P, P, I, I, I, I, I, I, F, I, P],
     # as the exact forms, with the address of an AttentionRule before the stream

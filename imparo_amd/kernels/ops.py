@@ -571,13 +571,14 @@ def attention_decode_qkv(qkv, q_weight, k_weight, eps: float, inv_freq, k_cache,
                          rows, n_rows: int, seg_start, positions, block_table, heads: int, scale: float,
                          window: Optional[int], max_context: int, interleaved: bool = False,
                          write_kv: bool = True, rule: Optional[AttentionRule] = None, magnitude: float = 1.0,
-                         whole: bool = False) -> torch.Tensor:
+                         whole: bool = False, row_store: bool = False) -> torch.Tensor:
     """qk_norm_rope_store and attention_decode in one launch less, for a step whose rows all bring one
     token: `qkv` is the fused projection's float32 rows; the new keys and values are weighed in from
     registers and, with `write_kv`, written into their pages (V pages transposed). With a `rule` (and exact weights) the
     rows may be wider (gates behind the heads) and sines and cosines carry `magnitude`; without `write_kv` they then hold
     queries only, whose keys are all in the cache; `whole`: the norms run over all query heads and all key heads of a row,
-    weights as wide as those (without `write_kv` the key weight is not read)."""
+    weights as wide as those (without `write_kv` the key weight is not read). A row then has the bits of the two launches, the
+    first of them qk_norm_rope_store or, with `row_store`, qk_row_norm_rope_store."""
     n_pages, kv_heads, page_size, head_dim = k_cache.shape
     n = qkv.shape[0]
     if rule is None:
@@ -607,8 +608,8 @@ def attention_decode_qkv(qkv, q_weight, k_weight, eps: float, inv_freq, k_cache,
             qkv.data_ptr(), qkv.shape[1], int(bool(write_kv)),
             _dev(q_weight, "q norm weight", torch.float32, (heads * head_dim if whole else head_dim,)),
             _dev(k_weight, "k norm weight", torch.float32, (kv_heads * head_dim,) if whole and write_kv else None if whole else (head_dim,)),
-            float(eps), _dev(inv_freq, "inv_freq", torch.float32), n_freq, int(bool(interleaved)), float(magnitude), int(bool(whole)), k_cache.data_ptr(),
-            v_cache.data_ptr(), out.data_ptr(), _dev(part_o, "partial outputs", torch.float32),
+            float(eps), _dev(inv_freq, "inv_freq", torch.float32), n_freq, int(bool(interleaved)), float(magnitude), int(bool(whole)), int(bool(row_store)),
+            k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), _dev(part_o, "partial outputs", torch.float32),
             _dev(part_ml, "partial sums", torch.float32), _dev(rows, "decode rows", torch.int32), n_rows,
             _dev(seg_start, "seg_start", torch.int32), _dev(positions, "positions", torch.int32, (n,)),
             _dev(block_table, "block table", torch.int32), block_table.shape[1], page_size, heads, kv_heads, head_dim,

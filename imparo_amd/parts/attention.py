@@ -262,7 +262,8 @@ class Attention:
             ops.attention_decode_qkv(qkv, self.q_norm, self.k_norm, self.norm_eps, inv_freq, k_cache, v_cache, o,
                                      part_o, part_ml, ctx.single_rows, ctx.n_single_rows, ctx.seg_start,
                                      ctx.positions, table, self.heads, self.scale, self.window, ctx.max_context,
-                                     interleaved=interleaved, write_kv=owns_cache, rule=rule, magnitude=self.magnitude, whole=whole)
+                                     interleaved=interleaved, write_kv=owns_cache, rule=rule, magnitude=self.magnitude, whole=whole,
+                                     row_store=self.row_store)
             return self.out(ctx, o, torch.float32, "mixer_out", sliced_ok=True, into=ctx.stream)
         q = ctx.workspace.get("q", (T, self.heads, self.head_dim), ctx.dtype)
         where = (ctx.positions, ctx.row_of_token, table if owns_cache else None, ctx.page_size, q,
