@@ -349,16 +349,16 @@ __global__ __launch_bounds__(SplitF32<HD>::WAVES * WAVE, 1) void k_attention_spl
         there = p <= pos && (p >= lo || p < keep) && page >= 0 && page < n_pages;
         const int row = there ? (page * kv_heads + kvh) * page_size + p % page_size : 0;
         // 64 lanes ask for 1,024 bytes of neighbouring rows: a row a lane, each instruction would meet 64 lines
-        int at[PIECES];
+        unsigned at[PIECES];                                 // (a pool holds up to 2^32 numbers)
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
-            const int piece = i * WAVE + lane;
-            at[i] = __shfl(row, piece / PIECES) * HD + piece % PIECES * 4;
+            const unsigned piece = i * WAVE + lane;
+            at[i] = (unsigned)__shfl(row, piece / PIECES) * HD + piece % PIECES * 4;
         }
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) key[i] = *reinterpret_cast<const f32x4*>(k_cache + (size_t)(unsigned)at[i]);
+        for (int i = 0; i < PIECES; ++i) key[i] = *reinterpret_cast<const f32x4*>(k_cache + (size_t)at[i]);
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) v[i] = *reinterpret_cast<const f32x4*>(v_cache + (size_t)(unsigned)at[i]);
+        for (int i = 0; i < PIECES; ++i) v[i] = *reinterpret_cast<const f32x4*>(v_cache + (size_t)at[i]);
         }
         float* rows_lds = values + (size_t)wave * WAVE * LD;
         auto put = [&](const f32x4 (&piece)[PIECES]) __attribute__((always_inline)) {

@@ -35,3 +35,25 @@ def test_few_tokens_have_the_general_kernels_bits(H, Hk, D, window, keep, capped
         ops().attention(q, k, values, out, ctx.positions, ctx.row_of_token, table, 0.125, window, v_transposed=transposed, rule=rule)
         got.append(out.cpu())
     assert bool(torch.isfinite(got[0]).all()) and torch.equal(*got)
+
+
+def test_pages_behind_two_billion_numbers():
+    """A pool of more than 2^31 numbers (8 GiB of keys), keys in its last pages: a key's place is past what a signed int holds."""
+    H, Hk, D, page, n = 4, 2, 64, 16, 70
+    n_pages = 2 ** 31 // (Hk * page * D) + 40
+    held = list(range(n_pages - 5, n_pages))
+    ctx = hand_context([(n - 1, 1)], page, 8, torch.float32, DEV, kv_sites={0: (Hk, D)}, tables=[held])
+    g = torch.Generator().manual_seed(2)
+    k, v = (torch.empty(n_pages, Hk, page, D, device=DEV) for _ in range(2))
+    q = torch.randn(1, H, D, generator=g)
+    for cache in (k, v):
+        cache[held] = torch.randn(len(held), Hk, page, D, generator=g).to(DEV)
+    out = torch.full((1, H * D), float("nan"), device=DEV)
+    wide = torch.full((1, 8), -1, dtype=torch.int32, device=DEV)         # (room for more than one chunk of 64 keys)
+    wide[:, :len(held)] = ctx.block_tables[0]
+    ops().attention(q.to(DEV), k, v, out, ctx.positions, ctx.row_of_token, wide, 0.125, None)
+    keys, values = (c[held].cpu().double().transpose(0, 1).reshape(Hk, -1, D)[:, :n].repeat_interleave(H // Hk, 0) for c in (k, v))
+    weights = torch.softmax((keys @ q[0].double()[:, :, None])[..., 0] * 0.125, -1)
+    want = (weights[:, None] @ values)[:, 0].reshape(1, -1)
+    # (sums of 64 and of 70 products in float32)
+    torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -18, atol=2 ** -20)
