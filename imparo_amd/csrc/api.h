@@ -687,6 +687,7 @@ int imparo_stream_norm(const float* x, int in_streams, float* x_out, const float
 // a mixture's router (+ router_bias) in the same launch: route_choice and route_weight [n_rows, route_top + always] as
 // imparo_moe_route leaves them. The bits are those of imparo_stream_norm, of the product of few rows, and of imparo_moe_route.
 int imparo_stream_step_takes(int n_rows, int streams, int width, int n_delta, int top);
+int imparo_stream_step_pays(int streams, int width, int top);
 int imparo_stream_step_routes(int width, int n_router, int top);
 int imparo_stream_step(const float* x, int in_streams, float* x_out, const float* delta, int n_delta, const float* y,
                        const void* h, int h_dtype, const int32_t* choice, const float* choice_weight, int top, int n_experts,

@@ -428,6 +428,13 @@ extern "C" int imparo_stream_step_takes(int n_rows, int streams, int width, int 
     return n_rows >= 1 && n_rows <= 16 && streams >= 1 && streams <= 4 && width >= 256 && width <= 4096 && width % 256 == 0 &&
            (top > 0 ? top <= STREAM_STEP_TOP && n_delta == 0 : n_delta >= 1 && n_delta <= STREAM_STEP_DELTAS);
 }
+// ... and where that is the faster way without a router: a thread's copies and all that joins them, asked for at once, fit the registers
+// of a block of 1,024 threads in part only. One row, us here | k_stream_norm: a tensor joins, four copies of 1,024 3.45 | 3.62, of 1,280
+// 3.96 | 3.72, of 4,096 5.60 | 4.59, two of 4,096 3.98 | 4.04; eight experts' rows join, four copies of 1,280 4.96 | 4.56, of 4,096
+// 7.31 | 5.65, one or two of 2,048 faster here, one of 2,304 4.43 | 4.09, of 4,096 5.15 | 4.65.
+extern "C" int imparo_stream_step_pays(int streams, int width, int top) {
+    return streams > 2 ? width <= 1024 : top == 0 || width <= 2048;
+}
 // ... and whether a router of so many outputs rides: widths whose chunks of 128 come out as the product of few rows sums them.
 extern "C" int imparo_stream_step_routes(int width, int n_router, int top) {
     return width % 256 == 0 && (width <= 1024 || width == 2048) && n_router >= 1 && n_router <= STREAM_STEP_ROUTER && top >= 1 &&

@@ -90,6 +90,7 @@ _SIGNATURES = {
     "imparo_stream_norm": [P, I, P, P, I, P, P, I, P, P, P, I, I, I, P, I, P, P, P, I, P, P, F, P, I, I, I, P],
     "imparo_stream_max": [],
     "imparo_stream_step_takes": [I, I, I, I, I],
+    "imparo_stream_step_pays": [I, I, I],
     "imparo_stream_step_routes": [I, I, I],
     # x, in_streams, x_out, delta, n_delta, y, h, h_dtype, choice, choice_weight, top, n_experts, n_rows, streams, mix, join, read,
     # norm, weight, bias, eps, out, out_dtype, width, router_w, router_bias, correction, n_router, route_top, scoring, normalize,

@@ -168,7 +168,8 @@ def stream_norm(x: torch.Tensor, norm: str, weight: Optional[torch.Tensor], bias
         if rows is not None or delta is None:
             raise KernelArgumentError("stream_norm: the copies are written for every row, and where something joins them")
         _dev(x_out, "stream out", torch.float32, (n_x, width) if streams == 1 and x_out.dim() == 2 else (n_x, streams, width))
-    if x_out is not None and _stream_step_takes(x, out, delta, slices, n_delta, streams, weight, bias, x_out):
+    if (x_out is not None and _stream_step_takes(x, out, delta, slices, n_delta, streams, weight, bias, x_out)
+            and (route is not None or library().imparo_stream_step_pays(streams, width, delta.choice.shape[1] if moe[0] else 0))):
         by_entry = moe[0:5] + moe[6:] if moe[0] else (0, 0, 0, 0, 0, 0, 0)
         router = (0, 0, 0, 0, 0, 0, 0, 0.0, 0, 0, 0)
         if route is not None:
@@ -199,7 +200,7 @@ def stream_norm(x: torch.Tensor, norm: str, weight: Optional[torch.Tensor], bias
 
 
 def _stream_step_takes(x, out, delta, slices, n_delta: int, streams: int, weight, bias, x_out) -> bool:
-    """Whether stream_norm's call goes to the kernel of a decode step's rows."""
+    """Whether the kernel of a decode step's rows takes stream_norm's call; without a router it goes there where that pays too."""
     top = 0
     if delta is not None and not isinstance(delta, torch.Tensor):
         if not getattr(delta, "by_entry", False):
