@@ -754,8 +754,9 @@ int imparo_moe_route_plan(const float* logits, const float* correction, int32_t*
                           int32_t* slot_of_entry, int32_t* entry_of_slot, int32_t* tiles, int max_tiles,
                           int logits_ld, int groups, int keep, int normalize, float scale, int always, imparo_stream stream);
 // The router's product (x [n_tokens, k] by w [n_router, k], both bfloat16, plus bias), choice and plan of many tokens in two launches,
-// where imparo_moe_router_takes says so. counts: scratch of imparo_moe_router_blocks(n_tokens) x n_experts.
+// where imparo_moe_router_takes says so (and, to be the faster way, _pays). counts: scratch of imparo_moe_router_blocks(n_tokens) x n_experts.
 int imparo_moe_router_takes(int n_tokens, int n_router, int n_experts, int top, int groups, int always, int k);
+int imparo_moe_router_pays(int n_tokens, int n_router, int top, int k);
 int imparo_moe_router_blocks(int n_tokens);
 int imparo_moe_router_plan(const void* x, const void* w, const float* bias, const float* correction, int32_t* choice,
                            float* weight, int32_t* counts, int n_tokens, int n_router, int k, int top, int scoring,

@@ -488,6 +488,21 @@ extern "C" int imparo_moe_router_takes(int n_tokens, int n_router, int n_experts
            k >= 128 && k % 128 == 0;
 }
 
+// ... and where they are faster than the three. What they save is the plan by one block, 0.7 ns an entry, and a launch; what they cost is
+// that each 16 tokens read the whole router and one wave walks K, in rounds of as many blocks as the CUs' LDS holds at once (three a CU
+// with up to 9 outputs, two up to 21, one above). In one round K is walked as fast as the tiles walk it, in more it
+// is not, and the entries have to pay for that. Measured, us three launches | two, 4 chosen: 2,048 tokens of 1,024, 8 outputs 18.9 | 11.1, 32
+// outputs 20.0 | 14.5, of 8,192 46.2 | 49.0; 8,192 of 2,048, 32 outputs 44.8 | 35.9, of 4,096 52.2 | 61.9; 16,384 of 8,192, 22 outputs 102.5 | 164;
+// one chosen, 16 outputs of 2,048 37.0 | 38.4; 512 tokens of 128, 32 outputs 12.1 | 12.9. Of 931 forms one is slower by more than 2 %, by 3.
+extern "C" int imparo_moe_router_pays(int n_tokens, int n_router, int top, int k) {
+    const bool one_round = n_tokens <= (n_router <= 9 ? 3 : n_router <= 21 ? 2 : 1) * 256 * MOE_ROUTER_TOKENS;
+    if (n_router <= 9) return one_round || k <= 4096 * top;
+    if (n_router <= 21) return one_round ? k <= 4096 || n_tokens <= 4096 || top >= 4 : k <= 1280 * top;
+    if (!one_round) return top >= 2 && k <= 512 * top;
+    if (n_tokens < 2048) return n_router <= 24 || k >= 512 || n_tokens * top >= 4096;
+    return k <= 3072 || (top >= 4 && k <= 4096) || top >= 8;
+}
+
 extern "C" int imparo_moe_router_blocks(int n_tokens) { return (n_tokens + MOE_ROUTER_TOKENS - 1) / MOE_ROUTER_TOKENS; }
 
 extern "C" int imparo_moe_router_plan(const void* x, const void* w, const float* bias, const float* correction, int32_t* choice,

@@ -144,6 +144,7 @@ _SIGNATURES = {
     "imparo_moe_route_plan_tokens": [],
     "imparo_moe_route_plan": [P, P, P, P, I, I, I, I, I, I, P, P, P, I, I, I, I, I, F, I, P],
     "imparo_moe_router_takes": [I, I, I, I, I, I, I],
+    "imparo_moe_router_pays": [I, I, I, I],
     "imparo_moe_router_blocks": [I],
     # x, w, bias, correction, choice, weight, counts, n_tokens, n_router, k, top, scoring, normalize, scale, always, n_experts,
     # tile_rows, slot_of_entry, entry_of_slot, tiles, max_tiles, stream

@@ -1171,6 +1171,11 @@ def moe_router_takes(n_tokens: int, n_router: int, n_experts: int, top: int, gro
     return bool(library().imparo_moe_router_takes(int(n_tokens), int(n_router), int(n_experts), int(top), int(groups), int(always), int(k)))
 
 
+def moe_router_pays(n_tokens: int, n_router: int, top: int, k: int) -> bool:
+    """Whether that is faster than the product, the choice and the plan in launches of their own."""
+    return bool(library().imparo_moe_router_pays(int(n_tokens), int(n_router), int(top), int(k)))
+
+
 def moe_router_blocks(n_tokens: int) -> int:
     """The rows of `moe_router_plan`'s counts."""
     return int(library().imparo_moe_router_blocks(int(n_tokens)))

@@ -245,7 +245,8 @@ class RoutedExperts:
         # a prompt's router takes choice and plan along, where nothing else reads its logits
         rides = (routed is None and X > 0 and n.dtype == torch.bfloat16
                  and self.router.weight.dtype == torch.bfloat16 and not (self.shared is not None and self.shared_gated)
-                 and ops.moe_router_takes(T, self.n_router, X, top, self.group_count, self.always, self.width))
+                 and ops.moe_router_takes(T, self.n_router, X, top, self.group_count, self.always, self.width)
+                 and ops.moe_router_pays(T, self.n_router, top, self.width))
         z = None if routed is not None or rides else self.router(ctx, n, torch.float32, "router_logits")
         if shared_out is not None:
             shared_out.append(z)

@@ -10,3 +10,14 @@ from imparo_amd.kernels import library
 def test_a_step_norm_without_a_router(streams, width, top, pays):
     assert library().imparo_stream_step_takes(8, streams, width, 0 if top else 1, top)
     assert library().imparo_stream_step_pays(streams, width, top) == pays
+
+
+@pytest.mark.parametrize("tokens,outputs,top,k,pays", [
+    (129, 8, 1, 128, 1), (12288, 9, 1, 8192, 1), (12289, 9, 1, 4096, 1), (12289, 9, 1, 4224, 0), (16384, 8, 2, 8192, 1),
+    (4096, 16, 1, 8192, 1), (8192, 16, 1, 4096, 1), (8192, 16, 1, 8192, 0), (8192, 16, 4, 8192, 1), (8193, 21, 1, 1280, 1), (8193, 21, 1, 1408, 0),
+    (8193, 21, 2, 3072, 0), (129, 24, 4, 128, 1), (129, 32, 4, 128, 0), (1023, 32, 4, 384, 0), (1024, 32, 4, 384, 1), (512, 32, 4, 512, 1), (2048, 32, 4, 128, 1),
+    (2048, 32, 2, 3072, 1), (2048, 32, 2, 4096, 0), (2048, 32, 4, 4096, 1), (2048, 32, 4, 8192, 0), (4096, 32, 8, 8192, 1),
+    (4097, 32, 1, 128, 0), (8192, 22, 2, 1024, 1), (8192, 22, 2, 2048, 0), (8192, 32, 4, 2048, 1), (16384, 32, 4, 4096, 0)])
+def test_a_prompts_router_with_choice_and_plan(tokens, outputs, top, k, pays):
+    assert library().imparo_moe_router_takes(tokens, outputs, outputs, top, 1, 0, k)
+    assert library().imparo_moe_router_pays(tokens, outputs, top, k) == pays
