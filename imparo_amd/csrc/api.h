@@ -697,9 +697,10 @@ int imparo_stream_step(const float* x, int in_streams, float* x_out, const float
                        int scoring, int normalize, float route_scale, int always, int32_t* route_choice, float* route_weight,
                        imparo_stream stream);
 // A mixture's bfloat16 products for a step of few tokens (imparo_moe_direct_takes) straight from the tokens' choices [n_tokens,
-// used], without a plan: out has a row an entry, token * used + place in its list; own_rows: row t of `a` is read for every entry of
+// used], without a plan and faster by the launches of one where _pays says so; a token's choices differ. out has a row an entry, token * used + place in its list; own_rows: row t of `a` is read for every entry of
 // token t, else row t * used + j. w [n_experts, n, k], epilogues and limits as imparo_moe_gemm (gated: bfloat16 out, else float32).
 int imparo_moe_direct_takes(int n_tokens, int used, int n_experts);
+int imparo_moe_direct_pays(int n_tokens, int used, int n_experts, int width, int hidden);
 int imparo_moe_gemm_direct(const void* a, int a_ld, int own_rows, const int32_t* choice, int n_tokens, int used, int n_experts,
                            const void* w, void* out, int out_dtype, int n, int k, int epilogue, const float* limits, float alpha,
                            imparo_stream stream);

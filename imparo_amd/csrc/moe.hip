@@ -897,9 +897,10 @@ __global__ __launch_bounds__(512) void k_moe_gemm_dma(const bf16_t* __restrict__
 // few rows, by 12 % at the most.
 // DIRECT: no plan at all. A step of at most 16 tokens fits one tile of slots, so a block of expert `y` takes all tokens, finds
 // in their choices (`tiles`: [max_tiles tokens, gather_div used]) which of them use the expert, and leaves where nobody does;
-// rows of `out` (and of A, unless the tokens' own rows are read: bit 0 of `own_rows`) go by entry, token * used + place in its list. A row of the tile sums
-// over k as it does in any other, so results have the bits of planned ones. Worth the launch of the plan and not faster by
-// itself, cold weights, direct | planned us, gate and up, way back: 9 experts of 768 by 1,024, five a token, 1 token 6.8 | 5.9, 4.6 | 4.5,
+// rows of `out` (and of A, unless the tokens' own rows are read: bit 0 of `own_rows`) go by entry, token * used + place in its list
+// (a token's choices differ: of two entries with the same expert the first is made). A row of the tile sums
+// over k as it does in any other, so results have the bits of planned ones. Not faster by itself, and worth it for the launches that go
+// with the plan (imparo_moe_direct_pays): cold weights, direct | planned us, gate and up, way back: 9 experts of 768 by 1,024, five a token, 1 token 6.8 | 5.9, 4.6 | 4.5,
 // 8 tokens 8.1 | 8.3, 6.0 | 5.8; 16 of 512 by 2,048, four a token, 1 token 9.1 | 7.1, 4.5 | 4.0, 8 tokens 13.5 | 13.3, 8.1 | 7.5; 32 of
 // 512 by 1,024, four a token, whose blocks mostly leave, 8 tokens 11.0 | 9.9, 6.8 | 5.9.
 #define MOE_ROWS_WAVES 4
@@ -965,7 +966,9 @@ __global__ __launch_bounds__(MOE_ROWS_WAVES * 64) void k_moe_gemm_rows16(const b
             arow = A + (size_t)token * a_ld;
             ask_rows(run_lo);
         }
-        // (where hardly an expert goes unchosen its rows are asked for before that is known: one trip to memory less)
+        // (where hardly an expert goes unchosen its rows are asked for before that is known: one trip to memory less. From four
+        // entries an expert on; at two one in eight is unchosen, and its weights cost more than the trip: 16 experts of
+        // 2,048 by 1,024, two a token, 16 tokens a layer 46.3 -> 40.9 us without)
         if (own_rows & 2) ask_weights(run_lo);
         const unsigned long long lo = __ballot(lane < entries && choice[0] == expert);
         const unsigned long long hi = __ballot(lane + 64 < entries && choice[1] == expert);
@@ -1096,6 +1099,15 @@ static void launch_rows16(const bf16_t* a, int a_ld, int gather_div, const int32
 extern "C" int imparo_moe_direct_takes(int n_tokens, int used, int n_experts) {
     return n_tokens >= 1 && n_tokens <= MOE_DIRECT_TOKENS && used >= 1 && used <= MOE_DIRECT_USED && n_experts >= 1 && n_experts <= 24;
 }
+// ... and where a layer with them is the faster one, its router riding with the norm. That saves two launches, 4 to 6 us; the blocks of
+// experts that nobody chose, which grow with all experts' weights, cost more than that past some size. Norm, router, choice, both products
+// and the next norm in us, planned | so: 9 experts of 768 by 1,024, five a token, 1 token 25.2 | 21.3, 8 tokens 31.6 | 25.2; 16 of 2,048 by
+// 1,024, four, 8 tokens 43.7 | 38.8, of 4,096 by 1,024 16 tokens 76.0 | 80.7; 8 of 1,408 by 2,048, four, 1 token 36.1 | 35.8, 16 of 1,024
+// by 2,048 31.0 | 33.2. Of 864 forms with up to 16 experts none that goes this way is more than 1 % slower.
+extern "C" int imparo_moe_direct_pays(int n_tokens, int used, int n_experts, int width, int hidden) {
+    const long long all = (long long)n_experts * width * hidden;
+    return n_tokens * used <= 2 || (width <= 1024 ? all <= 32LL << 20 : all < 24LL << 20);
+}
 
 // own_rows: row t of `a` is read for every entry of token t, else row t * used + j for its j-th; out has a row an entry.
 extern "C" int imparo_moe_gemm_direct(const void* a, int a_ld, int own_rows, const int32_t* choice, int n_tokens, int used,
@@ -1106,7 +1118,7 @@ extern "C" int imparo_moe_gemm_direct(const void* a, int a_ld, int own_rows, con
     if (epilogue < MOE_EPI_NONE || epilogue > MOE_EPI_GATED) return IMPARO_BAD_ARGUMENT;
     hipStream_t s = (hipStream_t)stream;
     const MoeGate gate{limits, alpha, nullptr, 0};
-    const int flags = (own_rows ? 1 : 0) | (n_tokens * used >= 2 * n_experts ? 2 : 0);
+    const int flags = (own_rows ? 1 : 0) | (n_tokens * used >= 4 * n_experts ? 2 : 0);
     if (epilogue == MOE_EPI_GATED) {
         if (out_dtype != IMPARO_BF16 || n % 64) return IMPARO_BAD_ARGUMENT;
         launch_rows16<bf16_t, true, true>((const bf16_t*)a, a_ld, used, nullptr, (const bf16_t*)w, (bf16_t*)out, choice, n_tokens, n, k,

@@ -97,6 +97,7 @@ _SIGNATURES = {
     # route_scale, always, route_choice, route_weight, stream
     "imparo_stream_step": [P, I, P, P, I, P, P, I, P, P, I, I, I, I, P, P, P, I, P, P, F, P, I, I, P, P, P, I, I, I, I, F, I, P, P, P],
     "imparo_moe_direct_takes": [I, I, I],
+    "imparo_moe_direct_pays": [I, I, I, I, I],
     # a, a_ld, own_rows, choice, n_tokens, used, n_experts, w, out, out_dtype, n, k, epilogue, limits, alpha, stream
     "imparo_moe_gemm_direct": [P, I, I, P, I, I, I, P, P, I, I, I, I, P, F, P],
     # table, bigram, dtype, ids, positions, row_of_token, seg_start, seg_len, slot, state, x, n_tokens, n_rows, width, vocab,

@@ -1253,10 +1253,16 @@ def moe_direct_takes(n_tokens: int, used: int, n_experts: int) -> bool:
     return bool(library().imparo_moe_direct_takes(int(n_tokens), int(used), int(n_experts)))
 
 
+def moe_direct_pays(n_tokens: int, used: int, n_experts: int, width: int, hidden: int) -> bool:
+    """Whether a layer with such experts is faster so, its router riding with the norm, than with a plan."""
+    return bool(library().imparo_moe_direct_pays(int(n_tokens), int(used), int(n_experts), int(width), int(hidden)))
+
+
 def moe_gemm_direct(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, choice: torch.Tensor, own_rows: bool = False,
                     epilogue: Optional[str] = None, limits: Optional[torch.Tensor] = None, alpha: float = 1.0) -> torch.Tensor:
     """`moe_gemm` without a plan, for few tokens: out[entry] = epilogue(a[row] . w[choice of the entry]^T), entry = token * used +
-    place in `choice` [tokens, used], row the entry, or with `own_rows` the token. Entries of no expert are left as they are."""
+    place in `choice` [tokens, used], row the entry, or with `own_rows` the token. Entries of no expert are left as they are, and
+    so is a token's second entry with the same expert: a router's choices differ."""
     n_experts, n, k = w.shape
     tokens, used = choice.shape
     gated = epilogue == "gated"

@@ -217,7 +217,8 @@ class RoutedExperts:
         """The router, for the norm that hands this part its rows; None where it goes a launch of its own. The products then go
         by the tokens' choices: the plan, which takes all tokens, would be a launch again."""
         if (self.shared is not None or self.group_count > 1 or not self.fused or self.weigh != "output"
-                or not ops.moe_direct_takes(T, self.used, self.n_experts)):
+                or not ops.moe_direct_takes(T, self.used, self.n_experts)
+                or not ops.moe_direct_pays(T, self.used, self.n_experts, self.width, self.hidden_rows)):
             return None
         ws = ctx.workspace
         return RouterRide(self.router.weight, self.router.bias, self.correction, self.top, self.always, self.scoring, self.normalize,

@@ -21,3 +21,11 @@ def test_a_step_norm_without_a_router(streams, width, top, pays):
 def test_a_prompts_router_with_choice_and_plan(tokens, outputs, top, k, pays):
     assert library().imparo_moe_router_takes(tokens, outputs, outputs, top, 1, 0, k)
     assert library().imparo_moe_router_pays(tokens, outputs, top, k) == pays
+
+
+@pytest.mark.parametrize("tokens,used,experts,width,hidden,pays", [
+    (8, 5, 9, 1024, 768, 1), (16, 4, 16, 1024, 2048, 1), (16, 4, 16, 1024, 2080, 0), (16, 2, 8, 1024, 4096, 1), (4, 2, 12, 512, 5632, 0),
+    (1, 4, 8, 2048, 1408, 1), (1, 4, 12, 2048, 1024, 0), (1, 2, 16, 2048, 4096, 1), (2, 1, 16, 2048, 4096, 1), (1, 3, 16, 2048, 4096, 0)])
+def test_products_by_the_tokens_choices(tokens, used, experts, width, hidden, pays):
+    assert library().imparo_moe_direct_takes(tokens, used, experts)
+    assert library().imparo_moe_direct_pays(tokens, used, experts, width, hidden) == pays
