@@ -348,7 +348,7 @@ int imparo_attention_decode_qkv(const float* qkv, const float* q_weight, const f
 // query heads and over all key heads, weights as wide. far_first: a norm a head adds its squares in the order of
 // imparo_qk_row_norm_rope_store, else of imparo_qk_norm_rope_store: a row has the bits of the two launches.
 int imparo_attention_decode_qkv_ruled_takes(int heads, int kv_heads, int head_dim, int n_freq, int whole);
-int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int whole);
+int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int heads, int kv_heads, int brings, int whole, int far_first);
 int imparo_attention_decode_qkv_ruled(const float* qkv, int row_ld, int brings, const float* q_weight, const float* k_weight,
                                       float eps, const float* inv_freq, int n_freq, int interleaved, float magnitude, int whole, int far_first,
                                       void* k_cache, void* v_cache, void* out, float* part_o, float* part_ml,

@@ -1776,11 +1776,19 @@ extern "C" int imparo_attention_decode_qkv_ruled_takes(int heads, int kv_heads, 
     return head_dim == 64 && (n_freq == 0 || n_freq == 32) &&
            (!whole || ((long long)heads * head_dim <= WHOLE_Q && (long long)kv_heads * head_dim <= WHOLE_K));
 }
-// ... and for how many rows over how many splits it is the faster way. Launch behind launch, 16 heads by 8, one launch | two, us:
-// norms over all heads 1 row over 50 keys 7.2 | 8.3, 8 over 200 8.5 | 9.7, 8 over 1,000 12.0 | 13.4, 8 over 4,000 23.0 | 22.7, 16 over
-// 4,000 33.0 | 32.1, queries alone 30.0 | 31.2; a norm a head 8 over 200 8.2 | 10.9, 16 over 4,000 29.4 | 33.1.
-extern "C" int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int whole) {
-    return n_rows <= 16 && (long long)n_rows * n_splits <= (whole ? 128 : 1024);
+// ... and for how many rows over how many splits it is the faster way. Every block norms its queries, over whole rows the row, which
+// many rows of many kv heads over long contexts pay for more than for the launch. Launch behind launch, us, one launch | two. Norms over
+// all heads, 16 by 8: 1 row over 50 keys 7.8 | 8.8, 8 over 200 9.0 | 10.2, 16 over 1,900 21.0 | 23.2, 8 over 4,000 22.9 | 23.1, queries alone
+// 16 over 1,900 20.3 | 22.4; 32 by 16: 8 over 1,000 16.2 | 18.2, over 2,000 24.7 | 23.4, 1 over 16,000 21.7 | 23.4. A norm a head, 16 by 8:
+// 8 over 200 8.7 | 9.7, 16 over 4,000 30.5 | 31.3; 32 by 16: 16 over 1,900 28.9 | 31.7, over 4,000 52.3 | 49.7, queries alone 46.3 | 49.3. With
+// scaled sines (far_first), 8 by 8: 16 over 1,900 21.1 | 23.5, over 4,000 33.6 | 32.5.
+extern "C" int imparo_attention_decode_qkv_ruled_pays(int n_rows, int n_splits, int heads, int kv_heads, int brings, int whole,
+                                                      int far_first) {
+    const long long rows = n_rows, each = rows * kv_heads;
+    if (n_rows > 16 || rows * n_splits > (whole ? 128 : 1024)) return 0;
+    if (!brings) return 1;
+    if (whole) return n_splits <= 4 || each * (heads + kv_heads) <= 5120;
+    return n_splits <= 8 || each < (far_first && n_splits > 12 ? 128 : 256);
 }
 
 // The same under a rule, with exact weights, out of rows that may be wider than the heads (row_ld floats apart). brings: the

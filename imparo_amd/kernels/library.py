@@ -51,7 +51,7 @@ _SIGNATURES = {
     "imparo_attention_decode_qkv_takes": [I, I],
     "imparo_attention_decode_qkv_pays": [I, I],
     "imparo_attention_decode_qkv_ruled_takes": [I, I, I, I, I],
-    "imparo_attention_decode_qkv_ruled_pays": [I, I, I],
+    "imparo_attention_decode_qkv_ruled_pays": [I, I, I, I, I, I, I],
     "imparo_attention_prefill": [P, P, P, P, P, P, I, P, I, I, P, P, P, P, I, I, I, I, I, I, F, I, P],
     "imparo_attention_prefill_splits": [I, I, I, I, I],
     "imparo_attention_decode_split": [],

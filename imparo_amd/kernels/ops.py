@@ -563,9 +563,10 @@ def attention_decode_qkv_ruled_takes(heads: int, kv_heads: int, head_dim: int, n
     return bool(library().imparo_attention_decode_qkv_ruled_takes(int(heads), int(kv_heads), int(head_dim), int(n_freq), int(whole)))
 
 
-def attention_decode_qkv_ruled_pays(n_rows: int, keys: int, whole: bool) -> bool:
-    """Whether the one launch is the faster way under a rule, for rows that see at most so many `keys`."""
-    return bool(library().imparo_attention_decode_qkv_ruled_pays(int(n_rows), max(1, -(-int(keys) // decode_split())), int(whole)))
+def attention_decode_qkv_ruled_pays(n_rows: int, keys: int, heads: int, kv_heads: int, brings: bool, whole: bool, row_store: bool) -> bool:
+    """Whether the one launch is the faster way under a rule, for rows that see at most so many `keys`; `brings`: as `write_kv`."""
+    return bool(library().imparo_attention_decode_qkv_ruled_pays(int(n_rows), max(1, -(-int(keys) // decode_split())), int(heads),
+                                                                 int(kv_heads), int(brings), int(whole), int(row_store)))
 
 
 def attention_decode_qkv(qkv, q_weight, k_weight, eps: float, inv_freq, k_cache, v_cache, out, part_o, part_ml,

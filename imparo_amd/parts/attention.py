@@ -229,7 +229,8 @@ class Attention:
             return (owns_cache and not self.exact_weights and not self.row_store
                     and ops.attention_decode_qkv_pays(T, ctx.max_context) and ops.attention_decode_qkv_takes(self.head_dim, n_freq))
         keys = ops.attention_ruled_keys(ctx.max_context, self.window, self.rule)
-        return (row_ld % 4 == 0 and ops.attention_decode_qkv_ruled_pays(T, keys, whole)
+        return (row_ld % 4 == 0
+                and ops.attention_decode_qkv_ruled_pays(T, keys, self.heads, self.kv_heads, owns_cache, whole, self.row_store)
                 and ops.attention_decode_qkv_ruled_takes(self.heads, self.kv_heads, self.head_dim, n_freq, whole))
 
     def forward(self, ctx: StepContext, site: int, owns_cache: bool, h: torch.Tensor) -> torch.Tensor:

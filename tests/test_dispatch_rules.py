@@ -29,3 +29,13 @@ def test_a_prompts_router_with_choice_and_plan(tokens, outputs, top, k, pays):
 def test_products_by_the_tokens_choices(tokens, used, experts, width, hidden, pays):
     assert library().imparo_moe_direct_takes(tokens, used, experts)
     assert library().imparo_moe_direct_pays(tokens, used, experts, width, hidden) == pays
+
+
+@pytest.mark.parametrize("rows,splits,heads,kv_heads,brings,whole,far_first,pays", [
+    (16, 8, 16, 8, 1, 1, 1, 1), (16, 9, 16, 8, 1, 1, 1, 0), (16, 8, 32, 8, 1, 1, 1, 1), (8, 4, 32, 16, 1, 1, 1, 1), (8, 5, 32, 16, 1, 1, 1, 0),
+    (8, 8, 32, 16, 0, 1, 1, 1), (1, 64, 32, 16, 1, 1, 1, 1), (17, 1, 16, 8, 0, 0, 0, 0), (16, 64, 16, 8, 1, 0, 0, 1), (16, 65, 16, 8, 1, 0, 0, 0),
+    (16, 8, 32, 16, 1, 0, 0, 1), (16, 9, 32, 16, 1, 0, 0, 0), (16, 64, 32, 16, 0, 0, 0, 1), (8, 64, 32, 16, 1, 0, 0, 1),
+    (16, 12, 8, 8, 1, 0, 1, 1), (16, 13, 8, 8, 1, 0, 1, 0), (8, 64, 8, 8, 1, 0, 1, 1)])
+def test_attention_under_a_rule_from_the_projections_rows(rows, splits, heads, kv_heads, brings, whole, far_first, pays):
+    assert library().imparo_attention_decode_qkv_ruled_takes(heads, kv_heads, 64, 32, whole)
+    assert library().imparo_attention_decode_qkv_ruled_pays(rows, splits, heads, kv_heads, brings, whole, far_first) == pays
