@@ -1026,21 +1026,55 @@ __global__ void k_head_prepare(float* __restrict__ rows, int ld, int off, int n_
     for (int i = 2 * n_freq + lane; i < dim; i += WAVE) x[i] *= f;
 }
 
-// The same without a rotation, for heads of whole 16-byte pieces, at most one a lane: LANES lanes a head, which keep it in registers
-// where it was read twice, a value a lane at a time. Bound by its bytes. 3,328 rows of 8 heads of 128 as unit vectors 9.9 -> 6.5 us.
-template <int LANES>
+// The sum of squares of numbers that lie four a lane over 16 lanes, Q times (y[q][i]: number 64 q + 4 lane + i, zeros past the end), in
+// the order of a wave with a value a lane: a lane's numbers, 64 apart, one after the other, then lanes 32, 16, 8, 4, 2, 1 apart. So the
+// kernels in pieces and those that take any length give the same bits.
+template <int Q>
+__device__ __forceinline__ float squares_of_pieces(const float (&y)[Q][4]) {
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] = fmaf(y[q][i], y[q][i], s[i]);
+    // (the four sums go on in a quarter of the lanes each: seven moves between lanes and not sixteen)
+    const bool b8 = threadIdx.x & 8, b4 = threadIdx.x & 4;
+    const float first = (b8 ? s[2] : s[0]) + lane_xor<8>(b8 ? s[0] : s[2]);
+    const float second = (b8 ? s[3] : s[1]) + lane_xor<8>(b8 ? s[1] : s[3]);
+    float sum = (b4 ? second : first) + lane_xor<4>(b4 ? first : second);
+    sum += lane_xor<2>(sum);
+    sum += lane_xor<1>(sum);
+    sum += lane_xor<8>(sum);
+    sum += lane_xor<4>(sum);
+    return sum;
+}
+
+// The same without a rotation, for heads of whole 16-byte pieces: 16 lanes a head, four heads a wave, which keep it in registers where
+// it was read twice, a value a lane at a time. Bound by its bytes. 3,328 rows of 8 heads as unit vectors, us before and so: of 128 9.8 and
+// 5.5, of 64 7.5 and 4.0, of 256 16.0 and 8.1. (In 32 lanes a head with a sum of its own order 5.6, 4.8 and, in 64, 11.5.)
+template <int Q>
 __global__ __launch_bounds__(256) void k_head_prepare_four(float* __restrict__ rows, int ld, int off, int n_tokens, int heads, int dim,
                                                            int unit, float unit_eps, int n_first, float scale_first, float scale_rest) {
-    const int lane = threadIdx.x % LANES;
-    const long long all = (long long)n_tokens * heads, at = (long long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const int lane = threadIdx.x % 16;
+    const long long all = (long long)n_tokens * heads, at = (long long)blockIdx.x * 16 + threadIdx.x / 16;
     const long long id = at < all ? at : all - 1;            // (no lane leaves before the sums)
     const int t = (int)(id / heads), j = (int)(id - (long long)t * heads);
-    float4* x = reinterpret_cast<float4*>(rows + (size_t)t * ld + off + (size_t)j * dim) + min(lane, dim / 4 - 1);
-    const bool on = lane < dim / 4;
-    const float4 v = *x;
+    float* x = rows + (size_t)t * ld + off + (size_t)j * dim;
+    float y[Q][4];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = 64 * q + 4 * lane;
+        const float4 v = *reinterpret_cast<const float4*>(x + min(i, dim - 4));
+        const bool on = i < dim;
+        y[q][0] = on ? v.x : 0.f, y[q][1] = on ? v.y : 0.f, y[q][2] = on ? v.z : 0.f, y[q][3] = on ? v.w : 0.f;
+    }
     float f = j < n_first ? scale_first : scale_rest;
-    if (unit) f *= 1.0f / sqrtf(sum_near_first<LANES>(on ? fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, v.w * v.w))) : 0.f) + unit_eps);
-    if (on && at < all) *x = make_float4(v.x * f, v.y * f, v.z * f, v.w * f);
+    if (unit) f *= 1.0f / sqrtf(squares_of_pieces<Q>(y) + unit_eps);
+    if (at >= all) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int i = 64 * q + 4 * lane;
+        if (i < dim) *reinterpret_cast<float4*>(x + i) = make_float4(y[q][0] * f, y[q][1] * f, y[q][2] * f, y[q][3] * f);
+    }
 }
 
 extern "C" int imparo_head_prepare(float* rows, int ld, int off, int n_tokens, int heads, int dim, int unit,
@@ -1052,12 +1086,13 @@ extern "C" int imparo_head_prepare(float* rows, int ld, int off, int n_tokens, i
     if (n_tokens == 0) return IMPARO_OK;
     const long long waves = (long long)n_tokens * heads;
     if (!n_freq && dim % 4 == 0 && dim <= 256 && ld % 4 == 0 && off % 4 == 0 && !((uintptr_t)rows & 15)) {
-        if (dim <= 128)
-            k_head_prepare_four<32><<<(unsigned)((waves + 7) / 8), 256, 0, (hipStream_t)stream>>>(rows, ld, off, n_tokens, heads, dim, unit,
-                                                                                                unit_eps, n_first, scale_first, scale_rest);
-        else
-            k_head_prepare_four<64><<<(unsigned)((waves + 3) / 4), 256, 0, (hipStream_t)stream>>>(rows, ld, off, n_tokens, heads, dim, unit,
-                                                                                                unit_eps, n_first, scale_first, scale_rest);
+#define HEAD_FOUR(Q)                                                                                                 \
+    k_head_prepare_four<Q><<<(unsigned)((waves + 15) / 16), 256, 0, (hipStream_t)stream>>>(rows, ld, off, n_tokens, heads, dim, unit, \
+                                                                                         unit_eps, n_first, scale_first, scale_rest)
+        if (dim <= 64) HEAD_FOUR(1);
+        else if (dim <= 128) HEAD_FOUR(2);
+        else HEAD_FOUR(4);
+#undef HEAD_FOUR
         return launch_status();
     }
     k_head_prepare<<<(unsigned)((waves + 3) / 4), 4 * WAVE, 0, (hipStream_t)stream>>>(
@@ -1104,16 +1139,16 @@ __global__ __launch_bounds__(256) void k_gated_group_norm(const float* __restric
     }
 }
 
-// A short part of whole 16-byte pieces, Q of them a lane at most: LANES lanes a part, everything asked for at once and kept, where a
-// wave asked value by value and read the part and its gate again behind the sum. Bound by its bytes. 3,328 rows of 8 parts of 128, bfloat16
-// out, 15.5 -> 10.6 us.
-template <typename TOut, int LANES, int Q>
+// A short part of whole 16-byte pieces, Q of them a lane at most: 16 lanes a part, everything asked for at once and kept, where a wave
+// asked value by value and read the part and its gate again behind the sum. Bound by its bytes. 3,328 rows of 8 parts of 64, bfloat16 out,
+// 9.4 -> 6.5 us.
+template <typename TOut, int Q>
 __global__ __launch_bounds__(256) void k_gated_group_norm_four(const float* __restrict__ x, const float* __restrict__ gate,
                                                                int gate_ld, int gate_off, const float* __restrict__ w,
                                                                TOut* __restrict__ out, int n_tokens, int width, int groups,
                                                                float eps, int gate_first, int gate_act) {
-    const int lane = threadIdx.x % LANES, part = width / groups;
-    const long long all = (long long)n_tokens * groups, at = (long long)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
+    const int lane = threadIdx.x % 16, part = width / groups;
+    const long long all = (long long)n_tokens * groups, at = (long long)blockIdx.x * 16 + threadIdx.x / 16;
     const long long id = at < all ? at : all - 1;            // (no lane leaves before the sum)
     const int t = (int)(id / groups), g = (int)(id - (long long)t * groups);
     const float* xr = x + (size_t)t * width + (size_t)g * part;
@@ -1121,7 +1156,7 @@ __global__ __launch_bounds__(256) void k_gated_group_norm_four(const float* __re
     float y[Q][4], gv[Q][4], wv[Q][4];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const int i = min((lane + q * LANES) * 4, part - 4);
+        const int i = min(64 * q + 4 * lane, part - 4);
         const float4 a = *reinterpret_cast<const float4*>(xr + i);
         const float4 one = make_float4(1.f, 1.f, 1.f, 1.f);
         const float4 b = gr ? *reinterpret_cast<const float4*>(gr + i) : one;
@@ -1130,19 +1165,18 @@ __global__ __launch_bounds__(256) void k_gated_group_norm_four(const float* __re
         gv[q][0] = b.x, gv[q][1] = b.y, gv[q][2] = b.z, gv[q][3] = b.w;
         wv[q][0] = c.x, wv[q][1] = c.y, wv[q][2] = c.z, wv[q][3] = c.w;
     }
-    float ss = 0.f;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             gv[q][i] = gr ? ds_gate(gv[q][i], gate_act) : 1.f;
             if (gate_first) y[q][i] *= gv[q][i];
-            if ((lane + q * LANES) * 4 < part) ss = fmaf(y[q][i], y[q][i], ss);
+            if (64 * q + 4 * lane >= part) y[q][i] = 0.f;
         }
-    const float rs = 1.0f / sqrtf(sum_near_first<LANES>(ss) / (float)part + eps);
+    const float rs = 1.0f / sqrtf(squares_of_pieces<Q>(y) / (float)part + eps);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        const int i = (lane + q * LANES) * 4;
+        const int i = 64 * q + 4 * lane;
         float v[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
@@ -1155,6 +1189,46 @@ __global__ __launch_bounds__(256) void k_gated_group_norm_four(const float* __re
             *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
         else
             *reinterpret_cast<uint2*>(to) = make_uint2(f32x2_to_bf16x2(v[0], v[1]), f32x2_to_bf16x2(v[2], v[3]));
+    }
+}
+
+// A longer part of up to 64 PER numbers: a wave a part and a value a lane, as below, but everything asked for at once and kept, and a gate's
+// activation made once. 3,328 rows of 8 parts, bfloat16 out, of 128 13.7 -> 10.1 us, of 256 19.4 -> 15.1, of 512 33.9 -> 24.6 (16 bytes a
+// lane and 64 lanes a part, whose sum has to change lanes in mid-chain, 10.4, 18.3 and 33.6).
+template <typename TOut, int PER>
+__global__ __launch_bounds__(256) void k_gated_group_norm_kept(const float* __restrict__ x, const float* __restrict__ gate,
+                                                               int gate_ld, int gate_off, const float* __restrict__ w,
+                                                               TOut* __restrict__ out, int n_tokens, int width, int groups,
+                                                               float eps, int gate_first, int gate_act) {
+    const int lane = threadIdx.x & (WAVE - 1), part = width / groups;
+    const long long id = (long long)blockIdx.x * (256 / WAVE) + threadIdx.x / WAVE;
+    if (id >= (long long)n_tokens * groups) return;          // (whole waves)
+    const int t = (int)(id / groups), g = (int)(id - (long long)t * groups);
+    const float* xr = x + (size_t)t * width + (size_t)g * part;
+    const float* gr = gate ? gate + (size_t)t * gate_ld + gate_off + (size_t)g * part : nullptr;
+    float y[PER], gv[PER], wv[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int i = min(lane + 64 * p, part - 1);
+        y[p] = xr[i];
+        gv[p] = gr ? gr[i] : 1.f;
+        wv[p] = w ? w[(size_t)g * part + i] : 1.f;
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        if (gr) gv[p] = ds_gate(gv[p], gate_act);
+        if (gate_first) y[p] *= gv[p];
+        const float mine = lane + 64 * p < part ? y[p] : 0.f;
+        ss = fmaf(mine, mine, ss);
+    }
+    const float rs = 1.0f / sqrtf(wave_sum(ss) / (float)part + eps);
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int i = lane + 64 * p;
+        float v = y[p] * rs * wv[p];
+        if (!gate_first) v *= gv[p];
+        if (i < part) store_f32<TOut>(out, (size_t)t * width + (size_t)g * part + i, v);
     }
 }
 
@@ -1222,15 +1296,26 @@ extern "C" int imparo_gated_group_norm(const float* x, const float* gate, int ga
     }
     if (part % 4 == 0 && part <= 512 && gate_ld % 4 == 0 && gate_off % 4 == 0 &&
         !(((uintptr_t)x | (uintptr_t)gate | (uintptr_t)w | (uintptr_t)out) & 15)) {
-#define GGN_FOUR(T, LANES, Q)                                                                                        \
-    k_gated_group_norm_four<T, LANES, Q><<<(unsigned)((parts + 256 / LANES - 1) / (256 / LANES)), 256, 0, s>>>(      \
-        x, gate, gate_ld, gate_off, w, (T*)out, n_tokens, width, groups, eps, gate_first, gate_act)
+        // 16 lanes a part need fewer waves but go through a lane's numbers one after the other: for short parts, longer ones where there
+        // are very many. us, 16 lanes | a wave a part: 512 parts of 64 3.0 | 2.4; 106,000 of 96 26.1 | 32.8, of 128 31.9 |
+        // 35.3, 8,192 of 96 4.8 | 4.4, 26,624 9.5 | 10.0, of 128 11.2 | 10.3.
+        const bool few = part > 32 && parts < 4096, many = parts >= (part <= 96 ? 16384 : 65536);
+#define GGN_FOUR(T, Q)                                                                                               \
+    k_gated_group_norm_four<T, Q><<<(unsigned)((parts + 15) / 16), 256, 0, s>>>(x, gate, gate_ld, gate_off, w, (T*)out, n_tokens, width, \
+                                                                              groups, eps, gate_first, gate_act)
+#define GGN_KEPT(T, PER)                                                                                             \
+    k_gated_group_norm_kept<T, PER><<<(unsigned)((parts + 3) / 4), 256, 0, s>>>(x, gate, gate_ld, gate_off, w, (T*)out, n_tokens, width, \
+                                                                              groups, eps, gate_first, gate_act)
 #define GGN_FIT(T)                                                                                                   \
-    if (part <= 128) GGN_FOUR(T, 32, 1);                                                                             \
-    else if (part <= 256) GGN_FOUR(T, 64, 1);                                                                        \
-    else GGN_FOUR(T, 64, 2)
+    if (part <= 64 && !few) GGN_FOUR(T, 1);                                                                          \
+    else if (part <= 64) GGN_KEPT(T, 1);                                                                             \
+    else if (part <= 128 && !many) GGN_KEPT(T, 2);                                                                   \
+    else if (part <= 128) GGN_FOUR(T, 2);                                                                            \
+    else if (part <= 256) GGN_KEPT(T, 4);                                                                            \
+    else GGN_KEPT(T, 8)
         if (out_dtype == IMPARO_BF16) { GGN_FIT(bf16_t); } else { GGN_FIT(float); }
 #undef GGN_FIT
+#undef GGN_KEPT
 #undef GGN_FOUR
         return launch_status();
     }
