@@ -685,7 +685,7 @@ int imparo_stream_norm(const float* x, int in_streams, float* x_out, const float
 // joins is n_delta slices, or experts' rows that lie by entry, row t * top + j of y for the j-th expert in token t's list. With
 // router_w [n_router, width] bfloat16 (imparo_stream_step_routes; bfloat16 out, no groups) the row, as it is stored, goes on through
 // a mixture's router (+ router_bias) in the same launch: route_choice and route_weight [n_rows, route_top + always] as
-// imparo_moe_route leaves them. The bits are those of imparo_stream_norm, of the product of few rows, and of imparo_moe_route.
+// imparo_moe_route leaves them; they share no buffer with choice and choice_weight unless rows of both are as long. The bits are those of imparo_stream_norm, of the product of few rows, and of imparo_moe_route.
 int imparo_stream_step_takes(int n_rows, int streams, int width, int n_delta, int top);
 int imparo_stream_step_pays(int streams, int width, int top);
 int imparo_stream_step_routes(int width, int n_router, int top);

@@ -246,6 +246,7 @@ __global__ __launch_bounds__(1024) void k_stream_norm(
 // waves' sums in order), and the first wave chooses. 8 rows of 1,024 on four copies, one of 33 such launches of a step: behind a
 // mixture 6.0 -> 4.7 us; behind attention, with a router of 8 outputs, 7.7, where norm, product and choice took 6.0 + 4.2 + 4.0.
 // 8 chats of a mixture of 8 experts 32.0 -> 28.4 ms.
+// (A block of the framework norms the mixer's result before its mixture, so no router rides behind experts' rows there; the entry takes it.)
 #define STREAM_STEP_DELTAS 4
 #define STREAM_STEP_TOP 8
 #define STREAM_STEP_ROUTER 16
@@ -465,6 +466,14 @@ extern "C" int imparo_stream_step(const float* x, int in_streams, float* x_out, 
         if (!route_choice || !route_weight || always < 0 || route_top + always > MOE_MAX_USED || !(route_scale == route_scale))
             return IMPARO_BAD_ARGUMENT;
         if (scoring < MOE_SCORE_SOFTMAX || scoring > MOE_SCORE_CHOSEN) return IMPARO_BAD_ARGUMENT;
+        // a block reads its row of the choices that join and writes its row of the new ones: where both lie in one buffer the rows have
+        // to be the same ones, or a block would write what another has yet to read
+        const int used = route_top + always;
+        auto crosses = [&](const void* joins, const void* chosen) {
+            const uintptr_t a = (uintptr_t)joins, b = (uintptr_t)chosen, rows = (uintptr_t)n_rows * 4;
+            return joins && a < b + rows * used && b < a + rows * top && !(a == b && used == top);
+        };
+        if (y && (crosses(choice, route_choice) || crosses(choice_weight, route_weight))) return IMPARO_BAD_ARGUMENT;
     }
     hipStream_t s = (hipStream_t)stream;
     const StreamExperts moe{y, h, choice, choice_weight, nullptr, h_dtype == IMPARO_BF16, top, n_experts};

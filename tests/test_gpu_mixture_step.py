@@ -82,3 +82,34 @@ def test_the_step_norm_and_its_router_have_the_bits_of_their_launches(T, width, 
         monkeypatch.setattr(ops(), "_stream_step_takes", lambda *a: False)
     for a, b in zip(*got):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("before,always,taken", [(5, 1, True), (6, 1, False), (4, 1, False)])
+def test_choices_in_place_of_the_ones_that_join(before, always, taken):
+    """A router that rides behind experts' rows may write its choices where theirs lay if the rows are as long; of other lengths a
+    row's choices would lie where another row's are still read, and the call is refused."""
+    from imparo_amd.kernels import KernelArgumentError
+    T, width, top = 16, 1024, 4
+    used = top + always
+    x, weight, router = rnd(T, width, seed=1), rnd(width, seed=2), rnd(8, width, seed=3, dtype=torch.bfloat16)
+    choice = torch.stack([torch.randperm(9, generator=torch.Generator().manual_seed(i))[:before] for i in range(T)]).to(torch.int32).to(DEV)
+    shares = rnd(T, before, seed=4).abs()
+    y, h = rnd(T * before, width, seed=5), rnd(T, width, seed=6, dtype=torch.bfloat16)
+    got = []
+    for shared in (False, True):
+        buffers = [torch.zeros(T * 8, dtype=t.dtype, device=DEV) for t in (choice, shares)]
+        joins = [b[:T * before].view(T, before).copy_(t) for b, t in zip(buffers, (choice, shares))]
+        chosen = [b[:T * used].view(T, used) if shared else torch.zeros(T, used, dtype=b.dtype, device=DEV) for b in buffers]
+        delta = types.SimpleNamespace(y=y, h=h, choice=joins[0], weight=joins[1], n_experts=9, extra=None, by_entry=True,
+                                      slot_of_entry=torch.arange(T * before, dtype=torch.int32, device=DEV))
+        ride = types.SimpleNamespace(weight=router, bias=None, correction=None, top=top, always=always, scoring="chosen", normalize=False,
+                                     scale=1.0, choice=chosen[0], shares=chosen[1])
+        out, moved = torch.empty(T, width, dtype=torch.bfloat16, device=DEV), torch.empty(T, 1, width, device=DEV)
+        run = lambda: ops().stream_norm(x, "rms", weight, None, 1e-5, out, delta=delta, x_out=moved, streams=1, route=ride)
+        if shared and not taken:
+            with pytest.raises(KernelArgumentError):
+                run()
+            return
+        run()
+        got.append((out, moved, *chosen))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
