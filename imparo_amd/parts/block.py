@@ -150,7 +150,7 @@ class HyperBlock:
         if len({self.ffn is None, self.ffn_norm is None, self.ffn_link is None}) > 1:
             raise ValueError("a block has a feed-forward, the norm before it and its link, or none of them")
         # whether the feed-forward's router may ride with the norm: both have to say so of the methods they run
-        self.routes = (emits(self.ffn_norm, "routes", "forward_linked")
+        self.routes = (all(emits(self.ffn_norm, "routes", run) for run in ("forward_linked", "_read"))
                        and all(emits(self.ffn, "router_ride", run) for run in ("forward", "forward_parts", "_parts", "_rows")))
 
     def cache_spec(self, page_size: int):

@@ -69,7 +69,8 @@ class LinkedNorm:
                        name: str = "normed", route=None) -> torch.Tensor:
         """`forward` for a sublayer with a link of its own: the normed sum of the copies, weighed by its `read`. `route`: the
         sublayer's router, which the launch takes along where it can."""
-        return self._read(ctx, res, link, ctx.workspace.get(name, tuple(res.x.shape), out_dtype), route=route)
+        more = {} if route is None else dict(route=route)        # (a norm with a `_read` of its own may know no routers)
+        return self._read(ctx, res, link, ctx.workspace.get(name, tuple(res.x.shape), out_dtype), **more)
 
 
 class RmsNorm(LinkedNorm):

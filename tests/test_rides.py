@@ -5,9 +5,9 @@ import types
 import pytest
 import torch
 
-from imparo_amd.parts import attention, channel_delta, ffn, mixer_pair, norm, retention
+from imparo_amd.parts import attention, channel_delta, ffn, mixer_pair, moe, norm, retention
 from imparo_amd.parts.base import Residual, emits
-from imparo_amd.parts.block import PreNormBlock
+from imparo_amd.parts.block import HyperBlock, PreNormBlock
 
 
 new = lambda cls: cls.__new__(cls)
@@ -118,3 +118,25 @@ def test_both_sides_of_a_pair_are_asked():
         assert pair.forward(ctx, 0, True, torch.zeros(2, 8)) is ctx.stream
         assert (left.ride is None) == isinstance(left, Silent) and (left.ride is None or left.ride.norm is None)
         assert (right.ride is ride) == (not isinstance(right, Silent)) and (right.ride in (None, ride))
+
+
+class OwnRead(norm.RmsNorm):                     # a norm from outside that reads the stream in its own way
+    def _read(self, ctx, res, link, out, rows=None):
+        return out.fill_(3.0)
+
+
+@pytest.mark.parametrize("ffn_norm,feed,routes", [
+    (norm.RmsNorm, moe.RoutedExperts, True), (norm.LayerNorm, moe.RoutedExperts, True), (OwnRead, moe.RoutedExperts, False),
+    (type("OwnLinked", (norm.RmsNorm,), dict(forward_linked=lambda self, *a, **k: None)), moe.RoutedExperts, False),
+    (norm.RmsNorm, type("OwnRows", (moe.RoutedExperts,), dict(_rows=lambda self, *a: None)), False),
+    (norm.RmsNorm, type("OwnParts", (moe.RoutedExperts,), dict(forward_parts=None)), False), (norm.RmsNorm, ffn.SwiGlu, False)])
+def test_a_router_rides_where_norm_and_mixture_say_so_of_what_they_run(ffn_norm, feed, routes):
+    block = HyperBlock(dict(mixer_norm=new(norm.RmsNorm), mixer=new(attention.Attention), mixer_link=object(), ffn_norm=new(ffn_norm),
+                            ffn=new(feed), ffn_link=object()))
+    assert block.routes == routes
+
+
+def test_a_norm_with_a_read_of_its_own_runs_behind_copies():
+    ctx = types.SimpleNamespace(workspace=types.SimpleNamespace(get=lambda name, shape, dtype: torch.zeros(shape, dtype=dtype)))
+    rows = new(OwnRead).forward_linked(ctx, Residual(torch.zeros(2, 4)), object(), torch.float32)
+    assert torch.equal(rows, torch.full((2, 4), 3.0))
