@@ -57,3 +57,26 @@ def test_pages_behind_two_billion_numbers():
     want = (weights[:, None] @ values)[:, 0].reshape(1, -1)
     # (sums of 64 and of 70 products in float32)
     torch.testing.assert_close(out.cpu().double(), want, rtol=2 ** -18, atol=2 ** -20)
+
+
+@pytest.mark.parametrize("H,Hk,D", [(16, 8, 64), (32, 8, 64), (8, 2, 128)])
+@pytest.mark.parametrize("page", [8, 32, 64])
+@pytest.mark.parametrize("gated", [False, True])
+def test_portions_gates_and_other_pages_have_the_general_kernels_bits(H, Hk, D, page, gated):
+    """Several tokens of a request beside single ones, rows with a gate a head, pages of other sizes, rows of one chunk among long
+    ones."""
+    segments = [(0, 3), (60, 6), (63, 1), (300, 4), (40, 1), (700, 2)]
+    T, n_pages = sum(n for _, n in segments), sum(-(-(p + n) // page) for p, n in segments) + 1
+    ctx = hand_context(segments, page, n_pages, torch.float32, DEV, kv_sites={0: (Hk, D)})
+    g = torch.Generator().manual_seed(page)
+    k, v, q = (torch.randn(*s, generator=g).to(DEV) for s in ((n_pages, Hk, page, D), (n_pages, Hk, page, D), (T, H, D)))
+    rule = ops().attention_rule(H, softcap=8.0, out_scale=0.9)
+    if gated:
+        rule = rule.with_gate(torch.randn(T, H + 4, generator=g).to(DEV), 4)
+    got = []
+    for transposed in (False, True):
+        out = torch.full((T, H * D), float("nan"), device=DEV)
+        ops().attention(q, k, v.transpose(2, 3).contiguous() if transposed else v, out, ctx.positions, ctx.row_of_token, ctx.block_tables[0],
+                        0.125, None, v_transposed=transposed, rule=rule)
+        got.append(out.cpu())
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(*got)

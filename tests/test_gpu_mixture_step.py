@@ -113,3 +113,42 @@ def test_choices_in_place_of_the_ones_that_join(before, always, taken):
         run()
         got.append((out, moved, *chosen))
     assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("width", [256, 512, 768, 1024, 2048])
+@pytest.mark.parametrize("outputs,top,always", [(1, 1, 0), (5, 3, 1), (8, 4, 1), (9, 1, 2), (16, 8, 0), (16, 16, 3)])
+@pytest.mark.parametrize("biased,corrected", [(False, False), (True, False), (True, True)])
+@pytest.mark.parametrize("scoring,normalize", [("chosen", False), ("softmax", True), ("sigmoid", False)])
+def test_riding_routers_of_all_forms(width, outputs, top, always, biased, corrected, scoring, normalize):
+    """Choices and weights as the norm, the product of few rows with its bias, and the choice leave them in launches of their own."""
+    T, streams = 7, 3
+    x, delta = rnd(T, streams, width, seed=1), rnd(T, width, seed=2)
+    weight, bias = rnd(width, seed=3), rnd(width, seed=4)
+    mix, join, read = rnd(streams, streams, seed=5), rnd(streams, seed=6), rnd(streams, seed=7)
+    router = (rnd(outputs, width, seed=8) * width ** -0.5).to(torch.bfloat16)
+    router_bias, correction = rnd(outputs, seed=9) if biased else None, 0.3 * rnd(outputs, seed=10) if corrected else None
+    used = top + always
+    assert ops().stream_step_routes(x, delta, streams, weight, bias, router, top)
+    got = []
+    for rides in (True, False):
+        out, moved = torch.empty(T, width, dtype=torch.bfloat16, device=DEV), torch.empty(T, streams, width, device=DEV)
+        chosen, shares = torch.full((T, used), -7, dtype=torch.int32, device=DEV), torch.full((T, used), -7.0, device=DEV)
+        call = dict(delta=delta, mix=mix, join=join, read=read, x_out=moved)
+        if rides:
+            ride = types.SimpleNamespace(weight=router, bias=router_bias, correction=correction, top=top, always=always, scoring=scoring,
+                                         normalize=normalize, scale=1.25, choice=chosen, shares=shares)
+            ops().stream_norm(x, "layer", weight, bias, 1e-5, out, route=ride, **call)
+        else:
+            ops().stream_norm(x, "layer", weight, bias, 1e-5, out, **call)
+            z = torch.empty(T, outputs, device=DEV)
+            ops().gemm(out, router, z, bias=router_bias)
+            ops().moe_route(z, correction, chosen, shares, top, scoring=scoring, normalize=normalize, scale=1.25, always=always)
+        got.append((out, moved, chosen, shares))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    z = got[0][0].double() @ router.double().t() + (0 if router_bias is None else router_bias.double())
+    score = {"chosen": z, "softmax": torch.softmax(z, -1), "sigmoid": torch.sigmoid(z)}[scoring]
+    ranked = (score if correction is None else score + correction.double()).sort(-1, descending=True)
+    # (where no rounding of a sum of products of about one turns a choice)
+    sure = ((ranked.values[:, :-1] - ranked.values[:, 1:])[:, :top] > 1e-5).all(-1) if outputs > 1 else torch.ones(T, dtype=torch.bool, device=DEV)
+    assert torch.equal(got[0][2][sure, :top].long(), ranked.indices[sure, :top])
+    assert torch.equal(got[0][2][:, top:].cpu(), (outputs + torch.arange(always, dtype=torch.int32)).expand(T, always))
