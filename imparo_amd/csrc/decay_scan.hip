@@ -349,25 +349,25 @@ __device__ __forceinline__ f32x4 dc_product(const f32x4& x, const f32x4& y, f32x
     return acc;
 }
 
-// A pair j < t belongs to the level s = 1, 2, 4, 8 or 16 of the highest bit in which t and j differ: t in the second half of a run
-// of 2 s tokens, j in the first. With e the first half's last token, g_t / g_j = (g_t / g_e) (g_e / g_j), both at most one, and
-// neither leaves float32's range where their product does not. So a level is one product of 16 tokens by 16 over the
-// state's rows, on the matrix cores, of whose result the pairs that share a run count, and needs one exponential a
-// token and row, 5 for all levels, where pair by pair it was 16 and five reads of LDS a pair and row. Each wave has a
-// quarter of the state's rows; the four sums meet in LDS. Every thread asks for its column of k, q and steps at once, and sums
-// the steps up in registers. The triangle is inverted in two halves side by side and the block below them by two products.
-// Bound by what it reads and writes, 106 KB a chunk and head. Measured, 4 requests of 1,024 tokens, 8 heads of 128: 78.5 -> 41.5 us; one of
-// 2,048 44.5 -> 27.3; results 2.8e-7 -> 2.3e-7 from 64 bits.
+// Where the entries of L that have a use, below its diagonal, lie by column: each column from the last multiple of four at or above its
+// first one, so that a lane reads four tokens at once.
+__host__ __device__ constexpr int channel_column(int j) {
+    const int q = (j + 1) / 4;                               // the column's rows from 4 q on
+    return q == 0 ? j * DC : 3 * DC + 4 * (q - 1) * DC - 8 * q * (q - 1) + (j + 1) % 4 * (DC - 4 * q);
+}
+
+// Ratios of decays are exponentials of differences of the logarithms' sums, a pair j <= t and state row at a time, and a pair's sums run over
+// the state's rows in order. A thread has two neighbouring j of a t (256 such pieces below the diagonal), whose rows it reads four
+// numbers at a time out of LDS; every thread asks for its column of k, q and steps at once, and sums the steps up in registers;
+// a solved token of the triangle's inverse goes into all later ones side by side, and the other waves make what is left of the diagonal
+// meanwhile. Bound by the pairs' exponentials and reads of LDS and by its bytes, 106 KB a chunk and head. Measured, 4 requests of 1,024
+// tokens, 8 heads of 128: 44.5 us; one of 2,048 27.9. (With a pair a lane and numbers read one by one 78.5 and 44.5; ratios split at a
+// token between the two, so that they become products of 16 tokens by 16 on the matrix cores, 41.5 and 27.3, and other bits.)
 template <int DP>
 __global__ __launch_bounds__(256, 3) void k_channel_delta_prepare(const DecayScanArgs A) {
-    constexpr int LD = DP + 4, RUNS = 256 / DP, TOK = DC / RUNS, KL = DP / 16, LEVELS = 5;
-    constexpr int PART = DC * DC, TRI = DC + 1;
-    constexpr int FLOATS = 3 * DC * LD > 8 * PART + DC * TRI ? 3 * DC * LD : 8 * PART + DC * TRI;
-    __shared__ __attribute__((aligned(16))) float mem[FLOATS];   // k | q | logarithms; then the waves' sums, and L
-    __shared__ float sb[DC], diagonal[DC], total[DP];
-    float* const sk = mem;
-    float* const sq = mem + DC * LD;
-    float* const lg = mem + 2 * DC * LD;
+    constexpr int LD = DP + 4, RUNS = 256 / DP, TOK = DC / RUNS;
+    __shared__ __attribute__((aligned(16))) float sk[DC * LD], sq[DC * LD], lg[DC * LD], sL[channel_column(DC - 1)];
+    __shared__ float sb[DC], total[DP];
     const int r = blockIdx.x / A.max_chunks, chunk = blockIdx.x - r * A.max_chunks, h = blockIdx.y;
     const int tid = threadIdx.x, dim = A.dim, heads = A.heads;
     const int n_all = A.seg_len[r];
@@ -438,98 +438,70 @@ __global__ __launch_bounds__(256, 3) void k_channel_delta_prepare(const DecaySca
         }
         if (run == 0) ke_out[DC * DP + col] = __builtin_amdgcn_exp2f(last);
     }
-    const int lane = tid & (WAVE - 1), wave = tid / WAVE, c = lane & 15, g = lane >> 4;
-    {                                                    // q_t . k_t: eight threads a token
-        const int t = tid >> 3, at = t * LD + (tid & 7) * (DP / 8);
-        float sum = 0.f;
+    auto four = [&](const float* rows, int t, int k) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f32x4*>(rows + t * LD + k);
+    };
+    {
+        // piece tid: tokens t = 2 m - 1 and 2 m have m pieces each (31 has 16), j and j + 1 of a piece; with t odd the last one's j + 1 is t
+        int m = (int)((1.0f + sqrtf(1.0f + 4.0f * (float)tid)) * 0.5f);
+        if (m * (m - 1) > tid) --m;
+        if (m * (m + 1) <= tid) ++m;
+        const int at = tid - m * (m - 1), t = 2 * m - 1 + (at >= m ? 1 : 0), j = 2 * (at >= m ? at - m : at);
+        float kk[2] = {0.f, 0.f}, qk[2] = {0.f, 0.f};
+#pragma unroll 2
+        for (int k = 0; k < dim; k += 4) {               // (past dim: zeros)
+            const f32x4 lt = four(lg, t, k), kt = four(sk, t, k), qt = four(sq, t, k);
 #pragma unroll
-        for (int i = 0; i < DP / 8; ++i) sum = fmaf(sq[at + i], sk[at + i], sum);
+            for (int p = 0; p < 2; ++p) {
+                const f32x4 lj = four(lg, j + p, k), kj = four(sk, j + p, k);
 #pragma unroll
-        for (int m = 1; m < 8; m *= 2) sum += __shfl_xor(sum, m, WAVE);
-        if ((tid & 7) == 0) diagonal[t] = sum;
-    }
-    f32x4 kk[LEVELS], qk[LEVELS];
-#pragma unroll
-    for (int lv = 0; lv < LEVELS; ++lv) {
-        const int s = 1 << lv, t = (c / s * 2 + 1) * s + c % s, e = (c / s * 2 + 1) * s - 1;
-        const int at = wave * (DP / 4) + g * KL;         // (the state's rows in any order, the same on both sides)
-        kk[lv] = qk[lv] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = at; k < at + KL; k += 4) {
-            const f32x4 lt = *reinterpret_cast<const f32x4*>(&lg[t * LD + k]), le = *reinterpret_cast<const f32x4*>(&lg[e * LD + k]);
-            const f32x4 lj = *reinterpret_cast<const f32x4*>(&lg[(t - s) * LD + k]), kj = *reinterpret_cast<const f32x4*>(&sk[(t - s) * LD + k]);
-            const f32x4 kt = *reinterpret_cast<const f32x4*>(&sk[t * LD + k]), qt = *reinterpret_cast<const f32x4*>(&sq[t * LD + k]);
-            f32x4 a, b;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                a[i] = __builtin_amdgcn_exp2f(lt[i] - le[i]);
-                b[i] = kj[i] * __builtin_amdgcn_exp2f(le[i] - lj[i]);
+                for (int i = 0; i < 4; ++i) {
+                    const float w = kj[i] * __builtin_amdgcn_exp2f(lt[i] - lj[i]);
+                    kk[p] = fmaf(kt[i], w, kk[p]);
+                    qk[p] = fmaf(qt[i], w, qk[p]);
+                }
             }
-            kk[lv] = dc_product(kt * a, b, kk[lv]);
-            qk[lv] = dc_product(qt * a, b, qk[lv]);
+        }
+        const float b = sb[t];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            // (column j's place is channel_column(j), rows from 4 ((j + 1) / 4) on)
+            if (j + p < t) sL[channel_column(j + p) + t - ((j + p + 1) & ~3)] = kk[p] * b;
+            M_out[t * DC + j + p] = qk[p];
         }
     }
-    __syncthreads();                                     // k, q and the logarithms have been read
-    float* const part = mem + wave * 2 * PART;           // [t][j], of K K^T and of Q K^T
-#pragma unroll
-    for (int lv = 0; lv < LEVELS; ++lv) {
-        const int s = 1 << lv, j = c / s * 2 * s + c % s;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = 4 * g + i, t = (row / s * 2 + 1) * s + row % s;
-            if (row / s != c / s) continue;
-            part[t * DC + j] = kk[lv][i];
-            part[PART + t * DC + j] = qk[lv][i];
-        }
-    }
+    for (int i = tid; i < DC * DC; i += 256)             // above the diagonal
+        if (i % DC > i / DC) M_out[i] = 0.f;
     __syncthreads();
-    float* const sL = mem + 8 * PART;                    // [DC][TRI]
-    for (int i = tid; i < PART; i += 256) {
-        const int t = i / DC, j = i - t * DC;
-        float l = 0.f, m = j == t ? diagonal[t] : 0.f;
-        if (j < t) {
-            l = ((mem[i] + mem[2 * PART + i]) + (mem[4 * PART + i] + mem[6 * PART + i])) * sb[t];
-            m = (mem[PART + i] + mem[3 * PART + i]) + (mem[5 * PART + i] + mem[7 * PART + i]);
+    if (tid >= 256 - 16) {                               // the diagonal's even tokens
+        const int t = 2 * (tid - (256 - 16));
+        float qk = 0.f;
+        for (int k = 0; k < dim; k += 4) {
+            const f32x4 lt = four(lg, t, k), kt = four(sk, t, k), qt = four(sq, t, k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) qk = fmaf(qt[i], kt[i] * __builtin_amdgcn_exp2f(lt[i] - lt[i]), qk);
         }
-        sL[t * TRI + j] = l;
-        M_out[i] = m;
+        M_out[t * DC + t] = qk;
     }
-    __syncthreads();
-    if (wave) return;
-    // (I + L)^-1 diag(b): lanes 0 .. 15 the columns of the upper half's inverse, 16 .. 31 of the lower's, by forward
-    // substitution; the block below is -(lower inverse) L21 (upper inverse)
-    float* const inverse = mem;                          // [2][16][17]
-    if (lane < DC) {
-        const float* L = sL + (lane & 16) * (TRI + 1);
-        float x[16];
+    if (tid < DC) {
+        // column tid of (I + L)^-1 by forward substitution, then times b of that column
+        float x[DC];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            float acc = t == c ? 1.f : 0.f;
+        for (int t = 0; t < DC; ++t) x[t] = t == tid ? 1.f : 0.f;
 #pragma unroll
-            for (int j = 0; j < t; ++j) acc = fmaf(-L[t * TRI + j], x[j], acc);
-            x[t] = acc;
+        for (int j = 0; j < DC - 1; ++j) {
+#pragma unroll
+            for (int t = (j + 1) & ~3; t < DC; t += 4) {
+                const f32x4 l = *reinterpret_cast<const f32x4*>(&sL[channel_column(j) + t - ((j + 1) & ~3)]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (t + i > j) x[t + i] = fmaf(-l[i], x[j], x[t + i]);
+            }
         }
-        const float b = sb[lane];
+        const float b = sb[tid];
 #pragma unroll
-        for (int t = 0; t < 16; ++t) {
-            inverse[(g * 16 + t) * 17 + c] = x[t];
-            T_out[((lane & 16) + t) * DC + lane] = x[t] * b;
-            if (g == 1) T_out[t * DC + lane] = 0.f;
-        }
+        for (int t = 0; t < DC; ++t) T_out[t * DC + tid] = x[t] * b;
     }
-    wave_lds_sync();
-    f32x4 l21, upper, lower;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        l21[i] = sL[(16 + c) * TRI + 4 * g + i];
-        upper[i] = inverse[(4 * g + i) * 17 + c];
-        lower[i] = -inverse[(16 + c) * 17 + 4 * g + i];
-    }
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 below = dc_product(lower, dc_product(l21, upper, zero), zero);
-    const float b = sb[c];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) T_out[(16 + 4 * g + i) * DC + c] = below[i] * b;
 }
 
 // The walk: a segment's chunks in order, a block a (segment, head, run of 16 value columns), every product on the

@@ -46,3 +46,25 @@ def test_chunks_are_the_recurrence(d, dv, strength):
     error = lambda got, ref: ((got.cpu().double() - ref).norm() / ref.norm()).item()
     assert error(out, want.view(n, -1)) < 5e-6
     assert error(S, state) < 5e-6
+
+
+@pytest.mark.parametrize("d", [4, 33, 64, 65, 128])
+def test_a_pairs_sum_runs_over_the_state_rows_in_order(d):
+    # nothing decays and the first token alone has a key, of ones, and values of one: the result of token t in its chunk is then the sum of
+    # its query, one number after the other in float32, and everything else on the way is exact
+    H, dv, n = 2, 16, 64
+    q = torch.randn(n, H, d, generator=torch.Generator().manual_seed(d)) * 2.0 ** torch.arange(n)[:, None, None].remainder(5)
+    k, v = torch.zeros(n, H, d), torch.zeros(n, H, dv)
+    k[0], v[0] = 1.0, 1.0
+    rows = torch.cat([q.reshape(n, -1), k.view(n, -1), v.view(n, -1), torch.full((n, H), 100.0)], 1).to(DEV)
+    out, S = torch.empty(n, H * dv, device=DEV), torch.zeros(1, H, d, dv, device=DEV)
+    chunk_tokens, max_chunks = ops.channel_delta_chunks(n, d)
+    scratch = torch.empty(ops.channel_delta_scratch(1, max_chunks, H, d), device=DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ops.channel_delta_scan(rows, 0, 1, rows, H * d, 1, rows, 2 * H * d, torch.zeros(n, H * d, device=DEV), 0, torch.zeros(H * d, device=DEV),
+                           torch.zeros(H, device=DEV), rows, 2 * H * d + H * dv, S, i32([0]), i32([n]), i32([0]), out, H, d, dv,
+                           chunk_tokens=chunk_tokens, max_chunks=max_chunks, scratch=scratch)
+    want = torch.zeros(n, H)
+    for i in range(d):
+        want += q[:, :, i]
+    assert torch.equal(out.cpu().view(n, H, dv)[:chunk_tokens], want[:chunk_tokens, :, None].expand(-1, -1, dv))
