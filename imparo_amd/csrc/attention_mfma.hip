@@ -268,7 +268,7 @@ __device__ __forceinline__ void decode_tile(DecodeState<ND>& st, const DecodeTil
 // or (2i, 2i + 1) sit in one lane. Under a rule (EXT) heads of 64 only; the new key and value take their places in the loaded tile
 // there, so that a row has the bits of the two launches, and a layer without keys of its own brings queries alone. Bound by the
 // trips to memory behind one another, the rotation's float64 and the tiles' exponentials; 16 heads by 8, exact weights and a cap,
-// 8 rows over 200 keys 9.7 us in two launches and 8.5 in one, queries alone 9.1 and 7.0; 8 chats of a mixture 33.0 -> 32.1 ms.
+// 8 rows over 200 keys 9.7 us in two launches and 8.7 in one (norms over all heads 10.2 and 9.0), queries alone 9.1 and 7.0; 8 chats of a mixture 33.0 -> 32.1 ms.
 #define WHOLE_Q 2048            // the widest query part of a row, all heads, whose norm over all of it the kernel makes
 #define WHOLE_K 1024            // and the widest key part
 struct FromQkv {

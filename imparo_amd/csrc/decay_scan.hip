@@ -515,7 +515,8 @@ __global__ __launch_bounds__(256, 3) void k_channel_delta_prepare(const DecaySca
 // right behind the last use of this chunk's, into the same registers. Bound by the chunk's chain: 60 to 68 products of 32
 // cycles a wave, with the exchange in the middle. Measured, 4 requests of 1,024 tokens, 8 heads of 128, decays a channel: 88.3 us
 // with a chunk's 27 requests in a row and the sums read from LDS one by one, 74.4 now (50 with neither requests nor results); one of
-// 2,048 158 -> 129. Uniform bases with 32-bit offsets in place of whole addresses: 73.9 and 128.8, not kept.
+// 2,048 158 -> 129. With the first launch, one segment of 2,048, 16 heads: the delta rule, of 128 216 -> 205, of 64 157 -> 154, of 65 (numbers
+// one by one) 300 -> 275; plain decays, of 128 157 -> 157, of 64 123 -> 117, of 65 183 -> 164; same bits. Uniform bases with 32-bit offsets in place of whole addresses: 73.9 and 128.8, not kept.
 // KIND: a plain decay (U is V itself), the delta rule, the delta rule with decays a channel (whose operands the first
 // launch has laid out; the others read K and Q where they lie and scale rows of the results instead). VEC: K's and
 // Q's rows can be read in 16-byte pieces.

@@ -87,6 +87,6 @@ __device__ __forceinline__ void moe_route_token_narrow(const float* __restrict__
 
 // Counting costs by the output, choosing in rounds by the choice: 8,192 rows, counted | in rounds, 64 outputs: the best one 9.8 |
 // 7.6 us, two 10.0 | 9.4, four 10.4 | 13.2; 32 outputs: the best one 6.7 | 7.6.
-__host__ __device__ __forceinline__ bool moe_routes_narrow(int n_router, int top, const MoeRouteRules& rules) {
+__device__ __forceinline__ bool moe_routes_narrow(int n_router, int top, const MoeRouteRules& rules) {
     return n_router <= WAVE && rules.groups == 1 && (n_router <= 32 || top >= 3);
 }
