@@ -131,6 +131,8 @@ int imparo_attention_prefill_exact(const void* q, const void* k_cache, const voi
 // walks over at positions below max_context (the splits of a decode launch are counted from it). The wave kernel
 // likewise.
 int imparo_attention_ruled_keys(int max_context, int window, int keep_first);
+// Whether float32 attention of so few tokens goes to a block of several waves a token's kv head, where its tables have room for more than 64 keys.
+int imparo_attention_f32_split_pays(int n_tokens, int heads, int kv_heads, int head_dim, int window, int keep_first);
 int imparo_attention_decode_ruled(const void* q, const void* k_cache, const void* v_cache, void* out, float* part_o,
                                   float* part_ml, const int32_t* rows, int n_rows, const int32_t* seg_start,
                                   const int32_t* positions, const int32_t* block_table, int table_stride, int page_size,

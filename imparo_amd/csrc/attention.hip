@@ -341,12 +341,16 @@ __global__ __launch_bounds__(SplitF32<HD>::WAVES * WAVE, 1) void k_attention_spl
 #pragma unroll
     for (int j = 0; j < DPL; ++j) acc[j] = 0.f;
     // A round: W chunks, one a wave. A walk of one chunk (`alone_as`) has nothing for the other waves but its heads: one a wave, each with
-    // the chunk's keys and values of its own. 16 heads by 4 of 128 over 40 keys 13.4 -> 10.2 us (a block a head 10.4), 32 by 8 of 64
-    // 10.1 -> 7.5 (8.7). As branches in the code of the other rounds this cost those 0.3 to 0.7 us.
+    // the chunk's keys and values of its own, of those the sixteens of rows that hold keys (what LDS has in place of the others is not
+    // looked at). Launch behind launch, a block a head | so, 16 heads by 4 of 128: 5 keys 6.0 | 6.1 us, 40 keys 9.1 | 7.7, 32 by 8 of 64
+    // 5.4 | 4.8, 7.3 | 5.6 (16 by 4 with the whole chunk asked for 8.8 over 5 keys). As branches in the code of the other rounds this cost those 0.3 to 0.7 us.
     auto round = [&](auto alone_as, int first) __attribute__((always_inline)) {
         constexpr bool alone = decltype(alone_as)::value;
         const int slot = alone ? 0 : wave;                   // the chunk of this round that the wave makes
         const bool busy = alone ? wave < G : first + wave < chunks;      // (the last round: a wave may have none)
+        constexpr int QUARTER = PIECES / 4;
+        const int first_row = keep > 0 ? 0 : lo - start_of(0), rows_end = pos + 1 - start_of(0);
+        auto wanted = [&](int i) { return i / QUARTER * 16 < rows_end && i / QUARTER * 16 + 16 > first_row; };
         f32x4 key[PIECES], v[PIECES];
         bool there = false;
         if (busy) {
@@ -362,15 +366,24 @@ __global__ __launch_bounds__(SplitF32<HD>::WAVES * WAVE, 1) void k_attention_spl
             at[i] = (unsigned)__shfl(row, piece / PIECES) * HD + piece % PIECES * 4;
         }
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) key[i] = *reinterpret_cast<const f32x4*>(k_cache + (size_t)at[i]);
+        for (int i = 0; i < PIECES; i += QUARTER)
+            if (!alone || wanted(i))
 #pragma unroll
-        for (int i = 0; i < PIECES; ++i) v[i] = *reinterpret_cast<const f32x4*>(v_cache + (size_t)at[i]);
+                for (int j = i; j < i + QUARTER; ++j) key[j] = *reinterpret_cast<const f32x4*>(k_cache + (size_t)at[j]);
+#pragma unroll
+        for (int i = 0; i < PIECES; i += QUARTER)
+            if (!alone || wanted(i))
+#pragma unroll
+                for (int j = i; j < i + QUARTER; ++j) v[j] = *reinterpret_cast<const f32x4*>(v_cache + (size_t)at[j]);
         }
         float* rows_lds = values + (size_t)wave * WAVE * LD;
         auto put = [&](const f32x4 (&piece)[PIECES]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int i = 0; i < PIECES; ++i)
-                *reinterpret_cast<f32x4*>(rows_lds + (i * WAVE + lane) / PIECES * LD + lane % PIECES * 4) = piece[i];
+            for (int i = 0; i < PIECES; i += QUARTER)
+                if (!alone || wanted(i))
+#pragma unroll
+                    for (int j = i; j < i + QUARTER; ++j)
+                        *reinterpret_cast<f32x4*>(rows_lds + (j * WAVE + lane) / PIECES * LD + lane % PIECES * 4) = piece[j];
         };
         __syncthreads();                                     // (queries are there; the values before are read)
         float s[GMAX];
@@ -538,6 +551,21 @@ static int check_attention_args(const void* q, const void* k_cache, const void* 
     return IMPARO_OK;
 }
 
+// Whether few float32 tokens take k_attention_split_f32: heads of 64 or 128, at most four a kv head, as long as each token's kv head has
+// a CU of its own. Few keys of a window or a chunk that lie in two runs of 64 are two runs' reads there, for all heads of a wave, and with
+// three or four heads a kv head a block a head is the faster way: us, a block a head | so, one token, a window of 20, 16 heads by 4 of 128
+// over 130 keys 11.4 | 14.2, 32 by 8 of 64 over 1,100 8.8 | 9.7. As times of a block a head at worst, 16 by 4 of 128: windows of 40 1.20, of 56
+// 1.14, of 64 1.11, of 72 1.04, of 96 0.81, chunks of 20 1.31 and of 100 1.24; 32 by 8 of 64: 1.08, 1.04, 1.02, 1.01, 0.82, 1.13 and 1.09; 12 by
+// 4 of 128: a window of 8 1.35, of 40 1.03; up to two heads a kv head 0.95 for all. Chunks that start with a run of 64 have few keys in one run only.
+extern "C" int imparo_attention_f32_split_pays(int n_tokens, int heads, int kv_heads, int head_dim, int window, int keep_first) {
+    if (heads < 1 || kv_heads < 1 || heads % kv_heads || (head_dim != 64 && head_dim != 128)) return 0;
+    const int G = heads / kv_heads;
+    if (G > 4 || (long long)n_tokens * kv_heads > 256) return 0;
+    if (window == 0 || keep_first > 0 || G <= 2) return 1;
+    if (G == 3) return head_dim == 64 || window >= 32 || window <= -32;
+    return window > 0 ? window >= 80 : window <= -128 || window % WAVE == 0;
+}
+
 // Keys of head_dim and values of value_dim a head: q [tokens, heads, head_dim], the value cache
 // [pages, kv_heads, page, value_dim] (or transposed inside the page), out [tokens, out_ld] with out_ld >=
 // heads * value_dim; what lies beyond the heads in a row is written as zeros.
@@ -571,9 +599,9 @@ static int attention_wave(const void* q, const void* k_cache, const void* v_cach
     // and 1,146) and short contexts (4 prompts of 100 tokens, 64 heads 251 and 216; one of 333 537 and 554).
     const long long room = (long long)table_stride * page_size;
     const bool one = room <= WAVE, few = total <= 4096;
-    // Few tokens: a block of several waves for a token's kv head (k_attention_split_f32), as long as each has a CU of its own.
+    // Few tokens: a block of several waves for a token's kv head (k_attention_split_f32).
     const int G = heads / kv_heads;
-    if (plain && (head_dim == 64 || head_dim == 128) && !one && G <= 4 && (long long)n_tokens * kv_heads <= 256 && !((uintptr_t)v_cache & 15) &&
+    if (plain && !one && imparo_attention_f32_split_pays(n_tokens, heads, kv_heads, head_dim, window, r.keep_first) && !((uintptr_t)v_cache & 15) &&
         (long long)n_pages * kv_heads * page_size * head_dim < (1LL << 32)) {
 #define SPLIT_F32(HD, GMAX)                                                                                             \
     return launch_split_f32<HD, GMAX>((const float*)q, (const float*)k_cache, (const float*)v_cache, (float*)out, positions, row_of_token, \

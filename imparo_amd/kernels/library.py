@@ -48,6 +48,7 @@ _SIGNATURES = {
     "imparo_attention_prefill_ruled": [P, P, P, P, P, P, I, P, I, I, P, P, P, P, I, I, I, I, I, I, F, I, P, P],
     "imparo_attention_ruled": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, I, F, I, I, P, P],
     "imparo_attention_ruled_keys": [I, I, I],
+    "imparo_attention_f32_split_pays": [I, I, I, I, I, I],
     "imparo_attention_decode_qkv_takes": [I, I],
     "imparo_attention_decode_qkv_pays": [I, I],
     "imparo_attention_decode_qkv_ruled_takes": [I, I, I, I, I],

@@ -39,3 +39,12 @@ def test_products_by_the_tokens_choices(tokens, used, experts, width, hidden, pa
 def test_attention_under_a_rule_from_the_projections_rows(rows, splits, heads, kv_heads, brings, whole, far_first, pays):
     assert library().imparo_attention_decode_qkv_ruled_takes(heads, kv_heads, 64, 32, whole)
     assert library().imparo_attention_decode_qkv_ruled_pays(rows, splits, heads, kv_heads, brings, whole, far_first) == pays
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,dim,window,keep,pays", [
+    (1, 16, 4, 128, 0, 0, 1), (64, 16, 4, 128, 0, 0, 1), (65, 16, 4, 128, 0, 0, 0), (1, 20, 4, 64, 0, 0, 0), (1, 16, 8, 96, 0, 0, 0),
+    (1, 16, 4, 128, 79, 0, 0), (1, 16, 4, 128, 80, 0, 1), (1, 32, 8, 64, 20, 0, 0), (1, 32, 8, 64, 20, 4, 1), (1, 32, 8, 64, -20, 0, 0), (1, 32, 8, 64, -64, 0, 1),
+    (1, 32, 8, 64, -100, 0, 0), (1, 32, 8, 64, -200, 0, 1), (1, 12, 4, 128, 31, 0, 0), (1, 12, 4, 128, 32, 0, 1), (1, 12, 4, 128, -20, 0, 0), (1, 24, 8, 64, 8, 0, 1),
+    (1, 16, 8, 128, 1, 0, 1), (1, 8, 8, 64, -20, 0, 1)])
+def test_float32_attention_of_few_tokens(tokens, heads, kv_heads, dim, window, keep, pays):
+    assert library().imparo_attention_f32_split_pays(tokens, heads, kv_heads, dim, window, keep) == pays

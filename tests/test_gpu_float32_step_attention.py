@@ -80,3 +80,20 @@ def test_portions_gates_and_other_pages_have_the_general_kernels_bits(H, Hk, D, 
                         0.125, None, v_transposed=transposed, rule=rule)
         got.append(out.cpu())
     assert bool(torch.isfinite(got[0]).all()) and torch.equal(*got)
+
+
+@pytest.mark.parametrize("H,Hk,D", [(16, 8, 64), (32, 8, 64), (4, 1, 128), (2, 2, 128)])
+@pytest.mark.parametrize("window", [None, 1, 16, 17, -64, -96])
+def test_sixteens_of_a_walks_only_chunk_have_the_general_kernels_bits(H, Hk, D, window):
+    """Contexts, and windows inside one run of 64 keys, that end or start on sixteens of its rows and beside them."""
+    lens, page = (1, 15, 16, 17, 31, 33, 48, 49, 63, 64, 80, 97, 128), 16
+    R, n_pages = len(lens), sum(-(-c // page) for c in lens) + 2
+    ctx = hand_context([(c - 1, 1) for c in lens], page, n_pages, torch.float32, DEV, kv_sites={0: (Hk, D)})
+    g = torch.Generator().manual_seed(2)
+    k, v, q = (torch.randn(*s, generator=g).to(DEV) for s in ((n_pages, Hk, page, D), (n_pages, Hk, page, D), (R, H, D)))
+    got = []
+    for values, transposed in ((v, False), (v.transpose(2, 3).contiguous(), True)):
+        out = torch.full((R, H * D), float("nan"), device=DEV)
+        ops().attention(q, k, values, out, ctx.positions, ctx.row_of_token, ctx.block_tables[0], 0.125, window, v_transposed=transposed)
+        got.append(out.cpu())
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(*got)
